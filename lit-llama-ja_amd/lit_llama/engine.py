@@ -23,6 +23,8 @@ ones.
 """
 from __future__ import annotations
 
+import weakref
+
 import torch
 
 from . import _hip
@@ -30,13 +32,26 @@ from .model import LLaMA, _Work, _enable_i8_handoff
 from .state import Rows
 
 
-class LLaMAProgram:
+class _Program:
+    """The session owns its program; the program only refers to it. A reference cycle would leave the session's captured
+    graph to the garbage collector, and freeing a graph synchronizes the device, which aborts the process when it
+    happens in the middle of another session's capture."""
+
+    def __init__(self, sess: "DecodeSession"):
+        self._sess = weakref.ref(sess)
+
+    @property
+    def sess(self) -> "DecodeSession":
+        return self._sess()
+
+
+class LLaMAProgram(_Program):
     """Prompt and step launches of LLaMA.forward's blocks over the ring K / V caches; one position for all rows."""
 
     npos = 1
 
     def __init__(self, sess: "DecodeSession"):
-        self.sess = sess
+        super().__init__(sess)
         self.dev = sess.model.transformer.wte.weight.device
         _hip.require_device(sess.model.transformer.wte.weight, "model")
 
@@ -98,11 +113,11 @@ class LLaMAProgram:
         raise NotImplementedError("rows of this model share one position: the batch ends together")
 
 
-class HybridProgram:
+class HybridProgram(_Program):
     """Prompt and step launches of a model with per-sequence state (run / new_state); a position per row."""
 
     def __init__(self, sess: "DecodeSession"):
-        self.sess = sess
+        super().__init__(sess)
         self.npos = sess.B
         self.dev = sess.model.device
         self.state = sess.state if sess.state is not None else sess.model.new_state(sess.B, sess.S)
