@@ -333,6 +333,12 @@ int llj_g_rmsnorm(const void* x, int ldx, const void* w, float eps, void* y, int
  * (q - zero) * scale in fp32 (quantization.py:250-267, 390-409). */
 int llj_g_linear(int wkind, const void* x, int ldx, int M, int K, const void* W, const float* scales, const float* zeros,
                  int bits, int group, int N, void* y, int ldy, const void* resid, int ldr, int dt, void* stream);
+/* The same with scratch: the K range of a product with few output tiles is split over workgroups, whose fp32 sums meet in ws
+ * (llj_g_linear_ws_bytes of it; 0: not split. A smaller or NULL ws: not split either). */
+size_t llj_g_linear_ws_bytes(int wkind, int M, int N, int K, int dt);
+int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void* W, const float* scales, const float* zeros,
+                    int bits, int group, int N, void* y, int ldy, const void* resid, int ldr, int dt, void* ws, size_t ws_bytes,
+                    void* stream);
 /* c_attn output qkv (B*T, 3C) -> q_out (B*T, C) with RoPE, k (RoPE) / v into cache slot pos[t] % S
  * (model.py:204-228, 312-329); rope (block_size, hs/2, 2) fp32; head size even. */
 int llj_g_rope_kv(const void* qkv, void* q_out, void* kcache, void* vcache, const float* rope, const int* pos, int B, int T,

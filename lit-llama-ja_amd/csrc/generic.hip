@@ -1,14 +1,14 @@
 // The any-shape path: LLaMA configurations the streaming kernels do not tile -- n_embd % 128 != 0
 // or a head size other than 64 / 128. The JA fork's own 125M config (n_embd 780, head 78; reference
 // lit_llama/model.py:48-51) and the reference test's n_embd 32 / head 2 (tests/test_model.py:108-112)
-// run here. Plain kernels: one output per wave (linear) or per thread, fp32 accumulation, the
-// reference's bf16 rounding points (the same ones the fast kernels keep). Slower by design: these
-// shapes are small models, and none of them is the headline workload.
+// run here: tiled matrix products from 9 rows on (generic_gemm.h), below that one output column per
+// wave, fp32 accumulation, the reference's bf16 rounding points (the same ones the fast kernels keep).
 // Every kernel also runs in fp32 (dt = 1: activations, dense weights, KV cache and logits fp32, no
 // bf16 rounding -- the reference's float32 model, e.g. evaluate/full.py's default dtype and the
 // CPU config of generate.py:121): LLaMA.forward routes an fp32 model here whatever its shape.
 #include "common.h"
 #include "elem.h"
+#include "generic_gemm.h"
 #include "lit_llama_amd.h"
 
 namespace llj {
@@ -314,21 +314,99 @@ int llj_g_rmsnorm(const void* x, int ldx, const void* w, float eps, void* y, int
   return 0;
 }
 
-int llj_g_linear(int wkind, const void* x, int ldx, int M, int K, const void* W, const float* scales, const float* zeros,
-                 int bits, int group, int N, void* y, int ldy, const void* resid, int ldr, int dt, void* stream) {
+size_t llj_g_linear_ws_bytes(int wkind, int M, int N, int K, int dt) {
+  if (M <= GL_ROWS || N <= 0 || K <= 0) return 0;
+  const int s = gg_splits(M, N, K, dt == 1 || wkind == 0, dt == 1 && K <= kGgFineK);
+  return s > 1 ? (size_t)s * M * N * 4 : 0;
+}
+
+int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void* W, const float* scales, const float* zeros,
+                    int bits, int group, int N, void* y, int ldy, const void* resid, int ldr, int dt, void* ws, size_t ws_bytes,
+                    void* stream) {
   LLJ_REQUIRE(x && W && y && M > 0 && K > 0 && N > 0 && ldx >= K && ldy >= N && (!resid || ldr >= N) && (dt == 0 || dt == 1));
   LLJ_REQUIRE(wkind == 1 || (wkind == 0 && scales && zeros && (bits == 2 || bits == 4 || bits == 8) && group > 0 &&
                              K % (8 / bits) == 0));
-  const dim3 grid((N + 3) / 4, (M + GL_ROWS - 1) / GL_ROWS);
   hipStream_t s = (hipStream_t)stream;
+  if (M <= GL_ROWS) {
+    const dim3 grid((N + 3) / 4, 1);
 #define LLJ_GL(WK, T) \
   hipLaunchKernelGGL((g_linear_kernel<WK, T>), grid, dim3(256), 0, s, (const T*)x, ldx, M, K, W, scales, zeros, \
                      WK == 1 ? 16 : bits, WK == 1 ? K : group, N, (T*)y, ldy, (const T*)resid, ldr)
-  if (wkind == 1) LLJ_DT(dt, LLJ_GL(1, bf16_t), LLJ_GL(1, float));
-  else LLJ_DT(dt, LLJ_GL(0, bf16_t), LLJ_GL(0, float));
+    if (wkind == 1) LLJ_DT(dt, LLJ_GL(1, bf16_t), LLJ_GL(1, float));
+    else LLJ_DT(dt, LLJ_GL(0, bf16_t), LLJ_GL(0, float));
 #undef LLJ_GL
+    LLJ_CHECK_LAUNCH();
+    return 0;
+  }
+  const bool f32 = dt == 1 || wkind == 0;  // bf16 rows on codes: the weight element (q - zero) * scale is fp32
+  int splits = ws ? gg_splits(M, N, K, f32, dt == 1 && K <= kGgFineK) : 1;
+  if (splits > 1 && ws_bytes < (size_t)splits * M * N * 4) splits = 1;
+  const int kt = kGgRow / (f32 ? 4 : 2), all = (K + kt - 1) / kt, per = (all + splits - 1) / splits;
+  const int mt = (M + kGgBM - 1) / kGgBM, nt = (N + kGgBN - 1) / kGgBN;
+  LLJ_REQUIRE((long)((nt + 7) / 8) * 8 * mt < (1L << 31));
+  const dim3 grid((nt + 7) / 8 * 8 * mt, splits);
+  float* part = splits > 1 ? (float*)ws : nullptr;
+  // elements per load: 16, 8 (bf16) or single elements, as the rows of x and of a dense W are aligned
+  const int el = dt == 1 ? 4 : 2;
+  auto fits = [&](const void* p, int ld, int n) { return (uintptr_t)p % (n * el) == 0 && ld % n == 0 && K % n == 0; };
+  // WL: loader of J accumulators per wave (512 / J threads)
+#define LLJ_GG_RUN(T, CT, VEX, J, FINE, ...)                                                                                  \
+  do {                                                                                                                        \
+    typedef __VA_ARGS__ wl;                                                                                                   \
+    hipLaunchKernelGGL((gg_kernel<wl, T, CT, VEX, J, FINE>), grid, dim3(512 / J), 0, s, (const T*)x, ldx, M, K, W, scales,    \
+                       zeros, wkind == 1 ? K : group, N, (T*)y, ldy, (const T*)resid, ldr, part, per);                        \
+  } while (0)
+  const bool fine = dt == 1 && K <= kGgFineK;
+#define LLJ_GG_F32(VE)                                                      \
+  do {                                                                      \
+    if (fine) LLJ_GG_RUN(float, float, VE, 1, true, GgWeightDense<float, VE, 512>); \
+    else LLJ_GG_RUN(float, float, VE, 2, false, GgWeightDense<float, VE, 256>);     \
+  } while (0)
+#define LLJ_GG_BF16(VE) LLJ_GG_RUN(bf16_t, bf16_t, VE, 1, false, GgWeightDense<bf16_t, VE, 512>)
+#define LLJ_GG_BITS(B, VE)                                                                 \
+  do {                                                                                     \
+    if (dt == 0) LLJ_GG_RUN(bf16_t, float, VE, 2, false, GgWeightCodes<B, 256>);           \
+    else if (fine) LLJ_GG_RUN(float, float, VE, 1, true, GgWeightCodes<B, 512>);           \
+    else LLJ_GG_RUN(float, float, VE, 2, false, GgWeightCodes<B, 256>);                    \
+  } while (0)
+#define LLJ_GG_CODES(VE)                  \
+  do {                                    \
+    if (bits == 4) LLJ_GG_BITS(4, VE);    \
+    else if (bits == 8) LLJ_GG_BITS(8, VE); \
+    else LLJ_GG_BITS(2, VE);              \
+  } while (0)
+  if (wkind == 0) {
+    if (fits(x, ldx, 4)) LLJ_GG_CODES(4);
+    else LLJ_GG_CODES(1);
+  } else if (dt == 1) {
+    if (fits(x, ldx, 4) && fits(W, K, 4)) LLJ_GG_F32(4);
+    else LLJ_GG_F32(1);
+  } else {
+    if (fits(x, ldx, 8) && fits(W, K, 8)) LLJ_GG_BF16(8);
+    else if (fits(x, ldx, 4) && fits(W, K, 4)) LLJ_GG_BF16(4);
+    else LLJ_GG_BF16(1);
+  }
+#undef LLJ_GG_CODES
+#undef LLJ_GG_BITS
+#undef LLJ_GG_BF16
+#undef LLJ_GG_F32
+#undef LLJ_GG_RUN
+  if (part) {
+    LLJ_CHECK_LAUNCH();
+    const size_t blocks = ((size_t)M * N + 255) / 256;
+    const unsigned g = blocks < 4096 ? (unsigned)blocks : 4096u;
+    LLJ_DT(dt, hipLaunchKernelGGL(gg_reduce_kernel<bf16_t>, dim3(g), dim3(256), 0, s, part, splits, M, N, (bf16_t*)y, ldy,
+                                  (const bf16_t*)resid, ldr),
+           hipLaunchKernelGGL(gg_reduce_kernel<float>, dim3(g), dim3(256), 0, s, part, splits, M, N, (float*)y, ldy,
+                              (const float*)resid, ldr));
+  }
   LLJ_CHECK_LAUNCH();
   return 0;
+}
+
+int llj_g_linear(int wkind, const void* x, int ldx, int M, int K, const void* W, const float* scales, const float* zeros,
+                 int bits, int group, int N, void* y, int ldy, const void* resid, int ldr, int dt, void* stream) {
+  return llj_g_linear_ws(wkind, x, ldx, M, K, W, scales, zeros, bits, group, N, y, ldy, resid, ldr, dt, nullptr, 0, stream);
 }
 
 int llj_g_rope_kv(const void* qkv, void* q_out, void* kcache, void* vcache, const float* rope, const int* pos, int B, int T,

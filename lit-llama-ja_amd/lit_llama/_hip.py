@@ -77,6 +77,7 @@ SIGNATURES = {
     "llj_g_embedding": [_P, _P, _P, _I, _I, _P, _I, _P],
     "llj_g_rmsnorm": [_P, _I, _P, _F, _P, _I, _I, _I, _I, _P],
     "llj_g_linear": [_I, _P, _I, _I, _I, _P, _P, _P, _I, _I, _I, _P, _I, _P, _I, _I, _P],
+    "llj_g_linear_ws": [_I, _P, _I, _I, _I, _P, _P, _P, _I, _I, _I, _P, _I, _P, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_g_rope_kv": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "llj_g_attention": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "llj_g_silu_mul": [_P, _P, _P, ctypes.c_size_t, _I, _P],
@@ -131,6 +132,7 @@ SIZE_SIGNATURES = {
     "llj_i8_rowstats_bytes": [_I],
     "llj_gemm_resid_ws_bytes": [_I, _I, _I, _I],
     "llj_gemm_swiglu_ws_bytes": [_I, _I, _I, _I],
+    "llj_g_linear_ws_bytes": [_I, _I, _I, _I, _I],
     "llj_gemm_bf16_ws_bytes": [_I, _I, _I],
 }
 
@@ -189,6 +191,14 @@ def call(name: str, *args) -> None:
     if rc != 0:
         what = "unsupported shape/argument (EINVAL)" if rc == 1000 else f"hipError {rc}"
         raise HipError(f"{name} failed: {what}")
+
+
+def g_linear(wkind: int, x, M: int, K: int, W, scales, zeros, bits: int, group: int, N: int, y, resid, dt: int, st: int) -> None:
+    """llj_g_linear_ws with its scratch (stream-ordered: reused only by later work on the stream)."""
+    nb = lib().llj_g_linear_ws_bytes(wkind, M, N, K, dt)
+    ws = torch.empty(nb // 4, dtype=torch.float32, device=y.device) if nb else None
+    call("llj_g_linear_ws", wkind, x.data_ptr(), x.stride(0), M, K, W.data_ptr(), ptr(scales), ptr(zeros), bits, group, N,
+         y.data_ptr(), y.stride(0), ptr(resid), 0 if resid is None else resid.stride(0), dt, ptr(ws), nb, st)
 
 
 def stream() -> int:

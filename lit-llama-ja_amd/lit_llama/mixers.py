@@ -94,8 +94,7 @@ class PackedLinear:
         act, bias = (2 if self.unit else int(relu2)), _hip.ptr(self.bias)
         if self.dtype == torch.float32:
             y = torch.empty(M, self.Np, dtype=torch.float32, device=out.device) if self.unit else out
-            _hip.call("llj_g_linear", 1, a.data_ptr(), a.stride(0), M, self.Kp, self.w.data_ptr(), None, None, 16, self.Kp,
-                      self.Np, y.data_ptr(), y.stride(0), None, 0, 1, st)
+            _hip.g_linear(1, a, M, self.Kp, self.w, None, None, 16, self.Kp, self.Np, y, None, 1, st)
             if self.unit:
                 _hip.call("llj_g_bias_act", 2, y.data_ptr(), y.stride(0), bias, out.data_ptr(), out.stride(0), M, self.Np,
                           limit, alpha, 1, st)

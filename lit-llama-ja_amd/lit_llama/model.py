@@ -623,9 +623,7 @@ class LLaMA(nn.Module):
             return
         if kind == 1 and W.dtype != A.dtype:
             raise TypeError(f"dense Linear weight {W.dtype} with {A.dtype} activations")
-        _hip.call("llj_g_linear", kind, A.data_ptr(), A.stride(0), M, K, W.data_ptr(), _hip.ptr(sc), _hip.ptr(zr), bits,
-                  group, N, out.data_ptr(), out.stride(0), None if resid is None else resid.data_ptr(),
-                  0 if resid is None else resid.stride(0), _dt_code(A.dtype), st)
+        _hip.g_linear(kind, A, M, K, W, sc, zr, bits, group, N, out, resid, _dt_code(A.dtype), st)
 
     def _blocks_generic(self, w, specs, kv, pos, B, T, S, st):
         """The blocks on the any-shape kernels (csrc/generic.hip), per layer (model.py:162-175):

@@ -238,8 +238,8 @@ class ColBlockQuantizedLinear(torch.nn.Module):
             x2 = inp.reshape(-1, K).contiguous()
             out = torch.empty((x2.shape[0], N), dtype=inp.dtype, device=inp.device)
             kind, qw, sc, zr, bits, group = self._gspec()
-            _hip.call("llj_g_linear", kind, x2.data_ptr(), K, x2.shape[0], K, qw.data_ptr(), sc.data_ptr(), zr.data_ptr(),
-                      bits, group, N, out.data_ptr(), N, None, 0, 0 if inp.dtype == torch.bfloat16 else 1, _hip.stream())
+            _hip.g_linear(kind, x2, x2.shape[0], K, qw, sc, zr, bits, group, N, out, None,
+                          0 if inp.dtype == torch.bfloat16 else 1, _hip.stream())
             return out.reshape(*inp.shape[:-1], N)
         self._prepare()
         x2 = _as_rows(inp, K)

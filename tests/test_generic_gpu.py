@@ -172,3 +172,54 @@ def test_generic_int8_linear_vs_oracle(M, K, N, outliers):
     err = np.abs(got - ref32)
     assert (err <= 2e-3 * np.abs(ref32) + 1e-3 * np.abs(ref32).max()).all(), err.max()
     np.testing.assert_allclose(yr32.cpu().numpy(), res + got, rtol=0, atol=1e-6)
+
+
+# ---- matrix products of more than 8 rows (generic_gemm.h)
+def _g_linear_operands(kind, bits, group, dt, M, K, N, ldx, seed):
+    rng = np.random.default_rng(seed)
+    dtype = torch.float32 if dt else torch.bfloat16
+    buf = torch.from_numpy(rng.standard_normal(M * ldx + 1).astype(np.float32)).cuda().to(dtype)
+    G = -(-K // group)
+    if kind == 1:
+        w = torch.from_numpy(rng.standard_normal((N, K)).astype(np.float32)).cuda().to(dtype)
+        return buf, w, None, None, w.double()
+    q = torch.from_numpy(rng.integers(0, 1 << bits, (N, K)).astype(np.uint8)).cuda()
+    sc = torch.from_numpy((rng.random((N, G)) * 0.01 + 0.001).astype(np.float32)).cuda()
+    zr = torch.from_numpy(rng.integers(0, 1 << bits, (N, G)).astype(np.float32)).cuda()
+    epb = 8 // bits
+    packed = sum(q[:, r::epb].int() << (r * bits) for r in range(epb)).to(torch.uint8).t().contiguous()
+    cols = torch.arange(K, device="cuda") // group
+    return buf, packed, sc, zr, (q.double() - zr[:, cols].double()) * sc[:, cols].double()
+
+
+@pytest.mark.parametrize("kind,bits,group", [(1, 16, 0), (0, 2, 0), (0, 4, 0), (0, 8, 0), (0, 4, 100)])
+@pytest.mark.parametrize("dt", [0, 1])
+@pytest.mark.parametrize("M,N,K,pad,off", [(9, 1, 4, 0, 0), (9, 127, 32, 0, 0), (64, 128, 36, 4, 0), (65, 129, 780, 0, 0),
+                                           (129, 255, 1028, 1, 1), (33, 780, 2304, 8, 0), (70, 36, 4100, 0, 1)])
+def test_generic_gemm_edges_vs_float64(kind, bits, group, dt, M, N, K, pad, off):
+    """Partial tiles, the K tail, loads of 16 / 8 / 4 / 2 bytes (strides and pointers off the alignment), the K split, groups,
+    and the residual in place. Bound: fp32 sums over chains of at most 32, 8, K / 128 and 16 (splits) terms lose half an
+    ulp of sum |x w| per term; a weight element from codes two more; bf16 results (8 significant bits) round by 2^-8, once more with the
+    residual."""
+    from lit_llama import _hip
+
+    group = group or K
+    ldx = K + pad
+    buf, w, sc, zr, w64 = _g_linear_operands(kind, bits, group, dt, M, K, N, ldx, M * N + K)
+    x = buf[off:off + M * ldx].view(M, ldx)
+    x64 = x[:, :K].double()
+    res = torch.randn(M, N, device="cuda", generator=torch.Generator("cuda").manual_seed(K)).to(x.dtype)
+    want, mass = x64 @ w64.T, x64.abs() @ w64.abs().T
+    bound = mass * 2.0 ** -24 * (32 + 8 + K // 128 + 16 + 4)
+    half = 0.0 if dt else 2.0 ** -8 * 1.01
+    for resid in (None, res):
+        ref = want if resid is None else want + resid.double()
+        lim = bound + half * want.abs() + (0.0 if resid is None else (half + 2.0 ** -24) * (ref.abs() + half * want.abs()))
+        y = torch.empty(M, N, dtype=x.dtype, device="cuda") if resid is None else resid.clone()
+        _hip.g_linear(kind, x, M, K, w, sc, zr, bits, group, N, y, None if resid is None else y, dt, _hip.stream())
+        one = torch.empty_like(y) if resid is None else resid.clone()
+        _hip.call("llj_g_linear", kind, x.data_ptr(), ldx, M, K, w.data_ptr(), _hip.ptr(sc), _hip.ptr(zr), bits, group, N,
+                  one.data_ptr(), N, None if resid is None else one.data_ptr(), 0 if resid is None else N, dt, _hip.stream())
+        for got in (y, one):
+            bad = (got.double() - ref).abs() > lim + 1e-30
+            assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside the bound"
