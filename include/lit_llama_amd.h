@@ -339,6 +339,18 @@ size_t llj_g_linear_ws_bytes(int wkind, int M, int N, int K, int dt);
 int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void* W, const float* scales, const float* zeros,
                     int bits, int group, int N, void* y, int ldy, const void* resid, int ldr, int dt, void* ws, size_t ws_bytes,
                     void* stream);
+/* llj_g_rmsnorm and a dense product of its rows in one launch: y = norm(x) . W^T, and h = silu(norm(x) . W1^T) * (norm(x) . W2^T)
+ * (model.py:256-260), each step rounded as the separate calls round. For the rows that llj_g_norm_ok takes (returns 1). */
+int llj_g_norm_ok(int M, int K, int dt);
+int llj_g_norm_linear(const void* x, int ldx, const void* nw, float eps, int M, int K, const void* W, int N, void* y, int ldy,
+                      int dt, void* stream);
+int llj_g_norm_swiglu(const void* x, int ldx, const void* nw, float eps, int M, int K, const void* W1, const void* W2, int N,
+                      void* y, int ldy, int dt, void* stream);
+/* llj_g_rope_kv and llj_g_attention of one token per sequence (all at position pos[0]) in one launch: qkv (B, 3C) -> y (B, C); for the
+ * cache and head sizes that llj_g_rope_attention_ok takes (returns 1). */
+int llj_g_rope_attention_ok(int S, int hs);
+int llj_g_rope_attention(const void* qkv, void* kcache, void* vcache, const float* rope, const int* pos, void* y, int B, int C,
+                         int n_head, int S, int dt, void* stream);
 /* c_attn output qkv (B*T, 3C) -> q_out (B*T, C) with RoPE, k (RoPE) / v into cache slot pos[t] % S
  * (model.py:204-228, 312-329); rope (block_size, hs/2, 2) fp32; head size even. */
 int llj_g_rope_kv(const void* qkv, void* q_out, void* kcache, void* vcache, const float* rope, const int* pos, int B, int T,

@@ -2,13 +2,14 @@
 // or a head size other than 64 / 128. The JA fork's own 125M config (n_embd 780, head 78; reference
 // lit_llama/model.py:48-51) and the reference test's n_embd 32 / head 2 (tests/test_model.py:108-112)
 // run here: tiled matrix products from 9 rows on (generic_gemm.h), below that one output column per
-// wave, fp32 accumulation, the reference's bf16 rounding points (the same ones the fast kernels keep).
+// wave (generic_rows.h), fp32 accumulation, the reference's bf16 rounding points (the same ones the fast kernels keep).
 // Every kernel also runs in fp32 (dt = 1: activations, dense weights, KV cache and logits fp32, no
 // bf16 rounding -- the reference's float32 model, e.g. evaluate/full.py's default dtype and the
 // CPU config of generate.py:121): LLaMA.forward routes an fp32 model here whatever its shape.
 #include "common.h"
 #include "elem.h"
 #include "generic_gemm.h"
+#include "generic_rows.h"
 #include "lit_llama_amd.h"
 
 namespace llj {
@@ -45,23 +46,19 @@ __global__ __launch_bounds__(256) void g_rmsnorm_kernel(const T* __restrict__ x,
 }
 
 // ---- y[m, n] = bf16(sum_k x[m, k] W[n, k]) or, with resid, bf16(resid[m, n] + that) (the residual
-// adds of model.py:172-173). WK 1: dense bf16 W (N, K) row-major (F.linear). WK 0: the reference's
-// ColBlockQuantizedLinear buffers untouched -- codes in quant_weight's column-major storage (byte
-// (n, j) at j N + n, 8 / bits codes per byte, code of k = j epb + r at bits r * bits), per-group
-// fp32 scales / zeros (N, G), group = tile_cols (K for -1); the weight element is the Triton path's
+// adds of model.py:172-173) of up to 8 rows on the reference's ColBlockQuantizedLinear buffers untouched -- codes in
+// quant_weight's column-major storage (byte (n, j) at j N + n, 8 / bits codes per byte, code of k = j epb + r at bits
+// r * bits), per-group fp32 scales / zeros (N, G), group = tile_cols (K for -1); the weight element is the Triton path's
 // (q - zero) * scale in fp32 (quantization.py:250-267, 390-409). One wave per output column, lanes
-// over k, up to 8 rows per wave. T: activation (and dense weight) type.
-constexpr int GL_ROWS = 8;
-template <int WK, typename T>
-__global__ __launch_bounds__(256) void g_linear_kernel(const T* __restrict__ x, int ldx, int M, int K,
-                                                       const void* __restrict__ W, const float* __restrict__ sc,
-                                                       const float* __restrict__ zr, int bits, int group, int N,
-                                                       T* __restrict__ y, int ldy, const T* resid, int ldr) {
+// over k. T: activation type.
+template <typename T>
+__global__ __launch_bounds__(256) void g_code_rows_kernel(const T* __restrict__ x, int ldx, int M, int K,
+                                                          const unsigned char* __restrict__ W, const float* __restrict__ sc,
+                                                          const float* __restrict__ zr, int bits, int group, int N,
+                                                          T* __restrict__ y, int ldy, const T* resid, int ldr) {
   const int lane = threadIdx.x & 63;
   const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (n >= N) return;
-  const int m0 = blockIdx.y * GL_ROWS;
-  const int mr = M - m0 < GL_ROWS ? M - m0 : GL_ROWS;
   const int G = (K + group - 1) / group;
   const int epb = 8 / bits;
   const uint32_t mask = (1u << bits) - 1u;
@@ -69,27 +66,21 @@ __global__ __launch_bounds__(256) void g_linear_kernel(const T* __restrict__ x, 
 #pragma unroll
   for (int r = 0; r < GL_ROWS; ++r) acc[r] = 0.f;
   for (int k = lane; k < K; k += 64) {
-    float wv;
-    if (WK == 1) {
-      wv = ldv(reinterpret_cast<const T*>(W), (size_t)n * K + k);
-    } else {
-      const int j = k / epb, sh = (k - j * epb) * bits;
-      const uint32_t q = ((uint32_t)reinterpret_cast<const unsigned char*>(W)[(size_t)j * N + n] >> sh) & mask;
-      const int g = k / group;
-      wv = ((float)q - zr[(size_t)n * G + g]) * sc[(size_t)n * G + g];
-    }
+    const int j = k / epb, sh = (k - j * epb) * bits;
+    const uint32_t q = ((uint32_t)W[(size_t)j * N + n] >> sh) & mask;
+    const int g = k / group;
+    const float wv = ((float)q - zr[(size_t)n * G + g]) * sc[(size_t)n * G + g];
 #pragma unroll
     for (int r = 0; r < GL_ROWS; ++r)
-      if (r < mr) acc[r] += ldv(x, (size_t)(m0 + r) * ldx + k) * wv;
+      if (r < M) acc[r] += ldv(x, (size_t)r * ldx + k) * wv;
   }
 #pragma unroll
   for (int r = 0; r < GL_ROWS; ++r) {
     const float s = wave_sum(acc[r]);
-    if (lane == r && r < mr) {
-      const size_t m = (size_t)(m0 + r);
+    if (lane == r && r < M) {
       float v = rnd<T>(s);
-      if (resid) v = ldv(resid, m * ldr + n) + v;
-      stv(y, m * ldy + n, v);
+      if (resid) v = ldv(resid, (size_t)r * ldr + n) + v;
+      stv(y, (size_t)r * ldy + n, v);
     }
   }
 }
@@ -293,8 +284,84 @@ __global__ __launch_bounds__(256) void g_i8_linear_kernel(const T* __restrict__ 
   }
 }
 
+// Elements per load: 16 bytes, 8 or single elements, as x, its rows and the weights' rows are aligned. Columns per wave: four from
+// 8192 on (every CU then still has 8 waves), one below.
+template <typename T>
+static int gr_launch(int mode, const void* x, int ldx, const void* nw, float eps, int M, int K, const void* W, const void* W2,
+                     int N, void* y, int ldy, const void* resid, int ldr, hipStream_t s) {
+  const int el = (int)sizeof(T), nc = N >= 8192 && mode != GR_SWIGLU ? 4 : 1;
+  auto fits = [&](int n) {
+    return K % n == 0 && (uintptr_t)W % (n * el) == 0 && (uintptr_t)W2 % (n * el) == 0 &&
+           (mode != GR_PLAIN || ((uintptr_t)x % (n * el) == 0 && (ldx % n == 0 || M == 1)));
+  };
+  const size_t lds = mode == GR_PLAIN ? 0 : (size_t)M * K * el;
+  const dim3 grid((N + 4 * nc - 1) / (4 * nc));
+#define LLJ_GR(VE, MB, NC, MODE)                                                                                               \
+  hipLaunchKernelGGL((g_rows_kernel<T, VE, MB, NC, MODE>), grid, dim3(256), lds, s, (const T*)x, ldx, (const T*)nw, eps, M, K, \
+                     (const T*)W, (const T*)W2, N, (T*)y, ldy, (const T*)resid, ldr)
+#define LLJ_GR_MODE(VE, MB)                                  \
+  do {                                                       \
+    if (mode == GR_SWIGLU) LLJ_GR(VE, MB, 1, GR_SWIGLU);     \
+    else if (mode == GR_NORM && nc == 4) LLJ_GR(VE, MB, 4, GR_NORM); \
+    else if (mode == GR_NORM) LLJ_GR(VE, MB, 1, GR_NORM);    \
+    else if (nc == 4) LLJ_GR(VE, MB, 4, GR_PLAIN);           \
+    else LLJ_GR(VE, MB, 1, GR_PLAIN);                        \
+  } while (0)
+#define LLJ_GR_ROWS(VE)            \
+  do {                             \
+    if (M == 1) LLJ_GR_MODE(VE, 1); \
+    else LLJ_GR_MODE(VE, GL_ROWS); \
+  } while (0)
+  if (sizeof(T) == 2 && fits(8)) LLJ_GR_ROWS(sizeof(T) == 2 ? 8 : 4);
+  else if (fits(4)) LLJ_GR_ROWS(4);
+  else LLJ_GR_ROWS(1);
+#undef LLJ_GR_ROWS
+#undef LLJ_GR_MODE
+#undef LLJ_GR
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
 extern "C" {
 LLJ_TRACE_EXPORT(generic)
+
+int llj_g_norm_ok(int M, int K, int dt) {
+  return M > 0 && M <= GL_ROWS && K > 0 && (dt == 0 || dt == 1) && (size_t)M * K * (dt ? 4 : 2) <= (size_t)kGrNormLds;
+}
+
+int llj_g_norm_linear(const void* x, int ldx, const void* nw, float eps, int M, int K, const void* W, int N, void* y, int ldy,
+                      int dt, void* stream) {
+  LLJ_REQUIRE(x && nw && W && y && llj_g_norm_ok(M, K, dt) && N > 0 && ldx >= K && ldy >= N);
+  hipStream_t s = (hipStream_t)stream;
+  return dt == 0 ? gr_launch<bf16_t>(GR_NORM, x, ldx, nw, eps, M, K, W, nullptr, N, y, ldy, nullptr, 0, s)
+                 : gr_launch<float>(GR_NORM, x, ldx, nw, eps, M, K, W, nullptr, N, y, ldy, nullptr, 0, s);
+}
+
+int llj_g_norm_swiglu(const void* x, int ldx, const void* nw, float eps, int M, int K, const void* W1, const void* W2, int N,
+                      void* y, int ldy, int dt, void* stream) {
+  LLJ_REQUIRE(x && nw && W1 && W2 && y && llj_g_norm_ok(M, K, dt) && N > 0 && ldx >= K && ldy >= N);
+  hipStream_t s = (hipStream_t)stream;
+  return dt == 0 ? gr_launch<bf16_t>(GR_SWIGLU, x, ldx, nw, eps, M, K, W1, W2, N, y, ldy, nullptr, 0, s)
+                 : gr_launch<float>(GR_SWIGLU, x, ldx, nw, eps, M, K, W1, W2, N, y, ldy, nullptr, 0, s);
+}
+
+static size_t gr_attention_lds(int S, int hs) { return ((size_t)S + (size_t)hs * (3 + gr_groups(hs / 2))) * 4; }
+
+int llj_g_rope_attention_ok(int S, int hs) { return S > 0 && hs > 0 && hs % 2 == 0 && gr_attention_lds(S, hs) <= 64 * 1024; }
+
+int llj_g_rope_attention(const void* qkv, void* kcache, void* vcache, const float* rope, const int* pos, void* y, int B, int C,
+                         int n_head, int S, int dt, void* stream) {
+  LLJ_REQUIRE(qkv && kcache && vcache && rope && pos && y && B > 0 && n_head > 0 && C % n_head == 0 && (dt == 0 || dt == 1) &&
+              llj_g_rope_attention_ok(S, C / n_head) && ((uintptr_t)kcache | (uintptr_t)vcache) % (dt ? 8 : 4) == 0);
+  const size_t lds = gr_attention_lds(S, C / n_head);
+  hipStream_t s = (hipStream_t)stream;
+  LLJ_DT(dt, hipLaunchKernelGGL(g_rope_attention_kernel<bf16_t>, dim3(B, n_head), dim3(kGrThreads), lds, s, (const bf16_t*)qkv,
+                                (bf16_t*)kcache, (bf16_t*)vcache, rope, pos, (bf16_t*)y, C, n_head, S),
+         hipLaunchKernelGGL(g_rope_attention_kernel<float>, dim3(B, n_head), dim3(kGrThreads), lds, s, (const float*)qkv, (float*)kcache,
+                            (float*)vcache, rope, pos, (float*)y, C, n_head, S));
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
 
 int llj_g_embedding(const int* idx, const void* wte, void* out, int M, int C, int* pos_inc, int dt, void* stream) {
   LLJ_REQUIRE(idx && wte && out && M > 0 && C > 0 && (dt == 0 || dt == 1));
@@ -327,13 +394,14 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
   LLJ_REQUIRE(wkind == 1 || (wkind == 0 && scales && zeros && (bits == 2 || bits == 4 || bits == 8) && group > 0 &&
                              K % (8 / bits) == 0));
   hipStream_t s = (hipStream_t)stream;
+  if (M <= GL_ROWS && wkind == 1)
+    return dt == 0 ? gr_launch<bf16_t>(GR_PLAIN, x, ldx, nullptr, 0.f, M, K, W, nullptr, N, y, ldy, resid, ldr, s)
+                   : gr_launch<float>(GR_PLAIN, x, ldx, nullptr, 0.f, M, K, W, nullptr, N, y, ldy, resid, ldr, s);
   if (M <= GL_ROWS) {
-    const dim3 grid((N + 3) / 4, 1);
-#define LLJ_GL(WK, T) \
-  hipLaunchKernelGGL((g_linear_kernel<WK, T>), grid, dim3(256), 0, s, (const T*)x, ldx, M, K, W, scales, zeros, \
-                     WK == 1 ? 16 : bits, WK == 1 ? K : group, N, (T*)y, ldy, (const T*)resid, ldr)
-    if (wkind == 1) LLJ_DT(dt, LLJ_GL(1, bf16_t), LLJ_GL(1, float));
-    else LLJ_DT(dt, LLJ_GL(0, bf16_t), LLJ_GL(0, float));
+#define LLJ_GL(T) \
+  hipLaunchKernelGGL(g_code_rows_kernel<T>, dim3((N + 3) / 4), dim3(256), 0, s, (const T*)x, ldx, M, K, (const unsigned char*)W, \
+                     scales, zeros, bits, group, N, (T*)y, ldy, (const T*)resid, ldr)
+    LLJ_DT(dt, LLJ_GL(bf16_t), LLJ_GL(float));
 #undef LLJ_GL
     LLJ_CHECK_LAUNCH();
     return 0;

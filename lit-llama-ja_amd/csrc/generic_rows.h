@@ -1,0 +1,259 @@
+// Up to 8 rows of the any-shape path on dense weights (generic.hip's llj_g_linear, llj_g_norm_linear, llj_g_norm_swiglu), and the
+// attention of decode rows with their rotary positions and cache writes (llj_g_rope_attention).
+//
+// Decode of these models (780 wide, 3.6 MB per matrix) is bound by latency: what counts is how many dependent memory trips and
+// launches a layer has. A wave takes one output column (four where there are columns enough for every CU), its lanes
+// consecutive pieces of K, and issues the weights' loads of up to 8 pieces at once before it needs the first, in the
+// norm-fused forms before the norm. The residual's RMSNorm is computed by every workgroup for itself (a read of a few KB) in the
+// order of g_rmsnorm_kernel, so a layer is 5 launches instead of 10. 125M bf16, one row, per launch: rms_1 and c_attn 4.4 + 10.1 ->
+// 4.9 us, c_proj and mlp.c_proj 15.8 -> 3.7 on average, rms_2, c_fc1, c_fc2 and silu * mul 29 -> 6.0, rotary positions and
+// attention over 130 keys 18.3 -> 8.2 (256 threads 9.8, and without the early loads 11.2); lm_head 51.7 -> 14.8 (3.7 TB/s).
+#pragma once
+#include "common.h"
+#include "elem.h"
+
+namespace llj {
+
+constexpr int GL_ROWS = 8;
+constexpr int kGrNormLds = 48 * 1024;  // the rows' normalized copy of the norm-fused forms
+
+enum { GR_PLAIN = 0, GR_NORM = 1, GR_SWIGLU = 2 };
+
+// y[m, n] = x[m] . W[n] (+ resid), x through an RMSNorm in the fused forms; GR_SWIGLU: silu(x . W[n]) * (x . W2[n]). VE elements
+// per load: a divisor of K (and of ldx), with x and W aligned to it. MB: 1 or 8 rows' accumulators; NC: columns per wave.
+template <typename T, int VE, int MB, int NC, int MODE>
+__global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, int ldx, const T* __restrict__ nw, float eps, int M,
+                                                     int K, const T* __restrict__ W, const T* __restrict__ W2, int N,
+                                                     T* __restrict__ y, int ldy, const T* resid, int ldr) {
+  extern __shared__ __align__(16) char gr_lds[];
+  typedef T vec __attribute__((ext_vector_type(VE)));
+  constexpr int U = NC == 1 ? 8 : 4, NT = MODE == GR_SWIGLU ? 2 : NC;
+  const int tid = threadIdx.x, lane = tid & 63, n0 = (blockIdx.x * 4 + (tid >> 6)) * NC;
+  const T* wr[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int n = MODE == GR_SWIGLU ? n0 : n0 + t;
+    wr[t] = (MODE == GR_SWIGLU && t ? W2 : W) + (size_t)(n < N ? n : N - 1) * K;
+  }
+  vec wv[NT][U];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + (u * 64 + lane) * VE;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wv[t][u] = k < K ? *reinterpret_cast<const vec*>(wr[t] + k) : vec(0);
+    }
+  };
+  fetch(0);
+  T* xs = reinterpret_cast<T*>(gr_lds);
+  if constexpr (MODE != GR_PLAIN) {
+    __shared__ float red[MB][4];
+#pragma unroll
+    for (int r = 0; r < MB; ++r) {
+      if (r < M) {
+        float ss = 0.f;
+        for (int k = tid; k < K; k += 256) {
+          const float v = ldv(x, (size_t)r * ldx + k);
+          ss += rnd<T>(v * v);
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) red[r][tid >> 6] = ss;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < MB; ++r) {
+      if (r < M) {
+        const float tot = red[r][0] + red[r][1] + red[r][2] + red[r][3];
+        const float s = rnd<T>(rsqrtf(rnd<T>(rnd<T>(tot / (float)K) + eps)));
+        for (int k = tid; k < K; k += 256) stv(xs, r * K + k, ldv(nw, k) * rnd<T>(ldv(x, (size_t)r * ldx + k) * s));
+      }
+    }
+    __syncthreads();
+  }
+  float acc[MB][NT];
+#pragma unroll
+  for (int r = 0; r < MB; ++r)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[r][t] = 0.f;
+  for (int k0 = 0; k0 < K; k0 += U * 64 * VE) {
+    if (k0) fetch(k0);
+#pragma unroll
+    for (int r = 0; r < MB; ++r) {
+      if (r < M) {
+        vec xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = k0 + (u * 64 + lane) * VE;
+          const T* xr = MODE == GR_PLAIN ? x + (size_t)r * ldx : xs + r * K;
+          xv[u] = k < K ? *reinterpret_cast<const vec*>(xr + k) : vec(0);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int e = 0; e < VE; ++e) {
+            T xe = xv[u][e];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              T we = wv[t][u][e];
+              acc[r][t] += ldv(&xe, 0) * ldv(&we, 0);
+            }
+          }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < MB; ++r) {
+    if (r < M) {
+      float s[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) s[t] = rnd<T>(wave_sum(acc[r][t]));
+      if constexpr (MODE == GR_SWIGLU) {
+        if (lane == 0 && n0 < N) stv(y, (size_t)r * ldy + n0, rnd<T>(s[0] / (1.f + expf(-s[0]))) * s[1]);
+      } else {
+#pragma unroll
+        for (int t = 0; t < NC; ++t) {
+          if (lane == t && n0 + t < N) {
+            float v = s[t];
+            if (resid) v = ldv(resid, (size_t)r * ldr + n0 + t) + v;
+            stv(y, (size_t)r * ldy + n0 + t, v);
+          }
+        }
+      }
+    }
+  }
+}
+
+// One token per sequence: rotary positions of q and k (g_rope_kv_kernel), k and v into cache slot p % S, and causal attention over
+// the cache (g_attention_kernel). Block (row, head) of 512 threads -- a few tens of blocks with a chain of memory trips each: 16
+// lanes per key and 128 keys at a time, then the values with the threads split over dimension pairs and up to kGrKeyGroups
+// interleaved groups of keys. The first keys and values are loaded before the rotation. LDS: S + hs (3 + groups) floats.
+constexpr int kGrThreads = 512, kGrKeyGroups = 14;
+__host__ __device__ inline int gr_groups(int P) { return P > kGrThreads ? 1 : P * kGrKeyGroups > kGrThreads ? kGrThreads / P : kGrKeyGroups; }
+template <typename T>
+__global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* __restrict__ qkv, T* __restrict__ kc, T* __restrict__ vc,
+                                                               const float* __restrict__ rope, const int* __restrict__ pos,
+                                                               T* __restrict__ y, int C, int nh, int S) {
+  extern __shared__ __align__(16) char gr_lds[];
+  __shared__ float red[kGrThreads / 64];
+  typedef T pair __attribute__((ext_vector_type(2)));
+  const int m = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int hs = C / nh, P = hs / 2, p = pos[0], slot = p % S, nvis = p < S ? p + 1 : S;
+  float* sc = reinterpret_cast<float*>(gr_lds);  // [S] scores, then weights
+  float* sq = sc + S;                            // [hs] the scaled query
+  float* sk = sq + hs;                           // [hs] the new key
+  float* sv = sk + hs;                           // [hs] and value
+  float* so = sv + hs;                           // [groups][hs] partial outputs
+  const float scale = 1.f / sqrtf((float)hs);
+  const T* row = qkv + (size_t)m * 3 * C + h * hs;
+  const size_t cb = ((size_t)m * nh + h) * S * hs, cbase = cb + (size_t)slot * hs;
+  // keys j0 + 16 u of this group of 16 lanes, 64 pairs from i0 on: up to 16 loads in flight
+  const int sub = tid & 15, kg = tid >> 4;
+  pair kw[4][4];
+  auto keys = [&](int j0, int i0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = j0 + 32 * u, i = i0 + 16 * q + sub;
+        kw[u][q] = j < nvis && i < P ? reinterpret_cast<const pair*>(kc + cb + (size_t)j * hs)[i] : pair(0);
+      }
+  };
+  const int G = gr_groups(P), g = P > kGrThreads ? 0 : tid / P;
+  const int pi = P > kGrThreads ? tid : tid % P;  // this thread's (first) pair of the values, keys g + G u
+  const pair* vr = reinterpret_cast<const pair*>(vc + cb) + pi;
+  constexpr int VU = 12;
+  pair vw[VU];
+  keys(kg, 0);
+#pragma unroll
+  for (int u = 0; u < VU; ++u) vw[u] = g < G && g + G * u < nvis ? vr[(size_t)(g + G * u) * P] : pair(0);
+  // in flight while q and k are rotated; the rows that this workgroup writes come from LDS
+  for (int i = tid; i < P; i += kGrThreads) {
+    const float c = rope[((size_t)p * P + i) * 2], s = rope[((size_t)p * P + i) * 2 + 1];
+    const float q0 = ldv(row, 2 * i), q1 = ldv(row, 2 * i + 1), k0 = ldv(row, C + 2 * i), k1 = ldv(row, C + 2 * i + 1);
+    sq[2 * i] = rnd<T>(q0 * c - q1 * s) * scale;
+    sq[2 * i + 1] = rnd<T>(q1 * c + q0 * s) * scale;
+    const float r0 = rnd<T>(k0 * c - k1 * s), r1 = rnd<T>(k1 * c + k0 * s);
+    sk[2 * i] = r0;
+    sk[2 * i + 1] = r1;
+    sv[2 * i] = ldv(row, 2 * C + 2 * i);
+    sv[2 * i + 1] = ldv(row, 2 * C + 2 * i + 1);
+    stv(kc, cbase + 2 * i, r0);
+    stv(kc, cbase + 2 * i + 1, r1);
+    vc[cbase + 2 * i] = row[2 * C + 2 * i];
+    vc[cbase + 2 * i + 1] = row[2 * C + 2 * i + 1];
+  }
+  __syncthreads();
+  float mx = -INFINITY;
+  for (int j0 = kg; j0 < nvis; j0 += 128) {
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < P; i0 += 64) {
+      if (j0 != kg || i0) keys(j0, i0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int i = i0 + 16 * q + sub;
+        if (i >= P) continue;
+        const float q0 = sq[2 * i], q1 = sq[2 * i + 1];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          T k0 = kw[u][q][0], k1 = kw[u][q][1];
+          const bool own = j0 + 32 * u == slot;
+          s[u] += q0 * (own ? sk[2 * i] : ldv(&k0, 0)) + q1 * (own ? sk[2 * i + 1] : ldv(&k1, 0));
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      s[u] = row16_sum(s[u]);
+      if (j0 + 32 * u < nvis) {
+        if (sub == 0) sc[j0 + 32 * u] = s[u];
+        mx = fmaxf(mx, s[u]);
+      }
+    }
+  }
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kGrThreads / 64; ++w) mx = fmaxf(mx, red[w]);
+  __syncthreads();
+  float l = 0.f;
+  for (int j = tid; j < nvis; j += kGrThreads) {
+    const float e = __expf(sc[j] - mx);
+    sc[j] = e;
+    l += e;
+  }
+  l = wave_sum(l);
+  if ((tid & 63) == 0) red[tid >> 6] = l;
+  __syncthreads();
+  l = 0.f;
+#pragma unroll
+  for (int w = 0; w < kGrThreads / 64; ++w) l += red[w];
+  const float inv = 1.f / l;
+  for (int i = pi; i < P && g < G; i += P > kGrThreads ? kGrThreads : P) {
+    float o0 = 0.f, o1 = 0.f;
+    auto add = [&](int j, pair v) {
+      T v0 = v[0], v1 = v[1];
+      o0 += sc[j] * (j == slot ? sv[2 * i] : ldv(&v0, 0));
+      o1 += sc[j] * (j == slot ? sv[2 * i + 1] : ldv(&v1, 0));
+    };
+    int j = g;
+    if (i == pi) {
+#pragma unroll
+      for (int u = 0; u < VU; ++u, j += G)
+        if (j < nvis) add(j, vw[u]);
+    }
+#pragma unroll 8
+    for (; j < nvis; j += G) add(j, vr[(i - pi) + (size_t)j * P]);
+    so[g * hs + 2 * i] = o0;
+    so[g * hs + 2 * i + 1] = o1;
+  }
+  __syncthreads();
+  for (int d = tid; d < hs; d += kGrThreads) {
+    float o = 0.f;
+    for (int k = 0; k < G; ++k) o += so[k * hs + d];
+    stv(y, (size_t)m * C + h * hs + d, o * inv);
+  }
+}
+
+}  // namespace llj

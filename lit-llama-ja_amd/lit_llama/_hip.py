@@ -78,6 +78,11 @@ SIGNATURES = {
     "llj_g_rmsnorm": [_P, _I, _P, _F, _P, _I, _I, _I, _I, _P],
     "llj_g_linear": [_I, _P, _I, _I, _I, _P, _P, _P, _I, _I, _I, _P, _I, _P, _I, _I, _P],
     "llj_g_linear_ws": [_I, _P, _I, _I, _I, _P, _P, _P, _I, _I, _I, _P, _I, _P, _I, _I, _P, ctypes.c_size_t, _P],
+    "llj_g_norm_ok": [_I, _I, _I],
+    "llj_g_norm_linear": [_P, _I, _P, _F, _I, _I, _P, _I, _P, _I, _I, _P],
+    "llj_g_norm_swiglu": [_P, _I, _P, _F, _I, _I, _P, _P, _I, _P, _I, _I, _P],
+    "llj_g_rope_attention_ok": [_I, _I],
+    "llj_g_rope_attention": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "llj_g_rope_kv": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "llj_g_attention": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "llj_g_silu_mul": [_P, _P, _P, ctypes.c_size_t, _I, _P],

@@ -628,27 +628,52 @@ class LLaMA(nn.Module):
     def _blocks_generic(self, w, specs, kv, pos, B, T, S, st):
         """The blocks on the any-shape kernels (csrc/generic.hip), per layer (model.py:162-175):
         rms_1 -> c_attn -> split + RoPE + KV write -> attention -> c_proj + residual -> rms_2 ->
-        c_fc1, c_fc2 -> silu * mul -> mlp.c_proj + residual."""
+        c_fc1, c_fc2 -> silu * mul -> mlp.c_proj + residual. Up to 8 rows on dense weights take each norm with
+        the products after it, decode rows the RoPE + KV write with the attention."""
         cfg = self.config
         C, H, nh = cfg.n_embd, MLP.hidden(cfg), cfg.n_head
-        M = B * T
+        M, L = B * T, _hip.lib()
+        norm = bool(L.llj_g_norm_ok(M, C, w.dt))
+        step = T == 1 and bool(L.llj_g_rope_attention_ok(S, C // nh))
         for i, blk in enumerate(self.transformer.h):
             sa, sp, s1, s2, sd = specs["layers"][i]
             kc, vc = kv[i]
-            _hip.call("llj_g_rmsnorm", w.x.data_ptr(), C, blk.rms_1.scale.data_ptr(), blk.rms_1.eps, w.xn.data_ptr(), C,
-                      M, C, w.dt, st)
-            self._glinear(sa, w.xn, M, C, 3 * C, w.qkv, None, st)
-            _hip.call("llj_g_rope_kv", w.qkv.data_ptr(), w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
-                      self.rope_cache.data_ptr(), pos.data_ptr(), B, T, C, nh, S, w.dt, st)
-            _hip.call("llj_g_attention", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(),
-                      B, T, C, nh, S, w.dt, st)
+            LLaMA._gnorm_linear(norm, w.x, blk.rms_1, sa, M, C, 3 * C, w.qkv, w, st)
+            if step:
+                _hip.call("llj_g_rope_attention", w.qkv.data_ptr(), kc.data_ptr(), vc.data_ptr(), self.rope_cache.data_ptr(),
+                          pos.data_ptr(), w.y.data_ptr(), B, C, nh, S, w.dt, st)
+            else:
+                _hip.call("llj_g_rope_kv", w.qkv.data_ptr(), w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                          self.rope_cache.data_ptr(), pos.data_ptr(), B, T, C, nh, S, w.dt, st)
+                _hip.call("llj_g_attention", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(),
+                          B, T, C, nh, S, w.dt, st)
             self._glinear(sp, w.y, M, C, C, w.x, w.x, st)
-            _hip.call("llj_g_rmsnorm", w.x.data_ptr(), C, blk.rms_2.scale.data_ptr(), blk.rms_2.eps, w.xn.data_ptr(), C,
-                      M, C, w.dt, st)
-            self._glinear(s1, w.xn, M, C, H, w.a1, None, st)
-            self._glinear(s2, w.xn, M, C, H, w.a2, None, st)
-            _hip.call("llj_g_silu_mul", w.a1.data_ptr(), w.a2.data_ptr(), w.h.data_ptr(), M * H, w.dt, st)
+            if norm and LLaMA._gdense(s1, w.x) and LLaMA._gdense(s2, w.x):
+                _hip.call("llj_g_norm_swiglu", w.x.data_ptr(), C, blk.rms_2.scale.data_ptr(), blk.rms_2.eps, M, C,
+                          s1[1].data_ptr(), s2[1].data_ptr(), H, w.h.data_ptr(), H, w.dt, st)
+            else:
+                _hip.call("llj_g_rmsnorm", w.x.data_ptr(), C, blk.rms_2.scale.data_ptr(), blk.rms_2.eps, w.xn.data_ptr(), C,
+                          M, C, w.dt, st)
+                self._glinear(s1, w.xn, M, C, H, w.a1, None, st)
+                self._glinear(s2, w.xn, M, C, H, w.a2, None, st)
+                _hip.call("llj_g_silu_mul", w.a1.data_ptr(), w.a2.data_ptr(), w.h.data_ptr(), M * H, w.dt, st)
             self._glinear(sd, w.h, M, H, C, w.x, w.x, st)
+
+    @staticmethod
+    def _gdense(spec, x) -> bool:
+        """A dense weight of x's type (the norm-fused products take no other; _glinear checks the type of the rest)."""
+        return spec[0] == 1 and spec[1].dtype == x.dtype
+
+    @staticmethod
+    def _gnorm_linear(fused, x, norm, spec, M, K, N, out, w, st):
+        """out = norm(x) . W^T, in one launch where the rows and the weight allow it (llj_g_norm_ok)."""
+        if fused and LLaMA._gdense(spec, x):
+            _hip.call("llj_g_norm_linear", x.data_ptr(), x.stride(0), norm.scale.data_ptr(), norm.eps, M, K,
+                      spec[1].data_ptr(), N, out.data_ptr(), out.stride(0), w.dt, st)
+            return
+        xn = w.xn if M <= w.xn.shape[0] else torch.empty_like(x)
+        _hip.call("llj_g_rmsnorm", x.data_ptr(), x.stride(0), norm.scale.data_ptr(), norm.eps, xn.data_ptr(), K, M, K, w.dt, st)
+        LLaMA._glinear(spec, xn, M, K, N, out, None, st)
 
     def _blocks(self, w, specs, kv, pos, B, T, S, st):
         cfg = self.config
@@ -760,10 +785,8 @@ class LLaMA(nn.Module):
         C, V = cfg.n_embd, cfg.padded_vocab_size
         ln = self.transformer.ln_f
         if w.generic:  # ln_f + lm_head on the any-shape kernels
-            xn = w.xn if M <= w.xn.shape[0] else torch.empty_like(x)
-            _hip.call("llj_g_rmsnorm", x.data_ptr(), x.stride(0), ln.scale.data_ptr(), ln.eps, xn.data_ptr(), C, M, C,
-                      w.dt, st)
-            self._glinear(specs["head"], xn, M, C, V, out, None, st)
+            fused = bool(_hip.lib().llj_g_norm_ok(M, C, w.dt))
+            LLaMA._gnorm_linear(fused, x, ln, specs["head"], M, C, V, out, w, st)
             return
         f, W, sz = specs["head"]
         rs = nst = None

@@ -223,3 +223,77 @@ def test_generic_gemm_edges_vs_float64(kind, bits, group, dt, M, N, K, pad, off)
         for got in (y, one):
             bad = (got.double() - ref).abs() > lim + 1e-30
             assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside the bound"
+
+
+# ---- up to 8 rows (generic_rows.h)
+@pytest.mark.parametrize("dt", [0, 1])
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N,K,off", [(1, 1, 0), (5, 6, 0), (780, 780, 0), (36, 2304, 0), (129, 4100, 1), (8200, 260, 0), (8193, 40, 0)])
+def test_generic_rows_vs_float64_and_fused_forms(dt, M, N, K, off):
+    """Rows of x at and off the loads' alignment, columns in ones and fours, K tails, the residual in place. Bound: a lane
+    sums ceil(K / 64) + 7 products, six more additions over the lanes, half an ulp of sum |x w| each; bf16 as above. The
+    norm-fused forms give bitwise what the separate calls give: the same sums in the same order."""
+    from lit_llama import _hip
+
+    g = torch.Generator("cuda").manual_seed(M * N + K)
+    dtype = torch.float32 if dt else torch.bfloat16
+    x = torch.randn(M * K + 1, device="cuda", generator=g).to(dtype)[off:off + M * K].view(M, K)
+    w, w2 = (torch.randn(N, K, device="cuda", generator=g).to(dtype) for _ in range(2))
+    nw = (1 + 0.1 * torch.randn(K, device="cuda", generator=g)).to(dtype)
+    res = torch.randn(M, N, device="cuda", generator=g).to(dtype)
+    want, mass = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    half = 0.0 if dt else 2.0 ** -8 * 1.01
+    st = _hip.stream()
+    for resid in (None, res):
+        ref = want if resid is None else want + resid.double()
+        lim = mass * 2.0 ** -24 * (K // 64 + 14) + half * want.abs()
+        lim = lim if resid is None else lim + (half + 2.0 ** -24) * (ref.abs() + half * want.abs())
+        y = torch.empty_like(res) if resid is None else resid.clone()
+        _hip.g_linear(1, x, M, K, w, None, None, 16, K, N, y, None if resid is None else y, dt, st)
+        assert ((y.double() - ref).abs() <= lim + 1e-30).all()
+    assert _hip.lib().llj_g_norm_ok(M, K, dt) == (M * K * (4 if dt else 2) <= 48 * 1024)
+    if not _hip.lib().llj_g_norm_ok(M, K, dt):
+        return
+    xn, one, two, sep = torch.empty(M, K, dtype=dtype, device="cuda"), *(torch.empty_like(res) for _ in range(3))
+    _hip.call("llj_g_rmsnorm", x.data_ptr(), K, nw.data_ptr(), 1e-5, xn.data_ptr(), K, M, K, dt, st)
+    _hip.g_linear(1, xn, M, K, w, None, None, 16, K, N, one, None, dt, st)
+    _hip.g_linear(1, xn, M, K, w2, None, None, 16, K, N, two, None, dt, st)
+    fused = torch.empty_like(one)
+    _hip.call("llj_g_norm_linear", x.data_ptr(), K, nw.data_ptr(), 1e-5, M, K, w.data_ptr(), N, fused.data_ptr(), N, dt, st)
+    assert torch.equal(fused, one)
+    _hip.call("llj_g_silu_mul", one.data_ptr(), two.data_ptr(), sep.data_ptr(), M * N, dt, st)
+    _hip.call("llj_g_norm_swiglu", x.data_ptr(), K, nw.data_ptr(), 1e-5, M, K, w.data_ptr(), w2.data_ptr(), N, fused.data_ptr(), N,
+              dt, st)
+    assert torch.equal(fused, sep)
+
+
+@pytest.mark.parametrize("dt", [0, 1])
+@pytest.mark.parametrize("B,nh,hs,S,p", [(1, 10, 78, 132, 0), (3, 10, 78, 132, 131), (2, 2, 2, 16, 40), (1, 3, 64, 300, 17),
+                                         (8, 2, 128, 1000, 999), (1, 1, 600, 40, 20), (1, 1, 1100, 40, 39)])
+def test_generic_rope_attention_vs_separate_calls(dt, B, nh, hs, S, p):
+    """First position, a full cache, a wrapped ring, head sizes from one pair to more pairs than threads: the caches bitwise as
+    llj_g_rope_kv leaves them, the output against attention in float64 over them. Bound: scores and weighted sums
+    lose half an ulp per term of hs and S (exp: 2 more), relative to sum |p v|; bf16 results round by 2^-8."""
+    from lit_llama import _hip
+
+    g = torch.Generator("cuda").manual_seed(B * S + p)
+    dtype, C, st = torch.float32 if dt else torch.bfloat16, nh * hs, _hip.stream()
+    qkv = torch.randn(B, 3 * C, device="cuda", generator=g).to(dtype)
+    kc, vc = (torch.randn(B, nh, S, hs, device="cuda", generator=g).to(dtype) for _ in range(2))
+    ang = torch.rand(p + 1, hs // 2, device="cuda", generator=g) * 6
+    rope = torch.stack([ang.cos(), ang.sin()], -1).contiguous()
+    pos = torch.tensor([p], dtype=torch.int32, device="cuda")
+    k2, v2, q, y = kc.clone(), vc.clone(), torch.empty(B, C, dtype=dtype, device="cuda"), torch.empty(B, C, dtype=dtype, device="cuda")
+    assert _hip.lib().llj_g_rope_attention_ok(S, hs) == 1
+    _hip.call("llj_g_rope_attention", qkv.data_ptr(), kc.data_ptr(), vc.data_ptr(), rope.data_ptr(), pos.data_ptr(), y.data_ptr(),
+              B, C, nh, S, dt, st)
+    _hip.call("llj_g_rope_kv", qkv.data_ptr(), q.data_ptr(), k2.data_ptr(), v2.data_ptr(), rope.data_ptr(), pos.data_ptr(), B, 1, C,
+              nh, S, dt, st)
+    assert torch.equal(kc, k2) and torch.equal(vc, v2)
+    n = min(p + 1, S)
+    s = (k2[:, :, :n].double() * q.view(B, nh, 1, hs).double()).sum(-1) * hs ** -0.5
+    size = (k2[:, :, :n].double() * q.view(B, nh, 1, hs).double()).abs().sum(-1) * hs ** -0.5
+    w = torch.softmax(s, -1)
+    want, mass = ((w[..., None] * t).sum(2).reshape(B, C) for t in (v2[:, :, :n].double(), v2[:, :, :n].double().abs()))
+    loss = 2.0 ** -24 * (n + 16 + 2 * (hs // 2 + 8) * float(size.max()))
+    assert ((y.double() - want).abs() <= mass * loss + (0.0 if dt else 2.0 ** -8 * 1.01) * want.abs() + 1e-30).all()
