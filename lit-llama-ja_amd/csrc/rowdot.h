@@ -1,0 +1,329 @@
+// One activation row times a bf16 weight (N, K): the decode step of a single sequence.
+//
+// Bound: the weights' bytes. A workgroup owns a range of output columns; each of its NW waves keeps its own slice of the row (SL
+// pieces of 512 values, 8 per lane) in registers and streams that slice of column after column -- 1 KiB of consecutive
+// bytes per load, two rounds of loads in flight -- into fp32 multiply-adds. The lanes' sums meet over 16 lanes (DPP), the rest
+// through LDS once per workgroup, where the epilogue also runs, a thread per column with its operands loaded ahead. The MFMA forms (gemv_impl.h,
+// post_gemv.hip), made for several rows, read 16 columns x 64 bytes per load and leave HBM at 60 % of what these reach. In a
+// graph, us (TB/s), MFMA form -> this:
+//   4096 -> 12288   22.0 (4.6) -> 19.0 (5.3)     4096 -> 22016   38.6 (4.7) -> 31.5 (5.7)     4096 -> 4096    8.6 (3.9) -> 8.3 (4.1)
+//   11008 -> 4096   21.7 (4.2) -> 17.3 (5.2)     4096 -> 32000   51.2 (5.1) -> 44.1 (5.9)     2048 -> 2048    7.0 (1.2) -> 4.8 (1.8)
+// (a wave per column, each with the whole row, measured the same without a prologue, but repeats the norm in ten times the
+// workgroups.) The grid is about 2048 waves, 8 per CU with 16 KiB in flight each; 256 or 1024 workgroups of the same waves
+// lose 1-4 %.
+//
+// Prologues (the weights' first loads are in flight meanwhile):
+//   plain    the row from memory, bf16;
+//   norm     RMSNorm with the reference's bf16 rounding points (model.py:281-283);
+//   post     the fp32 residual after a sublayer, x' = x + t / rms(t) * (1 + w), rounded to bf16 as the input and written
+//            once to x';
+//   streams  the residual streams after a sublayer, the mixed row and its layer norm (streams.hip), the new streams written
+//            once to x'.
+#pragma once
+#include "common.h"
+#include "elem.h"
+
+namespace llj {
+
+enum { RD_PLAIN = 0, RD_NORM = 1, RD_POST = 2, RD_STREAMS = 3 };
+// RD_STORE: + bias (fp32 or NULL). RD_RESID: out += . RD_QKV: RoPE, q to out, k / v to the caches. RD_SWIGLU: silu(. W) * (. W2).
+// RD_RELU2: max(., 0)^2. RD_GLU: the clamped gated unit of interleaved columns (elem.h), biased.
+enum { RD_STORE = 0, RD_RESID = 1, RD_QKV = 2, RD_SWIGLU = 3, RD_RELU2 = 4, RD_GLU = 5 };
+
+struct RowDotParams {
+  const bf16_t* A;  // plain, norm: the row
+  const bf16_t* w;  // norm, post, streams: norm weight
+  float eps;
+  int K, N;         // row stride of the weights; output columns (RD_SWIGLU: both weights' rows, 2 H)
+  int C;            // values of the row (<= K, the weights past it are not read)
+  const bf16_t* W;
+  const bf16_t* W2;
+  bf16_t* out;
+  const float* bias;
+  float limit, alpha;
+  const bf16_t* t;  // post, streams: the sublayer's output; residual in / out
+  const float* x;
+  float* xo;
+  const float* so;  // streams: output weights (S), mix (S, S), input weights (S) or NULL; x, xo: S rows of stride ldx
+  const float* sm;
+  const float* si;
+  int S, ldx;
+  bf16_t* kcache;  // RD_QKV
+  bf16_t* vcache;
+  const float* rope;
+  const int* pos;
+  int n_head, hs, ring, T, m;  // ring: cache slots; m: row of q (sequence m / T, position pos[m % T])
+};
+
+constexpr int kRdStreams = 4;
+constexpr int kRdMaxC = 16384;
+
+template <int NW, int SL, int PRO, int EPI>
+__global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
+  extern __shared__ __align__(16) float rd_part[];  // [column][NW * 4]
+  __shared__ float red[2][NW];
+  constexpr int CB = SL == 1 ? 8 : SL == 2 ? 4 : 2;  // columns per round of loads
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+  const int units = p.N >> 1;
+  const int c0 = 2 * (int)((long)blockIdx.x * units / gridDim.x), c1 = 2 * (int)((long)(blockIdx.x + 1) * units / gridDim.x);
+  const int k0 = wave * (SL * 512) + lane * 8;  // slice s: k0 + 512 s
+  u32x4 wv[2][CB][SL];
+  auto fetch = [&](int b, int c) {
+    if (c >= c1) return;
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      const int n = min(c + i, c1 - 1);
+      const bf16_t* r = EPI == RD_SWIGLU ? ((n & 1) ? p.W2 : p.W) + (size_t)(n >> 1) * p.K : p.W + (size_t)n * p.K;
+#pragma unroll
+      for (int s = 0; s < SL; ++s) {
+        const int k = k0 + 512 * s;
+        wv[b][i][s] = k < p.C ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(r + k)) : u32x4{0, 0, 0, 0};
+      }
+    }
+  };
+
+  // ---- the epilogue's operands of column c0 + tid: requested with the row, so that no memory trip follows the last barrier
+  struct Operand {
+    float v;    // RD_RESID: the residual; RD_STORE, RD_GLU: the bias
+    float2 cs;  // RD_QKV: the rotation (cos, sin)
+    size_t at;  // RD_QKV: place in q / k / v
+    int region, odd;
+  };
+  auto operand = [&](int j) {
+    const int n = c0 + j < c1 ? c0 + j : c0;
+    Operand o{};
+    if constexpr (EPI == RD_RESID) o.v = bf2f(p.out[n]);
+    if constexpr (EPI == RD_STORE || EPI == RD_GLU) o.v = p.bias ? p.bias[n] : 0.f;
+    if constexpr (EPI == RD_QKV) {  // model.py:204-228: RoPE in fp32 on the bf16 output, k / v to ring slot p % ring
+      const int Cd = p.n_head * p.hs, nc = n % Cd, h = nc / p.hs, dd = nc - h * p.hs;
+      const int b = p.T == 1 ? p.m : p.m / p.T, ps = p.pos[p.m - b * p.T];
+      o.region = n / Cd;
+      o.odd = dd & 1;
+      o.cs = o.region < 2 ? *reinterpret_cast<const float2*>(p.rope + ((size_t)ps * (p.hs >> 1) + (dd >> 1)) * 2) : float2{1.f, 0.f};
+      o.at = o.region == 0 ? (size_t)p.m * Cd + nc : (((size_t)b * p.n_head + h) * p.ring + ps % p.ring) * p.hs + dd;
+    }
+    return o;
+  };
+
+  // ---- prologue: this lane's values of the row, fp32 holding bf16 values
+  float xf[SL][8];
+  Operand first;
+  auto block_sum = [&](float v, int which) {
+    v = wave_sum(v);
+    if (lane == 0) red[which][wave] = v;
+    __syncthreads();
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) t += red[which][i];
+    return t;
+  };
+  if constexpr (PRO == RD_PLAIN || PRO == RD_NORM) {
+    u32x4 xv[SL], gv[SL];
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      const int k = k0 + 512 * s;
+      xv[s] = k < p.C ? *reinterpret_cast<const u32x4*>(p.A + k) : u32x4{0, 0, 0, 0};
+      if constexpr (PRO == RD_NORM) gv[s] = k < p.C ? *reinterpret_cast<const u32x4*>(p.w + k) : u32x4{0, 0, 0, 0};
+    }
+    fetch(0, c0);
+    first = operand(tid);
+#pragma unroll
+    for (int s = 0; s < SL; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[s][e] = (e & 1) ? bfhi(xv[s][e >> 1]) : bflo(xv[s][e >> 1]);
+    if constexpr (PRO == RD_NORM) {
+      float ss = 0.f;
+#pragma unroll
+      for (int s = 0; s < SL; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += round_bf(xf[s][e] * xf[s][e]);
+      const float r = round_bf(rsqrtf(round_bf(round_bf(block_sum(ss, 0) / (float)p.C) + p.eps)));
+#pragma unroll
+      for (int s = 0; s < SL; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          xf[s][e] = round_bf(((e & 1) ? bfhi(gv[s][e >> 1]) : bflo(gv[s][e >> 1])) * round_bf(xf[s][e] * r));
+    }
+  } else if constexpr (PRO == RD_POST) {
+    u32x4 tv[SL], gv[SL];
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      const int k = k0 + 512 * s, kk = k < p.C ? k : 0;
+      tv[s] = *reinterpret_cast<const u32x4*>(p.t + kk);
+      gv[s] = *reinterpret_cast<const u32x4*>(p.w + kk);
+      ld8(p.x + kk, xf[s]);
+    }
+    fetch(0, c0);
+    first = operand(tid);
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      if (k0 + 512 * s < p.C) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += bflo(tv[s][e]) * bflo(tv[s][e]) + bfhi(tv[s][e]) * bfhi(tv[s][e]);
+      }
+    }
+    const float r = 1.f / sqrtf(block_sum(ss, 0) / (float)p.C + p.eps);
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      const int k = k0 + 512 * s;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float tt = (e & 1) ? bfhi(tv[s][e >> 1]) : bflo(tv[s][e >> 1]);
+        const float gg = (e & 1) ? bfhi(gv[s][e >> 1]) : bflo(gv[s][e >> 1]);
+        xf[s][e] = k < p.C ? xf[s][e] + tt * r * (1.f + gg) : 0.f;
+      }
+      if (k < p.C && (unsigned)(k >> 3) % gridDim.x == blockIdx.x) st8(p.xo + k, xf[s]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[s][e] = round_bf(xf[s][e]);
+    }
+  } else {
+    u32x4 tv[SL], gv[SL];
+    float sv[SL][kRdStreams][8];
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      const int k = k0 + 512 * s, kk = k < p.C ? k : 0;
+      tv[s] = *reinterpret_cast<const u32x4*>(p.t + kk);
+      gv[s] = *reinterpret_cast<const u32x4*>(p.w + kk);
+#pragma unroll
+      for (int q = 0; q < kRdStreams; ++q) ld8(p.x + (size_t)(q < p.S ? q : 0) * p.ldx + kk, sv[s][q]);  // (past S: a copy)
+    }
+    fetch(0, c0);
+    first = operand(tid);
+    float sum = 0.f;
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      const int k = k0 + 512 * s;
+      const bool mine = k < p.C && (unsigned)(k >> 3) % gridDim.x == blockIdx.x;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[s][e] = 0.f;
+#pragma unroll
+      for (int t = 0; t < kRdStreams; ++t) {
+        if (t < p.S) {  // (uniform)
+          float n[8];
+          const float ot = p.so[t], in = p.si ? p.si[t] : 1.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) n[e] = ot * ((e & 1) ? bfhi(tv[s][e >> 1]) : bflo(tv[s][e >> 1]));
+#pragma unroll
+          for (int q = 0; q < kRdStreams; ++q) {
+            const float a = q < p.S ? p.sm[q * p.S + t] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) n[e] += a * sv[s][q][e];
+          }
+          if (mine) st8(p.xo + (size_t)t * p.ldx + k, n);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) xf[s][e] += in * n[e];
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum += k < p.C ? xf[s][e] : 0.f;
+    }
+    const float mean = block_sum(sum, 0) / (float)p.C;
+    sum = 0.f;
+#pragma unroll
+    for (int s = 0; s < SL; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        xf[s][e] -= mean;
+        sum += k0 + 512 * s < p.C ? xf[s][e] * xf[s][e] : 0.f;
+      }
+    const float r = 1.f / sqrtf(block_sum(sum, 1) / (float)p.C + p.eps);
+#pragma unroll
+    for (int s = 0; s < SL; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        xf[s][e] = k0 + 512 * s < p.C ? round_bf(xf[s][e] * r * ((e & 1) ? bfhi(gv[s][e >> 1]) : bflo(gv[s][e >> 1]))) : 0.f;
+  }
+
+  // ---- the stream
+  auto columns = [&](int b, int c) {
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+      float a = 0.f;
+#pragma unroll
+      for (int s = 0; s < SL; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          a = fmaf(bflo(wv[b][i][s][e]), xf[s][2 * e], a);
+          a = fmaf(bfhi(wv[b][i][s][e]), xf[s][2 * e + 1], a);
+        }
+      a = row16_sum(a);
+      if ((lane & 15) == 0 && c + i < c1) rd_part[(c + i - c0) * (NW * 4) + wave * 4 + (lane >> 4)] = a;
+    }
+  };
+  for (int c = c0; c < c1; c += 2 * CB) {
+    fetch(1, c + CB);
+    columns(0, c);
+    fetch(0, c + 2 * CB);
+    if (c + CB < c1) columns(1, c + CB);
+  }
+  __syncthreads();
+
+  // ---- epilogue: thread per column, neighbouring columns in neighbouring lanes (c0 is even)
+  const bool pairs = (((uintptr_t)p.out | (uintptr_t)p.kcache | (uintptr_t)p.vcache) & 3) == 0;
+  for (int j0 = 0; j0 < c1 - c0; j0 += NW * 64) {
+    const int j = j0 + tid, n = c0 + j;
+    const bool live = n < c1;
+    const f32x4* q = reinterpret_cast<const f32x4*>(rd_part + (live ? j : 0) * (NW * 4));
+    float y = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) y += (q[w][0] + q[w][1]) + (q[w][2] + q[w][3]);
+    const Operand op = j0 ? operand(j) : first;
+    if constexpr (EPI == RD_STORE || EPI == RD_GLU) y += op.v;
+    if constexpr (EPI == RD_SWIGLU) {
+      const float a = round_bf(y), b = lane_xor1(a);
+      if (live && !(n & 1)) p.out[n >> 1] = f2bf(round_bf(a / (1.f + __expf(-a))) * b);  // model.py:258 in bf16
+    } else if constexpr (EPI == RD_GLU) {
+      const float u = lane_xor1(y);
+      if (live && !(n & 1)) p.out[n >> 1] = f2bf(clamped_glu(y, u, p.limit, p.alpha));
+    } else {
+      float o = y;
+      if constexpr (EPI == RD_RELU2) o = fmaxf(y, 0.f) * fmaxf(y, 0.f);
+      if constexpr (EPI == RD_RESID) o = round_bf(op.v + round_bf(y));  // model.py:172-173
+      bf16_t* dst = p.out + n;
+      if constexpr (EPI == RD_QKV) {
+        o = round_bf(y);
+        const float partner = lane_xor1(o);
+        if (op.region < 2) o = op.odd ? o * op.cs.x + partner * op.cs.y : o * op.cs.x - partner * op.cs.y;
+        dst = (op.region == 0 ? p.out : op.region == 1 ? p.kcache : p.vcache) + op.at;
+      }
+      const uint32_t ob = (uint32_t)f2bf(o), pr = lane_xor1(ob);
+      if (pairs) {  // columns (n, n + 1) leave as one 4-byte store
+        if (live && !(n & 1)) st_out32(dst, ob | (pr << 16));
+      } else if (live) {
+        *dst = (bf16_t)ob;
+      }
+    }
+  }
+}
+
+template <int NW, int SL, int PRO, int EPI>
+static int rowdot_go(const RowDotParams& p, hipStream_t s) {
+  const int units = p.N / 2;
+  int grid = 2048 / NW;
+  grid = grid < units ? grid : units;
+  // [column][NW * 4] sums of the largest range in 48 KiB (very wide outputs: more workgroups)
+  const long most = 48 * 1024 / (NW * 16) - 2;
+  if ((long)p.N > most * grid) grid = (int)((p.N + most - 1) / most);
+  const size_t lds = (size_t)2 * ((units + grid - 1) / grid) * NW * 16;
+  hipLaunchKernelGGL((rowdot_kernel<NW, SL, PRO, EPI>), dim3(grid), dim3(NW * 64), lds, s, p);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+// The row's slices: as few waves as keep a wave's slice at 1024 values, 8 waves at most (streams, whose prologue reads 20 bytes per
+// value in every workgroup: 8 waves and half the workgroups from 2049 on). C <= kRdMaxC (streams, post: 8192).
+template <int PRO, int EPI>
+static int rowdot_launch(const RowDotParams& p, hipStream_t s) {
+  if (p.C <= 1024) return rowdot_go<2, 1, PRO, EPI>(p, s);
+  if (p.C <= 2048) return rowdot_go<4, 1, PRO, EPI>(p, s);
+  if (p.C <= 4096) return PRO == RD_STREAMS ? rowdot_go<8, 1, PRO, EPI>(p, s) : rowdot_go<4, 2, PRO, EPI>(p, s);
+  if (p.C <= 8192) return rowdot_go<8, 2, PRO, EPI>(p, s);
+  if constexpr (PRO <= RD_NORM) {
+    if (p.C <= 12288) return rowdot_go<8, 3, PRO, EPI>(p, s);
+    if (p.C <= kRdMaxC) return rowdot_go<8, 4, PRO, EPI>(p, s);
+  }
+  return LLJ_EINVAL;
+}
+
+}  // namespace llj

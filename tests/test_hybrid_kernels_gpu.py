@@ -635,3 +635,72 @@ def test_gqa_sink_takes_the_weight(hip, kind, dtype):
     c.inp, c.cache = dev(q, dtype), dev(k, dtype)
     c.run(kind)
     assert np.abs(c.want[0]).max() < 0.15
+
+
+# ------------------------------------------------------------------------------------ one row (rowdot.h)
+@pytest.mark.parametrize("K", [128, 1024, 1152, 2048, 2176, 4096, 4224, 8192, 8320, 12288, 12416, 16384, 16512])
+@pytest.mark.parametrize("N,act", [(16, 0), (4112, 1), (48, 2), (98304, 0)])
+def test_one_row_vs_float64(hip, K, N, act):
+    """Both sides of every slice size (16,512 runs on the MFMA form), fewer columns than workgroups, an output range past
+    one pass of the epilogue's threads. Bound: a lane sums at most 32 products, 4 + 8 more additions, half an ulp of sum
+    |x w| each; the result rounds to bf16 (2^-8), squared or through the unit (slope at most 1.5, values below 12) twice."""
+    if N * K > 1 << 29:
+        N = 8192
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    x = torch.randn(1, K, generator=g, device="cuda").to(torch.bfloat16)
+    W = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    bias = None if act == 1 else torch.randn(N, generator=g, device="cuda")
+    out = torch.empty(1, N // 2 if act == 2 else N, dtype=torch.bfloat16, device="cuda")
+    call("llj_rows_linear", act, x, K, W, bias, out, out.shape[1], 1, N, K, 1.25, 1.5)
+    y = (x.double() @ W.double().T)[0] + (0 if bias is None else bias.double())
+    lim = (x.double().abs() @ W.double().abs().T)[0] * 2.0 ** -24 * 64
+    if act == 1:
+        want, lim = y.clamp(min=0) ** 2, lim * 2 * (y.abs() + lim)
+    elif act == 2:
+        want = torch.from_numpy(_unit_ref(back(y)[None], 1.25, 1.5)[0]).cuda()
+        lim = (lim[0::2] + lim[1::2]) * 4
+    else:
+        want = y
+    assert ((out[0].double() - want).abs() <= lim + 2.0 ** -8 * 1.01 * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("K,H", [(512, 512), (640, 1792), (2048, 5632), (13824, 640)])
+def test_one_row_of_the_block_vs_float64(hip, K, H):
+    """The four ops of a LLaMA block on bf16 weights with one row, row 9 of a longer call included (the last slice of eight),
+    against float64 on the same rounding points. A pre-rounding difference of an fp32 sum can move a bf16 point by one
+    step (2^-7 of the value at most), of which the residual and RoPE outputs see one, the unit two."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    bf = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    r = lambda t: t.to(torch.bfloat16).double()  # noqa: E731
+    x, nw, W = bf(1, K), (1 + 0.1 * torch.randn(K, generator=g, device="cuda")).to(torch.bfloat16), bf(H, K) * K ** -0.5
+    W2, st = bf(H, K) * K ** -0.5, torch.cuda.current_stream().cuda_stream
+    xd = x.double()
+    xn = r(nw.double() * r(xd * r(torch.rsqrt(r(r(r(xd * xd).mean()) + 1e-5)))))
+    near = lambda got, want, steps: float(((got.double() - want).abs() / (want.abs() + 0.05)).max()) <= steps * 2.0 ** -7  # noqa: E731
+    res = bf(1, H)
+    y = res.clone()
+    call("llj_linear_resid", 1, x, K, W, None, y, H, 1, H, K, None, 0, None)
+    assert near(y, r(res.double() + r(xd @ W.double().T)), 2)
+    h = torch.empty(1, H, dtype=torch.bfloat16, device="cuda")
+    call("llj_norm_swiglu", 1, x, nw, 1e-5, W, None, W2, None, h, 1, H, K, None, 0, None, None, 0)
+    a, b = r(xn @ W.double().T), r(xn @ W2.double().T)
+    assert near(h, r(r(a * torch.sigmoid(a)) * b), 5)
+    call("llj_norm_linear", 1, x, nw, 1e-5, W, None, h, H, 1, H, K, None, 0, None, None, 0)
+    assert near(h, r(xn @ W.double().T), 2)
+    if K > 4096:
+        return
+    nh, hs, S, T = K // 64, 64, 16, 10
+    X, q = bf(T, K), torch.zeros(T, K, dtype=torch.bfloat16, device="cuda")
+    X[9] = x[0]
+    Wq = bf(3 * K, K) * K ** -0.5
+    kc, vc = (torch.zeros(1, nh, S, hs, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    ang = torch.rand(64, hs // 2, generator=g, device="cuda") * 6
+    rope = torch.stack([ang.cos(), ang.sin()], -1).contiguous()
+    pos = torch.arange(20, 20 + T, dtype=torch.int32, device="cuda")
+    call("llj_norm_qkv_rope", 1, X, nw, 1e-5, Wq, None, q, kc, vc, rope, pos, 1, T, K, nh, S, 9, 1, None, None, None, 0)
+    qkv = r(xn @ Wq.double().T).view(3, nh, hs)
+    c, s = rope[29, :, 0].double(), rope[29, :, 1].double()
+    rot = lambda t: torch.stack([t[..., 0::2] * c - t[..., 1::2] * s, t[..., 1::2] * c + t[..., 0::2] * s], -1).flatten(-2)  # noqa: E731
+    for got, want in ((q[9].view(nh, hs), rot(qkv[0])), (kc[0, :, 29 % S], rot(qkv[1])), (vc[0, :, 29 % S], qkv[2])):
+        assert float((got.double() - want).abs().max()) <= 2.0 ** -6 * float(want.abs().max())
+    assert float(q[:9].abs().max()) == 0.0
