@@ -23,6 +23,7 @@ ones.
 """
 from __future__ import annotations
 
+import collections
 import weakref
 
 import torch
@@ -30,6 +31,11 @@ import torch
 from . import _hip
 from .model import LLaMA, _Work, _enable_i8_handoff
 from .state import Rows
+
+
+# Captured graphs that nothing replays any more. Freeing one waits for the device; they are freed where the next capture waits
+# anyway, so that a program's next prompt is launched while the last session's steps still run. At most two are kept.
+_retired: collections.deque = collections.deque(maxlen=2)
 
 
 class _Program:
@@ -169,7 +175,7 @@ class HybridProgram(_Program):
     def room(self, n: int) -> None:
         """State for n more tokens per row."""
         if self.state.ensure(max(self.seen) + n):
-            self.sess.graph = None
+            self.sess._drop_graph()
 
     def finish(self, live: list) -> None:
         kept = set(live)
@@ -227,6 +233,15 @@ class DecodeSession:
             _hip.require_device(uniforms, "uniforms")
         self.uniforms = uniforms
 
+    def _drop_graph(self) -> None:
+        if self.graph is not None:
+            _retired.append(self.graph)
+            self.graph = None
+
+    def __del__(self):
+        if getattr(self, "graph", None) is not None and _retired is not None:  # (None: the interpreter is ending)
+            self._drop_graph()
+
     def _choose(self, st):
         """next token of every row from self.logits -> cur and tokens[:, pos + 1]"""
         _hip.call("llj_next_token", self.logits.data_ptr(), self.logits.stride(0), self.B, self.vocab, self.temperature,
@@ -249,7 +264,7 @@ class DecodeSession:
         self.lens = lens if self.ragged else [lens] * self.B
         self.t_prompt = max(self.lens)
         self.steps_done = 1
-        self.graph = None  # the caches / operands may have changed
+        self._drop_graph()  # the caches / operands may have changed
         self.program.prepare()
         return self.program.wanted if want is not None else None
 
@@ -261,6 +276,7 @@ class DecodeSession:
     def capture(self):
         if self.graph is not None or not self.use_graph:
             return
+        _retired.clear()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
             self._step()
@@ -317,7 +333,8 @@ class DecodeSession:
         if self.tokens is not None:
             self.tokens = self.tokens[idx]
         self.lens = [self.lens[b] for b in live]
-        self.B, self.graph = len(live), None
+        self.B = len(live)
+        self._drop_graph()
         if live:
             self.program.prepare()
 

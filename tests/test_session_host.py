@@ -40,3 +40,25 @@ def test_session_is_freed_without_the_collector(program, monkeypatch):
         assert gone() is None
     finally:
         gc.enable()
+
+
+def test_dropped_graphs_wait_for_the_next_capture(monkeypatch):
+    """A session's graph outlives it until the next capture, and at most two are kept."""
+    from lit_llama import engine
+
+    class Graph:
+        pass
+
+    monkeypatch.setattr(engine, "_retired", type(engine._retired)(maxlen=2))
+    refs = []
+    for _ in range(3):
+        sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+        sess.graph = Graph()
+        refs.append(weakref.ref(sess.graph))
+        del sess
+    assert refs[0]() is None and len(engine._retired) == 2
+    sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: 1 / 0)
+    with pytest.raises(ZeroDivisionError):
+        sess.capture()
+    assert refs[1]() is None and refs[2]() is None
