@@ -236,6 +236,32 @@ int llj_gemm_i8_silu_mul(const void* A, int lda, const void* CB, const void* SCB
 int llj_gemm_i8_qkv_rope(const void* x, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
                          const void* w16, int kpad, void* q_out, void* kcache, void* vcache, const float* rope,
                          const int* pos, int B, int T, int C, int n_head, int S, void* stream);
+/* The same products with scratch (llj_gemm_ws_bytes of it, which also serves llj_gemm_resid_ws; 0: not split. A smaller or NULL ws: not
+ * split either): fewer than 256 rows
+ * have few output tiles, so the K range of each is split over workgroups, whose sums meet in ws. */
+size_t llj_gemm_ws_bytes(int wfmt, int M, int N, int K);
+int llj_gemm_linear_ws(int wfmt, const void* A, int lda, const void* W, const void* sz, void* C, int ldc, int M, int N,
+                    int K, void* ws,
+    size_t ws_bytes, void* stream);
+int llj_gemm_silu_mul_ws(int wfmt, const void* A, int lda, const void* W, const void* sz, void* h, int ldh, int M, int N,
+                      int K, void* ws,
+    size_t ws_bytes, void* stream);
+int llj_gemm_qkv_rope_ws(int wfmt, const void* x, const void* W, const void* sz, void* q_out, void* kcache, void* vcache,
+                      const float* rope, const int* pos, int B, int T, int C, int n_head, int S, void* ws,
+    size_t ws_bytes, void* stream);
+int llj_gemm_i8_linear_ws(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                       const void* w16, int kpad, void* C, int ldc, int M, int N, int K, void* ws,
+    size_t ws_bytes, void* stream);
+int llj_gemm_i8_resid_ws(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                      const void* w16, int kpad, void* x, int ldx, int M, int N, int K, void* ws,
+    size_t ws_bytes, void* stream);
+int llj_gemm_i8_silu_mul_ws(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                         const void* w16, int kpad, void* h, int ldh, int M, int N, int K, void* ws,
+    size_t ws_bytes, void* stream);
+int llj_gemm_i8_qkv_rope_ws(const void* x, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                         const void* w16, int kpad, void* q_out, void* kcache, void* vcache, const float* rope,
+                         const int* pos, int B, int T, int C, int n_head, int S, void* ws,
+    size_t ws_bytes, void* stream);
 /* The outlier columns of an activation (its llj_i8_stats workspace) gathered as f16 rows
  * ao16[M][kpad] and of a weight (CB in I8P, SCB) as f16(CB * SCB / 127) rows w16[N][kpad], zero past
  * the outlier count up to the next multiple of 64: with both passed to llj_gemm_i8_* (else NULL,

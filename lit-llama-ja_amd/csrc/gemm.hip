@@ -24,7 +24,8 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 }
 
 template <int EP>
-static int gemm_run(int wfmt, GemmParams& p, void* stream) {
+static int gemm_run(int wfmt, GemmParams& p, void* ws, size_t ws_bytes, void* stream) {
+  p.ws = (float*)ws;  // K slices of fewer than 256 rows (llj_gemm_ws_bytes)
   const bool zint = (wfmt & LLJ_WF_ZINT) != 0;  // int4 only: every zero is an integer
   wfmt &= ~LLJ_WF_ZINT;
   if (zint && wfmt != GWF_W4) return LLJ_EINVAL;
@@ -38,19 +39,19 @@ static int gemm_run(int wfmt, GemmParams& p, void* stream) {
     if (zint && p.M >= 256 && w4z_enabled()) return gemm_glds_launch<GWF_W4Z, EP, 128>(p, s);
     if (p.M >= 256 && p.K % 128 == 0 && glds_enabled(GWF_W4)) return gemm_glds_run<GWF_W4, EP>(p, s);
     if (LLJ_GEMM_BM256_W4 && p.M >= 256) return gemm_launch<GWF_W4, EP, 256>(p, s);
-    return gemm_launch<GWF_W4, EP>(p, s);
+    return gemm_split_launch<GWF_W4, EP>(p, ws_bytes, s);
   }
-  if (wfmt == GWF_W8) return p.sz ? gemm_launch<GWF_W8, EP>(p, s) : LLJ_EINVAL;
+  if (wfmt == GWF_W8) return p.sz ? gemm_split_launch<GWF_W8, EP>(p, ws_bytes, s) : LLJ_EINVAL;
   if ((wfmt & 0xff) == GWF_W4G) {  // grouped int4: group size (128-deep chunks) in the bits above
     p.gch = wfmt >> 8;
-    return (p.sz && p.gch >= 1 && p.K % 128 == 0) ? gemm_launch<GWF_W4G, EP>(p, s) : LLJ_EINVAL;
+    return (p.sz && p.gch >= 1 && p.K % 128 == 0) ? gemm_split_launch<GWF_W4G, EP>(p, ws_bytes, s) : LLJ_EINVAL;
   }
-  if (wfmt == GWF_BF16) return gemm_bf16_run(EP, p, s);
+  if (wfmt == GWF_BF16) return gemm_bf16_run(EP, p, ws_bytes, s);
   if (wfmt == GWF_I8) {
     if (!p.sz || !p.i8ws || p.K % 128) return LLJ_EINVAL;
     if (!p.ao16 != !p.w16 || (p.ao16 && (p.kpad < 64 || p.kpad % 64))) return LLJ_EINVAL;
     if (LLJ_GEMM_BM256_I8 && p.M >= 256) return gemm_launch<GWF_I8, EP, 256>(p, s);
-    return gemm_launch<GWF_I8, EP>(p, s);
+    return gemm_split_launch<GWF_I8, EP>(p, ws_bytes, s);
   }
   return LLJ_EINVAL;
 }
@@ -61,12 +62,18 @@ using namespace llj;
 
 extern "C" {
 
-int llj_gemm_linear(int wfmt, const void* A, int lda, const void* W, const void* sz, void* C, int ldc, int M, int N,
-                    int K, void* stream) {
+int llj_gemm_linear_ws(int wfmt, const void* A, int lda, const void* W, const void* sz, void* C, int ldc, int M, int N,
+                    int K, void* ws,
+    size_t ws_bytes, void* stream) {
   GemmParams p{};
   p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = W; p.sz = (const float2*)sz;
   p.C = (bf16_t*)C; p.ldc = ldc;
-  return gemm_run<GEP_STORE>(wfmt, p, stream);
+  return gemm_run<GEP_STORE>(wfmt, p, ws, ws_bytes, stream);
+}
+
+int llj_gemm_linear(int wfmt, const void* A, int lda, const void* W, const void* sz, void* C, int ldc, int M, int N,
+                    int K, void* stream) {
+  return llj_gemm_linear_ws(wfmt, A, lda, W, sz, C, ldc, M, N, K, nullptr, 0, stream);
 }
 
 int llj_gemm_resid(int wfmt, const void* A, int lda, const void* W, const void* sz, void* x, int ldx, int M, int N,
@@ -74,24 +81,32 @@ int llj_gemm_resid(int wfmt, const void* A, int lda, const void* W, const void* 
   GemmParams p{};
   p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = W; p.sz = (const float2*)sz;
   p.C = (bf16_t*)x; p.ldc = ldx;
-  return gemm_run<GEP_RESID>(wfmt, p, stream);
+  return gemm_run<GEP_RESID>(wfmt, p, nullptr, 0, stream);
+}
+
+int llj_gemm_silu_mul_ws(int wfmt, const void* A, int lda, const void* W, const void* sz, void* h, int ldh, int M, int N,
+                      int K, void* ws,
+    size_t ws_bytes, void* stream) {
+  GemmParams p{};
+  p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = W; p.sz = (const float2*)sz;
+  p.C = (bf16_t*)h; p.ldc = ldh;
+  return gemm_run<GEP_SILU_MUL>(wfmt, p, ws, ws_bytes, stream);
 }
 
 int llj_gemm_silu_mul(int wfmt, const void* A, int lda, const void* W, const void* sz, void* h, int ldh, int M, int N,
                       int K, void* stream) {
-  GemmParams p{};
-  p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = W; p.sz = (const float2*)sz;
-  p.C = (bf16_t*)h; p.ldc = ldh;
-  return gemm_run<GEP_SILU_MUL>(wfmt, p, stream);
+  return llj_gemm_silu_mul_ws(wfmt, A, lda, W, sz, h, ldh, M, N, K, nullptr, 0, stream);
 }
 
-// Workspace bytes llj_gemm_resid_ws needs for this residual GEMM (0: it would not split K -- call
-// llj_gemm_resid).
+// Workspace bytes llj_gemm_resid_ws needs for this residual GEMM of 256 rows or more (0: it would not split K).
 size_t llj_gemm_resid_ws_bytes(int wfmt, int M, int N, int K) {
   int kcs = 0;
   const int ns = splitk_plan(wfmt, M, N, K, &kcs);
   return ns ? (size_t)ns * M * N * sizeof(float) : 0;
 }
+
+// Scratch of the _ws forms below 256 rows (0: they would not split K).
+size_t llj_gemm_ws_bytes(int wfmt, int M, int N, int K) { return gemm_split_bytes(wfmt & 0xff, M, N, K); }
 
 // llj_gemm_resid with the K range split over workgroups (few row tiles): fp32 partials into ws
 // (llj_gemm_resid_ws_bytes), then one reduce launch adds them in slice order and the residual.
@@ -99,14 +114,19 @@ int llj_gemm_resid_ws(int wfmt, const void* A, int lda, const void* W, const voi
                       int K, void* ws, size_t ws_bytes, void* stream) {
   int kcs = 0;
   const int ns = splitk_plan(wfmt, M, N, K, &kcs);
-  if (!ns) return llj_gemm_resid(wfmt, A, lda, W, sz, x, ldx, M, N, K, stream);
+  if (!ns) {
+    GemmParams p{};
+    p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = W; p.sz = (const float2*)sz;
+    p.C = (bf16_t*)x; p.ldc = ldx;
+    return gemm_run<GEP_RESID>(wfmt, p, ws, ws_bytes, stream);
+  }
   if (!ws || ws_bytes < (size_t)ns * M * N * sizeof(float) || (lda & 7) || (ldx & 3) || !A || !W || !x) return LLJ_EINVAL;
   if ((wfmt & ~LLJ_WF_ZINT) == GWF_W4 && !sz) return LLJ_EINVAL;
   GemmParams p{};
   p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = W; p.sz = (const float2*)sz;
   p.ws = (float*)ws; p.nsplit = ns; p.kcs = kcs;
   hipStream_t s = (hipStream_t)stream;
-  const int rc = wfmt == GWF_BF16 ? gemm_bf16_run(GEP_PARTIAL, p, s)
+  const int rc = wfmt == GWF_BF16 ? gemm_bf16_run(GEP_PARTIAL, p, ws_bytes, s)
                                   : gemm_glds_launch<GWF_W4Z, GEP_PARTIAL, 128>(p, s);
   if (rc) return rc;
   const size_t n4 = (size_t)M * N / 4;
@@ -219,36 +239,55 @@ int llj_gemm_swiglu_ws(int wfmt, const void* A, int lda, const void* W1, const v
 }
 
 // LLM.int8() forms (wfmt 2): W = CB in the I8P tiling, sz = SCB (fp32), i8ws = llj_i8_stats of A
-int llj_gemm_i8_linear(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
-                       const void* w16, int kpad, void* C, int ldc, int M, int N, int K, void* stream) {
+int llj_gemm_i8_linear_ws(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                       const void* w16, int kpad, void* C, int ldc, int M, int N, int K, void* ws,
+    size_t ws_bytes, void* stream) {
   GemmParams p{};
   p.ao16 = (const _Float16*)ao16; p.w16 = (const _Float16*)w16; p.kpad = kpad;
   p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = CB; p.sz = (const float2*)SCB;
   p.C = (bf16_t*)C; p.ldc = ldc; p.i8ws = (const char*)i8ws;
-  return gemm_run<GEP_STORE>(GWF_I8, p, stream);
+  return gemm_run<GEP_STORE>(GWF_I8, p, ws, ws_bytes, stream);
 }
 
-int llj_gemm_i8_resid(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
-                      const void* w16, int kpad, void* x, int ldx, int M, int N, int K, void* stream) {
+int llj_gemm_i8_linear(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                       const void* w16, int kpad, void* C, int ldc, int M, int N, int K, void* stream) {
+  return llj_gemm_i8_linear_ws(A, lda, CB, SCB, i8ws, ao16, w16, kpad, C, ldc, M, N, K, nullptr, 0, stream);
+}
+
+int llj_gemm_i8_resid_ws(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                      const void* w16, int kpad, void* x, int ldx, int M, int N, int K, void* ws,
+    size_t ws_bytes, void* stream) {
   GemmParams p{};
   p.ao16 = (const _Float16*)ao16; p.w16 = (const _Float16*)w16; p.kpad = kpad;
   p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = CB; p.sz = (const float2*)SCB;
   p.C = (bf16_t*)x; p.ldc = ldx; p.i8ws = (const char*)i8ws;
-  return gemm_run<GEP_RESID>(GWF_I8, p, stream);
+  return gemm_run<GEP_RESID>(GWF_I8, p, ws, ws_bytes, stream);
 }
 
-int llj_gemm_i8_silu_mul(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
-                         const void* w16, int kpad, void* h, int ldh, int M, int N, int K, void* stream) {
+int llj_gemm_i8_resid(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                      const void* w16, int kpad, void* x, int ldx, int M, int N, int K, void* stream) {
+  return llj_gemm_i8_resid_ws(A, lda, CB, SCB, i8ws, ao16, w16, kpad, x, ldx, M, N, K, nullptr, 0, stream);
+}
+
+int llj_gemm_i8_silu_mul_ws(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                         const void* w16, int kpad, void* h, int ldh, int M, int N, int K, void* ws,
+    size_t ws_bytes, void* stream) {
   GemmParams p{};
   p.ao16 = (const _Float16*)ao16; p.w16 = (const _Float16*)w16; p.kpad = kpad;
   p.A = (const bf16_t*)A; p.lda = lda; p.M = M; p.N = N; p.K = K; p.W = CB; p.sz = (const float2*)SCB;
   p.C = (bf16_t*)h; p.ldc = ldh; p.i8ws = (const char*)i8ws;
-  return gemm_run<GEP_SILU_MUL>(GWF_I8, p, stream);
+  return gemm_run<GEP_SILU_MUL>(GWF_I8, p, ws, ws_bytes, stream);
 }
 
-int llj_gemm_i8_qkv_rope(const void* x, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+int llj_gemm_i8_silu_mul(const void* A, int lda, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                         const void* w16, int kpad, void* h, int ldh, int M, int N, int K, void* stream) {
+  return llj_gemm_i8_silu_mul_ws(A, lda, CB, SCB, i8ws, ao16, w16, kpad, h, ldh, M, N, K, nullptr, 0, stream);
+}
+
+int llj_gemm_i8_qkv_rope_ws(const void* x, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
                          const void* w16, int kpad, void* q_out, void* kcache, void* vcache, const float* rope,
-                         const int* pos, int B, int T, int C, int n_head, int S, void* stream) {
+                         const int* pos, int B, int T, int C, int n_head, int S, void* ws,
+    size_t ws_bytes, void* stream) {
   if (B < 1 || T < 1 || n_head < 1 || C % n_head || S < 1 || !pos || !rope) return LLJ_EINVAL;
   GemmParams p{};
   p.ao16 = (const _Float16*)ao16; p.w16 = (const _Float16*)w16; p.kpad = kpad;
@@ -256,18 +295,30 @@ int llj_gemm_i8_qkv_rope(const void* x, const void* CB, const void* SCB, const v
   p.q_out = (bf16_t*)q_out; p.kcache = (bf16_t*)kcache; p.vcache = (bf16_t*)vcache; p.rope = rope; p.pos = pos;
   p.n_head = n_head; p.head_size = C / n_head; p.S = S; p.T = T; p.i8ws = (const char*)i8ws;
   if (p.head_size & 1 || C % 16) return LLJ_EINVAL;
-  return gemm_run<GEP_QKV>(GWF_I8, p, stream);
+  return gemm_run<GEP_QKV>(GWF_I8, p, ws, ws_bytes, stream);
 }
 
-int llj_gemm_qkv_rope(int wfmt, const void* x, const void* W, const void* sz, void* q_out, void* kcache, void* vcache,
-                      const float* rope, const int* pos, int B, int T, int C, int n_head, int S, void* stream) {
+int llj_gemm_i8_qkv_rope(const void* x, const void* CB, const void* SCB, const void* i8ws, const void* ao16,
+                         const void* w16, int kpad, void* q_out, void* kcache, void* vcache, const float* rope,
+                         const int* pos, int B, int T, int C, int n_head, int S, void* stream) {
+  return llj_gemm_i8_qkv_rope_ws(x, CB, SCB, i8ws, ao16, w16, kpad, q_out, kcache, vcache, rope, pos, B, T, C, n_head, S, nullptr, 0, stream);
+}
+
+int llj_gemm_qkv_rope_ws(int wfmt, const void* x, const void* W, const void* sz, void* q_out, void* kcache, void* vcache,
+                      const float* rope, const int* pos, int B, int T, int C, int n_head, int S, void* ws,
+    size_t ws_bytes, void* stream) {
   if (B < 1 || T < 1 || n_head < 1 || C % n_head || S < 1 || !pos || !rope) return LLJ_EINVAL;
   GemmParams p{};
   p.A = (const bf16_t*)x; p.lda = C; p.M = B * T; p.N = 3 * C; p.K = C; p.W = W; p.sz = (const float2*)sz;
   p.q_out = (bf16_t*)q_out; p.kcache = (bf16_t*)kcache; p.vcache = (bf16_t*)vcache; p.rope = rope; p.pos = pos;
   p.n_head = n_head; p.head_size = C / n_head; p.S = S; p.T = T;
   if (p.head_size & 1 || C % 16) return LLJ_EINVAL;
-  return gemm_run<GEP_QKV>(wfmt, p, stream);
+  return gemm_run<GEP_QKV>(wfmt, p, ws, ws_bytes, stream);
+}
+
+int llj_gemm_qkv_rope(int wfmt, const void* x, const void* W, const void* sz, void* q_out, void* kcache, void* vcache,
+                      const float* rope, const int* pos, int B, int T, int C, int n_head, int S, void* stream) {
+  return llj_gemm_qkv_rope_ws(wfmt, x, W, sz, q_out, kcache, vcache, rope, pos, B, T, C, n_head, S, nullptr, 0, stream);
 }
 
 }  // extern "C"

@@ -5,21 +5,21 @@
 namespace llj {
 
 template <int EP>
-static int bf16_run(const GemmParams& p, hipStream_t s) {
+static int bf16_run(const GemmParams& p, size_t ws_bytes, hipStream_t s) {
   if (p.M >= 256 && glds_enabled(GWF_BF16)) return gemm_glds_run<GWF_BF16, EP>(p, s);
   if (LLJ_GEMM_BM256 && p.M >= 256) return gemm_launch<GWF_BF16, EP, 256>(p, s);
-  return gemm_launch<GWF_BF16, EP>(p, s);
+  return gemm_split_launch<GWF_BF16, EP>(p, ws_bytes, s);
 }
 
-int gemm_bf16_run(int ep, const GemmParams& p, hipStream_t s) {
+int gemm_bf16_run(int ep, const GemmParams& p, size_t ws_bytes, hipStream_t s) {
   switch (ep) {
-    case GEP_STORE: return bf16_run<GEP_STORE>(p, s);
-    case GEP_RESID: return bf16_run<GEP_RESID>(p, s);
-    case GEP_QKV: return bf16_run<GEP_QKV>(p, s);
-    case GEP_SILU_MUL: return bf16_run<GEP_SILU_MUL>(p, s);
-    case GEP_RELU2: return bf16_run<GEP_RELU2>(p, s);
-    case GEP_BIAS: return bf16_run<GEP_BIAS>(p, s);
-    case GEP_GLU: return bf16_run<GEP_GLU>(p, s);
+    case GEP_STORE: return bf16_run<GEP_STORE>(p, ws_bytes, s);
+    case GEP_RESID: return bf16_run<GEP_RESID>(p, ws_bytes, s);
+    case GEP_QKV: return bf16_run<GEP_QKV>(p, ws_bytes, s);
+    case GEP_SILU_MUL: return bf16_run<GEP_SILU_MUL>(p, ws_bytes, s);
+    case GEP_RELU2: return bf16_run<GEP_RELU2>(p, ws_bytes, s);
+    case GEP_BIAS: return bf16_run<GEP_BIAS>(p, ws_bytes, s);
+    case GEP_GLU: return bf16_run<GEP_GLU>(p, ws_bytes, s);
     case GEP_PARTIAL: return gemm_glds_launch<GWF_BF16, GEP_PARTIAL, 128>(p, s);
   }
   return LLJ_EINVAL;
@@ -53,7 +53,7 @@ LLJ_TRACE_EXPORT(gemm_bf16)
 size_t llj_gemm_bf16_ws_bytes(int M, int N, int K) {
   int kcs = 0;
   const int ns = splitk_plan(GWF_BF16, M, N, K, &kcs);
-  return ns ? (size_t)ns * M * N * sizeof(float) : 0;
+  return ns ? (size_t)ns * M * N * sizeof(float) : gemm_split_bytes(GWF_BF16, M, N, K);
 }
 
 int llj_gemm_bf16(int act, const void* A, int lda, const void* W, const float* bias, void* C, int ldc, int M, int N, int K,
@@ -67,10 +67,13 @@ int llj_gemm_bf16(int act, const void* A, int lda, const void* W, const float* b
   hipStream_t s = (hipStream_t)stream;
   int kcs = 0;
   const int ns = act == 0 && ws ? splitk_plan(GWF_BF16, M, N, K, &kcs) : 0;
-  if (!ns) return gemm_bf16_run(act == 2 ? GEP_GLU : act ? GEP_RELU2 : bias ? GEP_BIAS : GEP_STORE, p, s);
+  if (!ns) {
+    p.ws = (float*)ws;
+    return gemm_bf16_run(act == 2 ? GEP_GLU : act ? GEP_RELU2 : bias ? GEP_BIAS : GEP_STORE, p, ws_bytes, s);
+  }
   LLJ_REQUIRE(ws_bytes >= (size_t)ns * M * N * sizeof(float));
   p.ws = (float*)ws; p.nsplit = ns; p.kcs = kcs;
-  if (const int rc = gemm_bf16_run(GEP_PARTIAL, p, s)) return rc;
+  if (const int rc = gemm_bf16_run(GEP_PARTIAL, p, ws_bytes, s)) return rc;
   const size_t n4 = (size_t)M * N / 4;
   hipLaunchKernelGGL(gemm_splitk_store_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, (const float*)ws, ns, M,
                      N, bias, (bf16_t*)C, ldc);

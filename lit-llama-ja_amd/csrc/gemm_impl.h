@@ -62,8 +62,11 @@ enum : int { GWF_W4 = 0, GWF_BF16 = 1, GWF_I8 = 2, GWF_W8 = 3, GWF_W4G = 4, GWF_
 // blockIdx.x % nsplit into ws[slice][M][N]; llj_gemm_resid_ws's reduce adds them and the residual
 // GEP_SWIGLU_PART: split-K slice of the dual SwiGLU pass (its last partial wave of tiles) -- fp32 partials of
 // c_fc1 and c_fc2 (scales applied) into ws[slice][2][M][N]; llj_gemm_swiglu_ws's reduce finishes h
+// GEP_SPLIT: K slice blockIdx.x % slices of a 128-row tile (any format): the slice's sums into ws[slice][M][N] -- fp32 with the scale
+// applied, LLM.int8 its int32 accumulators and, from one more slice that multiplies nothing else, the fp16 side product;
+// gemm_finish_kernel adds them and runs the epilogue
 enum : int { GEP_STORE = 0, GEP_RESID = 1, GEP_QKV = 2, GEP_SILU_MUL = 3, GEP_SWIGLU = 4, GEP_PARTIAL = 5, GEP_SWIGLU_PART = 6, GEP_RELU2 = 7,
-               GEP_BIAS = 8, GEP_GLU = 9 };
+               GEP_BIAS = 8, GEP_GLU = 9, GEP_SPLIT = 10 };
 
 struct GemmParams {
   const bf16_t* A;  // (M, K) rows with stride lda
@@ -92,7 +95,7 @@ struct GemmParams {
   // GEP_SWIGLU: the second weight (c_fc2) and its (scale, 128 + zero) pairs
   const void* W2;
   const float2* sz2;
-  // GEP_PARTIAL: nsplit K slices of kcs 64-deep chunks each (kcs even), fp32 partials [nsplit][M][N]
+  // GEP_PARTIAL, GEP_SPLIT: nsplit K slices of kcs 64-deep chunks each (kcs even; LLM.int8: 128-deep), partials [nsplit][M][N]
   float* ws;
   int nsplit, kcs;
   // GEP_BIAS / GEP_GLU: fp32 bias (N) or NULL, the unit's constants
@@ -269,8 +272,9 @@ constexpr size_t gemm_lds_bytes() {
 }
 
 // BM: rows per tile (128, or 256 for bf16 with 8 waves: 4 row groups x 2 column groups of 64 x 64)
+// (two waves per SIMD: two 128-row workgroups per CU; gptq.int8 and grouped int4 took 268 and 324 registers without the bound)
 template <int WF, int EP, int BM = kGBM>
-__global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(GemmParams p) {
   static_assert(BM == kGBM || WF == GWF_BF16 || WF == GWF_I8 || WF == GWF_W4, "256-row tiles: bf16, int8, int4");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr bool NIB = WF == GWF_W4 || WF == GWF_W8;  // nibble-coded: offset removed with the A row sums
@@ -285,10 +289,21 @@ __global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmParams p) {
   constexpr int MI = BM / WRN / 16, NJ = kGBN / WCN / 16;
   const int wr = wave % WRN, wc = wave / WRN;
   const int row = lane & 15, g = lane >> 4;
-  const int M = p.M, K = p.K, KC = I8 ? K / 128 : K / kGBK, KC128 = K / 128;
+  constexpr bool SPLIT = EP == GEP_SPLIT;
+  const int M = p.M, K = p.K, KCA = I8 ? K / 128 : K / kGBK, KC128 = K / 128;
   const int mtiles = (M + BM - 1) / BM, ntiles = p.N / kGBN;
   const int total = mtiles * ntiles;
   int t = blockIdx.x;
+  // this workgroup's chunks: c0 + [0, KC) of KCA (LLM.int8: the last slice has none, only the side product)
+  int slice = 0, c0 = 0, KC = KCA;
+  if constexpr (SPLIT) {
+    const int ns = p.nsplit + (I8 ? 1 : 0);
+    slice = t % ns;
+    t /= ns;
+    c0 = slice * p.kcs;
+    KC = KCA - c0 < p.kcs ? KCA - c0 : p.kcs;
+    if (I8 && slice == p.nsplit) c0 = KC = 0;
+  }
   if (total % 8 == 0) t = (t % 8) * (total / 8) + t / 8;  // contiguous tile range per XCD
   // m fastest (LLJ_GEMM_MFAST): the workgroups resident on one XCD cover a few weight column
   // panels x every row panel, so a weight panel is fetched once and shared through L2 by all
@@ -328,7 +343,7 @@ __global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmParams p) {
   u32x4 areg[GDEPTH][4], breg[GDEPTH][BV];
   float2 szr[GDEPTH][4];  // GWF_W4G: (scale, 128 + zero) of the chunk's group for the lane's column of tile j
   auto load_chunk = [&](int slot, int c) {
-    c = c < KC ? c : KC - 1;  // past the end: a valid duplicate, never stored
+    c = c0 + (c < KC ? c : KC > 0 ? KC - 1 : 0);  // past the end: a valid duplicate, never stored
     if constexpr (I8) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) areg[slot][v] = *reinterpret_cast<const u32x4*>(aqsrc + (size_t)c * 128 + 16 * v);
@@ -512,7 +527,7 @@ __global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmParams p) {
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) sacc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if constexpr (I8) {
+  if (I8 && (!SPLIT || slice == p.nsplit)) {
     int* s_pre = reinterpret_cast<int*>(smem);  // [kNSB + 1] prefix of the per-block outlier counts
     int* s_k = s_pre + 64;                      // [kSideK] this round's columns
     _Float16* sa16 = reinterpret_cast<_Float16*>(smem + 512);          // [128 rows][kSideP]
@@ -664,6 +679,11 @@ __global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmParams p) {
           const int m = m0 + ml;
           float y = acc[i0 + i][j][r];
           if constexpr (NIB) y = szn.x * (y - szn.y * rs_lds[ml]);
+          if constexpr (SPLIT) {
+            if constexpr (I8) y = slice == p.nsplit ? sacc[i0 + i][j][r] : __int_as_float(iacc[i0 + i][j][r]);
+            if (m < M) p.ws[((size_t)slice * M + m) * p.N + n] = y;
+            continue;
+          }
           if constexpr (EP == GEP_BIAS || EP == GEP_GLU) y += bn;
           const bool live = m < M;
           if constexpr (I8) {  // mm_dequant in fp16, + the fp16 outlier product, in fp16 (the GEMV's epilogue)
@@ -679,6 +699,33 @@ __global__ __launch_bounds__(2 * BM) void gemm_kernel(GemmParams p) {
   }
 }
 
+// The slices of a GEP_SPLIT product in slice order, then epilogue EP: block (64 columns, 4 rows), a thread per element.
+template <int EP, bool I8>
+__global__ __launch_bounds__(256) void gemm_finish_kernel(GemmParams p) {
+  const int n = blockIdx.x * 64 + (threadIdx.x & 63), m = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const bool live = m < p.M;
+  const int mm = live ? m : p.M - 1;
+  const size_t MN = (size_t)p.M * p.N, at = (size_t)mm * p.N + n;
+  const int Cd = p.n_head * p.head_size;
+  const QkvRow qr = EP == GEP_QKV ? qkv_row(p, mm) : QkvRow{};
+  const QkvCol qc = EP == GEP_QKV ? qkv_col(p, n & ~15, n, Cd) : QkvCol{};
+  const float2 op = gemm_operand<EP>(p, mm, n, qr, qc);
+  float y;
+  if constexpr (I8) {
+    const I8WsHeader h8 = *reinterpret_cast<const I8WsHeader*>(p.i8ws);
+    const float sa = i8_layout(p.i8ws, h8.mtot, h8.K).sca[mm], sb = reinterpret_cast<const float*>(p.sz)[n];
+    int a = 0;
+    for (int s = 0; s < p.nsplit; ++s) a += __float_as_int(p.ws[s * MN + at]);
+    y = (float)a * (sa * sb * (1.f / (127.f * 127.f)));
+    y = (float)(_Float16)((float)(_Float16)y + p.ws[p.nsplit * MN + at]);
+  } else {
+    y = p.ws[at];
+    for (int s = 1; s < p.nsplit; ++s) y += p.ws[s * MN + at];
+    if (EP == GEP_BIAS || EP == GEP_GLU) y += p.bias ? p.bias[n] : 0.f;
+  }
+  gemm_store_elem<EP>(p, y, m, n, live, n & 15, Cd, op, qr, qc);
+}
+
 template <int WF, int EP, int BM = kGBM>
 static int gemm_launch(const GemmParams& p, hipStream_t s) {
   auto kern = gemm_kernel<WF, EP, BM>;
@@ -689,8 +736,55 @@ static int gemm_launch(const GemmParams& p, hipStream_t s) {
     if (e != hipSuccess) return (int)e;
     attr_set = true;
   }
-  const int tiles = ((p.M + BM - 1) / BM) * (p.N / kGBN);
+  int tiles = ((p.M + BM - 1) / BM) * (p.N / kGBN);
+  if (EP == GEP_SPLIT) tiles *= p.nsplit + (WF == GWF_I8 ? 1 : 0);
   hipLaunchKernelGGL(kern, dim3(tiles), dim3(2 * BM), lds, s, p);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+#ifndef LLJ_GSPLIT
+#define LLJ_GSPLIT 0  // A/B: slices forced (0: the rule)
+#endif
+// K slices of a product of less than 256 rows (128-row tiles): such a product has 32..172 tiles at 7B widths, one workgroup
+// each with a chain of K / 64 chunk loads, far from the memory and the matrix rate. Returns the slices (1: none), kcs = chunks each.
+// The rule weighs, in us, the chunks of the busiest CU (one chunk of one workgroup; two workgroups on a CU take 1.5, four 3 times
+// as long) against the second launch and the partial sums, and splits for a gain of a tenth. Measured at 128 / 154 rows, us unsplit ->
+// split (slices): 4096 -> 12288 int4 49 -> 39 (4), bf16 123 -> 62 (4), llm.int8 58 -> 33 (4), gptq.int8 80 -> 73 (2);
+// 11008 -> 4096 int4 121 -> 37 (12), bf16 325 -> 89 (8), llm.int8 119 -> 40 (8), gptq.int8 198 -> 58 (8).
+static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out) {
+  if (M >= 256 || M < 1 || N % kGBN || K < kGBK) return 1;
+  const int KC = wf == GWF_I8 ? K / 128 : K / kGBK, planes = wf == GWF_I8 ? 1 : 0;
+  const long tiles = (long)((M + kGBM - 1) / kGBM) * (N / kGBN);
+  const double chunk = wf == GWF_W4 ? 0.75 : wf == GWF_BF16 ? 1.85 : wf == GWF_I8 ? 1.7 : 1.2;
+  int best = 1, best_kcs = KC;
+  double least = 0;
+  for (int ns = LLJ_GSPLIT ? LLJ_GSPLIT : 1; ns <= (LLJ_GSPLIT ? LLJ_GSPLIT : 16); ++ns) {
+    int kcs = (KC + ns - 1) / ns;
+    kcs += kcs & 1;
+    if (ns > 1 && (kcs < 4 || (KC + kcs - 1) / kcs != ns)) continue;
+    const long q = (tiles * ns + 255) / 256;  // workgroups of the busiest CU
+    const double load = q == 1 ? 1.0 : q * 0.75 + (q & 1) * 0.25;
+    const double us = (ns > 1 ? kcs : KC) * chunk * load + (ns > 1 ? 4.0 + (ns + planes) * (double)M * N * 2e-6 : 0.0);
+    if (least == 0 || us < (best == 1 ? 0.9 : 1.0) * least) best = ns, best_kcs = kcs, least = us;
+  }
+  if (kcs_out) *kcs_out = best_kcs;
+  return best;
+}
+static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
+  const int ns = gemm_split_plan(wf, M, N, K, nullptr);
+  return ns < 2 ? 0 : (size_t)(ns + (wf == GWF_I8 ? 1 : 0)) * M * N * 4;
+}
+// The 128-row kernel of format WF, in K slices when p.ws holds ws_bytes enough for the plan.
+template <int WF, int EP>
+static int gemm_split_launch(GemmParams p, size_t ws_bytes, hipStream_t s) {
+  int kcs = 0;
+  const int ns = p.ws ? gemm_split_plan(WF, p.M, p.N, p.K, &kcs) : 1;
+  if (ns < 2 || ws_bytes < gemm_split_bytes(WF, p.M, p.N, p.K)) return gemm_launch<WF, EP>(p, s);
+  p.nsplit = ns;
+  p.kcs = kcs;
+  if (int e = gemm_launch<WF, GEP_SPLIT>(p, s)) return e;
+  hipLaunchKernelGGL((gemm_finish_kernel<EP, WF == GWF_I8>), dim3(p.N / 64, (p.M + 3) / 4), dim3(256), 0, s, p);
   LLJ_CHECK_LAUNCH();
   return 0;
 }
@@ -1472,6 +1566,6 @@ static inline int splitk_plan(int wfmt, int M, int N, int K, int* kcs_out) {
 }
 
 // bf16 (N, K) weights, any epilogue of the plain GEMMs: instantiated in gemm_bf16.hip
-int gemm_bf16_run(int ep, const GemmParams& p, hipStream_t s);
+int gemm_bf16_run(int ep, const GemmParams& p, size_t ws_bytes, hipStream_t s);
 
 }  // namespace llj

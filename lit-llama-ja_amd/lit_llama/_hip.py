@@ -36,9 +36,13 @@ SIGNATURES = {
                           _P],
     "llj_attention_split": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P],
     "llj_gemm_i8_linear": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+    "llj_gemm_i8_linear_ws": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_gemm_i8_resid": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+    "llj_gemm_i8_resid_ws": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_gemm_i8_silu_mul": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+    "llj_gemm_i8_silu_mul_ws": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_gemm_i8_qkv_rope": [_P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
+    "llj_gemm_i8_qkv_rope_ws": [_P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_i8_gather_act": [_P, _I, _I, _I, _P, _P, _I, _P],
     "llj_i8_gather_weight": [_P, _P, _I, _I, _P, _P, _I, _P],
     "llj_gptq_block": [_P, _I, _I, _P, _I, _P, _P, _I, _P, _P, _P, _P],
@@ -67,12 +71,15 @@ SIGNATURES = {
     "llj_i8_norm_rowstats": [_P, _P, _F, _P, _I, _I, _F, _P, _P, _P],
     "llj_i8_linear_resid": [_P, _I, _P, _P, _P, _I, _I, _I, _I, _P, _P],
     "llj_gemm_linear": [_I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
+    "llj_gemm_linear_ws": [_I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_gemm_resid": [_I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
     "llj_gemm_silu_mul": [_I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
+    "llj_gemm_silu_mul_ws": [_I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_gemm_swiglu": [_I, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "llj_gemm_swiglu_ws": [_I, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_gemm_resid_ws": [_I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_gemm_qkv_rope": [_I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
+    "llj_gemm_qkv_rope_ws": [_I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "llj_stream_read": [_P, ctypes.c_size_t, _P, _I, _P],
     "llj_g_embedding": [_P, _P, _P, _I, _I, _P, _I, _P],
     "llj_g_rmsnorm": [_P, _I, _P, _F, _P, _I, _I, _I, _I, _P],
@@ -138,6 +145,7 @@ SIZE_SIGNATURES = {
     "llj_gemm_resid_ws_bytes": [_I, _I, _I, _I],
     "llj_gemm_swiglu_ws_bytes": [_I, _I, _I, _I],
     "llj_g_linear_ws_bytes": [_I, _I, _I, _I, _I],
+    "llj_gemm_ws_bytes": [_I, _I, _I, _I],
     "llj_gemm_bf16_ws_bytes": [_I, _I, _I],
 }
 

@@ -106,7 +106,7 @@ class PackedLinear:
                 _hip.call("llj_rows_linear", act, a[r].data_ptr(), a.stride(0), self.w.data_ptr(), bias, out[r].data_ptr(),
                           out.stride(0), min(STREAM_ROWS, M - r), self.Np, self.Kp, limit, alpha, st)
         else:
-            nb = 0 if act else _hip.lib().llj_gemm_bf16_ws_bytes(M, self.Np, self.Kp)
+            nb = 0 if act and M >= 256 else _hip.lib().llj_gemm_bf16_ws_bytes(M, self.Np, self.Kp)
             ws = torch.empty(nb // 4, dtype=torch.float32, device=out.device) if nb else None
             _hip.call("llj_gemm_bf16", act, a.data_ptr(), a.stride(0), self.w.data_ptr(), bias, out.data_ptr(),
                       out.stride(0), M, self.Np, self.Kp, limit, alpha, _hip.ptr(ws), nb, st)

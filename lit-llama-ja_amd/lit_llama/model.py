@@ -304,6 +304,21 @@ class _Work:
             self.att_part = torch.empty(nb, dtype=torch.uint8, device=device)
 
 
+class _GemmScratch:
+    """Scratch of one prompt call's split products (llj_gemm_ws_bytes): the products of a stream use it in turn."""
+
+    def __init__(self, specs, M, C, H, device, head: Optional[int] = None):
+        L = _hip.lib()
+        nb = L.llj_gemm_ws_bytes(specs["head"][0], M, head, C) if head else 0
+        for f in {s[0] for layer in specs["layers"] for s in layer} if not head else ():
+            g = f | _hip.WF_ZINT if f == 0 and GEMM_ZINT else f  # the larger of the int4 forms
+            nb = max(nb, L.llj_gemm_ws_bytes(f, M, 3 * C, C), L.llj_gemm_ws_bytes(f, M, H, C),
+                     *(L.llj_gemm_ws_bytes(f, M, C, K) for K in (C, H)),
+                     *(L.llj_gemm_resid_ws_bytes(q, M, C, K) for K in (C, H) for q in (f, g) if f != 2))
+        self.buf = torch.empty(nb // 4, dtype=torch.float32, device=device) if nb else None
+        self.ptr, self.nb = _hip.ptr(self.buf), nb
+
+
 @register("LLaMA")
 class LLaMA(nn.Module):
     HIP_SOURCES = None  # every weight format: the whole library
@@ -547,31 +562,33 @@ class LLaMA(nn.Module):
         M = B * T
         P = _hip.ptr
         I8ws = P(w.i8ws)
+        sc = _GemmScratch(specs, M, C, H, w.x.device)
         for i, blk in enumerate(self.transformer.h):
             (fa, wa, sa), (fp, wp, sp), (f1, w1, s1), (f2, w2, s2), (fd, wd, sd) = specs["layers"][i]
             kc, vc = kv[i]
             if fa == 2:  # LLM.int8: the norm + the activation statistics of all M rows, then the int8 GEMM
                 self._i8_norm_prep(w.x, blk.rms_1, w.xn, M, C, w, st)
                 ao, (wg,), kp = self._i8_gathered(w.xn, M, C, [(wa, sa, 3 * C)], w, st)
-                _hip.call("llj_gemm_i8_qkv_rope", w.xn.data_ptr(), wa.data_ptr(), P(sa), I8ws, P(ao), P(wg), kp,
+                _hip.call("llj_gemm_i8_qkv_rope_ws", w.xn.data_ptr(), wa.data_ptr(), P(sa), I8ws, P(ao), P(wg), kp,
                           w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), self.rope_cache.data_ptr(), pos.data_ptr(),
-                          B, T, C, nh, S, st)
+                          B, T, C, nh, S, sc.ptr, sc.nb, st)
             else:
                 _hip.call("llj_rmsnorm_rows", w.x.data_ptr(), blk.rms_1.scale.data_ptr(), blk.rms_1.eps,
                           w.xn.data_ptr(), None, M, C, st)
-                _hip.call("llj_gemm_qkv_rope", _gz(fa, blk.attn.c_attn), w.xn.data_ptr(), wa.data_ptr(), P(sa), w.q.data_ptr(),
-                          kc.data_ptr(), vc.data_ptr(), self.rope_cache.data_ptr(), pos.data_ptr(), B, T, C, nh, S, st)
+                _hip.call("llj_gemm_qkv_rope_ws", _gz(fa, blk.attn.c_attn), w.xn.data_ptr(), wa.data_ptr(), P(sa),
+                          w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), self.rope_cache.data_ptr(), pos.data_ptr(), B, T, C,
+                          nh, S, sc.ptr, sc.nb, st)
             self._attention(w, kc, vc, pos, B, T, S, st)
-            self._gemm_resid(_gz(fp, blk.attn.c_proj), w.y, wp, sp, w.x, M, C, C, w, st)
+            self._gemm_resid(_gz(fp, blk.attn.c_proj), w.y, wp, sp, w.x, M, C, C, w, sc, st)
             if f1 != f2:
                 raise TypeError("c_fc1 and c_fc2 must share a weight format")
             if f1 == 2:
                 self._i8_norm_prep(w.x, blk.rms_2, w.xn, M, C, w, st)
                 ao, (g1, g2), kp = self._i8_gathered(w.xn, M, C, [(w1, s1, H), (w2, s2, H)], w, st)
-                _hip.call("llj_gemm_i8_linear", w.xn.data_ptr(), C, w1.data_ptr(), P(s1), I8ws, P(ao), P(g1), kp,
-                          w.h.data_ptr(), H, M, H, C, st)
-                _hip.call("llj_gemm_i8_silu_mul", w.xn.data_ptr(), C, w2.data_ptr(), P(s2), I8ws, P(ao), P(g2), kp,
-                          w.h.data_ptr(), H, M, H, C, st)
+                _hip.call("llj_gemm_i8_linear_ws", w.xn.data_ptr(), C, w1.data_ptr(), P(s1), I8ws, P(ao), P(g1), kp,
+                          w.h.data_ptr(), H, M, H, C, sc.ptr, sc.nb, st)
+                _hip.call("llj_gemm_i8_silu_mul_ws", w.xn.data_ptr(), C, w2.data_ptr(), P(s2), I8ws, P(ao), P(g2), kp,
+                          w.h.data_ptr(), H, M, H, C, sc.ptr, sc.nb, st)
             else:
                 _hip.call("llj_rmsnorm_rows", w.x.data_ptr(), blk.rms_2.scale.data_ptr(), blk.rms_2.eps,
                           w.xn.data_ptr(), None, M, C, st)
@@ -587,29 +604,23 @@ class LLaMA(nn.Module):
                         _hip.call("llj_gemm_swiglu", g1, w.xn.data_ptr(), C, w1.data_ptr(), P(s1), w2.data_ptr(),
                                   P(s2), w.h.data_ptr(), H, M, H, C, st)
                 else:
-                    _hip.call("llj_gemm_linear", g1, w.xn.data_ptr(), C, w1.data_ptr(), P(s1), w.h.data_ptr(), H, M,
-                              H, C, st)
-                    _hip.call("llj_gemm_silu_mul", g2, w.xn.data_ptr(), C, w2.data_ptr(), P(s2), w.h.data_ptr(), H,
-                              M, H, C, st)
-            self._gemm_resid(_gz(fd, blk.mlp.c_proj), w.h, wd, sd, w.x, M, C, H, w, st)
+                    _hip.call("llj_gemm_linear_ws", g1, w.xn.data_ptr(), C, w1.data_ptr(), P(s1), w.h.data_ptr(), H, M,
+                              H, C, sc.ptr, sc.nb, st)
+                    _hip.call("llj_gemm_silu_mul_ws", g2, w.xn.data_ptr(), C, w2.data_ptr(), P(s2), w.h.data_ptr(), H,
+                              M, H, C, sc.ptr, sc.nb, st)
+            self._gemm_resid(_gz(fd, blk.mlp.c_proj), w.h, wd, sd, w.x, M, C, H, w, sc, st)
 
-    def _gemm_resid(self, f, A, W, sz, x, M, N, K, w, st):
+    def _gemm_resid(self, f, A, W, sz, x, M, N, K, w, sc, st):
         """x += A . W^T for many rows (LLM.int8: the statistics of A first)."""
         if f == 2:
             self._i8_prep(A, M, K, w, st)
             ao, (wg,), kp = self._i8_gathered(A, M, K, [(W, sz, N)], w, st)
-            _hip.call("llj_gemm_i8_resid", A.data_ptr(), A.stride(0), W.data_ptr(), _hip.ptr(sz), _hip.ptr(w.i8ws),
-                      _hip.ptr(ao), _hip.ptr(wg), kp, x.data_ptr(), x.stride(0), M, N, K, st)
+            _hip.call("llj_gemm_i8_resid_ws", A.data_ptr(), A.stride(0), W.data_ptr(), _hip.ptr(sz), _hip.ptr(w.i8ws),
+                      _hip.ptr(ao), _hip.ptr(wg), kp, x.data_ptr(), x.stride(0), M, N, K, sc.ptr, sc.nb, st)
         else:
-            # few row tiles (256..1024 prompt rows): the K range split over workgroups (llj_gemm_resid_ws)
-            nb = _hip.lib().llj_gemm_resid_ws_bytes(f, M, N, K) if M >= 256 else 0
-            if nb:
-                ws = torch.empty(nb // 4, dtype=torch.float32, device=x.device)
-                _hip.call("llj_gemm_resid_ws", f, A.data_ptr(), A.stride(0), W.data_ptr(), _hip.ptr(sz), x.data_ptr(),
-                          x.stride(0), M, N, K, ws.data_ptr(), nb, st)
-            else:
-                _hip.call("llj_gemm_resid", f, A.data_ptr(), A.stride(0), W.data_ptr(), _hip.ptr(sz), x.data_ptr(),
-                          x.stride(0), M, N, K, st)
+            # few row tiles (up to 1024 prompt rows): the K range split over workgroups
+            _hip.call("llj_gemm_resid_ws", f, A.data_ptr(), A.stride(0), W.data_ptr(), _hip.ptr(sz), x.data_ptr(),
+                      x.stride(0), M, N, K, sc.ptr, sc.nb, st)
 
     @staticmethod
     def _glinear(spec, A, M, K, N, out, resid, st):
@@ -802,15 +813,17 @@ class LLaMA(nn.Module):
             self._i8_norm_prep(x, ln, xn, M, C, w, st)
             if M >= GEMM_MIN_ROWS and C % 128 == 0 and V % 128 == 0:  # many rows: the int8 GEMM
                 ao, (wg,), kp = self._i8_gathered(xn, M, C, [(W, sz, V)], w, st)
-                _hip.call("llj_gemm_i8_linear", xn.data_ptr(), C, W.data_ptr(), _hip.ptr(sz), _hip.ptr(w.i8ws),
-                          _hip.ptr(ao), _hip.ptr(wg), kp, out.data_ptr(), out.stride(0), M, V, C, st)
+                sc = _GemmScratch(specs, M, C, 0, x.device, head=V)
+                _hip.call("llj_gemm_i8_linear_ws", xn.data_ptr(), C, W.data_ptr(), _hip.ptr(sz), _hip.ptr(w.i8ws),
+                          _hip.ptr(ao), _hip.ptr(wg), kp, out.data_ptr(), out.stride(0), M, V, C, sc.ptr, sc.nb, st)
                 return
             src, nw = xn, None
         elif M >= GEMM_MIN_ROWS and _gemm_fmt(f) and C % 128 == 0 and V % 128 == 0:  # many rows: GEMM
             xn = torch.empty_like(x)
             _hip.call("llj_rmsnorm_rows", x.data_ptr(), ln.scale.data_ptr(), ln.eps, xn.data_ptr(), None, M, C, st)
-            _hip.call("llj_gemm_linear", _gz(f, self.lm_head), xn.data_ptr(), C, W.data_ptr(), _hip.ptr(sz),
-                      out.data_ptr(), out.stride(0), M, V, C, st)
+            sc = _GemmScratch(specs, M, C, 0, x.device, head=V)
+            _hip.call("llj_gemm_linear_ws", _gz(f, self.lm_head), xn.data_ptr(), C, W.data_ptr(), _hip.ptr(sz),
+                      out.data_ptr(), out.stride(0), M, V, C, sc.ptr, sc.nb, st)
             return
         elif x is w.x and w.hand and f != 2 and len(self.transformer.h) > 0:  # the last mlp.c_proj's partials
             nst = w.nst

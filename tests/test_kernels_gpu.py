@@ -1793,3 +1793,73 @@ def test_attention_part_merged_in_cproj(hip, nsplit, p0, S):
     assert_bf16_close(xb.float().cpu().numpy(), ref, "one-block attention + resid", rel=2e-2)
     assert_bf16_close(xa.float().cpu().numpy(), ref, f"merged attn.c_proj nsplit={nsplit} p={p0}", rel=2e-2)
     assert_bf16_close(xa.float().cpu().numpy(), xb.float().cpu().numpy(), "merged vs one-block + resid", rel=2e-2)
+
+
+@pytest.mark.parametrize("M", [32, 129, 255])
+@pytest.mark.parametrize("N,K", [(128, 1024), (384, 4224), (256, 11008)])
+@pytest.mark.parametrize("wfmt", [0, 1, 2, 3, W4G_128])
+def test_gemm_split_below_256_rows(hip, wfmt, M, N, K):
+    """K slices (llj_gemm_*_ws) against the unsplit kernel on the same operands, partial row tiles and an odd last slice
+    included. LLM.int8: bitwise (int32 sums, the side product in a slice of its own). The others add the same products in
+    another fp32 order, which can move a rounding to bf16 by one step (2^-7 of the value at most): the product's, and the
+    result's -- next to a residual the product's step counts at the product's size, which may exceed the sum's; the unit's
+    factor is the old value at most 1.1 times itself, so two steps of the result. 1e-3 of the largest for the fp32 sums
+    themselves where codes' offsets cancel."""
+    rng = np.random.default_rng(M + N + K + wfmt)
+    assert hip.llj_gemm_ws_bytes(wfmt, M, N, K) >= 2 * M * N * 4 and hip.llj_gemm_ws_bytes(wfmt, 256, N, K) == 0
+    scr = torch.full((hip.llj_gemm_ws_bytes(wfmt, M, N, K) // 4,), float("nan"), device=dev)
+    ws = (scr.data_ptr(), scr.numel() * 4)
+    x = T(_i8_act(rng, M, K, 6 if wfmt == 2 else 0), torch.bfloat16)
+    res = T(bf16(rng.standard_normal((M, N))), torch.bfloat16)
+    if wfmt == 2:
+        iws = torch.empty(hip.llj_i8_ws_bytes(M, K), dtype=torch.uint8, device=dev)
+        call(hip, "llj_i8_stats", x.data_ptr(), K, M, K, 6.0, iws.data_ptr(), st())
+        W, sz = _i8_operands(hip, bf16(rng.standard_normal((N, K)) * 0.02))[:2]
+        ao, (g1,), kp, keep = _i8_gather(hip, x, M, K, iws, [(W, sz, N)], M == 129)
+        pre = (x.data_ptr(), K, W.data_ptr(), sz.data_ptr(), iws.data_ptr(), ao, g1, kp)
+        names = ("llj_gemm_i8_linear", "llj_gemm_i8_resid", "llj_gemm_i8_silu_mul")
+    else:
+        _, W, sz = quant_operands(hip, rng, wfmt, N, K)
+        pre = (wfmt, x.data_ptr(), K, W.data_ptr(), None if sz is None else sz.data_ptr())
+        names = ("llj_gemm_linear", "llj_gemm_resid", "llj_gemm_silu_mul")
+    for name in names:
+        a, b = res.clone(), res.clone()
+        call(hip, name, *pre, a.data_ptr(), N, M, N, K, st())
+        call(hip, name + "_ws", *pre, b.data_ptr(), N, M, N, K, *ws, st())
+        torch.cuda.synchronize()
+        if wfmt == 2:
+            assert torch.equal(a, b), name
+        else:
+            step = a.float().abs() + ((a.float() - res.float()).abs() if "resid" in name else a.float().abs())
+            assert ((a.float() - b.float()).abs() <= 2.0 ** -7 * 1.01 * step + 1e-3 * a.float().abs().max()).all(), name
+
+
+@pytest.mark.parametrize("wfmt", [0, 1, 2, 3, W4G_128])
+def test_gemm_split_qkv(hip, wfmt):
+    """The c_attn product in K slices: q and the cache rows as the unsplit kernel leaves them, two sequences of 45 tokens."""
+    rng = np.random.default_rng(wfmt)
+    B, T_, nh, hs, S = 2, 45, 16, 128, 64
+    C, M = nh * hs, B * T_
+    assert hip.llj_gemm_ws_bytes(wfmt, M, 3 * C, C) > 0
+    scr = torch.empty(hip.llj_gemm_ws_bytes(wfmt, M, 3 * C, C) // 4, device=dev)
+    x, rope = T(_i8_act(rng, M, C, 6 if wfmt == 2 else 0), torch.bfloat16), T(O.build_rope_cache(128, hs))
+    pos = T(np.arange(7, 7 + T_, dtype=np.int32))
+    if wfmt == 2:
+        iws = torch.empty(hip.llj_i8_ws_bytes(M, C), dtype=torch.uint8, device=dev)
+        call(hip, "llj_i8_stats", x.data_ptr(), C, M, C, 6.0, iws.data_ptr(), st())
+        W, sz = _i8_operands(hip, bf16(rng.standard_normal((3 * C, C)) * 0.02))[:2]
+        name, pre = "llj_gemm_i8_qkv_rope", (x.data_ptr(), W.data_ptr(), sz.data_ptr(), iws.data_ptr(), None, None, 0)
+    else:
+        _, W, sz = quant_operands(hip, rng, wfmt, 3 * C, C)
+        name, pre = "llj_gemm_qkv_rope", (wfmt, x.data_ptr(), W.data_ptr(), None if sz is None else sz.data_ptr())
+    outs = []
+    for tail in ((), (scr.data_ptr(), scr.numel() * 4)):
+        q, kc, vc = (torch.zeros(*s, dtype=torch.bfloat16, device=dev) for s in ((M, C), (B, nh, S, hs), (B, nh, S, hs)))
+        call(hip, name + ("_ws" if tail else ""), *pre, q.data_ptr(), kc.data_ptr(), vc.data_ptr(), rope.data_ptr(),
+             pos.data_ptr(), B, T_, C, nh, S, *tail, st())
+        torch.cuda.synchronize()
+        outs.append([t.float().cpu().numpy() for t in (q, kc, vc)])
+    for a, b in zip(*outs):
+        if wfmt == 2:
+            np.testing.assert_array_equal(a, b)
+        assert_bf16_close(b, a, name, rel=2.0 ** -6, abs_frac=4e-3)
