@@ -224,9 +224,15 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logi
 // from the same distribution with its own generator (exponential race); u is either given
 // (u_in, tests) or a counter-based hash of (seed, decode position, row), so a captured decode
 // graph samples a fresh u every step without the host.
-// One 1024-thread block per row. The top_k threshold is an exact radix select on the 16-bit
-// order-preserving keys of the bf16 values (a 2048-bin histogram of key >> 5, then a 32-bin one
-// inside the selected bin, each walked with a block suffix scan), so no sort is needed.
+// One 1024-thread block per row, bound by its chain of block-wide steps and, the row being one CU's, by the instructions per
+// value. The row is read once, as order-preserving keys, into LDS (rows of more than kSampRow bytes are read again by each pass).
+// Each thread keeps the largest key it loaded; for top_k <= 1024 the top_k-th largest of those 1024 keys, rounded down to its
+// histogram bin, cannot lie above the top_k-th largest key of all, so only keys from there on -- a few hundred -- enter the exact
+// radix select (histograms of 11 + 5 bits of the bf16 keys, of 11 + 11 + 10 of the fp32 keys) and the passes after it: the set
+// bits of a mask over a thread's range. The running sum over the threads is one chain of additions in thread order, of the threads
+// that keep anything (a zero adds nothing), along the lanes of a wave. Where every pass read the row in memory and the chain
+// ran through LDS, us a launch, before -> now, V = 32000 bf16: top_k 200 55.1 -> 16.3, 1100 55.2 -> 32.5, all 55.2 -> 29.0;
+// V = 35008 bf16: 47.4 -> 17.8; V = 32000 fp32: 62.2 -> 19.9; V = 100278 bf16 (not in LDS): 147 -> 66.
 __device__ __forceinline__ uint32_t bf_key(uint32_t b) { return (b & 0x8000u) ? (~b & 0xFFFFu) : (b | 0x8000u); }
 __device__ __forceinline__ float key_bf(uint32_t k) {
   const uint32_t b = (k & 0x8000u) ? (k & 0x7FFFu) : (~k & 0xFFFFu);
@@ -240,33 +246,47 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
 }
 
 constexpr int kSampNT = 1024;
-// Exclusive suffix sum over the block (thread order): sum of v over threads > tid.
-__device__ __forceinline__ uint32_t block_suffix_excl(uint32_t v, uint32_t* wsum) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  uint32_t x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_down((int)x, o, 64);
-    if (lane + o < 64) x += y;
+// inclusive prefix over the wave in lane order (OP 0: sum, 1: maximum)
+template <int OP>
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
+#define LLJ_DPP_STEP(ctrl, rows)                                                                  \
+  {                                                                                               \
+    const uint32_t t = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false);  \
+    v = OP ? max(v, t) : v + t;                                                                   \
   }
-  if (lane == 0) wsum[wv] = x;
-  __syncthreads();
-  uint32_t above = 0;
-  for (int w = wv + 1; w < kSampNT / 64; ++w) above += wsum[w];
-  __syncthreads();
-  return x - v + above;
+  LLJ_DPP_STEP(0x111, 0xf)  // row_shr 1, 2, 4, 8: within 16 lanes
+  LLJ_DPP_STEP(0x112, 0xf)
+  LLJ_DPP_STEP(0x114, 0xf)
+  LLJ_DPP_STEP(0x118, 0xf)
+  LLJ_DPP_STEP(0x142, 0xa)  // the last lane of rows 0, 2 into rows 1, 3; then of the first half into the second
+  LLJ_DPP_STEP(0x143, 0xc)
+#undef LLJ_DPP_STEP
+  return v;
+}
+constexpr int kSampWaves = kSampNT / 64;
+// one value per wave, all read at once
+__device__ __forceinline__ void per_wave(const uint32_t* w, uint32_t (&o)[kSampWaves]) {
+#pragma unroll
+  for (int i = 0; i < kSampWaves / 4; ++i) {
+    const uint4 q = reinterpret_cast<const uint4*>(w)[i];
+    o[4 * i] = q.x;
+    o[4 * i + 1] = q.y;
+    o[4 * i + 2] = q.z;
+    o[4 * i + 3] = q.w;
+  }
 }
 
 // The logits type of the sampler: bf16 (the reference's GPU precision: x = bf16(logits * (1/T)),
-// probabilities rounded to bf16; 16-bit keys selected in passes of 11 + 5 bits) or fp32 (its
-// float32 model: x = logits / T, fp32 softmax; 32-bit keys in passes of 11 + 11 + 10 bits).
+// probabilities rounded to bf16) or fp32 (its
+// float32 model: x = logits / T, fp32 softmax).
 template <typename T>
 struct SampTraits;
 template <>
 struct SampTraits<bf16_t> {
   static constexpr int NP = 2;
   static constexpr int SH[3] = {5, 0, 0}, W[3] = {11, 5, 0};
-  __device__ static uint32_t key(const bf16_t* l, int i, float inv_t, float) { return bf_key(f2bf(bf2f(l[i]) * inv_t)); }
+  using Key = uint16_t;
+  __device__ static uint32_t key(bf16_t l, float inv_t, float) { return bf_key(f2bf(bf2f(l) * inv_t)); }
   __device__ static float val(uint32_t k) { return key_bf(k); }
   __device__ static float ex(float d) { return __expf(d); }
   __device__ static float prob(float e) { return bf2f(f2bf(e)); }
@@ -280,144 +300,272 @@ template <>
 struct SampTraits<float> {
   static constexpr int NP = 3;
   static constexpr int SH[3] = {21, 10, 0}, W[3] = {11, 11, 10};
-  __device__ static uint32_t key(const float* l, int i, float, float t) { return f_key(l[i] / t); }
+  using Key = uint32_t;
+  __device__ static uint32_t key(float l, float, float t) { return f_key(l / t); }
   __device__ static float val(uint32_t k) { return key_f(k); }
   __device__ static float ex(float d) { return expf(d); }
   __device__ static float prob(float e) { return e; }
 };
 
+constexpr size_t kSampRow = 144 * 1024;  // largest row of keys held in LDS
+
+// stride: Keys from one thread's range to the next in LDS (0: not there; more than the range: an odd number of words, so that
+// the threads' places lie in different banks, and 16-byte pieces of the row are each one thread's)
 template <typename T>
 __global__ __launch_bounds__(kSampNT) void sample_kernel(const T* __restrict__ logits, int ldl, int V, float inv_t,
                                                         float temp, int top_k, const float* __restrict__ u_in,
                                                         uint64_t seed, int* __restrict__ out_idx,
                                                         int* __restrict__ tokens_out, int tok_stride,
-                                                        const int* __restrict__ pos, int pos_step) {
+                                                        const int* __restrict__ pos, int pos_step, int stride) {
   using Tr = SampTraits<T>;
+  using Key = typename Tr::Key;
   constexpr int HB = 2048;  // the widest pass: 11 bits
-  __shared__ uint32_t hist[HB];
-  __shared__ float fred[kSampNT / 64];
-  __shared__ uint32_t ured[kSampNT / 64];
-  __shared__ float chunk_excl[kSampNT];
+  extern __shared__ __attribute__((aligned(16))) unsigned char samp_row[];
+  __shared__ __attribute__((aligned(16))) uint32_t hist[HB];  // the histograms; then the kept threads' sums and what precedes each
+  __shared__ __attribute__((aligned(16))) uint32_t ured[2][kSampWaves];
+  __shared__ float fred[kSampWaves];
   __shared__ uint32_t sel[4];
   const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const T* lr = logits + (size_t)m * ldl;
-  auto xkey = [&](int i) -> uint32_t { return Tr::key(lr, i, inv_t, temp); };
+  const int place = pos ? pos[m * pos_step] + 1 : 0;
+  // row m of the uniforms of this position (or of the only position without pos)
+  const float u = u_in ? u_in[(size_t)place * gridDim.x + m]
+                       : (float)(splitmix64(seed ^ ((uint64_t)place << 20) ^ (uint64_t)m) >> 40) * (1.0f / 16777216.0f);
   const int k = top_k < 1 || top_k > V ? V : top_k;
-  // ---- radix select: thr = the k-th largest key; keep key >= thr
-  uint32_t prefix = 0, want = (uint32_t)k;
-#pragma unroll
-  for (int pass = 0; pass < Tr::NP; ++pass) {
-    const int sh = Tr::SH[pass], nbins = 1 << Tr::W[pass];
-    for (int b = tid; b < HB; b += kSampNT) hist[b] = 0;
-    __syncthreads();
-    for (int i = tid; i < V; i += kSampNT) {
-      const uint32_t key = xkey(i);
-      if (pass == 0 || (key >> (sh + Tr::W[pass])) == prefix) atomicAdd(&hist[(key >> sh) & (nbins - 1)], 1u);
-    }
-    __syncthreads();
-    // thread t owns bins [b0, b0 + nb): counts above them by a suffix scan
-    const int nb = nbins >= kSampNT ? nbins / kSampNT : (tid < nbins ? 1 : 0);
-    const int b0 = nbins >= kSampNT ? nb * tid : tid;
-    uint32_t c = 0;
-    for (int q = 0; q < nb; ++q) c += hist[b0 + q];
-    const uint32_t above = block_suffix_excl(c, ured);
-    if (above < want && want <= above + c) {  // exactly one thread
-      uint32_t a = above;
-      int b = b0 + nb - 1;
-      for (; b > b0; --b) {
-        if (a + hist[b] >= want) break;
-        a += hist[b];
-      }
-      sel[0] = (uint32_t)b;
-      sel[1] = want - a;
-    }
-    __syncthreads();
-    prefix = pass == 0 ? sel[0] : (prefix << Tr::W[pass]) | sel[0];
-    want = sel[1];
-    __syncthreads();
-  }
-  const uint32_t thr = prefix;
-  // ---- max and sum of exp over the kept values (fp32, fixed reduction order)
-  uint32_t kmax = 0;
-  for (int i = tid; i < V; i += kSampNT) kmax = max(kmax, xkey(i));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o, 64));
-  if (lane == 0) ured[wv] = kmax;
-  __syncthreads();
-  if (tid == 0) {
-    uint32_t mk = 0;
-    for (int w = 0; w < kSampNT / 64; ++w) mk = max(mk, ured[w]);
-    sel[2] = mk;
-  }
-  __syncthreads();
-  const float xmax = Tr::val(sel[2]);
   // each thread owns a contiguous index range (the CDF is taken in index order)
   const int per = (V + kSampNT - 1) / kSampNT;
-  const int i0 = tid * per, i1 = min(V, i0 + per);
-  float esum = 0.f;
-  for (int i = i0; i < i1; ++i) {
-    const uint32_t key = xkey(i);
-    if (key >= thr) esum += Tr::ex(Tr::val(key) - xmax);
+  const int i0 = min(V, tid * per), i1 = min(V, i0 + per);
+  Key* own = reinterpret_cast<Key*>(samp_row) + tid * stride;
+  auto key_at = [&](int i) -> uint32_t { return stride ? (uint32_t)own[i - i0] : Tr::key(lr[i], inv_t, temp); };
+
+  // ---- the keys, and this thread's largest (any partition of the row serves for that)
+  for (int b = tid; b < HB; b += kSampNT) hist[b] = 0;
+  uint32_t tmax = 0;
+  constexpr int E = 16 / sizeof(T);
+  auto piece = [&](const uint4 w, Key (&ks)[E]) {
+    const T* x = reinterpret_cast<const T*>(&w);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const uint32_t key = Tr::key(x[e], inv_t, temp);
+      tmax = max(tmax, key);
+      ks[e] = (Key)key;
+    }
+  };
+  const bool ranges = stride > per;
+  const int nv = ((uintptr_t)lr & 15) ? 0 : ranges ? (i1 - i0) / E : V / E;
+  const uint4* src = reinterpret_cast<const uint4*>(ranges ? lr + i0 : lr);
+#pragma unroll 4
+  for (int v = ranges ? 0 : tid; v < nv; v += ranges ? 1 : kSampNT) {
+    Key ks[E];
+    piece(src[v], ks);
+    if (ranges) {  // (rows of an odd number of words: 4-byte places)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) reinterpret_cast<uint32_t*>(own + v * E)[e] = reinterpret_cast<const uint32_t*>(ks)[e];
+    } else if (stride) {  // ranges follow each other
+      reinterpret_cast<uint4*>(samp_row)[v] = *reinterpret_cast<const uint4*>(ks);
+    }
   }
+  for (int i = ranges ? i0 + nv * E : nv * E + tid; i < (ranges ? i1 : V); i += ranges ? 1 : kSampNT) {
+    const uint32_t key = Tr::key(lr[i], inv_t, temp);
+    tmax = max(tmax, key);
+    if (ranges) own[i - i0] = (Key)key;
+    else if (stride) reinterpret_cast<Key*>(samp_row)[i] = (Key)key;
+  }
+  const uint32_t wmax = wave_prefix<1>(tmax);
+  if (lane == 63) ured[0][wv] = wmax;
+  __syncthreads();
+  uint32_t each_wave[kSampWaves], kmax = 0;
+  per_wave(ured[0], each_wave);
+#pragma unroll
+  for (int w = 0; w < kSampWaves; ++w) kmax = max(kmax, each_wave[w]);
+  const float xmax = Tr::val(kmax);
+
+  // ---- the bin of the want-th largest key counted in hist (nbins bins), and the rank within it: sel[0], sel[1]. hist is left
+  // cleared: the next pass may count after it.
+  auto find = [&](int nbins, uint32_t want) {
+    __syncthreads();
+    // thread t owns bins [b0, b0 + nb), nb <= 2: counts above them by a suffix sum
+    const int nb = nbins > kSampNT ? 2 : (tid < nbins ? 1 : 0), b0 = nb * tid;
+    const uint32_t h0 = nb ? hist[b0] : 0, h1 = nb == 2 ? hist[b0 + 1] : 0, c = h0 + h1;
+    if (nb) hist[b0] = 0;
+    if (nb == 2) hist[b0 + 1] = 0;
+    const uint32_t incl = wave_prefix<0>(c);
+    if (lane == 63) ured[1][wv] = incl;
+    __syncthreads();
+    per_wave(ured[1], each_wave);
+    uint32_t above = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63) - incl;
+#pragma unroll
+    for (int w = 0; w < kSampWaves; ++w) above += w > wv ? each_wave[w] : 0;
+    if (above < want && want <= above + c) {  // exactly one thread
+      const bool upper = nb == 2 && above + h1 >= want;
+      sel[0] = (uint32_t)(upper ? b0 + 1 : b0);
+      sel[1] = want - (nb == 2 && !upper ? above + h1 : above);
+    }
+    __syncthreads();
+  };
+  uint32_t low = 0;  // no candidate lies below
+  const bool few = k < V && k <= kSampNT;
+  if (few) {
+    atomicAdd(&hist[tmax >> Tr::SH[0]], 1u);
+    find(1 << Tr::W[0], (uint32_t)k);
+    low = sel[0] << Tr::SH[0];
+  }
+  // ---- candidates: bit e of the mask stands for 1 << qs elements of this thread's range
+  int qs = 0;
+  while ((per - 1) >> qs > 63) ++qs;
+  uint64_t mask = 0;
+  if (few && ranges && qs == 0 && sizeof(Key) == 2) {  // two keys per word: the upper decides a comparison of whole words
+    if (tmax >= low) {
+      const uint32_t* pairs = reinterpret_cast<const uint32_t*>(own);
+      const uint32_t bar = low << 16;
+      uint32_t half[2] = {0, 0};
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll 8
+        for (int i = 16 * h; i < min(per / 2, 16 * h + 16); ++i) {
+          const uint32_t w = pairs[i], two = ((w << 16) >= bar ? 1u : 0u) | (w >= bar ? 2u : 0u);
+          half[h] |= two << (2 * (i & 15));
+        }
+      mask = ((uint64_t)half[1] << 32) | half[0];
+      if (i1 - i0 < 64) mask &= (1ull << (i1 - i0)) - 1;
+    }
+  } else if (few && !(ranges && tmax < low)) {
+    uint32_t half[2] = {0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll 8
+      for (int i = i0 + (h << (5 + qs)); i < min(i1, i0 + (32 << qs) + (h << (5 + qs))); ++i)
+        half[h] |= (key_at(i) >= low ? 1u : 0u) << (((i - i0) >> qs) & 31);
+    mask = ((uint64_t)half[1] << 32) | half[0];
+  }
+  auto each = [&](auto&& f) {  // f(index, key) over the candidates in index order, until it returns false
+    if (!few) {
+      for (int i = i0; i < i1; ++i)
+        if (!f(i, key_at(i))) return;
+      return;
+    }
+    for (uint64_t b = mask; b; b &= b - 1) {
+      const int s0 = i0 + ((int)__builtin_ctzll(b) << qs), s1 = min(i1, s0 + (1 << qs));
+      for (int i = s0; i < s1; ++i) {
+        const uint32_t key = key_at(i);
+        if (key >= low && !f(i, key)) return;
+      }
+    }
+  };
+  // ---- radix select among them: thr = the k-th largest key; keep key >= thr
+  uint32_t thr = 0;
+  if (k < V) {
+    uint32_t prefix = 0, want = (uint32_t)k;
+#pragma unroll
+    for (int pass = 0; pass < Tr::NP; ++pass) {
+      const int sh = Tr::SH[pass], nbins = 1 << Tr::W[pass];
+      auto count = [&](int, uint32_t key) {
+        if (pass == 0 || (key >> (sh + Tr::W[pass])) == prefix) atomicAdd(&hist[(key >> sh) & (nbins - 1)], 1u);
+        return true;
+      };
+      if (few || stride) each(count);
+      else
+        for (int i = tid; i < V; i += kSampNT) count(i, key_at(i));
+      find(nbins, want);
+      prefix = pass == 0 ? sel[0] : (prefix << Tr::W[pass]) | sel[0];
+      want = sel[1];
+    }
+    thr = prefix;
+  }
+  // ---- sum of exp over the kept values (fp32, fixed reduction order)
+  float esum = 0.f;
+  each([&](int, uint32_t key) {
+    if (key >= thr) esum += Tr::ex(Tr::val(key) - xmax);
+    return true;
+  });
   float t = wave_sum(esum);
   if (lane == 0) fred[wv] = t;
+  if (tid == 0) sel[2] = sel[3] = 0;
   __syncthreads();
   float tot = 0.f;
 #pragma unroll
-  for (int w = 0; w < kSampNT / 64; ++w) tot += fred[w];
+  for (int w = 0; w < kSampWaves; ++w) tot += fred[w];
   const float rinv = 1.f / tot;
-  // probabilities, chunk sums, exclusive scan over the chunks (thread order = index order)
+  // probabilities, the threads' sums, exclusive scan over the threads that have one (thread order = index order)
   float csum = 0.f;
-  for (int i = i0; i < i1; ++i) {
-    const uint32_t key = xkey(i);
-    if (key >= thr) csum += Tr::prob(Tr::ex(Tr::val(key) - xmax) * rinv);
-  }
-  chunk_excl[tid] = csum;
-  __syncthreads();
-  if (tid == 0) {  // sequential scan of 1024 chunk sums: deterministic
-    float run = 0.f;
-    for (int c = 0; c < kSampNT; ++c) {
-      const float v = chunk_excl[c];
-      chunk_excl[c] = run;
-      run += v;
-    }
-    float u;
-    if (u_in) {  // row m of the uniforms of this position (or of the only position without pos)
-      u = u_in[(size_t)(pos ? pos[m * pos_step] + 1 : 0) * gridDim.x + m];
-    } else {
-      const uint64_t h = splitmix64(seed ^ ((uint64_t)(pos ? pos[m * pos_step] + 1 : 0) << 20) ^ (uint64_t)m);
-      u = (float)(h >> 40) * (1.0f / 16777216.0f);
-    }
-    fred[0] = u * run;
-    sel[3] = 0xFFFFFFFFu;
-  }
-  __syncthreads();
-  const float target = fred[0];
-  const float base = chunk_excl[tid];
-  const float next = tid + 1 < kSampNT ? chunk_excl[tid + 1] : 3.4e38f;
-  if (i0 < i1 && base <= target && target < next) {
-    float run = base;
-    int pick = -1, last = -1;
-    for (int i = i0; i < i1; ++i) {
-      const uint32_t key = xkey(i);
-      if (key < thr) continue;
+  int last = -1;
+  each([&](int i, uint32_t key) {
+    if (key >= thr) {
+      csum += Tr::prob(Tr::ex(Tr::val(key) - xmax) * rinv);
       last = i;
-      run += Tr::prob(Tr::ex(Tr::val(key) - xmax) * rinv);
-      if (run > target) { pick = i; break; }
     }
-    if (pick < 0) pick = last;
-    if (pick >= 0) atomicMin(&sel[3], (uint32_t)pick);
+    return true;
+  });
+  if (last >= 0) atomicMax(&sel[2], (uint32_t)last);
+  const bool some = csum != 0.f;  // (NaN too)
+  const unsigned long long bal = __ballot(some);
+  if (lane == 0) ured[0][wv] = (uint32_t)__popcll(bal);
+  __syncthreads();
+  per_wave(ured[0], each_wave);
+  int at = __popcll(bal & ((1ull << lane) - 1ull)), n = 0;
+#pragma unroll
+  for (int w = 0; w < kSampWaves; ++w) {
+    at += w < wv ? (int)each_wave[w] : 0;
+    n += (int)each_wave[w];
+  }
+  float* sums = reinterpret_cast<float*>(hist);
+  float* excl = sums + kSampNT;
+  if (some) sums[at] = csum;
+  __syncthreads();
+  if (wv == 0) {  // one chain of additions: after step j the lanes up to j hold their sum, each its neighbour's plus its own
+    float run = 0.f;
+    for (int j = 0; j < n; j += 64) {
+      const float c = j + lane < n ? sums[j + lane] : 0.f, carry = run;
+      float before = carry;
+#pragma unroll 8
+      for (int e = 0; e < 64; ++e) {
+        before = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(carry), __float_as_int(run), 0x138, 0xf, 0xf, false));
+        run = before + c;
+      }
+      excl[j + lane] = before;
+      run = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(run), 63));
+    }
+    if (lane == 0) fred[0] = run;
+  }
+  __syncthreads();
+  const float run = fred[0], target = u * run;
+  if (some) {
+    const float base = excl[at], next = at + 1 < n ? excl[at + 1] : run;
+    if (base <= target && target < next) {  // one thread at most
+      float r = base;
+      int pick = last;
+      each([&](int i, uint32_t key) {
+        if (key < thr) return true;
+        r += Tr::prob(Tr::ex(Tr::val(key) - xmax) * rinv);
+        if (r > target) pick = i;
+        return !(r > target);
+      });
+      sel[3] = (uint32_t)pick + 1;
+    }
   }
   __syncthreads();
   if (tid == 0) {
-    uint32_t pick = sel[3];
-    if (pick == 0xFFFFFFFFu) {  // u * sum at the very end (rounding): the last kept index
-      for (int i = V - 1; i >= 0; --i)
-        if (xkey(i) >= thr) { pick = (uint32_t)i; break; }
-    }
-    out_idx[m] = (int)pick;
-    if (tokens_out) tokens_out[(size_t)m * tok_stride + pos[m * pos_step] + 1] = (int)pick;
+    const int pick = sel[3] ? (int)sel[3] - 1 : (int)sel[2];  // u * sum at the very end (rounding): the last kept index
+    out_idx[m] = pick;
+    if (tokens_out) tokens_out[(size_t)m * tok_stride + place] = pick;
   }
+}
+
+template <typename T>
+static int sample_launch(const T* logits, int ldl, int M, int V, float temperature, int top_k, const float* u, uint64_t seed,
+                         int* out_idx, int* tokens_out, int tok_stride, const int* pos, int pos_step, hipStream_t s) {
+  constexpr int KB = sizeof(typename SampTraits<T>::Key), E = 16 / sizeof(T);
+  const int per = (V + kSampNT - 1) / kSampNT;
+  // ranges of whole 16-byte pieces lie an even number of words apart: one more word between them
+  int stride = per % E == 0 && ((uintptr_t)logits & 15) == 0 && ldl % E == 0 ? per + 4 / KB : per;
+  if ((size_t)stride * kSampNT * KB > kSampRow) stride = 0;
+  static const hipError_t set =
+      hipFuncSetAttribute((const void*)sample_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSampRow);
+  if (set != hipSuccess) return -(int)set;
+  hipLaunchKernelGGL(sample_kernel<T>, dim3(M), dim3(kSampNT), (size_t)stride * kSampNT * KB, s, logits, ldl, V, 1.f / temperature,
+                     temperature, top_k, u, seed, out_idx, tokens_out, tok_stride, pos, pos_step, stride);
+  LLJ_CHECK_LAUNCH();
+  return 0;
 }
 
 // Streaming read of n16 16-byte words (the achievable HBM read rate the decode kernels are priced
@@ -597,19 +745,15 @@ int llj_attention_i8(const void* q, const void* kcache, const void* vcache, void
 int llj_sample(const void* logits, int ldl, int M, int V, float temperature, int top_k, const float* u,
                unsigned long long seed, int* out_idx, int* tokens_out, int tok_stride, const int* pos, void* stream) {
   LLJ_REQUIRE(M > 0 && V > 0 && temperature > 0.f && (!tokens_out || pos) && (u || pos));
-  hipLaunchKernelGGL(sample_kernel<bf16_t>, dim3(M), dim3(kSampNT), 0, (hipStream_t)stream, (const bf16_t*)logits, ldl,
-                     V, 1.f / temperature, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride, pos, 0);
-  LLJ_CHECK_LAUNCH();
-  return 0;
+  return sample_launch((const bf16_t*)logits, ldl, M, V, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride, pos,
+                       0, (hipStream_t)stream);
 }
 
 int llj_g_sample(const float* logits, int ldl, int M, int V, float temperature, int top_k, const float* u,
                  unsigned long long seed, int* out_idx, int* tokens_out, int tok_stride, const int* pos, void* stream) {
   LLJ_REQUIRE(logits && out_idx && M > 0 && V > 0 && ldl >= V && temperature > 0.f && (!tokens_out || pos) && (u || pos));
-  hipLaunchKernelGGL(sample_kernel<float>, dim3(M), dim3(kSampNT), 0, (hipStream_t)stream, logits, ldl, V,
-                     1.f / temperature, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride, pos, 0);
-  LLJ_CHECK_LAUNCH();
-  return 0;
+  return sample_launch(logits, ldl, M, V, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride, pos, 0,
+                       (hipStream_t)stream);
 }
 
 int llj_argmax(const void* logits, int ldl, int M, int V, int* out_idx, int* tokens_out, int tok_stride,
@@ -641,13 +785,12 @@ int llj_next_token(const void* logits, int ldl, int M, int V, float temperature,
                                   tokens_out, tok_stride, pos, pos_step),
            hipLaunchKernelGGL(argmax_kernel<float>, dim3(M), dim3(1024), 0, s, (const float*)logits, ldl, V, out_idx,
                               tokens_out, tok_stride, pos, pos_step));
+  } else if (dt == 0) {
+    return sample_launch((const bf16_t*)logits, ldl, M, V, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride,
+                         pos, pos_step, s);
   } else {
-    LLJ_DT(dt, hipLaunchKernelGGL(sample_kernel<bf16_t>, dim3(M), dim3(kSampNT), 0, s, (const bf16_t*)logits, ldl, V,
-                                  1.f / temperature, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride,
-                                  pos, pos_step),
-           hipLaunchKernelGGL(sample_kernel<float>, dim3(M), dim3(kSampNT), 0, s, (const float*)logits, ldl, V,
-                              1.f / temperature, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride, pos,
-                              pos_step));
+    return sample_launch((const float*)logits, ldl, M, V, temperature, top_k, u, (uint64_t)seed, out_idx, tokens_out, tok_stride,
+                         pos, pos_step, s);
   }
   LLJ_CHECK_LAUNCH();
   return 0;

@@ -1096,6 +1096,44 @@ def test_sample_inverse_cdf_vs_oracle(hip, temperature, top_k):
         assert mism <= 2, mism
 
 
+@pytest.mark.parametrize("V", [2, 63, 1024, 1025, 8192, 32000, 35008, 36865, 73728, 73729, 100278])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sample_forms(hip, dtype, V):
+    """The sampler over its forms: rows kept in LDS in 16-byte pieces, in single values (odd ranges, unaligned rows) and not at
+    all; the threshold from the threads' maxima (top_k <= 1024) and from the whole row; ties, infinities, the ends of u.
+    The drawn index is kept and lies where u falls in the kept probabilities' running sum, up to the rounding of that sum:
+    each bf16 probability may round the other way (2^-8 of it); fp32: 2^-21 for exp and one rounding per addition, of which a
+    value passes at most V / 1024 in its thread and 1024 over the threads."""
+    gen = torch.Generator(device=dev).manual_seed(V)
+    M, temp = 12, 0.8
+    slack = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-20 + (V / 1024 + 1024) * 2.0**-24
+    for top_k in (2, 200, 1024, 1025, V - 1, 0):
+        for ldl in (V + -V % 8, V + 1):
+            k = V if top_k < 1 or top_k > V else top_k
+            L = torch.randn(M, ldl, device=dev, generator=gen) * 3
+            L[1] = (L[1] * 2).round() / 2  # ties
+            L[2, : V // 2] = -float("inf")
+            L[3] = 0.25
+            L = L.to(dtype)
+            u = torch.rand(M, device=dev, generator=gen)
+            u[4], u[5] = 0.0, 1 - 2.0**-24
+            out = torch.full((M,), -1, dtype=torch.int32, device=dev)
+            call(hip, "llj_sample" if dtype == torch.bfloat16 else "llj_g_sample", L.data_ptr(), ldl, M, V, temp, top_k, u.data_ptr(),
+                 0, out.data_ptr(), None, 0, None, st())
+            torch.cuda.synchronize()
+            got = out.long()
+            assert int(got.min()) >= 0 and int(got.max()) < V
+            x = (L[:, :V].float() * (1 / temp)).to(dtype).float() if dtype == torch.bfloat16 else L[:, :V] / temp
+            kept = x >= torch.topk(x, k, dim=1).values[:, -1:]
+            assert bool(kept.gather(1, got[:, None]).all())
+            p = torch.softmax(torch.where(kept, x, torch.full_like(x, -float("inf"))), 1)
+            p = (p.to(dtype).double() * kept) if dtype == torch.bfloat16 else p.double()
+            cdf = p.cumsum(1)
+            at, total = cdf.gather(1, got[:, None])[:, 0], cdf[:, -1]
+            target, tol = u.double() * total, slack * total
+            assert bool((target <= at + tol).all()) and bool((target >= at - p.gather(1, got[:, None])[:, 0] - tol).all()), (top_k, ldl)
+
+
 def test_sample_device_rng_distribution(hip):
     """The in-graph path (u from the counter hash of seed, position and row): 8192 rows of the same
     logits draw from the top_k = 8 softmax with the oracle's probabilities (4-sigma bound per
