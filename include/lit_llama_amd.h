@@ -154,6 +154,12 @@ int llj_attention_part(const void* q, const void* kcache, const void* vcache, co
                        int n_head, int head_size, int S, int nsplit, void* part_ws, void* stream);
 int llj_attention_split(const void* q, const void* kcache, const void* vcache, void* y, const int* pos, int B, int T,
                         int n_head, int head_size, int S, int nsplit, void* part_ws, void* stream);
+/* llj_attention_split with nsplit <= 64 in one launch: the last of a (row, head)'s blocks merges its partials. count: one int
+ * per (row, head), zero before the first call; every call leaves them zero. With y_stats (LLM.int8, B * T <= 8 rows) also y's
+ * statistics, and clr_words words at clr zeroed (llj_attention_i8). */
+int llj_attention_ranges(const void* q, const void* kcache, const void* vcache, void* y, const int* pos, int B, int T,
+                         int n_head, int head_size, int S, int nsplit, void* part_ws, int* count, void* y_stats, void* clr,
+                         int clr_words, float threshold, void* stream);
 
 /* x[M, N] += A[M, K] . W^T (attn.c_proj / mlp.c_proj + residual add, model.py:172-173).
  * nstat_out (optional, M <= 16, not int8): per 16-column tile t of the new x, the bf16-rounded

@@ -61,6 +61,19 @@ __device__ __forceinline__ void softmax_merge(float& mx, float& l, float* o, con
 template <int HS>
 constexpr int kAttPart = HS + 4;  // floats per partial record: HS outputs, max, sum, 2 pad (16-byte records)
 
+// count (with PART, else partials only; nsplit <= 64): zeroed arrival counters, one per (row, head), left zero: the last of the
+// ranges' blocks to finish merges them. The hand-off is device-scope stores, a wait for them, the counter, device-scope
+// loads; no block waits for another.
+
+// y[m, h * HS + d] of thread d < HS, adjacent dims as one 4-byte store; with st the LLM.int8 statistics of y, one slot per head
+template <int HS>
+__device__ __forceinline__ void attention_out(float v, bf16_t* __restrict__ y, uint32_t* st, float thr, int h, int m, int C) {
+  const int d = threadIdx.x;
+  const uint32_t ob = (uint32_t)f2bf(v), pr = lane_xor1(ob);
+  if (!(d & 1)) st_out32(y + (size_t)m * C + h * HS + d, ob | (pr << 16));
+  if (st) i8_emit_stats64(st, thr, m, h * HS + (d & ~63), ob, h);  // (uniform)
+}
+
 template <int HS, int U, int NTH, bool PART = false, int SPECU = U / 2, bool ILV = false>
 __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                const bf16_t* __restrict__ vc, bf16_t* __restrict__ y,
@@ -69,7 +82,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
                                                int split = 0, float* __restrict__ part = nullptr,
                                                uint32_t* __restrict__ st = nullptr, float thr = 0.f,
                                                uint32_t* __restrict__ clr = nullptr, int clr_words = 0,
-                                               bool spec_ok = false) {
+                                               bool spec_ok = false, int* __restrict__ count = nullptr) {
   constexpr int DPL = HS / 16;
   constexpr int NG = NTH / 16;
   constexpr int NWV = NTH / 64;
@@ -218,23 +231,60 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
     }
     if constexpr (PART) {  // unnormalized partial: outputs, then (max, sum)
       float* dst = part + ((size_t)(m * nh + h) * nsplit + split) * kAttPart<HS>;
-      dst[d] = O;
-      if (d == 0) {
-        dst[HS] = M;
-        dst[HS + 1] = L;
+      if (count) {
+        const float O1 = lane_xor1(O);
+        if (!(d & 1)) put2(dst + d, O, O1);
+        if (d == 0) put2(dst + HS, M, L);
+      } else {
+        dst[d] = O;
+        if (d == 0) {
+          dst[HS] = M;
+          dst[HS + 1] = L;
+        }
       }
       LLJ_STAMP(5);
-      return;
+    } else {
+      attention_out<HS>(O / L, y, st, thr, h, m, C);
     }
-    const uint32_t ob = (uint32_t)f2bf(O / L);
-    const uint32_t pr = lane_xor1(ob);
-    if (!(d & 1)) {
-      const size_t eo = (size_t)m * C + h * HS + d;
-      st_out32(y + eo, ob | (pr << 16));
-    }
-    if (st) i8_emit_stats64(st, thr, m, h * HS + (d & ~63), ob, h);  // uniform; one SCA slot per head
   }
   LLJ_STAMP(5);
+  if constexpr (PART) {
+    if (!count) return;
+    // ---- the last of the ranges' blocks merges them: every range's pieces requested at once, added in range order
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials are out
+    __syncthreads();
+    int* last = reinterpret_cast<int*>(s_m);
+    if (threadIdx.x == 0) {
+      int* c = count + m * nh + h;
+      const int done = __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *last = done == nsplit - 1;
+      if (done == nsplit - 1) __hip_atomic_store(c, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!*last || threadIdx.x >= HS) return;
+    const int d = threadIdx.x, lane = d & 63;
+    const float* src = part + (size_t)(m * nh + h) * nsplit * kAttPart<HS>;
+    float O = 0.f;
+    constexpr int R = 16;
+    float pc[R];
+    auto pieces = [&](int s0) {  // (past the end: a copy, its weight is 0)
+#pragma unroll
+      for (int e = 0; e < R; ++e) pc[e] = get1(src + (size_t)min(s0 + e, nsplit - 1) * kAttPart<HS> + d);
+    };
+    pieces(0);
+    float2 ml = make_float2(-INFINITY, 0.f);  // lane s: range s (nsplit <= 64)
+    if (lane < nsplit) ml = get2(src + (size_t)lane * kAttPart<HS> + HS);
+    const float M = wave_max(ml.x);  // (in every lane: not inside the selection)
+    const float w = ml.x == -INFINITY ? 0.f : exp2f(ml.x - M);
+    const float L = wave_sum(w * ml.y);
+    for (int s0 = 0; s0 < nsplit; s0 += R) {
+      if (s0) pieces(s0);
+#pragma unroll
+      for (int e = 0; e < R; ++e)  // (s0 + e < 64; ranges past nsplit weigh 0)
+        O += pc[e] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s0 + e));
+    }
+    attention_out<HS>(O / L, y, st, thr, h, m, C);
+  }
 }
 
 // Merge the nsplit partials of one (head, row) in split order: y = sum_s O_s f_s / sum_s L_s f_s

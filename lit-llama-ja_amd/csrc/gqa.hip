@@ -37,16 +37,6 @@ struct GqaParams {
   float scale;
 };
 
-// device-scope accesses of the decode hand-off, two floats each
-__device__ __forceinline__ void put2(float* p, float a, float b) {
-  const unsigned long long v = (unsigned long long)__float_as_uint(a) | ((unsigned long long)__float_as_uint(b) << 32);
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float2 get2(const float* p) {
-  const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
-}
-
 __device__ __forceinline__ void turn_cs(const double* __restrict__ turns, int i, int pos, float& c, float& s) {
   const double t = (double)pos * turns[i];
   sincospif(2.f * (float)(t - rint(t)), &s, &c);

@@ -141,6 +141,23 @@ __global__ __launch_bounds__(NTH) void attention_part_kernel(const bf16_t* __res
                                    blockIdx.z, part);
 }
 
+// interleaved key ranges merged by the last block of each (row, head): one launch. Against the two launches (contiguous ranges
+// of 256 keys, then the merge), us in a graph, hs 128: 32 heads, 1010 of 1033 keys 10.1 -> 8.6; 2000 of 2048 15.5 -> 11.9; 40 heads,
+// 1400 keys 13.5 -> 10.6; 8 rows, 900 keys 27.8 -> 25.9. Contiguous ranges, merged the same way: 8.9, 11.9, 11.1, 27.1; interleaved
+// ranges of 128 keys: 8.7, 12.0, 10.9, 27.5; half a pass loaded before the position is known: 8.7, 12.1, 10.7, 25.3 but 6.8
+// against 5.7 where 100 of 2048 slots are in use.
+template <int HS, int U, int NTH>
+__global__ __launch_bounds__(NTH) void attention_ranges_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
+                                                               const bf16_t* __restrict__ vc, bf16_t* __restrict__ y,
+                                                               const int* __restrict__ pos, int T, int S, int nh,
+                                                               float scale_log2, int nsplit, float* __restrict__ part,
+                                                               int* __restrict__ count, uint32_t* st, float thr,
+                                                               uint32_t* clr, int clr_words) {
+  __shared__ float lds[attention_lds_floats<HS, NTH>()];
+  attention_body<HS, U, NTH, true, U / 2, true>(q, kc, vc, y, pos, T, S, nh, scale_log2, blockIdx.x, blockIdx.y, lds, nsplit,
+                                                blockIdx.z, part, st, thr, clr, clr_words, false, count);
+}
+
 // interleaved key splits of a short cache (attention.h ILV), partials merged by the consumer
 template <int HS, int U, int NTH, int SPECU>
 __global__ __launch_bounds__(NTH) void attention_ilv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
@@ -705,6 +722,25 @@ int llj_attention_split(const void* q, const void* kcache, const void* vcache, v
                         int n_head, int head_size, int S, int nsplit, void* part_ws, void* stream) {
   return attention_split_run(q, kcache, vcache, y, pos, B, T, n_head, head_size, S, nsplit, part_ws, nullptr, 0.f,
                              nullptr, 0, stream);
+}
+
+int llj_attention_ranges(const void* q, const void* kcache, const void* vcache, void* y, const int* pos, int B, int T,
+                         int n_head, int head_size, int S, int nsplit, void* part_ws, int* count, void* y_stats, void* clr,
+                         int clr_words, float threshold, void* stream) {
+  LLJ_REQUIRE(q && kcache && vcache && y && pos && B > 0 && T > 0 && n_head > 0 && S > 0 && nsplit >= 1 && nsplit <= 64 && part_ws &&
+              ((uintptr_t)part_ws & 7) == 0 && count && (!y_stats || B * T <= 8) && clr_words >= 0 && (!clr_words || clr));
+  const float sl2 = 1.4426950408889634f / sqrtf((float)head_size);
+  const dim3 grid(n_head, B * T, nsplit);
+#define LLJ_ATT_RANGES(HS_)                                                                                              \
+  hipLaunchKernelGGL((attention_ranges_kernel<HS_, LLJ_ATT_U, LLJ_ATT_NTH>), grid, dim3(LLJ_ATT_NTH), 0, (hipStream_t)stream, \
+                     (const bf16_t*)q, (const bf16_t*)kcache, (const bf16_t*)vcache, (bf16_t*)y, pos, T, S, n_head, sl2, nsplit, \
+                     (float*)part_ws, count, (uint32_t*)y_stats, threshold, (uint32_t*)clr, clr_words)
+  if (head_size == 128) LLJ_ATT_RANGES(128);
+  else if (head_size == 64) LLJ_ATT_RANGES(64);
+  else return LLJ_EINVAL;
+#undef LLJ_ATT_RANGES
+  LLJ_CHECK_LAUNCH();
+  return 0;
 }
 
 // Decode attention (one-block or split over nsplit key ranges) that also writes the LLM.int8

@@ -96,10 +96,10 @@ LIN_ROWS = 16   # plain linear kernels take <= 16 rows per launch
 I8_ROWS = 8     # int8 kernels quantize <= 8 rows in LDS
 if os.environ.get("LLJ_I8_ROWS"):  # profiling only: smaller int8 row slices (A images under 64 KiB of LDS)
     I8_ROWS = max(1, min(8, int(os.environ["LLJ_I8_ROWS"])))
-# long caches: attention split over the keys (llj_attention_split) into ATTN_SPLIT_KEYS-key
-# ranges once the cache holds >= ATTN_SPLIT_MIN_S slots (32 heads x 1 row leave most CUs idle)
+# long caches: attention split over the keys (llj_attention_ranges) into ranges of ATTN_SPLIT_KEYS
+# keys once the cache holds >= ATTN_SPLIT_MIN_S slots (32 heads x 1 row leave most CUs idle)
 ATTN_SPLIT_MIN_S = 512
-ATTN_SPLIT_KEYS = 256  # 7B bs=1 at p = 2000 (S = 2048): 33.1 us one block, 14.4 us in 8 ranges
+ATTN_SPLIT_KEYS = 256  # 7B bs=1 at p = 2000 (S = 2048): 33.1 us one block, 11.9 us in 8 ranges
 
 
 # prompts of at least this many tokens run the MFMA flash attention (llj_attention_prefill) when
@@ -290,12 +290,13 @@ class _Work:
             self.h_st = torch.zeros(L.llj_i8_rowstats_bytes(H) // 4, dtype=torch.int32, device=device)
             # the norm outputs' block (rms_1 / rms_2 / ln_f), rewritten whole by llj_i8_norm_rowstats
             self.n_st = torch.zeros(L.llj_i8_rowstats_bytes(C) // 4, dtype=torch.int32, device=device)
-        # split-K attention partials for long caches (llj_attention_split)
+        # attention over key ranges for long caches (llj_attention_ranges): partials, arrival counters (zero between launches)
         self.nsplit = attn_splits(S)
-        self.att_ws = None
+        self.att_ws = self.att_count = None
         if self.nsplit > 1:
             nb = _hip.lib().llj_attention_ws_bytes(M, cfg.n_head, C // cfg.n_head, self.nsplit)
             self.att_ws = torch.empty(nb, dtype=torch.uint8, device=device)
+            self.att_count = torch.zeros(M * cfg.n_head, dtype=torch.int32, device=device)
         # one decode row, short cache: interleaved split partials merged in attn.c_proj (ATT_MERGE)
         self.att_merge = ATT_MERGE if (ATT_MERGE > 1 and M == 1 and self.nsplit <= 1 and not need_i8) else 0
         self.att_part = None
@@ -540,8 +541,8 @@ class LLaMA(nn.Module):
             _hip.call("llj_attention_prefill", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(),
                       pos.data_ptr(), B, T, nh, C // nh, S, st)
         elif w.att_ws is not None:
-            _hip.call("llj_attention_split", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(),
-                      pos.data_ptr(), B, T, nh, C // nh, S, w.nsplit, w.att_ws.data_ptr(), st)
+            _hip.call("llj_attention_ranges", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(), B, T, nh,
+                      C // nh, S, w.nsplit, w.att_ws.data_ptr(), w.att_count.data_ptr(), None, None, 0, 0.0, st)
         else:
             _hip.call("llj_attention", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(),
                       pos.data_ptr(), B, T, nh, C // nh, S, st)
@@ -728,9 +729,14 @@ class LLaMA(nn.Module):
                           S, r0, r, P(w.i8ws), P(rs), P(nst), w.npart, st)
             # 2. attention, 3. c_proj + residual
             if w.i8s and not w.flash:  # y's LLM.int8 statistics from the attention (clears h's block)
-                _hip.call("llj_attention_i8", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(),
-                          B, T, nh, C // nh, S, w.nsplit, P(w.att_ws), w.y_st.data_ptr(), w.h_st.data_ptr(),
-                          w.h_st.numel(), Linear8bitLtThreshold, st)
+                if w.att_ws is not None:
+                    _hip.call("llj_attention_ranges", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(),
+                              B, T, nh, C // nh, S, w.nsplit, w.att_ws.data_ptr(), w.att_count.data_ptr(), w.y_st.data_ptr(),
+                              w.h_st.data_ptr(), w.h_st.numel(), Linear8bitLtThreshold, st)
+                else:
+                    _hip.call("llj_attention_i8", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(),
+                              B, T, nh, C // nh, S, 1, None, w.y_st.data_ptr(), w.h_st.data_ptr(), w.h_st.numel(),
+                              Linear8bitLtThreshold, st)
                 _hip.call("llj_i8_linear_resid", w.y.data_ptr(), C, wp.data_ptr(), P(sp), w.x.data_ptr(), C, M, C, C,
                           w.y_st.data_ptr(), st)
             elif w.att_merge and not w.flash and fp in (0, 1, 3):  # split partials, merged by c_proj (A/B)

@@ -809,6 +809,39 @@ def test_attention_split_keys(hip, hs, nh, B, T_, S, p0, nsplit):
     assert_bf16_close(y.float().cpu().numpy(), _attn_oracle(q, kc, vc, pos, S, T_, nh, hs), "split attention")
 
 
+@pytest.mark.parametrize("hs,nh,B,T_,S,p0,nsplit", [(128, 4, 1, 1, 2048, 2000, 8), (128, 3, 2, 1, 2048, 40, 16), (64, 4, 2, 5, 600, 300, 3),
+                                                   (128, 2, 1, 1, 512, 900, 1), (128, 5, 8, 1, 1033, 1010, 5), (64, 2, 3, 1, 700, 0, 64)])
+def test_attention_ranges(hip, hs, nh, B, T_, S, p0, nsplit):
+    """Interleaved key ranges merged by the last block, against the oracle: few to 64 ranges (most of them empty), heads and ranges
+    that are no multiple of the chiplets, prompt rows, the rolled ring; partials of the last call or NaN in the scratch make no
+    difference and the counters end at zero. With statistics: those of llj_i8_stats on the same y, and the other block zeroed."""
+    rng = np.random.default_rng(hs + S + p0 + nsplit)
+    C, M = nh * hs, B * T_
+    kc = bf16(rng.standard_normal((B, nh, S, hs)))
+    vc = bf16(rng.standard_normal((B, nh, S, hs)))
+    vc[:, 0, :, 9] = 9.0  # (a column past the LLM.int8 threshold)
+    q = bf16(rng.standard_normal((M, C)) * 2)
+    pos = np.arange(p0, p0 + T_, dtype=np.int32)
+    qd, kd, vd, pd = T(q, torch.bfloat16), T(kc, torch.bfloat16), T(vc, torch.bfloat16), T(pos)
+    part = torch.full((hip.llj_attention_ws_bytes(M, nh, hs, nsplit),), 0xFF, dtype=torch.uint8, device=dev)
+    count = torch.zeros(M * nh, dtype=torch.int32, device=dev)
+    stats = M <= 8 and C % 128 == 0
+    y_st = torch.zeros(hip.llj_i8_rowstats_bytes(C) // 4, dtype=torch.int32, device=dev)
+    clr = torch.full((700,), 7, dtype=torch.int32, device=dev)
+    want = _attn_oracle(q, kc, vc, pos, S, T_, nh, hs)
+    for rep in range(3):
+        y = torch.full((M, C), float("nan"), dtype=torch.bfloat16, device=dev)
+        y_st.zero_()
+        call(hip, "llj_attention_ranges", qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), y.data_ptr(), pd.data_ptr(), B, T_, nh, hs, S,
+             nsplit, part.data_ptr(), count.data_ptr(), y_st.data_ptr() if stats else None, clr.data_ptr(), 700, 6.0, st())
+        torch.cuda.synchronize()
+        assert not count.any() and not clr.any()
+        assert_bf16_close(y.float().cpu().numpy(), want, "attention over ranges")
+    if stats:
+        for got, ref in zip(_st_decode(y_st, M, C), _i8_ws_stats(hip, y, M, C)):
+            np.testing.assert_array_equal(got, ref)
+
+
 def _i8_ws_stats(hip, A, M, K):
     """(SCA (M,), outlier flags (K,) bool) of llj_i8_stats's workspace for the rows A (M, K)."""
     from lit_llama import _hip
