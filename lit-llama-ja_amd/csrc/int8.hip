@@ -213,6 +213,10 @@ __device__ __forceinline__ uint2 quant8(uint4 x, uint2 fl, float inv) {
   return make_uint2(o[0], o[1]);
 }
 
+// bits of the smallest bf16 value >= thr (thr finite, positive)
+__device__ __forceinline__ uint32_t first_not_below(float thr) { return (__float_as_uint(thr) + 0xFFFFu) >> 16; }
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
 // The whole activation preparation in ONE launch for decode batches (M <= 8 rows): one 1024-thread
 // block per k-block (kNSB blocks). Every block reads all M rows (four 256-thread groups, group g
 // taking rows g and g + 4 with llj_rmsnorm's thread-to-vector map, so with norm_w the sums of
@@ -220,9 +224,9 @@ __device__ __forceinline__ uint2 quant8(uint4 x, uint2 fl, float inv) {
 // elements below the threshold itself (redundant across blocks, no grid-wide dependency); then it
 // finishes its own k-block: outlier flags, the list, part, the normalized rows (xn) and the
 // quantized rows (aq). Block 0 writes the header and SCA.
-#ifndef LLJ_PREP_ABL
-#define LLJ_PREP_ABL 0  // timing ablations only (results wrong): 1 no sums of squares, 2 no row maxima, 4 no row loads, 8 no list
-#endif
+// Bound by instructions and by the steps that follow each other: the 32 CUs each see all rows. 8 rows of 4096 with the norm,
+// us a launch: 7.5 -> 7.1 since the maxima are taken on pairs of bf16 bits, the rows' factors by every wave for itself and the
+// row loads issued ahead of the own item's place.
 template <bool NORM, int VPT>
 __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restrict__ x, int lda,
                                                            const bf16_t* __restrict__ w, float eps,
@@ -231,8 +235,7 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
                                                            uint32_t* __restrict__ st = nullptr) {
   constexpr int MR = 8;
   __shared__ int flag[1024];
-  __shared__ float red[MR][4];
-  __shared__ float rr[MR];
+  __shared__ __attribute__((aligned(16))) float red[MR][4];
   __shared__ float mred[16][MR];
   __shared__ int pmax[MR];
   __shared__ uint4 vals[MR][1024 / 8];  // the own k-block's (normalized) rows, for aval
@@ -242,12 +245,6 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
   const int nvec = K >> 3;
   const int k0 = b * kb, k1 = min(K, k0 + kb);
   const int vpr = k1 > k0 ? (k1 - k0) >> 3 : 0;
-  // own k-block item (row, vector), loaded first (M * vpr <= 1024 on this path)
-  const bool own = tid < M * vpr;
-  const int om = own ? tid / vpr : 0, ov = own ? (k0 >> 3) + tid % vpr : 0;
-  const uint4 oa = reinterpret_cast<const uint4*>(x + (size_t)om * lda)[ov];
-  uint4 og = oa;
-  if (NORM) og = reinterpret_cast<const uint4*>(w)[ov];
   // rows grp and grp + 4, vectors lt + 256 j (past the row: zeros, which add nothing to either pass)
   uint4 xa[2][VPT], ga[VPT];
 #pragma unroll
@@ -256,16 +253,23 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
     for (int j = 0; j < VPT; ++j) {
       const bool ok = lt + 256 * j < nvec;
       const int m = grp + 4 * r < M ? grp + 4 * r : M - 1, v = ok ? lt + 256 * j : nvec - 1;
-      const uint4 t = (LLJ_PREP_ABL & 4) ? oa : reinterpret_cast<const uint4*>(x + (size_t)m * lda)[v];
+      const uint4 t = reinterpret_cast<const uint4*>(x + (size_t)m * lda)[v];
       xa[r][j] = ok ? t : make_uint4(0u, 0u, 0u, 0u);
     }
   if (NORM) {
 #pragma unroll
     for (int j = 0; j < VPT; ++j) ga[j] = reinterpret_cast<const uint4*>(w)[lt + 256 * j < nvec ? lt + 256 * j : nvec - 1];
   }
+  // own k-block item (row, vector; M * vpr <= 1024 on this path): its place is computed over the loads above
+  const bool own = tid < M * vpr;
+  const int om = own ? tid / vpr : 0, ov = own ? (k0 >> 3) + tid % vpr : 0;
+  const uint4 oa = reinterpret_cast<const uint4*>(x + (size_t)om * lda)[ov];
+  uint4 og = oa;
+  if (NORM) og = reinterpret_cast<const uint4*>(w)[ov];
   for (int i = tid; i < kb; i += 1024) flag[i] = 0;
   if (tid < MR) pmax[tid] = 0;
-  if (NORM && !(LLJ_PREP_ABL & 1)) {
+  float rows = 1.f;
+  if (NORM) {
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
       float a = 0.f;
@@ -282,41 +286,43 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
       if (lane == 0) red[grp + 4 * r][gw] = a;
     }
     __syncthreads();
-    if (tid < MR) rr[tid] = round_bf(rsqrtf(round_bf(round_bf((red[tid][0] + red[tid][1] + red[tid][2] + red[tid][3]) / (float)K) + eps)));
-    __syncthreads();
+    // lane m & 7 of every wave: row m's factor (no second trip through LDS)
+    const f32x4 q = *reinterpret_cast<const f32x4*>(red[lane & 7]);
+    rows = round_bf(rsqrtf(round_bf(round_bf((q[0] + q[1] + q[2] + q[3]) / (float)K) + eps)));
   }
-  if ((LLJ_PREP_ABL & 1) && tid < MR) rr[tid] = 1.f;
-  if (LLJ_PREP_ABL & 1) __syncthreads();
   // each row's maximum of the (normalized) elements below the threshold. The elements are bf16
   // values, exact in fp16 wherever |v| >= 2^-14, and fp16 rounding is monotonic: for a threshold
   // >= 2^-14, max f16(|v|) over f16(|v|) < thr is f16(max |v| over |v| < thr) -- no per-element
-  // conversion (the i8_stats_kernel rule, bit for bit)
+  // conversion (the i8_stats_kernel rule, bit for bit). |v| orders as its bits, two values per word: minus the
+  // bits of the first bf16 value not below thr (>= 1), modulo 2^16, the values below it come last, in order.
+  const uint32_t tb = first_not_below(thr), tb2 = tb | (tb << 16);
 #pragma unroll
-  for (int r = 0; r < ((LLJ_PREP_ABL & 2) ? 0 : 2); ++r) {
-    const float rn = NORM ? rr[grp + 4 * r < M ? grp + 4 * r : M - 1] : 1.f;
+  for (int r = 0; r < 2; ++r) {
+    const float rn = NORM ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rows), uniform(grp + 4 * r))) : 1.f;
     const f32x2 rn2 = {rn, rn};
-    float mx = 0.f;
+    u16x2 mx = {0, 0};
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const uint32_t aw[4] = {xa[r][j].x, xa[r][j].y, xa[r][j].z, xa[r][j].w};
       const uint32_t gw4[4] = {ga[j].x, ga[j].y, ga[j].z, ga[j].w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        f32x2 v = unpk(aw[i]);
-        if (NORM) v = unpk(cvt_pk(unpk(gw4[i]) * unpk(cvt_pk(v * rn2))));  // g * bf16(x * r), rounded
-        const float a0 = fabsf(v.x), a1 = fabsf(v.y);
-        mx = fmaxf(mx, a0 < thr ? a0 : 0.f);
-        mx = fmaxf(mx, a1 < thr ? a1 : 0.f);
+        uint32_t v = aw[i];
+        if (NORM) v = cvt_pk(unpk(gw4[i]) * unpk(cvt_pk(unpk(v) * rn2)));  // g * bf16(x * r), rounded
+        const u16x2 a = __builtin_bit_cast(u16x2, v & 0x7fff7fffu) - __builtin_bit_cast(u16x2, tb2);
+        mx = __builtin_elementwise_max(mx, a);
       }
     }
-    mx = to_f16f(wave_max(mx));
-    if (lane == 0) mred[tid >> 6][r] = mx;  // wave (grp, gw): slot r <-> row grp + 4 r
+    const uint32_t top = max((uint32_t)mx[0], (uint32_t)mx[1]);
+    const float m = wave_max(top >= 0x10000u - tb ? __uint_as_float((top + tb) << 16) : 0.f);  // (top + tb - 2^16: bf16 bits)
+    if (lane == 0) mred[tid >> 6][r] = to_f16f(m);  // wave (grp, gw): slot r <-> row grp + 4 r
   }
   if (!NORM) __syncthreads();  // flag / pmax zeroed before any thread sets them (NORM: synced above)
   // own k-block: normalize, flags, per-row maximum
   uint4 on = oa;
+  const float orow = NORM ? __shfl(rows, om, 64) : 1.f;  // (in every lane)
   if (NORM && own) {
-    const float rn = rr[om];
+    const float rn = orow;
     on = make_uint4(norm_pair(oa.x, og.x, rn), norm_pair(oa.y, og.y, rn), norm_pair(oa.z, og.z, rn),
                     norm_pair(oa.w, og.w, rn));
   }
@@ -364,8 +370,7 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
       st[kI8StFlags + (k0 >> 5) + wd] = bits;
     }
   }
-  if ((LLJ_PREP_ABL & 8) && tid == 0) L.cnt[b] = 0;  // the ablation skips the list, never the count a consumer reads
-  if (tid < 64 && !(LLJ_PREP_ABL & 8)) {  // compact the flags into the list, 64 columns per ballot
+  if (tid < 64) {  // compact the flags into the list, 64 columns per ballot
     int c = 0;
     for (int i0 = 0; i0 < k1 - k0; i0 += 64) {
       const bool f = i0 + lane < k1 - k0 && flag[i0 + lane];
@@ -506,8 +511,11 @@ __device__ __forceinline__ int i8_flat_list(const I8Layout& L, const I8WsHeader&
   }
   __syncthreads();
   if (s_pre[nsb] > cap) return s_pre[nsb];  // over capacity: the caller gathers nothing
-  for (int b = 0; b < nsb; ++b)
-    for (int j = tid; j < s_pre[b + 1] - s_pre[b]; j += blockDim.x)
+  // a few threads per k-block, so that all k-blocks' entries are requested at once (k-block after k-block: a memory trip each;
+  // 128 rows of 4096 or 11008, i8_gather_act_kernel 9.2 -> 5.4 us a launch)
+  const int tpb = blockDim.x / kNSB, b = tid / tpb;
+  if (b < nsb)
+    for (int j = tid % tpb; j < s_pre[b + 1] - s_pre[b]; j += tpb)
       s_list[s_pre[b] + j] = i8_col_clamp(L.list[b * h.kb + j], h.K);
   __syncthreads();
   return s_pre[nsb];
