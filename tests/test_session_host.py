@@ -43,22 +43,45 @@ def test_session_is_freed_without_the_collector(program, monkeypatch):
 
 
 def test_dropped_graphs_wait_for_the_next_capture(monkeypatch):
-    """A session's graph outlives it until the next capture, and at most two are kept."""
+    """A session's graph outlives it until a capture has ended -- freeing one inside a capture aborts -- and at most two are kept;
+    every few captures the allocator gives back what the freed graphs' steps had allocated. A step that raises ends its capture."""
+    import contextlib
+
     from lit_llama import engine
 
+    log = []
+
     class Graph:
-        pass
+        def capture_begin(self):
+            log.append("begin")
+
+        def capture_end(self):
+            log.append("end")
 
     monkeypatch.setattr(engine, "_retired", type(engine._retired)(maxlen=2))
-    refs = []
+    monkeypatch.setattr(engine, "_captures", engine.itertools.count(1))
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", Graph)
+    monkeypatch.setattr(torch.cuda, "Stream", lambda dev: None)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "empty_cache", lambda: log.append("trim"))
+    monkeypatch.setattr(DecodeSession, "_step", lambda self: log.append("step"))
     for _ in range(3):
         sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
         sess.graph = Graph()
-        refs.append(weakref.ref(sess.graph))
+        gone = weakref.ref(sess.graph)
+        weakref.finalize(sess.graph, log.append, "free")
         del sess
-    assert refs[0]() is None and len(engine._retired) == 2
+    assert gone() is not None and log == ["free"]
     sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
-    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: 1 / 0)
+    sess.capture()
+    assert log == ["free", "begin", "step", "end", "free", "free"] and gone() is None and sess.graph is not None
+    sess.capture()
+    assert len(log) == 6  # captured already
+    for _ in range(engine._TRIM - 1):
+        DecodeSession(_Model(HybridProgram), 1, 16, 16).capture()
+    assert log.count("trim") == 1 and log[-1] == "trim"
+    sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+    monkeypatch.setattr(DecodeSession, "_step", lambda self: 1 / 0)
     with pytest.raises(ZeroDivisionError):
         sess.capture()
-    assert refs[1]() is None and refs[2]() is None
+    assert log[-2:] == ["begin", "end"] and sess.graph is None
