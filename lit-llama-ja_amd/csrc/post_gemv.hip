@@ -1,16 +1,11 @@
-// Decode products of hybrid models with bf16 weights (N, K): few activation rows (M <= 16), each
-// weight read once and fed straight from its registers to the MFMA units.
+// Decode products of hybrid models with bf16 weights (N, K): few activation rows (M <= 16), each weight read once.
 //
 // One row runs on rowdot.h, also as the residual after a sublayer (llj_post_linear) and as the residual streams
-// (llj_streams_linear). From two rows on (and for a row of more than kRdMaxC values):
-// a workgroup owns 16 output columns; its NW waves take the 128-deep K chunks round robin, D chunks in
-// flight per wave (a chunk of a column is 256 contiguous bytes, 16 B per lane and MFMA step), and their
-// partial tiles are summed through LDS. Activation rows are read as MFMA fragments from memory (L2) next to the weights:
-// no staging, no barrier before the stream; lanes of rows past M read row 0 and their results are dropped.
-// Few columns (N / 16 workgroups would leave CUs idle): HALF forms take 8 columns per workgroup and up to 8 rows
-// and put the two halves of K side by side in the MFMA tile -- operand rows 0-7 / columns 0-7 the first
-// half, rows 8-15 / columns 8-15 the second; the two diagonal quarters of the result are added.
-// Output bf16, plus a bias, optionally max(., 0)^2 or the clamped gated unit of interleaved columns (elem.h).
+// (llj_streams_linear). 2 to 8 rows run on rows_gemv_kernel, 9 to 16 (and rows of values that do not fit its registers) on
+// post_gemv_kernel. Output bf16, plus a bias, optionally max(., 0)^2 or the clamped gated unit of interleaved columns (elem.h).
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "elem.h"
 #include "lit_llama_amd.h"
@@ -28,16 +23,174 @@ struct PostGemvParams {
   float limit, alpha;  // clamped gated unit
 };
 
-template <int NW, int D, int ACT, bool HALF>
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// the 4x4 MFMA, 16 blocks: lane 4 b + j holds 4 values of row / column j of block b; result r of the lane: row r, column j
+__device__ __forceinline__ f32x4 mfma4(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, u32x2{a0, a1}), __builtin_bit_cast(s16x4, u32x2{b0, b1}), c, 0, 0, 0);
+}
+// x summed over the two halves of the wave (WIDE) or of each 32 lanes in the lower half's lanes, y likewise in the upper half's
+template <bool WIDE>
+__device__ __forceinline__ float lane_split(float x, float y) {
+  if constexpr (WIDE) asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+  else asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+  return x + y;
+}
+// with the value 4 (8) lanes further on within 16 lanes
+template <int N>
+__device__ __forceinline__ float quad_add(float v) { return v + dpp_f32<0x120 + N>(v); }  // row_ror
+
+// 2 to 8 rows. Bound: the weights' bytes, and at these sizes (tens of MB) the first bytes' latency. Each of a workgroup's NW waves
+// keeps the rows' values of its own share of K (up to S chunks of 128) in registers, as operands of the 4x4 MFMA whose 16 blocks
+// take 16 neighbouring pieces of K: a load is 256 consecutive bytes of each of 4 columns, and the sums of a group of 4 columns
+// leave the blocks once per wave, by lane swaps that halve the rows a lane holds. G groups' loads are in flight per wave, each
+// chunk's register loaded anew as soon as its products are done. The 16x16 form (below) reads its rows again from L2 for every 16
+// columns and, at 8 rows, multiplies as many zeros. us in a graph (TB/s), 8 rows, 16x16 form -> this:
+//   2048 -> 8448   12.5 (2.8) -> 9.3 (3.7)      8448 -> 2048   13.4 (2.6) -> 10.9 (3.2)    2048 -> 6272   9.3 (2.8) -> 7.6 (3.4)
+//   2048 -> 2048    6.7 (1.3) -> 5.1 (1.7)      2048 -> 32000  31.8 (4.1) -> 23.1 (5.7)    4096 -> 4096  10.6 (3.2) -> 9.0 (3.7)
+//   4096 -> 26112  54.1 (4.0) -> 35.0 (6.1)    16512 -> 4096   37.6 (3.6) -> 33.4 (4.1)   13056 -> 4096  28.5 (3.8) -> 22.1 (4.8)
+//   2 rows: 2048 -> 8448 11.1 -> 7.9, 4096 -> 26112 47.3 -> 35.8, 16512 -> 4096 34.8 -> 28.4
+template <int NW, int S, int G, int MG, int ACT>
+__global__ __launch_bounds__(NW * 64) void rows_gemv_kernel(PostGemvParams p) {
+  extern __shared__ __align__(16) float part[];  // [column][NW][RW]
+  constexpr int RW = 4 * MG;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), b = lane >> 2, j = lane & 3;
+  const int K = p.K, KC = K >> 7, groups = p.N >> 2;
+  const int g0 = (int)((long)blockIdx.x * groups / gridDim.x), g1 = (int)((long)(blockIdx.x + 1) * groups / gridDim.x);
+  const int k0 = KC * wave / NW, n = KC * (wave + 1) / NW - k0;  // this wave's chunks, at most S
+  u32x4 a[S][MG], wr[G][S];
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int g = 0; g < MG; ++g) {
+      const int m = 4 * g + j, c = k0 + s < KC ? k0 + s : KC - 1;
+      a[s][g] = *reinterpret_cast<const u32x4*>(p.A + (size_t)(m < p.M ? m : 0) * p.lda + 128 * c + 8 * b);
+    }
+  // This workgroup's columns as a buffer: a load past this wave's chunks or past the columns fetches nothing, so that the count of
+  // loads in flight is the same everywhere.
+  const __amdgpu_buffer_rsrc_t weights =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + (size_t)4 * g0 * K), 0, (g1 - g0) * 8 * K, 0x00020000);
+  const int lane_at = 2 * (j * K + 128 * k0 + 8 * b);
+  auto load = [&](int g, int s, int grp) {
+    const int at = s < n && grp < g1 ? lane_at + 8 * (grp - g0) * K + 256 * s : 0x7ffffff0;  // (all of it in the checked offset)
+    wr[g][s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(weights, at, 0, 2));  // non-temporal
+  };
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int s = 0; s < S; ++s) load(g, s, g0 + g);
+  auto round = [&](int grp, auto more) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      f32x4 acc[MG];
+#pragma unroll
+      for (int i = 0; i < MG; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const u32x4 w = wr[g][s];
+        if (s < n) {  // (uniform)
+#pragma unroll
+          for (int i = 0; i < MG; ++i) {
+            acc[i] = mfma4(a[s][i][0], a[s][i][1], w[0], w[1], acc[i]);
+            acc[i] = mfma4(a[s][i][2], a[s][i][3], w[2], w[3], acc[i]);
+          }
+        }
+        if constexpr (decltype(more)::value) load(g, s, grp + G + g);
+      }
+      if (grp + g >= g1) continue;
+      // acc[i][r]: row 4 i + r, column j, block b's share. Lanes 0-31 / 32-63, then the 16-lane rows, keep half of the rows each.
+      // (The first additions are the compiler's, which waits for the products; the swaps' asm does not.)
+#pragma unroll
+      for (int i = 0; i < MG; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][r] = quad_add<4>(acc[i][r]);
+      float* dst = part + ((size_t)(4 * (grp + g - g0) + j) * NW + wave) * RW + (RW / 2) * (lane >> 5) + (RW / 4) * ((lane >> 4) & 1);
+      if constexpr (MG == 2) {
+        f32x4 h;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h[r] = lane_split<true>(acc[0][r], acc[1][r]);
+        const float y0 = quad_add<8>(lane_split<false>(h[0], h[2])), y1 = quad_add<8>(lane_split<false>(h[1], h[3]));
+        if ((lane & 15) < 4) *reinterpret_cast<float2*>(dst) = make_float2(y0, y1);
+      } else {
+        const float y = quad_add<8>(lane_split<false>(lane_split<true>(acc[0][0], acc[0][2]), lane_split<true>(acc[0][1], acc[0][3])));
+        if ((lane & 15) < 4) *dst = y;
+      }
+    }
+  };
+  int grp = g0;
+  for (; grp + G < g1; grp += G) round(grp, std::true_type{});
+  round(grp, std::false_type{});
+  __syncthreads();
+  auto column = [&](int m, int c) {
+    float y = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) y += part[((size_t)c * NW + w) * RW + m];
+    if (ACT != 1) y += p.bias ? p.bias[4 * g0 + c] : 0.f;
+    return y;
+  };
+  const int cols = (4 * (g1 - g0)) >> (ACT == 2 ? 1 : 0), o0 = (4 * g0) >> (ACT == 2 ? 1 : 0);
+  for (int i = tid; i < cols * RW; i += NW * 64) {
+    const int m = i % RW, c = i / RW;
+    if (m >= p.M) continue;
+    float y;
+    if constexpr (ACT == 2) {
+      y = clamped_glu(column(m, 2 * c), column(m, 2 * c + 1), p.limit, p.alpha);
+    } else {
+      y = column(m, c);
+      if (ACT == 1) y = fmaxf(y, 0.f) * fmaxf(y, 0.f);
+    }
+    p.out[(size_t)m * p.ldo + o0 + c] = f2bf(y);
+  }
+}
+
+constexpr int kRowsMaxK = 8 * 17 * 128;
+
+template <int NW, int S, int G, int MG, int ACT>
+static int rows_gemv_go(const PostGemvParams& p, hipStream_t s) {
+  // one, two, four .. workgroups per CU, 8 waves per CU at most, at least 8 column groups each: the rows' loads are the same in
+  // every workgroup (2048 -> 8448, 8 rows: 512 workgroups 10.7 us, 256 9.3; 2048 -> 2048: 512 7.7, 256 5.1). Very wide outputs: the
+  // sums of a share stay within 48 KiB.
+  const int groups = p.N / 4, most = 48 * 1024 / (4 * NW * 4 * MG * 4) - 1;
+  int grid = 2048 / NW;
+  while (grid > 256 && groups < 8 * grid) grid /= 2;
+  grid = std::max(std::min(grid, groups), (groups + most - 1) / most);
+  const size_t lds = (size_t)((groups + grid - 1) / grid) * 4 * NW * 4 * MG * 4;
+  hipLaunchKernelGGL((rows_gemv_kernel<NW, S, G, MG, ACT>), dim3(grid), dim3(NW * 64), lds, s, p);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+template <int MG, int ACT>
+static int rows_gemv_k(const PostGemvParams& p, hipStream_t s) {
+  const int KC = p.K / 128;  // chunks; S: the least that covers them
+  if (KC <= 8) return rows_gemv_go<2, 4, 4, MG, ACT>(p, s);
+  if (KC <= 16) return rows_gemv_go<4, 4, 4, MG, ACT>(p, s);
+  if (KC <= 32) return rows_gemv_go<8, 4, 4, MG, ACT>(p, s);
+  if (KC <= 56) return rows_gemv_go<8, 7, 2, MG, ACT>(p, s);
+  if (KC <= 72) return rows_gemv_go<8, 9, 2, MG, ACT>(p, s);
+  if (KC <= 104) return rows_gemv_go<8, 13, 1, MG, ACT>(p, s);
+  return rows_gemv_go<8, 17, 1, MG, ACT>(p, s);
+}
+
+template <int ACT>
+static int rows_gemv_launch(const PostGemvParams& p, hipStream_t s) {
+  return p.M <= 4 ? rows_gemv_k<1, ACT>(p, s) : rows_gemv_k<2, ACT>(p, s);
+}
+
+// 9 to 16 rows: a workgroup owns 16 output columns; its NW waves take the 128-deep K chunks round robin, D chunks in
+// flight per wave (a chunk of a column is 256 contiguous bytes, 16 B per lane and MFMA step), and their partial tiles are summed
+// through LDS. Activation rows are read as MFMA fragments from memory (L2) next to the weights: no staging, no barrier before
+// the stream; lanes of rows past M read row 0 and their results are dropped.
+template <int NW, int D, int ACT>
 __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
   __shared__ __align__(16) float red[NW * 256];  // [NW][64][4]
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
   const int row = lane & 15, g = lane >> 4;
-  constexpr int CW = HALF ? 8 : 16;
-  const int K = p.K, KC = HALF ? K >> 8 : K >> 7, n0 = blockIdx.x * CW;
-  const int rc = HALF ? row & 7 : row, koff = HALF && row >= 8 ? K >> 1 : 0;  // column / row of the lane, its K half
-  const u32x4* wp = reinterpret_cast<const u32x4*>(p.W + (size_t)(n0 + rc) * K + koff + 8 * g);
-  const u32x4* ap = reinterpret_cast<const u32x4*>(p.A + (size_t)(rc < p.M ? rc : 0) * p.lda + koff + 8 * g);
+  constexpr int CW = 16;
+  const int K = p.K, KC = K >> 7, n0 = blockIdx.x * CW;
+  const u32x4* wp = reinterpret_cast<const u32x4*>(p.W + (size_t)(n0 + row) * K + 8 * g);
+  const u32x4* ap = reinterpret_cast<const u32x4*>(p.A + (size_t)(row < p.M ? row : 0) * p.lda + 8 * g);
   u32x4 wr[D][4], ar[D][4];
   auto load = [&](int d, int i) {
     int c = wave + NW * i;
@@ -71,10 +224,7 @@ __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
   auto column = [&](int m, int c) {
     float y = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      y += red[(w * 64 + (m >> 2) * 16 + c) * 4 + (m & 3)];
-      if (HALF) y += red[(w * 64 + ((m + 8) >> 2) * 16 + c + 8) * 4 + (m & 3)];
-    }
+    for (int w = 0; w < NW; ++w) y += red[(w * 64 + (m >> 2) * 16 + c) * 4 + (m & 3)];
     if (ACT != 1) y += p.bias ? p.bias[n0 + c] : 0.f;
     return y;
   };
@@ -92,24 +242,21 @@ __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
   }
 }
 
-template <int NW, int D, bool HALF>
+template <int NW, int D>
 static int post_gemv_go(const PostGemvParams& p, int act, hipStream_t s) {
-  const dim3 grid(p.N / (HALF ? 8 : 16)), nt(NW * 64);
-  if (act == 2) hipLaunchKernelGGL((post_gemv_kernel<NW, D, 2, HALF>), grid, nt, 0, s, p);
-  else if (act) hipLaunchKernelGGL((post_gemv_kernel<NW, D, 1, HALF>), grid, nt, 0, s, p);
-  else hipLaunchKernelGGL((post_gemv_kernel<NW, D, 0, HALF>), grid, nt, 0, s, p);
+  const dim3 grid(p.N / 16), nt(NW * 64);
+  if (act == 2) hipLaunchKernelGGL((post_gemv_kernel<NW, D, 2>), grid, nt, 0, s, p);
+  else if (act) hipLaunchKernelGGL((post_gemv_kernel<NW, D, 1>), grid, nt, 0, s, p);
+  else hipLaunchKernelGGL((post_gemv_kernel<NW, D, 0>), grid, nt, 0, s, p);
   LLJ_CHECK_LAUNCH();
   return 0;
 }
 
-#ifndef LLJ_PG_HALF_M
-#define LLJ_PG_HALF_M 8  // largest row count that takes the half-K form where it applies (A/B; 0: never)
-#endif
 static int post_gemv_launch(const PostGemvParams& p, int act, hipStream_t s) {
+  if (p.M <= 8 && p.K <= kRowsMaxK)
+    return act == 2 ? rows_gemv_launch<2>(p, s) : act ? rows_gemv_launch<1>(p, s) : rows_gemv_launch<0>(p, s);
   // waves: 8 for long K, so that a wave's chunks stay within a few rounds of the D in flight
-  if (p.M <= LLJ_PG_HALF_M && p.N / 16 < 256 && p.K % 256 == 0 && p.K >= 1024)
-    return p.K > 4096 ? post_gemv_go<8, 5, true>(p, act, s) : post_gemv_go<4, 4, true>(p, act, s);
-  return p.K > 2048 ? post_gemv_go<8, 4, false>(p, act, s) : post_gemv_go<4, 4, false>(p, act, s);
+  return p.K > 2048 ? post_gemv_go<8, 4>(p, act, s) : post_gemv_go<4, 4>(p, act, s);
 }
 
 constexpr int kPostMaxK = 28544;  // widest weight rows of the post and streams forms

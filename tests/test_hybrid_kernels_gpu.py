@@ -102,6 +102,29 @@ def test_rows_linear(hip, M, N, K, act):
     assert float((out[:, N:] - 3.0).abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("K", [128, 1024, 1152, 2048, 2176, 4096, 4224, 7168, 7296, 9216, 9344, 13312, 13440, 17408, 17536])
+@pytest.mark.parametrize("M", [2, 4, 5, 8])
+def test_rows_linear_shares(hip, M, K):
+    """2 to 8 rows at both ends of every share of K a wave can take, columns that leave workgroups unequal (or no) shares, up to
+    several rounds of loads; weights past a workgroup's columns and rows past M hold NaN and are not used. The tolerance: the
+    rounding of the bf16 output (2^-9) at twice its size, for the largest of a few thousand results."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    for N in (16, 1040, 3088) if K <= 4224 else (16, 528):
+        A = torch.full((9, K + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+        A[:M, :K] = torch.randn(M, K, generator=g, device="cuda")
+        W = torch.full((N + 16, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+        W[:N] = torch.randn(N, K, generator=g, device="cuda") * K ** -0.5
+        bias = torch.randn(N, generator=g, device="cuda")
+        want = back(A)[:M, :K] @ back(W)[:N].T
+        for act in (0, 1, 2):
+            w = N // 2 if act == 2 else N
+            out = torch.full((M + 1, w + 16), 3.0, dtype=torch.bfloat16, device="cuda")
+            call("llj_rows_linear", act, A, K + 8, W, None if act == 1 else bias, out, w + 16, M, N, K, 1.25, 1.5)
+            ref = np.maximum(want, 0) ** 2 if act == 1 else want + back(bias)
+            close(back(out)[:M, :w], _unit_ref(ref, 1.25, 1.5) if act == 2 else ref, 4e-3)
+            assert float((out[:, w:] - 3.0).abs().max()) == 0.0 and float((out[M] - 3.0).abs().max()) == 0.0
+
+
 @pytest.mark.parametrize("C,K,N", [(72, 128, 256), (2048, 2048, 384), (4096, 4096, 128), (8192, 8192, 4224), (1000, 1024, 8448)])
 @pytest.mark.parametrize("act", [0, 1])
 def test_post_linear(hip, C, K, N, act):
