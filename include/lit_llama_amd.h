@@ -68,8 +68,8 @@ int llj_set_stream_a(int mode);
  * first use; -1 = unset = the build default) and can be set per process; launches never read the
  * environment. Returns the previous value, or -1000 for an unknown option / out-of-range value.
  *   LLJ_OPT_ATT_SPEC_FULL  0..1  decode attention loads a whole (1) or half (0) key pass before the position (LLJ_ATT_SPEC)
- *   LLJ_OPT_FLASH_QB       1..2  flash prefill: 16-query blocks per wave (LLJ_FLASH_QB)
- *   LLJ_OPT_FLASH_PAIR     0..1  flash prefill: (long, short) query-block pairs per workgroup (LLJ_FLASH_PAIR)
+ *   LLJ_OPT_FLASH_QB       1..2  flash prefill: 16-query blocks per wave (default 1)
+ *   LLJ_OPT_FLASH_PAIR     0..1  flash prefill: (long, short) query-block pairs per workgroup (default 0)
  *   LLJ_OPT_GEMM_GLDS      0..1  prefill GEMMs: LDS-DMA (1) or register-staged (0) kernel for every format (LLJ_GEMM_GLDS)
  *   LLJ_OPT_GLDS_COST128   0..   LDS-DMA GEMM: cost of a 256 x 128 tile in % of a 256 x 256 one (LLJ_GLDS_COST128)
  *   LLJ_OPT_GEMV_LDS_A_KB  56..96 decode GEMVs: cap of the staged A image in KiB (LLJ_GEMV_LDS_A_KB)

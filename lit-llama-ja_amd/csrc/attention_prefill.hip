@@ -15,7 +15,8 @@
 // delivered column-major); staging V^T with 2-byte scattered stores cost 8-way bank conflicts
 // and 32 LDS writes per thread per tile (7B T = 2048: 357 us per layer). Keys are the cache slots
 // 0 .. p of a query at position p (no ring wrap: p0 + T <= S, checked by the caller), masked on
-// the diagonal tile.
+// the diagonal tile. Bound: the chain of each tile's steps, so what counts is waves per SIMD (3) without a spilled register: one
+// register set holds the next tile, and the loop body stands in the code once.
 #include <cstdlib>
 
 #include "common.h"
@@ -26,31 +27,13 @@ namespace llj {
 constexpr int kFK = 64;   // keys per tile
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-#ifndef LLJ_FLASH_OCC
-#define LLJ_FLASH_OCC 3  // workgroups per CU the QB = 1 register budget is sized for (152 VGPRs, no spill; 2: 7B T=2048 window 40.0 vs 39.5 ms)
-#endif
-#ifndef LLJ_FLASH_PAIR
-#define LLJ_FLASH_PAIR 1  // causal balance: one workgroup per (long, short) pair of query blocks (7B window -1.0 ms)
-#endif
 #ifndef LLJ_FLASH_FAST
 #define LLJ_FLASH_FAST 1  // softmax: mask only the diagonal tiles, raw-score max, v_exp_f32, rescale only when a max moved
 #endif
-#ifndef LLJ_FLASH_NWQ
-#define LLJ_FLASH_NWQ 4  // waves per workgroup (16 queries each) of the head-size-128 one-block form (8: 128 queries share a K / V tile)
-#endif
-#ifndef LLJ_FLASH_PF
-#define LLJ_FLASH_PF 1  // K / V tiles in flight in registers (2: two register sets; 7B window 32.03-32.06 ms at 1 vs 32.13-32.31 at 2)
-#endif
-#ifndef LLJ_FLASH_QB2_MIN_T
-#define LLJ_FLASH_QB2_MIN_T 2048
-#endif
-#ifndef LLJ_FLASH_QB
-#define LLJ_FLASH_QB 1  // 16-query blocks per wave (2: every K / V fragment read feeds two MFMAs; with the pairing 1 is faster)
-#endif
 // QB 16-query blocks per wave: 64 QB queries per workgroup; a K fragment (S^T) and a V^T fragment
 // (O^T) read from LDS feed QB MFMAs, and the tile's staging and barriers are shared by 4 x 16 QB queries
-template <int HS, int QB, bool PAIR, int NWQ = 4>
-__global__ __launch_bounds__(64 * NWQ, NWQ == 8 ? 1 : QB == 1 && LLJ_FLASH_PF == 1 ? LLJ_FLASH_OCC : 2) void flash_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
+template <int HS, int QB, bool PAIR>
+__global__ __launch_bounds__(256, QB == 1 ? 3 : 2) void flash_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                             const bf16_t* __restrict__ vc, bf16_t* __restrict__ y,
                                                             const int* __restrict__ pos, int T, int S, int nh,
                                                             float sl2) {
@@ -62,10 +45,10 @@ __global__ __launch_bounds__(64 * NWQ, NWQ == 8 ? 1 : QB == 1 && LLJ_FLASH_PF ==
   __shared__ __attribute__((aligned(16))) bf16_t Vs[kFK * VP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, g = lane >> 4;
-  constexpr int NT = 64 * NWQ;       // threads per workgroup
-  constexpr int kFQ = 16 * NWQ * QB;  // queries per workgroup
+  constexpr int NT = 256;       // threads per workgroup
+  constexpr int kFQ = 64 * QB;  // queries per workgroup
   auto run = [&](const int qb) {
-    const int h = blockIdx.y, b = blockIdx.z;
+    const int h = PAIR ? blockIdx.y : blockIdx.x % nh, b = PAIR ? blockIdx.z : blockIdx.x / nh;
     const int C = nh * HS;
     const int p0 = pos[0];
     int t[QB], qpos[QB];  // this lane's query rows (rows past T are computed on a copy, never stored)
@@ -87,10 +70,8 @@ __global__ __launch_bounds__(64 * NWQ, NWQ == 8 ? 1 : QB == 1 && LLJ_FLASH_PF ==
     const bf16_t* vbase = vc + ((size_t)(b * nh + h) * S) * HS;
     // staging map: 64 keys x HS/8 vectors = 64 * HS / 8 16-B pieces over NT threads
     constexpr int PV = kFK * HS / 8 / NT;
-    // two register sets (LLJ_FLASH_PF 2): tile kt + 2's loads are issued while tile kt is multiplied,
-    // so each tile's K / V loads have two tiles of MFMA work to land in (one with LLJ_FLASH_PF 1)
-    u32x4 kA[PV], vA[PV], kB[PV], vB[PV];
-    auto load_into = [&](int kt, u32x4 (&kr)[PV], u32x4 (&vr)[PV]) {
+    u32x4 kr[PV], vr[PV];  // the next tile, in flight over this one's products
+    auto load = [&](int kt) {
   #pragma unroll
       for (int i = 0; i < PV; ++i) {
         const int piece = tid + NT * i;
@@ -110,7 +91,8 @@ __global__ __launch_bounds__(64 * NWQ, NWQ == 8 ? 1 : QB == 1 && LLJ_FLASH_PF ==
   #pragma unroll
       for (int d = 0; d < DB; ++d) acc_o[qi][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    auto step = [&](int kt, u32x4 (&kr)[PV], u32x4 (&vr)[PV], u32x4 (&kn)[PV], u32x4 (&vn)[PV]) {
+    load(0);
+    for (int kt = 0; kt < ntile; ++kt) {
       __syncthreads();  // the previous tile's readers are done with Ks / Vt
   #pragma unroll
       for (int i = 0; i < PV; ++i) {
@@ -120,11 +102,7 @@ __global__ __launch_bounds__(64 * NWQ, NWQ == 8 ? 1 : QB == 1 && LLJ_FLASH_PF ==
         *reinterpret_cast<u32x4*>(Vs + key * VP + 8 * v8) = vr[i];
       }
       __syncthreads();
-      if (LLJ_FLASH_PF == 2) {
-        if (kt + 2 < ntile) load_into(kt + 2, kr, vr);  // the set just staged is free
-      } else {
-        if (kt + 1 < ntile) load_into(kt + 1, kn, vn);  // in flight during this tile's MFMAs
-      }
+      if (kt + 1 < ntile) load(kt + 1);
       // S^T = K . Q^T for the tile's four 16-key blocks
       f32x4 s[QB][4];
   #pragma unroll
@@ -215,27 +193,14 @@ __global__ __launch_bounds__(64 * NWQ, NWQ == 8 ? 1 : QB == 1 && LLJ_FLASH_PF ==
         for (int d = 0; d < DB; ++d) {
           // lane 4q + p of group g addresses keys 32u + 4g + q (+16), dims 16d + 4p .. +3; lane col
           // receives dim 16d + col of those 4 keys
-          const bf16_t* vr = Vs + (32 * u + 4 * g + ((lane >> 2) & 3)) * VP + 16 * d + 4 * (lane & 3);
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)vr);
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vr + 16 * VP));
+          const bf16_t* va = Vs + (32 * u + 4 * g + ((lane >> 2) & 3)) * VP + 16 * d + 4 * (lane & 3);
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)va);
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(va + 16 * VP));
           const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
           const u32x4 aw = {l2.x, l2.y, h2.x, h2.y};
   #pragma unroll
           for (int qi = 0; qi < QB; ++qi) acc_o[qi][d] = mfma_bf16(__builtin_bit_cast(bf16x8, aw), bfrag[qi], acc_o[qi][d]);
         }
-      }
-    };
-    load_into(0, kA, vA);
-    if (LLJ_FLASH_PF == 2) {
-      if (ntile > 1) load_into(1, kB, vB);
-      for (int kt = 0; kt < ntile; kt += 2) {
-        step(kt, kA, vA, kB, vB);
-        if (kt + 1 < ntile) step(kt + 1, kB, vB, kA, vA);
-      }
-    } else {
-      for (int kt = 0; kt < ntile; kt += 2) {
-        step(kt, kA, vA, kB, vB);
-        if (kt + 1 < ntile) step(kt + 1, kB, vB, kA, vA);
       }
     }
     // y[b*T + t][h*HS + d] = O / l; lane holds d = 16 db + 4 g + r of its query
@@ -255,26 +220,29 @@ __global__ __launch_bounds__(64 * NWQ, NWQ == 8 ? 1 : QB == 1 && LLJ_FLASH_PF ==
   };
   const int nqb = (T + kFQ - 1) / kFQ;
   if constexpr (PAIR) {  // block x takes query blocks nqb - 1 - x (long) and x (short): equal work per workgroup
-    const int qz = nqb - 1 - (int)blockIdx.x, qa = blockIdx.x;
-    run(qz);
-    if (qa < qz) {
+    for (int qb = nqb - 1 - (int)blockIdx.x;; qb = blockIdx.x) {
+      run(qb);
+      if (qb <= nqb - 1 - qb) break;
       __syncthreads();  // the first block's last readers are done with Ks / Vs
-      run(qa);
     }
   } else {
-    run(gridDim.x - 1 - blockIdx.x);  // long (late) query blocks first
+    // heads x sequences vary fastest (a chiplet then sees few heads' keys); query blocks from the last, longest one on, every other
+    // row of workgroups that fills the CUs once in reverse, so that workgroups that share a CU add up to the same work
+    const int R = max(1, 256 / (int)gridDim.x), r = blockIdx.y / R, j = blockIdx.y % R;
+    const int rank = r & 1 ? r * R + min(R, nqb - r * R) - 1 - j : (int)blockIdx.y;
+    run(nqb - 1 - rank);
   }
 }
 
-template <int HS, int QB, int NWQ = 4>
+template <int HS, int QB>
 static void flash_launch(const void* q, const void* kcache, const void* vcache, void* y, const int* pos, int B, int T,
                          int n_head, int S, float sl2, bool pair, hipStream_t st) {
-  const int nqb = (T + 16 * NWQ * QB - 1) / (16 * NWQ * QB);
+  const int nqb = (T + 64 * QB - 1) / (64 * QB);
   if (pair) {
-    hipLaunchKernelGGL((flash_prefill_kernel<HS, QB, true, NWQ>), dim3((nqb + 1) / 2, n_head, B), dim3(64 * NWQ), 0, st,
+    hipLaunchKernelGGL((flash_prefill_kernel<HS, QB, true>), dim3((nqb + 1) / 2, n_head, B), dim3(256), 0, st,
                        (const bf16_t*)q, (const bf16_t*)kcache, (const bf16_t*)vcache, (bf16_t*)y, pos, T, S, n_head, sl2);
   } else {
-    hipLaunchKernelGGL((flash_prefill_kernel<HS, QB, false, NWQ>), dim3(nqb, n_head, B), dim3(64 * NWQ), 0, st,
+    hipLaunchKernelGGL((flash_prefill_kernel<HS, QB, false>), dim3(n_head * B, nqb), dim3(256), 0, st,
                        (const bf16_t*)q, (const bf16_t*)kcache, (const bf16_t*)vcache, (bf16_t*)y, pos, T, S, n_head, sl2);
   }
 }
@@ -291,13 +259,15 @@ int llj_attention_prefill(const void* q, const void* kcache, const void* vcache,
   const float sl2 = 1.4426950408889634f / sqrtf((float)head_size);
   hipStream_t st = (hipStream_t)stream;
   const int oq = opt(LLJ_OPT_FLASH_QB), op = opt(LLJ_OPT_FLASH_PAIR);  // A/B options (llj_set_option)
-  // 1 or 2 query blocks per wave: 2 from LLJ_FLASH_QB2_MIN_T queries on (7B T = 2048: 29.28 / 29.43 vs
-  // 29.45 / 29.67 ms per window, profiles/r06aa_flash_qb.jsonl), where the grid still fills the CUs
-  const int qbw = oq > 0 ? oq : (T >= LLJ_FLASH_QB2_MIN_T ? 2 : LLJ_FLASH_QB);
-  const bool pair = op >= 0 ? op != 0 : LLJ_FLASH_PAIR != 0;  // a long and a short query block per workgroup
+  // One query block per wave, workgroups of one block each (the kernel orders them). 32 heads, T x sequences, us, before -> now:
+  // 301 20.9 -> 10.2, 512 33.3 -> 14.5, 1001 64.8 -> 26.8, 1500 104 -> 42.8, 2048 127 -> 67.6, 300 x 4 32.9 -> 13.3, 1001 x 2
+  // 85.8 -> 39.1. Before, the forms that the options still choose, which also spilled registers. Without the spills: two query
+  // blocks per wave 301 13.0, 1001 36.6, 2048 71.1; a workgroup taking a long and a short block in turn 301 13.3, 1001 31.8,
+  // 2048 79.4; 8 waves per K / V tile 301 11.7, 1001 33.3, 2048 66.3.
+  const int qbw = oq > 0 ? oq : 1;
+  const bool pair = op > 0;
   if (head_size == 128) {
     if (qbw == 2) flash_launch<128, 2>(q, kcache, vcache, y, pos, B, T, n_head, S, sl2, pair, st);
-    else if (LLJ_FLASH_NWQ == 8) flash_launch<128, 1, 8>(q, kcache, vcache, y, pos, B, T, n_head, S, sl2, pair, st);
     else flash_launch<128, 1>(q, kcache, vcache, y, pos, B, T, n_head, S, sl2, pair, st);
   } else if (head_size == 64) {
     if (qbw == 2) flash_launch<64, 2>(q, kcache, vcache, y, pos, B, T, n_head, S, sl2, pair, st);
