@@ -109,7 +109,7 @@ struct GemmParams {
 // load -> store dependence per element (7B 2048-token window: the QKV and silu * mul GEMMs ran
 // 20-26 % slower than the plain store GEMM of the same shape with per-element loads).
 #ifndef LLJ_QKV_LDS
-#define LLJ_QKV_LDS 1  // LDS-DMA GEMM at 256 x 128 (bf16, convert-once int4): QKV epilogue through LDS, 16-byte row stores
+#define LLJ_QKV_LDS 1  // LDS-DMA GEMM (bf16, convert-once int4): QKV epilogue through LDS, 16-byte row stores
 #endif
 #ifndef LLJ_GLDS_LDS_EPI
 #define LLJ_GLDS_LDS_EPI 1  // LDS-DMA GEMM at 256 x 128: store / residual / SwiGLU epilogues through LDS, 16-byte rows
@@ -871,7 +871,8 @@ struct GldsGeo {
   // convert-once int4: two bf16 (q - z) B tiles (BN rows x 128 B, the bf16 image) after the stages
   static constexpr size_t BF = CVT ? 2 * (size_t)BN * 128 : 0;
   static constexpr int NST = 3 * STAGE + BF + 1024 <= 160 * 1024 ? 3 : 2;
-  static constexpr size_t LDS = NST * STAGE + BF + 1024;  // + the row sums (per-fragment int4)
+  // + the row sums (per-fragment int4); the 256 x 256 QKV epilogue lays its bf16 tile over the stages and past them
+  static constexpr size_t LDS = NST * STAGE + BF + (BN == 256 ? 4096 : 1024);
   static constexpr int NG = 4 + ((WF == GWF_W4 || CVT) ? 1 : BN / 64);  // glds per thread per chunk
 };
 
@@ -1240,11 +1241,12 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
   }
 
   // ---- epilogue: lane holds rows m0 + wr * 16 MI + 16 i + 4 g + r, column n0 + wc * 16 NJ + 16 j + row
-  if constexpr (EP == GEP_QKV && LLJ_QKV_LDS && !NIB && BN == 128 && MI <= 4) if ((p.head_size & 7) == 0) {
+  if constexpr (EP == GEP_QKV && LLJ_QKV_LDS && !NIB) if (BN == 256 || (p.head_size & 7) == 0) {  // (256: gemm_glds_run)
     // QKV through LDS: the tile's bf16 c_attn outputs (model.py:204) go to LDS in the accumulator layout,
     // then every thread takes 8 consecutive columns (4 RoPE pairs: no lane exchange) of one row and
     // stores them as one 16-byte vector -- a tile row is 256 contiguous bytes of q, or of one K / V cache
-    // row (the head dimension), instead of 4-byte pairs from every other lane
+    // row (the head dimension), instead of 4-byte pairs from every other lane. At 256 x 256 the other form also computes
+    // every row's place again for each of its four column blocks and spills 88 registers (7B, 1001 rows bf16: 185 -> 115 us)
     constexpr int TP = BN + 8;  // row pitch (elements): 16-B aligned rows on shifted banks
     bf16_t* Ts = reinterpret_cast<bf16_t*>(smem);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1259,12 +1261,13 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
         for (int r = 0; r < 4; ++r) Ts[(wr * 16 * MI + 16 * i + 4 * g + r) * TP + nl] = f2bf(sc * acc[i][j][r]);
     }
     __syncthreads();
-    const int Cd = p.n_head * p.head_size, seg = tid & 15;
+    constexpr int SEGS = BN / 8, RPP = 512 / SEGS;
+    const int Cd = p.n_head * p.head_size, seg = tid % SEGS;
     const int nc0 = n0 + 8 * seg, region = nc0 / Cd, nc = nc0 - region * Cd;
     const int h = nc / p.head_size, dd = nc - h * p.head_size;  // 8 | head_size: the 8 columns share a head
 #pragma unroll 2
-    for (int k = 0; k < 8; ++k) {
-      const int rl = (tid >> 4) + 32 * k, m = m0 + rl;
+    for (int k = 0; k < 256 / RPP; ++k) {
+      const int rl = tid / SEGS + RPP * k, m = m0 + rl;
       if (m >= M) continue;
       const uint4 v = *reinterpret_cast<const uint4*>(Ts + rl * TP + 8 * seg);
       const QkvRow qr = qkv_row(p, m);
@@ -1518,7 +1521,9 @@ static int gemm_glds_run(const GemmParams& p, hipStream_t s) {
     cus = cached;
   }
   const long mt = (p.M + 255) / 256;
-  const long w256 = p.N % 256 == 0 ? (mt * (p.N / 256) + cus - 1) / cus : -1;
+  // (the 256 x 256 QKV epilogue of bf16 stores 8 columns of one head at a time)
+  const bool whole = EP != GEP_QKV || WF == GWF_W4 || (p.head_size & 7) == 0;
+  const long w256 = p.N % 256 == 0 && whole ? (mt * (p.N / 256) + cus - 1) / cus : -1;
   const long w128 = (mt * (p.N / 128) + cus - 1) / cus;
   const int oc = opt(LLJ_OPT_GLDS_COST128);  // A/B and tests: 0 forces 256 x 128, >= 100 prefers 256 x 256
   const long cost = oc >= 0 ? oc : LLJ_GLDS_COST128;

@@ -1934,3 +1934,33 @@ def test_gemm_split_qkv(hip, wfmt):
         if wfmt == 2:
             np.testing.assert_array_equal(a, b)
         assert_bf16_close(b, a, name, rel=2.0 ** -6, abs_frac=4e-3)
+
+
+@pytest.mark.parametrize("nh,hs,B,T_,S", [(16, 64, 1, 300, 320), (6, 128, 2, 257, 257), (16, 80, 1, 513, 600), (32, 40, 1, 256, 200),
+                                         (64, 20, 1, 300, 300)])
+def test_gemm_qkv_tiles(hip, nh, hs, B, T_, S):
+    """The bf16 c_attn product on 256 x 256 tiles against 256 x 128 ones: the same sums in the same order, so the same bits, over
+    head sizes that are no power of two, tiles across heads and the q / k / v borders, ragged rows, two sequences, a wrapped ring
+    and head sizes whose rows are not 16-byte pieces (256 x 128 tiles in both)."""
+    g = torch.Generator(device=dev).manual_seed(nh * hs + T_)
+    C, M = nh * hs, B * T_
+    x = torch.randn(M, C, device=dev, generator=g).to(torch.bfloat16)
+    W = (torch.randn(3 * C, C, device=dev, generator=g) * C ** -0.5).to(torch.bfloat16)
+    rope, pos = T(O.build_rope_cache(T_ + 8, hs)), T(np.arange(3, 3 + T_, dtype=np.int32))
+    outs = []
+    for cost in (0, 400):
+        q, kc, vc = (torch.full(s, 3.0, dtype=torch.bfloat16, device=dev) for s in ((M, C), (B, nh, S, hs), (B, nh, S, hs)))
+        with option(hip, _hip.OPT_GLDS_COST128, cost):
+            call(hip, "llj_gemm_qkv_rope", 1, x.data_ptr(), W.data_ptr(), None, q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                 rope.data_ptr(), pos.data_ptr(), B, T_, C, nh, S, st())
+        torch.cuda.synchronize()
+        outs.append((q, kc, vc))
+    keep = T_ <= S  # a ring shorter than the prompt: two rows per slot, either may stay
+    assert torch.equal(outs[0][0], outs[1][0])
+    if keep:
+        assert torch.equal(outs[0][1], outs[1][1]) and torch.equal(outs[0][2], outs[1][2])
+    y = x.float() @ W.float().T
+    if keep:
+        v = y[:, 2 * C:].view(B, T_, nh, hs).transpose(1, 2)
+        slots = ((pos.long()) % S)
+        assert_bf16_close(outs[1][2][:, :, slots].float().cpu().numpy(), v.cpu().numpy(), "v rows", rel=2.0 ** -7, abs_frac=2e-3)
