@@ -1,6 +1,6 @@
 """Build the in-tree HIP library (`_lljamd.so`) for gfx950 with hipcc. No torch in the ABI,
 so plain `hipcc` objects linked with `-shared` are enough; the .so lives next to this file so
-it travels with the repository snapshot to the GPU box. The translation units compile in
+it travels with a copy of the tree to machines without a compiler. The translation units compile in
 parallel (one hipcc per .hip file), then link."""
 from __future__ import annotations
 
