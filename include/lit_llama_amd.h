@@ -472,7 +472,10 @@ int llj_g_relu2(void* h, size_t n, int dt, void* stream);
  * llj_g_bias_act, any sizes, after a product: act 0 y += bias in place (out NULL), act 2 out[M, N / 2]. */
 int llj_g_bias_act(int act, void* y, int ldy, const float* bias, void* out, int ldo, int M, int N, float limit, float alpha,
                    int dt, void* stream);
-/* out[m] = act(A[m] . W^T + bias) for M <= 16 bf16 rows, the weight (N, K) read once. N % 16 == 0, K % 128 == 0. */
+/* out[m] = act(A[m] . W^T + bias) for M <= 16 bf16 rows, the weight (N, K) read once. N % 16 == 0, K % 128 == 0.
+ * act | LLJ_ACT_TILES: always on 16 x 16 tiles, so that a row's sums are the same whether it comes alone or among up to 8 (without
+ * it 1, and 2 to 8 rows take faster kernels that add in an order of their own). */
+#define LLJ_ACT_TILES 16
 int llj_rows_linear(int act, const void* A, int lda, const void* W, const float* bias, void* out, int ldo, int M, int N, int K,
                     float limit, float alpha, void* stream);
 /* One bf16 row with llj_post_norm in front: x_out = x + t / rms(t) * (1 + norm_w) (fp32, width C <= K, C % 8

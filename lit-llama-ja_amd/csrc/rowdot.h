@@ -15,8 +15,6 @@
 // Prologues (the weights' first loads are in flight meanwhile):
 //   plain    the row from memory, bf16;
 //   norm     RMSNorm with the reference's bf16 rounding points (model.py:281-283);
-//   post     the fp32 residual after a sublayer, x' = x + t / rms(t) * (1 + w), rounded to bf16 as the input and written
-//            once to x';
 //   streams  the residual streams after a sublayer, the mixed row and its layer norm (streams.hip), the new streams written
 //            once to x'.
 #pragma once
@@ -25,14 +23,14 @@
 
 namespace llj {
 
-enum { RD_PLAIN = 0, RD_NORM = 1, RD_POST = 2, RD_STREAMS = 3 };
+enum { RD_PLAIN = 0, RD_NORM = 1, RD_STREAMS = 2 };
 // RD_STORE: + bias (fp32 or NULL). RD_RESID: out += . RD_QKV: RoPE, q to out, k / v to the caches. RD_SWIGLU: silu(. W) * (. W2).
 // RD_RELU2: max(., 0)^2. RD_GLU: the clamped gated unit of interleaved columns (elem.h), biased.
 enum { RD_STORE = 0, RD_RESID = 1, RD_QKV = 2, RD_SWIGLU = 3, RD_RELU2 = 4, RD_GLU = 5 };
 
 struct RowDotParams {
   const bf16_t* A;  // plain, norm: the row
-  const bf16_t* w;  // norm, post, streams: norm weight
+  const bf16_t* w;  // norm, streams: norm weight
   float eps;
   int K, N;         // row stride of the weights; output columns (RD_SWIGLU: both weights' rows, 2 H)
   int C;            // values of the row (<= K, the weights past it are not read)
@@ -41,7 +39,7 @@ struct RowDotParams {
   bf16_t* out;
   const float* bias;
   float limit, alpha;
-  const bf16_t* t;  // post, streams: the sublayer's output; residual in / out
+  const bf16_t* t;  // streams: the sublayer's output; residual in / out
   const float* x;
   float* xo;
   const float* so;  // streams: output weights (S), mix (S, S), input weights (S) or NULL; x, xo: S rows of stride ldx
@@ -143,39 +141,6 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e)
           xf[s][e] = round_bf(((e & 1) ? bfhi(gv[s][e >> 1]) : bflo(gv[s][e >> 1])) * round_bf(xf[s][e] * r));
-    }
-  } else if constexpr (PRO == RD_POST) {
-    u32x4 tv[SL], gv[SL];
-#pragma unroll
-    for (int s = 0; s < SL; ++s) {
-      const int k = k0 + 512 * s, kk = k < p.C ? k : 0;
-      tv[s] = *reinterpret_cast<const u32x4*>(p.t + kk);
-      gv[s] = *reinterpret_cast<const u32x4*>(p.w + kk);
-      ld8(p.x + kk, xf[s]);
-    }
-    fetch(0, c0);
-    first = operand(tid);
-    float ss = 0.f;
-#pragma unroll
-    for (int s = 0; s < SL; ++s) {
-      if (k0 + 512 * s < p.C) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ss += bflo(tv[s][e]) * bflo(tv[s][e]) + bfhi(tv[s][e]) * bfhi(tv[s][e]);
-      }
-    }
-    const float r = 1.f / sqrtf(block_sum(ss, 0) / (float)p.C + p.eps);
-#pragma unroll
-    for (int s = 0; s < SL; ++s) {
-      const int k = k0 + 512 * s;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float tt = (e & 1) ? bfhi(tv[s][e >> 1]) : bflo(tv[s][e >> 1]);
-        const float gg = (e & 1) ? bfhi(gv[s][e >> 1]) : bflo(gv[s][e >> 1]);
-        xf[s][e] = k < p.C ? xf[s][e] + tt * r * (1.f + gg) : 0.f;
-      }
-      if (k < p.C && (unsigned)(k >> 3) % gridDim.x == blockIdx.x) st8(p.xo + k, xf[s]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) xf[s][e] = round_bf(xf[s][e]);
     }
   } else {
     u32x4 tv[SL], gv[SL];
@@ -312,7 +277,7 @@ static int rowdot_go(const RowDotParams& p, hipStream_t s) {
 }
 
 // The row's slices: as few waves as keep a wave's slice at 1024 values, 8 waves at most (streams, whose prologue reads 20 bytes per
-// value in every workgroup: 8 waves and half the workgroups from 2049 on). C <= kRdMaxC (streams, post: 8192).
+// value in every workgroup: 8 waves and half the workgroups from 2049 on). C <= kRdMaxC (streams: 8192).
 template <int PRO, int EPI>
 static int rowdot_launch(const RowDotParams& p, hipStream_t s) {
   if (p.C <= 1024) return rowdot_go<2, 1, PRO, EPI>(p, s);

@@ -42,9 +42,12 @@ class PackedLinear:
     at a multiple of PART_ALIGN), zero rows and columns up to the kernels' tiles. `offset[i]` is part i's
     first output column. `biases`: one per part (None: none). `unit` = (limit, alpha): two parts of equal size, gate
     and up, interleaved row by row, and the output is their clamped gated unit -- one column per pair, the
-    first lane_pad(part rows) columns."""
+    first lane_pad(part rows) columns. `tiles`: bf16 rows always on the 16 x 16 tiles (LLJ_ACT_TILES) and prompts below 256 rows
+    with unsplit sums, for models whose logits move with the order of a product's sums: Mugivik's recurrence carries every
+    flipped rounding on (bf16 logits from float64 ones, tiles and the other kernels: 1B, 2 prompts of 48, 0.013 and 0.029; 7B,
+    5 prompts of 49, 0.039 and 0.042; the two 0.030 and 0.039 apart)."""
 
-    def __init__(self, parts: list, dtype, device, biases: Optional[list] = None, unit: Optional[tuple] = None):
+    def __init__(self, parts: list, dtype, device, biases: Optional[list] = None, unit: Optional[tuple] = None, tiles: bool = False):
         if unit is not None:
             biases = biases or [None, None]
             n, pad = parts[0].shape[0], lane_pad(parts[0].shape[0], dtype)
@@ -57,7 +60,7 @@ class PackedLinear:
                 if b is not None:
                     bb[:n, j] = b.float().cpu()
             parts, biases = [both.view(2 * pad, -1)], [bb.view(-1)]
-        self.unit = unit
+        self.unit, self.tiles = unit, tiles
         self.K = parts[0].shape[1]
         self.Kp = lane_pad(self.K, dtype)
         self.offset, n = [], 0
@@ -102,11 +105,12 @@ class PackedLinear:
             if relu2:
                 _hip.call("llj_g_relu2", out.data_ptr(), M * out.stride(0), 1, st)
         elif M < GEMM_MIN_ROWS:  # weight-streaming rows
+            act |= _hip.ACT_TILES if self.tiles else 0
             for r in range(0, M, STREAM_ROWS):
                 _hip.call("llj_rows_linear", act, a[r].data_ptr(), a.stride(0), self.w.data_ptr(), bias, out[r].data_ptr(),
                           out.stride(0), min(STREAM_ROWS, M - r), self.Np, self.Kp, limit, alpha, st)
         else:
-            nb = 0 if act and M >= 256 else _hip.lib().llj_gemm_bf16_ws_bytes(M, self.Np, self.Kp)
+            nb = 0 if (act if M >= 256 else self.tiles) else _hip.lib().llj_gemm_bf16_ws_bytes(M, self.Np, self.Kp)
             ws = torch.empty(nb // 4, dtype=torch.float32, device=out.device) if nb else None
             _hip.call("llj_gemm_bf16", act, a.data_ptr(), a.stride(0), self.w.data_ptr(), bias, out.data_ptr(),
                       out.stride(0), M, self.Np, self.Kp, limit, alpha, _hip.ptr(ws), nb, st)
@@ -173,8 +177,8 @@ class GatedLinearAttention:
         """t: this mixer's tensors by their names."""
         self.rank = t["a1"].shape[0]
         _check_shapes(t, self.shapes(self.rank))
-        self.inp = PackedLinear([t["q"], t["k"], t["v"], t["g"], t["a1"]], dtype, device)
-        self.out = PackedLinear([t["o"]], dtype, device)
+        self.inp = PackedLinear([t["q"], t["k"], t["v"], t["g"], t["a1"]], dtype, device, tiles=True)
+        self.out = PackedLinear([t["o"]], dtype, device, tiles=True)
         self.norm = t["norm"].to(device=device, dtype=dtype).contiguous()
         self.a2 = t["a2"].to(device=device, dtype=dtype).contiguous()
         self.a2b = t["a2.b"].to(device=device, dtype=dtype).contiguous()
@@ -261,9 +265,9 @@ class LatentAttention:
         _check_shapes(t, self.shapes())
         s = self.spec
         own = s.kv_from is None
-        self.inp = PackedLinear([t["q"], t["g"]] + ([t["dkv"]] if own else []), dtype, device)
-        self.out = PackedLinear([t["o"]], dtype, device)
-        self.up = PackedLinear([t["uk"], t["uv"]], dtype, device)
+        self.inp = PackedLinear([t["q"], t["g"]] + ([t["dkv"]] if own else []), dtype, device, tiles=True)
+        self.out = PackedLinear([t["o"]], dtype, device, tiles=True)
+        self.up = PackedLinear([t["uk"], t["uv"]], dtype, device, tiles=True)
         self.kv_norm = t["dkv.norm"].to(device=device, dtype=dtype).contiguous() if own else None
         self.turns = rotation_turns(s.rot_dim, s.rot_base, device)
         self.dtype = dtype
@@ -491,8 +495,8 @@ class ReluSquaredMLP:
 
     def load(self, t: dict, dtype, device) -> None:
         _check_shapes(t, self.shapes())
-        self.up = PackedLinear([t["up"]], dtype, device)
-        self.down = PackedLinear([t["down"]], dtype, device)
+        self.up = PackedLinear([t["up"]], dtype, device, tiles=True)
+        self.down = PackedLinear([t["down"]], dtype, device, tiles=True)
 
     def linears(self) -> list:
         return [self.up, self.down]

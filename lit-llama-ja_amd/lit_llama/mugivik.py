@@ -165,7 +165,7 @@ class Mugivik(HybridModel):
         C = config.n_embd
         m.Cp = lane_pad(C, dtype)
         # one copy of the table for the lookup and the tied head
-        m.embed = m.head = PackedLinear([take("embed", (config.vocab_size, C))], dtype, m.device)
+        m.embed = m.head = PackedLinear([take("embed", (config.vocab_size, C))], dtype, m.device, tiles=True)
         m.bigram = take("bigram", (config.buckets + 1, C)).to(device=m.device, dtype=dtype).contiguous()
         m.embed_norm, m.final_norm = vec("embed.norm"), vec("final.norm")
         m.norm1, m.norm2 = [], []

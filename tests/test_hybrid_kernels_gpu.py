@@ -125,6 +125,55 @@ def test_rows_linear_shares(hip, M, K):
             assert float((out[:, w:] - 3.0).abs().max()) == 0.0 and float((out[M] - 3.0).abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("N,K", [(128, 128), (2048, 2048), (2048, 8448), (4096, 4096), (8448, 2048), (512, 17536)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_rows_on_tiles(hip, N, K, act):
+    """On the tiles a row's result is the same bits alone, among others, and with the norm that formed it in front
+    (both sides of the half-K forms' rule: few columns of a long K, up to 8 rows)."""
+    from lit_llama import _hip
+
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    W = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    A = torch.randn(8, K, generator=g, device="cuda").to(torch.bfloat16)
+    C = min(K, 8192)
+    t, w, x = (torch.randn(C, generator=g, device="cuda") for _ in range(3))
+    t, w, xo = t.to(torch.bfloat16), (0.3 * w).to(torch.bfloat16), torch.zeros(C, device="cuda")
+    post = torch.empty(N, dtype=torch.bfloat16, device="cuda")
+    call("llj_post_linear", act, t, w, 1e-5, x, xo, C, W, post, N, K)
+    A[0, :C], A[0, C:] = xo, 0
+    rows = {}
+    for M in (1, 2, 5, 8):
+        rows[M] = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        call("llj_rows_linear", act | _hip.ACT_TILES, A, K, W, None, rows[M], N, M, N, K, 0.0, 0.0)
+    want = back(A) @ back(W).T
+    close(back(rows[8]), np.maximum(want, 0) ** 2 if act else want, 5e-3)
+    for M in (1, 2, 5):
+        assert torch.equal(rows[M], rows[8][:M])
+    if N < 4096 or not 2048 < K <= 4096:  # (there the plain form splits K over twice the waves)
+        assert torch.equal(post, rows[8][0])
+
+
+@pytest.mark.parametrize("M", [1, 7, 40, 64, 154, 255])
+def test_packed_linear_on_tiles(hip, M):
+    """PackedLinear(tiles=True): rows and prompts below 256 rows as the tiles and the unsplit product give them, bit for bit."""
+    from lit_llama import _hip
+    from lit_llama.mixers import PackedLinear
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    K, N, st = 8448, 2048, torch.cuda.current_stream().cuda_stream
+    lin = PackedLinear([torch.randn(N, K, generator=g, device="cuda") * K ** -0.5], torch.bfloat16, "cuda", tiles=True)
+    a = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    got, want = (torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    lin.apply(a, M, got, st)
+    if M < 64:
+        for r in range(0, M, 16):
+            call("llj_rows_linear", _hip.ACT_TILES, a[r:], K, lin.w, None, want[r:], N, min(16, M - r), N, K, 0.0, 0.0)
+    else:
+        call("llj_gemm_bf16", 0, a, K, lin.w, None, want, N, M, N, K, 0.0, 0.0, None, 0)
+    assert torch.equal(got, want)
+    close(back(got), back(a) @ back(lin.w).T, 5e-3)
+
+
 @pytest.mark.parametrize("C,K,N", [(72, 128, 256), (2048, 2048, 384), (4096, 4096, 128), (8192, 8192, 4224), (1000, 1024, 8448)])
 @pytest.mark.parametrize("act", [0, 1])
 def test_post_linear(hip, C, K, N, act):
