@@ -267,7 +267,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
     float O = 0.f;
     constexpr int R = 16;
     float pc[R];
-    auto pieces = [&](int s0) {  // (past the end: a copy, its weight is 0)
+    auto pieces = [&](int s0) {  // (past the end: a copy, not used)
 #pragma unroll
       for (int e = 0; e < R; ++e) pc[e] = get1(src + (size_t)min(s0 + e, nsplit - 1) * kAttPart<HS> + d);
     };
@@ -276,12 +276,17 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
     if (lane < nsplit) ml = get2(src + (size_t)lane * kAttPart<HS> + HS);
     const float M = wave_max(ml.x);  // (in every lane: not inside the selection)
     const float w = ml.x == -INFINITY ? 0.f : exp2f(ml.x - M);
-    const float L = wave_sum(w * ml.y);
+    auto of_range = [](float v, int s) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), s)); };
+    float L = 0.f;  // both sums in attention_combine_kernel's order: the same bits
     for (int s0 = 0; s0 < nsplit; s0 += R) {
       if (s0) pieces(s0);
 #pragma unroll
-      for (int e = 0; e < R; ++e)  // (s0 + e < 64; ranges past nsplit weigh 0)
-        O += pc[e] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s0 + e));
+      for (int e = 0; e < R; ++e) {
+        if (s0 + e >= nsplit) break;  // (uniform; s0 + e < 64)
+        const float f = of_range(w, s0 + e);
+        L += of_range(ml.y, s0 + e) * f;
+        O += pc[e] * f;
+      }
     }
     attention_out<HS>(O / L, y, st, thr, h, m, C);
   }

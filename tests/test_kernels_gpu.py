@@ -812,7 +812,7 @@ def test_attention_split_keys(hip, hs, nh, B, T_, S, p0, nsplit):
 @pytest.mark.parametrize("hs,nh,B,T_,S,p0,nsplit", [(128, 4, 1, 1, 2048, 2000, 8), (128, 3, 2, 1, 2048, 40, 16), (64, 4, 2, 5, 600, 300, 3),
                                                    (128, 2, 1, 1, 512, 900, 1), (128, 5, 8, 1, 1033, 1010, 5), (64, 2, 3, 1, 700, 0, 64)])
 def test_attention_ranges(hip, hs, nh, B, T_, S, p0, nsplit):
-    """Interleaved key ranges merged by the last block, against the oracle: few to 64 ranges (most of them empty), heads and ranges
+    """Key ranges merged by the last block, against the oracle: few to 64 ranges (most of them empty), heads and ranges
     that are no multiple of the chiplets, prompt rows, the rolled ring; partials of the last call or NaN in the scratch make no
     difference and the counters end at zero. With statistics: those of llj_i8_stats on the same y, and the other block zeroed."""
     rng = np.random.default_rng(hs + S + p0 + nsplit)
@@ -840,6 +840,29 @@ def test_attention_ranges(hip, hs, nh, B, T_, S, p0, nsplit):
     if stats:
         for got, ref in zip(_st_decode(y_st, M, C), _i8_ws_stats(hip, y, M, C)):
             np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("hs,nh,B,T_,S,p0,nsplit", [(128, 32, 1, 1, 2048, 2000, 8), (128, 5, 2, 1, 2048, 40, 16), (64, 4, 2, 5, 600, 300, 3),
+                                                   (128, 2, 1, 1, 512, 900, 2), (128, 5, 8, 1, 1033, 1010, 5), (64, 2, 3, 1, 700, 699, 64)])
+def test_attention_ranges_are_the_split_ones(hip, hs, nh, B, T_, S, p0, nsplit):
+    """One launch or two (llj_attention_split: the same ranges, then the merge): the same bits, so that a sequence's tokens do not
+    depend on which of them its steps take. Infinite values too."""
+    rng = np.random.default_rng(hs + S + p0 + nsplit)
+    C, M = nh * hs, B * T_
+    kc, vc = (bf16(rng.standard_normal((B, nh, S, hs))) for _ in range(2))
+    vc[:, 0, p0 % S, 3] = np.inf
+    qd, kd, vd = T(bf16(rng.standard_normal((M, C)) * 2), torch.bfloat16), T(kc, torch.bfloat16), T(vc, torch.bfloat16)
+    pd = T(np.arange(p0, p0 + T_, dtype=np.int32))
+    part = torch.empty(hip.llj_attention_ws_bytes(M, nh, hs, nsplit), dtype=torch.uint8, device=dev)
+    count = torch.zeros(M * nh, dtype=torch.int32, device=dev)
+    one, two = (torch.empty(M, C, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    args = (qd.data_ptr(), kd.data_ptr(), vd.data_ptr())
+    call(hip, "llj_attention_split", *args, two.data_ptr(), pd.data_ptr(), B, T_, nh, hs, S, nsplit, part.data_ptr(), st())
+    part.fill_(0xFF)
+    call(hip, "llj_attention_ranges", *args, one.data_ptr(), pd.data_ptr(), B, T_, nh, hs, S, nsplit, part.data_ptr(), count.data_ptr(),
+         None, None, 0, 0.0, st())
+    torch.cuda.synchronize()
+    assert torch.equal(one.view(torch.int16), two.view(torch.int16))
 
 
 def _i8_ws_stats(hip, A, M, K):
