@@ -278,17 +278,32 @@ class DecodeSession:
         self.program.step(st)
         self._choose(st)
 
-    def capture(self):
-        if self.graph is not None or not self.use_graph:
-            return
+    def _record(self, last: bool = False):
+        """The step as a graph. What a step allocates comes out of the graph's own pool, for which the allocator gives back no cached
+        blocks while a capture is underway: None if that found no room (`last`: the error instead)."""
         # (not torch.cuda.graph: it waits for the device, here the prompt, and empties the allocator's cache first)
-        g = torch.cuda.CUDAGraph()
+        g, full = torch.cuda.CUDAGraph(), False
         with torch.cuda.stream(torch.cuda.Stream(self.dev)):
             g.capture_begin()
             try:
                 self._step()
+            except torch.OutOfMemoryError:
+                if last:
+                    raise
+                full = True
             finally:
                 g.capture_end()
+        return None if full else g
+
+    def capture(self):
+        if self.graph is not None or not self.use_graph:
+            return
+        g = self._record()
+        if g is None:
+            _retired.clear()
+            torch.cuda.synchronize()
+            torch.cuda.empty_cache()
+            g = self._record(last=True)
         self.graph = g
         _retired.clear()
         if next(_captures) % _TRIM == 0:

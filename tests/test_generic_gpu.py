@@ -98,6 +98,42 @@ def test_125m_generate_graph_matches_eager_and_wraps():
     assert outs[0].shape == (28,) and ((outs[0] >= 0) & (outs[0] < C125.vocab_size + 64)).all()
 
 
+def test_decode_on_a_device_full_of_cached_blocks(monkeypatch):
+    """A step that allocates where everything the process may use lies in the allocator's cache (after a large prompt): the capture
+    makes room, and the tokens are those of eager steps."""
+    from lit_llama.engine import DecodeSession
+
+    m, _ = _setup(REF_TEST, None, 7)
+    prompt = torch.from_numpy(np.random.default_rng(5).integers(3, REF_TEST.vocab_size, (2, 8))).cuda()
+    plain, attempts = DecodeSession._step, []
+
+    def step(self):
+        attempts.append(1)
+        room = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")  # (a step's own buffers)
+        plain(self)
+        del room
+
+    monkeypatch.setattr(DecodeSession, "_step", step)
+    outs = []
+    try:
+        for graph in (False, True):
+            s = DecodeSession(m, 2, 32, 32, use_graph=graph)
+            s.prefill(prompt)
+            if graph:
+                torch.cuda.empty_cache()
+                full = torch.empty(256 << 20, dtype=torch.uint8, device="cuda")
+                del full
+                total = torch.cuda.get_device_properties(0).total_memory
+                torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (16 << 20)) / total)
+                attempts.clear()
+            s.decode(12)
+            outs.append(s.output().cpu().numpy())
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert len(attempts) == 2  # captured at the second attempt, then replayed
+    np.testing.assert_array_equal(outs[0], outs[1])
+
+
 def test_generic_linear_grouped_int8_codes_vs_numpy():
     """llj_g_linear on ColBlock bits=8 codes with groups (tile_cols 256 over K 780 -> 4 groups, the
     last partial) and the residual form, against numpy (q - z) * s in fp32."""

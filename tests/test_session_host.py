@@ -85,3 +85,50 @@ def test_dropped_graphs_wait_for_the_next_capture(monkeypatch):
     with pytest.raises(ZeroDivisionError):
         sess.capture()
     assert log[-2:] == ["begin", "end"] and sess.graph is None
+
+
+def test_capture_makes_room_once(monkeypatch):
+    """A step whose buffers find no room during its capture: what the allocator and the dropped graphs hold is given back, with the
+    first attempt's graph, and the step captured again; the second time the error is the caller's."""
+    import contextlib
+
+    from lit_llama import engine
+
+    log = []
+
+    class Graph:
+        def __init__(self):
+            weakref.finalize(self, log.append, "free")
+
+        def capture_begin(self):
+            log.append("begin")
+
+        def capture_end(self):
+            log.append("end")
+
+    monkeypatch.setattr(engine, "_retired", type(engine._retired)(maxlen=2))
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", Graph)
+    monkeypatch.setattr(torch.cuda, "Stream", lambda dev: None)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: log.append("wait"))
+    monkeypatch.setattr(torch.cuda, "empty_cache", lambda: log.append("trim"))
+    failures = [1]
+
+    def step(self):
+        if failures:
+            failures.pop()
+            raise torch.OutOfMemoryError("no room")
+        log.append("step")
+
+    monkeypatch.setattr(DecodeSession, "_step", step)
+    old = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+    old.graph = Graph()
+    del old
+    sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+    sess.capture()
+    assert log == ["begin", "end", "free", "free", "wait", "trim", "begin", "step", "end"] and sess.graph is not None
+    sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+    failures += [1, 1]
+    with pytest.raises(torch.OutOfMemoryError):
+        sess.capture()
+    assert sess.graph is None and log.count("begin") == log.count("end") == 4
