@@ -24,7 +24,9 @@ ones.
 from __future__ import annotations
 
 import collections
+import contextlib
 import itertools
+import threading
 import weakref
 
 import torch
@@ -34,11 +36,42 @@ from .model import LLaMA, _Work, _enable_i8_handoff
 from .state import Rows
 
 
-# Captured graphs that nothing replays any more. Freeing one waits for the device; they are freed after the next capture, so that
-# a program's next prompt is launched while the last session's steps still run, and its first step captured while the prompt
-# runs. At most two are kept. Freed graphs leave what their steps allocated with the allocator, which gives it back after every
-# _TRIM captures (each time costs the next prompt its buffers anew: 7B gptq.int4, 8 prompts, 0.5 ms).
-_retired: collections.deque = collections.deque(maxlen=2)
+class _Retired:
+    """Captured graphs that nothing replays any more. Freeing one waits for the device; they are freed after the next capture, so that
+    a program's next prompt is launched while the last session's steps still run, and its first step captured while the prompt
+    runs. At most `maxlen` are kept, more only while a capture is underway: freeing a graph inside a capture, of whichever session,
+    thread or device, aborts it. `lock` is held by a capture and by whoever frees, so sessions of several threads capture one
+    after the other; dropping a graph never waits for it (a drop can come out of the garbage collector, anywhere)."""
+
+    def __init__(self, maxlen: int):
+        self.maxlen, self.graphs, self.lock, self.capturing = maxlen, collections.deque(), threading.RLock(), False
+
+    def append(self, graph) -> None:
+        self.graphs.append(graph)
+        self.clear(self.maxlen)
+
+    def clear(self, keep: int = 0) -> None:
+        """Free all but the `keep` newest; left to the end of a capture that is underway."""
+        if self.lock.acquire(blocking=False):
+            try:
+                while len(self.graphs) > keep and not self.capturing:
+                    self.graphs.popleft()
+            finally:
+                self.lock.release()
+
+    @contextlib.contextmanager
+    def capture(self):
+        with self.lock:
+            self.capturing = True
+            try:
+                yield
+            finally:
+                self.capturing = False
+
+
+# Freed graphs leave what their steps allocated with the allocator, which gives it back after every _TRIM captures (each time costs
+# the next prompt its buffers anew: 7B gptq.int4, 8 prompts, 0.5 ms).
+_retired = _Retired(maxlen=2)
 _TRIM = 16
 _captures = itertools.count(1)
 
@@ -283,7 +316,7 @@ class DecodeSession:
         blocks while a capture is underway: None if that found no room (`last`: the error instead)."""
         # (not torch.cuda.graph: it waits for the device, here the prompt, and empties the allocator's cache first)
         g, full = torch.cuda.CUDAGraph(), False
-        with torch.cuda.stream(torch.cuda.Stream(self.dev)):
+        with torch.cuda.stream(torch.cuda.Stream(self.dev)), _retired.capture():
             g.capture_begin()
             try:
                 self._step()
@@ -298,16 +331,17 @@ class DecodeSession:
     def capture(self):
         if self.graph is not None or not self.use_graph:
             return
-        g = self._record()
-        if g is None:
+        with _retired.lock:
+            g = self._record()
+            if g is None:
+                _retired.clear()
+                torch.cuda.synchronize()
+                torch.cuda.empty_cache()
+                g = self._record(last=True)
+            self.graph = g
             _retired.clear()
-            torch.cuda.synchronize()
-            torch.cuda.empty_cache()
-            g = self._record(last=True)
-        self.graph = g
-        _retired.clear()
-        if next(_captures) % _TRIM == 0:
-            torch.cuda.empty_cache()
+            if next(_captures) % _TRIM == 0:
+                torch.cuda.empty_cache()
 
     @torch.no_grad()
     def decode(self, n: int) -> None:

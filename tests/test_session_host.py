@@ -132,3 +132,60 @@ def test_capture_makes_room_once(monkeypatch):
     with pytest.raises(torch.OutOfMemoryError):
         sess.capture()
     assert sess.graph is None and log.count("begin") == log.count("end") == 4
+
+
+def test_graphs_dropped_during_a_capture_wait_for_its_end(monkeypatch):
+    """Sessions that end while another one captures, in its own thread (the garbage collector) or in others: their graphs are freed
+    after the capture, however many; two threads' captures follow each other."""
+    import contextlib
+    import threading
+
+    from lit_llama import engine
+
+    log, inside = [], []
+
+    class Graph:
+        def __init__(self):
+            weakref.finalize(self, lambda: log.append("freed inside" if inside else "free"))
+
+        def capture_begin(self):
+            assert not inside
+            inside.append(1)
+
+        def capture_end(self):
+            inside.pop()
+
+    def drop(n):
+        for _ in range(n):
+            sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+            sess.graph = Graph()
+            del sess
+
+    monkeypatch.setattr(engine, "_retired", type(engine._retired)(maxlen=2))
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", Graph)
+    monkeypatch.setattr(torch.cuda, "Stream", lambda dev: None)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "empty_cache", lambda: None)
+    other = [DecodeSession(_Model(HybridProgram), 1, 16, 16)]
+    threads = []
+
+    def step(self):
+        if not threads:
+            drop(4)
+            t = threading.Thread(target=drop, args=(4,))
+            t.start()
+            t.join(20)
+            assert not t.is_alive()  # (a drop does not wait for the capture)
+            threads.append(threading.Thread(target=other[0].capture))
+            threads[0].start()
+            threads[0].join(0.2)
+        log.append("step")
+
+    monkeypatch.setattr(DecodeSession, "_step", step)
+    sess = DecodeSession(_Model(HybridProgram), 1, 16, 16)
+    sess.capture()
+    threads[0].join(20)
+    assert sess.graph is not None and other[0].graph is not None
+    assert log.count("free") == 8 and log.count("step") == 2 and "freed inside" not in log
+    drop(3)
+    assert log.count("free") == 9  # two are kept
