@@ -407,7 +407,8 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
     return 0;
   }
   const bool f32 = dt == 1 || wkind == 0;  // bf16 rows on codes: the weight element (q - zero) * scale is fp32
-  int splits = ws ? gg_splits(M, N, K, f32, dt == 1 && K <= kGgFineK) : 1;
+  const bool fine = dt == 1 && K <= kGgFineK;  // fp32 operands: short chains of sums
+  int splits = ws ? gg_splits(M, N, K, f32, fine) : 1;
   if (splits > 1 && ws_bytes < (size_t)splits * M * N * 4) splits = 1;
   const int kt = kGgRow / (f32 ? 4 : 2), all = (K + kt - 1) / kt, per = (all + splits - 1) / splits;
   const int mt = (M + kGgBM - 1) / kGgBM, nt = (N + kGgBN - 1) / kGgBN;
@@ -418,13 +419,17 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
   const int el = dt == 1 ? 4 : 2;
   auto fits = [&](const void* p, int ld, int n) { return (uintptr_t)p % (n * el) == 0 && ld % n == 0 && K % n == 0; };
   // WL: loader of J accumulators per wave (512 / J threads)
-#define LLJ_GG_RUN(T, CT, VEX, J, FINE, ...)                                                                                  \
+#define LLJ_GG_GO(T, CT, VEX, J, FINE, HALVES, ...)                                                                           \
   do {                                                                                                                        \
     typedef __VA_ARGS__ wl;                                                                                                   \
-    hipLaunchKernelGGL((gg_kernel<wl, T, CT, VEX, J, FINE>), grid, dim3(512 / J), 0, s, (const T*)x, ldx, M, K, W, scales,    \
+    hipLaunchKernelGGL((gg_kernel<wl, T, CT, VEX, J, FINE, HALVES>), grid, dim3(512 / J), 0, s, (const T*)x, ldx, M, K, W, scales,    \
                        zeros, wkind == 1 ? K : group, N, (T*)y, ldy, (const T*)resid, ldr, part, per);                        \
   } while (0)
-  const bool fine = dt == 1 && K <= kGgFineK;
+#define LLJ_GG_RUN(T, CT, VEX, J, FINE, ...)                                                      \
+  do {                                                                                            \
+    if (FINE && splits == 1 && all >= 8) LLJ_GG_GO(T, CT, VEX, J, FINE, FINE, __VA_ARGS__);       \
+    else LLJ_GG_GO(T, CT, VEX, J, FINE, false, __VA_ARGS__);                                      \
+  } while (0)
 #define LLJ_GG_F32(VE)                                                      \
   do {                                                                      \
     if (fine) LLJ_GG_RUN(float, float, VE, 1, true, GgWeightDense<float, VE, 512>); \
@@ -459,6 +464,7 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
 #undef LLJ_GG_BF16
 #undef LLJ_GG_F32
 #undef LLJ_GG_RUN
+#undef LLJ_GG_GO
   if (part) {
     LLJ_CHECK_LAUNCH();
     const size_t blocks = ((size_t)M * N + 255) / 256;

@@ -18,7 +18,8 @@
 //
 // fp32 sums are no further from exact ones than the per-lane sums of K / 64 terms that they replace (2-norm error against
 // float64, random operands): from K = kGgFineK down an accumulator runs over 8 values of K, four of those are added pairwise, four of
-// these sums in a second and the rest in a third accumulator; above it 32 values, eight of those, and the rest.
+// these sums in a second and the rest in a third accumulator, and from 8 tiles on each half of K by itself (K = 780: error 9.5e-8
+// in one piece, 9.0e-8 in two or more, 9.3e-8 before); above it 32 values, eight of those, and the rest.
 #pragma once
 #include "common.h"
 #include "elem.h"
@@ -31,6 +32,7 @@ constexpr int kGgBM = 64, kGgBN = 128;
 constexpr int kGgRow = 128;  // bytes of one operand row in LDS
 constexpr int kGgMaxSplit = 16;
 constexpr int kGgFineK = 3071;
+constexpr size_t kGgForced = (size_t)128 << 20;  // most scratch of two ranges that are not there for speed
 
 __device__ __forceinline__ f32x16 gg_mma(f32x4 a, f32x4 b, f32x16 c, float) {
 #pragma unroll
@@ -131,10 +133,11 @@ struct GgWeightCodes {
 };
 
 // WL: the weight tile's loader; T: activations and output, CT: compute type, VEX: elements per load of x, J: accumulators per wave.
-// part (splits > 1): this split's fp32 sums at [split][M][N], summed by gg_reduce_kernel. FINE: short chains of sums (above).
+// part (splits > 1): this split's fp32 sums at [split][M][N], summed by gg_reduce_kernel. FINE: short chains of sums (above), HALVES:
+// those of each half of K by themselves.
 // Blocks: (8 * ceil(column tiles / 8) * row tiles, splits); block b runs on XCD b % 8, whose L2 keeps a column tile's weights
 // for its row tiles.
-template <typename WL, typename T, typename CT, int VEX, int J, bool FINE>
+template <typename WL, typename T, typename CT, int VEX, int J, bool FINE, bool HALVES>
 __global__ __launch_bounds__(512 / J) void gg_kernel(const T* __restrict__ x, int ldx, int M, int K, const void* __restrict__ W,
                                                      const float* __restrict__ sc, const float* __restrict__ zr, int group,
                                                      int N, T* __restrict__ y, int ldy, const T* resid, int ldr,
@@ -165,12 +168,20 @@ __global__ __launch_bounds__(512 / J) void gg_kernel(const T* __restrict__ x, in
     w.store(b + kGgBM * kGgRow, group, G, t * KT, K, tid);
   };
 
-  f32x16 acc[J] = {}, mid[J] = {}, tot[J] = {};
+  f32x16 acc[J] = {}, mid[J] = {}, tot[J] = {}, front[J] = {};
+  const int th = HALVES ? t0 + (t1 - t0 + 1) / 2 : t1;  // the second half's first tile
   const int nw = (wave >> 1) * 32 * J;  // the wave's first column
   const int ra = gg_at((wave & 1) * 32 + (lane & 31), lane >> 5), rb = gg_at(kGgBM + nw + (lane & 31), lane >> 5);
   fetch(t0);
   stage(t0);
   for (int t = t0; t < t1; ++t) {
+    if (HALVES && t == th) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        front[j] = tot[j] + mid[j];
+        tot[j] = mid[j] = f32x16{};
+      }
+    }
     __syncthreads();  // tile t is staged, and every wave is done with the other buffer
     if (t + 1 < t1) fetch(t + 1);
     const char* b = lds[t & 1];
@@ -199,7 +210,7 @@ __global__ __launch_bounds__(512 / J) void gg_kernel(const T* __restrict__ x, in
         }
       }
     }
-    if (sizeof(CT) == 4 && ((t - t0) & (FINE ? 3 : 7)) == (FINE ? 3 : 7)) {
+    if (sizeof(CT) == 4 && ((t - (HALVES && t >= th ? th : t0)) & (FINE ? 3 : 7)) == (FINE ? 3 : 7)) {
 #pragma unroll
       for (int j = 0; j < J; ++j) {
         tot[j] += mid[j];
@@ -212,6 +223,7 @@ __global__ __launch_bounds__(512 / J) void gg_kernel(const T* __restrict__ x, in
   for (int j = 0; j < J; ++j) {
     if constexpr (sizeof(CT) == 4) tot[j] += mid[j];
     else tot[j] = acc[j];
+    if constexpr (HALVES) tot[j] = front[j] + tot[j];
     const int n = n0 + nw + 32 * j + (lane & 31);
     if (n >= N) continue;
 #pragma unroll
@@ -250,15 +262,17 @@ __global__ __launch_bounds__(256) void gg_reduce_kernel(const float* __restrict_
 
 // K ranges of a product: what makes the last round of workgroups over the 256 CUs cheapest, against the partial sums'
 // traffic and launch. Microseconds: a tile step at the MFMA rate of one CU (0.9 fp32, 0.2 bf16), partials
-// written and read at 4.9 TB/s, 3 for the second launch. fine (fp32 operands, K <= kGgFineK): at least two ranges, for the
-// shorter sums (K = 780: error 9.5e-8 in one, 9.0e-8 in more, 9.3e-8 before).
+// written and read at 4.9 TB/s, 3 for the second launch. fine (fp32 operands, K <= kGgFineK): at least two ranges while their scratch
+// is small, for the shorter sums; larger outputs keep the halves apart inside one workgroup (HALVES). fp32, K = 780, us in two
+// ranges / in halves: 1000 x 2304 77 / 96, 100 x 35008 120 / 143, 300 x 35008 (80 MiB of scratch) 264 / 284, 1000 x 35008
+// (267 MiB) 875 / 842, 2048 x 35008 1757 / 1647.
 inline int gg_splits(int M, int N, int K, bool f32, bool fine) {
   const int KT = kGgRow / (f32 ? 4 : 2), all = (K + KT - 1) / KT;
   const long tiles = (long)((M + kGgBM - 1) / kGgBM) * ((N + kGgBN - 1) / kGgBN);
   const double step = f32 ? 0.9 : 0.2;
   int best = 1;
   double least = 0;
-  for (int s = fine && all >= 8 ? 2 : 1; s <= kGgMaxSplit && s <= all; ++s) {
+  for (int s = fine && all >= 8 && (size_t)M * N * 8 <= kGgForced ? 2 : 1; s <= kGgMaxSplit && s <= all; ++s) {
     const int per = (all + s - 1) / s;
     if ((all + per - 1) / per != s) continue;
     const double us = (double)((tiles * s + 255) / 256) * per * step + (s > 1 ? 3.0 + s * (double)M * N * 8 / 4.9e6 : 0.0);

@@ -228,6 +228,32 @@ def _g_linear_operands(kind, bits, group, dt, M, K, N, ldx, seed):
     return buf, packed, sc, zr, (q.double() - zr[:, cols].double()) * sc[:, cols].double()
 
 
+@pytest.mark.parametrize("kind,bits", [(1, 16), (0, 4), (0, 8)])
+def test_generic_gemm_fp32_halves_need_no_scratch(kind, bits):
+    """fp32, short K: the sums of the two halves of K are kept apart inside one workgroup (the same bits as the two halves' own
+    products, 7 tiles each, added), so large outputs take no scratch: twice the output's size for a head's logits otherwise."""
+    from lit_llama import _hip
+
+    for M in (1000, 2048, 16384):
+        assert _hip.lib().llj_g_linear_ws_bytes(kind, M, 35008, 780, 1) == 0
+    M, N, K, group = 77, 300, 448, 32
+    buf, w, sc, zr, _ = _g_linear_operands(kind, bits, group, 1, M, K, N, K, 5)
+    x = buf[:M * K].view(M, K)
+
+    def product(a, w, sc, zr):
+        y = torch.empty(M, N, device="cuda")
+        _hip.call("llj_g_linear", kind, a.data_ptr(), a.stride(0), M, a.shape[1], w.data_ptr(), _hip.ptr(sc), _hip.ptr(zr), bits, group, N,
+                  y.data_ptr(), N, None, 0, 1, _hip.stream())
+        return y
+
+    half = []
+    for lo, hi in ((0, 224), (224, 448)):
+        ww = w[:, lo:hi] if kind == 1 else w[lo * bits // 8:hi * bits // 8]
+        s = (None, None) if kind == 1 else (sc[:, lo // group:hi // group].contiguous(), zr[:, lo // group:hi // group].contiguous())
+        half.append(product(x[:, lo:hi], ww.contiguous(), *s))
+    assert torch.equal(product(x, w, sc, zr), half[0] + half[1])
+
+
 @pytest.mark.parametrize("kind,bits,group", [(1, 16, 0), (0, 2, 0), (0, 4, 0), (0, 8, 0), (0, 4, 100)])
 @pytest.mark.parametrize("dt", [0, 1])
 @pytest.mark.parametrize("M,N,K,pad,off", [(9, 1, 4, 0, 0), (9, 127, 32, 0, 0), (64, 128, 36, 4, 0), (65, 129, 780, 0, 0),
