@@ -647,6 +647,8 @@ class LLaMA(nn.Module):
         M, L = B * T, _hip.lib()
         norm = bool(L.llj_g_norm_ok(M, C, w.dt))
         step = T == 1 and bool(L.llj_g_rope_attention_ok(S, C // nh))
+        # (it reads pairs; caches of the caller's own may start anywhere)
+        step = step and not any((k.data_ptr() | v.data_ptr()) % (2 * k.element_size()) for k, v in kv)
         for i, blk in enumerate(self.transformer.h):
             sa, sp, s1, s2, sd = specs["layers"][i]
             kc, vc = kv[i]

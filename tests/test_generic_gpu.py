@@ -98,6 +98,25 @@ def test_125m_generate_graph_matches_eager_and_wraps():
     assert outs[0].shape == (28,) and ((outs[0] >= 0) & (outs[0] < C125.vocab_size + 64)).all()
 
 
+@pytest.mark.parametrize("odd", ["keys", "values"])
+def test_decode_over_caches_at_odd_places(odd):
+    """Caches that the caller laid out, starting at an odd element (decode rows on the fused launch read pairs): the same logits
+    as over the model's own, to the rounding of the separate launches."""
+    m, _ = _setup(REF_TEST, None, 9)
+    ids = torch.from_numpy(np.random.default_rng(4).integers(0, REF_TEST.vocab_size, (2, 9))).cuda()
+    outs = []
+    for own in (True, False):
+        m.reset_cache()
+        if not own:
+            for k, v in m._alloc_kv(2, 16, ids.device):
+                at = torch.zeros(k.numel() + 1, dtype=k.dtype, device=k.device)[1:].view(k.shape)
+                m.kv_caches.append((at, v) if odd == "keys" else (k, at))
+        m(ids[:, :8], 16, torch.arange(8).cuda())
+        outs.append(m(ids[:, 8:], 16, torch.tensor([8]).cuda()).float())
+    m.reset_cache()
+    assert float((outs[0] - outs[1]).norm() / outs[0].norm()) < 2e-2
+
+
 def test_decode_on_a_device_full_of_cached_blocks(monkeypatch):
     """A step that allocates where everything the process may use lies in the allocator's cache (after a large prompt): the capture
     makes room, and the tokens are those of eager steps."""
