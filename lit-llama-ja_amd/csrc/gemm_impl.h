@@ -272,9 +272,13 @@ constexpr size_t gemm_lds_bytes() {
 }
 
 // BM: rows per tile (128, or 256 for bf16 with 8 waves: 4 row groups x 2 column groups of 64 x 64)
-// (two waves per SIMD: two 128-row workgroups per CU; gptq.int8 and grouped int4 took 268 and 324 registers without the bound)
+// Two waves per SIMD: two 128-row workgroups per CU (grouped int4 took 324 registers without the bound: 1000 rows 4096 -> 12288 246
+// us, 175 with it). Unsplit gptq.int8 fits 256 registers by itself and spills 16 under the bound: 512 rows without / with it,
+// 4096 -> 12288 111 / 116 us, 11008 -> 4096 190 / 200.
+template <int WF, int EP>
+constexpr int gemm_waves = WF == GWF_W8 && EP != GEP_SPLIT ? 1 : 2;
 template <int WF, int EP, int BM = kGBM>
-__global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_waves<WF, EP>))) void gemm_kernel(GemmParams p) {
   static_assert(BM == kGBM || WF == GWF_BF16 || WF == GWF_I8 || WF == GWF_W4, "256-row tiles: bf16, int8, int4");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr bool NIB = WF == GWF_W4 || WF == GWF_W8;  // nibble-coded: offset removed with the A row sums
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
   u32x4 areg[GDEPTH][4], breg[GDEPTH][BV];
   float2 szr[GDEPTH][4];  // GWF_W4G: (scale, 128 + zero) of the chunk's group for the lane's column of tile j
   auto load_chunk = [&](int slot, int c) {
-    c = c0 + (c < KC ? c : KC > 0 ? KC - 1 : 0);  // past the end: a valid duplicate, never stored
+    c = c0 + (c < KC ? c : SPLIT && I8 && KC == 0 ? 0 : KC - 1);  // past the end: a valid duplicate, never stored
     if constexpr (I8) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) areg[slot][v] = *reinterpret_cast<const u32x4*>(aqsrc + (size_t)c * 128 + 16 * v);
