@@ -578,7 +578,7 @@ static int sample_launch(const T* logits, int ldl, int M, int V, float temperatu
   if ((size_t)stride * kSampNT * KB > kSampRow) stride = 0;
   static const hipError_t set =
       hipFuncSetAttribute((const void*)sample_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSampRow);
-  if (set != hipSuccess) return -(int)set;
+  if (set != hipSuccess) return (int)set;
   hipLaunchKernelGGL(sample_kernel<T>, dim3(M), dim3(kSampNT), (size_t)stride * kSampNT * KB, s, logits, ldl, V, 1.f / temperature,
                      temperature, top_k, u, seed, out_idx, tokens_out, tok_stride, pos, pos_step, stride);
   LLJ_CHECK_LAUNCH();
