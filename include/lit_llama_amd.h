@@ -482,8 +482,8 @@ int llj_rows_linear(int act, const void* A, int lda, const void* W, const float*
  * == 0, C <= 8192), out = act(bf16(x_out) . W^T). x_out must not be x. */
 int llj_post_linear(int act, const void* t, const void* norm_w, float eps, const float* x, float* x_out, int C,
                     const void* W, void* out, int N, int K, void* stream);
-/* C = act(A . W^T + bias) for many bf16 rows on the prefill GEMM (N, K multiples of 128); ws (act 0, optional,
- * llj_gemm_bf16_ws_bytes bytes): K split over workgroups when the row tiles leave most CUs idle. */
+/* C = act(A . W^T + bias) for many bf16 rows on the prefill GEMM (N, K multiples of 128); ws (optional, act 0 or fewer
+ * than 256 rows, llj_gemm_bf16_ws_bytes bytes): K split over workgroups when the row tiles leave most CUs idle. */
 size_t llj_gemm_bf16_ws_bytes(int M, int N, int K);
 int llj_gemm_bf16(int act, const void* A, int lda, const void* W, const float* bias, void* C, int ldc, int M, int N, int K,
                   float limit, float alpha, void* ws, size_t ws_bytes, void* stream);

@@ -61,10 +61,6 @@ __device__ __forceinline__ void softmax_merge(float& mx, float& l, float* o, con
 template <int HS>
 constexpr int kAttPart = HS + 4;  // floats per partial record: HS outputs, max, sum, 2 pad (16-byte records)
 
-// count (with PART, else partials only; nsplit <= 64): zeroed arrival counters, one per (row, head), left zero: the last of the
-// ranges' blocks to finish merges them. The hand-off is device-scope stores, a wait for them, the counter, device-scope
-// loads; no block waits for another.
-
 // y[m, h * HS + d] of thread d < HS, adjacent dims as one 4-byte store; with st the LLM.int8 statistics of y, one slot per head
 template <int HS>
 __device__ __forceinline__ void attention_out(float v, bf16_t* __restrict__ y, uint32_t* st, float thr, int h, int m, int C) {
@@ -74,6 +70,9 @@ __device__ __forceinline__ void attention_out(float v, bf16_t* __restrict__ y, u
   if (st) i8_emit_stats64(st, thr, m, h * HS + (d & ~63), ob, h);  // (uniform)
 }
 
+// count (with PART, else partials only; nsplit <= 64): zeroed arrival counters, one per (row, head), left zero: the last of the
+// ranges' blocks to finish merges them. The hand-off is device-scope stores, a wait for them, the counter, device-scope
+// loads; no block waits for another.
 template <int HS, int U, int NTH, bool PART = false, int SPECU = U / 2, bool ILV = false>
 __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                const bf16_t* __restrict__ vc, bf16_t* __restrict__ y,

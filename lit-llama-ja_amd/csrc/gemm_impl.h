@@ -753,9 +753,14 @@ static int gemm_launch(const GemmParams& p, hipStream_t s) {
 // K slices of a product of less than 256 rows (128-row tiles): such a product has 32..172 tiles at 7B widths, one workgroup
 // each with a chain of K / 64 chunk loads, far from the memory and the matrix rate. Returns the slices (1: none), kcs = chunks each.
 // The rule weighs, in us, the chunks of the busiest CU (one chunk of one workgroup; two workgroups on a CU take 1.5, four 3 times
-// as long) against the second launch and the partial sums, and splits for a gain of a tenth. Measured at 128 / 154 rows, us unsplit ->
-// split (slices): 4096 -> 12288 int4 49 -> 39 (4), bf16 123 -> 62 (4), llm.int8 58 -> 33 (4), gptq.int8 80 -> 73 (2);
-// 11008 -> 4096 int4 121 -> 37 (12), bf16 325 -> 89 (8), llm.int8 119 -> 40 (8), gptq.int8 198 -> 58 (8).
+// as long) against the second launch and the partial sums, and splits for a gain of a tenth. What it chooses, us unsplit -> (slices) us:
+//                   4096 -> 12288, 128 rows    154 rows            11008 -> 4096, 128 rows    154 rows
+//   int4            58 -> (2) 42               61 -> (1) 50        148 -> (8) 38              149 -> (8) 46
+//   bf16            122 -> (5) 54              117 -> (4) 91       346 -> (15) 57             329 -> (8) 82
+//   llm.int8        60 -> (4) 32               53 -> (1) 53        142 -> (8) 35              126 -> (8) 40
+//   gptq.int8       74 -> (5) 46               76 -> (4) 66        187 -> (8) 43              187 -> (8) 58
+//   int4 groups     81 -> (5) 42               82 -> (4) 61        210 -> (8) 42              210 -> (8) 56
+// (unsplit: before the slices and the two-waves bound, which alone took int4 at 154 rows from 61 to 50)
 static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out) {
   if (M >= 256 || M < 1 || N % kGBN || K < kGBK) return 1;
   const int KC = wf == GWF_I8 ? K / 128 : K / kGBK, planes = wf == GWF_I8 ? 1 : 0;

@@ -170,7 +170,8 @@ static int rows_gemv_go(const PostGemvParams& p, hipStream_t s) {
 
 template <int MG, int ACT>
 static int rows_gemv_k(const PostGemvParams& p, hipStream_t s) {
-  const int KC = p.K / 128;  // chunks; S: the least that covers them
+  const int KC = p.K / 128;  // chunks; S: the least built that covers them (8 rows against the 16x16 form inside the steps: 3072 -> 3072
+                             // 10.7 -> 7.3 us, 5120 -> 5120 22.4 -> 12.9, 17408 -> 512 20.7 -> 13.6)
   if (KC <= 8) return rows_gemv_go<2, 4, 4, MG, ACT>(p, s);
   if (KC <= 16) return rows_gemv_go<4, 4, 4, MG, ACT>(p, s);
   if (KC <= 32) return rows_gemv_go<8, 4, 4, MG, ACT>(p, s);
@@ -342,7 +343,7 @@ static int post_gemv_launch(const PostGemvParams& p, int act, hipStream_t s) {
   }
 }
 
-constexpr int kPostMaxK = 28544;  // widest weight rows of the post form (its row lies in LDS) and of the streams form
+constexpr int kPostMaxK = 28544;  // widest weight rows of the post form, whose row lies in LDS; llj_streams_linear keeps the same limit
 
 template <int PRO>
 static int rowdot_act(const RowDotParams& r, int act, hipStream_t s) {
