@@ -302,10 +302,10 @@ int llj_i8_quant_weight(const void* W, int dtype, void* CB, void* SCB, int N, in
  * (quantize_weight, 470-473), propagate each column's error through the block with Hinv1 =
  * hinv[i1:i1+128, i1:i1+128] (593). wt: the (permuted, running) weight TRANSPOSED, (K, N) fp32,
  * its block rows updated in place; qt (K, N): reconstructions scale*(q - zero) of the block's
- * rows; err (128, N): Err1; loss[n] += Σ_i (w - q)² / d² (Losses1 before the / 2). hinv: (K, K)
+ * rows; err (128, N): Err1; loss[n] += Σ_i ((w - q) / d)² (Losses1 before the / 2). hinv: (K, K)
  * fp32 upper Cholesky factor of H⁻¹. Requires i1 % 128 == 0, i1 + 128 <= K, bits in {2,4,8}.
  * Each fp32 op rounded on its own in the reference's order (bitwise the reference's loop). The
- * trailing update W[:, i2:] -= Err1 · Hinv[i1:i2, i2:] is a plain GEMM left to the caller. */
+ * trailing update W[:, i2:] -= Err1 · Hinv[i1:i2, i2:] is llj_gptq_update. */
 int llj_gptq_block(const float* hinv, int K, int i1, float* wt, int N, const float* scale, const float* zero,
                    int bits, float* qt, float* err, float* loss, void* stream);
 /* llj_gptq_block for GPTQQuantizer(blocksize=b) (quantization.py:437, 557-596): the column loop over
@@ -313,11 +313,26 @@ int llj_gptq_block(const float* hinv, int K, int i1, float* wt, int N, const flo
  * i1 + b <= K. llj_gptq_block is this with b = 128. */
 int llj_gptq_block_bs(const float* hinv, int K, int i1, int blocksize, float* wt, int N, const float* scale,
                       const float* zero, int bits, float* qt, float* err, float* loss, void* stream);
+/* GPTQQuantizer.find_params_weight (475-514), per channel: (scale, zero) of N rows of K fp32 weights; sym: the symmetric range. */
+int llj_gptq_params(const float* w, int N, int K, int bits, int sym, float* scale, float* zero, void* stream);
+/* collect_input_stats (516-530): H = keep H + (alpha x)^T (alpha x), x (T, K) row-major, dt 0 = bf16, 1 = fp32, H (K, K) fp32
+ * symmetric. Any T, K; fp32 sums over the rows in order. */
+int llj_gptq_gram(const void* x, int dt, int T, int K, float keep, float alpha, float* H, void* stream);
+/* W (N, K) in the loop's layout and column order: wt (K, N) with wt[place[k]][n] = W[n][k] (place NULL: k), zero for dead[k]. */
+int llj_gptq_weight(const float* W, const int64_t* place, const void* dead, int N, int K, float* wt, void* stream);
+/* hinv = M on return: the upper Cholesky factor of (H[perm][:, perm] + damp I)^-1 (549-566), zeros below. K % 128 == 0, H is not
+ * changed. P: K x K floats of scratch, xt: 128 x 128, all on 16 bytes; *info = 1 if a pivot is not positive (M is then unusable). */
+int llj_gptq_factor(const float* H, const int64_t* perm, const float* damp, int K, float* M, float* P, float* xt, int* info, void* stream);
+/* W[:, i2:] -= Err1 Hinv[i1:i2, i2:] (596) behind a block of `blocksize` columns, transposed as llj_gptq_block keeps it. */
+int llj_gptq_update(const float* hinv, int K, int i1, int blocksize, const float* err, int N, float* wt, void* stream);
 /* ColBlockQuantizedLinear.pack_weight (quantization.py:374-388) from reconstructions qt (K, N)
  * fp32: code = uint8(clamp(q / scale + zero, 0, 2^bits - 1)) (truncating), entries_per_byte =
  * 8/bits codes per byte; qw is quant_weight in its column-major storage: byte (n, j) at j*N + n. */
 int llj_colblock_pack(const float* qt, int K, int N, const float* scale, const float* zero, int bits,
                       unsigned char* qw, void* stream);
+/* The same where column k is row order[k] of qt (order NULL: k). */
+int llj_colblock_pack_order(const float* qt, const int64_t* order, int K, int N, const float* scale, const float* zero, int bits,
+                            unsigned char* qw, void* stream);
 
 /* ---------------------------------------------------------------- small ops */
 /* out[m] = wte[idx[m]] (model.py:110), any C; if pos_inc != NULL, *pos_inc += 1 (device-side

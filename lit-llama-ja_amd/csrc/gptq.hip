@@ -4,9 +4,9 @@
 // the device, host side); what is specific to GPTQ is the sequential column loop inside a
 // 128-column block (quantization.py:568-596) and the ColBlock packing (pack_weight, 374-388).
 //
-// llj_gptq_block(_bs): 8 or 4 lanes per weight row (rows are independent inside a block: the update of
+// llj_gptq_block(_bs): 16 or 4 lanes per weight row (rows are independent inside a block: the update of
 // row r uses only its own error and the shared Hinv1 rows). The block's 128 columns of each row
-// and Hinv1^T sit in LDS (32 or 64 rows per workgroup: 20 + 66 KiB); 16 columns at a time are quantized
+// and Hinv1 sit in LDS (16 or 64 rows per workgroup: 10 / 40 + 66 KiB); 16 columns at a time are quantized
 // in registers, then the rest of the block takes their 16 updates per column in one LDS round
 // trip, the columns split over the row's lanes. Weights are passed
 // transposed (Wt: K x N, element (k, n) at k * N + n) so column i of 128 rows is one coalesced load.
@@ -22,42 +22,23 @@ namespace llj {
 constexpr int kGptqBlock = 128;
 
 constexpr int kGptqSub = 16;          // columns held in registers at a time
-// Two shapes, picked by N at launch (both 256 threads, one workgroup per CU by LDS):
-//   kGptqRows = 32 rows x 8 lanes, W1^T row stride 40: lane l's column j = b + 16 + l + 8k lands
-//     40 l (mod 64) banks over -> the 8 lanes x 8 rows of a wavefront hit 64 distinct banks;
-//   kGptqRows = 64 rows x 4 lanes, stride 80 (80 l mod 64 = 16 l; 16 rows per wavefront),
-//     for N > 8192 so N / 64 workgroups still fit the 256 CUs in one round.
-constexpr int kHs = kGptqBlock + 1;   // LDS row stride of Hinv1^T (odd: conflict-free staging)
+constexpr int kHs = kGptqBlock + 4;   // LDS row stride of Hinv1 (rows start on 16 bytes)
 
-// Each row's 16-column quantization group is computed redundantly by all kGptqLanes lanes of the
-// row (identical inputs, identical fp32 ops -> identical e[u]); the trailing update of the block's
-// remaining columns is split over the lanes (column j to lane (j - b - 16) % kGptqLanes). Every
-// column still receives the same updates in the same order, so results are unchanged bit for bit;
-// the serial chain per block shrinks from 16 + 112 updates to 16 + 14 (16 + 28) and N / 32
-// (N / 64) workgroups fill the chip (N / 128 single-lane workgroups used 32-96 CUs at 7B shapes).
-template <int kGptqRows, int kGptqLanes, int kWs>
-__global__ __launch_bounds__(kGptqRows * kGptqLanes) void gptq_block_kernel(const float* __restrict__ hinv, int K, int i1,
-                                                                  int blk,
-                                                                  float* __restrict__ wt, int N,
-                                                                  const float* __restrict__ scale,
-                                                                  const float* __restrict__ zero, float maxq,
-                                                                  float* __restrict__ qt, float* __restrict__ err,
-                                                                  float* __restrict__ loss) {
-  __shared__ float hsT[kGptqBlock * kHs];              // hsT[j * kHs + i] = Hinv1[i][j]
-  __shared__ float ws[kGptqBlock * kWs];               // ws[j * kWs + t] = W1[row t][j]
-  constexpr int kGptqThreads = kGptqRows * kGptqLanes;
-  const int tid = threadIdx.x;
-  const int t = tid / kGptqLanes, l = tid % kGptqLanes;
-  for (int v = tid; v < blk * blk; v += kGptqThreads) {
-    const int i = v / blk, j = v % blk;
-    hsT[j * kHs + i] = hinv[(size_t)(i1 + i) * K + i1 + j];
-  }
-  const int n = blockIdx.x * kGptqRows + t;
-  const int nn = n < N ? n : N - 1;  // clamped: loads stay in bounds, stores are guarded
-  const float s = scale[nn], z = zero[nn];
-  for (int j = l; j < blk; j += kGptqLanes) ws[j * kWs + t] = wt[(size_t)(i1 + j) * N + nn];
-  __syncthreads();
-  const bool writer = l == 0 && n < N;
+// a / b, correctly rounded, from y = 1 / b correctly rounded: two residual steps. The first makes the quotient faithful, the
+// second then gives the rounded one (Markstein, "Computation of elementary functions on the IBM RISC System/6000", 1990), for
+// operands whose residuals do not underflow. A third of the division sequence's instructions, and no dependent reciprocal.
+__device__ __forceinline__ float div_by(float a, float b, float y) {
+  float q = __fmul_rn(a, y);
+  q = __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+}
+__device__ __forceinline__ bool divides(float b) { return fabsf(b) > 0x1p-40f && fabsf(b) < 0x1p40f; }
+
+// One block of one row's columns (see gptq_block_kernel). FAST: every divisor is in div_by's range.
+template <int LANES, int kWs, bool FAST>
+__device__ __forceinline__ float gptq_columns(const float* hs, const float* rd, float* ws, int t, int l, int blk, float s, float z, float maxq,
+                                              bool writer, float* __restrict__ q_out, float* __restrict__ e_out, size_t N) {
+  const float rs = __fdiv_rn(1.f, s);
   float lsum = 0.f;
   for (int b = 0; b < blk; b += kGptqSub) {
     float r[kGptqSub], e[kGptqSub];
@@ -65,44 +46,98 @@ __global__ __launch_bounds__(kGptqRows * kGptqLanes) void gptq_block_kernel(cons
     for (int u = 0; u < kGptqSub; ++u) r[u] = ws[(b + u) * kWs + t];
 #pragma unroll
     for (int u = 0; u < kGptqSub; ++u) {
-      const int i = b + u;
-      const float w = r[u];
-      const float d = hsT[i * kHs + i];
+      const float* h = hs + (b + u) * kHs + b;  // Hinv1[b + u][b ..]: the same address in every lane
+      const float w = r[u], d = h[u];
       // quantize_weight (quantization.py:470-473): clamp(round(x / scale) + zero, 0, maxq)
-      const float qi = fminf(fmaxf(__fadd_rn(rintf(__fdiv_rn(w, s)), z), 0.f), maxq);
+      const float x = FAST ? div_by(w, s, rs) : __fdiv_rn(w, s);
+      const float qi = fminf(fmaxf(__fadd_rn(rintf(x), z), 0.f), maxq);
       const float q = __fmul_rn(s, __fsub_rn(qi, z));
       const float dq = __fsub_rn(w, q);
-      lsum = __fadd_rn(lsum, __fdiv_rn(__fmul_rn(dq, dq), __fmul_rn(d, d)));  // Losses1 (590)
-      e[u] = __fdiv_rn(dq, d);                                                  // err1 (592)
+      e[u] = FAST ? div_by(dq, d, rd[b + u]) : __fdiv_rn(dq, d);  // err1 (592)
+      lsum = __fadd_rn(lsum, __fmul_rn(e[u], e[u]));               // Losses1 (590): (w - q)^2 / d^2
       if (writer) {
-        qt[(size_t)(i1 + i) * N + n] = q;
-        err[(size_t)i * N + n] = e[u];
+        q_out[(size_t)(b + u) * N] = q;
+        e_out[(size_t)(b + u) * N] = e[u];
       }
       // W1[:, i:] -= err1 (x) Hinv1[i, i:] (593) inside the register group (columns <= i are
       // never read again)
 #pragma unroll
-      for (int v = u + 1; v < kGptqSub; ++v) r[v] = __fsub_rn(r[v], __fmul_rn(e[u], hsT[(b + v) * kHs + i]));
+      for (int v = u + 1; v < kGptqSub; ++v) r[v] = __fsub_rn(r[v], __fmul_rn(e[u], h[v]));
     }
     __syncthreads();  // every lane has read the group's columns before any lane rewrites ws
     // the rest of the block, column by column: the group's updates in increasing i, as the
     // reference applies them one column i at a time
-    for (int j = b + kGptqSub + l; j < blk; j += kGptqLanes) {
+    for (int j = b + kGptqSub + l; j < blk; j += LANES) {
       float acc = ws[j * kWs + t];
-      const float* hc = hsT + j * kHs + b;  // Hinv1[b .. b+15][j]
 #pragma unroll
-      for (int u = 0; u < kGptqSub; ++u) acc = __fsub_rn(acc, __fmul_rn(e[u], hc[u]));
+      for (int u = 0; u < kGptqSub; ++u) acc = __fsub_rn(acc, __fmul_rn(e[u], hs[(b + u) * kHs + j]));
       ws[j * kWs + t] = acc;
     }
     __syncthreads();  // the next group's columns are complete
   }
-  if (writer) loss[n] += lsum;
+  return lsum;
+}
+
+// Each row's 16-column quantization group is computed redundantly by all LANES lanes of the
+// row (identical inputs, identical fp32 ops -> identical e[u]); the trailing update of the block's
+// remaining columns is split over the lanes (column j to lane (j - b - 16) % LANES). Every
+// column still receives the same updates in the same order, so results are unchanged bit for bit.
+//
+// Bound: the chain of dependent instructions of a column, two divisions in it, times 128. 16 rows x 16 lanes put N = 4096 on
+// all 256 CUs (32 x 8: on half of them); above N = 8192 64 x 4 keep the workgroups of one round. kWs spreads a wavefront's
+// lanes x rows over the 64 banks (20 l + t, 80 l + t mod 64). us a block, before (32 x 8, three division sequences a column; 64 x 4
+// above 8192): N = 4096 52 and 34, 8192 54 and 38, 11008 63 and 54 (32 x 8 there: 79), 35008 196 and 169.
+template <int ROWS, int LANES, int kWs>
+__global__ __launch_bounds__(ROWS * LANES) void gptq_block_kernel(const float* __restrict__ hinv, int K, int i1,
+                                                                  int blk,
+                                                                  float* __restrict__ wt, int N,
+                                                                  const float* __restrict__ scale,
+                                                                  const float* __restrict__ zero, float maxq,
+                                                                  float* __restrict__ qt, float* __restrict__ err,
+                                                                  float* __restrict__ loss) {
+  __shared__ __align__(16) float hs[kGptqBlock * kHs];  // hs[i * kHs + j] = Hinv1[i][j]
+  __shared__ float ws[kGptqBlock * kWs];                // ws[j * kWs + t] = W1[row t][j]
+  __shared__ float rd[kGptqBlock];                      // 1 / Hinv1[i][i]
+  constexpr int NT = ROWS * LANES;
+  const int tid = threadIdx.x;
+  const int t = tid / LANES, l = tid % LANES;
+  const int n = blockIdx.x * ROWS + t;
+  const int nn = n < N ? n : N - 1;  // clamped: loads stay in bounds, stores are guarded
+  const float s = scale[nn], z = zero[nn];
+  bool fast = divides(s);
+  if (tid < blk) {
+    const float d = hinv[(size_t)(i1 + tid) * K + i1 + tid];
+    rd[tid] = __fdiv_rn(1.f, d);
+    fast = fast && divides(d);
+  }
+  if (((K | i1) & 3) == 0 && ((uintptr_t)hinv & 15) == 0) {
+    for (int v = tid; v < blk * (blk / 4); v += NT) {
+      const int i = v / (blk / 4), j = v % (blk / 4) * 4;
+      *reinterpret_cast<f32x4*>(hs + i * kHs + j) = *reinterpret_cast<const f32x4*>(hinv + (size_t)(i1 + i) * K + i1 + j);
+    }
+  } else {
+    for (int v = tid; v < blk * blk; v += NT) hs[v / blk * kHs + v % blk] = hinv[(size_t)(i1 + v / blk) * K + i1 + v % blk];
+  }
+  // a wavefront reads runs of ROWS neighbouring rows of the matrix
+  for (int v = tid; v < blk * ROWS; v += NT) {
+    const int j = v / ROWS, m = min((int)blockIdx.x * ROWS + v % ROWS, N - 1);
+    ws[j * kWs + v % ROWS] = wt[(size_t)(i1 + j) * N + m];
+  }
+  const bool all = __syncthreads_and(fast);
+  const bool writer = l == 0 && n < N;
+  float* q_out = qt + (size_t)i1 * N + nn;
+  float* e_out = err + nn;
+  const float sum = all ? gptq_columns<LANES, kWs, true>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N)
+                        : gptq_columns<LANES, kWs, false>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N);
+  if (writer) loss[n] += sum;
 }
 
 // pack_weight (quantization.py:374-388) of reconstructed weights Qt (K x N, fp32):
 // code = uint8(clamp(q / scale + zero, 0, 2^bits - 1)) (truncating cast, as the reference's
 // .to(torch.uint8)), entries_per_byte = 8 / bits codes per byte, column epb*j + nr in bits
 // [nr*bits, (nr+1)*bits) of byte (n, j); quant_weight is column-major: byte (n, j) at j * N + n.
-__global__ __launch_bounds__(256) void colblock_pack_kernel(const float* __restrict__ qt, int K, int N,
+// order: the row of Qt that holds column k (null: k), for a column order that the loop worked in.
+__global__ __launch_bounds__(256) void colblock_pack_kernel(const float* __restrict__ qt, const int64_t* __restrict__ order, int N,
                                                             const float* __restrict__ scale,
                                                             const float* __restrict__ zero, int bits,
                                                             unsigned char* __restrict__ qw) {
@@ -113,11 +148,49 @@ __global__ __launch_bounds__(256) void colblock_pack_kernel(const float* __restr
   const float s = scale[n], z = zero[n], maxq = (float)((1 << bits) - 1);
   unsigned v = 0;
   for (int nr = 0; nr < epb; ++nr) {
-    const float x = qt[(size_t)(epb * j + nr) * N + n];
+    const size_t k = order ? (size_t)order[epb * j + nr] : epb * j + nr;
+    const float x = qt[k * N + n];
     const float c = fminf(fmaxf(__fadd_rn(__fdiv_rn(x, s), z), 0.f), maxq);
     v += ((unsigned)c) << (nr * bits);
   }
   qw[(size_t)j * N + n] = (unsigned char)v;
+}
+
+// find_params_weight's per-row (scale, zero) (quantization.py:475-514) of rows of K weights: one workgroup per row. NaN weights
+// give NaN as torch's minimum and maximum do. The quotients are correctly rounded, as the reference's on the CPU.
+__global__ __launch_bounds__(256) void gptq_params_kernel(const float* __restrict__ w, int K, float maxq, bool sym, float* __restrict__ scale,
+                                                          float* __restrict__ zero) {
+  __shared__ float part[2][4];
+  const float* row = w + (size_t)blockIdx.x * K;
+  float lo = 0.f, hi = 0.f;
+  bool nan = false;
+#pragma unroll 4
+  for (int k = threadIdx.x; k < K; k += 256) {
+    const float v = row[k];
+    lo = fminf(lo, v);
+    hi = fmaxf(hi, v);
+    nan = nan || v != v;
+  }
+  lo = -wave_max(-lo);
+  hi = wave_max(hi);
+  if ((threadIdx.x & 63) == 0) {
+    part[0][threadIdx.x >> 6] = lo;
+    part[1][threadIdx.x >> 6] = hi;
+  }
+  nan = __syncthreads_or(nan);
+  if (threadIdx.x) return;
+  lo = fminf(fminf(part[0][0], part[0][1]), fminf(part[0][2], part[0][3]));
+  hi = fmaxf(fmaxf(part[1][0], part[1][1]), fmaxf(part[1][2], part[1][3]));
+  if (nan) lo = hi = __builtin_nanf("");
+  if (sym) {
+    const float neg = lo;
+    hi = nan ? hi : fmaxf(fabsf(lo), hi);
+    if (neg < 0.f) lo = -hi;
+  }
+  if (lo == 0.f && hi == 0.f) lo = -1.f, hi = 1.f;
+  const float s = __fdiv_rn(__fsub_rn(hi, lo), maxq);
+  scale[blockIdx.x] = s;
+  zero[blockIdx.x] = sym ? __fmul_rn(__fadd_rn(maxq, 1.f), 0.5f) : rintf(__fdiv_rn(-lo, s));
 }
 
 }  // namespace llj
@@ -137,7 +210,7 @@ int llj_gptq_block_bs(const float* hinv, int K, int i1, int blocksize, float* wt
     hipLaunchKernelGGL((gptq_block_kernel<64, 4, 80>), dim3((N + 63) / 64), dim3(256), 0, (hipStream_t)stream, hinv,
                        K, i1, blocksize, wt, N, scale, zero, maxq, qt, err, loss);
   else
-    hipLaunchKernelGGL((gptq_block_kernel<32, 8, 40>), dim3((N + 31) / 32), dim3(256), 0, (hipStream_t)stream, hinv,
+    hipLaunchKernelGGL((gptq_block_kernel<16, 16, 20>), dim3((N + 15) / 16), dim3(256), 0, (hipStream_t)stream, hinv,
                        K, i1, blocksize, wt, N, scale, zero, maxq, qt, err, loss);
   LLJ_CHECK_LAUNCH();
   return 0;
@@ -148,14 +221,26 @@ int llj_gptq_block(const float* hinv, int K, int i1, float* wt, int N, const flo
   return llj_gptq_block_bs(hinv, K, i1, kGptqBlock, wt, N, scale, zero, bits, qt, err, loss, stream);
 }
 
-int llj_colblock_pack(const float* qt, int K, int N, const float* scale, const float* zero, int bits,
-                      unsigned char* qw, void* stream) {
+int llj_gptq_params(const float* w, int N, int K, int bits, int sym, float* scale, float* zero, void* stream) {
+  LLJ_REQUIRE(w && scale && zero && N > 0 && K > 0 && bits > 0 && bits <= 16);
+  hipLaunchKernelGGL(gptq_params_kernel, dim3(N), dim3(256), 0, (hipStream_t)stream, w, K, (float)((1 << bits) - 1), sym != 0, scale, zero);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+int llj_colblock_pack_order(const float* qt, const int64_t* order, int K, int N, const float* scale, const float* zero, int bits,
+                            unsigned char* qw, void* stream) {
   LLJ_REQUIRE(K > 0 && N > 0 && (bits == 2 || bits == 4 || bits == 8) && K % (8 / bits) == 0);
   LLJ_REQUIRE(qt && scale && zero && qw);
   hipLaunchKernelGGL(colblock_pack_kernel, dim3((N + 255) / 256, K / (8 / bits)), dim3(256), 0, (hipStream_t)stream,
-                     qt, K, N, scale, zero, bits, qw);
+                     qt, order, N, scale, zero, bits, qw);
   LLJ_CHECK_LAUNCH();
   return 0;
+}
+
+int llj_colblock_pack(const float* qt, int K, int N, const float* scale, const float* zero, int bits,
+                      unsigned char* qw, void* stream) {
+  return llj_colblock_pack_order(qt, nullptr, K, N, scale, zero, bits, qw, stream);
 }
 
 }  // extern "C"

@@ -1,0 +1,487 @@
+// Matrix work of the GPTQ producer around the column loop (gptq.hip): the calibration Hessian, the inverse factor that the
+// loop reads, and the update of the columns behind a block (reference lit_llama/quantization.py:516-530, 549-566, 596).
+//
+// All three are C -= or += A^T B with both operands stored along their output index ("k-major": X of the Hessian is tokens x
+// columns, a block of the factor and the block's errors are 128 x columns), which v_mfma_f32_16x16x4_f32 takes from LDS without a
+// transposition: lane l reads element (k + l / 16, m + l % 16), rows 16 banks apart. One accumulator per output, ascending k.
+// Bound: the fp32 matrix rate (157 TFLOP/s dense). A step of 16 k of a 64 x 64 tile is 32 MFMAs of 32 cycles for 16 reads of 4
+// bytes a lane, so neither LDS nor the loads (the next tile's in registers while this one is multiplied) are near their limits.
+#include "common.h"
+
+namespace llj {
+
+constexpr int kFactor = 128;  // columns per elimination step
+
+__device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// four consecutive elements, zeros from `left` on
+template <bool VEC>
+__device__ __forceinline__ f32x4 ld4(const float* p, int left) {
+  if constexpr (VEC) return left > 0 ? *reinterpret_cast<const f32x4*>(p) : f32x4{};
+  f32x4 v = {};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i < left) v[i] = p[i];
+  return v;
+}
+template <bool VEC>
+__device__ __forceinline__ f32x4 ld4(const bf16_t* p, int left) {
+  f32x4 v = {};
+  if constexpr (VEC) {
+    if (left > 0) {
+      const uint2 w = *reinterpret_cast<const uint2*>(p);
+      v = f32x4{bflo(w.x), bfhi(w.x), bflo(w.y), bfhi(w.y)};
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < left) v[i] = bf2f(p[i]);
+  }
+  return v;
+}
+
+// acc = A^T B of one BM x BN tile by 256 threads (2 x 2 waves): A: kd x ma, B: kd x nb, k-major, pointers at the tile's first column,
+// ma / nb columns left from there (VEC: multiples of 4, rows aligned to four elements). SCALE: elements times alpha, rounded.
+template <int BM, int BN, typename S, bool VEC, bool SCALE>
+struct AtB {
+  static constexpr int KD = 32, SA = BM + 16, SB = BN + 16, MI = BM / 32, NI = BN / 32;
+  static constexpr int kLds = 2 * KD * (SA + SB);  // floats
+  static constexpr int TA = BM / 4, RA = 256 / TA, PA = KD / RA, TB = BN / 4, RB = 256 / TB, PB = KD / RB;
+
+  static __device__ __forceinline__ void run(const S* A, size_t lda, int ma, const S* B, size_t ldb, int nb, int kd, float alpha,
+                                             float* lds, f32x4 (&acc)[MI][NI]) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int ca = (tid % TA) * 4, cb = (tid % TB) * 4;
+    f32x4 fa[PA], fb[PB];
+    auto fetch = [&](int k) {
+#pragma unroll
+      for (int p = 0; p < PA; ++p) {
+        const int row = k + tid / TA + p * RA;
+        fa[p] = ld4<VEC>(A + (size_t)row * lda + ca, row < kd ? ma - ca : 0);
+      }
+#pragma unroll
+      for (int p = 0; p < PB; ++p) {
+        const int row = k + tid / TB + p * RB;
+        fb[p] = ld4<VEC>(B + (size_t)row * ldb + cb, row < kd ? nb - cb : 0);
+      }
+    };
+    auto stage = [&](int buf) {
+      float* a = lds + buf * KD * (SA + SB);
+      float* b = a + KD * SA;
+#pragma unroll
+      for (int p = 0; p < PA; ++p) *reinterpret_cast<f32x4*>(a + (tid / TA + p * RA) * SA + ca) = SCALE ? fa[p] * alpha : fa[p];
+#pragma unroll
+      for (int p = 0; p < PB; ++p) *reinterpret_cast<f32x4*>(b + (tid / TB + p * RB) * SB + cb) = SCALE ? fb[p] * alpha : fb[p];
+    };
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{};
+    const int oa = (lane >> 4) * SA + (wave & 1) * (BM / 2) + (lane & 15), ob = (lane >> 4) * SB + (wave >> 1) * (BN / 2) + (lane & 15);
+    fetch(0);
+    stage(0);
+    for (int k = 0, t = 0; k < kd; k += KD, ++t) {
+      __syncthreads();  // tile t is staged, and every wave is done with the other buffer
+      if (k + KD < kd) fetch(k + KD);
+      const float* a = lds + (t & 1) * KD * (SA + SB) + oa;
+      const float* b = lds + (t & 1) * KD * (SA + SB) + KD * SA + ob;
+#pragma unroll
+      for (int q = 0; q < KD / 4; ++q) {
+        float va[MI], vb[NI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) va[i] = a[4 * q * SA + 16 * i];
+#pragma unroll
+        for (int j = 0; j < NI; ++j) vb[j] = b[4 * q * SB + 16 * j];
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] = mma4(va[i], vb[j], acc[i][j]);
+      }
+      if (k + KD < kd) stage((t + 1) & 1);
+    }
+  }
+  // acc = f(row, column) of every output of the tile: all loads before the first use
+  template <typename F>
+  static __device__ __forceinline__ void load(f32x4 (&acc)[MI][NI], F f) {
+    each(acc, [&](int i, int j, float& v) { v = f(i, j); });
+  }
+  // f(row, column, sum) of every output of the tile
+  template <typename F>
+  static __device__ __forceinline__ void each(f32x4 (&acc)[MI][NI], F f) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float v = acc[i][j][r];
+          f((wave & 1) * (BM / 2) + 16 * i + 4 * (lane >> 4) + r, (wave >> 1) * (BN / 2) + 16 * j + (lane & 15), v);
+          acc[i][j][r] = v;
+        }
+  }
+  template <typename F>
+  static __device__ __forceinline__ void both(f32x4 (&acc)[MI][NI], f32x4 (&old)[MI][NI], F f) {
+    int at = 0;
+    each(acc, [&](int i, int j, float v) {
+      f(i, j, v, old[at / (4 * NI)][at / 4 % NI][at % 4]);
+      ++at;
+    });
+  }
+};
+
+// block b of a grid padded to a multiple of 8 -> its place in a list of n tiles that gives each XCD (b % 8) one run of neighbours
+__device__ __forceinline__ int xcd_run(int b, int n) {
+  const int per = (n + 7) / 8, t = (b & 7) * per + (b >> 3);
+  return (b >> 3) < per && t < n ? t : -1;
+}
+// t -> (i, j <= i) of a triangle's tiles, row by row
+__device__ __forceinline__ void triangle(int t, int& i, int& j) {
+  i = (int)((__builtin_sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
+  while (i * (i + 1) / 2 > t) --i;
+  while ((i + 1) * (i + 2) / 2 <= t) ++i;
+  j = t - i * (i + 1) / 2;
+}
+
+// H = keep H + (alpha X)^T (alpha X): the tiles on and below the diagonal, each written to its place and mirrored. The sums are those
+// of the library's product bit for bit (to 4,096 columns), at half its work: 2048 x 4096 385 us (89 TFLOP/s of the half) for 580 with
+// the two passes over H.
+template <int BT, typename S, bool VEC>
+__global__ __launch_bounds__(256) void gptq_gram_kernel(const S* __restrict__ x, int T, int K, float keep, float alpha, float* __restrict__ H) {
+  typedef AtB<BT, BT, S, VEC, true> G;
+  __shared__ __align__(16) float lds[G::kLds];
+  const int nt = (K + BT - 1) / BT, t = xcd_run(blockIdx.x, nt * (nt + 1) / 2);
+  if (t < 0) return;
+  int ti, tj;
+  triangle(t, ti, tj);
+  const int m0 = ti * BT, n0 = tj * BT;
+  f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
+  G::run(x + m0, K, K - m0, x + n0, K, K - n0, T, alpha, lds, acc);
+  G::load(old, [&](int i, int j) { return H[(size_t)min(m0 + i, K - 1) * K + min(n0 + j, K - 1)]; });
+  G::both(acc, old, [&](int i, int j, float v, float h) {
+    const int m = m0 + i, n = n0 + j;
+    if (m >= K || n >= K) return;
+    h = h * keep + v;
+    H[(size_t)m * K + n] = h;
+    if (ti != tj) H[(size_t)n * K + m] = h;
+  });
+}
+
+// Wt[i2 + m][n] -= sum_b hinv[i1 + b][i2 + m] err[b][n]. Bound: Wt in and out beside the products; what is subtracted from is read
+// after them, all of it before the first use. 3968 x 4096: 51 us for 73 as a product and a subtraction, the same bits.
+template <int BM, int BN, bool VEC>
+__global__ __launch_bounds__(256) void gptq_update_kernel(const float* __restrict__ hinv, int K, int i1, int blk, const float* __restrict__ err,
+                                                          int N, float* __restrict__ wt) {
+  typedef AtB<BM, BN, float, VEC, false> G;
+  __shared__ __align__(16) float lds[G::kLds];
+  const int i2 = i1 + blk, M = K - i2, mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN, t = xcd_run(blockIdx.x, mt * nt);
+  if (t < 0) return;
+  const int m0 = t / nt * BM, n0 = t % nt * BN;
+  f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
+  G::run(hinv + (size_t)i1 * K + i2 + m0, K, M - m0, err + n0, N, N - n0, blk, 1.f, lds, acc);
+  G::load(old, [&](int i, int j) { return wt[(size_t)(i2 + min(m0 + i, M - 1)) * N + min(n0 + j, N - 1)]; });
+  G::both(acc, old, [&](int i, int j, float v, float w) {
+    const int m = m0 + i, n = n0 + j;
+    if (m < M && n < N) wt[(size_t)(i2 + m) * N + n] = w - v;
+  });
+}
+
+// ---------------------------------------------------------------- the inverse factor
+// U upper triangular with U^T U = H^-1 (torch.linalg.cholesky(cholesky_inverse(cholesky(H)), upper=True)): with the order of the
+// columns reversed, H = L L^T gives U as L^-1 reversed -- one elimination instead of two factorizations and a product. Blocks of 128
+// columns; step k turns row block k of [H | I] into P_k = L_kk^-1 [X_k | H_k] (gptq_panel_kernel) and takes P_k[:, i]^T P_k off every
+// later row block i (gptq_step_kernel): in H's upper triangle the next matrix to factor, in the lower one the growing L^-1.
+// The next diagonal block is factored by one workgroup of that launch while the others work on the rest: its chain of 128 pivots (about
+// 35 us) bounds a step, the products (2 K^3 / 3 in all, 0.3 ms at K = 4096) run beside it. K = 4096: 1.7 ms for 29.2 with the library's
+// three calls, K = 512: 0.18 for 3.1; error against float64 2.5e-7 for 1.1e-6 (8,192 rows).
+constexpr int kFs = kFactor + 16;  // LDS row stride of the diagonal block
+
+__device__ __forceinline__ float lane_value(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+
+// S (LDS, 128 x 128, upper triangle, zeros below) -> L^-1 in the lower triangle with zeros above, S = L L^T. 32 columns at a time: one wave eliminates
+// the 32 x 32 block in registers (lane c a column of the block, lane 32 + c of the identity), the matrix cores do the rest.
+// Returns false (in every thread) if a pivot was not positive.
+__device__ __forceinline__ bool factor_block(float* S, int* bad) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c16 = lane & 15;
+  if (tid == 0) *bad = 0;
+  for (int s = 0; s < 4; ++s) {
+    __syncthreads();
+    if (wave == 0) {
+      const int c = lane & 31;
+      float* d = S + 32 * s * kFs + 32 * s;
+      float v[32];
+#pragma unroll
+      for (int i = 0; i < 32; ++i) v[i] = d[i * kFs + c];
+#pragma unroll
+      for (int i = 0; i < 32; ++i) v[i] = lane < 32 ? (i <= c ? v[i] : 0.f) : (i == c ? 1.f : 0.f);
+      bool ok = true;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        const float p = lane_value(v[j], j);
+        ok = ok && p > 0.f;
+        float r = __builtin_amdgcn_rsqf(p);
+        r = __builtin_fmaf(0.5f * r, __builtin_fmaf(-p * r, r, 1.f), r);  // one Newton step
+        v[j] *= r;
+#pragma unroll
+        for (int g = (j + 1) & ~7; g < 32; g += 8) {
+#pragma unroll
+          for (int i = g > j ? g : j + 1; i < g + 8; ++i) v[i] = __builtin_fmaf(-lane_value(v[j], i), v[j], v[i]);
+          // updated here, not where it is read next: the lane values would pile up and spill
+          asm volatile("" : "+v"(v[g]), "+v"(v[g + 1]), "+v"(v[g + 2]), "+v"(v[g + 3]), "+v"(v[g + 4]), "+v"(v[g + 5]), "+v"(v[g + 6]), "+v"(v[g + 7]));
+        }
+      }
+      if (lane >= 32) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) d[i * kFs + c] = v[i];
+      }
+      if (!ok && lane == 0) *bad = 1;
+    }
+    __syncthreads();
+    if (wave != s) {  // the other 32-column blocks of these rows, times the block's inverse
+      float* b = S + 32 * s * kFs + 32 * wave;
+      const float* a = S + 32 * s * kFs + 32 * s;
+      f32x4 o[2][2] = {};
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            o[i][j] = mma4(a[(16 * i + c16) * kFs + 4 * k + q], b[(4 * k + q) * kFs + 16 * j + c16], o[i][j]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) b[(16 * i + 4 * q + r) * kFs + 16 * j + c16] = o[i][j][r];
+    }
+    __syncthreads();
+    int n = 0;
+    for (int ib = s + 1; ib < 4; ++ib)
+      for (int jb = 0; jb < 4; ++jb) {
+        if (jb > s && jb < ib) continue;
+        if ((n++ & 3) != wave) continue;
+        const float* p = S + 32 * s * kFs;
+        float* o = S + 32 * ib * kFs + 32 * jb;
+        f32x4 d[2][2] = {}, old[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) old[i][j][r] = o[(16 * i + 4 * q + r) * kFs + 16 * j + c16];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              d[i][j] = mma4(p[(4 * k + q) * kFs + 32 * ib + 16 * i + c16], p[(4 * k + q) * kFs + 32 * jb + 16 * j + c16], d[i][j]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[(16 * i + 4 * q + r) * kFs + 16 * j + c16] = old[i][j][r] - d[i][j][r];
+      }
+  }
+  __syncthreads();
+  return *bad == 0;
+}
+
+// the factored block: its rows of P (zeros above the diagonal) and transposed for the panel product
+__device__ __forceinline__ void put_block(const float* S, int k, int K, float* __restrict__ P, float* __restrict__ xt, bool ok, int* info) {
+  const int j = threadIdx.x & 127;
+#pragma unroll 8
+  for (int i = threadIdx.x >> 7; i < kFactor; i += 2) {
+    const float a = S[i * kFs + j], t = S[j * kFs + i];
+    P[((size_t)k * kFactor + i) * K + (size_t)k * kFactor + j] = j <= i ? a : 0.f;
+    xt[i * kFactor + j] = i <= j ? t : 0.f;
+  }
+  if (!ok && threadIdx.x == 0) *info = 1;
+}
+
+// M (upper triangle) = H in the reversed order of perm (null: 0, 1, ..) with damp on the diagonal
+__global__ __launch_bounds__(256) void gptq_order_kernel(const float* __restrict__ H, const int64_t* __restrict__ perm, const float* __restrict__ damp,
+                                                         int K, float* __restrict__ M) {
+  const int a = blockIdx.y, b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= K || b < a) return;
+  const int ra = K - 1 - a, rb = K - 1 - b;
+  const size_t i = perm ? (size_t)perm[ra] : ra, j = perm ? (size_t)perm[rb] : rb;
+  M[(size_t)a * K + b] = a == b ? H[i * K + j] + *damp : H[i * K + j];
+}
+
+__global__ __launch_bounds__(256) void gptq_first_kernel(const float* __restrict__ M, int K, float* __restrict__ P, float* __restrict__ xt, int* info) {
+  __shared__ __align__(16) float S[kFactor * kFs];
+  __shared__ int bad;
+  float m[kFactor * kFactor / 256];  // every load in flight before the first is used (the lower triangle is not set)
+#pragma unroll
+  for (int r = 0; r < kFactor * kFactor / 256; ++r) m[r] = M[(size_t)(2 * r + (threadIdx.x >> 7)) * K + (threadIdx.x & 127)];
+#pragma unroll
+  for (int r = 0; r < kFactor * kFactor / 256; ++r) {
+    const int i = 2 * r + (threadIdx.x >> 7), j = threadIdx.x & 127;
+    S[i * kFs + j] = j >= i ? m[r] : 0.f;
+  }
+  const bool ok = factor_block(S, &bad);
+  put_block(S, 0, K, P, xt, ok, info);
+}
+
+// P's row block k outside the diagonal block: xt^T M's row block. Workgroup: 64 rows x 64 columns.
+__global__ __launch_bounds__(256) void gptq_panel_kernel(const float* __restrict__ M, const float* __restrict__ xt, int k, int K, float* __restrict__ P) {
+  typedef AtB<64, 64, float, true, false> G;
+  __shared__ __align__(16) float lds[G::kLds];
+  const int m0 = (blockIdx.x & 1) * 64, n0 = (blockIdx.x >> 1) * 64;
+  if (n0 / kFactor == k) return;
+  f32x4 acc[G::MI][G::NI];
+  const size_t row = (size_t)k * kFactor;
+  G::run(xt + m0, kFactor, kFactor - m0, M + row * K + n0, K, K - n0, kFactor, 1.f, lds, acc);
+  G::each(acc, [&](int i, int j, float v) { P[(row + m0 + i) * K + n0 + j] = v; });
+}
+
+// Workgroup 0: the next diagonal block, updated and factored. The others: 64 x 64 tiles of the rows below, the lower triangle's columns
+// up to block k (first sums in block k's own) and the upper triangle's.
+__global__ __launch_bounds__(256) void gptq_step_kernel(float* __restrict__ M, float* __restrict__ P, int k, int K, float* __restrict__ xt, int* info) {
+  typedef AtB<128, 128, float, true, false> D;
+  typedef AtB<64, 64, float, true, false> G;
+  constexpr int kS = kFactor * kFs;
+  __shared__ __align__(16) float lds[kS > D::kLds ? kS : D::kLds];
+  __shared__ int bad;
+  const float* p = P + (size_t)k * kFactor * K;
+  const int r0 = (k + 1) * kFactor;
+  if (blockIdx.x == 0) {
+    __builtin_amdgcn_s_setprio(3);  // the longest chain of the launch, beside another workgroup's products
+    f32x4 acc[D::MI][D::NI], old[D::MI][D::NI];
+    D::load(old, [&](int i, int j) { return M[(size_t)(r0 + i) * K + r0 + j]; });
+    D::run(p + r0, K, kFactor, p + r0, K, kFactor, kFactor, 1.f, lds, acc);
+    __syncthreads();
+    D::both(acc, old, [&](int i, int j, float v, float m) { lds[i * kFs + j] = j >= i ? m - v : 0.f; });
+    const bool ok = factor_block(lds, &bad);
+    put_block(lds, k + 1, K, P, xt, ok, info);
+    return;
+  }
+  const int R = (K - r0) / 64, C = r0 / 64, upper = R * (R + 1) / 2;
+  const int t = xcd_run(blockIdx.x - 1, R * C + upper);
+  if (t < 0) return;
+  int m0, n0;
+  if (t < R * C) {
+    m0 = r0 + t / C * 64;
+    n0 = t % C * 64;
+  } else {
+    int i, j;
+    triangle(t - R * C, i, j);
+    if (i < 2) return;  // workgroup 0's
+    m0 = r0 + j * 64;
+    n0 = r0 + i * 64;
+  }
+  f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
+  G::load(old, [&](int i, int j) { return M[(size_t)(m0 + i) * K + n0 + j]; });
+  G::run(p + m0, K, 64, p + n0, K, 64, kFactor, 1.f, lds, acc);
+  const bool first = n0 / kFactor == k;
+  G::both(acc, old, [&](int i, int j, float v, float m) { M[(size_t)(m0 + i) * K + n0 + j] = (first ? 0.f : m) - v; });
+}
+
+// Wt[place[k]][n] = W[n][k] (null: k), zero where dead[k]: 64 x 64 through LDS, whole rows of Wt moved to their places
+__global__ __launch_bounds__(256) void gptq_weight_kernel(const float* __restrict__ W, const int64_t* __restrict__ place, const bool* __restrict__ dead,
+                                                          int N, int K, float* __restrict__ Wt) {
+  __shared__ float t[64][65];
+  const int n0 = blockIdx.x * 64, k0 = blockIdx.y * 64, c = threadIdx.x & 63, r = threadIdx.x >> 6;
+  const int k = min(k0 + c, K - 1);
+  const bool zero = dead[k];
+  float v[16];
+  size_t to[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    v[i] = W[(size_t)min(n0 + r + 4 * i, N - 1) * K + k];
+    const int row = min(k0 + r + 4 * i, K - 1);
+    to[i] = place ? (size_t)place[row] : row;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) t[r + 4 * i][c] = zero ? 0.f : v[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if (n0 + c < N && k0 + r + 4 * i < K) Wt[to[i] * N + n0 + c] = t[c][r + 4 * i];
+}
+
+// U = P's lower triangle in reversed order, zeros below the diagonal
+__global__ __launch_bounds__(256) void gptq_reverse_kernel(const float* __restrict__ P, int K, float* __restrict__ U) {
+  const int a = blockIdx.y, b = blockIdx.x * 256 + threadIdx.x;
+  if (b < K) U[(size_t)a * K + b] = b >= a ? P[(size_t)(K - 1 - a) * K + K - 1 - b] : 0.f;
+}
+
+}  // namespace llj
+
+using namespace llj;
+
+extern "C" {
+
+int llj_gptq_gram(const void* x, int dt, int T, int K, float keep, float alpha, float* H, void* stream) {
+  LLJ_REQUIRE(x && H && T > 0 && K > 0 && (dt == 0 || dt == 1));
+  // 64 x 64 tiles, 32 x 32 while those leave CUs idle (1467 x 512: 49 us and 20, 357 x 1152: 17 and 12)
+  const long n64 = (K + 63) / 64, n32 = (K + 31) / 32;
+  const bool small = n64 * (n64 + 1) / 2 < 256;
+  const long tiles = small ? n32 * (n32 + 1) / 2 : n64 * (n64 + 1) / 2, grid = (tiles + 7) / 8 * 8;
+  const bool vec = K % 4 == 0 && ((uintptr_t)x & (dt ? 15 : 7)) == 0;
+  LLJ_REQUIRE(grid < (1l << 31));
+  const hipStream_t s = (hipStream_t)stream;
+#define LLJ_GRAM_T(B, S, V) \
+  hipLaunchKernelGGL((gptq_gram_kernel<B, S, V>), dim3((unsigned)grid), dim3(256), 0, s, (const S*)x, T, K, keep, alpha, H)
+#define LLJ_GRAM(S, V)                 \
+  do {                                 \
+    if (small) LLJ_GRAM_T(32, S, V);   \
+    else LLJ_GRAM_T(64, S, V);         \
+  } while (0)
+  if (dt) {
+    if (vec) LLJ_GRAM(float, true);
+    else LLJ_GRAM(float, false);
+  } else {
+    if (vec) LLJ_GRAM(bf16_t, true);
+    else LLJ_GRAM(bf16_t, false);
+  }
+#undef LLJ_GRAM
+#undef LLJ_GRAM_T
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+int llj_gptq_update(const float* hinv, int K, int i1, int blocksize, const float* err, int N, float* wt, void* stream) {
+  LLJ_REQUIRE(hinv && err && wt && K > 0 && N > 0 && i1 >= 0 && blocksize > 0 && i1 + blocksize <= K);
+  const int M = K - i1 - blocksize;
+  if (M == 0) return 0;
+  const bool vec = K % 4 == 0 && N % 4 == 0 && (i1 + blocksize) % 4 == 0 && (((uintptr_t)hinv | (uintptr_t)err) & 15) == 0;
+  const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64), grid = (tiles + 7) / 8 * 8;
+  LLJ_REQUIRE(grid < (1l << 31));
+  if (vec)
+    hipLaunchKernelGGL((gptq_update_kernel<64, 64, true>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, hinv, K, i1, blocksize, err, N, wt);
+  else
+    hipLaunchKernelGGL((gptq_update_kernel<64, 64, false>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, hinv, K, i1, blocksize, err, N, wt);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+int llj_gptq_weight(const float* W, const int64_t* place, const void* dead, int N, int K, float* Wt, void* stream) {
+  LLJ_REQUIRE(W && dead && Wt && N > 0 && K > 0 && (K + 63) / 64 <= 65535);
+  hipLaunchKernelGGL(gptq_weight_kernel, dim3((N + 63) / 64, (K + 63) / 64), dim3(256), 0, (hipStream_t)stream, W, place, (const bool*)dead, N, K, Wt);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+int llj_gptq_factor(const float* H, const int64_t* perm, const float* damp, int K, float* M, float* P, float* xt, int* info, void* stream) {
+  LLJ_REQUIRE(H && damp && M && P && xt && info && K >= kFactor && K % kFactor == 0 && K <= 65535);
+  LLJ_REQUIRE((((uintptr_t)M | (uintptr_t)P | (uintptr_t)xt) & 15) == 0);
+  const hipStream_t s = (hipStream_t)stream;
+  const int nb = K / kFactor;
+  hipLaunchKernelGGL(gptq_order_kernel, dim3((K + 255) / 256, K), dim3(256), 0, s, H, perm, damp, K, M);
+  hipLaunchKernelGGL(gptq_first_kernel, dim3(1), dim3(256), 0, s, M, K, P, xt, info);
+  for (int k = 0; k < nb; ++k) {
+    hipLaunchKernelGGL(gptq_panel_kernel, dim3(K / 64 * 2), dim3(256), 0, s, M, xt, k, K, P);
+    if (k + 1 == nb) break;
+    const long R = (K - (k + 1) * kFactor) / 64, C = (k + 1) * kFactor / 64, tiles = R * C + R * (R + 1) / 2;
+    hipLaunchKernelGGL(gptq_step_kernel, dim3((unsigned)(1 + (tiles + 7) / 8 * 8)), dim3(256), 0, s, M, P, k, K, xt, info);
+  }
+  hipLaunchKernelGGL(gptq_reverse_kernel, dim3((K + 255) / 256, K), dim3(256), 0, s, P, K, M);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // extern "C"

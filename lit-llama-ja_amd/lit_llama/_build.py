@@ -25,7 +25,7 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-variable", "-Wno-un
 
 # per-file flags: the GPTQ column loop reproduces the reference's fp32 op order bit for bit, so
 # no multiply-add contraction there (hipcc contracts by default and ignores the fp pragma)
-FILE_FLAGS = {"gptq.hip": ["-ffp-contract=off"]}
+FILE_FLAGS = {f: ["-ffp-contract=off"] for f in ("gptq.hip", "gptq_factor.hip")}
 
 
 def sources():

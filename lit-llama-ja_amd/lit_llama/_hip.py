@@ -48,6 +48,12 @@ SIGNATURES = {
     "llj_i8_gather_weight": [_P, _P, _I, _I, _P, _P, _I, _P],
     "llj_gptq_block": [_P, _I, _I, _P, _I, _P, _P, _I, _P, _P, _P, _P],
     "llj_gptq_block_bs": [_P, _I, _I, _I, _P, _I, _P, _P, _I, _P, _P, _P, _P],
+    "llj_gptq_gram": [_P, _I, _I, _I, _F, _F, _P, _P],
+    "llj_gptq_update": [_P, _I, _I, _I, _P, _I, _P, _P],
+    "llj_gptq_params": [_P, _I, _I, _I, _I, _P, _P, _P],
+    "llj_gptq_weight": [_P, _P, _P, _I, _I, _P, _P],
+    "llj_colblock_pack_order": [_P, _P, _I, _I, _P, _P, _I, _P, _P],
+    "llj_gptq_factor": [_P, _P, _P, _I, _P, _P, _P, _P, _P],
     "llj_colblock_pack": [_P, _I, _I, _P, _P, _I, _P, _P],
     "llj_attention": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "llj_attention_prefill": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],

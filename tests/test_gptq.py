@@ -485,3 +485,128 @@ def test_grouped_gptq_quantizer_vs_oracle(hip, t):
         y = qm(x).float()
         yr = x.float() @ qm.get_weight(torch.float).t()
     assert (y - yr).norm() / yr.norm() < 1e-2
+
+
+def _f64_factor(H, perm, percdamp=0.01):
+    H = H.double()[perm][:, perm]
+    H.diagonal().add_(percdamp * H.diagonal().mean())
+    return torch.linalg.cholesky(torch.cholesky_inverse(torch.linalg.cholesky(H)), upper=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,K,dtype", [(1, 128, torch.float32), (33, 130, torch.float32), (300, 129, torch.bfloat16), (95, 640, torch.bfloat16),
+                                       (257, 2048, torch.float32), (64, 1500, torch.float16)])
+def test_hessian_kernel(hip, T, K, dtype):
+    """collect_input_stats over two windows, the second not contiguous: both tile sizes, remainders of rows and columns, symmetric bits;
+    against float64 within T roundings of the largest partial sum."""
+    from lit_llama.quantization import GPTQQuantizer
+    g = torch.Generator(device=dev).manual_seed(T)
+    gq = GPTQQuantizer(torch.nn.Linear(128, 16, bias=False, device=dev), bits=4)
+    gq.H = torch.zeros(K, K, device=dev)
+    x = [torch.randn(1, T, K, generator=g, device=dev).to(dtype), torch.randn(1, K, T, generator=g, device=dev).to(dtype).transpose(1, 2)]
+    for w in x:
+        gq.collect_input_stats(None, (w,), None)
+    assert gq.tokens == 2 * T and torch.equal(gq.H, gq.H.t())
+    a = torch.cat([w[0] for w in x]).double()
+    bound = (2 * T + 8) * 2.0 ** -24 * (a.abs().t() @ a.abs())
+    assert ((gq.H.double() - a.t() @ a).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [128, 256, 384, 1152])
+def test_inverse_factor_kernel(hip, K):
+    """llj_gptq_factor against float64: one block, two, and several, with and without an order; the input stays as it is, zeros below
+    the diagonal. Its error is held to the library's chain's on the same matrix."""
+    from lit_llama import _hip
+    g = torch.Generator(device=dev).manual_seed(K)
+    x = torch.randn(2 * K, K, generator=g, device=dev) * torch.exp(0.5 * torch.randn(K, generator=g, device=dev))
+    H = x.t() @ x
+    H = (H + H.t()) / 2
+    for perm in (torch.arange(K, device=dev), torch.argsort(torch.diag(H), descending=True)):
+        damp = 0.01 * H.diagonal().mean()
+        kept, M, P = H.clone(), torch.full_like(H, float("nan")), torch.full_like(H, float("nan"))
+        xt, info = torch.empty(128, 128, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
+        order = 0 if torch.equal(perm, torch.arange(K, device=dev)) else perm.data_ptr()
+        _hip.call("llj_gptq_factor", H.data_ptr(), order, damp.data_ptr(), K, M.data_ptr(), P.data_ptr(), xt.data_ptr(), info.data_ptr(), _st())
+        torch.cuda.synchronize()
+        assert info.item() == 0 and torch.equal(H, kept) and torch.equal(M, M.triu())
+        ref = _f64_factor(H, perm)
+        h = H[perm][:, perm]
+        h.diagonal().add_(damp)
+        lib = torch.linalg.cholesky(torch.cholesky_inverse(torch.linalg.cholesky(h)), upper=True)
+        err = lambda u: ((u - ref).norm() / ref.norm()).item()  # noqa: E731
+        assert err(M) <= max(err(lib), K ** 0.5 * 2.0 ** -24)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,i1,blk", [(64, 256, 0, 128), (37, 256, 128, 64), (130, 384, 128, 128), (352, 128, 96, 16), (8, 128, 0, 128)])
+def test_block_update_kernel(hip, N, K, i1, blk):
+    """llj_gptq_update: the columns behind the block alone change, for row counts off the tiles and off four; nothing behind the last."""
+    from lit_llama import _hip
+    g = torch.Generator(device=dev).manual_seed(N)
+    hinv, err, w = (torch.randn(*s, generator=g, device=dev) for s in ((K, K), (blk, N), (K, N)))
+    ref = w.double()
+    i2 = i1 + blk
+    ref[i2:] -= hinv[i1:i2, i2:].double().t() @ err.double()
+    mag = w.abs().double()
+    mag[i2:] += hinv[i1:i2, i2:].double().abs().t() @ err.double().abs()
+    before = w.clone()
+    _hip.call("llj_gptq_update", hinv.data_ptr(), K, i1, blk, err.data_ptr(), N, w.data_ptr(), _st())
+    torch.cuda.synchronize()
+    assert torch.equal(w[:i2], before[:i2])
+    assert ((w.double() - ref).abs() <= (blk + 2) * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits,sym", [(4, False), (8, True), (2, False)])
+def test_row_parameters_kernel(hip, bits, sym):
+    """find_params_weight on the device against the host's: rows of one sign, of zeros, with NaN and infinities."""
+    from lit_llama.quantization import GPTQQuantizer
+    g = torch.Generator().manual_seed(bits)
+    w = torch.randn(40, 384, generator=g)
+    w[0], w[1], w[2] = 0, w[1].abs(), -w[2].abs()
+    w[3, 5], w[4, 9], w[5, 383] = float("nan"), float("inf"), float("-inf")
+    w[6] = 0
+    w[6, 200] = 1e-38
+    gq = GPTQQuantizer(torch.nn.Linear(384, 40, bias=False, device=dev), bits=bits, sym=sym)
+    for a, b in zip(gq.find_params_weight(w.to(dev)), gq.find_params_weight(w)):
+        assert a.shape == b.shape
+        np.testing.assert_array_equal(a.cpu().numpy(), b.numpy())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("small", [1.0, 2.0 ** -70])
+def test_gptq_block_kernel_divisions_bitwise(hip, small):
+    """Quotients by a reciprocal (scales and diagonals of ordinary size) and by the division instruction sequence (2^-70): bit for bit the
+    oracle's, many mantissas."""
+    from lit_llama import _hip
+    rng = np.random.default_rng(3)
+    N, K = 272, 128
+    W = (rng.standard_normal((N, K)) * small).astype(np.float32)
+    scale = (rng.uniform(0.05, 0.4, N) * small).astype(np.float32)
+    zero = rng.integers(4, 12, N).astype(np.float32)
+    Hinv = np.triu(rng.standard_normal((K, K)) * 0.02).astype(np.float32)
+    Hinv[np.arange(K), np.arange(K)] = rng.uniform(0.01, 3, K).astype(np.float32)
+    Q1, E1, L1 = G.gptq_block(W, Hinv, scale, zero, 4)
+    wt = torch.from_numpy(np.ascontiguousarray(W.T)).to(dev)
+    qt, err, loss = torch.empty(K, N, device=dev), torch.empty(128, N, device=dev), torch.zeros(N, device=dev)
+    hd, sd, zd = (torch.from_numpy(a).to(dev) for a in (Hinv, scale, zero))
+    _hip.call("llj_gptq_block", hd.data_ptr(), K, 0, wt.data_ptr(), N, sd.data_ptr(), zd.data_ptr(), 4, qt.data_ptr(), err.data_ptr(),
+              loss.data_ptr(), _st())
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(qt.cpu().numpy().T, Q1)
+    np.testing.assert_array_equal(err.cpu().numpy().T, E1)
+    if small == 1.0:
+        np.testing.assert_allclose(loss.cpu().numpy(), L1.sum(1), rtol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [64, 384])
+def test_quantizer_refuses_an_indefinite_hessian(hip, tokens):
+    """Negative damping: the same error below and above the calibration rows from which the factor is this library's own."""
+    from lit_llama.quantization import GPTQQuantizer
+    lin = torch.nn.Linear(128, 32, bias=False, device=dev)
+    gq = GPTQQuantizer(lin, bits=4, percdamp=-10.0, actorder=True)
+    gq.collect_input_stats(None, (torch.randn(1, tokens, 128, device=dev),), None)
+    with pytest.raises(torch.linalg.LinAlgError):
+        gq.quantize()
