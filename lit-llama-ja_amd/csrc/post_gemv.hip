@@ -187,8 +187,15 @@ static int rows_gemv_launch(const PostGemvParams& p, hipStream_t s) {
 }
 
 // A workgroup owns 16 output columns; its NW waves take the 128-deep K chunks round robin, D chunks in
-// flight per wave (a chunk of a column is 256 contiguous bytes, 16 B per lane and MFMA step), and their
-// partial tiles are summed through LDS. Activation rows:
+// flight per wave, and their partial tiles are summed through LDS. A load is 256 contiguous bytes of each of 4 columns;
+// the MFMA's operand (one column per lane and 16 bytes of four pieces of it) is made from four of them in a 4 KB
+// patch of LDS that is the wave's own. Loads in the operand's own order touch 64 bytes of each of 16 columns. us in a graph
+// (TB/s), that form -> this, the same sums:
+//   8 rows: 2048 -> 8448 13.3 (2.6) -> 10.3 (3.4)   8448 -> 2048 14.8 (2.3) -> 10.3 (3.4)   2048 -> 6272 9.6 (2.7) -> 8.1 (3.2)
+//           2048 -> 2048 6.7 (1.3) -> 4.2 (2.0)     2048 -> 32000 34.6 (3.8) -> 26.2 (5.0)  4096 -> 12544 32.4 (3.2) -> 22.4 (4.6)
+//           4096 -> 16512 40.5 (3.3) -> 27.6 (4.9)  16512 -> 4096 40.9 (3.3) -> 32.9 (4.1)
+//   post:   2048 -> 8448 11.7 -> 9.7, 4096 -> 16512 34.4 -> 28.5, 2048 -> 2048 4.9 -> 4.0
+// Activation rows:
 //   plain   read as MFMA fragments from memory (L2) next to the weights: no staging, no barrier before
 //           the stream; lanes of rows past M read row 0 and their results are dropped;
 //   post    one row (M = 1) that is the fp32 residual after a sublayer: x' = x + t / rms(t) * (1 + w) is formed
@@ -204,13 +211,22 @@ __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* red = reinterpret_cast<float*>(smem);            // [NW][64][4]
   float* rs = red + NW * 256;                             // [2][NW]
-  bf16_t* As = reinterpret_cast<bf16_t*>(rs + 16);        // post: the row (K)
+  constexpr int kOwn = (NW * 256 + 16) * 4;               // a chunk of weights per wave
+  bf16_t* As = reinterpret_cast<bf16_t*>(smem + kOwn + NW * 4096);  // post: the row (K)
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
   const int row = lane & 15, g = lane >> 4;
   constexpr int CW = HALF ? 8 : 16;
   const int K = p.K, KC = HALF ? K >> 8 : K >> 7, n0 = blockIdx.x * CW;
   const int rc = HALF ? row & 7 : row, koff = HALF && row >= 8 ? K >> 1 : 0;  // column / row of the lane, its K half
-  const u32x4* wp = reinterpret_cast<const u32x4*>(p.W + (size_t)(n0 + rc) * K + koff + 8 * g);
+  // load s of a chunk: operand column 4 s + g, 16 bytes each of its 16 lanes -> LDS, 16-byte piece q of column v at place q ^ v -> as
+  // the MFMA reads them
+  unsigned char* mine = smem + kOwn + wave * 4096;
+  const u32x4* wp[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int v = 4 * s + g;
+    wp[s] = reinterpret_cast<const u32x4*>(p.W + (size_t)(n0 + (HALF ? v & 7 : v)) * K + (HALF && v >= 8 ? K >> 1 : 0)) + row;
+  }
   const u32x4* ap = POST ? nullptr : reinterpret_cast<const u32x4*>(p.A + (size_t)(rc < p.M ? rc : 0) * p.lda + koff + 8 * g);
   u32x4 wr[D][4], ar[POST ? 1 : D][4];
   auto load = [&](int d, int i) {
@@ -219,7 +235,7 @@ __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       if constexpr (!POST) ar[d][s] = ap[(size_t)c * 16 + 4 * s];
-      wr[d][s] = __builtin_nontemporal_load(wp + (size_t)c * 16 + 4 * s);
+      wr[d][s] = __builtin_nontemporal_load(wp[s] + (size_t)c * 16);
     }
   };
   const int n = KC > wave ? (KC - wave + NW - 1) / NW : 0;
@@ -278,11 +294,16 @@ __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
       const int i = i0 + d;
       if (i < n) {  // (uniform)
 #pragma unroll
+        for (int s = 0; s < 4; ++s) *reinterpret_cast<u32x4*>(mine + 256 * (4 * s + g) + 16 * (row ^ (4 * s + g))) = wr[d][s];
+        u32x4 wt[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) wt[s] = *reinterpret_cast<const u32x4*>(mine + 256 * row + 16 * ((4 * s + g) ^ row));
+#pragma unroll
         for (int s = 0; s < 4; ++s) {
           u32x4 a;
           if constexpr (POST) a = *reinterpret_cast<const u32x4*>(As + koff + 128 * (wave + NW * i) + 32 * s + 8 * g);
           else a = ar[d][s];
-          acc = mfma_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, wr[d][s]), acc);
+          acc = mfma_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, wt[s]), acc);
         }
         if (i + D < n) load(d, i + D);
       }
@@ -317,8 +338,8 @@ __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
 
 template <int NW, int D, int NV, bool HALF>
 static int post_gemv_go(const PostGemvParams& p, int act, hipStream_t s) {
-  const size_t lds = (size_t)(NW * 256 + 16) * 4 + (NV > 0 ? (size_t)p.K * 2 : 0);
-  if (lds > 64 * 1024) return LLJ_EINVAL;
+  const size_t lds = (size_t)(NW * 256 + 16) * 4 + NW * 4096 + (NV > 0 ? (size_t)p.K * 2 : 0);
+  if (lds > 160 * 1024) return LLJ_EINVAL;
   const dim3 grid(p.N / (HALF ? 8 : 16)), nt(NW * 64);
   if (act == 2) hipLaunchKernelGGL((post_gemv_kernel<NW, D, NV, 2, HALF>), grid, nt, lds, s, p);
   else if (act) hipLaunchKernelGGL((post_gemv_kernel<NW, D, NV, 1, HALF>), grid, nt, lds, s, p);
@@ -335,11 +356,13 @@ static int post_gemv_launch(const PostGemvParams& p, int act, hipStream_t s) {
   const bool half = p.M <= kHalfRows && p.N / 16 < 256 && p.K % 256 == 0 && p.K >= 1024;
   if constexpr (NV > 0) {  // (the thread count is post_threads')
     if (post_threads(p.K) == 512) return half ? post_gemv_go<8, 4, NV, true>(p, act, s) : post_gemv_go<8, 4, NV, false>(p, act, s);
-    return half ? post_gemv_go<4, 4, NV, true>(p, act, s) : post_gemv_go<4, 4, NV, false>(p, act, s);
+    return half ? post_gemv_go<4, 3, NV, true>(p, act, s) : post_gemv_go<4, 4, NV, false>(p, act, s);
   } else {
-    // waves: 8 for long K, so that a wave's chunks stay within a few rounds of the D in flight
-    if (half) return p.K > 4096 ? post_gemv_go<8, 5, 0, true>(p, act, s) : post_gemv_go<4, 4, 0, true>(p, act, s);
-    return p.K > 2048 ? post_gemv_go<8, 4, 0, false>(p, act, s) : post_gemv_go<4, 4, 0, false>(p, act, s);
+    // waves: 8 for long K, so that a wave's chunks stay within a few rounds of the D in flight. D: few enough that two workgroups
+    // share a CU and one streams while the other starts and ends (8 rows, us at D = 2 / 3 / 4: 4096 -> 12544 22.4 / 25.6 / 26.3,
+    // 2048 -> 8448 10.9 / 10.3 / 10.6; halves, 16512 -> 4096 34.1 / 32.9 / 34.8, 2048 -> 2048, whose waves have two chunks, 4.2 / 4.9 / 5.4)
+    if (half) return p.K > 4096 ? post_gemv_go<8, 3, 0, true>(p, act, s) : post_gemv_go<4, 2, 0, true>(p, act, s);
+    return p.K > 2048 ? post_gemv_go<8, 2, 0, false>(p, act, s) : post_gemv_go<4, 3, 0, false>(p, act, s);
   }
 }
 
