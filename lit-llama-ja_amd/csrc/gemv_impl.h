@@ -1736,11 +1736,12 @@ static inline int device_cus() {
 // (M >= 2: one staged A image of M rows per CU instead of per tile, 1.966 -> 1.865 ms at 7B
 // bs=8); a single row keeps one tile per workgroup, where several workgroups per CU interleave
 // on each SIMD (measured 7B bs=1: 1.205 ms with one tile, 1.305 ms with three per workgroup).
-// Below LLJ_TPW_MIN_M rows the staged image is small and one tile per workgroup wins (7B
-// decode ms/token, tiles per workgroup 1 vs ceil(tiles / CUs): bs=2 1.427 vs 1.509, bs=4 1.574
-// vs 1.646, bs=6 1.683 vs 1.722, bs=8 1.889 vs 1.793).
+// All batched rows (2..8), streamed rows among them: each chunk's rows are read, normalized and turned into fragments once for
+// the workgroup's tiles. us per step, one tile per workgroup and ceil(tiles / CUs): 7B gptq.int4 2 rows 1,431 and 1,288, 4 rows
+// 1,457 and 1,304; 13B 2 rows 2,705 and 2,056, 6 rows 2,879 and 2,360; 7B gptq.int8 2 rows 1,922 and 1,873, 4 rows 1,983 and 1,950.
+// The same sums.
 #ifndef LLJ_TPW_MIN_M
-#define LLJ_TPW_MIN_M 7
+#define LLJ_TPW_MIN_M 2
 #endif
 static inline int pick_tpw(int ntiles, int M) {
   if (M < LLJ_TPW_MIN_M) return 1;

@@ -339,13 +339,19 @@ __global__ __launch_bounds__(NW * 64) void post_gemv_kernel(PostGemvParams p) {
 template <int NW, int D, int NV, bool HALF>
 static int post_gemv_go(const PostGemvParams& p, int act, hipStream_t s) {
   const size_t lds = (size_t)(NW * 256 + 16) * 4 + NW * 4096 + (NV > 0 ? (size_t)p.K * 2 : 0);
-  if (lds > 160 * 1024) return LLJ_EINVAL;
   const dim3 grid(p.N / (HALF ? 8 : 16)), nt(NW * 64);
-  if (act == 2) hipLaunchKernelGGL((post_gemv_kernel<NW, D, NV, 2, HALF>), grid, nt, lds, s, p);
-  else if (act) hipLaunchKernelGGL((post_gemv_kernel<NW, D, NV, 1, HALF>), grid, nt, lds, s, p);
-  else hipLaunchKernelGGL((post_gemv_kernel<NW, D, NV, 0, HALF>), grid, nt, lds, s, p);
-  LLJ_CHECK_LAUNCH();
-  return 0;
+  auto go = [&](auto kern) -> int {
+    if (lds > 64 * 1024) {
+      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(kern, grid, nt, lds, s, p);
+    LLJ_CHECK_LAUNCH();
+    return 0;
+  };
+  if (act == 2) return go(post_gemv_kernel<NW, D, NV, 2, HALF>);
+  if (act) return go(post_gemv_kernel<NW, D, NV, 1, HALF>);
+  return go(post_gemv_kernel<NW, D, NV, 0, HALF>);
 }
 
 constexpr int kHalfRows = 8;  // most rows of the half-K forms
@@ -366,7 +372,7 @@ static int post_gemv_launch(const PostGemvParams& p, int act, hipStream_t s) {
   }
 }
 
-constexpr int kPostMaxK = 28544;  // widest weight rows of the post form, whose row lies in LDS; llj_streams_linear keeps the same limit
+constexpr int kPostMaxK = 28544;  // widest weight rows of the post form, whose row lies in LDS (96 KB with the waves' patches); llj_streams_linear keeps the same limit
 
 template <int PRO>
 static int rowdot_act(const RowDotParams& r, int act, hipStream_t s) {

@@ -776,3 +776,9 @@ def test_one_row_of_the_block_vs_float64(hip, K, H):
     for got, want in ((q[9].view(nh, hs), rot(qkv[0])), (kc[0, :, 29 % S], rot(qkv[1])), (vc[0, :, 29 % S], qkv[2])):
         assert float((got.double() - want).abs().max()) <= 2.0 ** -6 * float(want.abs().max())
     assert float(q[:9].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("N", [48, 4096])
+def test_post_linear_widest_row(hip, N):
+    """The post form at its widest row, whose LDS is past 64 KB, in both tile widths."""
+    test_post_linear(hip, 8192, 28544, N, 0)
