@@ -8,6 +8,7 @@
 // CPU config of generate.py:121): LLaMA.forward routes an fp32 model here whatever its shape.
 #include "common.h"
 #include "elem.h"
+#include "generic_attention.h"
 #include "generic_gemm.h"
 #include "generic_rows.h"
 #include "lit_llama_amd.h"
@@ -503,6 +504,14 @@ int llj_g_attention(const void* q, const void* kcache, const void* vcache, void*
   const size_t lds = (size_t)(S + C / n_head) * 4;
   LLJ_REQUIRE(lds <= 64 * 1024);
   hipStream_t s = (hipStream_t)stream;
+  // The tiles from 1,024 (row, head) pairs on: below, one workgroup per pair is a shorter chain (us, pairs -> tiles; fp32, heads of 78:
+  // 4 rows of 10 heads 4.8 and 7.6, 100 rows 9.2 and 10.4, 128 rows 15.0 and 10.3, 1,000 rows 397 and 74; 301 rows of 32 heads of
+  // 128 137 and 37).
+  if (T >= kGaRows && (long)B * T * n_head >= 1024) {
+    const int e = dt == 0 ? ga_launch((const bf16_t*)q, (const bf16_t*)kcache, (const bf16_t*)vcache, (bf16_t*)y, pos, B, T, C, n_head, S, s)
+                          : ga_launch((const float*)q, (const float*)kcache, (const float*)vcache, (float*)y, pos, B, T, C, n_head, S, s);
+    if (e != 1) return e;
+  }
   LLJ_DT(dt, hipLaunchKernelGGL(g_attention_kernel<bf16_t>, dim3(B * T, n_head), dim3(256), lds, s, (const bf16_t*)q,
                                 (const bf16_t*)kcache, (const bf16_t*)vcache, (bf16_t*)y, pos, T, C, n_head, S),
          hipLaunchKernelGGL(g_attention_kernel<float>, dim3(B * T, n_head), dim3(256), lds, s, (const float*)q,

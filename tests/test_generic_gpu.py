@@ -378,3 +378,29 @@ def test_generic_rope_attention_vs_separate_calls(dt, B, nh, hs, S, p):
     want, mass = ((w[..., None] * t).sum(2).reshape(B, C) for t in (v2[:, :, :n].double(), v2[:, :, :n].double().abs()))
     loss = 2.0 ** -24 * (n + 16 + 2 * (hs // 2 + 8) * float(size.max()))
     assert ((y.double() - want).abs() <= mass * loss + (0.0 if dt else 2.0 ** -8 * 1.01) * want.abs() + 1e-30).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,nh,hs,S,p0", [(1, 301, 32, 128, 301, 0), (2, 67, 10, 78, 80, 5), (1, 130, 8, 1, 130, 0), (3, 49, 8, 13, 64, 40),
+                                            (1, 1030, 1, 256, 1030, 0), (2, 129, 5, 101, 200, 0), (1, 70, 16, 64, 72, 60), (1, 128, 9, 250, 128, 0)])
+def test_prompt_attention_tiles(hip, dtype, B, T, nh, hs, S, p0):
+    """llj_g_attention on tiles of 16 rows and 64 keys, any head size (also one whose vectors are too many for the tiles), remainders of
+    both, rows whose positions have gone round the cache, unseen slots that hold NaN. Against float64: the output's own rounding, and in
+    fp32 the scores' (values of some units, sums of hs products)."""
+    from lit_llama import _hip
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    C = nh * hs
+    q, k, v = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((B, T, C), (B, nh, S, hs), (B, nh, S, hs)))
+    pos = torch.arange(p0, p0 + T, dtype=torch.int32, device="cuda")
+    seen = (pos + 1).clamp(max=S)
+    k[:, :, int(seen.max()):], v[:, :, int(seen.max()):] = float("nan"), float("nan")
+    y = torch.full((B, T, C), float("nan"), dtype=dtype, device="cuda")
+    _hip.call("llj_g_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), y.data_ptr(), pos.data_ptr(), B, T, C, nh, S,
+              int(dtype == torch.float32), _hip.stream())
+    torch.cuda.synchronize()
+    mask = torch.arange(S, device="cuda")[None] < seen[:, None]
+    s = q.double().view(B, T, nh, hs).transpose(1, 2).contiguous() @ k.double().nan_to_num().transpose(2, 3).contiguous() * hs ** -0.5
+    want = (torch.softmax(s.masked_fill(~mask, float("-inf")), -1) @ v.double().nan_to_num()).transpose(1, 2).reshape(B, T, C)
+    assert (y.double() - want).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
