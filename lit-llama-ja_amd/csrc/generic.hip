@@ -449,7 +449,21 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
     else if (bits == 8) LLJ_GG_BITS(8, VE); \
     else LLJ_GG_BITS(2, VE);              \
   } while (0)
-  if (wkind == 0) {
+  if (wkind == 1 && dt == 1 && !fine && K % 32 == 0 && fits(x, ldx, 4) && fits(W, K, 4)) {
+    auto go = [&](auto kern, int stages) {
+      const size_t lds = (size_t)stages * (kGgBM + kGgBN) * kGgRow;
+      const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return (int)e;
+      hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, (const float*)x, ldx, M, K, (const float*)W, N, (float*)y, ldy, (const float*)resid, ldr,
+                         part, per);
+      return 0;
+    };
+    // three buffers, except where three workgroups to a CU are one round and two are not (37 rows, 4096 -> 12288, 768 workgroups: 79 us
+    // for 94 with three buffers; 301 rows, 480 workgroups: 278 with three, 291 with two, 324 through registers)
+    const long wgs = (long)mt * nt * splits;
+    const int e = wgs > 512 && wgs <= 768 ? go(gg_dma_kernel<2>, 2) : go(gg_dma_kernel<3>, 3);
+    if (e) return e;
+  } else if (wkind == 0) {
     if (fits(x, ldx, 4)) LLJ_GG_CODES(4);
     else LLJ_GG_CODES(1);
   } else if (dt == 1) {

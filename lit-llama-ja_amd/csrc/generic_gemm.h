@@ -243,6 +243,91 @@ __global__ __launch_bounds__(512 / J, 2) void gg_kernel(const T* __restrict__ x,
   }
 }
 
+// gg_kernel's dense fp32 form above kGgFineK for rows of whole tiles (K and the row strides multiples of 32 and 4 elements, rows aligned):
+// the same sums, the tiles brought to LDS by global_load_lds (no registers, no store), ST - 1 ahead of the one in use. The wait for a
+// tile is a counted vmcnt and a plain barrier. Three buffers leave two workgroups to a CU, two buffers three.
+typedef __attribute__((address_space(3))) void gg_lds_t;
+template <int N>
+__device__ __forceinline__ void gg_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+template <int ST>
+__global__ __launch_bounds__(256, ST == 2 ? 3 : 2) void gg_dma_kernel(const float* __restrict__ x, int ldx, int M, int K, const float* __restrict__ W, int N,
+                                                        float* __restrict__ y, int ldy, const float* resid, int ldr, float* __restrict__ part,
+                                                        int split_tiles) {
+  constexpr int J = 2, KT = 32, kStage = (kGgBM + kGgBN) * kGgRow, ND = (kGgBM + kGgBN) / 32;
+  extern __shared__ __align__(16) char gg_stages[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+  const int mt = (M + kGgBM - 1) / kGgBM, local = blockIdx.x >> 3;
+  const int nt = (int)(blockIdx.x & 7) + 8 * (local / mt);
+  if (nt * kGgBN >= N) return;
+  const int m0 = (local % mt) * kGgBM, n0 = nt * kGgBN;
+  const int t0 = blockIdx.y * split_tiles, all = K / KT, t1 = min(all, t0 + split_tiles);
+  // eight rows of 128 bytes an instruction; lane l's 16 bytes land at place l % 8 of row l / 8, so they are chunk (l % 8) ^ (row / 2 % 8)
+  const float* src[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const int row = 8 * (4 * i + wave) + (lane >> 3), c = (lane & 7) ^ (row >> 1 & 7);  // of the stage: 64 of x, 128 of W
+    src[i] = (i < 2 ? x + (size_t)min(m0 + row, M - 1) * ldx : W + (size_t)min(n0 + row - kGgBM, N - 1) * K) + 4 * c;
+  }
+  auto stage = [&](int buf, int t) {
+    const int tt = t < t1 ? t : t1 - 1;  // past the range: a copy that is not read
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+      __builtin_amdgcn_global_load_lds(src[i] + (size_t)tt * KT, (gg_lds_t*)(gg_stages + buf * kStage + (4 * i + wave) * 1024), 16, 0, 0);
+  };
+  f32x16 mid[J] = {}, tot[J] = {};
+  const int nw = (wave >> 1) * 32 * J;  // the wave's first column
+  const int ra = gg_at((wave & 1) * 32 + (lane & 31), lane >> 5), rb = gg_at(kGgBM + nw + (lane & 31), lane >> 5);
+  stage(0, t0);
+  if constexpr (ST == 3) stage(1, t0 + 1);
+  int buf = 0;
+  for (int t = t0; t < t1; ++t) {
+    gg_wait<(ST - 2) * ND>();  // tile t has landed, the next one may be on its way
+    __builtin_amdgcn_s_barrier();  // for every wave; and all are done with the buffer of tile t - 1
+    stage(buf == 0 ? ST - 1 : buf - 1, t + ST - 1);
+    const char* b = gg_stages + buf * kStage;
+    f32x4 fa[4], fb[J][4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      fa[g] = *reinterpret_cast<const f32x4*>(b + (ra ^ g << 5));
+#pragma unroll
+      for (int j = 0; j < J; ++j) fb[j][g] = *reinterpret_cast<const f32x4*>(b + (rb ^ g << 5) + 32 * j * kGgRow);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (read one by one in front of their products, each waited alone)
+    f32x16 acc[J] = {};
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[g][e], fb[j][g][e], acc[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < J; ++j) mid[j] += acc[j];
+    if (((t - t0) & 7) == 7) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        tot[j] += mid[j];
+        mid[j] = f32x16{};
+      }
+    }
+    buf = buf == ST - 1 ? 0 : buf + 1;
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    tot[j] += mid[j];
+    const int n = n0 + nw + 32 * j + (lane & 31);
+    if (n >= N) continue;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int m = m0 + (wave & 1) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+      if (m >= M) continue;
+      if (part) part[((size_t)blockIdx.y * M + m) * N + n] = tot[j][i];
+      else y[(size_t)m * ldy + n] = resid ? resid[(size_t)m * ldr + n] + tot[j][i] : tot[j][i];
+    }
+  }
+}
+
 // y = the splits' sums, added pairwise (and the residual), as gg_kernel's own epilogue
 template <typename T>
 __global__ __launch_bounds__(256) void gg_reduce_kernel(const float* __restrict__ part, int splits, int M, int N, T* __restrict__ y,
