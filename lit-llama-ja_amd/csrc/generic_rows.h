@@ -127,7 +127,9 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
 // One token per sequence: rotary positions of q and k (g_rope_kv_kernel), k and v into cache slot p % S, and causal attention over
 // the cache (g_attention_kernel). Block (row, head) of 512 threads -- a few tens of blocks with a chain of memory trips each: 16
 // lanes per key and 128 keys at a time, then the values with the threads split over dimension pairs and up to kGrKeyGroups
-// interleaved groups of keys. The first keys and values are loaded before the rotation. LDS: S + hs (3 + groups) floats.
+// interleaved groups of keys. The first keys and values are loaded before the rotation, without a branch around any of them (10 heads
+// of 78, bf16, us behind branches -> this: 40 keys 6.4 -> 5.8, 110 keys 7.0 -> 6.1, 500 keys 16.7 -> 14.8; the next 128 keys
+// requested a pass ahead as well: 6.2, 6.5, 14.6). LDS: S + hs (3 + groups) floats.
 constexpr int kGrThreads = 512, kGrKeyGroups = 14;
 __host__ __device__ inline int gr_groups(int P) { return P > kGrThreads ? 1 : P * kGrKeyGroups > kGrThreads ? kGrThreads / P : kGrKeyGroups; }
 template <typename T>
@@ -155,8 +157,8 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
     for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int j = j0 + 32 * u, i = i0 + 16 * q + sub;
-        kw[u][q] = j < nvis && i < P ? reinterpret_cast<const pair*>(kc + cb + (size_t)j * hs)[i] : pair(0);
+        const int j = min(j0 + 32 * u, S - 1), i = min(i0 + 16 * q + sub, P - 1);  // (a valid pair, not used past the last: no branch)
+        kw[u][q] = reinterpret_cast<const pair*>(kc + cb + (size_t)j * hs)[i];
       }
   };
   const int G = gr_groups(P), g = P > kGrThreads ? 0 : tid / P;
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
   pair vw[VU];
   keys(kg, 0);
 #pragma unroll
-  for (int u = 0; u < VU; ++u) vw[u] = g < G && g + G * u < nvis ? vr[(size_t)(g + G * u) * P] : pair(0);
+  for (int u = 0; u < VU; ++u) vw[u] = vr[(size_t)min(min(g, G - 1) + G * u, S - 1) * P];
   // in flight while q and k are rotated; the rows that this workgroup writes come from LDS
   for (int i = tid; i < P; i += kGrThreads) {
     const float c = rope[((size_t)p * P + i) * 2], s = rope[((size_t)p * P + i) * 2 + 1];
