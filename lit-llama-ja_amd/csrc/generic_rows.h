@@ -3,11 +3,15 @@
 //
 // Decode of these models (780 wide, 3.6 MB per matrix) is bound by latency: what counts is how many dependent memory trips and
 // launches a layer has. A wave takes one output column (four where there are columns enough for every CU), its lanes
-// consecutive pieces of K, and issues the weights' loads of up to 8 pieces at once before it needs the first, in the
-// norm-fused forms before the norm. The residual's RMSNorm is computed by every workgroup for itself (a read of a few KB) in the
-// order of g_rmsnorm_kernel, so a layer is 5 launches instead of 10. 125M bf16, one row, per launch: rms_1 and c_attn 4.4 + 10.1 ->
-// 4.9 us, c_proj and mlp.c_proj 15.8 -> 3.7 on average, rms_2, c_fc1, c_fc2 and silu * mul 29 -> 6.0, rotary positions and
-// attention over 130 keys 18.3 -> 8.2 (256 threads 9.8, and without the early loads 11.2); lm_head 51.7 -> 14.8 (3.7 TB/s).
+// consecutive pieces of K. The residual's RMSNorm is computed by every workgroup for itself (a read of a few KB) in the order of
+// g_rmsnorm_kernel, so a layer is 5 launches instead of 10. Loads come back in order, so each wave requests what it needs first
+// first: the norm's row and weights (up to 1,024 values; beyond that they are read again), the residual, then the weights' pieces,
+// and all without a branch, from clamped addresses whose values go unused. Where the next pieces would be mostly past K (the
+// plain form's 5th to 8th) a branch is cheaper than the loads. us per launch, one row, weights first and all loads in
+// branches -> this: bf16, K = 780: rms_1 and c_attn 4.6 -> 4.0, c_proj 2.8 -> 2.6, rms_2, c_fc1, c_fc2 and silu * mul 5.8 -> 4.6,
+// mlp.c_proj (K = 2,080) 3.2 -> 3.0, lm_head 14.7 -> 11.0 (5.1 TB/s); four rows 10.6 -> 8.3, 4.7 -> 4.5, 13.1 -> 9.7, 5.7 -> 5.5,
+// 35.1 -> 29.4; fp32, K = 512: the same to 0.2 less, lm_head 15.2 -> 12.6; bf16, K = 2,100: 12.2 -> 11.2, 16.4 -> 14.3. Two
+// sets of 4 pieces by turns instead: 4.1, 2.7, 4.8, 3.5, 11.2.
 #pragma once
 #include "common.h"
 #include "elem.h"
@@ -27,7 +31,7 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
                                                      T* __restrict__ y, int ldy, const T* resid, int ldr) {
   extern __shared__ __align__(16) char gr_lds[];
   typedef T vec __attribute__((ext_vector_type(VE)));
-  constexpr int U = NC == 1 ? 8 : 4, NT = MODE == GR_SWIGLU ? 2 : NC;
+  constexpr int U = MODE == GR_PLAIN && NC == 1 ? 8 : 4, NT = MODE == GR_SWIGLU ? 2 : NC;
   const int tid = threadIdx.x, lane = tid & 63, n0 = (blockIdx.x * 4 + (tid >> 6)) * NC;
   const T* wr[NT];
 #pragma unroll
@@ -35,14 +39,33 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
     const int n = MODE == GR_SWIGLU ? n0 : n0 + t;
     wr[t] = (MODE == GR_SWIGLU && t ? W2 : W) + (size_t)(n < N ? n : N - 1) * K;
   }
+  constexpr int RU = MODE == GR_PLAIN ? 1 : 4;
+  T xf[MB][RU], nf[RU], rv[MB];
+  if constexpr (MODE != GR_PLAIN) {
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      const int k = min(tid + 256 * u, K - 1);
+      nf[u] = nw[k];
+#pragma unroll
+      for (int r = 0; r < MB; ++r) xf[r][u] = x[(size_t)min(r, M - 1) * ldx + k];
+    }
+  }
+  if constexpr (MODE != GR_SWIGLU) {
+    const T* rp = resid ? resid + min(n0 + min(lane, NC - 1), N - 1) : x;
+#pragma unroll
+    for (int r = 0; r < MB; ++r) rv[r] = rp[resid ? (size_t)min(r, M - 1) * ldr : 0];
+  }
   vec wv[NT][U];
+  // piece u of a row: the first 4 from a valid address whatever k is
+  auto piece = [&](const T* p, int k, int u) {
+    if (u < 4 || k < K) return *reinterpret_cast<const vec*>(p + (u < 4 ? min(k, K - VE) : k));
+    return vec(0);
+  };
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + (u * 64 + lane) * VE;
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wv[t][u] = k < K ? *reinterpret_cast<const vec*>(wr[t] + k) : vec(0);
-    }
+      for (int t = 0; t < NT; ++t) wv[t][u] = piece(wr[t], k0 + (u * 64 + lane) * VE, u);
   };
   fetch(0);
   T* xs = reinterpret_cast<T*>(gr_lds);
@@ -52,10 +75,11 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
     for (int r = 0; r < MB; ++r) {
       if (r < M) {
         float ss = 0.f;
-        for (int k = tid; k < K; k += 256) {
-          const float v = ldv(x, (size_t)r * ldx + k);
-          ss += rnd<T>(v * v);
-        }
+        auto add = [&](float v) { ss += rnd<T>(v * v); };
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+          if (tid + 256 * u < K) add(ldv(&xf[r][u], 0));
+        for (int k = tid + 256 * RU; k < K; k += 256) add(ldv(x, (size_t)r * ldx + k));
         ss = wave_sum(ss);
         if (lane == 0) red[r][tid >> 6] = ss;
       }
@@ -66,7 +90,10 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
       if (r < M) {
         const float tot = red[r][0] + red[r][1] + red[r][2] + red[r][3];
         const float s = rnd<T>(rsqrtf(rnd<T>(rnd<T>(tot / (float)K) + eps)));
-        for (int k = tid; k < K; k += 256) stv(xs, r * K + k, ldv(nw, k) * rnd<T>(ldv(x, (size_t)r * ldx + k) * s));
+#pragma unroll
+        for (int u = 0; u < RU; ++u)
+          if (tid + 256 * u < K) stv(xs, r * K + tid + 256 * u, ldv(&nf[u], 0) * rnd<T>(ldv(&xf[r][u], 0) * s));
+        for (int k = tid + 256 * RU; k < K; k += 256) stv(xs, r * K + k, ldv(nw, k) * rnd<T>(ldv(x, (size_t)r * ldx + k) * s));
       }
     }
     __syncthreads();
@@ -81,15 +108,13 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
 #pragma unroll
     for (int r = 0; r < MB; ++r) {
       if (r < M) {
+        const T* xr = MODE == GR_PLAIN ? x + (size_t)r * ldx : xs + r * K;
         vec xv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int k = k0 + (u * 64 + lane) * VE;
-          const T* xr = MODE == GR_PLAIN ? x + (size_t)r * ldx : xs + r * K;
-          xv[u] = k < K ? *reinterpret_cast<const vec*>(xr + k) : vec(0);
-        }
+        for (int u = 0; u < U; ++u) xv[u] = piece(xr, k0 + (u * 64 + lane) * VE, u);
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+          if (k0 + (u * 64 + lane) * VE >= K) continue;
 #pragma unroll
           for (int e = 0; e < VE; ++e) {
             T xe = xv[u][e];
@@ -99,6 +124,7 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
               acc[r][t] += ldv(&xe, 0) * ldv(&we, 0);
             }
           }
+        }
       }
     }
   }
@@ -115,7 +141,7 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
         for (int t = 0; t < NC; ++t) {
           if (lane == t && n0 + t < N) {
             float v = s[t];
-            if (resid) v = ldv(resid, (size_t)r * ldr + n0 + t) + v;
+            if (resid) v = ldv(&rv[r], 0) + v;
             stv(y, (size_t)r * ldy + n0 + t, v);
           }
         }
