@@ -3,11 +3,19 @@
 // Bound: the weights' bytes. A workgroup owns a range of output columns; each of its NW waves keeps its own slice of the row (SL
 // pieces of 512 values, 8 per lane) in registers and streams that slice of column after column -- 1 KiB of consecutive
 // bytes per load, two rounds of loads in flight -- into fp32 multiply-adds. The lanes' sums meet over 16 lanes (DPP), the rest
-// through LDS once per workgroup, where the epilogue also runs, a thread per column with its operands loaded ahead. The MFMA forms (gemv_impl.h,
-// post_gemv.hip), made for several rows, read 16 columns x 64 bytes per load and leave HBM at 60 % of what these reach. In a
-// graph, us (TB/s), MFMA form -> this:
-//   4096 -> 12288   22.0 (4.6) -> 19.0 (5.3)     4096 -> 22016   38.6 (4.7) -> 31.5 (5.7)     4096 -> 4096    8.6 (3.9) -> 8.3 (4.1)
-//   11008 -> 4096   21.7 (4.2) -> 17.3 (5.2)     4096 -> 32000   51.2 (5.1) -> 44.1 (5.9)     2048 -> 2048    7.0 (1.2) -> 4.8 (1.8)
+// through LDS once per workgroup, where the epilogue also runs, a thread per column with its operands loaded ahead.
+//
+// Loads come back in order, and one behind a branch is waited for with all that precede it. So no load here is behind a branch
+// (a place past C or a column past the range is a valid one instead, left out of the sums), the row and the epilogue's operands
+// are requested before the weights, and the loop's last rounds are written out. A range of one round has a kernel of its own size,
+// since loads of columns that are not there cost as much in the caches as others. In a graph, us (TB/s), loads in branches
+// -> this:
+//   640 -> 1920, norm     4.9 -> 3.8           1792 -> 640            4.5 -> 3.6           640 -> 35008, norm   13.7 -> 10.6 (4.2)
+//   2048 -> 6144, norm    8.4 -> 6.6 (3.8)     2048 -> 2048           4.8 -> 4.1           2048 -> 2 x 5632    11.9 -> 10.4 (4.4)
+//   4096 -> 12288, norm  20.8 -> 20.0 (5.0)    4096 -> 4096           9.0 -> 8.1 (4.1)     4096 -> 2 x 11008   36.0 -> 34.3 (5.3)
+//   11008 -> 4096        19.0 -> 18.6 (4.8)    4096 -> 32000, norm   50.3 -> 48.9 (5.4)    13824 -> 5120       28.4 -> 27.9 (5.1)
+// Rounds of 8 columns up to 2048 values: 11.5, 8.4, 11.1 for 10.6, 6.6, 10.4; of 2: 11.8, 6.8, 10.4. The MFMA forms (gemv_impl.h,
+// post_gemv.hip), made for several rows, read 16 columns x 64 bytes per load: 21.7 for 11008 -> 4096, 7.0 for 2048 -> 2048.
 // (a wave per column, each with the whole row, measured the same without a prologue, but repeats the norm in ten times the
 // workgroups.) The grid is about 2048 waves, 8 per CU with 16 KiB in flight each; 256 or 1024 workgroups of the same waves
 // lose 1-4 %.
@@ -56,27 +64,27 @@ struct RowDotParams {
 constexpr int kRdStreams = 4;
 constexpr int kRdMaxC = 16384;
 
-template <int NW, int SL, int PRO, int EPI>
+// ONE: columns of the largest range where a single round of loads holds them, or 0.
+template <int NW, int SL, int PRO, int EPI, int ONE>
 __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
   extern __shared__ __align__(16) float rd_part[];  // [column][NW * 4]
   __shared__ float red[2][NW];
-  constexpr int CB = SL == 1 ? 8 : SL == 2 ? 4 : 2;  // columns per round of loads
+  constexpr int CB = ONE ? ONE : SL <= 2 ? 4 : 2;  // columns per round of loads
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
   const int units = p.N >> 1;
   const int c0 = 2 * (int)((long)blockIdx.x * units / gridDim.x), c1 = 2 * (int)((long)(blockIdx.x + 1) * units / gridDim.x);
   const int k0 = wave * (SL * 512) + lane * 8;  // slice s: k0 + 512 s
+  int kv[SL];  // (past C: a valid place, whose values are left out of the sums)
+#pragma unroll
+  for (int s = 0; s < SL; ++s) kv[s] = k0 + 512 * s < p.C ? k0 + 512 * s : 0;
   u32x4 wv[2][CB][SL];
-  auto fetch = [&](int b, int c) {
-    if (c >= c1) return;
+  auto fetch = [&](int b, int c) {  // (columns past c1: the last pair again)
 #pragma unroll
     for (int i = 0; i < CB; ++i) {
-      const int n = min(c + i, c1 - 1);
-      const bf16_t* r = EPI == RD_SWIGLU ? ((n & 1) ? p.W2 : p.W) + (size_t)(n >> 1) * p.K : p.W + (size_t)n * p.K;
+      const int n = min(c + (i & ~1), c1 - 2) + (i & 1);
+      const bf16_t* r = EPI == RD_SWIGLU ? ((i & 1) ? p.W2 : p.W) + (size_t)(n >> 1) * p.K : p.W + (size_t)n * p.K;
 #pragma unroll
-      for (int s = 0; s < SL; ++s) {
-        const int k = k0 + 512 * s;
-        wv[b][i][s] = k < p.C ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(r + k)) : u32x4{0, 0, 0, 0};
-      }
+      for (int s = 0; s < SL; ++s) wv[b][i][s] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(r + kv[s]));
     }
   };
 
@@ -91,13 +99,16 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
     const int n = c0 + j < c1 ? c0 + j : c0;
     Operand o{};
     if constexpr (EPI == RD_RESID) o.v = bf2f(p.out[n]);
-    if constexpr (EPI == RD_STORE || EPI == RD_GLU) o.v = p.bias ? p.bias[n] : 0.f;
+    if constexpr (EPI == RD_STORE || EPI == RD_GLU) {
+      const float v = (p.bias ? p.bias : reinterpret_cast<const float*>(p.W))[p.bias ? n : 0];
+      o.v = p.bias ? v : 0.f;
+    }
     if constexpr (EPI == RD_QKV) {  // model.py:204-228: RoPE in fp32 on the bf16 output, k / v to ring slot p % ring
       const int Cd = p.n_head * p.hs, nc = n % Cd, h = nc / p.hs, dd = nc - h * p.hs;
       const int b = p.T == 1 ? p.m : p.m / p.T, ps = p.pos[p.m - b * p.T];
       o.region = n / Cd;
       o.odd = dd & 1;
-      o.cs = o.region < 2 ? *reinterpret_cast<const float2*>(p.rope + ((size_t)ps * (p.hs >> 1) + (dd >> 1)) * 2) : float2{1.f, 0.f};
+      o.cs = *reinterpret_cast<const float2*>(p.rope + ((size_t)ps * (p.hs >> 1) + (dd >> 1)) * 2);
       o.at = o.region == 0 ? (size_t)p.m * Cd + nc : (((size_t)b * p.n_head + h) * p.ring + ps % p.ring) * p.hs + dd;
     }
     return o;
@@ -119,12 +130,15 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
     u32x4 xv[SL], gv[SL];
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
-      const int k = k0 + 512 * s;
-      xv[s] = k < p.C ? *reinterpret_cast<const u32x4*>(p.A + k) : u32x4{0, 0, 0, 0};
-      if constexpr (PRO == RD_NORM) gv[s] = k < p.C ? *reinterpret_cast<const u32x4*>(p.w + k) : u32x4{0, 0, 0, 0};
+      xv[s] = *reinterpret_cast<const u32x4*>(p.A + kv[s]);
+      if constexpr (PRO == RD_NORM) gv[s] = *reinterpret_cast<const u32x4*>(p.w + kv[s]);
     }
-    fetch(0, c0);
     first = operand(tid);
+    fetch(0, c0);
+    if constexpr (!ONE) fetch(1, c0 + CB);
+#pragma unroll
+    for (int s = 0; s < SL; ++s)
+      if (k0 + 512 * s >= p.C) xv[s] = u32x4{0, 0, 0, 0};
 #pragma unroll
     for (int s = 0; s < SL; ++s)
 #pragma unroll
@@ -147,14 +161,23 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
     float sv[SL][kRdStreams][8];
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
-      const int k = k0 + 512 * s, kk = k < p.C ? k : 0;
-      tv[s] = *reinterpret_cast<const u32x4*>(p.t + kk);
-      gv[s] = *reinterpret_cast<const u32x4*>(p.w + kk);
+      tv[s] = *reinterpret_cast<const u32x4*>(p.t + kv[s]);
+      gv[s] = *reinterpret_cast<const u32x4*>(p.w + kv[s]);
 #pragma unroll
-      for (int q = 0; q < kRdStreams; ++q) ld8(p.x + (size_t)(q < p.S ? q : 0) * p.ldx + kk, sv[s][q]);  // (past S: a copy)
+      for (int q = 0; q < kRdStreams; ++q) ld8(p.x + (size_t)(q < p.S ? q : 0) * p.ldx + kv[s], sv[s][q]);  // (past S: a copy)
     }
-    fetch(0, c0);
+    float ot[kRdStreams], mx[kRdStreams][kRdStreams], in[kRdStreams];
+#pragma unroll
+    for (int t = 0; t < kRdStreams; ++t) {
+      const int tt = t < p.S ? t : 0;
+      ot[t] = p.so[tt];
+      in[t] = (p.si ? p.si : p.so)[tt];
+#pragma unroll
+      for (int q = 0; q < kRdStreams; ++q) mx[t][q] = p.sm[(q < p.S ? q : 0) * p.S + tt];
+    }
     first = operand(tid);
+    fetch(0, c0);
+    if constexpr (!ONE) fetch(1, c0 + CB);
     float sum = 0.f;
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
@@ -166,18 +189,18 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
       for (int t = 0; t < kRdStreams; ++t) {
         if (t < p.S) {  // (uniform)
           float n[8];
-          const float ot = p.so[t], in = p.si ? p.si[t] : 1.f;
+          const float it = p.si ? in[t] : 1.f;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) n[e] = ot * ((e & 1) ? bfhi(tv[s][e >> 1]) : bflo(tv[s][e >> 1]));
+          for (int e = 0; e < 8; ++e) n[e] = ot[t] * ((e & 1) ? bfhi(tv[s][e >> 1]) : bflo(tv[s][e >> 1]));
 #pragma unroll
           for (int q = 0; q < kRdStreams; ++q) {
-            const float a = q < p.S ? p.sm[q * p.S + t] : 0.f;
+            const float a = q < p.S ? mx[t][q] : 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) n[e] += a * sv[s][q][e];
           }
           if (mine) st8(p.xo + (size_t)t * p.ldx + k, n);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) xf[s][e] += in * n[e];
+          for (int e = 0; e < 8; ++e) xf[s][e] += it * n[e];
         }
       }
 #pragma unroll
@@ -206,21 +229,36 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
     for (int i = 0; i < CB; ++i) {
       float a = 0.f;
 #pragma unroll
-      for (int s = 0; s < SL; ++s)
+      for (int s = 0; s < SL; ++s) {
+        if (k0 + 512 * s >= p.C) continue;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           a = fmaf(bflo(wv[b][i][s][e]), xf[s][2 * e], a);
           a = fmaf(bfhi(wv[b][i][s][e]), xf[s][2 * e + 1], a);
         }
+      }
       a = row16_sum(a);
       if ((lane & 15) == 0 && c + i < c1) rd_part[(c + i - c0) * (NW * 4) + wave * 4 + (lane >> 4)] = a;
     }
   };
-  for (int c = c0; c < c1; c += 2 * CB) {
-    fetch(1, c + CB);
+  if constexpr (ONE) {
+    columns(0, c0);
+  } else {
+    int c = c0;
+    for (; c + 3 * CB < c1; c += 2 * CB) {
+      columns(0, c);
+      fetch(0, c + 2 * CB);
+      columns(1, c + CB);
+      fetch(1, c + 3 * CB);
+    }
     columns(0, c);
-    fetch(0, c + 2 * CB);
-    if (c + CB < c1) columns(1, c + CB);
+    if (c + 2 * CB < c1) {
+      fetch(0, c + 2 * CB);
+      columns(1, c + CB);
+      columns(0, c + 2 * CB);
+    } else if (c + CB < c1) {
+      columns(1, c + CB);
+    }
   }
   __syncthreads();
 
@@ -271,7 +309,12 @@ static int rowdot_go(const RowDotParams& p, hipStream_t s) {
   const long most = 48 * 1024 / (NW * 16) - 2;
   if ((long)p.N > most * grid) grid = (int)((p.N + most - 1) / most);
   const size_t lds = (size_t)2 * ((units + grid - 1) / grid) * NW * 16;
-  hipLaunchKernelGGL((rowdot_kernel<NW, SL, PRO, EPI>), dim3(grid), dim3(NW * 64), lds, s, p);
+  const int range = 2 * ((units + grid - 1) / grid);
+#define LLJ_RD(ONE) hipLaunchKernelGGL((rowdot_kernel<NW, SL, PRO, EPI, ONE>), dim3(grid), dim3(NW * 64), lds, s, p)
+  if (range <= 2) LLJ_RD(2);
+  else if (SL <= 2 && range <= 4) LLJ_RD(SL <= 2 ? 4 : 0);
+  else LLJ_RD(0);
+#undef LLJ_RD
   LLJ_CHECK_LAUNCH();
   return 0;
 }

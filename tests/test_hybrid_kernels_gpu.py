@@ -736,6 +736,24 @@ def test_one_row_vs_float64(hip, K, N, act):
     assert ((out[0].double() - want).abs() <= lim + 2.0 ** -8 * 1.01 * want.abs() + 1e-30).all()
 
 
+@pytest.mark.parametrize("K,grid", [(896, 1024), (4096, 512), (12288, 256)])
+def test_one_row_every_range(hip, K, grid):
+    """Ranges of 2 to 20 columns a workgroup (one round of loads, two, three, with and without a rest; N not a multiple of the
+    grid too): a column's sum has one order whatever the range, so 512 columns at a time (ranges of 2) give the same bits."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(1, K, generator=g, device="cuda").to(torch.bfloat16)
+    most = 2 * grid * 10
+    W = (torch.randn(most, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    want = torch.empty(1, most, dtype=torch.bfloat16, device="cuda")
+    for n in range(0, most, 512):
+        call("llj_rows_linear", 0, x, K, W[n:], None, want[:, n:], 512, 1, 512, K, 0.0, 0.0)
+    for units in range(1, 11):
+        for N in (2 * grid * units, 2 * grid * units - 320):
+            out = torch.full((1, most), -7.0, dtype=torch.bfloat16, device="cuda")
+            call("llj_rows_linear", 0, x, K, W, None, out, N, 1, N, K, 0.0, 0.0)
+            assert torch.equal(out[:, :N], want[:, :N]) and (out[:, N:] == -7).all(), N
+
+
 @pytest.mark.parametrize("K,H", [(512, 512), (640, 1792), (2048, 5632), (13824, 640)])
 def test_one_row_of_the_block_vs_float64(hip, K, H):
     """The four ops of a LLaMA block on bf16 weights with one row, row 9 of a longer call included (the last slice of eight),
