@@ -1261,6 +1261,11 @@ __device__ __forceinline__ void gemv_body(const GemvParams& p, const int nt0, un
   }
 #pragma unroll
   for (int d = 0; d < D; ++d) load(d, d);  // the weight stream starts before any A wait
+  if constexpr (EP == EP_QKV && FLAT) {  // the positions (their RoPE rows' addresses) are first read behind the weight requests:
+    // the compiler moved that arithmetic up, and its wait held the requests back (no instruction; 7B gptq.int4, 8 rows 10.2 -> 9.1 us).
+#pragma unroll
+    for (int q = 0; q < FQ; ++q) asm volatile("" : "+v"(f_ps[q])::"memory");  // One row keeps the wait: 7.6 us with and 8.2 without
+  }
   if constexpr (SNRM) {  // every wave reduces the partials itself (same order everywhere: one rstd per row)
     float ss[8];
 #pragma unroll
@@ -1827,7 +1832,9 @@ static int launch_mb(const GemvParams& p, hipStream_t s) {
   if constexpr (tpw_ok<WF, AM>() && MB > 1) {  // M == 1 (MB 1) always one tile: pick_tpw
     // the residual ops (8 chunks in flight) take at most 2 tiles per workgroup (3 and 4 spill;
     // C / 16 tiles need 2 only past 256 CUs' worth: 13B / 30B / 65B)
-    const int t = pick_tpw(p.N / 16, p.M);
+    // 2 and 3 rows on 8-bit codes keep one tile in the SwiGLU: 2 rows of 4096 -> 2 x 11008 19.9 us, 20.6 with three; 4 rows
+    // 20.8 and 20.8
+    const int t = WF == WF_W8 && EP == EP_SWIGLU && p.M < 4 ? 1 : pick_tpw(p.N / 16, p.M);
     switch (EP == EP_RESID && t > 2 ? 2 : t) {
       case 2: return launch_t<WF, AM, EP, MB, NW, 2>(p, s);
       case 3: if constexpr (EP != EP_RESID) return launch_t<WF, AM, EP, MB, NW, 3>(p, s); break;
