@@ -213,18 +213,24 @@ __device__ void stage_a(const GemvParams& p, bf16_t* As, int a_stride, float* re
 }
 
 // int8: copy rows [0, M) of the activation quantized once by llj_i8_stats (outlier columns
-// already 0) into LDS int8 rows (stride K + 16 bytes); sca[] receives SCA per local row.
+// already 0) into LDS int8 rows (stride K + 16 bytes). The rows are first in the workspace (i8ws.h):
+// their place does not depend on its header. One row is in registers by now (row0).
+constexpr int kQRow0 = 4;  // 16-byte registers of row 0 per thread
 template <int NW>
-__device__ void stage_i8(const GemvParams& p, int8_t* Aq, int q_stride, float* sca) {
+__device__ void stage_i8(const GemvParams& p, int8_t* Aq, int q_stride, const u32x4 (&row0)[kQRow0]) {
   const int tid = threadIdx.x;
   constexpr int NT = NW * 64;
   const int K = p.K, M = p.M;
-  const I8WsHeader h = *reinterpret_cast<const I8WsHeader*>(p.i8ws);
-  const I8Layout L = i8_layout(p.i8ws, h.mtot, h.K);
-  if (tid < M) sca[tid] = L.sca[p.m0 + tid];
   const int nv = K >> 4;
+  if (M == 1 && nv <= kQRow0 * NT) {
+#pragma unroll
+    for (int j = 0; j < kQRow0; ++j)
+      if (tid + NT * j < nv) reinterpret_cast<u32x4*>(Aq)[tid + NT * j] = row0[j];
+    return;
+  }
   for (int m = 0; m < M; ++m) {
-    const uint4* src = reinterpret_cast<const uint4*>(L.aq + (size_t)(p.m0 + m) * K);
+    const uint4* src = reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(p.i8ws) + i8_offsets(1, K).aq +
+                                                      (size_t)(p.m0 + m) * K);
     uint4* dst = reinterpret_cast<uint4*>(Aq + (size_t)m * q_stride);
     for (int v = tid; v < nv; v += NT) dst[v] = src[v];
   }
@@ -823,12 +829,13 @@ __device__ __forceinline__ void gemv_body(const GemvParams& p, const int nt0, un
     if constexpr (SIS) {
       if (sis) {  // uniform
         const int n = uniform(scn[d]);
-        u32x4 c0 = r1[d][0][0], c1 = r1[d][0][1];
-        u32x4 e0 = DUAL ? r2[d][0][0] : c0, e1 = DUAL ? r2[d][0][1] : c1;
-        if (n > 0) {  // pinned before the loops (see the AM_I8Q side product)
-          asm volatile("" : "+v"(c0), "+v"(c1));
-          if constexpr (DUAL) asm volatile("" : "+v"(e0), "+v"(e1));
+        if (n > 0) {  // pinned before the loops (see the AM_I8Q side product), in place: copies took the main loop
+          // registers of its own, and filling these waited for all the first chunks
+          asm volatile("" : "+v"(r1[d][0][0]), "+v"(r1[d][0][1]));
+          if constexpr (DUAL) asm volatile("" : "+v"(r2[d][0][0]), "+v"(r2[d][0][1]));
         }
+        const u32x4 c0 = r1[d][0][0], c1 = r1[d][0][1];
+        const u32x4 e0 = DUAL ? r2[d][0][0] : c0, e1 = DUAL ? r2[d][0][1] : c1;
         auto side_col = [&](int k, const u32x4 ov) {  // one outlier column k of this chunk (uniform)
           const int kk = k - 128 * c, t = kk >> 6;
           if (((kk >> 4) & 3) == grp) {  // the lanes holding CB[n, k]
@@ -1259,8 +1266,46 @@ __device__ __forceinline__ void gemv_body(const GemvParams& p, const int nt0, un
       snv[i][1] = *reinterpret_cast<const float4*>(p.nstat + (size_t)q * kNstRows + 4);
     }
   }
+  // int8 workspace (not the hand-off): its header, outlier counts, `avh`, SCA and the side product's speculative
+  // list entries, from the places they have when it holds exactly this launch's rows (always inside it: the
+  // offsets grow with the rows), so nothing here waits for the header. Read after the weight requests: the header
+  // first and the rest from it cost four dependent latencies, each of which waited for the weights as well (4096 ->
+  // 12288 with 8 rows 12.8 -> 12.3 us, with one 12.2 -> 11.7; 4096 -> 2 x 11008 18.9 -> 18.7 and 17.9 -> 17.8).
+  constexpr bool I8W = I8 && !I8Q;
+  constexpr int SPC = kSpE<NW> * NT / kNSB;
+  u32x4 i8h = {0, 0, 0, 0}, i8x[I8W && !I8S ? kQRow0 : 1];
+  int i8cnt = 0, i8avh = 0, i8spk[kSpE<NW>] = {};
+  float i8sca = 0.f;
+  if constexpr (I8W) {
+    const int vq = vzero();  // uniform values stay in VGPRs
+    const I8Layout Lq = i8_layout(p.i8ws, M, K);
+    i8h = reinterpret_cast<const u32x4*>(p.i8ws)[vq];
+    i8cnt = Lq.cnt[lane < kNSB ? lane : 0];
+    i8avh = Lq.avh[vq];
+    i8sca = Lq.sca[tid < M ? tid : M - 1];
+    if constexpr (!I8S) {
+      const u32x4* a0 = reinterpret_cast<const u32x4*>(reinterpret_cast<const int8_t*>(p.i8ws) + i8_offsets(1, K).aq +
+                                                       (size_t)p.m0 * K);
+#pragma unroll
+      for (int j = 0; j < kQRow0; ++j) i8x[j] = a0[tid + NT * j < (K >> 4) ? tid + NT * j : (K >> 4) - 1];
+    }
+#pragma unroll
+    for (int e = 0; e < kSpE<NW>; ++e) {
+      const int q = tid + NT * e, sb = q / SPC < kNSB ? q / SPC : 0;
+      i8spk[e] = Lq.list[sb * i8_kb(K) + q % SPC];
+    }
+    asm volatile("" ::: "memory");  // these requests stay ahead of the weights'
+  }
 #pragma unroll
   for (int d = 0; d < D; ++d) load(d, d);  // the weight stream starts before any A wait
+  // What follows is first read behind the weight requests: without these pins (no instruction) the compiler moves
+  // arithmetic on it up, and its wait holds the requests back. The hand-off form measured nothing from them (8 rows of
+  // 11008 -> 4096 17.4 and 17.3 us, of 4096 -> 4096 7.7 and 7.8).
+  if constexpr (I8W) {
+    asm volatile("" : "+v"(e_a[0].x)::"memory");
+    if constexpr (DUAL) asm volatile("" : "+v"(e_b[0].x)::"memory");
+    asm volatile("" : "+v"(i8h), "+v"(i8cnt), "+v"(i8avh), "+v"(i8sca)::"memory");
+  }
   if constexpr (EP == EP_QKV && FLAT) {  // the positions (their RoPE rows' addresses) are first read behind the weight requests:
     // the compiler moved that arithmetic up, and its wait held the requests back (no instruction; 7B gptq.int4, 8 rows 10.2 -> 9.1 us).
 #pragma unroll
@@ -1311,26 +1356,28 @@ __device__ __forceinline__ void gemv_body(const GemvParams& p, const int nt0, un
     i8scb = e_a[0].x / 127.f;
     if constexpr (DUAL) i8scb2 = e_b[0].x / 127.f;
   }
-  // int8: the per-k-block outlier counts the side product starts from, loaded now (one memory
-  // latency less in the tail; needed once the stream is done)
-  int i8cnt = 0, i8spk[kSpE<NW>] = {};
-  if constexpr (I8 && !I8Q) {  // + the speculative outlier-list entries of the side product's fast path
-    const I8WsHeader h = *reinterpret_cast<const I8WsHeader*>(p.i8ws);
-    const I8Layout L8 = i8_layout(p.i8ws, h.mtot, h.K);
-    i8cnt = L8.cnt[lane < kNSB ? lane : 0];
+  if constexpr (I8W) {
+    const I8WsHeader h = {uniform((int)i8h[0]), uniform((int)i8h[1]), uniform((int)i8h[2]), uniform((int)i8h[3])};
+    const bool exact = h.mtot == M && h.K == K && p.m0 == 0 && h.kb == i8_kb(K);
+    if (!exact) {  // rows of a larger workspace: from the places its header gives
+      const I8Layout L8 = i8_layout(p.i8ws, h.mtot, h.K);
+      i8cnt = L8.cnt[lane < kNSB ? lane : 0];
+      i8sca = L8.sca[p.m0 + (tid < M ? tid : M - 1)];
+#pragma unroll
+      for (int e = 0; e < kSpE<NW>; ++e) {
+        const int q = tid + NT * e, sb = q / SPC < kNSB ? q / SPC : 0;
+        i8spk[e] = L8.list[sb * h.kb + q % SPC];
+        asm volatile("" : "+v"(i8spk[e]));  // waited for here, not on the other path
+      }
+      asm volatile("" : "+v"(i8cnt), "+v"(i8sca));
+    }
     if constexpr (SIS) {
       // in-stream only when every chunk's outlier columns are among its prefetched entries (no
       // load inside a loop in the stream: that would wait for the weight prefetch); else after it
       const float most = wave_max((float)(lane < h.nsb ? i8cnt : 0));
-      sis = h.kb == 128 && h.mtot == M && h.K == p.K && p.m0 == 0 && M <= 8 && L8.avh[0] == 1 && most <= (float)SE;
+      sis = exact && h.kb == 128 && M <= 8 && uniform(i8avh) == 1 && most <= (float)SE;
       i8scb = e_a[0].x / 127.f;
       if constexpr (DUAL) i8scb2 = e_b[0].x / 127.f;
-    }
-    constexpr int SPC = kSpE<NW> * NT / kNSB;
-#pragma unroll
-    for (int e = 0; e < kSpE<NW>; ++e) {
-      const int q = tid + NT * e, sb = q / SPC < kNSB ? q / SPC : 0;
-      i8spk[e] = L8.list[sb * h.kb + q % SPC];
     }
   }
   LLJ_STAMP(1);
@@ -1358,10 +1405,10 @@ __device__ __forceinline__ void gemv_body(const GemvParams& p, const int nt0, un
   if constexpr ((LLJ_ABL & 1) != 0) {  // ablation: no A prologue (garbage A)
   } else if constexpr (I8Q) {
   } else if constexpr (I8S) {  // the epilogue's SCA only (read after the reduction barrier)
-    const I8WsHeader h = *reinterpret_cast<const I8WsHeader*>(p.i8ws);
-    if (tid < M) sca[tid] = i8_layout(p.i8ws, h.mtot, h.K).sca[p.m0 + tid];
+    if (tid < M) sca[tid] = i8sca;
   } else if constexpr (I8) {
-    stage_i8<NW>(p, reinterpret_cast<int8_t*>(smem), a_stride, sca);
+    if (tid < M) sca[tid] = i8sca;
+    stage_i8<NW>(p, reinterpret_cast<int8_t*>(smem), a_stride, i8x);
     __syncthreads();
   } else if constexpr (ALDS) {
     if (rs == 0) {

@@ -284,6 +284,33 @@ def test_int8_linear_vs_restatement(hip, M, outliers):
     assert_bf16_close(out.float().cpu().numpy(), ref, f"int8 M={M} outliers={outliers}", rel=2e-2)
 
 
+@pytest.mark.parametrize("row0,M", [(0, 8), (8, 4), (11, 1)])
+@pytest.mark.parametrize("K,outliers", [(4096, 3), (4096, 120), (8192, 300)])
+def test_int8_linear_rows_of_a_larger_workspace(hip, row0, M, K, outliers):
+    """Statistics of 12 rows, a product of some of them: the workspace's places are those of its own row count, not of
+    the launch's. Tolerance: test_int8_linear_vs_restatement's."""
+    rng = np.random.default_rng(K + outliers + M)
+    N, R = 64, 12
+    W = bf16(rng.standard_normal((N, K)) * 0.02)
+    x = rng.standard_normal((R, K)).astype(np.float32)
+    x[:, rng.choice(K, outliers, replace=False)] *= 25.0
+    x = bf16(x)
+    Wd, xd = T(W, torch.bfloat16), T(x, torch.bfloat16)
+    cb = torch.empty(N, K, dtype=torch.int8, device=dev)
+    scb = torch.empty(N, dtype=torch.float32, device=dev)
+    call(hip, "llj_i8_quant_weight", Wd.data_ptr(), 1, cb.data_ptr(), scb.data_ptr(), N, K, st())
+    cbt = torch.empty_like(cb)
+    call(hip, "llj_i8_repack", cb.data_ptr(), cbt.data_ptr(), N, K, st())
+    ws = torch.empty(hip.llj_i8_ws_bytes(R, K), dtype=torch.uint8, device=dev)
+    call(hip, "llj_i8_stats", xd.data_ptr(), K, R, K, 6.0, ws.data_ptr(), st())
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    call(hip, "llj_linear", 2, xd[row0:].data_ptr(), K, cbt.data_ptr(), scb.data_ptr(), None, out.data_ptr(), N, M, N, K,
+         ws.data_ptr(), row0, None, st())
+    torch.cuda.synchronize()
+    ref = O.int8_linear(x, *O.int8_quantize_weight(W))[row0:row0 + M]
+    assert_bf16_close(out.float().cpu().numpy(), ref, f"int8 rows {row0}..{row0 + M - 1} of {R}", rel=2e-2)
+
+
 @pytest.mark.parametrize("C", [256, 4096, 5120])
 def test_rmsnorm_kernel(hip, golden, C):
     rng = np.random.default_rng(C)
