@@ -552,7 +552,8 @@ class GPTQQuantizer:
     def quantize(self):
         """reference 532-614 with the column loop on the GPU: returns (ColBlockQuantizedLinear, error)."""
         _hip.require_device(self.linear_module.weight, "GPTQQuantizer linear_module.weight")
-        W = self.linear_module.weight.detach().to(dtype=torch.float, copy=True)
+        # (row-major however the parameter is stored: the kernels take its address)
+        W = self.linear_module.weight.detach().to(dtype=torch.float, copy=True, memory_format=torch.contiguous_format)
         scale, zero = self.find_params_weight(W)
         self.scales[:] = scale
         self.zeros[:] = zero

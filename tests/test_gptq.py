@@ -610,3 +610,22 @@ def test_quantizer_refuses_an_indefinite_hessian(hip, tokens):
     gq.collect_input_stats(None, (torch.randn(1, tokens, 128, device=dev),), None)
     with pytest.raises(torch.linalg.LinAlgError):
         gq.quantize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("actorder", [False, True])
+def test_quantizer_weight_in_another_layout(hip, actorder):
+    """A weight whose storage is column-major (a tied or loaded transposed matrix): every output is the row-major weight's."""
+    from lit_llama.quantization import GPTQQuantizer
+    g = torch.Generator(device=dev).manual_seed(4)
+    w, x = torch.randn(96, 256, generator=g, device=dev), torch.randn(1, 512, 256, generator=g, device=dev)
+    outs = []
+    for weight in (w, w.t().contiguous().t()):
+        lin = torch.nn.Linear(256, 96, bias=False, device=dev)
+        lin.weight = torch.nn.Parameter(weight, requires_grad=False)
+        gq = GPTQQuantizer(lin, bits=4, actorder=actorder)
+        gq.collect_input_stats(None, (x,), None)
+        q, error = gq.quantize()
+        outs.append((q.quant_weight, q.scales, q.zeros, error))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
