@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void g_attention_tiles_kernel(const T* __re
   for (int i = 0; i < kGaMaxD / 64; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float mx[4], l[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) mx[r] = -INFINITY, l[r] = 0.f;
+  for (int r = 0; r < 4; ++r) mx[r] = -3.402823466e38f, l[r] = 0.f;  // (finite: a first tile of scores of minus infinity has weights of 0)
   for (int k0 = 0; k0 < nmax; k0 += kGaKeys) {
     put(kr);
     fetch(vr, vbuf, k0);
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256, 2) void g_attention_tiles_kernel(const T* __re
     for (int r = 0; r < 4; ++r) {
       const int i = 4 * g4 + r;
       const float m = fmaxf(fmaxf(fmaxf(red[i], red[kGaRows + i]), fmaxf(red[2 * kGaRows + i], red[3 * kGaRows + i])), mx[r]);
-      keep[r] = __expf(mx[r] - m);  // (every row sees key 0: m is finite from the first tile on)
+      keep[r] = __expf(mx[r] - m);
       mx[r] = m;
       const float p = __expf(s[r] - m);
       l[r] = l[r] * keep[r] + p;

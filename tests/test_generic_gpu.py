@@ -404,3 +404,37 @@ def test_prompt_attention_tiles(hip, dtype, B, T, nh, hs, S, p0):
     s = q.double().view(B, T, nh, hs).transpose(1, 2).contiguous() @ k.double().nan_to_num().transpose(2, 3).contiguous() * hs ** -0.5
     want = (torch.softmax(s.masked_fill(~mask, float("-inf")), -1) @ v.double().nan_to_num()).transpose(1, 2).reshape(B, T, C)
     assert (y.double() - want).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
+
+
+def _prompt_attention(dtype, B, T, nh, hs, S, p0, seed):
+    """(q, k, v, positions, a call of llj_g_attention)."""
+    from lit_llama import _hip
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q, k, v = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((B, T, nh * hs), (B, nh, S, hs), (B, nh, S, hs)))
+    pos = torch.arange(p0, p0 + T, dtype=torch.int32, device="cuda")
+
+    def run():
+        y = torch.empty(B, T, nh * hs, dtype=dtype, device="cuda")
+        _hip.call("llj_g_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), y.data_ptr(), pos.data_ptr(), B, T, nh * hs, nh, S,
+                  int(dtype == torch.float32), _hip.stream())
+        torch.cuda.synchronize()
+        return y.view(B, T, nh, hs).transpose(1, 2)
+
+    return q.view(B, T, nh, hs).transpose(1, 2), k, v, pos, run
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,nh,hs,dead", [(200, 8, 64, 64), (200, 8, 78, 70), (150, 8, 16, 128)])
+def test_prompt_attention_first_scores_minus_infinity(hip, dtype, T, nh, hs, dead):
+    """The first `dead` keys score minus infinity in every row: the rows that see a later one average the later ones."""
+    q, k, v, pos, run = _prompt_attention(dtype, 1, T, nh, hs, T, 0, dead)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[:, :, :dead, 0] = float("-inf")
+    y = run()
+    assert not y[:, :, :dead].isfinite().any()  # no score but minus infinity: as a softmax of those
+    s = (q.double() @ k.double().transpose(2, 3).contiguous()) * hs ** -0.5
+    s = s.masked_fill(pos[None, :] > pos[:, None], float("-inf"))[:, :, dead:]
+    want = torch.softmax(s, -1) @ v.double()
+    assert (y[:, :, dead:].double() - want).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
