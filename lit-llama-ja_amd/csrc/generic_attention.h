@@ -23,6 +23,37 @@ __host__ __device__ inline int ga_stride(int hs) { return ((hs + 15) & ~15) + 4;
 inline size_t ga_lds(int hs) { return ((size_t)(kGaRows + kGaKeys) * ga_stride(hs) + kGaRows * kGaPs + 8 * kGaRows) * 4; }
 inline int ga_vectors(int hs, int ve) { return (kGaKeys * hs / ve + 255) / 256; }  // per thread and tile
 
+// One row by g_attention_kernel's steps: y = softmax(q . K) V over its n keys and no other. q: the scaled row, lds: 264 floats.
+template <typename T>
+__device__ __forceinline__ void ga_row(const float* q, const T* __restrict__ k, const T* __restrict__ v, T* __restrict__ y, int n, int hs, float* lds, int tid) {
+  const int lane = tid & 63, wave = tid >> 6;
+  float *sc = lds, *top = lds + 256, *sum = lds + 260;
+  auto score = [&](int j) {
+    float s = 0.f;
+    for (int d = 0; d < hs; ++d) s += q[d] * ldv(k, (size_t)j * hs + d);
+    return s;
+  };
+  float mx = -INFINITY, l = 0.f, o = 0.f;
+  for (int j = tid; j < n; j += 256) mx = fmaxf(mx, score(j));
+  mx = wave_max(mx);
+  if (lane == 0) top[wave] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
+  for (int j0 = 0; j0 < n; j0 += 256) {
+    const float p = j0 + tid < n ? __expf(score(j0 + tid) - mx) : 0.f;
+    l += p;
+    sc[tid] = p;
+    __syncthreads();
+    if (tid < hs)
+      for (int j = 0; j < min(256, n - j0); ++j) o += sc[j] * ldv(v, (size_t)(j0 + j) * hs + tid);
+    __syncthreads();
+  }
+  l = wave_sum(l);
+  if (lane == 0) sum[wave] = l;
+  __syncthreads();
+  if (tid < hs) stv(y, tid, o * (1.f / (sum[0] + sum[1] + sum[2] + sum[3])));
+}
+
 template <typename T, int VE, int NL>
 __global__ __launch_bounds__(256, 2) void g_attention_tiles_kernel(const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc,
                                                                    T* __restrict__ y, const int* __restrict__ pos, int T_, int C, int nh, int S) {
@@ -34,7 +65,7 @@ __global__ __launch_bounds__(256, 2) void g_attention_tiles_kernel(const T* __re
   float* Ps = KV + kGaKeys * ST;        // [16][kGaPs]
   float* red = Ps + kGaRows * kGaPs;    // [4][16]
   int* s_n = reinterpret_cast<int*>(red + 4 * kGaRows);  // [16] visible keys of a row
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c16 = lane & 15, g4 = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), c16 = lane & 15, g4 = lane >> 4;
   const int QT = (T_ + kGaRows - 1) / kGaRows, b = blockIdx.x / QT, t0 = (QT - 1 - (int)blockIdx.x % QT) * kGaRows, h = blockIdx.y;
   const float scale = 1.f / sqrtf((float)hs);
   const size_t base = ((size_t)b * nh + h) * S * hs;
@@ -165,6 +196,8 @@ __global__ __launch_bounds__(256, 2) void g_attention_tiles_kernel(const T* __re
     const float v = row16_sum(l[r]);
     if (c16 == 0) red[wave * kGaRows + 4 * g4 + r] = v;
   }
+  int* odd = reinterpret_cast<int*>(Ps);  // [16] rows with an output that is not finite
+  if (tid < kGaRows) odd[tid] = 0;
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -174,8 +207,21 @@ __global__ __launch_bounds__(256, 2) void g_attention_tiles_kernel(const T* __re
 #pragma unroll
     for (int n = 0; n < kGaMaxD / 64; ++n) {
       const int d = 16 * (wave + 4 * n) + c16;
-      if (d < hs) stv(y, ((size_t)b * T_ + t0 + i) * C + h * hs + d, o[n][r] * inv);
+      const float v = o[n][r] * inv;
+      if (d < hs) stv(y, ((size_t)b * T_ + t0 + i) * C + h * hs + d, v);
+      if (d < hs && !(fabsf(v) < INFINITY)) odd[i] = 1;
     }
+  }
+  // A row that does not see a key takes 0 times its value above, and that is not 0 for a value that is not finite: where an output is
+  // not, its row again from its own keys alone. (lane2: the lane without a register held through the loop, which cost fp32 heads of 78
+  // their third wave per SIMD. Told apart in the loop, it took 10 registers.)
+  __syncthreads();
+  const int lane2 = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  unsigned again = (unsigned)__ballot(lane2 < kGaRows && odd[lane2 & (kGaRows - 1)]);
+  for (; again; again &= again - 1) {
+    const int i = __builtin_ctz(again);
+    ga_row(Qs + i * ST, kc + base, vc + base, y + ((size_t)b * T_ + t0 + i) * C + h * hs, uniform(s_n[i]), hs, KV, wave * 64 + lane2);
+    __syncthreads();
   }
 }
 

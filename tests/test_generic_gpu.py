@@ -438,3 +438,22 @@ def test_prompt_attention_first_scores_minus_infinity(hip, dtype, T, nh, hs, dea
     s = s.masked_fill(pos[None, :] > pos[:, None], float("-inf"))[:, :, dead:]
     want = torch.softmax(s, -1) @ v.double()
     assert (y[:, :, dead:].double() - want).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("T,nh,hs,p0,at", [(130, 8, 64, 0, 37), (130, 10, 78, 3, 64), (100, 12, 13, 0, 99), (129, 8, 200, 2, 0)])
+def test_prompt_attention_values_of_later_tokens(hip, dtype, value, T, nh, hs, p0, at):
+    """One value of key `at` is not finite: the rows before it give what they give without it (to the order of their sums), the rows
+    that see it one output that is not finite."""
+    q, k, v, pos, run = _prompt_attention(dtype, 1, T, nh, hs, T + p0, p0, at)
+    want = run()
+    v[0, 1, at, hs // 2] = value
+    got = run()
+    sees = (pos >= at).nonzero().flatten()
+    assert not got[0, 1, sees, hs // 2].isfinite().any()
+    got, want = got.clone(), want.clone()
+    got[0, 1, sees, hs // 2] = want[0, 1, sees, hs // 2] = 0
+    assert got.isfinite().all()
+    assert (got.double() - want.double()).norm() <= (2e-6 if dtype == torch.float32 else 2.0 ** -8) * want.double().norm()
