@@ -26,18 +26,30 @@ constexpr int kHs = kGptqBlock + 4;   // LDS row stride of Hinv1 (rows start on 
 
 // a / b, correctly rounded, from y = 1 / b correctly rounded: two residual steps. The first makes the quotient faithful, the
 // second then gives the rounded one (Markstein, "Computation of elementary functions on the IBM RISC System/6000", 1990), for
-// operands whose residuals do not underflow. A third of the division sequence's instructions, and no dependent reciprocal.
+// operands whose quotient does not overflow and whose residuals do not underflow (a zero's sign is not kept). A third of the division
+// sequence's instructions, and no dependent reciprocal.
 __device__ __forceinline__ float div_by(float a, float b, float y) {
   float q = __fmul_rn(a, y);
   q = __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
   return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
 }
 __device__ __forceinline__ bool divides(float b) { return fabsf(b) > 0x1p-40f && fabsf(b) < 0x1p40f; }
+// The range of the errors e = dq / d seen. From 2^-60 to 2^40, or zero, with divides(d): |dq| is in [2^-100, 2^80), its residuals are
+// multiples of 2^-147; and with divides(s) and |z| < 2^30: |w| < 2^81, w / s does not overflow (a small one rounds to code z either way).
+struct Errors {
+  unsigned hi = 0, lo = ~0u;  // bits of absolute values: NaN's are the largest, a zero's less one too
+  __device__ __forceinline__ void add(float e) {
+    const unsigned a = __float_as_uint(e) & 0x7fffffffu;
+    hi = max(hi, a);
+    lo = min(lo, a - 1u);
+  }
+  __device__ __forceinline__ bool fit() const { return hi < __float_as_uint(0x1p40f) && lo >= __float_as_uint(0x1p-60f) - 1u; }
+};
 
-// One block of one row's columns (see gptq_block_kernel). FAST: every divisor is in div_by's range.
+// One block of one row's columns (see gptq_block_kernel). FAST: every divisor is in div_by's range; seen: the errors.
 template <int LANES, int kWs, bool FAST>
 __device__ __forceinline__ float gptq_columns(const float* hs, const float* rd, float* ws, int t, int l, int blk, float s, float z, float maxq,
-                                              bool writer, float* __restrict__ q_out, float* __restrict__ e_out, size_t N) {
+                                              bool writer, float* __restrict__ q_out, float* __restrict__ e_out, size_t N, Errors& seen) {
   const float rs = __fdiv_rn(1.f, s);
   float lsum = 0.f;
   for (int b = 0; b < blk; b += kGptqSub) {
@@ -54,6 +66,7 @@ __device__ __forceinline__ float gptq_columns(const float* hs, const float* rd, 
       const float q = __fmul_rn(s, __fsub_rn(qi, z));
       const float dq = __fsub_rn(w, q);
       e[u] = FAST ? div_by(dq, d, rd[b + u]) : __fdiv_rn(dq, d);  // err1 (592)
+      if constexpr (FAST) seen.add(e[u]);
       lsum = __fadd_rn(lsum, __fmul_rn(e[u], e[u]));               // Losses1 (590): (w - q)^2 / d^2
       if (writer) {
         q_out[(size_t)(b + u) * N] = q;
@@ -86,7 +99,9 @@ __device__ __forceinline__ float gptq_columns(const float* hs, const float* rd, 
 // Bound: the chain of dependent instructions of a column, two divisions in it, times 128. 16 rows x 16 lanes put N = 4096 on
 // all 256 CUs (32 x 8: on half of them); above N = 8192 64 x 4 keep the workgroups of one round. kWs spreads a wavefront's
 // lanes x rows over the 64 banks (20 l + t, 80 l + t mod 64). us a block, before (32 x 8, three division sequences a column; 64 x 4
-// above 8192): N = 4096 52 and 34, 8192 54 and 38, 11008 63 and 54 (32 x 8 there: 79), 35008 196 and 169.
+// above 8192): N = 4096 52 and 35 (39 among the producer's other launches), 8192 54
+// and 37, 11008 63 and 55 (32 x 8 there: 79), 35008 196 and 173; of that 1 to 3 for the range of the errors (a block with one out of
+// range is done twice).
 template <int ROWS, int LANES, int kWs>
 __global__ __launch_bounds__(ROWS * LANES) void gptq_block_kernel(const float* __restrict__ hinv, int K, int i1,
                                                                   int blk,
@@ -104,7 +119,7 @@ __global__ __launch_bounds__(ROWS * LANES) void gptq_block_kernel(const float* _
   const int n = blockIdx.x * ROWS + t;
   const int nn = n < N ? n : N - 1;  // clamped: loads stay in bounds, stores are guarded
   const float s = scale[nn], z = zero[nn];
-  bool fast = divides(s);
+  bool fast = divides(s) && fabsf(z) < 0x1p30f;
   if (tid < blk) {
     const float d = hinv[(size_t)(i1 + tid) * K + i1 + tid];
     rd[tid] = __fdiv_rn(1.f, d);
@@ -118,17 +133,26 @@ __global__ __launch_bounds__(ROWS * LANES) void gptq_block_kernel(const float* _
   } else {
     for (int v = tid; v < blk * blk; v += NT) hs[v / blk * kHs + v % blk] = hinv[(size_t)(i1 + v / blk) * K + i1 + v % blk];
   }
-  // a wavefront reads runs of ROWS neighbouring rows of the matrix
-  for (int v = tid; v < blk * ROWS; v += NT) {
-    const int j = v / ROWS, m = min((int)blockIdx.x * ROWS + v % ROWS, N - 1);
-    ws[j * kWs + v % ROWS] = wt[(size_t)(i1 + j) * N + m];
-  }
-  const bool all = __syncthreads_and(fast);
+  auto stage = [&] {  // a wavefront reads runs of ROWS neighbouring rows of the matrix
+    for (int v = tid; v < blk * ROWS; v += NT) {
+      const int j = v / ROWS, m = min((int)blockIdx.x * ROWS + v % ROWS, N - 1);
+      ws[j * kWs + v % ROWS] = wt[(size_t)(i1 + j) * N + m];
+    }
+  };
+  stage();
+  bool done = __syncthreads_and(fast);
   const bool writer = l == 0 && n < N;
   float* q_out = qt + (size_t)i1 * N + nn;
   float* e_out = err + nn;
-  const float sum = all ? gptq_columns<LANES, kWs, true>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N)
-                        : gptq_columns<LANES, kWs, false>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N);
+  float sum = 0.f;
+  Errors seen;
+  if (done) {
+    sum = gptq_columns<LANES, kWs, true>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N, seen);
+    done = __syncthreads_and(seen.fit());
+    if (!done) stage();  // a quotient out of div_by's range: the block again
+    __syncthreads();
+  }
+  if (!done) sum = gptq_columns<LANES, kWs, false>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N, seen);
   if (writer) loss[n] += sum;
 }
 

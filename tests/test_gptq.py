@@ -629,3 +629,33 @@ def test_quantizer_weight_in_another_layout(hip, actorder):
         outs.append((q.quant_weight, q.scales, q.zeros, error))
     for a, b in zip(*outs):
         assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", [float("inf"), 2.0 ** 127, 2.0 ** 100, 2.0 ** -110, 2.0 ** -130])
+def test_gptq_block_kernel_dividends_bitwise(hip, size):
+    """Ordinary scales and diagonals with one row of weights whose quotients overflow or whose residuals underflow, or infinite last ones: bit
+    for bit the oracle's in every row, as with the division instruction sequence."""
+    from lit_llama import _hip
+    rng = np.random.default_rng(8)
+    N, K = 40, 128
+    W = rng.standard_normal((N, K)).astype(np.float32)
+    if np.isinf(size):
+        W[17, -1], W[18, -1] = size, -size
+    else:
+        W[17] = (rng.uniform(1, 1.9, K) * size).astype(np.float32)
+    scale = rng.uniform(0.05, 0.4, N).astype(np.float32)
+    zero = rng.integers(4, 12, N).astype(np.float32)
+    Hinv = np.triu(rng.standard_normal((K, K)) * 1e-4).astype(np.float32)
+    Hinv[np.arange(K), np.arange(K)] = rng.uniform(1.5, 3, K).astype(np.float32)
+    with np.errstate(over="ignore", invalid="ignore"):
+        Q1, E1, _ = G.gptq_block(W, Hinv, scale, zero, 4)
+    assert np.isfinite(Q1).all() and not np.isnan(E1).any()
+    wt = torch.from_numpy(np.ascontiguousarray(W.T)).to(dev)
+    qt, err, loss = torch.empty(K, N, device=dev), torch.empty(128, N, device=dev), torch.zeros(N, device=dev)
+    hd, sd, zd = (torch.from_numpy(a).to(dev) for a in (Hinv, scale, zero))
+    _hip.call("llj_gptq_block", hd.data_ptr(), K, 0, wt.data_ptr(), N, sd.data_ptr(), zd.data_ptr(), 4, qt.data_ptr(), err.data_ptr(),
+              loss.data_ptr(), _st())
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(qt.cpu().numpy().T, Q1)
+    np.testing.assert_array_equal(err.cpu().numpy().T, E1)
