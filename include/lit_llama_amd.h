@@ -321,7 +321,7 @@ int llj_gptq_gram(const void* x, int dt, int T, int K, float keep, float alpha, 
 /* W (N, K) in the loop's layout and column order: wt (K, N) with wt[place[k]][n] = W[n][k] (place NULL: k), zero for dead[k]. */
 int llj_gptq_weight(const float* W, const int64_t* place, const void* dead, int N, int K, float* wt, void* stream);
 /* hinv = M on return: the upper Cholesky factor of (H[perm][:, perm] + damp I)^-1 (549-566), zeros below. K % 128 == 0, H is not
- * changed. P: K x K floats of scratch, xt: 128 x 128, all on 16 bytes; *info = 1 if a pivot is not positive (M is then unusable). */
+ * changed. P: K x K floats of scratch, xt: 128 x 128, all on 16 bytes; *info = 1 if a pivot is not positive and normal (M is then unusable). */
 int llj_gptq_factor(const float* H, const int64_t* perm, const float* damp, int K, float* M, float* P, float* xt, int* info, void* stream);
 /* W[:, i2:] -= Err1 Hinv[i1:i2, i2:] (596) behind a block of `blocksize` columns, transposed as llj_gptq_block keeps it. */
 int llj_gptq_update(const float* hinv, int K, int i1, int blocksize, const float* err, int N, float* wt, void* stream);

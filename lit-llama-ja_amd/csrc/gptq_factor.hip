@@ -200,7 +200,7 @@ __device__ __forceinline__ float lane_value(float v, int lane) { return __uint_a
 
 // S (LDS, 128 x 128, upper triangle, zeros below) -> L^-1 in the lower triangle with zeros above, S = L L^T. 32 columns at a time: one wave eliminates
 // the 32 x 32 block in registers (lane c a column of the block, lane 32 + c of the identity), the matrix cores do the rest.
-// Returns false (in every thread) if a pivot was not positive.
+// Returns false (in every thread) if a pivot was not a positive normal number.
 __device__ __forceinline__ bool factor_block(float* S, int* bad) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c16 = lane & 15;
   if (tid == 0) *bad = 0;
@@ -218,7 +218,7 @@ __device__ __forceinline__ bool factor_block(float* S, int* bad) {
 #pragma unroll
       for (int j = 0; j < 32; ++j) {
         const float p = lane_value(v[j], j);
-        ok = ok && p > 0.f;
+        ok = ok && p >= 0x1p-126f && p < INFINITY;  // (the root's estimate takes normal numbers)
         float r = __builtin_amdgcn_rsqf(p);
         r = __builtin_fmaf(0.5f * r, __builtin_fmaf(-p * r, r, 1.f), r);  // one Newton step
         v[j] *= r;

@@ -531,7 +531,7 @@ class GPTQQuantizer:
         1.7 ms for 29.5 with the library's two factorizations and inverse, its error against float64 2.5e-7 for 1.1e-6. With
         fewer rows H is damping in most directions and the error feedback amplifies any rounding (other correct factors change
         1 to 5 % of the codes at 4,096 columns, 0.2 % from there on): those keep the library's. So does an H whose elimination
-        meets a pivot that is not positive, so that it is the library that decides whether that is an error."""
+        meets a pivot that is not positive and normal, so that it is the library that decides whether that is an error."""
         K = self.columns
         if 2 * self.tokens >= 3 * K and K <= 65535:
             Hinv, P, xt = torch.empty_like(H), torch.empty_like(H), torch.empty((128, 128), device=H.device)

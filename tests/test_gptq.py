@@ -659,3 +659,18 @@ def test_gptq_block_kernel_dividends_bitwise(hip, size):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(qt.cpu().numpy().T, Q1)
     np.testing.assert_array_equal(err.cpu().numpy().T, E1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 0.0, 2.0 ** -140])
+def test_inverse_factor_reports_the_last_pivot(hip, value):
+    """The last pivot of the elimination (column 0) is one that has no ordinary reciprocal root: reported, not written as numbers."""
+    from lit_llama import _hip
+    K = 256
+    H = torch.eye(K, device=dev)
+    H[0, 0] = value
+    damp, M, P = torch.zeros((), device=dev), torch.empty_like(H), torch.empty_like(H)
+    xt, info = torch.empty(128, 128, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
+    _hip.call("llj_gptq_factor", H.data_ptr(), 0, damp.data_ptr(), K, M.data_ptr(), P.data_ptr(), xt.data_ptr(), info.data_ptr(), _st())
+    torch.cuda.synchronize()
+    assert info.item() == 1
