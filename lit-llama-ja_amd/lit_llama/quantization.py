@@ -466,13 +466,13 @@ class GPTQQuantizer:
         self.zeros = torch.zeros_like(self.scales)
 
     def find_params_weight(self, x):
-        """reference 475-514, per channel in one kernel. Otherwise the min / max reduce on the device (exact) and the divisions
-        run on the host, because torch's device division by a scalar multiplies by its reciprocal
-        (not the reference's correctly rounded quotient). perchannel=False: one (scale, zero) over
+        """reference 475-514, per channel in one kernel (codes to 16 bits). Otherwise the min / max reduce on the device
+        (exact) and the divisions run on the host, because torch's device division by a scalar multiplies by its
+        reciprocal (not the reference's correctly rounded quotient). perchannel=False: one (scale, zero) over
         the whole matrix, repeated per row (481-482, 503-506); sym: the range symmetric about 0 and
         zero = (maxq + 1) / 2 (488-492, 498-499)."""
         rows = x.shape[0]
-        if self.perchannel and x.is_cuda and x.dtype == torch.float32 and x.numel():
+        if self.perchannel and x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and x.numel() and 1 <= self.bits <= 16:
             x = x.contiguous()
             scale, zero = torch.empty(2, rows, 1, device=x.device)
             with torch.cuda.device(x.device):

@@ -674,3 +674,14 @@ def test_inverse_factor_reports_the_last_pivot(hip, value):
     _hip.call("llj_gptq_factor", H.data_ptr(), 0, damp.data_ptr(), K, M.data_ptr(), P.data_ptr(), xt.data_ptr(), info.data_ptr(), _st())
     torch.cuda.synchronize()
     assert info.item() == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits,sym", [(17, False), (24, True)])
+def test_row_parameters_of_wide_codes(hip, bits, sym):
+    """Code widths that the per-row kernel does not take: as on the host."""
+    from lit_llama.quantization import GPTQQuantizer
+    w = torch.randn(8, 128, generator=torch.Generator().manual_seed(bits))
+    gq = GPTQQuantizer(torch.nn.Linear(128, 8, bias=False, device=dev), bits=bits, sym=sym)
+    for a, b in zip(gq.find_params_weight(w.to(dev)), gq.find_params_weight(w)):
+        np.testing.assert_array_equal(a.cpu().numpy(), b.numpy())
