@@ -306,6 +306,43 @@ def test_generic_gemm_edges_vs_float64(kind, bits, group, dt, M, N, K, pad, off)
             assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside the bound"
 
 
+@pytest.mark.parametrize("M,N,K,pad,ws", [
+    (9, 1, 3104, 0, True), (9, 129, 3104, 4, False), (64, 128, 4096, 0, True), (65, 129, 3104, 12, True), (65, 780, 4096, 0, False),
+    (301, 1000, 3104, 0, True), (37, 12288, 4096, 0, True), (301, 13200, 3104, 4, False), (513, 11000, 3104, 0, False),
+    (64, 16500, 3072, 0, False), (70, 256, 32 * 113, 0, True)])
+def test_generic_gemm_direct_tiles_equal_staged_ones(M, N, K, pad, ws):
+    """fp32 rows above K = 3,071 in whole tiles, brought to LDS without registers, against the same product through registers (x one
+    element off the alignment): the same sums bit for bit, with and without the residual in place. One workgroup and several rounds,
+    both buffer counts (513 to 768 workgroups take two), column and row remainders, padded rows, split K (32 x 113: splits of unequal
+    length), no split."""
+    from lit_llama import _hip
+
+    g = torch.Generator("cuda").manual_seed(M + N + K)
+    ldx = K + pad
+    w, res = torch.randn(N, K, device="cuda", generator=g), torch.randn(M, N, device="cuda", generator=g)
+    x = torch.randn(M, K, device="cuda", generator=g)
+    rows = []
+    for off in (0, 1):
+        buf = torch.full((M * ldx + 4,), float("nan"), device="cuda")
+        rows.append(buf[off:off + M * ldx].view(M, ldx))
+        rows[-1][:, :K] = x
+    nbytes = _hip.lib().llj_g_linear_ws_bytes(1, M, N, K, 1) if ws else 0
+    scratch = torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda")
+    for resid in (False, True):
+        outs = []
+        for r in rows:
+            y = res.clone() if resid else torch.full_like(res, float("nan"))
+            _hip.call("llj_g_linear_ws", 1, r.data_ptr(), ldx, M, K, w.data_ptr(), None, None, 16, K, N, y.data_ptr(), N,
+                      y.data_ptr() if resid else None, N if resid else 0, 1, scratch.data_ptr() if nbytes else None, nbytes, _hip.stream())
+            outs.append(y)
+        assert torch.equal(*outs)
+        if M * N < 200000:  # (the bound of the test above)
+            want, mass = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+            ref = want + res.double() if resid else want
+            lim = mass * 2.0 ** -24 * (32 + 8 + K // 128 + 16 + 4) + (2.0 ** -24 * ref.abs() if resid else 0.0)
+            assert ((outs[0].double() - ref).abs() <= lim + 1e-30).all()
+
+
 # ---- up to 8 rows (generic_rows.h)
 @pytest.mark.parametrize("dt", [0, 1])
 @pytest.mark.parametrize("M", [1, 3, 8])
@@ -383,7 +420,9 @@ def test_generic_rope_attention_vs_separate_calls(dt, B, nh, hs, S, p):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,T,nh,hs,S,p0", [(1, 301, 32, 128, 301, 0), (2, 67, 10, 78, 80, 5), (1, 130, 8, 1, 130, 0), (3, 49, 8, 13, 64, 40),
-                                            (1, 1030, 1, 256, 1030, 0), (2, 129, 5, 101, 200, 0), (1, 70, 16, 64, 72, 60), (1, 128, 9, 250, 128, 0)])
+                                            (1, 1030, 1, 256, 1030, 0), (2, 129, 5, 101, 200, 0), (1, 70, 16, 64, 72, 60), (1, 128, 9, 250, 128, 0),
+                                            (1, 130, 8, 17, 130, 0), (1, 140, 8, 63, 150, 7), (1, 131, 8, 82, 131, 0), (1, 129, 8, 126, 140, 9),
+                                            (1, 130, 8, 132, 130, 0)])
 def test_prompt_attention_tiles(hip, dtype, B, T, nh, hs, S, p0):
     """llj_g_attention on tiles of 16 rows and 64 keys, any head size (also one whose vectors are too many for the tiles), remainders of
     both, rows whose positions have gone round the cache, unseen slots that hold NaN. Against float64: the output's own rounding, and in

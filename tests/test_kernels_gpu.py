@@ -680,11 +680,12 @@ def test_rmsnorm_rows_rowsum_and_int4_rowsum_operand(hip, golden):
 
 
 @pytest.mark.parametrize("wfmt", [0, 3])
-@pytest.mark.parametrize("M", [7, 8])
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 6, 7, 8])
 def test_multi_tile_workgroups_equal_single_tile(hip, wfmt, M):
     """Several 16-column tiles per workgroup (7B / 13B shapes: QKV 768 tiles, SwiGLU 688 with a
     partial last workgroup, lm_head 2000, 13B mlp.c_proj 320 tiles at 8 waves) give bitwise
-    the results of one tile per workgroup (llj_set_tpw_max(1)), and match the oracle."""
+    the results of one tile per workgroup (llj_set_tpw_max(1)), and match the oracle; the norm-fused ops with the
+    rows in LDS and, as decode runs them, streamed with the producer's statistics."""
     rng = np.random.default_rng(100 + M + wfmt)
     P = lambda t: None if t is None else t.data_ptr()  # noqa: E731
     C, nh, H, V = 4096, 32, 11008, 32000
@@ -702,37 +703,42 @@ def test_multi_tile_workgroups_equal_single_tile(hip, wfmt, M):
     xr0 = T(bf16(rng.standard_normal((M, C13))), torch.bfloat16)
     rope, pos, S = T(O.build_rope_cache(256, 128)), T(np.array([37], np.int32)), 64
 
-    def run():
+    nst = torch.zeros(C // 16, 16, device=dev)
+    nst[:, :M] = (xd.float() * xd.float()).to(torch.bfloat16).float().view(M, C // 16, 16).sum(2).T
+
+    def run(*ns):
         q = torch.zeros(M, C, dtype=torch.bfloat16, device=dev)
         kc = torch.zeros(M, nh, S, 128, dtype=torch.bfloat16, device=dev)
         vc = torch.zeros_like(kc)
         call(hip, "llj_norm_qkv_rope", wfmt, xd.data_ptr(), gd.data_ptr(), 1e-5, Wqd.data_ptr(), P(sq), q.data_ptr(),
-             kc.data_ptr(), vc.data_ptr(), rope.data_ptr(), pos.data_ptr(), M, 1, C, nh, S, 0, M, None, None, None, 0, st())
+             kc.data_ptr(), vc.data_ptr(), rope.data_ptr(), pos.data_ptr(), M, 1, C, nh, S, 0, M, None, None, *ns, st())
         h = torch.empty(M, H, dtype=torch.bfloat16, device=dev)
         call(hip, "llj_norm_swiglu", wfmt, xd.data_ptr(), gd.data_ptr(), 1e-5, W1d.data_ptr(), P(s1), W2d.data_ptr(),
-             P(s2), h.data_ptr(), M, H, C, None, 0, None, None, 0, st())
+             P(s2), h.data_ptr(), M, H, C, None, 0, None, *ns, st())
         lg = torch.empty(M, V, dtype=torch.bfloat16, device=dev)
         call(hip, "llj_norm_linear", wfmt, xd.data_ptr(), gd.data_ptr(), 1e-5, Whd.data_ptr(), P(sh), lg.data_ptr(),
-             V, M, V, C, None, 0, None, None, 0, st())
+             V, M, V, C, None, 0, None, *ns, st())
         xr = xr0.clone()
         call(hip, "llj_linear_resid", wfmt, hxd.data_ptr(), H13, Wrd.data_ptr(), P(sr), xr.data_ptr(), C13, M, C13,
              H13, None, 0, None, st())
         torch.cuda.synchronize()
         return q, kc, vc, h, lg, xr
 
-    old = hip.llj_set_tpw_max(1)
-    try:
-        one = run()
-    finally:
-        hip.llj_set_tpw_max(old)
-    multi = run()
-    for name, a, b in zip(("q", "k cache", "v cache", "swiglu", "lm_head", "resid"), one, multi):
-        assert torch.equal(a, b), name
     hn = bf16(O.rmsnorm(x, g))
     hexp = bf16(bf16(O.silu(bf16(hn @ W1.T))) * bf16(hn @ W2.T))
-    assert_bf16_close(multi[3].float().cpu().numpy(), hexp, "swiglu", rel=3e-2)
-    assert_bf16_close(multi[4].float().cpu().numpy(), hn @ Wh.T, "lm_head")
-    assert_bf16_close(multi[5].float().cpu().numpy(), xr0.float().cpu().numpy() + bf16(hx @ Wr.T), "resid 13B")
+    lexp, rexp = hn @ Wh.T, xr0.float().cpu().numpy() + bf16(hx @ Wr.T)
+    for ns in ((None, 0), (nst.data_ptr(), C // 16)):
+        old = hip.llj_set_tpw_max(1)
+        try:
+            one = run(*ns)
+        finally:
+            hip.llj_set_tpw_max(old)
+        multi = run(*ns)
+        for name, a, b in zip(("q", "k cache", "v cache", "swiglu", "lm_head", "resid"), one, multi):
+            assert torch.equal(a, b), name
+        assert_bf16_close(multi[3].float().cpu().numpy(), hexp, "swiglu", rel=3e-2)
+        assert_bf16_close(multi[4].float().cpu().numpy(), lexp, "lm_head")
+        assert_bf16_close(multi[5].float().cpu().numpy(), rexp, "resid 13B")
 
 
 @pytest.mark.parametrize("M,K", [(1, 4096), (8, 4096), (13, 4096), (3, 256), (8, 5120), (16, 5120), (20, 4096), (5, 11008)])
