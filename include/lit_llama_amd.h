@@ -301,10 +301,10 @@ int llj_i8_quant_weight(const void* W, int dtype, void* CB, void* SCB, int N, in
  * -1): for rows n < N, quantize columns i1 .. i1+127 in order with the per-row (scale, zero)
  * (quantize_weight, 470-473), propagate each column's error through the block with Hinv1 =
  * hinv[i1:i1+128, i1:i1+128] (593). wt: the (permuted, running) weight TRANSPOSED, (K, N) fp32,
- * its block rows updated in place; qt (K, N): reconstructions scale*(q - zero) of the block's
+ * only read; qt (K, N): reconstructions scale*(q - zero) of the block's
  * rows; err (128, N): Err1; loss[n] += Σ_i ((w - q) / d)² (Losses1 before the / 2). hinv: (K, K)
  * fp32 upper Cholesky factor of H⁻¹. Requires i1 % 128 == 0, i1 + 128 <= K, bits in {2,4,8}.
- * Each fp32 op rounded on its own in the reference's order (bitwise the reference's loop). The
+ * Each fp32 op rounded on its own in the reference's order (bitwise the reference's loop, the signs of zeros aside). The
  * trailing update W[:, i2:] -= Err1 · Hinv[i1:i2, i2:] is llj_gptq_update. */
 int llj_gptq_block(const float* hinv, int K, int i1, float* wt, int N, const float* scale, const float* zero,
                    int bits, float* qt, float* err, float* loss, void* stream);

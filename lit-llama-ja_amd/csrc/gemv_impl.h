@@ -1879,8 +1879,9 @@ static int launch_mb(const GemvParams& p, hipStream_t s) {
   if constexpr (tpw_ok<WF, AM>() && MB > 1) {  // M == 1 (MB 1) always one tile: pick_tpw
     // the residual ops (8 chunks in flight) take at most 2 tiles per workgroup (3 and 4 spill;
     // C / 16 tiles need 2 only past 256 CUs' worth: 13B / 30B / 65B)
-    // 2 and 3 rows on 8-bit codes keep one tile in the SwiGLU: 2 rows of 4096 -> 2 x 11008 19.9 us, 20.6 with three; 4 rows
-    // 20.8 and 20.8
+    // 2 and 3 rows on 8-bit codes keep one tile in the SwiGLU. us at 2, 3 and 4 rows, one tile -> share: 4096 -> 2 x 11008
+    // 21.4, 20.0, 20.4 -> 21.1, 20.6, 20.3; 4096 -> 2 x 14336 25.3, 24.8, 26.1 -> 26.2, 26.0, 26.1; 5120 -> 2 x 13824 30.3, 29.2,
+    // 29.7 -> 30.6, 29.7, 29.7; 2048 -> 2 x 5632 9.9, 10.2, 10.0 -> 9.9, 9.9, 10.0
     const int t = WF == WF_W8 && EP == EP_SWIGLU && p.M < 4 ? 1 : pick_tpw(p.N / 16, p.M);
     switch (EP == EP_RESID && t > 2 ? 2 : t) {
       case 2: return launch_t<WF, AM, EP, MB, NW, 2>(p, s);
@@ -1904,8 +1905,8 @@ static int launch(const GemvParams& p, hipStream_t s) {
   if constexpr (EP == EP_RESID && AM != AM_GLOBAL && LLJ_NWR != kNW) {
     if (p.K >= LLJ_NWR_KMIN) {  // residual ops: 256 workgroups, more waves each
       if (WF != WF_I8 && p.M == 1) return launch_mb<WF, AM, EP, 1, LLJ_NWR>(p, s);
-      // one tile per workgroup: an 8-row image of K >= 8192 exceeds the LDS cap, so the multi-tile
-      // forms (M >= 7) were unreachable here (and spilled: 256 VGPRs + scratch)
+      // one tile per workgroup, also for the 2 to 5 rows whose image of K >= 8192 fits the LDS: the multi-tile
+      // forms of these waves spill (256 VGPRs + scratch)
       return launch_t<WF, AM, EP, 8, LLJ_NWR, 1>(p, s);
     }
   }

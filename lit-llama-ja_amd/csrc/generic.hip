@@ -458,7 +458,7 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
                          part, per);
       return 0;
     };
-    // three buffers, except where three workgroups to a CU are one round and two are not (37 rows, 4096 -> 12288, 768 workgroups: 79 us
+    // three buffers, except where three workgroups to a CU (of 256) are one round and two are not (37 rows, 4096 -> 12288, 768 workgroups: 79 us
     // for 94 with three buffers; 301 rows, 480 workgroups: 278 with three, 291 with two, 324 through registers)
     const long wgs = (long)mt * nt * splits;
     const int e = wgs > 512 && wgs <= 768 ? go(gg_dma_kernel<2>, 2) : go(gg_dma_kernel<3>, 3);

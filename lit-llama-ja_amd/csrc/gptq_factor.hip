@@ -4,8 +4,8 @@
 // All three are C -= or += A^T B with both operands stored along their output index ("k-major": X of the Hessian is tokens x
 // columns, a block of the factor and the block's errors are 128 x columns), which v_mfma_f32_16x16x4_f32 takes from LDS without a
 // transposition: lane l reads element (k + l / 16, m + l % 16), rows 16 banks apart. One accumulator per output, ascending k.
-// Bound: the fp32 matrix rate (157 TFLOP/s dense). A step of 16 k of a 64 x 64 tile is 32 MFMAs of 32 cycles for 16 reads of 4
-// bytes a lane, so neither LDS nor the loads (the next tile's in registers while this one is multiplied) are near their limits.
+// Bound: the fp32 matrix rate (157 TFLOP/s dense). A wave's 16 k of a 64 x 64 tile are 16 MFMAs of 32 cycles for 16 reads of
+// 4 bytes a lane, so neither LDS nor the loads (the next tile's in registers while this one is multiplied) are near their limits.
 #include "common.h"
 
 namespace llj {
@@ -144,7 +144,7 @@ __device__ __forceinline__ void triangle(int t, int& i, int& j) {
 }
 
 // H = keep H + (alpha X)^T (alpha X): the tiles on and below the diagonal, each written to its place and mirrored. The sums are those
-// of the library's product bit for bit (to 4,096 columns), at half its work: 2048 x 4096 385 us (89 TFLOP/s of the half) for 580 with
+// of the library's product bit for bit (to 4,096 columns), at half its work: 2048 x 4096 422 us (83 TFLOP/s of the half) for 580 with
 // the two passes over H.
 template <int BT, typename S, bool VEC>
 __global__ __launch_bounds__(256) void gptq_gram_kernel(const S* __restrict__ x, int T, int K, float keep, float alpha, float* __restrict__ H) {
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256) void gptq_gram_kernel(const S* __restrict__ x,
 }
 
 // Wt[i2 + m][n] -= sum_b hinv[i1 + b][i2 + m] err[b][n]. Bound: Wt in and out beside the products; what is subtracted from is read
-// after them, all of it before the first use. 3968 x 4096: 51 us for 73 as a product and a subtraction, the same bits.
+// after them, all of it before the first use. 3968 x 4096: 56 us for 73 as a product and a subtraction, the same bits.
 template <int BM, int BN, bool VEC>
 __global__ __launch_bounds__(256) void gptq_update_kernel(const float* __restrict__ hinv, int K, int i1, int blk, const float* __restrict__ err,
                                                           int N, float* __restrict__ wt) {
