@@ -1783,8 +1783,13 @@ static inline int device_cus() {
   }
   return cus[dev];
 }
-// tiles per workgroup: ceil(tiles / CUs), i.e. about one workgroup per CU with every CU's
-// share of tiles minimal, capped at LLJ_TPW_MAX and the run-time cap. Batched rows only
+// tiles per workgroup, to LLJ_TPW_MAX and the run-time cap: the t of the least rounds(t) (4 t + fixed), rounds the workgroups over the
+// CUs and fixed what a workgroup costs beside its tiles, in quarters of a tile. To 1,024 tiles (4 a CU) that is ceil(tiles / CUs),
+// every CU's share in one round; past that a share of 4 may leave a last round nearly empty. us at 1, 2, 3 and 4 tiles, 4 rows:
+// int4 SwiGLU 6656 -> 2 x 17920 (1,120 tiles) 34.0, 30.2, 29.1, 34.4; QKV 8192 (1,536) 38.7, 27.4, 24.3, 26.7; head 4096 -> 35008
+// (2,188) 29.7, 22.2, 18.5, 20.1; 8-bit head 5120 -> 35008 43.8, 37.8, 33.8, 41.1; 32000 columns (2,000) are best at 4. fixed is 4, and 1
+// for the SwiGLU on 8-bit codes, whose two matrices leave less beside them: 6656 46.7, 51.9, 48.0, 66.4, 8192 67.2, 63.6, 61.1, 84.3.
+// Batched rows only
 // (M >= 2: one staged A image of M rows per CU instead of per tile, 1.966 -> 1.865 ms at 7B
 // bs=8); a single row keeps one tile per workgroup, where several workgroups per CU interleave
 // on each SIMD (measured 7B bs=1: 1.205 ms with one tile, 1.305 ms with three per workgroup).
@@ -1795,12 +1800,17 @@ static inline int device_cus() {
 #ifndef LLJ_TPW_MIN_M
 #define LLJ_TPW_MIN_M 2
 #endif
-static inline int pick_tpw(int ntiles, int M) {
+static inline int pick_tpw(int ntiles, int M, int cap, int fixed) {
   if (M < LLJ_TPW_MIN_M) return 1;
   const int cu = device_cus();
-  const int cap = g_tpw_max < LLJ_TPW_MAX ? g_tpw_max : LLJ_TPW_MAX;
-  const int t = (ntiles + cu - 1) / cu;
-  return t < 1 ? 1 : (t > cap ? cap : t);
+  cap = g_tpw_max < cap ? g_tpw_max : cap;
+  int best = 1;
+  long least = 0;
+  for (int t = 1; t <= cap; ++t) {
+    const long rounds = ((ntiles + t - 1) / t + cu - 1) / cu, cost = rounds * (4 * t + fixed);
+    if (t == 1 || cost <= least) best = t, least = cost;
+  }
+  return best;
 }
 // multi-tile instantiations: nibble-coded weights with the LDS A image or streamed A
 template <int WF, int AM>
@@ -1882,8 +1892,10 @@ static int launch_mb(const GemvParams& p, hipStream_t s) {
     // 2 and 3 rows on 8-bit codes keep one tile in the SwiGLU. us at 2, 3 and 4 rows, one tile -> share: 4096 -> 2 x 11008
     // 21.4, 20.0, 20.4 -> 21.1, 20.6, 20.3; 4096 -> 2 x 14336 25.3, 24.8, 26.1 -> 26.2, 26.0, 26.1; 5120 -> 2 x 13824 30.3, 29.2,
     // 29.7 -> 30.6, 29.7, 29.7; 2048 -> 2 x 5632 9.9, 10.2, 10.0 -> 9.9, 9.9, 10.0
-    const int t = WF == WF_W8 && EP == EP_SWIGLU && p.M < 4 ? 1 : pick_tpw(p.N / 16, p.M);
-    switch (EP == EP_RESID && t > 2 ? 2 : t) {
+    // So does the QKV product that forms the norm itself (a step's first): 4096 11.5, 14.8, 15.5 -> 13.6, 15.1, 15.3; 6656 26.8, 32.0 at
+    // 2 and 3 rows -> 30.9, 37.3
+    constexpr bool w8dual = WF == WF_W8 && EP == EP_SWIGLU, w8few = w8dual || (WF == WF_W8 && EP == EP_QKV && AM == AM_NORM);
+    switch (w8few && p.M < 4 ? 1 : pick_tpw(p.N / 16, p.M, EP == EP_RESID ? 2 : LLJ_TPW_MAX, w8dual ? 1 : 4)) {
       case 2: return launch_t<WF, AM, EP, MB, NW, 2>(p, s);
       case 3: if constexpr (EP != EP_RESID) return launch_t<WF, AM, EP, MB, NW, 3>(p, s); break;
       case 4: if constexpr (EP != EP_RESID) return launch_t<WF, AM, EP, MB, NW, 4>(p, s); break;

@@ -741,6 +741,37 @@ def test_multi_tile_workgroups_equal_single_tile(hip, wfmt, M):
         assert_bf16_close(multi[5].float().cpu().numpy(), rexp, "resid 13B")
 
 
+@pytest.mark.parametrize("wfmt", [0, 3])
+@pytest.mark.parametrize("tiles", [1025, 1120, 1376, 2188])
+def test_tiles_per_workgroup_beyond_four_a_cu(hip, wfmt, tiles):
+    """Tile counts whose share of a CU is more than a workgroup takes (the count is then chosen by its rounds): bitwise one
+    tile per workgroup, in the product with a norm and in the two-matrix one."""
+    rng = np.random.default_rng(tiles + wfmt)
+    K, N = 256, 16 * tiles
+    _, W1, s1 = quant_operands(hip, rng, wfmt, N, K)
+    _, W2, s2 = quant_operands(hip, rng, wfmt, N, K)
+    g = T(bf16(rng.uniform(0.5, 1.5, K)), torch.bfloat16)
+    for M in (2, 5, 8):
+        x = T(bf16(rng.standard_normal((M, K))), torch.bfloat16)
+
+        def run():
+            y, h = (torch.empty(M, N, dtype=torch.bfloat16, device=dev) for _ in range(2))
+            call(hip, "llj_norm_linear", wfmt, x.data_ptr(), g.data_ptr(), 1e-5, W1.data_ptr(), s1.data_ptr(), y.data_ptr(), N, M, N, K,
+                 None, 0, None, None, 0, st())
+            call(hip, "llj_norm_swiglu", wfmt, x.data_ptr(), g.data_ptr(), 1e-5, W1.data_ptr(), s1.data_ptr(), W2.data_ptr(), s2.data_ptr(),
+                 h.data_ptr(), M, N, K, None, 0, None, None, 0, st())
+            torch.cuda.synchronize()
+            return y, h
+
+        old = hip.llj_set_tpw_max(1)
+        try:
+            one = run()
+        finally:
+            hip.llj_set_tpw_max(old)
+        for a, b in zip(one, run()):
+            assert torch.equal(a, b), M
+
+
 @pytest.mark.parametrize("M,K", [(1, 4096), (8, 4096), (13, 4096), (3, 256), (8, 5120), (16, 5120), (20, 4096), (5, 11008)])
 def test_i8_norm_stats_equals_separate_launches(hip, M, K):
     """llj_i8_norm_stats (one launch for M <= 8, K <= 4096; RMSNorm + pass 1, then the row
