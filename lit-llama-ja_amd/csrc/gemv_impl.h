@@ -215,7 +215,7 @@ __device__ void stage_a(const GemvParams& p, bf16_t* As, int a_stride, float* re
 // int8: copy rows [0, M) of the activation quantized once by llj_i8_stats (outlier columns
 // already 0) into LDS int8 rows (stride K + 16 bytes). The rows are first in the workspace (i8ws.h):
 // their place does not depend on its header. One row is in registers by now (row0).
-constexpr int kQRow0 = 4;  // 16-byte registers of row 0 per thread
+constexpr int kQRow0 = 2;  // 16-byte registers of row 0 per thread: 8,192 values for 4 waves, 16,384 for 8 (4 took the residual op of K >= 8192 its second workgroup a CU)
 template <int NW>
 __device__ void stage_i8(const GemvParams& p, int8_t* Aq, int q_stride, const u32x4 (&row0)[kQRow0]) {
   const int tid = threadIdx.x;

@@ -285,7 +285,7 @@ def test_int8_linear_vs_restatement(hip, M, outliers):
 
 
 @pytest.mark.parametrize("row0,M", [(0, 8), (8, 4), (11, 1)])
-@pytest.mark.parametrize("K,outliers", [(4096, 3), (4096, 120), (8192, 300)])
+@pytest.mark.parametrize("K,outliers", [(4096, 3), (4096, 120), (8192, 300), (9216, 40)])
 def test_int8_linear_rows_of_a_larger_workspace(hip, row0, M, K, outliers):
     """Statistics of 12 rows, a product of some of them: the workspace's places are those of its own row count, not of
     the launch's. Tolerance: test_int8_linear_vs_restatement's."""
