@@ -77,8 +77,16 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
   int kv[SL];  // (past C: a valid place, whose values are left out of the sums)
 #pragma unroll
   for (int s = 0; s < SL; ++s) kv[s] = k0 + 512 * s < p.C ? k0 + 512 * s : 0;
+  // A wave whose slices are all past the row (8 waves of 1,024 values; C = 5,120 has three): its loads, though unused, would all be
+  // issued at once, ahead of the others'. Plain and streams: no loop for it. Norm: no loads; the branch in front of every wave's also
+  // holds the range of an output head or a SwiGLU back to what it took before the loads left their branches, which at 5,120 to
+  // 5,632 and 8,192 is less. us, loads of all waves / no loop / no loads: 5120 -> 32000 58.7 / 55.8 / 55.8, -> 35008 62.1 / 59.6 / 57.5,
+  // -> 2 x 13824 50.5 / 48.4 / 46.5; 5632 -> 35008 67.4 / 66.5 / 63.2; 8192 -> 2 x 22016 117.7 / 117.1 / 114.7; plain 4224 -> 4224
+  // 9.4 / 8.8 / 10.0; streams 4224 -> 28000 47.7 / 46.4 / 48.1. With 4 waves, or slices of 512, the test costs 1 to 5 %.
+  const bool idle = NW == 8 && SL == 2 && wave * (SL * 512) >= p.C;
   u32x4 wv[2][CB][SL];
   auto fetch = [&](int b, int c) {  // (columns past c1: the last pair again)
+    if (idle && PRO == RD_NORM) return;
 #pragma unroll
     for (int i = 0; i < CB; ++i) {
       const int n = min(c + (i & ~1), c1 - 2) + (i & 1);
@@ -243,6 +251,8 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
   };
   if constexpr (ONE) {
     columns(0, c0);
+  } else if (idle && PRO != RD_NORM) {
+    for (int i = lane; i < (c1 - c0) * 4; i += 64) rd_part[(i >> 2) * (NW * 4) + wave * 4 + (i & 3)] = 0.f;
   } else {
     int c = c0;
     for (; c + 3 * CB < c1; c += 2 * CB) {
