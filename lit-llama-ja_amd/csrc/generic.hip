@@ -356,10 +356,25 @@ int llj_g_rope_attention(const void* qkv, void* kcache, void* vcache, const floa
               llj_g_rope_attention_ok(S, C / n_head) && ((uintptr_t)kcache | (uintptr_t)vcache) % (dt ? 8 : 4) == 0);
   const size_t lds = gr_attention_lds(S, C / n_head);
   hipStream_t s = (hipStream_t)stream;
-  LLJ_DT(dt, hipLaunchKernelGGL(g_rope_attention_kernel<bf16_t>, dim3(B, n_head), dim3(kGrThreads), lds, s, (const bf16_t*)qkv,
-                                (bf16_t*)kcache, (bf16_t*)vcache, rope, pos, (bf16_t*)y, C, n_head, S),
-         hipLaunchKernelGGL(g_rope_attention_kernel<float>, dim3(B, n_head), dim3(kGrThreads), lds, s, (const float*)qkv, (float*)kcache,
-                            (float*)vcache, rope, pos, (float*)y, C, n_head, S));
+  // fp32 with more than a workgroup per CU: masked loads (12 rows of 32 heads, us without and with: heads of 80, 16 slots 7.3 and 7.0,
+  // 1,700 keys 84.6 and 80.9; of 128 7.8 and 7.2, 131 and 131; 8 rows, one workgroup a CU: 80, 500 keys 17.8 and 18.7; bf16 is 3 to 20 %
+  // faster without at either)
+  const bool mask = dt == 1 && (long)B * n_head > 256;
+#define LLJ_GRA(T, NQ, MASK) \
+  hipLaunchKernelGGL((g_rope_attention_kernel<T, NQ, MASK>), dim3(B, n_head), dim3(kGrThreads), lds, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
+#define LLJ_GRA_NQ(NQ)                        \
+  do {                                        \
+    if (dt == 0) LLJ_GRA(bf16_t, NQ, false);  \
+    else if (mask) LLJ_GRA(float, NQ, true);  \
+    else LLJ_GRA(float, NQ, false);           \
+  } while (0)
+  const int hs = C / n_head;
+  if (hs <= 32) LLJ_GRA_NQ(1);
+  else if (hs <= 64) LLJ_GRA_NQ(2);
+  else if (hs <= 96) LLJ_GRA_NQ(3);
+  else LLJ_GRA_NQ(4);
+#undef LLJ_GRA_NQ
+#undef LLJ_GRA
   LLJ_CHECK_LAUNCH();
   return 0;
 }

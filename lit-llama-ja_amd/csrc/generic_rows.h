@@ -153,12 +153,14 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
 // One token per sequence: rotary positions of q and k (g_rope_kv_kernel), k and v into cache slot p % S, and causal attention over
 // the cache (g_attention_kernel). Block (row, head) of 512 threads -- a few tens of blocks with a chain of memory trips each: 16
 // lanes per key and 128 keys at a time, then the values with the threads split over dimension pairs and up to kGrKeyGroups
-// interleaved groups of keys. The first keys and values are loaded before the rotation, without a branch around any of them (10 heads
+// interleaved groups of keys. The first keys and values are loaded before the rotation, without a branch around any of them but in MASK (10 heads
 // of 78, bf16, us behind branches -> this: 40 keys 6.4 -> 5.8, 110 keys 7.0 -> 6.1, 500 keys 16.7 -> 14.8; the next 128 keys
-// requested a pass ahead as well: 6.2, 6.5, 14.6). LDS: S + hs (3 + groups) floats.
+// requested a pass ahead as well: 6.2, 6.5, 14.6; fp32, 12 rows of 32 heads of 16, 1,700 keys, with 4 loads a key whatever the head 43.8,
+// with NQ 29.6). LDS: S + hs (3 + groups) floats.
 constexpr int kGrThreads = 512, kGrKeyGroups = 14;
 __host__ __device__ inline int gr_groups(int P) { return P > kGrThreads ? 1 : P * kGrKeyGroups > kGrThreads ? kGrThreads / P : kGrKeyGroups; }
-template <typename T>
+// NQ: pairs of a key's 16 lanes each, ceil(hs / 32) to 4. MASK: only what is seen is loaded, behind branches.
+template <typename T, int NQ, bool MASK>
 __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* __restrict__ qkv, T* __restrict__ kc, T* __restrict__ vc,
                                                                const float* __restrict__ rope, const int* __restrict__ pos,
                                                                T* __restrict__ y, int C, int nh, int S) {
@@ -175,16 +177,17 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
   const float scale = 1.f / sqrtf((float)hs);
   const T* row = qkv + (size_t)m * 3 * C + h * hs;
   const size_t cb = ((size_t)m * nh + h) * S * hs, cbase = cb + (size_t)slot * hs;
-  // keys j0 + 16 u of this group of 16 lanes, 64 pairs from i0 on: up to 16 loads in flight
+  // keys j0 + 32 u of this group of 16 lanes, 16 NQ pairs from i0 on: up to 16 loads in flight
   const int sub = tid & 15, kg = tid >> 4;
-  pair kw[4][4];
+  pair kw[4][NQ];
   auto keys = [&](int j0, int i0) {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < NQ; ++q) {
         const int j = min(j0 + 32 * u, S - 1), i = min(i0 + 16 * q + sub, P - 1);  // (a valid pair, not used past the last: no branch)
-        kw[u][q] = reinterpret_cast<const pair*>(kc + cb + (size_t)j * hs)[i];
+        if (MASK && !(j0 + 32 * u < nvis && i0 + 16 * q + sub < P)) kw[u][q] = pair(0);
+        else kw[u][q] = reinterpret_cast<const pair*>(kc + cb + (size_t)j * hs)[i];
       }
   };
   const int G = gr_groups(P), g = P > kGrThreads ? 0 : tid / P;
@@ -194,7 +197,10 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
   pair vw[VU];
   keys(kg, 0);
 #pragma unroll
-  for (int u = 0; u < VU; ++u) vw[u] = vr[(size_t)min(min(g, G - 1) + G * u, S - 1) * P];
+  for (int u = 0; u < VU; ++u) {
+    if (MASK && !(g < G && g + G * u < nvis)) vw[u] = pair(0);
+    else vw[u] = vr[(size_t)min(min(g, G - 1) + G * u, S - 1) * P];
+  }
   // in flight while q and k are rotated; the rows that this workgroup writes come from LDS
   for (int i = tid; i < P; i += kGrThreads) {
     const float c = rope[((size_t)p * P + i) * 2], s = rope[((size_t)p * P + i) * 2 + 1];
@@ -215,10 +221,10 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
   float mx = -INFINITY;
   for (int j0 = kg; j0 < nvis; j0 += 128) {
     float s[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int i0 = 0; i0 < P; i0 += 64) {
+    for (int i0 = 0; i0 < P; i0 += 16 * NQ) {
       if (j0 != kg || i0) keys(j0, i0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < NQ; ++q) {
         const int i = i0 + 16 * q + sub;
         if (i >= P) continue;
         const float q0 = sq[2 * i], q1 = sq[2 * i + 1];

@@ -387,9 +387,12 @@ def test_generic_rows_vs_float64_and_fused_forms(dt, M, N, K, off):
 
 @pytest.mark.parametrize("dt", [0, 1])
 @pytest.mark.parametrize("B,nh,hs,S,p", [(1, 10, 78, 132, 0), (3, 10, 78, 132, 131), (2, 2, 2, 16, 40), (1, 3, 64, 300, 17),
-                                         (8, 2, 128, 1000, 999), (1, 1, 600, 40, 20), (1, 1, 1100, 40, 39)])
+                                         (8, 2, 128, 1000, 999), (1, 1, 600, 40, 20), (1, 1, 1100, 40, 39), (1, 5, 32, 40, 10),
+                                         (2, 3, 34, 50, 49), (1, 2, 96, 200, 150), (33, 8, 16, 20, 7), (26, 10, 78, 132, 131), (13, 20, 128, 64, 100),
+                                         (300, 1, 66, 30, 0)])
 def test_generic_rope_attention_vs_separate_calls(dt, B, nh, hs, S, p):
-    """First position, a full cache, a wrapped ring, head sizes from one pair to more pairs than threads: the caches bitwise as
+    """First position, a full cache, a wrapped ring, head sizes from one pair to more pairs than threads, few and many (more than
+    256) rows and heads: the caches bitwise as
     llj_g_rope_kv leaves them, the output against attention in float64 over them. Bound: scores and weighted sums
     lose half an ulp per term of hs and S (exp: 2 more), relative to sum |p v|; bf16 results round by 2^-8."""
     from lit_llama import _hip
