@@ -287,6 +287,18 @@ __global__ __launch_bounds__(256) void g_i8_linear_kernel(const T* __restrict__ 
 
 // Elements per load: 16 bytes, 8 or single elements, as x, its rows and the weights' rows are aligned. Columns per wave: four from
 // 8192 on (every CU then still has 8 waves), one below.
+// Pieces per round for K of n: as many as there are up to 4; then 3 or 4, whichever leaves fewer past K; single elements from 20 on 8
+// (one column), where what counts is how much is in flight. 2 to 8 rows of four columns, whose loads per piece are 4 weights and
+// as many rows: one at a time to 8 pieces, 3 to 12, then 4. Time against 4 a round in every case (one column of the plain form 8, the last
+// 4 in branches), mean over sizes, bf16 / fp32: one column, n = 1 0.86 / 0.92, 2 0.90 / 0.94, 3 0.98 / 0.97, 9 0.91 / 0.94, 40 0.79 /
+// 0.88; four columns, one row, 1 0.76 / 0.71, 2 to 8 rows 1 0.65 / 0.65, 3 0.81 / 0.83, 9 0.89 / 0.92, 40 0.74 / 0.78.
+static int gr_pieces(int n, int ve, int nc, int M) {
+  if (nc > 1 && M > 1) return n <= 8 ? 1 : n <= 12 ? 3 : 4;
+  if (n <= 4) return n;
+  if (n >= 20 && ve == 1 && nc == 1) return 8;
+  return (n + 2) / 3 * 3 < (n + 3) / 4 * 4 ? 3 : 4;
+}
+
 template <typename T>
 static int gr_launch(int mode, const void* x, int ldx, const void* nw, float eps, int M, int K, const void* W, const void* W2,
                      int N, void* y, int ldy, const void* resid, int ldr, hipStream_t s) {
@@ -297,9 +309,21 @@ static int gr_launch(int mode, const void* x, int ldx, const void* nw, float eps
   };
   const size_t lds = mode == GR_PLAIN ? 0 : (size_t)M * K * el;
   const dim3 grid((N + 4 * nc - 1) / (4 * nc));
-#define LLJ_GR(VE, MB, NC, MODE)                                                                                               \
-  hipLaunchKernelGGL((g_rows_kernel<T, VE, MB, NC, MODE>), grid, dim3(256), lds, s, (const T*)x, ldx, (const T*)nw, eps, M, K, \
+#define LLJ_GR_U(VE, MB, NC, MODE, U, APART)                                                                                             \
+  hipLaunchKernelGGL((g_rows_kernel<T, VE, MB, NC, MODE, U, APART>), grid, dim3(256), lds, s, (const T*)x, ldx, (const T*)nw, eps, M, K, \
                      (const T*)W, (const T*)W2, N, (T*)y, ldy, (const T*)resid, ldr)
+#define LLJ_GR(VE, MB, NC, MODE)                                                                          \
+  do {                                                                                                    \
+    constexpr bool loop = MB > 1 && NC == 1 && MODE != GR_SWIGLU, many = MB > 1 && NC > 1;                \
+    const int n = (K + 64 * (VE) - 1) / (64 * (VE)), u = gr_pieces(n, VE, NC, M);                         \
+    if (u == 1) LLJ_GR_U(VE, MB, NC, MODE, 1, !loop);                                                     \
+    else if (u == 2 && !many) LLJ_GR_U(VE, MB, NC, MODE, (many ? 1 : 2), !loop);                          \
+    else if (u == 3 && loop && n == 3) LLJ_GR_U(VE, MB, NC, MODE, 3, !loop);                              \
+    else if (u == 3) LLJ_GR_U(VE, MB, NC, MODE, 3, true);                                                 \
+    else if (u == 4 && loop && n == 4) LLJ_GR_U(VE, MB, NC, MODE, 4, !loop);                              \
+    else if (u == 8 && VE == 1 && NC == 1) LLJ_GR_U(VE, MB, NC, MODE, (VE == 1 && NC == 1 ? 8 : 4), true); \
+    else LLJ_GR_U(VE, MB, NC, MODE, 4, true);                                                             \
+  } while (0)
 #define LLJ_GR_MODE(VE, MB)                                  \
   do {                                                       \
     if (mode == GR_SWIGLU) LLJ_GR(VE, MB, 1, GR_SWIGLU);     \
@@ -313,12 +337,13 @@ static int gr_launch(int mode, const void* x, int ldx, const void* nw, float eps
     if (M == 1) LLJ_GR_MODE(VE, 1); \
     else LLJ_GR_MODE(VE, GL_ROWS); \
   } while (0)
-  if (sizeof(T) == 2 && fits(8)) LLJ_GR_ROWS(sizeof(T) == 2 ? 8 : 4);
+  if (sizeof(T) == 2 && fits(8)) LLJ_GR_ROWS((sizeof(T) == 2 ? 8 : 4));
   else if (fits(4)) LLJ_GR_ROWS(4);
   else LLJ_GR_ROWS(1);
 #undef LLJ_GR_ROWS
 #undef LLJ_GR_MODE
 #undef LLJ_GR
+#undef LLJ_GR_U
   LLJ_CHECK_LAUNCH();
   return 0;
 }

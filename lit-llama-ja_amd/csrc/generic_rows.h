@@ -6,9 +6,8 @@
 // consecutive pieces of K. The residual's RMSNorm is computed by every workgroup for itself (a read of a few KB) in the order of
 // g_rmsnorm_kernel, so a layer is 5 launches instead of 10. Loads come back in order, so each wave requests what it needs first
 // first: the norm's row and weights (up to 1,024 values; beyond that they are read again), the residual, then the weights' pieces,
-// and all without a branch, from clamped addresses whose values go unused. Where the next pieces would be mostly past K (the
-// plain form's 5th to 8th) a branch is cheaper than the loads. us per launch, one row, weights first and all loads in
-// branches -> this: bf16, K = 780: rms_1 and c_attn 4.6 -> 4.0, c_proj 2.8 -> 2.6, rms_2, c_fc1, c_fc2 and silu * mul 5.8 -> 4.6,
+// and all without a branch, from clamped addresses whose values go unused; so a round has as many pieces as K needs (gr_pieces).
+// us per launch, one row, weights first and all loads in branches -> this with 4 a round: bf16, K = 780: rms_1 and c_attn 4.6 -> 4.0, c_proj 2.8 -> 2.6, rms_2, c_fc1, c_fc2 and silu * mul 5.8 -> 4.6,
 // mlp.c_proj (K = 2,080) 3.2 -> 3.0, lm_head 14.7 -> 11.0 (5.1 TB/s); four rows 10.6 -> 8.3, 4.7 -> 4.5, 13.1 -> 9.7, 5.7 -> 5.5,
 // 35.1 -> 29.4; fp32, K = 512: the same to 0.2 less, lm_head 15.2 -> 12.6; bf16, K = 2,100: 12.2 -> 11.2, 16.4 -> 14.3. Two
 // sets of 4 pieces by turns instead: 4.1, 2.7, 4.8, 3.5, 11.2.
@@ -24,14 +23,15 @@ constexpr int kGrNormLds = 48 * 1024;  // the rows' normalized copy of the norm-
 enum { GR_PLAIN = 0, GR_NORM = 1, GR_SWIGLU = 2 };
 
 // y[m, n] = x[m] . W[n] (+ resid), x through an RMSNorm in the fused forms; GR_SWIGLU: silu(x . W[n]) * (x . W2[n]). VE elements
-// per load: a divisor of K (and of ldx), with x and W aligned to it. MB: 1 or 8 rows' accumulators; NC: columns per wave.
-template <typename T, int VE, int MB, int NC, int MODE>
+// per load: a divisor of K (and of ldx), with x and W aligned to it. MB: 1 or 8 rows' accumulators; NC: columns per wave; U: pieces of 64
+// lanes x VE elements per round (gr_pieces). APART: the last round's code by itself.
+template <typename T, int VE, int MB, int NC, int MODE, int U, bool APART>
 __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, int ldx, const T* __restrict__ nw, float eps, int M,
                                                      int K, const T* __restrict__ W, const T* __restrict__ W2, int N,
                                                      T* __restrict__ y, int ldy, const T* resid, int ldr) {
   extern __shared__ __align__(16) char gr_lds[];
   typedef T vec __attribute__((ext_vector_type(VE)));
-  constexpr int U = MODE == GR_PLAIN && NC == 1 ? 8 : 4, NT = MODE == GR_SWIGLU ? 2 : NC;
+  constexpr int NT = MODE == GR_SWIGLU ? 2 : NC;
   const int tid = threadIdx.x, lane = tid & 63, n0 = (blockIdx.x * 4 + (tid >> 6)) * NC;
   const T* wr[NT];
 #pragma unroll
@@ -56,16 +56,12 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
     for (int r = 0; r < MB; ++r) rv[r] = rp[resid ? (size_t)min(r, M - 1) * ldr : 0];
   }
   vec wv[NT][U];
-  // piece u of a row: the first 4 from a valid address whatever k is
-  auto piece = [&](const T* p, int k, int u) {
-    if (u < 4 || k < K) return *reinterpret_cast<const vec*>(p + (u < 4 ? min(k, K - VE) : k));
-    return vec(0);
-  };
+  auto piece = [&](const T* p, int k) { return *reinterpret_cast<const vec*>(p + min(k, K - VE)); };  // (a valid address whatever k is)
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wv[t][u] = piece(wr[t], k0 + (u * 64 + lane) * VE, u);
+      for (int t = 0; t < NT; ++t) wv[t][u] = piece(wr[t], k0 + (u * 64 + lane) * VE);
   };
   fetch(0);
   T* xs = reinterpret_cast<T*>(gr_lds);
@@ -103,18 +99,22 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
   for (int r = 0; r < MB; ++r)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[r][t] = 0.f;
-  for (int k0 = 0; k0 < K; k0 += U * 64 * VE) {
-    if (k0) fetch(k0);
+  // One round; only the last asks of each piece whether it is past K (asked in every round, single elements, 8 rows of K = 6,400, bf16,
+  // -> 20,000: 145 us for 101). Its code is apart from the others', or with theirs in the loop, which one column of 2 to 8 rows prefers
+  // where K is a single round (fp32, K = 780 -> 780, norm: 4 rows 6.4 us apart, 5.5 in the loop; several rounds, bf16, 8 rows of 6,400 ->
+  // 3,000 21.3 and 24.0).
+  auto round = [&](int k0, bool last) {
 #pragma unroll
     for (int r = 0; r < MB; ++r) {
       if (r < M) {
         const T* xr = MODE == GR_PLAIN ? x + (size_t)r * ldx : xs + r * K;
         vec xv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) xv[u] = piece(xr, k0 + (u * 64 + lane) * VE, u);
-#pragma unroll
         for (int u = 0; u < U; ++u) {
-          if (k0 + (u * 64 + lane) * VE >= K) continue;
+          const int k = k0 + (u * 64 + lane) * VE;
+          xv[u] = APART && !last ? *reinterpret_cast<const vec*>(xr + k) : piece(xr, k);
+        }
+        auto add = [&](int u) {
 #pragma unroll
           for (int e = 0; e < VE; ++e) {
             T xe = xv[u][e];
@@ -124,8 +124,29 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
               acc[r][t] += ldv(&xe, 0) * ldv(&we, 0);
             }
           }
+        };
+        if (last) {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (k0 + (u * 64 + lane) * VE < K) add(u);
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u) add(u);
         }
       }
+    }
+  };
+  int k0 = 0;
+  if constexpr (APART) {
+    for (; k0 + U * 64 * VE < K; k0 += U * 64 * VE) {
+      round(k0, false);
+      fetch(k0 + U * 64 * VE);
+    }
+    round(k0, true);
+  } else {
+    for (; k0 < K; k0 += U * 64 * VE) {
+      if (k0) fetch(k0);
+      round(k0, k0 + U * 64 * VE > K);
     }
   }
 #pragma unroll
