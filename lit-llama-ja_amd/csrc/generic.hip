@@ -288,14 +288,15 @@ __global__ __launch_bounds__(256) void g_i8_linear_kernel(const T* __restrict__ 
 // Elements per load: 16 bytes, 8 or single elements, as x, its rows and the weights' rows are aligned. Columns per wave: four from
 // 8192 on (every CU then still has 8 waves), one below.
 // Pieces per round for K of n: as many as there are up to 4; then 3 or 4, whichever leaves fewer past K; single elements from 20 on 8
-// (one column), where what counts is how much is in flight. 2 to 8 rows of four columns, whose loads per piece are 4 weights and
+// (one column), where what counts is how much is in flight, and so one row of vectors to 8 in the plain form (bf16, 2080 -> 780 3.0 us, in
+// rounds of 3 3.2), the last 4 behind branches. 2 to 8 rows of four columns, whose loads per piece are 4 weights and
 // as many rows: one at a time to 8 pieces, 3 to 12, then 4. Time against 4 a round in every case (one column of the plain form 8, the last
 // 4 in branches), mean over sizes, bf16 / fp32: one column, n = 1 0.86 / 0.92, 2 0.90 / 0.94, 3 0.98 / 0.97, 9 0.91 / 0.94, 40 0.79 /
 // 0.88; four columns, one row, 1 0.76 / 0.71, 2 to 8 rows 1 0.65 / 0.65, 3 0.81 / 0.83, 9 0.89 / 0.92, 40 0.74 / 0.78.
-static int gr_pieces(int n, int ve, int nc, int M) {
+static int gr_pieces(int n, int ve, int nc, int M, bool plain) {
   if (nc > 1 && M > 1) return n <= 8 ? 1 : n <= 12 ? 3 : 4;
   if (n <= 4) return n;
-  if (n >= 20 && ve == 1 && nc == 1) return 8;
+  if (nc == 1 && (ve == 1 ? n >= 20 : n <= 8 && M == 1 && plain)) return 8;
   return (n + 2) / 3 * 3 < (n + 3) / 4 * 4 ? 3 : 4;
 }
 
@@ -315,13 +316,13 @@ static int gr_launch(int mode, const void* x, int ldx, const void* nw, float eps
 #define LLJ_GR(VE, MB, NC, MODE)                                                                          \
   do {                                                                                                    \
     constexpr bool loop = MB > 1 && NC == 1 && MODE != GR_SWIGLU, many = MB > 1 && NC > 1;                \
-    const int n = (K + 64 * (VE) - 1) / (64 * (VE)), u = gr_pieces(n, VE, NC, M);                         \
+    const int n = (K + 64 * (VE) - 1) / (64 * (VE)), u = gr_pieces(n, VE, NC, M, MODE == GR_PLAIN);       \
     if (u == 1) LLJ_GR_U(VE, MB, NC, MODE, 1, !loop);                                                     \
     else if (u == 2 && !many) LLJ_GR_U(VE, MB, NC, MODE, (many ? 1 : 2), !loop);                          \
     else if (u == 3 && loop && n == 3) LLJ_GR_U(VE, MB, NC, MODE, 3, !loop);                              \
     else if (u == 3) LLJ_GR_U(VE, MB, NC, MODE, 3, true);                                                 \
     else if (u == 4 && loop && n == 4) LLJ_GR_U(VE, MB, NC, MODE, 4, !loop);                              \
-    else if (u == 8 && VE == 1 && NC == 1) LLJ_GR_U(VE, MB, NC, MODE, (VE == 1 && NC == 1 ? 8 : 4), true); \
+    else if (u == 8) LLJ_GR_U(VE, MB, NC, MODE, (NC == 1 && (VE == 1 || (MB == 1 && MODE == GR_PLAIN)) ? 8 : 4), true); \
     else LLJ_GR_U(VE, MB, NC, MODE, 4, true);                                                             \
   } while (0)
 #define LLJ_GR_MODE(VE, MB)                                  \
@@ -389,7 +390,7 @@ int llj_g_rope_attention(const void* qkv, void* kcache, void* vcache, const floa
   hipLaunchKernelGGL((g_rope_attention_kernel<T, NQ, MASK>), dim3(B, n_head), dim3(kGrThreads), lds, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
 #define LLJ_GRA_NQ(NQ)                        \
   do {                                        \
-    if (dt == 0) LLJ_GRA(bf16_t, NQ, false);  \
+    if (dt == 0) LLJ_GRA(bf16_t, (NQ == 3 ? 4 : NQ), false);  \
     else if (mask) LLJ_GRA(float, NQ, true);  \
     else LLJ_GRA(float, NQ, false);           \
   } while (0)
