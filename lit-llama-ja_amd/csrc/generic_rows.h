@@ -56,12 +56,16 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
     for (int r = 0; r < MB; ++r) rv[r] = rp[resid ? (size_t)min(r, M - 1) * ldr : 0];
   }
   vec wv[NT][U];
-  auto piece = [&](const T* p, int k) { return *reinterpret_cast<const vec*>(p + min(k, K - VE)); };  // (a valid address whatever k is)
+  // piece u at k: from a valid address whatever k is; of 8 vectors, the last 4 behind branches
+  auto piece = [&](const T* p, int k, int u) {
+    if (U < 8 || VE == 1 || u < 4 || k < K) return *reinterpret_cast<const vec*>(p + min(k, K - VE));
+    return vec(0);
+  };
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wv[t][u] = piece(wr[t], k0 + (u * 64 + lane) * VE);
+      for (int t = 0; t < NT; ++t) wv[t][u] = piece(wr[t], k0 + (u * 64 + lane) * VE, u);
   };
   fetch(0);
   T* xs = reinterpret_cast<T*>(gr_lds);
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const int k = k0 + (u * 64 + lane) * VE;
-          xv[u] = APART && !last ? *reinterpret_cast<const vec*>(xr + k) : piece(xr, k);
+          xv[u] = APART && !last ? *reinterpret_cast<const vec*>(xr + k) : piece(xr, k, u);
         }
         auto add = [&](int u) {
 #pragma unroll
