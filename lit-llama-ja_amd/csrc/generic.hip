@@ -499,10 +499,13 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
                          part, per);
       return 0;
     };
-    // three buffers, except where three workgroups to a CU (of 256) are one round and two are not (37 rows, 4096 -> 12288, 768 workgroups: 79 us
-    // for 94 with three buffers; 301 rows, 480 workgroups: 278 with three, 291 with two, 324 through registers)
-    const long wgs = (long)mt * nt * splits;
-    const int e = wgs > 512 && wgs <= 768 ? go(gg_dma_kernel<2>, 2) : go(gg_dma_kernel<3>, 3);
+    // an XCD's tiles over its 32 CUs, three to a CU with two buffers and two with three: three buffers where more than one round of
+    // three remains and the last round of two is at least three quarters full, two otherwise (us with two, three buffers, through registers:
+    // 60 tiles, 301 rows 4096 -> 12288: 272, 280, 309; 96, 384 rows 5120 -> 64: 49, 59, 49, 37 rows 4096 -> 12288: 77, 93, 77; 128, 2048
+    // rows 4096 -> 4096: 570, 551, 603; 150, 300 rows 4096 -> 10240: 250, 289, 264; 256, 2048 rows 11008 -> 8192: 2964, 2875, 3127;
+    // 288, 100 rows 4096 -> 36000: 350, 380, 368)
+    const long tiles = (long)((nt + 7) / 8) * mt * splits;
+    const int e = tiles > 96 && (tiles - 1) % 64 >= 47 ? go(gg_dma_kernel<3>, 3) : go(gg_dma_kernel<2>, 2);
     if (e) return e;
   } else if (wkind == 0) {
     if (fits(x, ldx, 4)) LLJ_GG_CODES(4);

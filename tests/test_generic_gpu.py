@@ -309,11 +309,11 @@ def test_generic_gemm_edges_vs_float64(kind, bits, group, dt, M, N, K, pad, off)
 @pytest.mark.parametrize("M,N,K,pad,ws", [
     (9, 1, 3104, 0, True), (9, 129, 3104, 4, False), (64, 128, 4096, 0, True), (65, 129, 3104, 12, True), (65, 780, 4096, 0, False),
     (301, 1000, 3104, 0, True), (37, 12288, 4096, 0, True), (301, 13200, 3104, 4, False), (513, 11000, 3104, 0, False),
-    (64, 16500, 3072, 0, False), (70, 256, 32 * 113, 0, True)])
+    (64, 16500, 3072, 0, False), (70, 256, 32 * 113, 0, True), (1000, 7900, 3104, 0, False), (301, 5000, 3104, 4, True)])
 def test_generic_gemm_direct_tiles_equal_staged_ones(M, N, K, pad, ws):
     """fp32 rows above K = 3,071 in whole tiles, brought to LDS without registers, against the same product through registers (x one
     element off the alignment): the same sums bit for bit, with and without the residual in place. One workgroup and several rounds,
-    both buffer counts (513 to 768 workgroups take two), column and row remainders, padded rows, split K (32 x 113: splits of unequal
+    both buffer counts (the last two shapes take three), column and row remainders, padded rows, split K (32 x 113: splits of unequal
     length), no split."""
     from lit_llama import _hip
 
