@@ -289,12 +289,20 @@ __global__ __launch_bounds__(256) void g_i8_linear_kernel(const T* __restrict__ 
 // 8192 on (every CU then still has 8 waves), one below.
 // Pieces per round for K of n: as many as there are up to 4; then 3 or 4, whichever leaves fewer past K; single elements from 20 on 8
 // (one column), where what counts is how much is in flight, and so one row of vectors to 8 in the plain form (bf16, 2080 -> 780 3.0 us, in
-// rounds of 3 3.2), the last 4 behind branches. 2 to 8 rows of four columns, whose loads per piece are 4 weights and
-// as many rows: one at a time to 8 pieces, 3 to 12, then 4. Time against 4 a round in every case (one column of the plain form 8, the last
+// rounds of 3 3.2), the last 4 behind branches. Time against 4 a round in every case (one column of the plain form 8, the last
 // 4 in branches), mean over sizes, bf16 / fp32: one column, n = 1 0.86 / 0.92, 2 0.90 / 0.94, 3 0.98 / 0.97, 9 0.91 / 0.94, 40 0.79 /
-// 0.88; four columns, one row, 1 0.76 / 0.71, 2 to 8 rows 1 0.65 / 0.65, 3 0.81 / 0.83, 9 0.89 / 0.92, 40 0.74 / 0.78.
+// 0.88; four columns of one row, 1 0.76 / 0.71.
+// 2 to 8 rows of four columns (4 weights a piece, and in the plain form as many of x as there are rows, from the caches; formed rows lie
+// in LDS): fewer a round the wider the pieces. Time of 1, 2, 3, 4 a round in hundredths of what 8 behind branches took; plain, single
+// elements, fp32 6 pieces 114 103 95 99, 8 126 112 107 99; of 4, bf16 6 109 92 89 101, 8 128 100 99 98; of 8, 6 98 89 94 102, 40 119 89
+// 112 97; formed, single elements, fp32 6 99 88 86 89, 10 - 83 83 81; of 4, fp32 4 68 68 76 75, 12 - 89 88 87; of 8, 8 85 89 90 110, 24 92
+// 94 98 132.
 static int gr_pieces(int n, int ve, int nc, int M, bool plain) {
-  if (nc > 1 && M > 1) return n <= 8 ? 1 : n <= 12 ? 3 : 4;
+  if (nc > 1 && M > 1) {
+    if (plain) return ve == 8 ? (n > 1 ? 2 : 1) : n <= 3 ? n : n == 4 ? (ve == 4 ? 2 : 4) : n <= 6 || n == 9 ? 3 : 4;
+    if (ve == 1) return n == 1 ? 1 : n <= 6 ? 2 : 4;
+    return n <= ve ? 1 : ve == 8 || n <= 10 ? 2 : 4;
+  }
   if (n <= 4) return n;
   if (nc == 1 && (ve == 1 ? n >= 20 : n <= 8 && M == 1 && plain)) return 8;
   return (n + 2) / 3 * 3 < (n + 3) / 4 * 4 ? 3 : 4;
@@ -315,15 +323,16 @@ static int gr_launch(int mode, const void* x, int ldx, const void* nw, float eps
                      (const T*)W, (const T*)W2, N, (T*)y, ldy, (const T*)resid, ldr)
 #define LLJ_GR(VE, MB, NC, MODE)                                                                          \
   do {                                                                                                    \
-    constexpr bool loop = MB > 1 && NC == 1 && MODE != GR_SWIGLU, many = MB > 1 && NC > 1;                \
+    constexpr bool loop = MB > 1 && NC == 1 && MODE != GR_SWIGLU;                                         \
+    constexpr bool many = MB > 1 && NC > 1, few = many && VE == 8, none3 = few || (many && MODE == GR_NORM); \
     const int n = (K + 64 * (VE) - 1) / (64 * (VE)), u = gr_pieces(n, VE, NC, M, MODE == GR_PLAIN);       \
     if (u == 1) LLJ_GR_U(VE, MB, NC, MODE, 1, !loop);                                                     \
-    else if (u == 2 && !many) LLJ_GR_U(VE, MB, NC, MODE, (many ? 1 : 2), !loop);                          \
+    else if (u == 2) LLJ_GR_U(VE, MB, NC, MODE, 2, !loop);                                                \
     else if (u == 3 && loop && n == 3) LLJ_GR_U(VE, MB, NC, MODE, 3, !loop);                              \
-    else if (u == 3) LLJ_GR_U(VE, MB, NC, MODE, 3, true);                                                 \
+    else if (u == 3 && !none3) LLJ_GR_U(VE, MB, NC, MODE, (none3 ? 2 : 3), true);                         \
     else if (u == 4 && loop && n == 4) LLJ_GR_U(VE, MB, NC, MODE, 4, !loop);                              \
     else if (u == 8) LLJ_GR_U(VE, MB, NC, MODE, (NC == 1 && (VE == 1 || (MB == 1 && MODE == GR_PLAIN)) ? 8 : 4), true); \
-    else LLJ_GR_U(VE, MB, NC, MODE, 4, true);                                                             \
+    else LLJ_GR_U(VE, MB, NC, MODE, (few ? 2 : 4), true);                                                 \
   } while (0)
 #define LLJ_GR_MODE(VE, MB)                                  \
   do {                                                       \

@@ -348,7 +348,8 @@ def test_generic_gemm_direct_tiles_equal_staged_ones(M, N, K, pad, ws):
 @pytest.mark.parametrize("M", [1, 3, 8])
 @pytest.mark.parametrize("N,K,off", [(1, 1, 0), (5, 6, 0), (780, 780, 0), (36, 2304, 0), (129, 4100, 1), (8200, 260, 0), (8193, 40, 0),
                                      (70, 500, 0), (70, 700, 0), (70, 900, 0), (70, 1500, 0), (40, 5200, 0), (36, 1283, 0), (36, 1285, 1),
-                                     (8200, 700, 0), (8200, 1000, 0), (8200, 701, 0), (8195, 1030, 0), (8200, 2600, 0), (8200, 3300, 0)])
+                                     (8200, 700, 0), (8200, 1000, 0), (8200, 701, 0), (8195, 1030, 0), (8200, 2600, 0), (8200, 3300, 0),
+                                     (8200, 101, 0), (8200, 201, 0), (8195, 321, 0), (8200, 1020, 0)])
 def test_generic_rows_vs_float64_and_fused_forms(dt, M, N, K, off):
     """Rows of x at and off the loads' alignment, columns in ones and fours, K of 1 to 8 pieces a round and of several rounds, K tails, the
     residual in place. Bound: a lane
