@@ -573,8 +573,10 @@ int llj_g_attention(const void* q, const void* kcache, const void* vcache, void*
   hipStream_t s = (hipStream_t)stream;
   // The tiles from 1,024 (row, head) pairs on: below, one workgroup per pair is a shorter chain (us, pairs -> tiles; fp32, heads of 78:
   // 4 rows of 10 heads 4.8 and 7.6, 100 rows 9.2 and 10.4, 128 rows 15.0 and 10.3, 1,000 rows 397 and 74; 301 rows of 32 heads of
-  // 128 137 and 37).
-  if (T >= kGaRows && (long)B * T * n_head >= 1024) {
+  // 128 137 and 37), below 48 rows from 2,048 on: a prompt at the sequence's start then has one short tile of keys (fp32, heads of 80: 36 rows of
+  // 32 heads 6.5 and 7.1, 24 of 80 0.89 of the tiles, 64 rows of 32 heads 1.3; from position 200 on the tiles are ahead from some 500
+  // pairs, but the host does not know where the rows stand).
+  if (T >= kGaRows && (long)B * T * n_head >= (T < 48 ? 2048 : 1024)) {
     const int e = dt == 0 ? ga_launch((const bf16_t*)q, (const bf16_t*)kcache, (const bf16_t*)vcache, (bf16_t*)y, pos, B, T, C, n_head, S, s)
                           : ga_launch((const float*)q, (const float*)kcache, (const float*)vcache, (float*)y, pos, B, T, C, n_head, S, s);
     if (e != 1) return e;

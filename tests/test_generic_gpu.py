@@ -429,7 +429,7 @@ def test_generic_rope_attention_vs_separate_calls(dt, B, nh, hs, S, p):
 @pytest.mark.parametrize("B,T,nh,hs,S,p0", [(1, 301, 32, 128, 301, 0), (2, 67, 10, 78, 80, 5), (1, 130, 8, 1, 130, 0), (3, 49, 8, 13, 64, 40),
                                             (1, 1030, 1, 256, 1030, 0), (2, 129, 5, 101, 200, 0), (1, 70, 16, 64, 72, 60), (1, 128, 9, 250, 128, 0),
                                             (1, 130, 8, 17, 130, 0), (1, 140, 8, 63, 150, 7), (1, 131, 8, 82, 131, 0), (1, 129, 8, 126, 140, 9),
-                                            (1, 130, 8, 132, 130, 0)])
+                                            (1, 130, 8, 132, 130, 0), (1, 36, 32, 80, 36, 0), (4, 36, 16, 80, 40, 2), (1, 48, 22, 64, 48, 0)])
 def test_prompt_attention_tiles(hip, dtype, B, T, nh, hs, S, p0):
     """llj_g_attention on tiles of 16 rows and 64 keys, any head size (also one whose vectors are too many for the tiles), remainders of
     both, rows whose positions have gone round the cache, unseen slots that hold NaN. Against float64: the output's own rounding, and in
