@@ -395,6 +395,8 @@ int llj_g_rope_attention(const void* qkv, void* kcache, void* vcache, const floa
   // 1,700 keys 84.6 and 80.9; of 128 7.8 and 7.2, 131 and 131; 8 rows, one workgroup a CU: 80, 500 keys 17.8 and 18.7; bf16 is 3 to 20 %
   // faster without at either)
   const bool mask = dt == 1 && (long)B * n_head > 256;
+  // bf16 heads of 65 to 96 take four pairs a lane: with three the compiler puts the loads of the new token's row one behind the other's
+  // wait (in a decode step of 10 heads of 78 7.7 us and 6.7)
 #define LLJ_GRA(T, NQ, MASK) \
   hipLaunchKernelGGL((g_rope_attention_kernel<T, NQ, MASK>), dim3(B, n_head), dim3(kGrThreads), lds, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
 #define LLJ_GRA_NQ(NQ)                        \

@@ -4,7 +4,7 @@
 // Decode of these models (780 wide, 3.6 MB per matrix) is bound by latency: what counts is how many dependent memory trips and
 // launches a layer has. A wave takes one output column (four where there are columns enough for every CU), its lanes
 // consecutive pieces of K. The residual's RMSNorm is computed by every workgroup for itself (a read of a few KB) in the order of
-// g_rmsnorm_kernel, so a layer is 5 launches instead of 10. Loads come back in order, so each wave requests what it needs first
+// g_rmsnorm_kernel, so a layer is 5 launches instead of 10. Loads come back in order, so each wave requests first what it needs
 // first: the norm's row and weights (up to 1,024 values; beyond that they are read again), the residual, then the weights' pieces,
 // and all without a branch, from clamped addresses whose values go unused; so a round has as many pieces as K needs (gr_pieces).
 // us per launch, one row, weights first and all loads in branches -> this with 4 a round: bf16, K = 780: rms_1 and c_attn 4.6 -> 4.0, c_proj 2.8 -> 2.6, rms_2, c_fc1, c_fc2 and silu * mul 5.8 -> 4.6,
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
 // with NQ 29.6). LDS: S + hs (3 + groups) floats.
 constexpr int kGrThreads = 512, kGrKeyGroups = 14;
 __host__ __device__ inline int gr_groups(int P) { return P > kGrThreads ? 1 : P * kGrKeyGroups > kGrThreads ? kGrThreads / P : kGrKeyGroups; }
-// NQ: pairs of a key's 16 lanes each, ceil(hs / 32) to 4. MASK: only what is seen is loaded, behind branches.
+// NQ: pairs of a key's 16 lanes each, ceil(hs / 32) to 4 (bf16: 4 for 3). MASK: only what is seen is loaded, behind branches.
 template <typename T, int NQ, bool MASK>
 __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* __restrict__ qkv, T* __restrict__ kc, T* __restrict__ vc,
                                                                const float* __restrict__ rope, const int* __restrict__ pos,
