@@ -11,6 +11,7 @@
 #include "generic_attention.h"
 #include "generic_gemm.h"
 #include "generic_rows.h"
+#include "generic_split.h"
 #include "lit_llama_amd.h"
 
 namespace llj {
@@ -436,7 +437,7 @@ int llj_g_rmsnorm(const void* x, int ldx, const void* w, float eps, void* y, int
 
 size_t llj_g_linear_ws_bytes(int wkind, int M, int N, int K, int dt) {
   if (M <= GL_ROWS || N <= 0 || K <= 0) return 0;
-  const int s = gg_splits(M, N, K, dt == 1 || wkind == 0, dt == 1 && K <= kGgFineK);
+  const int s = gs_takes(wkind, dt) ? gs_plan(M, N, K, true).splits : gg_splits(M, N, K, dt == 1 || wkind == 0, dt == 1 && K <= kGgFineK);
   return s > 1 ? (size_t)s * M * N * 4 : 0;
 }
 
@@ -458,6 +459,13 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
 #undef LLJ_GL
     LLJ_CHECK_LAUNCH();
     return 0;
+  }
+  if (gs_takes(wkind, dt)) {
+    GsPlan p = gs_plan(M, N, K, ws != nullptr);
+    if (p.splits > 1 && ws_bytes < (size_t)p.splits * M * N * 4) p = gs_plan(M, N, K, false);
+    const int e = gs_launch(p, (const float*)x, ldx, M, K, (const float*)W, N, (float*)y, ldy, (const float*)resid, ldr, (float*)ws, s);
+    if (e) return e;
+    return p.splits > 1 ? gg_reduce((const float*)ws, p.splits, M, N, (float*)y, ldy, (const float*)resid, ldr, s) : 0;
   }
   const bool f32 = dt == 1 || wkind == 0;  // bf16 rows on codes: the weight element (q - zero) * scale is fp32
   const bool fine = dt == 1 && K <= kGgFineK;  // fp32 operands: short chains of sums
@@ -483,11 +491,6 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
     if (FINE && splits == 1 && all >= 8) LLJ_GG_GO(T, CT, VEX, J, FINE, FINE, __VA_ARGS__);       \
     else LLJ_GG_GO(T, CT, VEX, J, FINE, false, __VA_ARGS__);                                      \
   } while (0)
-#define LLJ_GG_F32(VE)                                                      \
-  do {                                                                      \
-    if (fine) LLJ_GG_RUN(float, float, VE, 1, true, GgWeightDense<float, VE, 512>); \
-    else LLJ_GG_RUN(float, float, VE, 2, false, GgWeightDense<float, VE, 256>);     \
-  } while (0)
 #define LLJ_GG_BF16(VE) LLJ_GG_RUN(bf16_t, bf16_t, VE, 1, false, GgWeightDense<bf16_t, VE, 512>)
 #define LLJ_GG_BITS(B, VE)                                                                 \
   do {                                                                                     \
@@ -501,29 +504,9 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
     else if (bits == 8) LLJ_GG_BITS(8, VE); \
     else LLJ_GG_BITS(2, VE);              \
   } while (0)
-  if (wkind == 1 && dt == 1 && !fine && K % 32 == 0 && fits(x, ldx, 4) && fits(W, K, 4)) {
-    auto go = [&](auto kern, int stages) {
-      const size_t lds = (size_t)stages * (kGgBM + kGgBN) * kGgRow;
-      const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return (int)e;
-      hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, (const float*)x, ldx, M, K, (const float*)W, N, (float*)y, ldy, (const float*)resid, ldr,
-                         part, per);
-      return 0;
-    };
-    // an XCD's tiles over its 32 CUs, three to a CU with two buffers and two with three: three buffers where more than one round of
-    // three remains and the last round of two is at least three quarters full, two otherwise (us with two, three buffers, through registers:
-    // 60 tiles, 301 rows 4096 -> 12288: 272, 280, 309; 96, 384 rows 5120 -> 64: 49, 59, 49, 37 rows 4096 -> 12288: 77, 93, 77; 128, 2048
-    // rows 4096 -> 4096: 570, 551, 603; 150, 300 rows 4096 -> 10240: 250, 289, 264; 256, 2048 rows 11008 -> 8192: 2964, 2875, 3127;
-    // 288, 100 rows 4096 -> 36000: 350, 380, 368)
-    const long tiles = (long)((nt + 7) / 8) * mt * splits;
-    const int e = tiles > 96 && (tiles - 1) % 64 >= 47 ? go(gg_dma_kernel<3>, 3) : go(gg_dma_kernel<2>, 2);
-    if (e) return e;
-  } else if (wkind == 0) {
+  if (wkind == 0) {
     if (fits(x, ldx, 4)) LLJ_GG_CODES(4);
     else LLJ_GG_CODES(1);
-  } else if (dt == 1) {
-    if (fits(x, ldx, 4) && fits(W, K, 4)) LLJ_GG_F32(4);
-    else LLJ_GG_F32(1);
   } else {
     if (fits(x, ldx, 8) && fits(W, K, 8)) LLJ_GG_BF16(8);
     else if (fits(x, ldx, 4) && fits(W, K, 4)) LLJ_GG_BF16(4);
@@ -532,20 +515,12 @@ int llj_g_linear_ws(int wkind, const void* x, int ldx, int M, int K, const void*
 #undef LLJ_GG_CODES
 #undef LLJ_GG_BITS
 #undef LLJ_GG_BF16
-#undef LLJ_GG_F32
 #undef LLJ_GG_RUN
 #undef LLJ_GG_GO
-  if (part) {
-    LLJ_CHECK_LAUNCH();
-    const size_t blocks = ((size_t)M * N + 255) / 256;
-    const unsigned g = blocks < 4096 ? (unsigned)blocks : 4096u;
-    LLJ_DT(dt, hipLaunchKernelGGL(gg_reduce_kernel<bf16_t>, dim3(g), dim3(256), 0, s, part, splits, M, N, (bf16_t*)y, ldy,
-                                  (const bf16_t*)resid, ldr),
-           hipLaunchKernelGGL(gg_reduce_kernel<float>, dim3(g), dim3(256), 0, s, part, splits, M, N, (float*)y, ldy,
-                              (const float*)resid, ldr));
-  }
   LLJ_CHECK_LAUNCH();
-  return 0;
+  if (!part) return 0;
+  return dt == 0 ? gg_reduce(part, splits, M, N, (bf16_t*)y, ldy, (const bf16_t*)resid, ldr, s)
+                 : gg_reduce(part, splits, M, N, (float*)y, ldy, (const float*)resid, ldr, s);
 }
 
 int llj_g_linear(int wkind, const void* x, int ldx, int M, int K, const void* W, const float* scales, const float* zeros,

@@ -1,25 +1,22 @@
 // Tiled matrix products of the any-shape path (generic.hip's llj_g_linear / _ws for more than GL_ROWS rows): y = x . W^T for
-// any M, N, K and strides, on the matrix cores.
+// any M, N, K and strides, on the matrix cores: bf16 rows, and rows of either type on codes (dense fp32: generic_split.h).
 //
-// A workgroup computes 64 rows x 128 columns: fp32 four waves of two 32x32 accumulators (eight of one: 332 us for 310 at
-// 301 x 11008 x 4096), bf16 and short fp32 chains eight of one (four of two: 136 us for 120 at 2048 x 4096 x 4096 bf16, more
-// steps between barriers that one wave cannot fill). Both operands go through
+// A workgroup computes 64 rows x 128 columns: fp32 four waves of two 32x32 accumulators, bf16 and short fp32 chains eight of one (four of
+// two: 136 us for 120 at 2048 x 4096 x 4096 bf16, more steps between barriers that one wave cannot fill). Both operands go through
 // LDS as rows of 128 bytes of K (32 fp32 / 64 bf16 values), the 16-byte chunk c of row r at place c ^ (r / 2 % 8): 16 lanes
 // reading one chunk of 16 consecutive rows then fall on 16 different groups of four banks (padded rows, as free of
-// conflicts, left room for two workgroups per CU instead of three: 651 us for 642 at 2048 x 4096 x 4096 fp32). One read of 16 bytes per lane (lanes 0-31 the even
+// conflicts, left room for two workgroups per CU instead of three). One read of 16 bytes per lane (lanes 0-31 the even
 // chunks, 32-63 the odd ones) is four fp32 or one bf16 MFMA step -- the products' order over K is free as long as both
 // operands agree. Two LDS buffers, the next tile's loads in registers while the current one is multiplied, one barrier
 // per tile.
 //
-// Bound: the fp32 MFMA rate (v_mfma_f32_32x32x2_f32, 157 TFLOP/s dense; its operands need 32 of LDS's 128 bytes per clock), so
-// no larger tile is needed to feed it; 64 rows waste little on prompts of some hundred rows. One output column per wave, which this
-// replaces from 9 rows on, read x through the cache 8 times per weight element. fp32, 301 rows, 4096 -> 12288: 7,369 us before
-// (4.1 TFLOP/s), 354 now (86); 11008 -> 4096: 6,543 and 285 (95). bf16, 100 rows, 780 -> 2304: 87 and 11.
+// Bound: the MFMA rate (fp32 operands: v_mfma_f32_32x32x2_f32, 157 TFLOP/s dense; they need 32 of LDS's 128 bytes per clock), so
+// no larger tile is needed to feed it; 64 rows waste little on prompts of some hundred rows. bf16, 100 rows, 780 -> 2304: 11 us (87 with
+// one output column per wave, which reads x through the cache 8 times per weight element).
 //
-// fp32 sums are no further from exact ones than the per-lane sums of K / 64 terms that they replace (2-norm error against
-// float64, random operands): from K = kGgFineK down an accumulator runs over 8 values of K, four of those are added pairwise, four of
-// these sums in a second and the rest in a third accumulator, and from 8 tiles on each half of K by itself (K = 780: error 9.5e-8
-// in one piece, 9.0e-8 in two or more, 9.3e-8 before); above it 32 values, eight of those, and the rest.
+// fp32 sums (codes): from K = kGgFineK down an accumulator runs over 8 values of K, four of those are added pairwise, four of
+// these sums in a second and the rest in a third accumulator, and from 8 tiles on each half of K by itself; above it 32 values,
+// eight of those, and the rest (2-norm error against float64, random operands: 9.0e-8 at K = 780, 1.3e-7 to 1.7e-7 at 4096 and above).
 #pragma once
 #include "common.h"
 #include "elem.h"
@@ -138,7 +135,7 @@ struct GgWeightCodes {
 // Blocks: (8 * ceil(column tiles / 8) * row tiles, splits); block b runs on XCD b % 8, whose L2 keeps a column tile's weights
 // for its row tiles.
 // (At least two waves per SIMD: registers stay below 256, where the compiler keeps the accumulators in plain registers and the sums
-// need no copies out of the accumulation registers. 301 rows, 4096 -> 12288: 385 us and 352, 2048 rows, 4096 -> 4096: 647 and 605.)
+// need no copies out of the accumulation registers.)
 template <typename WL, typename T, typename CT, int VEX, int J, bool FINE, bool HALVES>
 __global__ __launch_bounds__(512 / J, 2) void gg_kernel(const T* __restrict__ x, int ldx, int M, int K, const void* __restrict__ W,
                                                      const float* __restrict__ sc, const float* __restrict__ zr, int group,
@@ -243,91 +240,6 @@ __global__ __launch_bounds__(512 / J, 2) void gg_kernel(const T* __restrict__ x,
   }
 }
 
-// gg_kernel's dense fp32 form above kGgFineK for rows of whole tiles (K and the row strides multiples of 32 and 4 elements, rows aligned):
-// the same sums, the tiles brought to LDS by global_load_lds (no registers, no store), ST - 1 ahead of the one in use. The wait for a
-// tile is a counted vmcnt and a plain barrier. Three buffers leave two workgroups to a CU, two buffers three.
-typedef __attribute__((address_space(3))) void gg_lds_t;
-template <int N>
-__device__ __forceinline__ void gg_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-template <int ST>
-__global__ __launch_bounds__(256, ST == 2 ? 3 : 2) void gg_dma_kernel(const float* __restrict__ x, int ldx, int M, int K, const float* __restrict__ W, int N,
-                                                        float* __restrict__ y, int ldy, const float* resid, int ldr, float* __restrict__ part,
-                                                        int split_tiles) {
-  constexpr int J = 2, KT = 32, kStage = (kGgBM + kGgBN) * kGgRow, ND = (kGgBM + kGgBN) / 32;
-  extern __shared__ __align__(16) char gg_stages[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
-  const int mt = (M + kGgBM - 1) / kGgBM, local = blockIdx.x >> 3;
-  const int nt = (int)(blockIdx.x & 7) + 8 * (local / mt);
-  if (nt * kGgBN >= N) return;
-  const int m0 = (local % mt) * kGgBM, n0 = nt * kGgBN;
-  const int t0 = blockIdx.y * split_tiles, all = K / KT, t1 = min(all, t0 + split_tiles);
-  // eight rows of 128 bytes an instruction; lane l's 16 bytes land at place l % 8 of row l / 8, so they are chunk (l % 8) ^ (row / 2 % 8)
-  const float* src[ND];
-#pragma unroll
-  for (int i = 0; i < ND; ++i) {
-    const int row = 8 * (4 * i + wave) + (lane >> 3), c = (lane & 7) ^ (row >> 1 & 7);  // of the stage: 64 of x, 128 of W
-    src[i] = (i < 2 ? x + (size_t)min(m0 + row, M - 1) * ldx : W + (size_t)min(n0 + row - kGgBM, N - 1) * K) + 4 * c;
-  }
-  auto stage = [&](int buf, int t) {
-    const int tt = t < t1 ? t : t1 - 1;  // past the range: a copy that is not read
-#pragma unroll
-    for (int i = 0; i < ND; ++i)
-      __builtin_amdgcn_global_load_lds(src[i] + (size_t)tt * KT, (gg_lds_t*)(gg_stages + buf * kStage + (4 * i + wave) * 1024), 16, 0, 0);
-  };
-  f32x16 mid[J] = {}, tot[J] = {};
-  const int nw = (wave >> 1) * 32 * J;  // the wave's first column
-  const int ra = gg_at((wave & 1) * 32 + (lane & 31), lane >> 5), rb = gg_at(kGgBM + nw + (lane & 31), lane >> 5);
-  stage(0, t0);
-  if constexpr (ST == 3) stage(1, t0 + 1);
-  int buf = 0;
-  for (int t = t0; t < t1; ++t) {
-    gg_wait<(ST - 2) * ND>();  // tile t has landed, the next one may be on its way
-    __builtin_amdgcn_s_barrier();  // for every wave; and all are done with the buffer of tile t - 1
-    stage(buf == 0 ? ST - 1 : buf - 1, t + ST - 1);
-    const char* b = gg_stages + buf * kStage;
-    f32x4 fa[4], fb[J][4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      fa[g] = *reinterpret_cast<const f32x4*>(b + (ra ^ g << 5));
-#pragma unroll
-      for (int j = 0; j < J; ++j) fb[j][g] = *reinterpret_cast<const f32x4*>(b + (rb ^ g << 5) + 32 * j * kGgRow);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // (read one by one in front of their products, each waited alone)
-    f32x16 acc[J] = {};
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int j = 0; j < J; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[g][e], fb[j][g][e], acc[j], 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < J; ++j) mid[j] += acc[j];
-    if (((t - t0) & 7) == 7) {
-#pragma unroll
-      for (int j = 0; j < J; ++j) {
-        tot[j] += mid[j];
-        mid[j] = f32x16{};
-      }
-    }
-    buf = buf == ST - 1 ? 0 : buf + 1;
-  }
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    tot[j] += mid[j];
-    const int n = n0 + nw + 32 * j + (lane & 31);
-    if (n >= N) continue;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = m0 + (wave & 1) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-      if (m >= M) continue;
-      if (part) part[((size_t)blockIdx.y * M + m) * N + n] = tot[j][i];
-      else y[(size_t)m * ldy + n] = resid ? resid[(size_t)m * ldr + n] + tot[j][i] : tot[j][i];
-    }
-  }
-}
-
 // y = the splits' sums, added pairwise (and the residual), as gg_kernel's own epilogue
 template <typename T>
 __global__ __launch_bounds__(256) void gg_reduce_kernel(const float* __restrict__ part, int splits, int M, int N, T* __restrict__ y,
@@ -347,12 +259,18 @@ __global__ __launch_bounds__(256) void gg_reduce_kernel(const float* __restrict_
   }
 }
 
+template <typename T>
+inline int gg_reduce(const float* part, int splits, int M, int N, T* y, int ldy, const T* resid, int ldr, hipStream_t s) {
+  const size_t blocks = ((size_t)M * N + 255) / 256;
+  hipLaunchKernelGGL(gg_reduce_kernel<T>, dim3(blocks < 4096 ? (unsigned)blocks : 4096u), dim3(256), 0, s, part, splits, M, N, y, ldy, resid, ldr);
+  LLJ_CHECK_LAUNCH();
+  return 0;
+}
+
 // K ranges of a product: what makes the last round of workgroups over the 256 CUs cheapest, against the partial sums'
 // traffic and launch. Microseconds: a tile step at the MFMA rate of one CU (0.9 fp32, 0.2 bf16), partials
 // written and read at 4.9 TB/s, 3 for the second launch. fine (fp32 operands, K <= kGgFineK): at least two ranges while their scratch
-// is small, for the shorter sums; larger outputs keep the halves apart inside one workgroup (HALVES). fp32, K = 780, us in two
-// ranges / in halves: 1000 x 2304 77 / 96, 100 x 35008 120 / 143, 300 x 35008 (80 MiB of scratch) 264 / 284, 1000 x 35008
-// (267 MiB) 875 / 842, 2048 x 35008 1757 / 1647.
+// is small, for the shorter sums; larger outputs keep the halves apart inside one workgroup (HALVES).
 inline int gg_splits(int M, int N, int K, bool f32, bool fine) {
   const int KT = kGgRow / (f32 ? 4 : 2), all = (K + KT - 1) / KT;
   const long tiles = (long)((M + kGgBM - 1) / kGgBM) * ((N + kGgBN - 1) / kGgBN);

@@ -13,6 +13,8 @@ ids and steps (tools/noise_floor.py --generic, profiles/r03_noise_floor_generic.
 carry more of it than the 2-layer width tests: n_embd 32 x 16 layers floor max 2.87e-2 / mean
 2.9e-3; 125M (12 layers) max 1.71e-2 (bf16) / 1.88e-2 (int4), mean <= 1.56e-2. Every row / step is
 held to 2x the max and the mean over rows to 2x the floor mean."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -341,6 +343,39 @@ def test_generic_gemm_direct_tiles_equal_staged_ones(M, N, K, pad, ws):
             ref = want + res.double() if resid else want
             lim = mass * 2.0 ** -24 * (32 + 8 + K // 128 + 16 + 4) + (2.0 ** -24 * ref.abs() if resid else 0.0)
             assert ((outs[0].double() - ref).abs() <= lim + 1e-30).all()
+
+
+@pytest.mark.parametrize("M", [9, 17, 40, 64, 80, 96, 100])
+@pytest.mark.parametrize("N,K,off", [(260, 3104, 0), (260, 3104, 1), (1200, 1028, 0), (130, 775, 1), (9, 40, 0)])
+def test_generic_gemm_fp32_sums_and_values_out_of_range(M, N, K, off):
+    """fp32 products as sums of bf16 ones, every height of a tile, all three kinds of loads. Rows of ordinary values are as near to float64 as fp32 sums
+    (the 2-norm of half an ulp for the result and one for the sums of a tile, of eight and of the rest); infinities, NaN, values that round to
+    infinity in bf16 and very small ones give what fp32 sums give: non-finite outputs where float64 has them, the bound of the tests above where no
+    partial sum can overflow."""
+    from lit_llama import _hip
+
+    g = torch.Generator("cuda").manual_seed(M + N + K)
+    x = torch.randn(M * K + 1, device="cuda", generator=g)[off:off + M * K].view(M, K)
+    w = torch.randn(N, K, device="cuda", generator=g)
+
+    def product():
+        y = torch.empty(M, N, device="cuda")
+        _hip.g_linear(1, x, M, K, w, None, None, 16, K, N, y, None, 1, _hip.stream())
+        return y.double()
+
+    want = x.double() @ w.double().T
+    assert ((product() - want).norm() / want.norm()).item() < 2.0 ** -24 * (0.5 + 3 * 0.5)
+    x[1, 5], x[2, 7], x[3, K - 1], w[7, 5], w[8, 3] = math.inf, -math.inf, math.nan, 0.0, math.inf
+    x[4] *= 1e37
+    x[5, ::2] = 3.4e38  # above bf16's largest
+    x[6] *= 1e-30
+    want, mass = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    got = product()
+    rows = [0, 1, 2, 3, 6, 7, 8]
+    assert torch.equal(torch.isnan(got[rows]), torch.isnan(want[rows])) and torch.equal(torch.isinf(got[rows]), torch.isinf(want[rows]))
+    safe = mass < 1e38
+    lim = mass * 2.0 ** -24 * (32 + 8 + K // 128 + 16 + 4)
+    assert safe[0, :7].all() and ((got - want).abs()[safe] <= lim[safe]).all()
 
 
 # ---- up to 8 rows (generic_rows.h)
