@@ -4,17 +4,17 @@
 // the device, host side); what is specific to GPTQ is the sequential column loop inside a
 // 128-column block (quantization.py:568-596) and the ColBlock packing (pack_weight, 374-388).
 //
-// llj_gptq_block(_bs): 16 or 4 lanes per weight row (rows are independent inside a block: the update of
-// row r uses only its own error and the shared Hinv1 rows). The block's 128 columns of each row
-// and Hinv1 sit in LDS (16 or 64 rows per workgroup: 10 / 40 + 66 KiB); 16 columns at a time are quantized
-// in registers, then the rest of the block takes their 16 updates per column in one LDS round
-// trip, the columns split over the row's lanes. Weights are passed
-// transposed (Wt: K x N, element (k, n) at k * N + n) so column i of 128 rows is one coalesced load.
+// llj_gptq_block(_bs): 16 lanes per weight row (rows are independent inside a block: the update of
+// row r uses only its own error and the shared Hinv1 rows). The block's 128 columns of each row are in its lanes'
+// registers, Hinv1 in LDS; 16 columns at a time are quantized one by one, then the rest of the block takes their 16 updates per
+// column. Weights are passed transposed (Wt: K x N, element (k, n) at k * N + n).
 // The block is the reference's `blocksize` (557; 16 / 32 / 64 / 128: whole 16-column register
 // groups, at most the 128 columns the LDS holds).
 // Every arithmetic step is the reference's fp32 op in the reference's order, rounded on its own
 // (this file is built with -ffp-contract=off, lit_llama/_build.py), so a block reproduces the torch CPU
 // loop bitwise given the same W1 and Hinv1.
+#include <utility>
+
 #include "common.h"
 
 namespace llj {
@@ -46,83 +46,122 @@ struct Errors {
   __device__ __forceinline__ bool fit() const { return hi < __float_as_uint(0x1p40f) && lo >= __float_as_uint(0x1p-60f) - 1u; }
 };
 
-// One block of one row's columns (see gptq_block_kernel). FAST: every divisor is in div_by's range; seen: the errors.
-template <int LANES, int kWs, bool FAST>
-__device__ __forceinline__ float gptq_columns(const float* hs, const float* rd, float* ws, int t, int l, int blk, float s, float z, float maxq,
-                                              bool writer, float* __restrict__ q_out, float* __restrict__ e_out, size_t N, Errors& seen) {
+// What a group of 16 columns needs of Hinv1: column l's values in lane l, the diagonal and its reciprocals in every lane
+struct Group {
+  float h[kGptqSub];
+  f32x4 d[kGptqSub / 4], rd[kGptqSub / 4];
+  __device__ __forceinline__ void load(const float* hs, const float (*diag)[kGptqBlock], int b, int l) {
+#pragma unroll
+    for (int u = 0; u < kGptqSub; ++u) h[u] = hs[(b + u) * kHs + b + l];
+#pragma unroll
+    for (int c = 0; c < kGptqSub / 4; ++c) {
+      d[c] = *reinterpret_cast<const f32x4*>(diag[0] + b + 4 * c);
+      rd[c] = *reinterpret_cast<const f32x4*>(diag[1] + b + 4 * c);
+    }
+  }
+};
+
+// A group's columns of a row, r: column l in lane l. Every lane of the row forms every column's code and error from the owner's weight.
+template <bool FAST>
+struct Columns {
+  const Group& grp;
+  const int l;
+  const float s, z, rs, maxq;
+  float r, lsum, q_own, e_own;
+  float e[kGptqSub];
+
+  template <int U>
+  __device__ __forceinline__ int column() {
+    const float w = __uint_as_float(dpp_u32<0x150 + U>(__float_as_uint(r)));  // lane U's, of the row's 16
+    const float d = grp.d[U / 4][U % 4];
+    // quantize_weight (quantization.py:470-473): clamp(round(x / scale) + zero, 0, maxq)
+    const float x = FAST ? div_by(w, s, rs) : __fdiv_rn(w, s);
+    const float qi = fminf(fmaxf(__fadd_rn(rintf(x), z), 0.f), maxq);
+    const float q = __fmul_rn(s, __fsub_rn(qi, z));
+    const float dq = __fsub_rn(w, q);
+    e[U] = FAST ? div_by(dq, d, grp.rd[U / 4][U % 4]) : __fdiv_rn(dq, d);  // err1 (592)
+    // W1[:, i:] -= err1 (x) Hinv1[i, i:] (593) inside the group (columns <= i are never read again)
+    r = __fsub_rn(r, __fmul_rn(e[U], grp.h[U]));
+    lsum = __fadd_rn(lsum, __fmul_rn(e[U], e[U]));  // Losses1 (590): (w - q)^2 / d^2
+    q_own = l == U ? q : q_own;
+    e_own = l == U ? e[U] : e_own;
+    return U;
+  }
+  template <int... U>
+  __device__ __forceinline__ void all(std::integer_sequence<int, U...>) {
+    int done[] = {column<U>()...};
+    (void)done;
+  }
+};
+
+// One block of one row's columns, column 16 i + l in r[i] of lane l (see gptq_block_kernel). FAST: every divisor is in div_by's range; seen: the
+// errors of the lane's columns.
+template <bool FAST>
+__device__ __forceinline__ float gptq_columns(const float* hs, const float (*diag)[kGptqBlock], float (&r)[kGptqBlock / kGptqSub], int l, int blk, float s,
+                                              float z, float maxq, bool live, float* __restrict__ q_out, float* __restrict__ e_out, size_t N, Errors& seen) {
   const float rs = __fdiv_rn(1.f, s);
   float lsum = 0.f;
+  Group grp;
+  grp.load(hs, diag, 0, l);
   for (int b = 0; b < blk; b += kGptqSub) {
-    float r[kGptqSub], e[kGptqSub];
+    Columns<FAST> c = {grp, l, s, z, rs, maxq, r[0], lsum, 0.f, 0.f};
+    c.all(std::make_integer_sequence<int, kGptqSub>());
+    lsum = c.lsum;
+    if constexpr (FAST) seen.add(c.e_own);
+    if (live) {
+      q_out[(size_t)(b + l) * N] = c.q_own;
+      e_out[(size_t)(b + l) * N] = c.e_own;
+    }
+    const float* h = hs + b * kHs + b + l;
+    if (b + kGptqSub < blk) grp.load(hs, diag, b + kGptqSub, l);
+    // the rest of the block: the group's updates of a column in increasing i, as the reference applies them one column i at a time
 #pragma unroll
-    for (int u = 0; u < kGptqSub; ++u) r[u] = ws[(b + u) * kWs + t];
+    for (int i = 1; i < kGptqBlock / kGptqSub; ++i) {
+      if (b + i * kGptqSub < blk) {
+        float hv[kGptqSub];
 #pragma unroll
-    for (int u = 0; u < kGptqSub; ++u) {
-      const float* h = hs + (b + u) * kHs + b;  // Hinv1[b + u][b ..]: the same address in every lane
-      const float w = r[u], d = h[u];
-      // quantize_weight (quantization.py:470-473): clamp(round(x / scale) + zero, 0, maxq)
-      const float x = FAST ? div_by(w, s, rs) : __fdiv_rn(w, s);
-      const float qi = fminf(fmaxf(__fadd_rn(rintf(x), z), 0.f), maxq);
-      const float q = __fmul_rn(s, __fsub_rn(qi, z));
-      const float dq = __fsub_rn(w, q);
-      e[u] = FAST ? div_by(dq, d, rd[b + u]) : __fdiv_rn(dq, d);  // err1 (592)
-      if constexpr (FAST) seen.add(e[u]);
-      lsum = __fadd_rn(lsum, __fmul_rn(e[u], e[u]));               // Losses1 (590): (w - q)^2 / d^2
-      if (writer) {
-        q_out[(size_t)(b + u) * N] = q;
-        e_out[(size_t)(b + u) * N] = e[u];
+        for (int u = 0; u < kGptqSub; ++u) hv[u] = h[u * kHs + i * kGptqSub];
+#pragma unroll
+        for (int u = 0; u < kGptqSub; ++u) r[i] = __fsub_rn(r[i], __fmul_rn(c.e[u], hv[u]));
       }
-      // W1[:, i:] -= err1 (x) Hinv1[i, i:] (593) inside the register group (columns <= i are
-      // never read again)
-#pragma unroll
-      for (int v = u + 1; v < kGptqSub; ++v) r[v] = __fsub_rn(r[v], __fmul_rn(e[u], h[v]));
+      r[i - 1] = r[i];
     }
-    __syncthreads();  // every lane has read the group's columns before any lane rewrites ws
-    // the rest of the block, column by column: the group's updates in increasing i, as the
-    // reference applies them one column i at a time
-    for (int j = b + kGptqSub + l; j < blk; j += LANES) {
-      float acc = ws[j * kWs + t];
-#pragma unroll
-      for (int u = 0; u < kGptqSub; ++u) acc = __fsub_rn(acc, __fmul_rn(e[u], hs[(b + u) * kHs + j]));
-      ws[j * kWs + t] = acc;
-    }
-    __syncthreads();  // the next group's columns are complete
   }
   return lsum;
 }
 
-// Each row's 16-column quantization group is computed redundantly by all LANES lanes of the
-// row (identical inputs, identical fp32 ops -> identical e[u]); the trailing update of the block's
-// remaining columns is split over the lanes (column j to lane (j - b - 16) % LANES). Every
-// column still receives the same updates in the same order, so results are unchanged bit for bit.
+// A row's 128 columns are in the registers of 16 lanes, four rows to a wave; a column's weight goes from its lane to the row's others
+// (DPP), which all form its code and error (identical inputs, identical fp32 ops) and then update their own columns. Every
+// column receives the updates in the reference's order, so results are its bit for bit.
 //
-// Bound: the chain of dependent instructions of a column, two divisions in it, times 128. 16 rows x 16 lanes put N = 4096 on
-// all 256 CUs (32 x 8: on half of them); above N = 8192 64 x 4 keep the workgroups of one round. kWs spreads a wavefront's
-// lanes x rows over the 64 banks (20 l + t, 80 l + t mod 64). us a block, before (32 x 8, three division sequences a column; 64 x 4
-// above 8192): N = 4096 52 and 35 (39 among the producer's other launches), 8192 54
-// and 37, 11008 63 and 55 (32 x 8 there: 79), 35008 196 and 173; of that 1 to 3 for the range of the errors (a block with one out of
-// range is done twice).
-template <int ROWS, int LANES, int kWs>
-__global__ __launch_bounds__(ROWS * LANES) void gptq_block_kernel(const float* __restrict__ hinv, int K, int i1,
-                                                                  int blk,
-                                                                  float* __restrict__ wt, int N,
-                                                                  const float* __restrict__ scale,
-                                                                  const float* __restrict__ zero, float maxq,
-                                                                  float* __restrict__ qt, float* __restrict__ err,
-                                                                  float* __restrict__ loss) {
-  __shared__ __align__(16) float hs[kGptqBlock * kHs];  // hs[i * kHs + j] = Hinv1[i][j]
-  __shared__ float ws[kGptqBlock * kWs];                // ws[j * kWs + t] = W1[row t][j]
-  __shared__ float rd[kGptqBlock];                      // 1 / Hinv1[i][i]
-  constexpr int NT = ROWS * LANES;
-  const int tid = threadIdx.x;
-  const int t = tid / LANES, l = tid % LANES;
+// Bound: the chain of dependent instructions of a column, two divisions in it, times 128. A lone wave on a SIMD issues one instruction every 7 to
+// 8 cycles whether it depends on the last or not, so their number counts: 570 a group of 16 columns (890 with a row's 16 columns in every
+// lane's registers: 23.6 us at N = 4096; interleaving those updates with the chain, or Hinv1's values a step ahead: no faster). 16 rows put
+// N = 4096 on all 256 CUs, one wave per SIMD; above, more rows to a workgroup share Hinv1. us a block with the rows in LDS, Hinv1 waited for
+// column by column, and now: N = 256 33 and 17, 4096 35 and 19, 8192 38 and 21, 11008 54 and 31, 35008 171 and 88 (a block with an error out
+// of div_by's range is done twice).
+template <int ROWS>
+__global__ __launch_bounds__(ROWS * 16) void gptq_block_kernel(const float* __restrict__ hinv, int K, int i1, int blk, float* __restrict__ wt, int N,
+                                                               const float* __restrict__ scale, const float* __restrict__ zero, float maxq,
+                                                               float* __restrict__ qt, float* __restrict__ err, float* __restrict__ loss) {
+  __shared__ __align__(16) float hs[kGptqBlock * kHs];    // hs[i * kHs + j] = Hinv1[i][j]
+  __shared__ __align__(16) float diag[2][kGptqBlock];     // Hinv1[i][i], 1 / Hinv1[i][i]
+  constexpr int NT = ROWS * 16;
+  const int tid = threadIdx.x, t = tid >> 4, l = tid & 15;
   const int n = blockIdx.x * ROWS + t;
   const int nn = n < N ? n : N - 1;  // clamped: loads stay in bounds, stores are guarded
+  float r[kGptqBlock / kGptqSub];
+  auto stage = [&] {
+#pragma unroll
+    for (int i = 0; i < kGptqBlock / kGptqSub; ++i) r[i] = i * kGptqSub < blk ? wt[(size_t)(i1 + i * kGptqSub + l) * N + nn] : 0.f;
+  };
+  stage();
   const float s = scale[nn], z = zero[nn];
   bool fast = divides(s) && fabsf(z) < 0x1p30f;
   if (tid < blk) {
     const float d = hinv[(size_t)(i1 + tid) * K + i1 + tid];
-    rd[tid] = __fdiv_rn(1.f, d);
+    diag[0][tid] = d;
+    diag[1][tid] = __fdiv_rn(1.f, d);
     fast = fast && divides(d);
   }
   if (((K | i1) & 3) == 0 && ((uintptr_t)hinv & 15) == 0) {
@@ -133,27 +172,19 @@ __global__ __launch_bounds__(ROWS * LANES) void gptq_block_kernel(const float* _
   } else {
     for (int v = tid; v < blk * blk; v += NT) hs[v / blk * kHs + v % blk] = hinv[(size_t)(i1 + v / blk) * K + i1 + v % blk];
   }
-  auto stage = [&] {  // a wavefront reads runs of ROWS neighbouring rows of the matrix
-    for (int v = tid; v < blk * ROWS; v += NT) {
-      const int j = v / ROWS, m = min((int)blockIdx.x * ROWS + v % ROWS, N - 1);
-      ws[j * kWs + v % ROWS] = wt[(size_t)(i1 + j) * N + m];
-    }
-  };
-  stage();
   bool done = __syncthreads_and(fast);
-  const bool writer = l == 0 && n < N;
+  const bool live = n < N;
   float* q_out = qt + (size_t)i1 * N + nn;
   float* e_out = err + nn;
   float sum = 0.f;
   Errors seen;
   if (done) {
-    sum = gptq_columns<LANES, kWs, true>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N, seen);
+    sum = gptq_columns<true>(hs, diag, r, l, blk, s, z, maxq, live, q_out, e_out, N, seen);
     done = __syncthreads_and(seen.fit());
     if (!done) stage();  // a quotient out of div_by's range: the block again
-    __syncthreads();
   }
-  if (!done) sum = gptq_columns<LANES, kWs, false>(hs, rd, ws, t, l, blk, s, z, maxq, writer, q_out, e_out, N, seen);
-  if (writer) loss[n] += sum;
+  if (!done) sum = gptq_columns<false>(hs, diag, r, l, blk, s, z, maxq, live, q_out, e_out, N, seen);
+  if (live && l == 0) loss[n] += sum;
 }
 
 // pack_weight (quantization.py:374-388) of reconstructed weights Qt (K x N, fp32):
@@ -230,12 +261,13 @@ int llj_gptq_block_bs(const float* hinv, int K, int i1, int blocksize, float* wt
   LLJ_REQUIRE(bits == 2 || bits == 4 || bits == 8);
   LLJ_REQUIRE(hinv && wt && scale && zero && qt && err && loss);
   const float maxq = (float)((1 << bits) - 1);
-  if (N > 8192)
-    hipLaunchKernelGGL((gptq_block_kernel<64, 4, 80>), dim3((N + 63) / 64), dim3(256), 0, (hipStream_t)stream, hinv,
-                       K, i1, blocksize, wt, N, scale, zero, maxq, qt, err, loss);
-  else
-    hipLaunchKernelGGL((gptq_block_kernel<16, 16, 20>), dim3((N + 15) / 16), dim3(256), 0, (hipStream_t)stream, hinv,
-                       K, i1, blocksize, wt, N, scale, zero, maxq, qt, err, loss);
+#define LLJ_BLOCK(ROWS)                                                                                                                \
+  hipLaunchKernelGGL((gptq_block_kernel<ROWS>), dim3((N + ROWS - 1) / ROWS), dim3(ROWS * 16), 0, (hipStream_t)stream, hinv, K, i1,    \
+                     blocksize, wt, N, scale, zero, maxq, qt, err, loss)
+  if (N <= 4096) LLJ_BLOCK(16);
+  else if (N <= 8192) LLJ_BLOCK(32);
+  else LLJ_BLOCK(64);
+#undef LLJ_BLOCK
   LLJ_CHECK_LAUNCH();
   return 0;
 }

@@ -154,6 +154,35 @@ def test_gptq_block_kernel_wide_bitwise(hip, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bs", [16, 128])
+@pytest.mark.parametrize("N", [1, 17, 4099, 8191, 8200])
+def test_gptq_block_kernel_rows_per_workgroup(hip, N, bs):
+    """16, 32 and 64 rows to a workgroup with a partial last one: each row as by itself in a product of 16 rows (which the tests above hold to
+    the oracle), the last block of the matrix, nothing outside it."""
+    from lit_llama import _hip
+    rng = np.random.default_rng(N)
+    K, n0 = 256, 16
+    W = torch.from_numpy(rng.standard_normal((K, n0)).astype(np.float32)).to(dev)
+    Hinv = np.triu(rng.standard_normal((K, K)) * 0.02).astype(np.float32)
+    Hinv[np.arange(K), np.arange(K)] = rng.uniform(0.1, 3, K)
+    hd = torch.from_numpy(Hinv).to(dev)
+    s, z = (torch.from_numpy(rng.uniform(a, b, n0).astype(np.float32).round(c)).to(dev) for a, b, c in ((0.05, 0.4, 7), (4, 12, 0)))
+
+    def run(idx):
+        n = len(idx)
+        w, sc, zr = W[:, idx].contiguous(), s[idx].contiguous(), z[idx].contiguous()
+        q, e, loss = torch.full((K, n), 7.0, device=dev), torch.empty(bs, n, device=dev), torch.zeros(n, device=dev)
+        _hip.call("llj_gptq_block_bs", hd.data_ptr(), K, K - bs, bs, w.data_ptr(), n, sc.data_ptr(), zr.data_ptr(), 4, q.data_ptr(), e.data_ptr(),
+                  loss.data_ptr(), _st())
+        assert bool((q[:K - bs] == 7).all())
+        return q, e, loss
+
+    idx = torch.arange(N, device=dev) % n0
+    for a, b in zip(run(idx), run(torch.arange(n0, device=dev))):
+        assert torch.equal(a, b[..., idx])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bits", [4, 8])
 def test_colblock_pack_kernel_bitwise(hip, bits):
     from lit_llama import _hip
