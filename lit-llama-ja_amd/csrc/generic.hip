@@ -123,10 +123,11 @@ __global__ __launch_bounds__(64) void g_rope_kv_kernel(const TT* __restrict__ qk
     const float c = rope[((size_t)p * (hs / 2) + i) * 2], s = rope[((size_t)p * (hs / 2) + i) * 2 + 1];
     const float q0 = ldv(row, 2 * i), q1 = ldv(row, 2 * i + 1);
     const float k0 = ldv(row, C + 2 * i), k1 = ldv(row, C + 2 * i + 1);
-    stv(q_out, (size_t)m * C + h * hs + 2 * i, q0 * c - q1 * s);
-    stv(q_out, (size_t)m * C + h * hs + 2 * i + 1, q1 * c + q0 * s);
-    stv(kc, cbase + 2 * i, k0 * c - k1 * s);
-    stv(kc, cbase + 2 * i + 1, k1 * c + k0 * s);
+    const float2 q = gr_rotate(q0, q1, c, s), k = gr_rotate(k0, k1, c, s);
+    stv(q_out, (size_t)m * C + h * hs + 2 * i, q.x);
+    stv(q_out, (size_t)m * C + h * hs + 2 * i + 1, q.y);
+    stv(kc, cbase + 2 * i, k.x);
+    stv(kc, cbase + 2 * i + 1, k.y);
     vc[cbase + 2 * i] = row[2 * C + 2 * i];
     vc[cbase + 2 * i + 1] = row[2 * C + 2 * i + 1];
   }
@@ -392,22 +393,27 @@ int llj_g_rope_attention(const void* qkv, void* kcache, void* vcache, const floa
               llj_g_rope_attention_ok(S, C / n_head) && ((uintptr_t)kcache | (uintptr_t)vcache) % (dt ? 8 : 4) == 0);
   const size_t lds = gr_attention_lds(S, C / n_head);
   hipStream_t s = (hipStream_t)stream;
-  // fp32 with more than a workgroup per CU: masked loads (12 rows of 32 heads, us without and with: heads of 80, 16 slots 7.3 and 7.0,
-  // 1,700 keys 84.6 and 80.9; of 128 7.8 and 7.2, 131 and 131; 8 rows, one workgroup a CU: 80, 500 keys 17.8 and 18.7; bf16 is 3 to 20 %
-  // faster without at either)
+  // fp32 with more than a workgroup per CU: nothing is loaded that is not seen (12 rows of 32 heads, us without and with: heads of 80, 16 slots 8.9 and 7.2,
+  // of 128 21.5 and 18.9). Heads of more than 64 there, and of more than 128, stay on the kernel with its scores in LDS, which has the registers for
+  // more waves (12 rows of 32 heads of 80, 1,700 keys 88 and 81, 26 rows of 10 heads of 78 12.8 and 11.3; bf16 is ahead in registers at every size)
   const bool mask = dt == 1 && (long)B * n_head > 256;
-  // bf16 heads of 65 to 96 take four pairs a lane: with three the compiler puts the loads of the new token's row one behind the other's
-  // wait (in a decode step of 10 heads of 78 7.7 us and 6.7)
 #define LLJ_GRA(T, NQ, MASK) \
-  hipLaunchKernelGGL((g_rope_attention_kernel<T, NQ, MASK>), dim3(B, n_head), dim3(kGrThreads), lds, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
+  hipLaunchKernelGGL((g_rope_attention16_kernel<T, NQ, 4, MASK>), dim3(B, n_head), dim3(kGrThreads), 0, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
 #define LLJ_GRA_NQ(NQ)                        \
   do {                                        \
-    if (dt == 0) LLJ_GRA(bf16_t, (NQ == 3 ? 4 : NQ), false);  \
-    else if (mask) LLJ_GRA(float, NQ, true);  \
+    if (dt == 0) LLJ_GRA(bf16_t, NQ, false);  \
+    else if (mask) LLJ_GRA(float, (NQ > 2 ? 2 : NQ), true);  \
     else LLJ_GRA(float, NQ, false);           \
   } while (0)
   const int hs = C / n_head;
-  if (hs <= 32) LLJ_GRA_NQ(1);
+  if (hs > (mask ? 64 : 128)) {
+#define LLJ_GRS(T, MASK) \
+  hipLaunchKernelGGL((g_rope_attention_kernel<T, 4, MASK>), dim3(B, n_head), dim3(kGrThreads), lds, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
+    if (dt == 0) LLJ_GRS(bf16_t, false);
+    else if (mask) LLJ_GRS(float, true);
+    else LLJ_GRS(float, false);
+#undef LLJ_GRS
+  } else if (hs <= 32) LLJ_GRA_NQ(1);
   else if (hs <= 64) LLJ_GRA_NQ(2);
   else if (hs <= 96) LLJ_GRA_NQ(3);
   else LLJ_GRA_NQ(4);

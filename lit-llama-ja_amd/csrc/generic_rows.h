@@ -12,6 +12,8 @@
 // 35.1 -> 29.4; fp32, K = 512: the same to 0.2 less, lm_head 15.2 -> 12.6; bf16, K = 2,100: 12.2 -> 11.2, 16.4 -> 14.3. Two
 // sets of 4 pieces by turns instead: 4.1, 2.7, 4.8, 3.5, 11.2.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 #include "elem.h"
 
@@ -178,10 +180,13 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
 // One token per sequence: rotary positions of q and k (g_rope_kv_kernel), k and v into cache slot p % S, and causal attention over
 // the cache (g_attention_kernel). Block (row, head) of 512 threads -- a few tens of blocks with a chain of memory trips each: 16
 // lanes per key and 128 keys at a time, then the values with the threads split over dimension pairs and up to kGrKeyGroups
-// interleaved groups of keys. The first keys and values are loaded before the rotation, without a branch around any of them but in MASK (10 heads
-// of 78, bf16, us behind branches -> this: 40 keys 6.4 -> 5.8, 110 keys 7.0 -> 6.1, 500 keys 16.7 -> 14.8; the next 128 keys
-// requested a pass ahead as well: 6.2, 6.5, 14.6; fp32, 12 rows of 32 heads of 16, 1,700 keys, with 4 loads a key whatever the head 43.8,
-// with NQ 29.6). LDS: S + hs (3 + groups) floats.
+// interleaved groups of keys. The first keys and values are loaded before the rotation, without a branch around any of them but in MASK. For heads
+// of more than 128 (fp32 with many workgroups: 64); the others below. LDS: S + hs (3 + groups) floats.
+// A pair in rotary position (c, s), rounded the same in every kernel that forms it
+__device__ __forceinline__ float2 gr_rotate(float x0, float x1, float c, float s) {
+  const float a = x1 * s, b = x1 * c;
+  return make_float2(__builtin_fmaf(x0, c, -a), __builtin_fmaf(x0, s, b));
+}
 constexpr int kGrThreads = 512, kGrKeyGroups = 14;
 __host__ __device__ inline int gr_groups(int P) { return P > kGrThreads ? 1 : P * kGrKeyGroups > kGrThreads ? kGrThreads / P : kGrKeyGroups; }
 // NQ: pairs of a key's 16 lanes each, ceil(hs / 32) to 4 (bf16: 4 for 3). MASK: only what is seen is loaded, behind branches.
@@ -230,9 +235,10 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
   for (int i = tid; i < P; i += kGrThreads) {
     const float c = rope[((size_t)p * P + i) * 2], s = rope[((size_t)p * P + i) * 2 + 1];
     const float q0 = ldv(row, 2 * i), q1 = ldv(row, 2 * i + 1), k0 = ldv(row, C + 2 * i), k1 = ldv(row, C + 2 * i + 1);
-    sq[2 * i] = rnd<T>(q0 * c - q1 * s) * scale;
-    sq[2 * i + 1] = rnd<T>(q1 * c + q0 * s) * scale;
-    const float r0 = rnd<T>(k0 * c - k1 * s), r1 = rnd<T>(k1 * c + k0 * s);
+    const float2 q = gr_rotate(q0, q1, c, s), k = gr_rotate(k0, k1, c, s);
+    sq[2 * i] = rnd<T>(q.x) * scale;
+    sq[2 * i + 1] = rnd<T>(q.y) * scale;
+    const float r0 = rnd<T>(k.x), r1 = rnd<T>(k.y);
     sk[2 * i] = r0;
     sk[2 * i + 1] = r1;
     sv[2 * i] = ldv(row, 2 * C + 2 * i);
@@ -312,6 +318,163 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
     float o = 0.f;
     for (int k = 0; k < G; ++k) o += so[k * hs + d];
     stv(y, (size_t)m * C + h * hs + d, o * inv);
+  }
+}
+
+
+// The same for heads of up to 128, in registers: lane l of 16 holds pairs l, l + 16 .. of the query, of its keys and of the outputs, so the rotation needs
+// no LDS, keys and values pass once (running maximum and sum per 16 lanes, key group + 32 i) and the workgroup meets once, at the end.
+// A chain of three memory trips: the first 128 keys and values with the position (not in MASK), then its rotary pairs, then (from 128 keys on) the next
+// keys, a pass ahead.
+// us with the scores in LDS (the kernel above) and so, bf16: 10 heads of 78, 40 keys 5.4 and 3.9, 110 keys 5.7 and 4.0, 500 keys 18.7 and 7.0; 8 rows
+// of 32 heads of 80, 500 keys 28.4 and 11.9; fp32: 10 heads of 78, 110 keys 5.7 and 5.1, 500 keys 12.9 and 9.5. 10 workgroups: bound by the
+// chain, not by the 16 KB a head.
+template <typename T, int NQ, int U, bool MASK>
+__global__ __launch_bounds__(kGrThreads) void g_rope_attention16_kernel(const T* __restrict__ qkv, T* __restrict__ kc, T* __restrict__ vc,
+                                                                 const float* __restrict__ rope, const int* __restrict__ pos,
+                                                                 T* __restrict__ y, int C, int nh, int S) {
+  constexpr int kWaves = kGrThreads / 64, kGroups = kGrThreads / 16, kMost = 32 * NQ;
+  __shared__ float so[kWaves][kMost], sm[kWaves], sl[kWaves];
+  typedef T pair __attribute__((ext_vector_type(2)));
+  typedef pair __attribute__((aligned(sizeof(T)))) any_pair;
+  const int m = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, sub = tid & 15, kg = tid >> 4;
+  const int hs = C / nh, P = hs / 2;
+  const size_t cb = ((size_t)m * nh + h) * S * hs;
+  const T* row = qkv + (size_t)m * 3 * C + h * hs;
+  int at[NQ];  // this lane's pairs (past the last: a valid one, not used)
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) at[q] = min(16 * q + sub, P - 1);
+  constexpr int kBufs = MASK ? 1 : 2;  // (many workgroups: two to a CU instead of a pass ahead)
+  pair kw[kBufs][U][NQ], vw[kBufs][U][NQ];
+  auto load = [&](int b, int j0, int lim) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t r = cb + (size_t)min(j0 + kGroups * u, lim - 1) * hs;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        kw[b][u][q] = reinterpret_cast<const pair*>(kc + r)[at[q]];
+        vw[b][u][q] = reinterpret_cast<const pair*>(vc + r)[at[q]];
+      }
+    }
+  };
+  pair qw[NQ], nk[NQ], nv[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    qw[q] = *reinterpret_cast<const any_pair*>(row + 2 * at[q]);
+    nk[q] = *reinterpret_cast<const any_pair*>(row + C + 2 * at[q]);
+    nv[q] = *reinterpret_cast<const any_pair*>(row + 2 * C + 2 * at[q]);
+  }
+  if constexpr (!MASK) load(0, kg, S);
+  const int p = pos[0], slot = p % S, nvis = p < S ? p + 1 : S;
+  typedef float any_rope __attribute__((ext_vector_type(2), aligned(4)));
+  any_rope cs[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) cs[q] = *reinterpret_cast<const any_rope*>(rope + ((size_t)p * P + at[q]) * 2);
+  if constexpr (MASK) load(0, kg, nvis);
+  const float scale = 1.f / sqrtf((float)hs);
+  float q0[NQ], q1[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    T a0 = qw[q][0], a1 = qw[q][1], b0 = nk[q][0], b1 = nk[q][1];
+    const float c = cs[q].x, s = cs[q].y, x0 = ldv(&a0, 0), x1 = ldv(&a1, 0), k0 = ldv(&b0, 0), k1 = ldv(&b1, 0);
+    const bool mine = 16 * q + sub < P;
+    const float2 rq = gr_rotate(x0, x1, c, s), rk = gr_rotate(k0, k1, c, s);
+    q0[q] = mine ? rnd<T>(rq.x) * scale : 0.f;
+    q1[q] = mine ? rnd<T>(rq.y) * scale : 0.f;
+    stv(&b0, 0, rk.x);
+    stv(&b1, 0, rk.y);
+    nk[q] = pair{b0, b1};
+    if (kg == 0 && mine) {
+      reinterpret_cast<pair*>(kc + cb + (size_t)slot * hs)[at[q]] = nk[q];
+      reinterpret_cast<pair*>(vc + cb + (size_t)slot * hs)[at[q]] = nv[q];
+    }
+  }
+  float mx = -INFINITY, l = 0.f, o[2 * NQ] = {};
+  auto pass = [&](int b, int base) {  // keys base + group + 32 u
+    if constexpr (MASK) {
+      if (base) load(0, base + kg, nvis);
+    } else if (base + kGroups * U < nvis) {
+      load(b ^ 1, base + kGroups * U + kg, nvis);
+    }
+    float s[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = base + kg + kGroups * u;
+      s[u] = 0.f;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        if (j == slot) kw[b][u][q] = nk[q], vw[b][u][q] = nv[q];
+        T k0 = kw[b][u][q][0], k1 = kw[b][u][q][1];
+        float v0 = ldv(&k0, 0), v1 = ldv(&k1, 0);
+        if (q == NQ - 1) {  // (a pair of another lane: no part of this one's sum, whatever it holds)
+          v0 = 16 * q + sub < P ? v0 : 0.f;
+          v1 = 16 * q + sub < P ? v1 : 0.f;
+        }
+        s[u] += q0[q] * v0 + q1[q] * v1;
+      }
+      s[u] = row16_sum(s[u]);
+      s[u] = j < nvis ? s[u] : -INFINITY;
+    }
+    float mn = mx;
+#pragma unroll
+    for (int u = 0; u < U; ++u) mn = fmaxf(mn, s[u]);
+    const float ref = mn == -INFINITY ? 0.f : mn, corr = __expf(mx - ref);  // (nothing seen yet: weights of zero)
+    mx = mn;
+    l *= corr;
+#pragma unroll
+    for (int i = 0; i < 2 * NQ; ++i) o[i] *= corr;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (base + kg + kGroups * u >= nvis) continue;
+      const float w = __expf(s[u] - ref);
+      l += w;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        T v0 = vw[b][u][q][0], v1 = vw[b][u][q][1];
+        o[2 * q] += w * ldv(&v0, 0);
+        o[2 * q + 1] += w * ldv(&v1, 0);
+      }
+    }
+  };
+  for (int base = 0; base < nvis; base += 2 * kGroups * U) {
+    pass(0, base);
+    if (base + kGroups * U < nvis) pass(kBufs - 1, base + kGroups * U);
+  }
+  auto merge = [&](auto wide) {  // two groups of 16 lanes, in every lane of both
+    constexpr bool W = decltype(wide)::value;
+    float mlo, mhi, llo, lhi;
+    lane_halves<W>(mx, mlo, mhi);
+    lane_halves<W>(l, llo, lhi);
+    const float M = fmaxf(mlo, mhi), flo = mlo == -INFINITY ? 0.f : __expf(mlo - M), fhi = mhi == -INFINITY ? 0.f : __expf(mhi - M);
+    mx = M;
+    l = llo * flo + lhi * fhi;
+#pragma unroll
+    for (int i = 0; i < 2 * NQ; ++i) {
+      float lo, hi;
+      lane_halves<W>(o[i], lo, hi);
+      o[i] = lo * flo + hi * fhi;
+    }
+  };
+  merge(std::false_type());
+  merge(std::true_type());
+  const int wave = tid >> 6;
+  if ((tid & 63) < 16) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) *reinterpret_cast<float2*>(&so[wave][2 * (16 * q + sub)]) = make_float2(o[2 * q], o[2 * q + 1]);
+    if (sub == 0) sm[wave] = mx, sl[wave] = l;
+  }
+  __syncthreads();
+  if (tid < hs) {
+    float M = sm[0], L = 0.f, O = 0.f;
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) M = fmaxf(M, sm[w]);
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const float f = sm[w] == -INFINITY ? 0.f : __expf(sm[w] - M);
+      L += sl[w] * f;
+      O += so[w][tid] * f;
+    }
+    stv(y, (size_t)m * C + h * hs + tid, O / L);
   }
 }
 

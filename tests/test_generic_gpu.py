@@ -459,6 +459,32 @@ def test_generic_rope_attention_vs_separate_calls(dt, B, nh, hs, S, p):
     assert ((y.double() - want).abs() <= mass * loss + (0.0 if dt else 2.0 ** -8 * 1.01) * want.abs() + 1e-30).all()
 
 
+@pytest.mark.parametrize("dt", [0, 1])
+@pytest.mark.parametrize("B,nh,hs,S,p", [(1, 2, 78, 300, 100), (2, 3, 30, 400, 255), (1, 2, 126, 400, 256), (33, 8, 50, 200, 5), (1, 2, 66, 140, 500)])
+def test_generic_rope_attention_unseen_slots(dt, B, nh, hs, S, p):
+    """Slots that hold nothing yet (NaN) and the slot that the token takes (NaN before it) are no part of the result:
+    the same bits as over a cache of zeros there; one pass of 128 keys, several, the last one partial, a ring that has gone round."""
+    from lit_llama import _hip
+
+    g = torch.Generator("cuda").manual_seed(p)
+    dtype, C = torch.float32 if dt else torch.bfloat16, nh * hs
+    qkv = torch.randn(B, 3 * C, device="cuda", generator=g).to(dtype)
+    ang = torch.rand(p + 1, hs // 2, device="cuda", generator=g)
+    rope, pos = torch.stack([ang.cos(), ang.sin()], -1).contiguous(), torch.tensor([p], dtype=torch.int32, device="cuda")
+    kv = [torch.randn(B, nh, S, hs, device="cuda", generator=g).to(dtype) for _ in range(2)]
+    outs = []
+    for fill in (float("nan"), 0.0):
+        k, v = (t.clone() for t in kv)
+        for t in (k, v):
+            t[:, :, p + 1:] = fill
+            t[:, :, p % S] = fill
+        y = torch.empty(B, C, dtype=dtype, device="cuda")
+        _hip.call("llj_g_rope_attention", qkv.data_ptr(), k.data_ptr(), v.data_ptr(), rope.data_ptr(), pos.data_ptr(), y.data_ptr(), B, C, nh, S, dt,
+                  _hip.stream())
+        outs.append(y)
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,T,nh,hs,S,p0", [(1, 301, 32, 128, 301, 0), (2, 67, 10, 78, 80, 5), (1, 130, 8, 1, 130, 0), (3, 49, 8, 13, 64, 40),
