@@ -141,6 +141,13 @@ GEMM_MIN_ROWS = 32
 _GEMM_FMTS = (0, 1, 2, 3, 4)  # weight formats (low byte of wfmt; 4 = grouped int4) the prefill GEMMs take
 
 
+def _gemm_rows(fmts) -> int:
+    """GEMM_MIN_ROWS, or past its half where every format is bf16 or LLM.int8, whose slices past the second cost more than the tiles
+    (ms of a prompt, slices and GEMMs: 7B bf16 16 rows 7.0 and 7.5, 17 rows 9.8 and 7.6, 31 rows 12.6 and 7.7; LLM.int8 16 rows 7.0 and 7.0, 17 rows
+    8.9 and 7.1, 31 rows 13.3 and 8.7; 49M 16 rows 0.99 and 1.11, 24 rows 1.22 and 1.13; codes 24 rows 4.2 and 5.5, 31 rows 5.0 and 5.6)."""
+    return GEMM_MIN_ROWS // 2 + 1 if all((f & 0xFF) in (1, 2) for f in fmts) else GEMM_MIN_ROWS
+
+
 def _gemm_fmt(wfmt: int) -> bool:
     return (wfmt & 0xFF) in _GEMM_FMTS
 
@@ -551,7 +558,7 @@ class LLaMA(nn.Module):
         cfg = self.config
         C, H = cfg.n_embd, MLP.hidden(cfg)
         fmts = {s[0] for layer in specs["layers"] for s in layer}
-        return (M >= GEMM_MIN_ROWS and all(_gemm_fmt(f) for f in fmts) and C % 128 == 0 and H % 128 == 0
+        return (M >= _gemm_rows(fmts) and all(_gemm_fmt(f) for f in fmts) and C % 128 == 0 and H % 128 == 0
                 and _gemm_fmt(specs["head"][0]))
 
     def _blocks_gemm(self, w, specs, kv, pos, B, T, S, st):
@@ -819,14 +826,14 @@ class LLaMA(nn.Module):
         if f == 2:
             xn = torch.empty_like(x)
             self._i8_norm_prep(x, ln, xn, M, C, w, st)
-            if M >= GEMM_MIN_ROWS and C % 128 == 0 and V % 128 == 0:  # many rows: the int8 GEMM
+            if M >= _gemm_rows((f,)) and C % 128 == 0 and V % 128 == 0:  # many rows: the int8 GEMM
                 ao, (wg,), kp = self._i8_gathered(xn, M, C, [(W, sz, V)], w, st)
                 sc = _GemmScratch(specs, M, C, 0, x.device, head=V)
                 _hip.call("llj_gemm_i8_linear_ws", xn.data_ptr(), C, W.data_ptr(), _hip.ptr(sz), _hip.ptr(w.i8ws),
                           _hip.ptr(ao), _hip.ptr(wg), kp, out.data_ptr(), out.stride(0), M, V, C, sc.ptr, sc.nb, st)
                 return
             src, nw = xn, None
-        elif M >= GEMM_MIN_ROWS and _gemm_fmt(f) and C % 128 == 0 and V % 128 == 0:  # many rows: GEMM
+        elif M >= _gemm_rows((f,)) and _gemm_fmt(f) and C % 128 == 0 and V % 128 == 0:  # many rows: GEMM
             xn = torch.empty_like(x)
             _hip.call("llj_rmsnorm_rows", x.data_ptr(), ln.scale.data_ptr(), ln.eps, xn.data_ptr(), None, M, C, st)
             sc = _GemmScratch(specs, M, C, 0, x.device, head=V)

@@ -576,6 +576,36 @@ def test_generate_main_end_to_end(tmp_path, capsys):
     assert err.count("tokens/sec") == 2 and "Time to load model" in err and "Memory used" in err
 
 
+@pytest.mark.parametrize("mode,rows,takes", [(None, 16, False), (None, 17, True), (None, 31, True), ("llm.int8", 16, False), ("llm.int8", 17, True),
+                                             ("llm.int8", 31, True), ("gptq.int4", 31, False), ("gptq.int4", 32, True)])
+def test_rows_from_which_prompts_take_the_gemms(mode, rows, takes):
+    """model._gemm_rows: the logits of the row slices within two bf16 paths' noise on either side of the line (LLM.int8: one flipped rounding of
+    an activation is a whole int8 step)."""
+    from lit_llama import model as MD
+
+    m = _random_int4_model(1024, 8, mode=None if mode == "llm.int8" else mode, seed=96)
+    if mode == "llm.int8":
+        from lit_llama import LLaMA
+        from lit_llama.utils import EmptyInitOnDevice
+
+        with EmptyInitOnDevice(device=torch.device("cuda"), dtype=torch.bfloat16, quantization_mode=mode):
+            q = LLaMA(m.config)
+        q.load_state_dict(m.state_dict())
+        m = q.eval()
+    prompt = torch.randint(3, 2048, (1, rows), generator=torch.Generator().manual_seed(4)).cuda()
+    assert m._gemm_ok(m._layer_specs(), rows) == takes
+    outs, saved = [], MD.GEMM_MIN_ROWS
+    try:
+        for thr in (10 ** 9, saved):
+            MD.GEMM_MIN_ROWS = thr
+            m.reset_cache()
+            outs.append(m(prompt).float())
+    finally:
+        MD.GEMM_MIN_ROWS = saved
+    rel = ((outs[0] - outs[1]).norm() / outs[0].norm()).item()
+    assert rel < (3e-2 if mode == "llm.int8" else 2e-2), rel
+
+
 @pytest.mark.parametrize("mode", ["gptq.int4", "gptq.int8", None])
 def test_prefill_gemm_path_equals_gemv_path(mode):
     """A 96-token prompt through the prefill GEMMs (model.GEMM_MIN_ROWS) gives the logits of the
