@@ -22,13 +22,15 @@
 // tile is staged:
 //   y[m,n] = s[n] * (sum_k A[m,k] (128 + q[k,n]) - (128 + z[n]) * sum_k A[m,k]).
 // gptq.int8 (W8P: per 16 columns x 128 k the W4P tile of the low nibbles, then that of the high
-// nibbles) stages both planes' halves (8 KiB per chunk) and feeds both to the same accumulator,
-// the high plane dequantized to bf16 2048 + 16 hi (exponent 0x45): the epilogue is the int4 one
-// with the offset 2176 + zero (llj_w8_scale_zero).
-// Grouped int4 (ColBlock tile_cols = g, g % 128 == 0) stages the W4P tiles like int4 and
-// dequantizes each B fragment to bf16((q - z_g) * s_g) with its chunk's group pair -- exactly the
-// weights of the reference's grouped forward, F.linear over get_weight(bf16)
-// (quantization.py:390-421) -- so its epilogue takes the accumulator as is.
+// nibbles): a thread joins the nibbles of 32 k of one column to bytes and writes them to the chunk's
+// bf16 B tile (0 .. 255 are exact), laid out as bf16 weights' is: one conversion per workgroup and
+// one product per fragment (two products of 128 + lo and 2048 + 16 hi, put together by each wave:
+// 128 / 1000 rows 4096 -> 12288 46 / 205 us, 37 / 157 so); the epilogue is the int4 one with the
+// offset zero (llj_w8_scale_zero's pair less its 2176).
+// Grouped int4 (ColBlock tile_cols = g, g % 128 == 0) is converted in the same place, to
+// bf16((q - z_g) * s_g) with its chunk's group pair -- exactly the weights of the reference's grouped
+// forward, F.linear over get_weight(bf16) (quantization.py:390-421) -- so its epilogue takes the
+// accumulator as is (128 / 1000 rows 4096 -> 12288 41 / 181 us converted by each wave, 36 / 142 so).
 // LLM.int8() (Linear8bitLt, reference quantization.py:36-75 over bitsandbytes' MatMul8bitLt):
 // the activation quantized once by llj_i8_stats (aq rows, outlier columns 0, SCA per row) and CB
 // in the I8P tiling (per 16 columns x 128 k: 2 KiB = the two 64-deep MFMA steps, a lane's 16 B
@@ -244,6 +246,9 @@ constexpr int kGBM = 128, kGBN = 128, kGBK = 64, kGNT = 256;
 #ifndef LLJ_GDEPTH_W4_256
 #define LLJ_GDEPTH_W4_256 LLJ_GDEPTH  // int4 256-row tiles (188 VGPRs at 2 chunks in flight)
 #endif
+#ifndef LLJ_GDEPTH_ONCE
+#define LLJ_GDEPTH_ONCE 3  // codes converted as they are staged (gptq.int8 11008 -> 4096, 256 rows: 2 / 3 / 4 chunks 183 / 148 / 149 us)
+#endif
 #ifndef LLJ_GDEPTH_DENSE
 #define LLJ_GDEPTH_DENSE 1  // bf16 / int8 in 128-row tiles (32 VGPRs of A + B per chunk in flight)
 #endif
@@ -254,10 +259,9 @@ constexpr int kAP = kGBK + 8;  // A / bf16-B LDS row pitch (elements): 144 B
 
 template <int WF>
 constexpr size_t gemm_b_bytes() {
-  return (WF == GWF_W4 || WF == GWF_W4G) ? (size_t)kGBN * kGBK / 2
-         : WF == GWF_W8                  ? (size_t)kGBN * kGBK
-         : WF == GWF_I8                  ? (size_t)kGBN * 128  // 8 I8P tile blocks of 2 KiB
-                                         : (size_t)kGBN * kAP * 2;
+  return WF == GWF_W4   ? (size_t)kGBN * kGBK / 2
+         : WF == GWF_I8 ? (size_t)kGBN * 128  // 8 I8P tile blocks of 2 KiB
+                        : (size_t)kGBN * kAP * 2;
 }
 // GWF_I8 side product staging (in the A / B buffers after the K loop): 32 outlier columns per
 // round, f16 rows of 64 B at a pitch of 80 B
@@ -272,17 +276,14 @@ constexpr size_t gemm_lds_bytes() {
 }
 
 // BM: rows per tile (128, or 256 for bf16 with 8 waves: 4 row groups x 2 column groups of 64 x 64)
-// Two waves per SIMD: two 128-row workgroups per CU (grouped int4 took 324 registers without the bound: 1000 rows 4096 -> 12288 246
-// us, 175 with it). Unsplit gptq.int8 fits 256 registers by itself and spills 16 under the bound: 512 rows without / with it,
-// 4096 -> 12288 111 / 116 us, 11008 -> 4096 190 / 200.
-template <int WF, int EP>
-constexpr int gemm_waves = WF == GWF_W8 && EP != GEP_SPLIT ? 1 : 2;
+// Two waves per SIMD: two 128-row workgroups per CU.
 template <int WF, int EP, int BM = kGBM>
-__global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_waves<WF, EP>))) void gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(GemmParams p) {
   static_assert(BM == kGBM || WF == GWF_BF16 || WF == GWF_I8 || WF == GWF_W4, "256-row tiles: bf16, int8, int4");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr bool NIB = WF == GWF_W4 || WF == GWF_W8;  // nibble-coded: offset removed with the A row sums
   constexpr bool GRP = WF == GWF_W4G;                  // grouped int4: dequantized to the weight values
+  constexpr bool ONCE = WF == GWF_W8 || GRP;           // codes converted to bf16 as they are staged, once per workgroup
   constexpr bool I8 = WF == GWF_I8;                    // LLM.int8(): int8 MFMA + fp16 outlier side product
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // wave grid: WRN row groups x WCN column groups of (16 MI) x (16 NJ) outputs; int4 256-row tiles
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
   const int8_t* aqsrc = I8 ? L8.aq + (size_t)agm * K + ah * 64 : nullptr;
   // register ring of GDEPTH chunks in flight (chunk c lives in slot c % GDEPTH)
   constexpr int GDEPTH = (WF == GWF_W4 && BM == 256) ? LLJ_GDEPTH_W4_256
-                         : (NIB || GRP) ? LLJ_GDEPTH : BM == 256 ? LLJ_GDEPTH_DENSE256 : LLJ_GDEPTH_DENSE;
+                         : ONCE ? LLJ_GDEPTH_ONCE : NIB ? LLJ_GDEPTH : BM == 256 ? LLJ_GDEPTH_DENSE256 : LLJ_GDEPTH_DENSE;
   constexpr int BV = (WF == GWF_W4 || GRP) ? 1 : WF == GWF_W8 ? 2 : BM == 256 ? 2 : 4;  // GWF_I8: 4 (64 B of its tile block)
   // bf16 B with 256-row tiles: 512 threads over the 128 weight rows, a quarter row (32 B) each
   const int br = BM == 256 ? tid >> 2 : ar, bq = BM == 256 ? tid & 3 : ah;
@@ -345,7 +346,8 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
   constexpr int TPB = BM / 4;
   const int bt = tid & 255;
   u32x4 areg[GDEPTH][4], breg[GDEPTH][BV];
-  float2 szr[GDEPTH][4];  // GWF_W4G: (scale, 128 + zero) of the chunk's group for the lane's column of tile j
+  float2 szr[GDEPTH];  // GWF_W4G: (scale, 128 + zero) of the chunk's group for the column whose codes this thread converts
+  const int ccol = 16 * (bt >> 5) + (bt & 15), cseg = 32 * ((bt >> 4) & 1);  // W4P lane bt & 31 of tile bt >> 5: column, first k
   auto load_chunk = [&](int slot, int c) {
     c = c0 + (c < KC ? c : SPLIT && I8 && KC == 0 ? 0 : KC - 1);  // past the end: a valid duplicate, never stored
     if constexpr (I8) {
@@ -364,9 +366,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
       const size_t nt = (size_t)(n0 / 16 + (bt >> 5));  // (256-row tiles: threads 256.. load a copy, never stored)
       breg[slot][0] = __builtin_nontemporal_load(w + (nt * KC128 + (c >> 1)) * 64 + 32 * (c & 1) + (bt & 31));
       if constexpr (GRP) {
-        const size_t go = (size_t)((c >> 1) / p.gch) * p.N + n0 + wc * 16 * NJ + row;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) szr[slot][j] = p.sz[go + 16 * j];
+        szr[slot] = p.sz[(size_t)((c >> 1) / p.gch) * p.N + n0 + ccol];
       }
     } else if constexpr (WF == GWF_W8) {  // the same W4P lane of the low plane and of the high plane
       const u32x4* w = reinterpret_cast<const u32x4*>(p.W);
@@ -380,6 +380,9 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
       for (int v = 0; v < BV; ++v) breg[slot][v] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(w + 8 * v));
     }
   };
+  uint32_t msk = 0x000F000Fu, mag = 0x43004300u;
+  asm volatile("" : "+s"(msk));
+  asm volatile("" : "+v"(mag));
   f32x2 rsum2 = {0.f, 0.f};  // this thread's share of sum_k A[ar, k]
   auto store_chunk = [&](int slot, int buf) {
     if constexpr (I8) {  // A rows of 128 B at the bf16 pitch (144 B); B: the 8 tile blocks as stored
@@ -399,11 +402,30 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
         rsum2 += unpk(areg[slot][v][2]) + unpk(areg[slot][v][3]);
       }
     }
-    if constexpr (WF == GWF_W4 || GRP) {
+    if constexpr (WF == GWF_W4) {
       if (BM == 128 || tid < 256) reinterpret_cast<u32x4*>(Bs(buf))[tid] = breg[slot][0];
-    } else if constexpr (WF == GWF_W8) {  // [low plane halves 4 KiB][high plane halves 4 KiB]
-      reinterpret_cast<u32x4*>(Bs(buf))[tid] = breg[slot][0];
-      reinterpret_cast<u32x4*>(Bs(buf))[kGNT + tid] = breg[slot][1];
+    } else if constexpr (ONCE) {  // 32 consecutive k of one column, word v: k = 8 v + [0, 8), pair e in nibbles e and e + 4
+      bf16_t* b = reinterpret_cast<bf16_t*>(Bs(buf)) + ccol * kAP + cseg;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const uint32_t wl = breg[slot][0][v];
+        u32x4 o;
+        if constexpr (GRP) {
+          // bf16(fp32(q - z) * s), the reference's get_weight(bf16) (quantization.py:402-408: the bf16
+          // weight times the scale in the scale's precision, then stored to bf16): (128 + q) - (128 + z)
+          // is an exact small integer, its product with s rounds once to fp32 (exact for bf16 / fp16
+          // scales, the reference's fp32 product for fp32 scales), the conversion once to bf16
+          const f32x2 sc = {szr[slot].x, szr[slot].x}, zz = {szr[slot].y, szr[slot].y};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = cvt_pk((unpk(and_or(wl >> (4 * e), msk, mag)) - zz) * sc);
+        } else {  // the two planes' nibbles to bytes: codes (0, 4, 1, 5) and (2, 6, 3, 7), exact in bf16
+          const uint32_t wh = breg[slot][1][v];
+          const uint32_t b0 = (wl & 0x0F0F0F0Fu) | ((wh << 4) & 0xF0F0F0F0u), b1 = ((wl >> 4) & 0x0F0F0F0Fu) | (wh & 0xF0F0F0F0u);
+          auto pair = [](uint32_t x, int at) { return cvt_pk(f32x2{(float)((x >> at) & 255u), (float)((x >> (at + 16)) & 255u)}); };
+          o = u32x4{pair(b0, 0), pair(b1, 0), pair(b0, 8), pair(b1, 8)};
+        }
+        *reinterpret_cast<u32x4*>(b + 8 * v) = o;
+      }
     } else {
       bf16_t* b = reinterpret_cast<bf16_t*>(Bs(buf)) + br * kAP + bq * 8 * BV;
 #pragma unroll
@@ -411,10 +433,6 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
     }
   };
 
-  uint32_t msk = 0x000F000Fu, mag = 0x43004300u, mag_hi = 0x45004500u;  // mag_hi: W8 high nibbles, 2048 + 16 hi
-  asm volatile("" : "+s"(msk));
-  asm volatile("" : "+v"(mag));
-  if constexpr (WF == GWF_W8) asm volatile("" : "+v"(mag_hi));
   f32x4 acc[MI][NJ];
   i32x4 iacc[MI][NJ];  // GWF_I8
 #pragma unroll
@@ -427,9 +445,6 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
 
   auto step = [&](int slot, int c) {  // chunk c: stage it, refill its slot with c + GDEPTH, multiply
     const int buf = c & 1;
-    float2 gsz[4];  // GWF_W4G: this chunk's group pairs (the slot is refilled below)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) gsz[j] = szr[slot][j];
     store_chunk(slot, buf);
     __syncthreads();  // chunk c staged; every wave is done with chunk c - 1's buffer
     load_chunk(slot, c + GDEPTH);
@@ -455,7 +470,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
     const bf16_t* a = As(buf);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {  // MFMA k-steps of the chunk: k = 32 s + 8 g + [0, 8)
-      bf16x8 af[MI], bfr[NJ], bhi[NJ];
+      bf16x8 af[MI], bfr[NJ];
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         const int r = wr * 16 * MI + 16 * i + row;
@@ -469,25 +484,6 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
           const uint4 d = make_uint4(and_or(w, msk, mag), and_or(w >> 4, msk, mag), and_or(w >> 8, msk, mag),
                                      and_or(w >> 12, msk, mag));
           bfr[j] = __builtin_bit_cast(bf16x8, d);
-        } else if constexpr (GRP) {
-          // bf16(fp32(q - z) * s), the reference's get_weight(bf16) (quantization.py:402-408: the bf16
-          // weight times the scale in the scale's precision, then stored to bf16): (128 + q) - (128 + z)
-          // is an exact small integer, its product with s rounds once to fp32 (exact for bf16 / fp16
-          // scales, the reference's fp32 product for fp32 scales), the conversion once to bf16
-          const uint32_t w = reinterpret_cast<const uint32_t*>(Bs(buf))[((wc * NJ + j) * 32 + 16 * s + row) * 4 + g];
-          const f32x2 sc = {gsz[j].x, gsz[j].x}, zz = {gsz[j].y, gsz[j].y};
-          uint32_t o[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = cvt_pk((unpk(and_or(w >> (4 * e), msk, mag)) - zz) * sc);
-          bfr[j] = __builtin_bit_cast(bf16x8, make_uint4(o[0], o[1], o[2], o[3]));
-        } else if constexpr (WF == GWF_W8) {
-          const uint32_t* b32 = reinterpret_cast<const uint32_t*>(Bs(buf));
-          const int wi = ((wc * NJ + j) * 32 + 16 * s + row) * 4 + g;
-          const uint32_t wl = b32[wi], wh = b32[kGNT * 4 + wi];
-          bfr[j] = __builtin_bit_cast(bf16x8, make_uint4(and_or(wl, msk, mag), and_or(wl >> 4, msk, mag),
-                                                         and_or(wl >> 8, msk, mag), and_or(wl >> 12, msk, mag)));
-          bhi[j] = __builtin_bit_cast(bf16x8, make_uint4(and_or(wh, msk, mag_hi), and_or(wh >> 4, msk, mag_hi),
-                                                         and_or(wh >> 8, msk, mag_hi), and_or(wh >> 12, msk, mag_hi)));
         } else {
           const int n = wc * 16 * NJ + 16 * j + row;
           bfr[j] = __builtin_bit_cast(
@@ -498,10 +494,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          acc[i][j] = mfma_bf16(af[i], bfr[j], acc[i][j]);
-          if constexpr (WF == GWF_W8) acc[i][j] = mfma_bf16(af[i], bhi[j], acc[i][j]);
-        }
+        for (int j = 0; j < NJ; ++j) acc[i][j] = mfma_bf16(af[i], bfr[j], acc[i][j]);
       if (LLJ_GEMM_PRIO) __builtin_amdgcn_s_setprio(0);
     }
   };
@@ -659,6 +652,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(gemm_wav
     const int n = n0 + wc * 16 * NJ + 16 * j + row;
     float2 szn = make_float2(1.f, 0.f);
     if constexpr (NIB) szn = p.sz[n];
+    if constexpr (WF == GWF_W8) szn.y -= 2176.f;  // the codes carry no offset here
     if constexpr (I8) szn.x = reinterpret_cast<const float*>(p.sz)[n];  // SCB
     float bn = 0.f;
     if constexpr (EP == GEP_BIAS || EP == GEP_GLU) bn = p.bias ? p.bias[n] : 0.f;
@@ -758,9 +752,9 @@ static int gemm_launch(const GemmParams& p, hipStream_t s) {
 //   int4            58 -> (2) 42               61 -> (1) 50        148 -> (8) 38              149 -> (8) 46
 //   bf16            122 -> (5) 54              117 -> (4) 91       346 -> (15) 57             329 -> (8) 82
 //   llm.int8        60 -> (4) 32               53 -> (1) 53        142 -> (8) 35              126 -> (8) 40
-//   gptq.int8       74 -> (5) 46               76 -> (4) 66        187 -> (8) 43              187 -> (8) 58
-//   int4 groups     81 -> (5) 42               82 -> (4) 61        210 -> (8) 42              210 -> (8) 56
-// (unsplit: before the slices and the two-waves bound, which alone took int4 at 154 rows from 61 to 50)
+//   gptq.int8       62 -> (5) 37               62 -> (4) 54        148 -> (8) 37              148 -> (8) 47
+//   int4 groups     60 -> (5) 36               60 -> (4) 53        149 -> (8) 37              149 -> (8) 47
+// (unsplit int4, bf16 and llm.int8: before the slices and the two-waves bound, which alone took int4 at 154 rows from 61 to 50)
 static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out) {
   if (M >= 256 || M < 1 || N % kGBN || K < kGBK) return 1;
   const int KC = wf == GWF_I8 ? K / 128 : K / kGBK, planes = wf == GWF_I8 ? 1 : 0;

@@ -1404,6 +1404,30 @@ def test_gemm_w4z_exact_on_integer_rows(hip):
     np.testing.assert_array_equal(out.float().cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (127, 128, 384), (128, 256, 640), (129, 128, 4224), (300, 384, 256)])
+def test_gemm_w8_exact_on_integer_rows(hip, M, N, K):
+    """gptq.int8 prompt products, every code value, two chunks (fewer than are in flight) to many: with small-integer
+    activations every product and fp32 partial sum is an integer below 2^24, so the result is bitwise
+    bf16(s * sum_k a (q - z)); the scales are powers of two because K slices add s * their partial sums, which any other
+    scale rounds."""
+    rng = np.random.default_rng(M + K)
+    qw, sc, z = rand_w8(rng, N, K)
+    sc = np.exp2(np.round(np.log2(sc)))
+    qw.flat[:256] = np.arange(256)
+    Wd, szd = repack8(hip, qw), sz_of(hip, sc, z, 8)
+    a = rng.integers(-4, 5, size=(M, K)).astype(np.float32)
+    x = T(a, torch.bfloat16)
+    scr = torch.empty(max(4, hip.llj_gemm_ws_bytes(3, M, N, K)), dtype=torch.uint8, device=dev)
+    acc = a.astype(np.int64) @ (qw.astype(np.int64) - z.astype(np.int64)).T
+    want = bf16(sc.reshape(1, N) * acc.astype(np.float32))
+    for ws in (None, scr.data_ptr()):
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        call(hip, "llj_gemm_linear_ws", 3, x.data_ptr(), K, Wd.data_ptr(), szd.data_ptr(), out.data_ptr(), N, M, N, K, ws,
+             scr.numel() if ws else 0, st())
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.float().cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("M,H,K", [(256, 2816, 1024), (300, 11008, 4096), (2048, 11008, 4096), (520, 4096, 11008),
                                    (256, 128, 128)])
 def test_gemm_swiglu_dual_pass(hip, M, H, K):
