@@ -256,12 +256,22 @@ constexpr int kGBM = 128, kGBN = 128, kGBK = 64, kGNT = 256;
 #define LLJ_GDEPTH_DENSE256 2  // bf16 / int8 in 256-row tiles (7B bf16 window 59.6 ms at 1, 42.6 at 2)
 #endif
 constexpr int kAP = kGBK + 8;  // A / bf16-B LDS row pitch (elements): 144 B
+// Tiles of 160 rows: pitch 128 B, the eight 16-B segments of a row permuted by (row >> 1) & 7 (73 KiB of LDS; the padded pitch's
+// 83 would leave one workgroup per CU). 128 rows keep the padded pitch: both fit twice.
+template <int WF, int BM>
+constexpr int gemm_pitch = BM == 160 ? kGBK : kAP;
+template <int BM>
+constexpr int gemm_threads = BM == 256 ? 512 : 256;
+template <int WF, int BM>
+__device__ __forceinline__ int gemm_seg(int row, int seg) {  // element offset of 16-B segment seg of a tile row
+  return row * gemm_pitch<WF, BM> + 8 * (gemm_pitch<WF, BM> == kGBK ? seg ^ ((row >> 1) & 7) : seg);
+}
 
-template <int WF>
+template <int WF, int BM>
 constexpr size_t gemm_b_bytes() {
   return WF == GWF_W4   ? (size_t)kGBN * kGBK / 2
          : WF == GWF_I8 ? (size_t)kGBN * 128  // 8 I8P tile blocks of 2 KiB
-                        : (size_t)kGBN * kAP * 2;
+                        : (size_t)kGBN * gemm_pitch<WF, BM> * 2;
 }
 // GWF_I8 side product staging (in the A / B buffers after the K loop): 32 outlier columns per
 // round, f16 rows of 64 B at a pitch of 80 B
@@ -270,7 +280,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 template <int WF, int BM = kGBM>
 constexpr size_t gemm_lds_bytes() {
   // GWF_I8: also the dense side loop's two (A, B) f16 chunk buffers at the bf16 pitch
-  const size_t main = 2 * ((size_t)BM * kAP * 2 + gemm_b_bytes<WF>()) + BM * sizeof(float);
+  const size_t main = 2 * ((size_t)BM * gemm_pitch<WF, BM> * 2 + gemm_b_bytes<WF, BM>()) + BM * sizeof(float);
   const size_t side = 2 * ((size_t)BM * kAP * 2 + (size_t)kGBN * kAP * 2);
   return WF == GWF_I8 && side > main ? side : main;
 }
@@ -278,8 +288,12 @@ constexpr size_t gemm_lds_bytes() {
 // BM: rows per tile (128, or 256 for bf16 with 8 waves: 4 row groups x 2 column groups of 64 x 64)
 // Two waves per SIMD: two 128-row workgroups per CU.
 template <int WF, int EP, int BM = kGBM>
-__global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(GemmParams p) {
-  static_assert(BM == kGBM || WF == GWF_BF16 || WF == GWF_I8 || WF == GWF_W4, "256-row tiles: bf16, int8, int4");
+__global__ __launch_bounds__(gemm_threads<BM>) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(GemmParams p) {
+  constexpr bool SPLIT = EP == GEP_SPLIT;
+  static_assert(BM != 256 || WF == GWF_BF16 || WF == GWF_I8 || WF == GWF_W4, "256-row tiles: bf16, int8, int4");
+  static_assert(BM != 160 || ((WF == GWF_W8 || WF == GWF_W4G) && SPLIT), "160 rows: K slices");
+  constexpr int NT = gemm_threads<BM>;
+  constexpr bool TALL = BM == 160;  // a thread also stages one A segment of the 32 rows past 128
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr bool NIB = WF == GWF_W4 || WF == GWF_W8;  // nibble-coded: offset removed with the A row sums
   constexpr bool GRP = WF == GWF_W4G;                  // grouped int4: dequantized to the weight values
@@ -289,12 +303,11 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
   // wave grid: WRN row groups x WCN column groups of (16 MI) x (16 NJ) outputs; int4 256-row tiles
   // optionally 2 x 4 waves of 128 x 32 (LLJ_GEMM_W4_WIDE: each B fragment dequantized by 2 waves, not 4)
   constexpr bool WIDE = WF == GWF_W4 && BM == 256 && LLJ_GEMM_W4_WIDE;
-  constexpr int WRN = WIDE ? 2 : BM / 64;  // row groups of waves
-  constexpr int WCN = 2 * BM / 64 / WRN;   // column groups (2 * BM threads = 2 * BM / 64 waves)
+  constexpr int WRN = WIDE || BM < 256 ? 2 : 4;  // row groups of waves
+  constexpr int WCN = NT / 64 / WRN;             // column groups
   constexpr int MI = BM / WRN / 16, NJ = kGBN / WCN / 16;
   const int wr = wave % WRN, wc = wave / WRN;
   const int row = lane & 15, g = lane >> 4;
-  constexpr bool SPLIT = EP == GEP_SPLIT;
   const int M = p.M, K = p.K, KCA = I8 ? K / 128 : K / kGBK, KC128 = K / 128;
   const int mtiles = (M + BM - 1) / BM, ntiles = p.N / kGBN;
   const int total = mtiles * ntiles;
@@ -319,7 +332,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int m0 = mb * BM, n0 = nb * kGBN;
 
   // LDS: [A buf 0][A buf 1][B buf 0][B buf 1][row sums]
-  constexpr size_t kAB = (size_t)BM * kAP * 2, kBB = gemm_b_bytes<WF>();
+  constexpr size_t kAB = (size_t)BM * gemm_pitch<WF, BM> * 2, kBB = gemm_b_bytes<WF, BM>();
   auto As = [&](int b) { return reinterpret_cast<bf16_t*>(smem + b * kAB); };
   auto Bs = [&](int b) { return smem + 2 * kAB + b * kBB; };
   float* rs_lds = reinterpret_cast<float*>(smem + 2 * (kAB + kBB));
@@ -329,6 +342,8 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int ar = tid >> 1, ah = tid & 1;
   const int agm = m0 + ar < M ? m0 + ar : M - 1;  // rows past M: a clamped copy, never stored
   const bf16_t* asrc = p.A + (size_t)agm * p.lda + ah * 32;
+  const int xr = kGBM + (tid >> 3), xm = m0 + xr < M ? m0 + xr : M - 1;
+  const bf16_t* xsrc = p.A + (size_t)xm * p.lda + 8 * (tid & 7);
   I8Layout L8{};
   if constexpr (I8) {
     const I8WsHeader h8 = *reinterpret_cast<const I8WsHeader*>(p.i8ws);
@@ -338,16 +353,17 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int8_t* aqsrc = I8 ? L8.aq + (size_t)agm * K + ah * 64 : nullptr;
   // register ring of GDEPTH chunks in flight (chunk c lives in slot c % GDEPTH)
   constexpr int GDEPTH = (WF == GWF_W4 && BM == 256) ? LLJ_GDEPTH_W4_256
+                         : TALL ? 2  // (3 spill; gptq.int8 154 rows 11008 -> 4096 at 1 / 2: 51 / 40 us)
                          : ONCE ? LLJ_GDEPTH_ONCE : NIB ? LLJ_GDEPTH : BM == 256 ? LLJ_GDEPTH_DENSE256 : LLJ_GDEPTH_DENSE;
   constexpr int BV = (WF == GWF_W4 || GRP) ? 1 : WF == GWF_W8 ? 2 : BM == 256 ? 2 : 4;  // GWF_I8: 4 (64 B of its tile block)
   // bf16 B with 256-row tiles: 512 threads over the 128 weight rows, a quarter row (32 B) each
   const int br = BM == 256 ? tid >> 2 : ar, bq = BM == 256 ? tid & 3 : ah;
   // int8 B: the 8 tile blocks of 128 x 16 B over TPB threads each; int4 B: the first 256 threads
-  constexpr int TPB = BM / 4;
+  constexpr int TPB = NT / 8;
   const int bt = tid & 255;
-  u32x4 areg[GDEPTH][4], breg[GDEPTH][BV];
+  u32x4 areg[GDEPTH][4 + TALL], breg[GDEPTH][BV];
   float2 szr[GDEPTH];  // GWF_W4G: (scale, 128 + zero) of the chunk's group for the column whose codes this thread converts
-  const int ccol = 16 * (bt >> 5) + (bt & 15), cseg = 32 * ((bt >> 4) & 1);  // W4P lane bt & 31 of tile bt >> 5: column, first k
+  const int ccol = 16 * (bt >> 5) + (bt & 15), cseg = 4 * ((bt >> 4) & 1);  // W4P lane bt & 31 of tile bt >> 5: column, first segment of 8 k
   auto load_chunk = [&](int slot, int c) {
     c = c0 + (c < KC ? c : SPLIT && I8 && KC == 0 ? 0 : KC - 1);  // past the end: a valid duplicate, never stored
     if constexpr (I8) {
@@ -361,6 +377,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) areg[slot][v] = *reinterpret_cast<const u32x4*>(asrc + (size_t)c * kGBK + 8 * v);
+    if constexpr (TALL) areg[slot][4] = *reinterpret_cast<const u32x4*>(xsrc + (size_t)c * kGBK);
     if constexpr (WF == GWF_W4 || GRP) {
       const u32x4* w = reinterpret_cast<const u32x4*>(p.W);
       const size_t nt = (size_t)(n0 / 16 + (bt >> 5));  // (256-row tiles: threads 256.. load a copy, never stored)
@@ -384,6 +401,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
   asm volatile("" : "+s"(msk));
   asm volatile("" : "+v"(mag));
   f32x2 rsum2 = {0.f, 0.f};  // this thread's share of sum_k A[ar, k]
+  f32x2 rsumx = {0.f, 0.f};  // and of A[xr, k]
   auto store_chunk = [&](int slot, int buf) {
     if constexpr (I8) {  // A rows of 128 B at the bf16 pitch (144 B); B: the 8 tile blocks as stored
       unsigned char* a8 = reinterpret_cast<unsigned char*>(As(buf)) + ar * (kAP * 2) + ah * 64;
@@ -393,19 +411,27 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
       for (int v = 0; v < BV; ++v) reinterpret_cast<u32x4*>(Bs(buf))[(tid / TPB) * 128 + tid % TPB + TPB * v] = breg[slot][v];
       return;
     }
-    bf16_t* a = As(buf) + ar * kAP + ah * 32;
+    bf16_t* a = As(buf);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      *reinterpret_cast<u32x4*>(a + 8 * v) = areg[slot][v];
+      *reinterpret_cast<u32x4*>(a + gemm_seg<WF, BM>(ar, 4 * ah + v)) = areg[slot][v];
       if constexpr (NIB) {
         rsum2 += unpk(areg[slot][v][0]) + unpk(areg[slot][v][1]);
         rsum2 += unpk(areg[slot][v][2]) + unpk(areg[slot][v][3]);
       }
     }
+    if constexpr (TALL) {
+      const u32x4 t = areg[slot][4];
+      *reinterpret_cast<u32x4*>(a + gemm_seg<WF, BM>(xr, tid & 7)) = t;
+      if constexpr (NIB) {
+        rsumx += unpk(t[0]) + unpk(t[1]);
+        rsumx += unpk(t[2]) + unpk(t[3]);
+      }
+    }
     if constexpr (WF == GWF_W4) {
-      if (BM == 128 || tid < 256) reinterpret_cast<u32x4*>(Bs(buf))[tid] = breg[slot][0];
+      if (NT == 256 || tid < 256) reinterpret_cast<u32x4*>(Bs(buf))[tid] = breg[slot][0];
     } else if constexpr (ONCE) {  // 32 consecutive k of one column, word v: k = 8 v + [0, 8), pair e in nibbles e and e + 4
-      bf16_t* b = reinterpret_cast<bf16_t*>(Bs(buf)) + ccol * kAP + cseg;
+      bf16_t* b = reinterpret_cast<bf16_t*>(Bs(buf));
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const uint32_t wl = breg[slot][0][v];
@@ -424,12 +450,12 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
           auto pair = [](uint32_t x, int at) { return cvt_pk(f32x2{(float)((x >> at) & 255u), (float)((x >> (at + 16)) & 255u)}); };
           o = u32x4{pair(b0, 0), pair(b1, 0), pair(b0, 8), pair(b1, 8)};
         }
-        *reinterpret_cast<u32x4*>(b + 8 * v) = o;
+        *reinterpret_cast<u32x4*>(b + gemm_seg<WF, BM>(ccol, cseg + v)) = o;
       }
     } else {
-      bf16_t* b = reinterpret_cast<bf16_t*>(Bs(buf)) + br * kAP + bq * 8 * BV;
+      bf16_t* b = reinterpret_cast<bf16_t*>(Bs(buf));
 #pragma unroll
-      for (int v = 0; v < BV; ++v) *reinterpret_cast<u32x4*>(b + 8 * v) = breg[slot][v];
+      for (int v = 0; v < BV; ++v) *reinterpret_cast<u32x4*>(b + gemm_seg<WF, BM>(br, bq * BV + v)) = breg[slot][v];
     }
   };
 
@@ -474,7 +500,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         const int r = wr * 16 * MI + 16 * i + row;
-        af[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(a + r * kAP + 32 * s + 8 * g));
+        af[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(a + gemm_seg<WF, BM>(r, 4 * s + g)));
       }
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
@@ -487,7 +513,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
         } else {
           const int n = wc * 16 * NJ + 16 * j + row;
           bfr[j] = __builtin_bit_cast(
-              bf16x8, *reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(Bs(buf)) + n * kAP + 32 * s + 8 * g));
+              bf16x8, *reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(Bs(buf)) + gemm_seg<WF, BM>(n, 4 * s + g)));
         }
       }
       if (LLJ_GEMM_PRIO) __builtin_amdgcn_s_setprio(1);  // the MFMA cluster ahead of the other waves' staging
@@ -516,6 +542,12 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
   // row sums of A (both halves of a row are adjacent lanes)
   rsum += lane_xor1(rsum);
   if (!ah) rs_lds[ar] = rsum;
+  if constexpr (TALL) {  // (the eight segments of a row are adjacent lanes)
+    float r = rsumx.x + rsumx.y;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) r += __shfl_xor(r, o, 64);
+    if ((tid & 7) == 0) rs_lds[xr] = r;
+  }
   __syncthreads();
 
   // ---- GWF_I8: fp16 outlier side product into sacc (the K loop's LDS is free now)
@@ -658,7 +690,7 @@ __global__ __launch_bounds__(2 * BM) __attribute__((amdgpu_waves_per_eu(2))) voi
     if constexpr (EP == GEP_BIAS || EP == GEP_GLU) bn = p.bias ? p.bias[n] : 0.f;
     const int nblk = n0 + wc * 16 * NJ + 16 * j;  // first column of this 16-column block
     const QkvCol qc = EP == GEP_QKV ? qkv_col(p, nblk, n, Cd) : QkvCol{};
-    constexpr int GI = I8 ? (EP == GEP_QKV ? 1 : 2) : 4;  // row blocks whose operands are in flight together (LLM.int8: 3 accumulator sets live)
+    constexpr int GI = I8 ? (EP == GEP_QKV ? 1 : 2) : MI % 4 ? MI : 4;  // row blocks whose operands are in flight together (LLM.int8: 3 accumulator sets live)
 #pragma unroll
     for (int i0 = 0; i0 < MI; i0 += GI) {
       float2 opv[GI][4];
@@ -736,7 +768,7 @@ static int gemm_launch(const GemmParams& p, hipStream_t s) {
   }
   int tiles = ((p.M + BM - 1) / BM) * (p.N / kGBN);
   if (EP == GEP_SPLIT) tiles *= p.nsplit + (WF == GWF_I8 ? 1 : 0);
-  hipLaunchKernelGGL(kern, dim3(tiles), dim3(2 * BM), lds, s, p);
+  hipLaunchKernelGGL(kern, dim3(tiles), dim3(gemm_threads<BM>), lds, s, p);
   LLJ_CHECK_LAUNCH();
   return 0;
 }
@@ -745,20 +777,27 @@ static int gemm_launch(const GemmParams& p, hipStream_t s) {
 #define LLJ_GSPLIT 0  // A/B: slices forced (0: the rule)
 #endif
 // K slices of a product of less than 256 rows (128-row tiles): such a product has 32..172 tiles at 7B widths, one workgroup
-// each with a chain of K / 64 chunk loads, far from the memory and the matrix rate. Returns the slices (1: none), kcs = chunks each.
+// each with a chain of K / 64 chunk loads, far from the memory and the matrix rate. Returns the slices (1: none), kcs = chunks each, rows = of a tile.
 // The rule weighs, in us, the chunks of the busiest CU (one chunk of one workgroup; two workgroups on a CU take 1.5, four 3 times
 // as long) against the second launch and the partial sums, and splits for a gain of a tenth. What it chooses, us unsplit -> (slices) us:
 //                   4096 -> 12288, 128 rows    154 rows            11008 -> 4096, 128 rows    154 rows
 //   int4            58 -> (2) 42               61 -> (1) 50        148 -> (8) 38              149 -> (8) 46
 //   bf16            122 -> (5) 54              117 -> (4) 91       346 -> (15) 57             329 -> (8) 82
 //   llm.int8        60 -> (4) 32               53 -> (1) 53        142 -> (8) 35              126 -> (8) 40
-//   gptq.int8       62 -> (5) 37               62 -> (4) 54        148 -> (8) 37              148 -> (8) 47
-//   int4 groups     60 -> (5) 36               60 -> (4) 53        149 -> (8) 37              149 -> (8) 47
+//   gptq.int8       62 -> (5) 37               62 -> (4) 43        148 -> (8) 37              148 -> (8) 40
+//   int4 groups     60 -> (5) 36               60 -> (4) 43        149 -> (8) 37              149 -> (8) 43
 // (unsplit int4, bf16 and llm.int8: before the slices and the two-waves bound, which alone took int4 at 154 rows from 61 to 50)
-static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out) {
+// 129 to 160 rows are one tile of 160 where the codes are converted as they are staged (two tiles of 128 convert, read and multiply
+// for 256 rows), us two of 128 -> one of 160 at 154 rows: 4096 -> 12288 gptq.int8 54 -> 43, int4 groups 53 -> 43; 11008 -> 4096
+// 47 -> 40, 47 -> 43; 4096 -> 4096 30 -> 28, 28 -> 27. int4 per row spills there and gains nothing (50 -> 49, 45 -> 43, 29 -> 32), nor
+// does a tile of 192 for more rows (one chunk in flight: gptq.int8 11008 -> 4096, 192 rows 47 -> 53).
+static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int* rows_out) {
+  if (kcs_out) *kcs_out = K / kGBK;
+  if (rows_out) *rows_out = kGBM;
   if (M >= 256 || M < 1 || N % kGBN || K < kGBK) return 1;
   const int KC = wf == GWF_I8 ? K / 128 : K / kGBK, planes = wf == GWF_I8 ? 1 : 0;
-  const long tiles = (long)((M + kGBM - 1) / kGBM) * (N / kGBN);
+  const int rows = (wf == GWF_W8 || wf == GWF_W4G) && M > kGBM && M <= 160 ? 160 : kGBM;
+  const long tiles = (long)((M + rows - 1) / rows) * (N / kGBN);
   const double chunk = wf == GWF_W4 ? 0.75 : wf == GWF_BF16 ? 1.85 : wf == GWF_I8 ? 1.7 : 1.2;
   int best = 1, best_kcs = KC;
   double least = 0;
@@ -772,21 +811,27 @@ static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out) {
     if (least == 0 || us < (best == 1 ? 0.9 : 1.0) * least) best = ns, best_kcs = kcs, least = us;
   }
   if (kcs_out) *kcs_out = best_kcs;
+  if (rows_out) *rows_out = best > 1 ? rows : kGBM;
   return best;
 }
 static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
-  const int ns = gemm_split_plan(wf, M, N, K, nullptr);
+  const int ns = gemm_split_plan(wf, M, N, K, nullptr, nullptr);
   return ns < 2 ? 0 : (size_t)(ns + (wf == GWF_I8 ? 1 : 0)) * M * N * 4;
 }
-// The 128-row kernel of format WF, in K slices when p.ws holds ws_bytes enough for the plan.
+// The 128- or 160-row kernel of format WF, in K slices when p.ws holds ws_bytes enough for the plan.
 template <int WF, int EP>
 static int gemm_split_launch(GemmParams p, size_t ws_bytes, hipStream_t s) {
-  int kcs = 0;
-  const int ns = p.ws ? gemm_split_plan(WF, p.M, p.N, p.K, &kcs) : 1;
+  int kcs = 0, rows = kGBM;
+  const int ns = p.ws ? gemm_split_plan(WF, p.M, p.N, p.K, &kcs, &rows) : 1;
   if (ns < 2 || ws_bytes < gemm_split_bytes(WF, p.M, p.N, p.K)) return gemm_launch<WF, EP>(p, s);
   p.nsplit = ns;
   p.kcs = kcs;
-  if (int e = gemm_launch<WF, GEP_SPLIT>(p, s)) return e;
+  int e;
+  if constexpr (WF == GWF_W8 || WF == GWF_W4G)
+    e = rows == 160 ? gemm_launch<WF, GEP_SPLIT, 160>(p, s) : gemm_launch<WF, GEP_SPLIT>(p, s);
+  else
+    e = gemm_launch<WF, GEP_SPLIT>(p, s);
+  if (e) return e;
   hipLaunchKernelGGL((gemm_finish_kernel<EP, WF == GWF_I8>), dim3(p.N / 64, (p.M + 3) / 4), dim3(256), 0, s, p);
   LLJ_CHECK_LAUNCH();
   return 0;

@@ -1404,12 +1404,13 @@ def test_gemm_w4z_exact_on_integer_rows(hip):
     np.testing.assert_array_equal(out.float().cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (127, 128, 384), (128, 256, 640), (129, 128, 4224), (300, 384, 256)])
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (127, 128, 384), (128, 256, 640), (129, 128, 4224), (150, 128, 384), (160, 256, 1024),
+                                   (161, 128, 2176), (300, 384, 256)])
 def test_gemm_w8_exact_on_integer_rows(hip, M, N, K):
-    """gptq.int8 prompt products, every code value, two chunks (fewer than are in flight) to many: with small-integer
-    activations every product and fp32 partial sum is an integer below 2^24, so the result is bitwise
-    bf16(s * sum_k a (q - z)); the scales are powers of two because K slices add s * their partial sums, which any other
-    scale rounds."""
+    """gptq.int8 prompt products, every code value, tiles of 128 and of 160 rows, two chunks (fewer than are in flight) to
+    many: with small-integer activations every product and fp32 partial sum is an integer below 2^24, so the result is
+    bitwise bf16(s * sum_k a (q - z)); the scales are powers of two because K slices add s * their partial sums, which any
+    other scale rounds."""
     rng = np.random.default_rng(M + K)
     qw, sc, z = rand_w8(rng, N, K)
     sc = np.exp2(np.round(np.log2(sc)))
@@ -1850,6 +1851,27 @@ def test_gemm_grouped_dequant_equals_get_weight_bf16(hip, scale_kind):
     torch.cuda.synchronize()
     wref = O.colblock_get_weight(qw, sc, z, 4, tile_cols=g, bf16=True)
     np.testing.assert_array_equal(out.float().cpu().numpy().T, wref)
+
+
+@pytest.mark.parametrize("M", [128, 129, 150, 160, 161])
+def test_gemm_grouped_dequant_in_k_slices(hip, M):
+    """Rows of the identity as in the test above, K in slices, tiles of 128 and of 160 rows: a row's one product, and zeros
+    from the other slices, so the dequantized weight bit for bit."""
+    rng = np.random.default_rng(M)
+    N, K, g = 256, 2048, 256
+    qw, sc, z = rand_w4g(rng, N, K, g)
+    k = rng.permutation(K)[:M]
+    x = np.zeros((M, K), np.float32)
+    x[np.arange(M), k] = 1
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    f = 4 | (2 << 8)
+    ws = torch.empty(hip.llj_gemm_ws_bytes(f, M, N, K), dtype=torch.uint8, device=dev)
+    assert ws.numel() > 0
+    xd, wd, szd = T(x, torch.bfloat16), repack(hip, qw), sz_grouped(hip, sc, z)
+    call(hip, "llj_gemm_linear_ws", f, xd.data_ptr(), K, wd.data_ptr(), szd.data_ptr(), out.data_ptr(), N, M, N, K, ws.data_ptr(),
+         ws.numel(), st())
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.float().cpu().numpy(), O.colblock_get_weight(qw, sc, z, 4, tile_cols=g, bf16=True).T[k])
 
 
 def _i8_ws_offsets(M, K):
