@@ -776,29 +776,47 @@ static int gemm_launch(const GemmParams& p, hipStream_t s) {
 #ifndef LLJ_GSPLIT
 #define LLJ_GSPLIT 0  // A/B: slices forced (0: the rule)
 #endif
-// K slices of a product of less than 256 rows (128-row tiles): such a product has 32..172 tiles at 7B widths, one workgroup
+#ifndef LLJ_GEMM_GLDS_BF16
+#define LLJ_GEMM_GLDS_BF16 1  // 7B 2048-token bf16 window 43.1 -> 36.5 ms (profiles/r04_prefill_ab.json)
+#endif
+#ifndef LLJ_GEMM_GLDS_W4
+#define LLJ_GEMM_GLDS_W4 0  // int4: 42.5 ms vs 37.6 with the register-staged 256-row kernel
+#endif
+// option LLJ_OPT_GEMM_GLDS (llj_set_option / LLJ_GEMM_GLDS) 1 / 0: the LDS-DMA / the register-staged
+// kernels for every format (A/B in one process); unset: the per-format default
+static inline bool glds_enabled(int wf) {
+  const int o = opt(LLJ_OPT_GEMM_GLDS);
+  if (o >= 0) return o != 0;
+  return wf == GWF_BF16 ? LLJ_GEMM_GLDS_BF16 != 0 : LLJ_GEMM_GLDS_W4 != 0;
+}
+// K slices of a product of less than 256 rows (128-row tiles, bf16 256): such a product has 32..172 tiles at 7B widths, one workgroup
 // each with a chain of K / 64 chunk loads, far from the memory and the matrix rate. Returns the slices (1: none), kcs = chunks each, rows = of a tile.
 // The rule weighs, in us, the chunks of the busiest CU (one chunk of one workgroup; two workgroups on a CU take 1.5, four 3 times
 // as long) against the second launch and the partial sums, and splits for a gain of a tenth. What it chooses, us unsplit -> (slices) us:
 //                   4096 -> 12288, 128 rows    154 rows            11008 -> 4096, 128 rows    154 rows
 //   int4            58 -> (2) 42               61 -> (1) 50        148 -> (8) 38              149 -> (8) 46
-//   bf16            122 -> (5) 54              117 -> (4) 91       346 -> (15) 57             329 -> (8) 82
+//   bf16            56 -> (2) 38               58 -> (2) 38        129 -> (8) 31              131 -> (8) 34
 //   llm.int8        60 -> (4) 32               53 -> (1) 53        142 -> (8) 35              126 -> (8) 40
 //   gptq.int8       62 -> (5) 37               62 -> (4) 43        148 -> (8) 37              148 -> (8) 40
 //   int4 groups     60 -> (5) 36               60 -> (4) 43        149 -> (8) 37              149 -> (8) 43
-// (unsplit int4, bf16 and llm.int8: before the slices and the two-waves bound, which alone took int4 at 154 rows from 61 to 50)
+// (unsplit int4 and llm.int8: before the slices and the two-waves bound, which alone took int4 at 154 rows from 61 to 50)
 // 129 to 160 rows are one tile of 160 where the codes are converted as they are staged (two tiles of 128 convert, read and multiply
 // for 256 rows), us two of 128 -> one of 160 at 154 rows: 4096 -> 12288 gptq.int8 54 -> 43, int4 groups 53 -> 43; 11008 -> 4096
 // 47 -> 40, 47 -> 43; 4096 -> 4096 30 -> 28, 28 -> 27. int4 per row spills there and gains nothing (50 -> 49, 45 -> 43, 29 -> 32), nor
 // does a tile of 192 for more rows (one chunk in flight: gptq.int8 11008 -> 4096, 192 rows 47 -> 53).
+// bf16 takes one tile of 256 rows per 128 columns (gemm_glds_kernel; a chunk there is 0.87 us, one workgroup per CU) at any count of
+// rows: the register-staged tiles of 128 rows cost 1.85 a chunk, and split better to 42 / 53 / 90 us 4096 -> 12288 at 32 / 128 / 154
+// rows and 44 / 55 / 82 11008 -> 4096, 32 / 38 / 38 and 27 / 31 / 34 so.
 static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int* rows_out) {
   if (kcs_out) *kcs_out = K / kGBK;
   if (rows_out) *rows_out = kGBM;
   if (M >= 256 || M < 1 || N % kGBN || K < kGBK) return 1;
   const int KC = wf == GWF_I8 ? K / 128 : K / kGBK, planes = wf == GWF_I8 ? 1 : 0;
-  const int rows = (wf == GWF_W8 || wf == GWF_W4G) && M > kGBM && M <= 160 ? 160 : kGBM;
+  const bool dma = wf == GWF_BF16;
+  if (dma && !glds_enabled(wf)) return 1;
+  const int rows = dma ? 256 : (wf == GWF_W8 || wf == GWF_W4G) && M > kGBM && M <= 160 ? 160 : kGBM;
   const long tiles = (long)((M + rows - 1) / rows) * (N / kGBN);
-  const double chunk = wf == GWF_W4 ? 0.75 : wf == GWF_BF16 ? 1.85 : wf == GWF_I8 ? 1.7 : 1.2;
+  const double chunk = wf == GWF_W4 ? 0.75 : dma ? 0.87 : wf == GWF_I8 ? 1.7 : 1.2;
   int best = 1, best_kcs = KC;
   double least = 0;
   for (int ns = LLJ_GSPLIT ? LLJ_GSPLIT : 1; ns <= (LLJ_GSPLIT ? LLJ_GSPLIT : 16); ++ns) {
@@ -806,8 +824,9 @@ static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int
     kcs += kcs & 1;
     if (ns > 1 && (kcs < 4 || (KC + kcs - 1) / kcs != ns)) continue;
     const long q = (tiles * ns + 255) / 256;  // workgroups of the busiest CU
-    const double load = q == 1 ? 1.0 : q * 0.75 + (q & 1) * 0.25;
-    const double us = (ns > 1 ? kcs : KC) * chunk * load + (ns > 1 ? 4.0 + (ns + planes) * (double)M * N * 2e-6 : 0.0);
+    const double load = dma ? q : q == 1 ? 1.0 : q * 0.75 + (q & 1) * 0.25;
+    const double us = (ns > 1 ? kcs : KC) * chunk * load + (dma ? 2.0 * q : 0.0) +
+                      (ns > 1 ? 4.0 + (ns + planes) * (double)M * N * (dma ? 1e-6 : 2e-6) : 0.0);
     if (least == 0 || us < (best == 1 ? 0.9 : 1.0) * least) best = ns, best_kcs = kcs, least = us;
   }
   if (kcs_out) *kcs_out = best_kcs;
@@ -818,26 +837,6 @@ static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
   const int ns = gemm_split_plan(wf, M, N, K, nullptr, nullptr);
   return ns < 2 ? 0 : (size_t)(ns + (wf == GWF_I8 ? 1 : 0)) * M * N * 4;
 }
-// The 128- or 160-row kernel of format WF, in K slices when p.ws holds ws_bytes enough for the plan.
-template <int WF, int EP>
-static int gemm_split_launch(GemmParams p, size_t ws_bytes, hipStream_t s) {
-  int kcs = 0, rows = kGBM;
-  const int ns = p.ws ? gemm_split_plan(WF, p.M, p.N, p.K, &kcs, &rows) : 1;
-  if (ns < 2 || ws_bytes < gemm_split_bytes(WF, p.M, p.N, p.K)) return gemm_launch<WF, EP>(p, s);
-  p.nsplit = ns;
-  p.kcs = kcs;
-  int e;
-  if constexpr (WF == GWF_W8 || WF == GWF_W4G)
-    e = rows == 160 ? gemm_launch<WF, GEP_SPLIT, 160>(p, s) : gemm_launch<WF, GEP_SPLIT>(p, s);
-  else
-    e = gemm_launch<WF, GEP_SPLIT>(p, s);
-  if (e) return e;
-  hipLaunchKernelGGL((gemm_finish_kernel<EP, WF == GWF_I8>), dim3(p.N / 64, (p.M + 3) / 4), dim3(256), 0, s, p);
-  LLJ_CHECK_LAUNCH();
-  return 0;
-}
-
-
 // ---------------------------------------------------------------------------------------------
 // 256-row LDS-DMA GEMM (bf16 and int4 W4P weights, M >= 256): a 512-thread workgroup (8 waves, one
 // per CU) owns a 256 x BN output tile (BN 256: waves 2 x 4 of 128 x 64; BN 128: 4 x 2 of 64 x 64)
@@ -852,12 +851,6 @@ static int gemm_split_launch(GemmParams p, size_t ws_bytes, hipStream_t s) {
 // hits 16 distinct bank slots. int4: the 128 + zero offset is removed with the row sums of A,
 // which the waves form from the A fragments they already hold (v_dot2 with (1, 1); wave column wc
 // sums the 16-row blocks i = wc mod WN) and combine through LDS after the loop.
-#ifndef LLJ_GEMM_GLDS_BF16
-#define LLJ_GEMM_GLDS_BF16 1  // 7B 2048-token bf16 window 43.1 -> 36.5 ms (profiles/r04_prefill_ab.json)
-#endif
-#ifndef LLJ_GEMM_GLDS_W4
-#define LLJ_GEMM_GLDS_W4 0  // int4: 42.5 ms vs 37.6 with the register-staged 256-row kernel
-#endif
 #ifndef LLJ_GLDS_W4_WN
 #define LLJ_GLDS_W4_WN 4
 #endif
@@ -1545,13 +1538,6 @@ static int gemm_glds_launch(const GemmParams& p, hipStream_t s) {
   return 0;
 }
 
-// option LLJ_OPT_GEMM_GLDS (llj_set_option / LLJ_GEMM_GLDS) 1 / 0: the LDS-DMA / the register-staged
-// kernels for every format (A/B in one process); unset: the per-format default
-static inline bool glds_enabled(int wf) {
-  const int o = opt(LLJ_OPT_GEMM_GLDS);
-  if (o >= 0) return o != 0;
-  return wf == GWF_BF16 ? LLJ_GEMM_GLDS_BF16 != 0 : LLJ_GEMM_GLDS_W4 != 0;
-}
 
 // 256 x 256 or 256 x 128 tiles: the shape with the fewer tile-time units over the CUs (waves of
 // tiles rounded up, a 256 x 128 tile costing LLJ_GLDS_COST128 % of a 256 x 256 one)
@@ -1577,6 +1563,31 @@ static int gemm_glds_run(const GemmParams& p, hipStream_t s) {
   const long cost = oc >= 0 ? oc : LLJ_GLDS_COST128;
   if (w256 > 0 && 100 * w256 <= cost * w128) return gemm_glds_launch<WF, EP, 256>(p, s);
   return gemm_glds_launch<WF, EP, 128>(p, s);
+}
+
+// Less than 256 rows, and the formats without a kernel of 256: in K slices when p.ws holds ws_bytes enough for the plan.
+template <int WF, int EP>
+static int gemm_split_launch(GemmParams p, size_t ws_bytes, hipStream_t s) {
+  int kcs = 0, rows = kGBM;
+  const int ns = p.ws ? gemm_split_plan(WF, p.M, p.N, p.K, &kcs, &rows) : 1;
+  if (ns < 2 || ws_bytes < gemm_split_bytes(WF, p.M, p.N, p.K)) {
+    if constexpr (WF == GWF_BF16)
+      if (glds_enabled(WF)) return gemm_glds_run<WF, EP>(p, s);
+    return gemm_launch<WF, EP>(p, s);
+  }
+  p.nsplit = ns;
+  p.kcs = kcs;
+  int e;
+  if constexpr (WF == GWF_BF16)
+    e = gemm_glds_launch<WF, GEP_PARTIAL, 128>(p, s);
+  else if constexpr (WF == GWF_W8 || WF == GWF_W4G)
+    e = rows == 160 ? gemm_launch<WF, GEP_SPLIT, 160>(p, s) : gemm_launch<WF, GEP_SPLIT>(p, s);
+  else
+    e = gemm_launch<WF, GEP_SPLIT>(p, s);
+  if (e) return e;
+  hipLaunchKernelGGL((gemm_finish_kernel<EP, WF == GWF_I8>), dim3(p.N / 64, (p.M + 3) / 4), dim3(256), 0, s, p);
+  LLJ_CHECK_LAUNCH();
+  return 0;
 }
 
 // K slices for a residual GEMM on the LDS-DMA kernels (0: none): when the row tiles x 128-column tiles

@@ -1404,6 +1404,29 @@ def test_gemm_w4z_exact_on_integer_rows(hip):
     np.testing.assert_array_equal(out.float().cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (17, 128, 384), (64, 256, 640), (129, 384, 4224), (255, 128, 2176)])
+def test_gemm_bf16_exact_below_256_rows(hip, M, N, K):
+    """Small integers: every product and fp32 partial sum is an integer below 2^24, whole or in K slices, so the product is
+    bitwise bf16 of the exact sums, and with a residual bf16 of the residual plus that."""
+    rng = np.random.default_rng(M + K)
+    a = rng.integers(-4, 5, size=(M, K)).astype(np.float32)
+    w = rng.integers(-3, 4, size=(N, K)).astype(np.float32)
+    x, W = T(a, torch.bfloat16), T(w, torch.bfloat16)
+    res = rng.integers(-64, 65, size=(M, N)).astype(np.float32)
+    y = bf16(a @ w.T)
+    n = hip.llj_gemm_ws_bytes(1, M, N, K)
+    assert (n > 0) == (K >= 640)
+    scr = torch.empty(max(4, n), dtype=torch.uint8, device=dev)
+    for ws in (None, scr.data_ptr()):
+        out, r = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev), T(res, torch.bfloat16)
+        tail = (N, M, N, K, ws, n if ws else 0, st())
+        call(hip, "llj_gemm_linear_ws", 1, x.data_ptr(), K, W.data_ptr(), None, out.data_ptr(), *tail)
+        call(hip, "llj_gemm_resid_ws", 1, x.data_ptr(), K, W.data_ptr(), None, r.data_ptr(), *tail)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.float().cpu().numpy(), y)
+        np.testing.assert_array_equal(r.float().cpu().numpy(), bf16(res + y))
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 128, 128), (127, 128, 384), (128, 256, 640), (129, 128, 4224), (150, 128, 384), (160, 256, 1024),
                                    (161, 128, 2176), (300, 384, 256)])
 def test_gemm_w8_exact_on_integer_rows(hip, M, N, K):
