@@ -381,6 +381,36 @@ def _attention_case(hip, hs, nh, B, T_, S, p0):
     assert_bf16_close(y.float().cpu().numpy(), _attn_oracle(q, kc, vc, pos, S, T_, nh, hs), "attention")
 
 
+@pytest.mark.parametrize("V", [7, 1000, 32000, 32776, 70001])
+def test_argmax_ties_and_values_out_of_range(hip, V):
+    """Lowest index of the largest value: equal values in other threads, vectors and rounds of the row, -0 equal to 0, NaNs
+    passed over; a row of -inf or of NaN gives 0."""
+    rng = np.random.default_rng(V)
+    rows = []
+    for _ in range(4):
+        r = bf16(rng.standard_normal(V))
+        at = np.sort(rng.choice(V, 3, replace=False))
+        r[at] = 9.0
+        rows.append((r, at[0]))
+    r = bf16(rng.standard_normal(V))
+    r[: V - 1] = np.nan
+    rows.append((r, V - 1))
+    r = -np.abs(bf16(rng.standard_normal(V))) - 1
+    r[V // 2], r[V - 1] = -0.0, 0.0
+    rows.append((r, V // 2))
+    r = np.full(V, -np.inf)
+    r[0] = np.nan
+    rows.append((r, 1))
+    rows += [(np.full(V, -np.inf), 0), (np.full(V, np.nan), 0)]
+    L = np.stack([r for r, _ in rows]).astype(np.float32)
+    want = np.array([i for _, i in rows])
+    for name, t in (("llj_argmax", T(L, torch.bfloat16)), ("llj_g_argmax", T(L))):
+        out = torch.full((len(rows),), -1, dtype=torch.int32, device=dev)
+        call(hip, name, t.data_ptr(), V, len(rows), V, out.data_ptr(), None, 0, None, st())
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
 def test_argmax_and_advance(hip):
     rng = np.random.default_rng(3)
     V, M = 32000, 8
