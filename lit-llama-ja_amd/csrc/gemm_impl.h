@@ -795,7 +795,7 @@ static inline bool glds_enabled(int wf) {
 // as long) against the second launch and the partial sums, and splits for a gain of a tenth. What it chooses, us unsplit -> (slices) us:
 //                   4096 -> 12288, 128 rows    154 rows            11008 -> 4096, 128 rows    154 rows
 //   int4            58 -> (2) 42               61 -> (1) 50        148 -> (8) 38              149 -> (8) 46
-//   bf16            56 -> (2) 38               58 -> (2) 38        129 -> (8) 31              131 -> (8) 34
+//   bf16            56 -> (2) 36               58 -> (2) 37        129 -> (8) 31              131 -> (8) 34
 //   llm.int8        60 -> (4) 32               53 -> (1) 53        142 -> (8) 35              126 -> (8) 40
 //   gptq.int8       62 -> (5) 37               62 -> (4) 43        148 -> (8) 37              148 -> (8) 40
 //   int4 groups     60 -> (5) 36               60 -> (4) 43        149 -> (8) 37              149 -> (8) 43
@@ -804,9 +804,9 @@ static inline bool glds_enabled(int wf) {
 // for 256 rows), us two of 128 -> one of 160 at 154 rows: 4096 -> 12288 gptq.int8 54 -> 43, int4 groups 53 -> 43; 11008 -> 4096
 // 47 -> 40, 47 -> 43; 4096 -> 4096 30 -> 28, 28 -> 27. int4 per row spills there and gains nothing (50 -> 49, 45 -> 43, 29 -> 32), nor
 // does a tile of 192 for more rows (one chunk in flight: gptq.int8 11008 -> 4096, 192 rows 47 -> 53).
-// bf16 takes one tile of 256 rows per 128 columns (gemm_glds_kernel; a chunk there is 0.87 us, one workgroup per CU) at any count of
+// bf16 takes one tile of 256 rows per 128 columns (gemm_glds_kernel; a chunk there is 0.7 us, one workgroup per CU) at any count of
 // rows: the register-staged tiles of 128 rows cost 1.85 a chunk, and split better to 42 / 53 / 90 us 4096 -> 12288 at 32 / 128 / 154
-// rows and 44 / 55 / 82 11008 -> 4096, 32 / 38 / 38 and 27 / 31 / 34 so.
+// rows and 44 / 55 / 82 11008 -> 4096, 32 / 36 / 37 and 27 / 31 / 34 so.
 static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int* rows_out) {
   if (kcs_out) *kcs_out = K / kGBK;
   if (rows_out) *rows_out = kGBM;
@@ -816,7 +816,7 @@ static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int
   if (dma && !glds_enabled(wf)) return 1;
   const int rows = dma ? 256 : (wf == GWF_W8 || wf == GWF_W4G) && M > kGBM && M <= 160 ? 160 : kGBM;
   const long tiles = (long)((M + rows - 1) / rows) * (N / kGBN);
-  const double chunk = wf == GWF_W4 ? 0.75 : dma ? 0.87 : wf == GWF_I8 ? 1.7 : 1.2;
+  const double chunk = wf == GWF_W4 ? 0.75 : dma ? 0.7 : wf == GWF_I8 ? 1.7 : 1.2;
   int best = 1, best_kcs = KC;
   double least = 0;
   for (int ns = LLJ_GSPLIT ? LLJ_GSPLIT : 1; ns <= (LLJ_GSPLIT ? LLJ_GSPLIT : 16); ++ns) {
@@ -858,7 +858,7 @@ static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
 #define LLJ_GLDS_PRE 1  // 256 x 128 tiles: read both MFMA steps' fragments of a chunk before its MFMAs (bf16 window 35.9 -> 35.4 ms)
 #endif
 #ifndef LLJ_GLDS_GROUPM
-#define LLJ_GLDS_GROUPM 0  // A/B only: grouped tile order (row tiles per group); 0 = the m- / n-fastest orders below
+#define LLJ_GLDS_GROUPM 4  // LDS-DMA GEMM of bf16 weights, more than 8 row tiles: row tiles that sweep the columns together
 #endif
 #ifndef LLJ_GLDS_NFAST_W4Z
 #define LLJ_GLDS_NFAST_W4Z 1  // convert-once int4 LDS-DMA GEMM: n-fastest tile order (A/B)
@@ -868,9 +868,6 @@ static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
 #endif
 #ifndef LLJ_GLDS_FDB
 #define LLJ_GLDS_FDB 1  // LDS-DMA GEMM at 256 x 128: chunk t + 1's fragments read during chunk t's MFMAs (A/B)
-#endif
-#ifndef LLJ_FDB_DSPM
-#define LLJ_FDB_DSPM 0  // fragment double buffering: LDS fragment reads per MFMA in the sched_group pattern (0: the scheduler's)
 #endif
 #ifndef LLJ_W4Z_PRIO
 #define LLJ_W4Z_PRIO 0  // convert-once int4: s_setprio around the MFMA clusters (1; 0: none, so the conversion interleaves with them)
@@ -885,13 +882,16 @@ static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
 #define LLJ_W4Z_IGLP 1  // convert-once int4: sched_group_barrier interleave of the conversion with the MFMAs
 #endif
 #ifndef LLJ_W4Z_VPM
-#define LLJ_W4Z_VPM 1  // VALU instructions per MFMA in that interleave (with fragment double buffering: 1 vs 2 vs 3 = 29.4-29.5 vs 29.9-30.0 vs 31.1 ms per 7B window)
+#define LLJ_W4Z_VPM 1  // VALU instructions per MFMA in that interleave, without fragment double buffering
 #endif
 #ifndef LLJ_W4Z_AFTER
 #define LLJ_W4Z_AFTER 0  // convert-once int4: the converting waves convert after their MFMAs (A/B)
 #endif
 #ifndef LLJ_GLDS_COST128
-#define LLJ_GLDS_COST128 55  // time of a 256 x 128 tile in % of a 256 x 256 one (tile-shape choice)
+// time of a 256 x 128 tile in % of a 256 x 256 one: less than half of it, so 256 x 128 always (4 row tiles at a time, bf16 rows 1024 /
+// 2048 / 4096 / 8192, 256 x 256 -> 256 x 128: 4096 -> 12288 108 / 203 / 343 / 687 -> 108 / 168 / 336 / 663 us, 11008 -> 4096
+// 246 / 246 / 292 / 595 -> 131 / 150 / 297 / 585)
+#define LLJ_GLDS_COST128 49
 #endif
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -958,9 +958,12 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
   // weight columns: the A re-reads go from one per column tile to one per XCD -- the int4 weights are a
   // quarter of the bf16 bytes, so re-reading them per row panel is the cheaper side)
   constexpr bool NFAST = CVT ? LLJ_GLDS_NFAST_W4Z != 0 : LLJ_GLDS_NFAST_BF16 != 0;
-  // (LLJ_GLDS_GROUPM > 0, A/B: groups of that many row tiles sweep the columns together, m fastest inside)
   int nb = NFAST ? t % ntiles : t / mtiles, mb = NFAST ? t / ntiles : t % mtiles;
-  if constexpr (LLJ_GLDS_GROUPM > 0) {
+  // many row tiles, m fastest: groups of LLJ_GLDS_GROUPM row tiles sweep the columns together, m fastest inside. The 32 tiles
+  // that an XCD has in flight then read 4 row and 8 column panels; m fastest over all rows, up to 32 row panels and one (bf16
+  // 256 x 128, 3000 / 6000 / 8192 rows: 4096 -> 12288 280 / 627 / 948 -> 253 / 474 / 663 us, 11008 -> 4096 287 / 604 / 881 ->
+  // 243 / 419 / 585; 2048 rows, 8 row tiles: 55 -> 58 4096 -> 4096, so those stay)
+  if (!NFAST && LLJ_GLDS_GROUPM > 0 && mtiles > 8) {
     const int gm = LLJ_GLDS_GROUPM, grp = t / (gm * ntiles), first = grp * gm;
     const int rows = mtiles - first < gm ? mtiles - first : gm;
     const int in = t - grp * gm * ntiles;
@@ -1087,13 +1090,25 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
   const unsigned char* bf_lds = smem + NST * G::STAGE;
   const int ctile = CW == 8 ? w : 2 * w + (lane >> 5), cl = CW == 8 ? lane >> 1 : lane & 31, ccol = cl & 15,
             cs = cl >> 4, cg = CW == 8 ? 2 * (lane & 1) : 0;
-  float zoff = 0.f;  // 128 + zero of this lane's column
+  float zero = 0.f;  // of this lane's column (an integer)
   if constexpr (CVT) {
-    if (CW == 8 || w < 4) zoff = DUAL ? (ctile < 4 ? p.sz : p.sz2)[n0 + 16 * (ctile & 3) + ccol].y : p.sz[n0 + 16 * ctile + ccol].y;
+    if (CW == 8 || w < 4) zero = (DUAL ? (ctile < 4 ? p.sz : p.sz2)[n0 + 16 * (ctile & 3) + ccol].y : p.sz[n0 + 16 * ctile + ccol].y) - 128.f;
   }
-  // CW 8, split: the codes read issued before the chunk's fragment reads (asm, no wait; LDS reads
-  // complete in order, so the compiler's own lgkmcnt waits for the later fragment reads cover it, and
-  // the explicit wait below ties the value to it), the conversion after them, in the MFMAs' block
+  // One word of codes: the nibbles as fp8 (e4m3) bytes are q * 2^-9, denormals included, so one conversion with the scale 512
+  // makes two of them fp32; minus the zero and to a bf16 pair, both exact. 19 instructions a word (28 through bf16(128 + q),
+  // unpacked): they take the matrix cores' issue slots, 4096 rows 4096 -> 12288 392 / 382 us.
+  auto cvt8 = [&](uint32_t wv) {
+    const uint32_t ev = wv & 0x0F0F0F0Fu, od = (wv >> 4) & 0x0F0F0F0Fu;  // bytes: codes 0, 4, 1, 5 and 2, 6, 3, 7
+    const auto e0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(ev, 512.f, false), e1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(ev, 512.f, true);
+    const auto o0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(od, 512.f, false), o1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(od, 512.f, true);
+    auto pair = [&](float x, float y) {
+      return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y} - f32x2{zero, zero}, bf16x2_t));
+    };
+    return u32x4{pair(e0[0], e1[0]), pair(o0[0], o1[0]), pair(e0[1], e1[1]), pair(o0[1], o1[1])};
+  };
+  // CW 8, split: the codes read issued before the chunk's fragment reads (asm, no wait; LDS reads complete in order, so the
+  // compiler's own lgkmcnt waits for the later fragment reads cover it, and an explicit wait ties the value to it: FDB's counts
+  // the fragment reads behind it), the conversion after them, in the MFMAs' block
   auto cread = [&](int buf) {
     const uint32_t ra = (uint32_t)(uintptr_t)(lds_void_t*)(smem + (size_t)buf * G::STAGE + G::SA + 512 * ctile + 16 * cl +
                                                            4 * cg);
@@ -1103,20 +1118,11 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
     return t;
   };
   auto cfinish = [&](uint2 t, int slot) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(t));
+    if constexpr (!FDB) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(t));
     const uint32_t da = (uint32_t)(uintptr_t)(lds_void_t*)(bf_lds + (size_t)slot * BN * 128 + (16 * ctile + ccol) * 128);
 #pragma unroll
     for (int g4 = 0; g4 < 2; ++g4) {
-      const uint32_t wv = g4 ? t.y : t.x;
-      uint32_t o[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t d = and_or(wv >> (4 * e), msk, mag);  // bf16 pair (128 + q_lo, 128 + q_hi)
-        // as fp32 (exact), minus 128 + z in one packed add, back to a bf16 pair in one convert (exact)
-        const f32x2 v = f32x2{__uint_as_float(d << 16), __uint_as_float(d & 0xFFFF0000u)} - f32x2{zoff, zoff};
-        o[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-      }
-      const u32x4 ov = {o[0], o[1], o[2], o[3]};
+      const u32x4 ov = cvt8(g4 ? t.y : t.x);
       asm volatile("ds_write_b128 %0, %1" ::"v"(da + (((4 * cs + cg + g4) ^ ((ccol >> 1) & 7)) * 16)), "v"(ov) : "memory");
     }
   };
@@ -1140,17 +1146,9 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
     const uint32_t da = (uint32_t)(uintptr_t)(lds_void_t*)(bf_lds + (size_t)slot * BN * 128 + (16 * ctile + ccol) * 128);
 #pragma unroll
     for (int g4 = 0; g4 < NWD; ++g4) {
-      const uint32_t wv = wv4[g4];
-      uint32_t o[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t d = and_or(wv >> (4 * e), msk, mag);  // bf16 pair (128 + q_lo, 128 + q_hi)
-        const float lo = __uint_as_float(d << 16) - zoff, hi = __uint_as_float(d & 0xFFFF0000u) - zoff;
-        o[e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);  // exact: small integers
-      }
+      const u32x4 ov = cvt8(wv4[g4]);
       // (asm too: hipcc also waits vmcnt(0) before a plain LDS store while LDS-DMAs are in flight; the
       // loop's lgkmcnt(0) before its barrier retires it)
-      const u32x4 ov = {o[0], o[1], o[2], o[3]};
       asm volatile("ds_write_b128 %0, %1" ::"v"(da + (((4 * cs + cg + g4) ^ ((ccol >> 1) & 7)) * 16)), "v"(ov) : "memory");
     }
   };
@@ -1176,7 +1174,12 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
   // ---- K loop, fragment double buffering (LLJ_GLDS_FDB, bf16 and convert-once int4 at 256 x 128): the
   // fragments of chunk t + 1 are read from LDS while chunk t's MFMAs run (two register sets), so the DMA
   // runs three chunks ahead (every stage issued, past the end with a clamped chunk index: equal DMA
-  // counts per wave in every iteration) and each iteration waits for chunk t + 1 instead of t
+  // counts per wave in every iteration) and each iteration waits for chunk t + 1 instead of t.
+  // A wave issues in order, and the 8 waves' 128 fragment reads and 40 to 48 DMAs of a chunk take the LDS about as long as
+  // the 256 products take the matrix cores, so all three are interleaved by hand: one read per product, then the DMAs among
+  // the last products (int4: after them, beside the conversion). Reads and DMAs first, products after: a chunk 0.78 us with a
+  // quarter of the CUs and 0.93 with all (int4 0.93 and 0.95), so 0.58 and 0.82 (0.77 and 0.85); 512 rows 4096 -> 4096 bf16
+  // 50 -> 39 us, int4 59 -> 49; 2048 rows 62 -> 57 and 67 -> 61; 2048 rows 4096 -> 12288 190 -> 168 and 197 -> 175.
   if constexpr (FDB) {
     struct Fr {
       bf16x8 a0[MI], b0[NJ], a1[MI], b1[NJ];
@@ -1187,28 +1190,59 @@ __global__ __launch_bounds__(512, 1) void gemm_glds_kernel(GemmParams p) {
       frags(Ab, Bb, 0, f.a0, f.b0);
       frags(Ab, Bb, 1, f.a1, f.b1);
     };
+    int b0 = 0;  // stage of chunk t: t % 3
     auto step = [&](int t, Fr& cur, Fr& nxt) {
       wait_vm<G::NG>();  // chunk t + 1 (and the codes of t + 2) landed; t + 2 in flight
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of chunk t's fragments (and codes) are done
+      // this wave's reads of chunk t's fragments (and codes) and its tile writes are done: lgkmcnt(0), as a wait that the compiler
+      // counts -- in asm it put another of its own after the next chunk's reads, before the products, which then hid none of them
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_s_barrier();
-      const int b0 = t % 3;
-      stage(b0, t + 3 < KC ? t + 3 : KC - 1);
+      asm volatile("" ::: "memory");
+      const int buf = b0, tn = t + 3 < KC ? t + 3 : KC - 1;
       uint2 ct = {0u, 0u};
-      if constexpr (CVT) ct = cread(b0 + 2 >= 3 ? b0 - 1 : b0 + 2);  // codes of chunk t + 2
-      if (t + 1 < KC) rd(b0 + 1 == 3 ? 0 : b0 + 1, (t + 1) & 1, nxt);
-      mma(0, cur.a0, cur.b0);
-      mma(1, cur.a1, cur.b1);
-      if constexpr (CVT) cfinish(ct, t & 1);  // chunk t + 2's tile into chunk t's slot (read in the previous iteration)
-      // the MFMAs interleaved with the next chunk's fragment reads (LLJ_FDB_DSPM per MFMA) and the
-      // conversion's VALU (LLJ_W4Z_VPM per MFMA)
-      if constexpr ((CVT && LLJ_W4Z_IGLP) || LLJ_FDB_DSPM > 0) {
+      if constexpr (CVT) ct = cread(b0 == 0 ? 2 : b0 - 1);  // codes of chunk t + 2
+      b0 = b0 == 2 ? 0 : b0 + 1;
+      const unsigned char* Ab = smem + (size_t)b0 * G::STAGE;
+      const unsigned char* Bb = CVT ? bf_lds + (size_t)((t + 1) & 1) * BN * 128 : Ab + G::SA;
+      auto one = [&](int n) {  // product n of 2 MI NJ
+        const int i = n / NJ % MI, j = n % NJ;
+        acc[i][j] = n < MI * NJ ? mfma_bf16(cur.a0[i], cur.b0[j], acc[i][j]) : mfma_bf16(cur.a1[i], cur.b1[j], acc[i][j]);
+      };
+      auto next = [&](int n) {  // fragment read n of 2 (MI + NJ) of the next chunk (past the last chunk: unused)
+        const int st = n / (MI + NJ), f = n % (MI + NJ), so = ((4 * st + g) ^ sw) * 16;
+        if (f < MI) (st ? nxt.a1 : nxt.a0)[f] = *reinterpret_cast<const bf16x8*>(Ab + aoff0 + 16 * f * 128 + so);
+        else (st ? nxt.b1 : nxt.b0)[f - MI] = *reinterpret_cast<const bf16x8*>(Bb + brow_off(f - MI) + so);
+      };
+      constexpr int NR = 2 * (MI + NJ), NP = 2 * MI * NJ, N0 = CVT ? 6 : NR;
 #pragma unroll
-        for (int q = 0; q < 2 * MI * NJ; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if constexpr (LLJ_FDB_DSPM > 0) __builtin_amdgcn_sched_group_barrier(0x100, LLJ_FDB_DSPM, 0);
-          if constexpr (CVT && LLJ_W4Z_IGLP) __builtin_amdgcn_sched_group_barrier(0x002, LLJ_W4Z_VPM, 0);
-        }
+      for (int n = 0; n < N0; ++n) {
+        next(n);
+        one(n);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      // the codes: their read went out before these N0, which "memory" keeps before this wait
+      if constexpr (CVT) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(ct) : "n"(N0) : "memory");
+#pragma unroll
+      for (int n = N0; n < NP; ++n) {
+        if (n < NR) next(n);
+        one(n);
+      }
+      if (!CVT) stage(buf, tn);
+      if constexpr (CVT) cfinish(ct, t & 1);  // chunk t + 2's tile into chunk t's slot (read in the previous iteration)
+#pragma unroll
+      for (int n = N0; n < NR; ++n) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if constexpr (CVT) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+      }
+#pragma unroll
+      for (int n = 0; n < NP - NR; ++n) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (!CVT && n % 3 == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        if constexpr (CVT) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+      }
+      if (CVT) stage(buf, tn);
     };
     // prologue: chunks 0 and 1 (CVT: and chunk 0's codes, then both tiles converted) before chunk 2 is
     // staged -- chunk 2's group carries chunk 3's codes into stage buffer 0, over chunk 0's
