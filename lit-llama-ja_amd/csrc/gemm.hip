@@ -1,5 +1,7 @@
 // C-ABI entry points of the prefill GEMMs and their instantiations for the quantized weight formats
 // (device code: gemm_impl.h; bf16 weights: gemm_bf16.hip).
+#include <algorithm>
+
 #include "gemm_impl.h"
 
 namespace llj {
@@ -37,6 +39,10 @@ static int gemm_run(int wfmt, GemmParams& p, void* ws, size_t ws_bytes, void* st
   if (wfmt == GWF_W4) {
     if (!p.sz) return LLJ_EINVAL;
     if (zint && p.M >= 256 && w4z_enabled()) return gemm_glds_launch<GWF_W4Z, EP, 128>(p, s);
+    // 129 to 255 rows: one convert-once tile of 256 against two of 128, us at 160 / 255 rows: 4096 -> 12288 50 / 50 -> 41 / 44,
+    // 11008 -> 4096 45 / 50 -> 36 / 39, 4096 -> 4096 29 / 32 -> 30 / 32. Up to 128 rows one tile of 128 is the cheaper (64 rows 35, 32,
+    // 23 -> 37, 32, 24), and for short sums, whose pipeline fills and drains more often (2048 -> 5632, 255 rows 28 -> 30).
+    if (zint && p.M > kGBM && p.M < 256 && p.K >= 4096 && w4z_enabled()) return gemm_split_launch<GWF_W4Z, EP>(p, ws_bytes, s);
     if (p.M >= 256 && p.K % 128 == 0 && glds_enabled(GWF_W4)) return gemm_glds_run<GWF_W4, EP>(p, s);
     if (LLJ_GEMM_BM256_W4 && p.M >= 256) return gemm_launch<GWF_W4, EP, 256>(p, s);
     return gemm_split_launch<GWF_W4, EP>(p, ws_bytes, s);
@@ -106,7 +112,10 @@ size_t llj_gemm_resid_ws_bytes(int wfmt, int M, int N, int K) {
 }
 
 // Scratch of the _ws forms below 256 rows (0: they would not split K).
-size_t llj_gemm_ws_bytes(int wfmt, int M, int N, int K) { return gemm_split_bytes(wfmt & 0xff, M, N, K); }
+size_t llj_gemm_ws_bytes(int wfmt, int M, int N, int K) {
+  const size_t n = gemm_split_bytes(wfmt & 0xff, M, N, K);
+  return (wfmt & 0xff) == GWF_W4 ? std::max(n, gemm_split_bytes(GWF_W4Z, M, N, K)) : n;  // (enough for either form of int4)
+}
 
 // llj_gemm_resid with the K range split over workgroups (few row tiles): fp32 partials into ws
 // (llj_gemm_resid_ws_bytes), then one reduce launch adds them in slice order and the residual.

@@ -804,7 +804,8 @@ static inline bool glds_enabled(int wf) {
 // for 256 rows), us two of 128 -> one of 160 at 154 rows: 4096 -> 12288 gptq.int8 54 -> 43, int4 groups 53 -> 43; 11008 -> 4096
 // 47 -> 40, 47 -> 43; 4096 -> 4096 30 -> 28, 28 -> 27. int4 per row spills there and gains nothing (50 -> 49, 45 -> 43, 29 -> 32), nor
 // does a tile of 192 for more rows (one chunk in flight: gptq.int8 11008 -> 4096, 192 rows 47 -> 53).
-// bf16 takes one tile of 256 rows per 128 columns (gemm_glds_kernel; a chunk there is 0.7 us, one workgroup per CU) at any count of
+// bf16 takes one tile of 256 rows per 128 columns (gemm_glds_kernel; a chunk there is 0.7 us, one workgroup per CU; convert-once
+// int4, GWF_W4Z, 0.82) at any count of
 // rows: the register-staged tiles of 128 rows cost 1.85 a chunk, and split better to 42 / 53 / 90 us 4096 -> 12288 at 32 / 128 / 154
 // rows and 44 / 55 / 82 11008 -> 4096, 32 / 36 / 37 and 27 / 31 / 34 so.
 static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int* rows_out) {
@@ -812,11 +813,11 @@ static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int
   if (rows_out) *rows_out = kGBM;
   if (M >= 256 || M < 1 || N % kGBN || K < kGBK) return 1;
   const int KC = wf == GWF_I8 ? K / 128 : K / kGBK, planes = wf == GWF_I8 ? 1 : 0;
-  const bool dma = wf == GWF_BF16;
-  if (dma && !glds_enabled(wf)) return 1;
+  const bool dma = wf == GWF_BF16 || wf == GWF_W4Z;
+  if (wf == GWF_BF16 && !glds_enabled(wf)) return 1;
   const int rows = dma ? 256 : (wf == GWF_W8 || wf == GWF_W4G) && M > kGBM && M <= 160 ? 160 : kGBM;
   const long tiles = (long)((M + rows - 1) / rows) * (N / kGBN);
-  const double chunk = wf == GWF_W4 ? 0.75 : dma ? 0.7 : wf == GWF_I8 ? 1.7 : 1.2;
+  const double chunk = wf == GWF_W4 ? 0.75 : wf == GWF_W4Z ? 0.82 : dma ? 0.7 : wf == GWF_I8 ? 1.7 : 1.2;
   int best = 1, best_kcs = KC;
   double least = 0;
   for (int ns = LLJ_GSPLIT ? LLJ_GSPLIT : 1; ns <= (LLJ_GSPLIT ? LLJ_GSPLIT : 16); ++ns) {
@@ -1605,6 +1606,7 @@ static int gemm_split_launch(GemmParams p, size_t ws_bytes, hipStream_t s) {
   int kcs = 0, rows = kGBM;
   const int ns = p.ws ? gemm_split_plan(WF, p.M, p.N, p.K, &kcs, &rows) : 1;
   if (ns < 2 || ws_bytes < gemm_split_bytes(WF, p.M, p.N, p.K)) {
+    if constexpr (WF == GWF_W4Z) return gemm_glds_launch<WF, EP, 128>(p, s);
     if constexpr (WF == GWF_BF16)
       if (glds_enabled(WF)) return gemm_glds_run<WF, EP>(p, s);
     return gemm_launch<WF, EP>(p, s);
@@ -1612,7 +1614,7 @@ static int gemm_split_launch(GemmParams p, size_t ws_bytes, hipStream_t s) {
   p.nsplit = ns;
   p.kcs = kcs;
   int e;
-  if constexpr (WF == GWF_BF16)
+  if constexpr (WF == GWF_BF16 || WF == GWF_W4Z)
     e = gemm_glds_launch<WF, GEP_PARTIAL, 128>(p, s);
   else if constexpr (WF == GWF_W8 || WF == GWF_W4G)
     e = rows == 160 ? gemm_launch<WF, GEP_SPLIT, 160>(p, s) : gemm_launch<WF, GEP_SPLIT>(p, s);

@@ -154,7 +154,7 @@ def _gemm_fmt(wfmt: int) -> bool:
 
 # int4 prompt GEMMs of Linears whose zeros are all integers (GPTQ's round(-min / scale)): each chunk's
 # codes converted once per workgroup into an exact bf16 (q - z) tile, the scale in the epilogue
-# (LLJ_WF_ZINT; csrc/gemm.hip, the convert-once LDS-DMA kernel at M >= 256)
+# (LLJ_WF_ZINT; csrc/gemm.hip, the convert-once LDS-DMA kernel at M > 128)
 GEMM_ZINT = True
 # ... and c_fc1 / c_fc2 of such weights in one dual pass (llj_gemm_swiglu: one A tile for both, silu * mul
 # in the epilogue, no h round trip) at M >= 256

@@ -1434,6 +1434,32 @@ def test_gemm_w4z_exact_on_integer_rows(hip):
     np.testing.assert_array_equal(out.float().cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("M,N,K", [(128, 128, 4096), (129, 128, 4096), (129, 384, 3968), (200, 256, 4224), (255, 128, 11008)])
+def test_gemm_w4z_exact_below_256_rows(hip, M, N, K):
+    """int4 with integral zeros, tiles of 128 and of 256 rows, K whole and in slices: with small-integer activations every product
+    and fp32 partial sum is an integer below 2^24 (128 + q codes: 4 * 143 * 11008 < 2^23), so the result is bitwise
+    bf16(s * sum_k a (q - z)); the scales are powers of two, as K slices add s * their sums."""
+    rng = np.random.default_rng(M + K)
+    qw, sc, z = rand_w4(rng, N, K)
+    sc = np.exp2(np.round(np.log2(sc)))
+    Wd, szd = repack(hip, qw), sz_of(hip, sc, z)
+    a = rng.integers(-4, 5, size=(M, K)).astype(np.float32)
+    x = T(a, torch.bfloat16)
+    codes = np.empty((N, K), dtype=np.int64)
+    codes[:, 0::2] = qw & 15
+    codes[:, 1::2] = qw >> 4
+    want = bf16(sc.reshape(1, N) * (a.astype(np.int64) @ (codes - z.astype(np.int64)).T).astype(np.float32))
+    n = hip.llj_gemm_ws_bytes(0, M, N, K)
+    assert n == hip.llj_gemm_ws_bytes(ZINT4, M, N, K) > 0
+    scr = torch.empty(n, dtype=torch.uint8, device=dev)
+    for ws in (None, scr.data_ptr()):
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+        call(hip, "llj_gemm_linear_ws", ZINT4, x.data_ptr(), K, Wd.data_ptr(), szd.data_ptr(), out.data_ptr(), N, M, N, K, ws,
+             n if ws else 0, st())
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.float().cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 128, 128), (17, 128, 384), (64, 256, 640), (129, 384, 4224), (255, 128, 2176)])
 def test_gemm_bf16_exact_below_256_rows(hip, M, N, K):
     """Small integers: every product and fp32 partial sum is an integer below 2^24, whole or in K slices, so the product is
