@@ -134,8 +134,8 @@ __device__ __forceinline__ float gptq_columns(const float* hs, const float (*dia
 // (DPP), which all form its code and error (identical inputs, identical fp32 ops) and then update their own columns. Every
 // column receives the updates in the reference's order, so results are its bit for bit.
 //
-// Bound: the chain of dependent instructions of a column, two divisions in it, times 128. A lone wave on a SIMD issues one instruction every 7 to
-// 8 cycles whether it depends on the last or not, so their number counts: 570 a group of 16 columns (890 with a row's 16 columns in every
+// Bound: the chain of dependent instructions of a column, two divisions in it, times 128. A lone wave on a SIMD issues an independent
+// instruction every 4.75 cycles and one that waits for the last every 8.1, so length and number both count: 570 a group of 16 columns (890 with a row's 16 columns in every
 // lane's registers: 23.6 us at N = 4096; interleaving those updates with the chain, or Hinv1's values a step ahead: no faster). 16 rows put
 // N = 4096 on all 256 CUs, one wave per SIMD; above, more rows to a workgroup share Hinv1. us a block with the rows in LDS, Hinv1 waited for
 // column by column, and now: N = 256 33 and 17, 4096 35 and 19, 8192 38 and 21, 11008 54 and 31, 35008 171 and 88 (a block with an error out
