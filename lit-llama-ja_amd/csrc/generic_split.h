@@ -19,7 +19,8 @@
 // Up to kGgFineK without K ranges the sums of K's halves are kept apart from 8 tiles on (the second half starts at the same sign).
 //
 // A value that is not finite, or rounds to infinity, spoils its outputs' other parts: outputs that are not finite are formed again on the
-// fp32 matrix cores at the end.
+// fp32 matrix cores at the end, a row of tiles at a time, in chains of 8 values, their pairs and eights (K = 4096 in one piece 1.16e-7 against
+// 1.15e-6 in one chain, 1.40e-7 in the fp32 products before; K = 780 9.6e-8 against 5.0e-7).
 //
 // Bound: the bf16 rate at the clock that it sustains (about 1.3 PFLOP/s, 217 TFLOP/s in sixths); below some 40 rows the weights' bytes. us before
 // (v_mfma_f32_32x32x2_f32) and now: 301 rows 4096 -> 12288 268, 186 (163 TFLOP/s), 4096 -> 4096 101, 69, 11008 -> 4096 252, 161, 2048 rows 4096 -> 4096 539,
@@ -176,37 +177,44 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
     if (hi < t1) flush();
   }
 
-  bool bad = false;
+  flush();
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int i = 0; i < MI; ++i) {
+    uint32_t bad = 0;  // a bit an output
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      tot[i][j] += mid[i][j];
-      mid[i][j] = f32x4{};
+    for (int u = 0; u < 8; ++u) bad |= fabsf(tot[i][u >> 2][u & 3]) < INFINITY ? 0u : 1u << u;
+    if (!__any(bad != 0)) continue;
+    // 8 values a chain, four of those in pairs, eight of these, and the rest: no further from float64 than the fp32 sums of gg_kernel
+    const float* row = x + (size_t)min(m0 + 16 * i + r, M - 1) * ldx;
+    const int k0 = t0 * kGsKT, k1 = min(t1 * kGsKT, K);
+    f32x4 part8[2] = {}, sum[2] = {};
+    for (int k = k0; k < k1; k += 32) {
+      f32x4 s[2][4] = {};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) bad = bad || !(fabsf(tot[i][j][e]) < INFINITY);
-    }
-  if (__any(bad)) {
-    for (int k = t0 * kGsKT; k < min(t1 * kGsKT, K); k += 16) {
-      f32x4 w[2];
+      for (int h = 0; h < 2; ++h) {
+        const int kh = k + 16 * h;
+        const f32x4 a = gs_ld<LD, true>(row, kh + 4 * g, kh + 16, K);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) w[j] = gs_ld<LD, true>(wr[j], k + 4 * g, k + 16, K);
+        for (int j = 0; j < 2; ++j) {
+          const f32x4 w = gs_ld<LD, true>(wr[j], kh + 4 * g, kh + 16, K);
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        const f32x4 a = gs_ld<LD, true>(x + (size_t)min(m0 + 16 * i + r, M - 1) * ldx, k + 4 * g, k + 16, K);
+          for (int e = 0; e < 4; ++e) {
+            f32x4& c = s[j][2 * h + (e >> 1)];
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], w[e], c, 0, 0, 0);
+          }
+        }
+      }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) mid[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], w[j][e], mid[i][j], 0, 0, 0);
+      for (int j = 0; j < 2; ++j) {
+        part8[j] += (s[j][0] + s[j][1]) + (s[j][2] + s[j][3]);
+        if (((k - k0) & 224) == 224 || k + 32 >= k1) {
+          sum[j] += part8[j];
+          part8[j] = f32x4{};
+        }
       }
     }
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (!(fabsf(tot[i][j][e]) < INFINITY)) tot[i][j][e] = mid[i][j][e];
+    for (int u = 0; u < 8; ++u) tot[i][u >> 2][u & 3] = bad >> u & 1 ? sum[u >> 2][u & 3] : tot[i][u >> 2][u & 3];
   }
 #pragma unroll
   for (int i = 0; i < MI; ++i)

@@ -378,6 +378,51 @@ def test_generic_gemm_fp32_sums_and_values_out_of_range(M, N, K, off):
     assert safe[0, :7].all() and ((got - want).abs()[safe] <= lim[safe]).all()
 
 
+# (rows, columns, K, K ranges): tiles of 16, 32 .. 96 rows in this order, then K in one piece (its halves kept apart at 780), then longer sums. The
+# ranges are asserted: a plan that chooses others has other heights as well, and shapes for it are to be looked for
+GEMM_HEIGHTS = [(9, 260, 800, 13), (9, 260, 780, 13), (33, 1100, 800, 13), (33, 1100, 780, 13), (33, 4100, 800, 9), (33, 4100, 780, 9),
+                (100, 6000, 800, 5), (100, 6000, 780, 5), (65, 11008, 800, 5), (65, 11008, 780, 5), (384, 2304, 800, 5), (384, 2304, 780, 5),
+                (70, 12288, 780, 1), (301, 11008, 800, 1), (301, 12288, 4096, 1), (301, 4096, 4096, 4), (90, 8200, 3108, 7)]
+
+
+def _gemm_heights_operands(M, N, K, ranges, off):
+    """fp32 x (M, K), `off` elements past an aligned address, w (N, K), a call of their product."""
+    from lit_llama import _hip
+
+    assert _hip.lib().llj_g_linear_ws_bytes(1, M, N, K, 1) == (ranges * M * N * 4 if ranges > 1 else 0)
+    g = torch.Generator("cuda").manual_seed(M + N + K)
+    x = torch.randn(M * K + 1, device="cuda", generator=g)[off:off + M * K].view(M, K)
+    w = torch.randn(N, K, device="cuda", generator=g)
+
+    def product():
+        y = torch.full((M, N), math.nan, device="cuda")
+        _hip.g_linear(1, x, M, K, w, None, None, 16, K, N, y, None, 1, _hip.stream())
+        return y.double()
+
+    return x, w, product
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("M,N,K,ranges", GEMM_HEIGHTS)
+def test_generic_gemm_fp32_outputs_formed_again(M, N, K, ranges, off):
+    """Finite values that bf16 parts cannot hold (3.4e38, times weights of 1e-38, and the other way round) and infinities, the last one in
+    W's last element (whose place past K is read with x's zeros). Bound of the finite outputs in the 2-norm: random roundings of 2^-24 / sqrt(3), for
+    the 8 values of a chain 4.5 of them, the pairs 2, eight of these 4.5 and the rest of K / 256 half as many."""
+    x, w, product = _gemm_heights_operands(M, N, K, ranges, off)
+    x[::2, 3], w[::3, K - 2] = 3.4e38, -3.4e38
+    w[:, 3], x[:, K - 2] = 1.2e-38 * torch.sign(w[:, 3]), 1.2e-38 * torch.sign(x[:, K - 2])
+    bound = 2.0 ** -24 / 3 ** 0.5 * (11 + (K / 256 + 1) / 2) ** 0.5
+    for step in range(2):
+        want, got = x.double() @ w.double().T, product()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+        for rows, cols in ((slice(0, None, 2), slice(None)), (slice(1, None, 2), slice(0, None, 3)), (slice(1, None, 2), slice(1, None, 3))):
+            a, b = got[rows, cols], want[rows, cols]
+            fin = torch.isfinite(b)
+            assert fin.all() if step == 0 else fin.any()
+            assert (((a - b)[fin].norm() / b[fin].norm()).item()) < bound
+        x[1, 0], x[2, 7], w[5, K - 1] = math.nan, -math.inf, math.inf
+
+
 # ---- up to 8 rows (generic_rows.h)
 @pytest.mark.parametrize("dt", [0, 1])
 @pytest.mark.parametrize("M", [1, 3, 8])
