@@ -14,13 +14,16 @@
 // a sum of products towards minus infinity, which would add up over K (a mean error of 0.6 of its deviation at K = 4096, 0.73 at 11008), so
 // every other tile is formed with -x and subtracted. Error against float64 in the 2-norm, random operands (fp32 MFMA before): 7.7e-8 at K = 780
 // (9.1e-8), 1.03e-7 at 4096 in one piece and 8.8e-8 in four (1.40e-7, 1.32e-7 in three), 1.01e-7 at 11008 in four (1.36e-7 in eight).
-// Values below 2^-109 keep fewer bits (their lowest parts are below bf16's range).
+// Both operands are multiplied by 2^24 before they are split and the sums by 2^-48 at the end: the lowest part of any fp32 value, the smallest
+// denormal's included, is then a normal bf16 number, and no part of a product falls below fp32's range (unscaled, rows of 1e-35 were 2.7e-6 from
+// float64, rows of 1e-37 2.6e-4; scaled 1.03e-7 as at any size). Sums past 2^79 and values past 2^103 leave the range at the other end and are
+// formed again as below. It costs an instruction a value: 301 rows 4096 -> 12288 216 us and 220, 11008 -> 4096 170 and 177, 780 -> 2048 the same.
 //
 // Up to kGgFineK without K ranges the sums of K's halves are kept apart from 8 tiles on (the second half starts at the same sign).
 //
 // A value that is not finite, or rounds to infinity, spoils its outputs' other parts: outputs that are not finite are formed again on the
-// fp32 matrix cores at the end, a row of tiles at a time, in chains of 8 values, their pairs and eights (K = 4096 in one piece 1.16e-7 against
-// 1.15e-6 in one chain, 1.40e-7 in the fp32 products before; K = 780 9.6e-8 against 5.0e-7).
+// fp32 matrix cores at the end, a row of tiles at a time, in chains of 4 values, their pairs up to two tiles, and fours (K = 4096 in one piece 1.10e-7 against
+// 1.15e-6 in one chain, 1.40e-7 in the fp32 products before; K = 780 8.9e-8, 5.0e-7 and 9.1e-8).
 //
 // Bound: the bf16 rate at the clock that it sustains (about 1.3 PFLOP/s, 217 TFLOP/s in sixths); below some 40 rows the weights' bytes. us before
 // (v_mfma_f32_32x32x2_f32) and now: 301 rows 4096 -> 12288 268, 186 (163 TFLOP/s), 4096 -> 4096 101, 69, 11008 -> 4096 252, 161, 2048 rows 4096 -> 4096 539,
@@ -32,6 +35,7 @@
 namespace llj {
 
 constexpr int kGsBN = 128, kGsKT = 32, kGsMostMI = 6;
+constexpr float kGsUp = 0x1p24f, kGsDown = 0x1p-48f;  // of both operands before they are split, of the sums
 
 // two fp32 values as three pairs of bf16
 __device__ __forceinline__ void gs_split(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
@@ -109,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
     for (int j = 0; j < JX; ++j)
       if (mine(j)) {
         uint2 p0, p1, p2;
-        const f32x4 v = negative ? -xv[j] : xv[j];
+        const f32x4 v = xv[j] * (negative ? -kGsUp : kGsUp);
         gs_split(v[0], v[1], p0.x, p1.x, p2.x);
         gs_split(v[2], v[3], p0.y, p1.y, p2.y);
         *reinterpret_cast<uint2*>(b + xo[j]) = p0;
@@ -129,6 +133,8 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
     uint4 w[2][3];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
+      wv[j][0] *= kGsUp;
+      wv[j][1] *= kGsUp;
       gs_split(wv[j][0][0], wv[j][0][1], w[j][0].x, w[j][1].x, w[j][2].x);
       gs_split(wv[j][0][2], wv[j][0][3], w[j][0].y, w[j][1].y, w[j][2].y);
       gs_split(wv[j][1][0], wv[j][1][1], w[j][0].z, w[j][1].z, w[j][2].z);
@@ -182,14 +188,17 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
   for (int i = 0; i < MI; ++i) {
     uint32_t bad = 0;  // a bit an output
 #pragma unroll
-    for (int u = 0; u < 8; ++u) bad |= fabsf(tot[i][u >> 2][u & 3]) < INFINITY ? 0u : 1u << u;
+    for (int u = 0; u < 8; ++u) {
+      bad |= fabsf(tot[i][u >> 2][u & 3]) < INFINITY ? 0u : 1u << u;
+      tot[i][u >> 2][u & 3] *= kGsDown;
+    }
     if (!__any(bad != 0)) continue;
-    // 8 values a chain, four of those in pairs, eight of these, and the rest: no further from float64 than the fp32 sums of gg_kernel
+    // 4 values a chain, pairs of those to two tiles, four of these, and the rest: no further from float64 than the fp32 sums of gg_kernel
     const float* row = x + (size_t)min(m0 + 16 * i + r, M - 1) * ldx;
     const int k0 = t0 * kGsKT, k1 = min(t1 * kGsKT, K);
-    f32x4 part8[2] = {}, sum[2] = {};
+    f32x4 held[2] = {}, part8[2] = {}, sum[2] = {};
     for (int k = k0; k < k1; k += 32) {
-      f32x4 s[2][4] = {};
+      f32x4 tile[2] = {};
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int kh = k + 16 * h;
@@ -197,17 +206,19 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const f32x4 w = gs_ld<LD, true>(wr[j], kh + 4 * g, kh + 16, K);
+          f32x4 s[4] = {};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            f32x4& c = s[j][2 * h + (e >> 1)];
-            c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], w[e], c, 0, 0, 0);
-          }
+          for (int e = 0; e < 4; ++e) s[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], w[e], s[e], 0, 0, 0);
+          tile[j] += (s[0] + s[1]) + (s[2] + s[3]);
         }
       }
+      const bool second = (k - k0) & 32, last = k + 32 >= k1;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        part8[j] += (s[j][0] + s[j][1]) + (s[j][2] + s[j][3]);
-        if (((k - k0) & 224) == 224 || k + 32 >= k1) {
+        if (second) part8[j] += held[j] + tile[j];
+        else if (last) part8[j] += tile[j];
+        held[j] = tile[j];
+        if (((k - k0) & 224) == 224 || last) {
           sum[j] += part8[j];
           part8[j] = f32x4{};
         }

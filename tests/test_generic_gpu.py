@@ -423,6 +423,19 @@ def test_generic_gemm_fp32_outputs_formed_again(M, N, K, ranges, off):
         x[1, 0], x[2, 7], w[5, K - 1] = math.nan, -math.inf, math.inf
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("M,N,K,ranges", GEMM_HEIGHTS)
+def test_generic_gemm_fp32_small_values(M, N, K, ranges, off):
+    """Operands down to fp32's smallest: as near to float64 as ordinary ones (the 2-norm of half an ulp for the result and one for the sums of a tile,
+    of eight and of the rest)."""
+    x, w, product = _gemm_heights_operands(M, N, K, ranges, off)
+    x0, w0 = x.clone(), w.clone()
+    for a, b in ((1.0, 1.0), (1e-34, 1.0), (1e-36, 1.0), (1.0, 1e-37), (1e-18, 1e-18), (1e-41, 1e11), (1e12, 1e-42)):
+        x.copy_(x0 * a), w.copy_(w0 * b)
+        want = x.double() @ w.double().T
+        assert ((product() - want).norm() / want.norm()).item() < 2.0 ** -24 * (0.5 + 3 * 0.5), (a, b)
+
+
 # ---- up to 8 rows (generic_rows.h)
 @pytest.mark.parametrize("dt", [0, 1])
 @pytest.mark.parametrize("M", [1, 3, 8])
