@@ -78,9 +78,14 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
   __shared__ __align__(16) char lds[2][3 * PL];
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), g = lane >> 4, r = lane & 15;
   const int mt = (M + BM - 1) / BM, cols = (N + kGsBN - 1) / kGsBN, local = blockIdx.x >> 3;
-  const int nt = cols < 8 ? (int)blockIdx.x / mt : (int)(blockIdx.x & 7) + 8 * (local / mt);
+  int nt = (int)(blockIdx.x & 7) + 8 * (local / mt), mb = local % mt;
+  if (cols < 8) {  // (gs_launch: tile by tile, or all on one XCD)
+    const int b = (int)gridDim.x == cols * mt ? (int)blockIdx.x : blockIdx.x & 7 ? cols * mt : local;
+    nt = b / mt;
+    mb = b % mt;
+  }
   if (nt >= cols) return;
-  const int m0 = (cols < 8 ? (int)blockIdx.x % mt : local % mt) * BM, n0 = nt * kGsBN + wave * 32;
+  const int m0 = mb * BM, n0 = nt * kGsBN + wave * 32;
   const int t0 = blockIdx.y * split_tiles, t1 = min((K + kGsKT - 1) / kGsKT, t0 + split_tiles);
 
   const float *xr[JX], *wr[2];
@@ -124,10 +129,12 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
 
   f32x4 mid[MI][2] = {}, tot[MI][2] = {};
   const int ra = r * 64 + ((g ^ (r >> 2)) << 4);
+  // past the last tile: its own elements again, not used; not at all where they may be single elements, each as many requests as 16 bytes
+  auto wanted = [&](int t) { return LD != 0 || t < t1; };
   fetch_x(t0);
+  fetch_w(t0);  // (before x is waited for)
   stage_x(t0, false);
-  fetch_w(t0);
-  fetch_x(min(t0 + 1, t1 - 1));
+  if (wanted(t0 + 1)) fetch_x(min(t0 + 1, t1 - 1));
   auto step = [&](int t, bool negative, bool next) {  // the signs of tile t and the next one (constants at every call)
     asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");  // tile t is staged, and every wave is done with the other buffer
     uint4 w[2][3];
@@ -140,9 +147,9 @@ __global__ __launch_bounds__(256, 2) void gs_kernel(const float* __restrict__ x,
       gs_split(wv[j][1][0], wv[j][1][1], w[j][0].z, w[j][1].z, w[j][2].z);
       gs_split(wv[j][1][2], wv[j][1][3], w[j][0].w, w[j][1].w, w[j][2].w);
     }
-    fetch_w(min(t + 1, t1 - 1));
+    if (wanted(t + 1)) fetch_w(min(t + 1, t1 - 1));
     if (t + 1 < t1) stage_x(t + 1, next);
-    fetch_x(min(t + 2, t1 - 1));
+    if (wanted(t + 2)) fetch_x(min(t + 2, t1 - 1));
     const char* b = lds[(t - t0) & 1] + ra;
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -274,7 +281,11 @@ inline bool gs_takes(int wkind, int dt) { return wkind == 1 && dt == 1; }
 inline int gs_launch(GsPlan p, const float* x, int ldx, int M, int K, const float* W, int N, float* y, int ldy, const float* resid, int ldr, float* part,
                      hipStream_t s) {
   const int mt = (M + 16 * p.mi - 1) / (16 * p.mi), nt = (N + kGsBN - 1) / kGsBN, all = (K + kGsKT - 1) / kGsKT, per = (all + p.splits - 1) / p.splits;
-  const long blocks = nt < 8 ? (long)nt * mt : (long)((nt + 7) / 8) * 8 * mt;
+  // below eight column tiles: tile by tile over the XCDs; an output of one workgroup of gg_reduce_kernel, where the parts' workgroups find a CU
+  // each on that one's XCD, there: its L2 then holds the parts (both launches: 29 rows 512 -> 1, 16 ranges 8.2 us tile by tile and 5.8; with more
+  // workgroups than CUs, 232 rows 2304 -> 1, 10.7 and 16.7)
+  const bool one = nt < 8 && p.splits > 1 && (long)M * N <= 256 && (long)nt * mt * p.splits <= 32;
+  const long blocks = one ? 8L * nt * mt : nt < 8 ? (long)nt * mt : (long)((nt + 7) / 8) * 8 * mt;
   LLJ_REQUIRE(blocks < (1L << 31));
   const dim3 grid((unsigned)blocks, p.splits);
   const bool vec = K % 4 == 0 && ldx % 4 == 0 && (((uintptr_t)x | (uintptr_t)W) & 15) == 0;

@@ -436,6 +436,30 @@ def test_generic_gemm_fp32_small_values(M, N, K, ranges, off):
         assert ((product() - want).norm() / want.norm()).item() < 2.0 ** -24 * (0.5 + 3 * 0.5), (a, b)
 
 
+@pytest.mark.parametrize("M,N,K", [(29, 1, 512), (10, 8, 512), (256, 1, 700), (128, 2, 4096), (18, 14, 3109), (15, 17, 1030), (13, 20, 310), (9, 28, 96),
+                                   (64, 130, 17), (70, 300, 1), (33, 129, 63)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_generic_gemm_fp32_small_outputs(M, N, K, off):
+    """K in ranges of one tile and of several whose sums fit one workgroup of the second launch (all on its XCD: up to 256 outputs) and just do not, and
+    K of a tile's part, whole and one more; the residual in place, nothing outside the output. Bound as in the first test."""
+    from lit_llama import _hip
+
+    g = torch.Generator("cuda").manual_seed(M + N + K)
+    x = torch.randn(M * K + 1, device="cuda", generator=g)[off:off + M * K].view(M, K)
+    w, res = torch.randn(N, K, device="cuda", generator=g), torch.randn(M, N, device="cuda", generator=g)
+    want, mass = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    lim = mass * 2.0 ** -24 * (32 + 8 + K // 128 + 16 + 4)
+    for resid in (False, True):
+        buf = torch.full((M + 1, N + 3), 7.0, device="cuda")
+        y = buf[:M, :N]
+        if resid:
+            y.copy_(res)
+        _hip.g_linear(1, x, M, K, w, None, None, 16, K, N, y, y if resid else None, 1, _hip.stream())
+        ref = want + res.double() if resid else want
+        assert ((y.double() - ref).abs() <= lim + (2.0 ** -24 * ref.abs() if resid else 0.0)).all()
+        assert (buf[M] == 7.0).all() and (buf[:M, N:] == 7.0).all()
+
+
 # ---- up to 8 rows (generic_rows.h)
 @pytest.mark.parametrize("dt", [0, 1])
 @pytest.mark.parametrize("M", [1, 3, 8])
