@@ -223,8 +223,8 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logi
     const float4 f = reinterpret_cast<const float4*>(sv)[q];
     top = fmaxf(fmaxf(top, fmaxf(f.x, f.y)), fmaxf(f.z, f.w));
   }
+  int bi = 0x7fffffff;
   if (mx == top) {
-    int bi = 0x7fffffff;
     if (vec) {
       for (int v0 = tid; v0 < nv && bi == 0x7fffffff; v0 += 4 * 1024) {
         if (nv > 4 * 1024) fetch(v0);  // (else the row is still in registers)
@@ -243,13 +243,20 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logi
       for (int v = tid; v < V && bi == 0x7fffffff; v += 1024)
         if (ldv(lr, v) == top) bi = v;
     }
-    if (bi != 0x7fffffff) atomicMin(&first, bi);
+  }
+  if (__any(bi != 0x7fffffff)) {  // (an atomic a lane is a turn a lane: where many hold the maximum, one of 16)
+    auto take_first = [&](uint32_t other) { bi = min(bi, (int)other); };
+    take_first(dpp_u32<kDppHalfMirror>(bi));
+    take_first(dpp_u32<kDppRowMirror>(bi));
+    take_first(dpp_u32<kDppXor1>(bi));
+    take_first(dpp_u32<kDppXor2>(bi));
+    if ((tid & 15) == 0 && bi != 0x7fffffff) atomicMin(&first, bi);
   }
   __syncthreads();
   if (tid == 0) {
-    const int bi = first == 0x7fffffff ? 0 : first;  // all-NaN row: 0
-    out_idx[m] = bi;
-    if (tokens_out) tokens_out[(size_t)m * tok_stride + at] = bi;
+    const int chosen = first == 0x7fffffff ? 0 : first;  // all-NaN row: 0
+    out_idx[m] = chosen;
+    if (tokens_out) tokens_out[(size_t)m * tok_stride + at] = chosen;
   }
 }
 

@@ -411,6 +411,22 @@ def test_argmax_ties_and_values_out_of_range(hip, V):
         np.testing.assert_array_equal(out.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("V", [1, 63, 250, 1000, 4100, 32000, 70001])
+def test_argmax_maximum_held_by_many(hip, V):
+    """The largest value in every place, in half of them, in the last 40 and in single lanes of every row of lanes: the lowest index."""
+    rng = np.random.default_rng(V)
+    every, half, last, lanes = (np.full(V, x, dtype=np.float32) for x in (0.5, -2.0, -2.0, -2.0))
+    half[rng.random(V) < 0.5] = 3.0
+    last[-40:] = 3.0
+    lanes[min(V - 1, 5)::16] = 3.0
+    L = np.stack([every, half, last, lanes])
+    for name, t in (("llj_argmax", T(L, torch.bfloat16)), ("llj_g_argmax", T(L))):
+        out = torch.full((4,), -1, dtype=torch.int32, device=dev)
+        call(hip, name, t.data_ptr(), V, 4, V, out.data_ptr(), None, 0, None, st())
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), L.argmax(1))
+
+
 def test_argmax_and_advance(hip):
     rng = np.random.default_rng(3)
     V, M = 32000, 8
