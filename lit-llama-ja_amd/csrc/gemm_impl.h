@@ -832,6 +832,9 @@ static inline int gemm_split_plan(int wf, int M, int N, int K, int* kcs_out, int
   if (wf == GWF_BF16 && !glds_enabled(wf)) return 1;
   const int rows = dma ? 256 : (wf == GWF_W8 || wf == GWF_W4G) && M > kGBM && M <= 160 ? 160 : kGBM;
   const long tiles = (long)((M + rows - 1) / rows) * (N / kGBN);
+  // more tiles than CUs: the parts of the whole output cost more than what a part-filled last round does (130 rows 4096 -> 33024, whole / 4 slices
+  // 102 / 126 us, int4's two tiles of 128 rows 111; 255 rows 8192 -> 40960 214 / 231)
+  if (wf == GWF_W4Z && tiles > 256) return 1;
   const double chunk = wf == GWF_W4 ? 0.75 : wf == GWF_W4Z ? 0.82 : dma ? 0.7 : wf == GWF_I8 ? 1.7 : 1.2;
   int best = 1, best_kcs = KC;
   double least = 0;

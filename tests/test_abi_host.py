@@ -71,6 +71,18 @@ def test_library_exports_every_header_symbol():
     assert not missing, f"declared but not exported: {sorted(missing)}"
 
 
+def test_wide_int4_prompt_products_are_not_split():
+    """int4 with integral zeros, 129 to 255 rows: K slices up to a tile per CU (256 columns of 128), none past that."""
+    from lit_llama import _hip
+
+    L = ctypes.CDLL(str(_lib_path()))
+    f = L.llj_gemm_ws_bytes
+    f.argtypes, f.restype = [ctypes.c_int] * 4, ctypes.c_size_t
+    assert f(_hip.WF_ZINT, 130, 12288, 4096) > 0
+    for M, N, K in ((130, 33024, 4096), (255, 33024, 4096), (192, 40960, 8192), (255, 49152, 8192)):
+        assert f(_hip.WF_ZINT, M, N, K) == 0
+
+
 def test_library_loads_and_binds_without_gpu():
     L = ctypes.CDLL(str(_lib_path()))
     for name in _header_decls():
