@@ -311,12 +311,15 @@ def test_generic_gemm_edges_vs_float64(kind, bits, group, dt, M, N, K, pad, off)
 @pytest.mark.parametrize("M,N,K,pad,ws", [
     (9, 1, 3104, 0, True), (9, 129, 3104, 4, False), (64, 128, 4096, 0, True), (65, 129, 3104, 12, True), (65, 780, 4096, 0, False),
     (301, 1000, 3104, 0, True), (37, 12288, 4096, 0, True), (301, 13200, 3104, 4, False), (513, 11000, 3104, 0, False),
-    (64, 16500, 3072, 0, False), (70, 256, 32 * 113, 0, True), (1000, 7900, 3104, 0, False), (301, 5000, 3104, 4, True)])
+    (64, 16500, 3072, 0, False), (70, 256, 32 * 113, 0, True), (1000, 7900, 3104, 0, False), (301, 5000, 3104, 4, True),
+    (33, 1100, 800, 0, True), (33, 4100, 780, 4, True), (100, 6000, 780, 0, True), (65, 11008, 800, 4, True), (384, 2304, 780, 0, True),
+    (301, 4096, 4100, 0, True), (90, 8200, 3108, 0, True), (70, 12288, 780, 0, False), (40, 500, 288, 0, False), (20, 2000, 260, 8, False),
+    (9, 1100, 36, 0, False)])
 def test_generic_gemm_direct_tiles_equal_staged_ones(M, N, K, pad, ws):
-    """fp32 rows above K = 3,071 in whole tiles, brought to LDS without registers, against the same product through registers (x one
-    element off the alignment): the same sums bit for bit, with and without the residual in place. One workgroup and several rounds,
-    both buffer counts (the last two shapes take three), column and row remainders, padded rows, split K (32 x 113: splits of unequal
-    length), no split."""
+    """fp32 rows in 16-byte loads (K a multiple of 32, and of 4 alone) against the same product in loads from any element on (x one element off the
+    alignment): the same sums bit for bit, with and without the residual in place. Tiles of every height, fewer than eight column tiles and
+    more, column and row remainders, padded rows, K in ranges (32 x 113: of unequal length), in one piece and in halves, one tile, odd and even
+    counts of them."""
     from lit_llama import _hip
 
     g = torch.Generator("cuda").manual_seed(M + N + K)
@@ -348,10 +351,10 @@ def test_generic_gemm_direct_tiles_equal_staged_ones(M, N, K, pad, ws):
 @pytest.mark.parametrize("M", [9, 17, 40, 64, 80, 96, 100])
 @pytest.mark.parametrize("N,K,off", [(260, 3104, 0), (260, 3104, 1), (1200, 1028, 0), (130, 775, 1), (9, 40, 0)])
 def test_generic_gemm_fp32_sums_and_values_out_of_range(M, N, K, off):
-    """fp32 products as sums of bf16 ones, every height of a tile, all three kinds of loads. Rows of ordinary values are as near to float64 as fp32 sums
-    (the 2-norm of half an ulp for the result and one for the sums of a tile, of eight and of the rest); infinities, NaN, values that round to
-    infinity in bf16 and very small ones give what fp32 sums give: non-finite outputs where float64 has them, the bound of the tests above where no
-    partial sum can overflow."""
+    """fp32 products as sums of bf16 ones, all three kinds of loads (every height of a tile: the tests below). Rows of ordinary values are as near to
+    float64 as fp32 sums (the 2-norm of half an ulp for the result and one for the sums of a tile, of eight and of the rest); infinities, NaN, values that
+    round to infinity in bf16, large and very small ones give what fp32 sums give: non-finite outputs where float64 has them, the bound of the tests
+    above where no partial sum can overflow."""
     from lit_llama import _hip
 
     g = torch.Generator("cuda").manual_seed(M + N + K)
@@ -366,16 +369,15 @@ def test_generic_gemm_fp32_sums_and_values_out_of_range(M, N, K, off):
     want = x.double() @ w.double().T
     assert ((product() - want).norm() / want.norm()).item() < 2.0 ** -24 * (0.5 + 3 * 0.5)
     x[1, 5], x[2, 7], x[3, K - 1], w[7, 5], w[8, 3] = math.inf, -math.inf, math.nan, 0.0, math.inf
-    x[4] *= 1e37
-    x[5, ::2] = 3.4e38  # above bf16's largest
+    x[4] *= 1e34
+    x[5, 2], w[:, 2] = 3.4e38, 1.2e-38 * torch.sign(w[:, 2])  # above bf16's largest, the products 4
     x[6] *= 1e-30
     want, mass = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
     got = product()
-    rows = [0, 1, 2, 3, 6, 7, 8]
-    assert torch.equal(torch.isnan(got[rows]), torch.isnan(want[rows])) and torch.equal(torch.isinf(got[rows]), torch.isinf(want[rows]))
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
     safe = mass < 1e38
     lim = mass * 2.0 ** -24 * (32 + 8 + K // 128 + 16 + 4)
-    assert safe[0, :7].all() and ((got - want).abs()[safe] <= lim[safe]).all()
+    assert safe[0, :7].all() and safe[4:7, :7].all() and ((got - want).abs()[safe] <= lim[safe]).all()
 
 
 # (rows, columns, K, K ranges): tiles of 16, 32 .. 96 rows in this order, then K in one piece (its halves kept apart at 780), then longer sums. The

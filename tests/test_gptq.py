@@ -126,9 +126,9 @@ def test_gptq_block_kernel_bitwise(hip, t):
 @pytest.mark.gpu
 @pytest.mark.parametrize("N", [8192, 8273])
 def test_gptq_block_kernel_wide_bitwise(hip, N):
-    """Both launch shapes of llj_gptq_block (32 rows x 8 lanes for N <= 8192, 64 rows x 4 lanes
-    above; 8273 also leaves a ragged last workgroup): the fixture's rows tiled to N rows (rows are
-    independent), first block, bit for bit against the oracle's gptq_block of the original rows."""
+    """The wider launch shapes of llj_gptq_block (16 lanes a row; 32 rows to a workgroup for N up to 8192, 64 above;
+    8273 also leaves a ragged last workgroup): the fixture's rows tiled to N rows (rows are independent), first block,
+    bit for bit against the oracle's gptq_block of the original rows."""
     W, X, H, bits, *_ = case(CASES[0])
     from lit_llama import _hip
     scale, zero = G.find_params_weight(W, bits)

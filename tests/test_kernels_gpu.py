@@ -1478,7 +1478,7 @@ def test_gemm_w4z_exact_below_256_rows(hip, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 128, 128), (17, 128, 384), (64, 256, 640), (129, 384, 4224), (255, 128, 2176)])
 def test_gemm_bf16_exact_below_256_rows(hip, M, N, K):
-    """Small integers: every product and fp32 partial sum is an integer below 2^24, whole or in K slices, so the product is
+    """Small integers: every product and fp32 partial sum is an integer below 2^24, whole (up to K = 640 here) or in K slices, so the product is
     bitwise bf16 of the exact sums, and with a residual bf16 of the residual plus that."""
     rng = np.random.default_rng(M + K)
     a = rng.integers(-4, 5, size=(M, K)).astype(np.float32)
@@ -1487,7 +1487,7 @@ def test_gemm_bf16_exact_below_256_rows(hip, M, N, K):
     res = rng.integers(-64, 65, size=(M, N)).astype(np.float32)
     y = bf16(a @ w.T)
     n = hip.llj_gemm_ws_bytes(1, M, N, K)
-    assert (n > 0 and K >= 2176) or (n == 0 and K <= 384) or K == 640  # (where the plan's line lies is its own affair)
+    assert (n > 0) == (K >= 2176)
     scr = torch.empty(max(4, n), dtype=torch.uint8, device=dev)
     for ws in (None, scr.data_ptr()):
         out, r = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev), T(res, torch.bfloat16)
