@@ -71,7 +71,7 @@ int llj_set_stream_a(int mode);
  *   LLJ_OPT_FLASH_QB       1..2  flash prefill: 16-query blocks per wave (default 1)
  *   LLJ_OPT_FLASH_PAIR     0..1  flash prefill: (long, short) query-block pairs per workgroup (default 0)
  *   LLJ_OPT_GEMM_GLDS      0..1  prefill GEMMs: LDS-DMA (1) or register-staged (0) kernel for every format (LLJ_GEMM_GLDS)
- *   LLJ_OPT_GLDS_COST128   0..   LDS-DMA GEMM: cost of a 256 x 128 tile in % of a 256 x 256 one (LLJ_GLDS_COST128)
+ *   LLJ_OPT_GLDS_COST128   0..   LDS-DMA GEMM: cost of a 256 x 128 tile in % of a 256 x 256 one (LLJ_GLDS_COST128; unset 49: always 256 x 128)
  *   LLJ_OPT_GEMV_LDS_A_KB  56..96 decode GEMVs: cap of the staged A image in KiB (LLJ_GEMV_LDS_A_KB)
  *   LLJ_OPT_ATT_SPEC_BATCH 0..1  decode attention: the half speculative key pass also past 64 blocks (LLJ_ATT_SPEC_BATCH)
  *   LLJ_OPT_GEMM_W4Z       0..1  prefill int4 GEMMs with LLJ_WF_ZINT: convert-once LDS-DMA kernel (1) or the int4 default (0) (LLJ_GEMM_W4Z) */
@@ -190,7 +190,7 @@ int llj_norm_linear(int wfmt, const void* x, const void* norm_w, float eps, cons
  * (group, column) as for llj_linear; B fragments dequantized to bf16((q - z) * s)).
  * N % 128 == 0, K % 128 == 0, lda % 8 == 0; any M >= 1. Same epilogue semantics as the GEMVs.
  * wfmt 0 | LLJ_WF_ZINT: int4 whose zeros are all integers (GPTQ's round(-min / scale); the caller
- * checks): for M >= 256 each chunk's codes are converted once per workgroup into an exact bf16
+ * checks): for M > 128 (up to 255 rows: K >= 4096) each chunk's codes are converted once per workgroup into an exact bf16
  * (q - z) tile and the scale is applied in the epilogue, y = s * sum_k A (q - z) -- the reference
  * kernel's ((q - zero) * scale) . A (quantization.py:263-267) with the scale factored out. */
 #define LLJ_WF_ZINT 0x20000

@@ -60,8 +60,9 @@ enum : int { GWF_W4 = 0, GWF_BF16 = 1, GWF_I8 = 2, GWF_W8 = 3, GWF_W4G = 4, GWF_
 // into column j of C (bf16 weights)
 // GEP_SWIGLU: h = bf16(silu(bf16(A . W1^T))) * bf16(A . W2^T) in one pass (convert-once int4: both weights'
 // codes staged per chunk, one A tile feeding both; W2 / sz2)
-// GEP_PARTIAL: split-K slice of a residual GEMM -- fp32 partials y (scale applied) of K range slice
-// blockIdx.x % nsplit into ws[slice][M][N]; llj_gemm_resid_ws's reduce adds them and the residual
+// GEP_PARTIAL: split-K slice in the LDS-DMA kernel -- fp32 partials y (scale applied) of K range slice
+// blockIdx.x % nsplit into ws[slice][M][N]; llj_gemm_resid_ws's reduce (M >= 256) adds them and the residual,
+// gemm_finish_kernel (below) adds them and runs any epilogue
 // GEP_SWIGLU_PART: split-K slice of the dual SwiGLU pass (its last partial wave of tiles) -- fp32 partials of
 // c_fc1 and c_fc2 (scales applied) into ws[slice][2][M][N]; llj_gemm_swiglu_ws's reduce finishes h
 // GEP_SPLIT: K slice blockIdx.x % slices of a 128-row tile (any format): the slice's sums into ws[slice][M][N] -- fp32 with the scale
@@ -857,7 +858,8 @@ static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
   return ns < 2 ? 0 : (size_t)(ns + (wf == GWF_I8 ? 1 : 0)) * M * N * 4;
 }
 // ---------------------------------------------------------------------------------------------
-// 256-row LDS-DMA GEMM (bf16 and int4 W4P weights, M >= 256): a 512-thread workgroup (8 waves, one
+// 256-row LDS-DMA GEMM (bf16 at any M; int4 W4P with integral zeros from 129 rows, or 256 by K and the columns,
+// gemm_run; other int4 and 256 x 256 tiles through the options alone): a 512-thread workgroup (8 waves, one
 // per CU) owns a 256 x BN output tile (BN 256: waves 2 x 4 of 128 x 64; BN 128: 4 x 2 of 64 x 64)
 // and walks K in 64-deep chunks. A chunk's A tile (256 rows x 128 B) and B tile (bf16: BN rows x
 // 128 B; W4P: the 512-B half of each of its BN / 16 tiles that holds the chunk) go global -> LDS
@@ -907,7 +909,8 @@ static inline size_t gemm_split_bytes(int wf, int M, int N, int K) {
 #define LLJ_W4Z_AFTER 0  // convert-once int4: the converting waves convert after their MFMAs (A/B)
 #endif
 #ifndef LLJ_GLDS_COST128
-// time of a 256 x 128 tile in % of a 256 x 256 one: less than half of it, so 256 x 128 always (4 row tiles at a time, bf16 rows 1024 /
+// time of a 256 x 128 tile in % of a 256 x 256 one: less than half of it, so 256 x 128 always, and 256 x 256 only with LLJ_OPT_GLDS_COST128
+// from 50 on (4 row tiles at a time, bf16 rows 1024 /
 // 2048 / 4096 / 8192, 256 x 256 -> 256 x 128: 4096 -> 12288 108 / 203 / 343 / 687 -> 108 / 168 / 336 / 663 us, 11008 -> 4096
 // 246 / 246 / 292 / 595 -> 131 / 150 / 297 / 585)
 #define LLJ_GLDS_COST128 49
@@ -1592,7 +1595,7 @@ static int gemm_glds_launch(const GemmParams& p, hipStream_t s) {
 }
 
 
-// 256 x 256 or 256 x 128 tiles: the shape with the fewer tile-time units over the CUs (waves of
+// 256 x 256 or 256 x 128 tiles (the first only under LLJ_OPT_GLDS_COST128, LLJ_GLDS_COST128 above): the shape with the fewer tile-time units over the CUs (waves of
 // tiles rounded up, a 256 x 128 tile costing LLJ_GLDS_COST128 % of a 256 x 256 one)
 template <int WF, int EP>
 static int gemm_glds_run(const GemmParams& p, hipStream_t s) {

@@ -408,7 +408,7 @@ int llj_g_rope_attention(const void* qkv, void* kcache, void* vcache, const floa
   const int hs = C / n_head;
   if (hs > (mask ? 64 : 128)) {
 #define LLJ_GRS(T, MASK) \
-  hipLaunchKernelGGL((g_rope_attention_kernel<T, 4, MASK>), dim3(B, n_head), dim3(kGrThreads), lds, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
+  hipLaunchKernelGGL((g_rope_attention_kernel<T, MASK>), dim3(B, n_head), dim3(kGrThreads), lds, s, (const T*)qkv, (T*)kcache, (T*)vcache, rope, pos, (T*)y, C, n_head, S)
     if (dt == 0) LLJ_GRS(bf16_t, false);
     else if (mask) LLJ_GRS(float, true);
     else LLJ_GRS(float, false);

@@ -177,26 +177,28 @@ __global__ __launch_bounds__(256) void g_rows_kernel(const T* __restrict__ x, in
   }
 }
 
-// One token per sequence: rotary positions of q and k (g_rope_kv_kernel), k and v into cache slot p % S, and causal attention over
-// the cache (g_attention_kernel). Block (row, head) of 512 threads -- a few tens of blocks with a chain of memory trips each: 16
-// lanes per key and 128 keys at a time, then the values with the threads split over dimension pairs and up to kGrKeyGroups
-// interleaved groups of keys. The first keys and values are loaded before the rotation, without a branch around any of them but in MASK. For heads
-// of more than 128 (fp32 with many workgroups: 64); the others below. LDS: S + hs (3 + groups) floats.
 // A pair in rotary position (c, s), rounded the same in every kernel that forms it
 __device__ __forceinline__ float2 gr_rotate(float x0, float x1, float c, float s) {
   const float a = x1 * s, b = x1 * c;
   return make_float2(__builtin_fmaf(x0, c, -a), __builtin_fmaf(x0, s, b));
 }
+
+// One token per sequence: rotary positions of q and k (g_rope_kv_kernel), k and v into cache slot p % S, and causal attention over
+// the cache (g_attention_kernel). Block (row, head) of 512 threads -- a few tens of blocks with a chain of memory trips each: 16
+// lanes per key and 128 keys at a time, then the values with the threads split over dimension pairs and up to kGrKeyGroups
+// interleaved groups of keys. The first keys and values are loaded before the rotation, without a branch around any of them but in MASK. For heads
+// of more than 128 (fp32 with many workgroups: 64); the others below. LDS: S + hs (3 + groups) floats.
 constexpr int kGrThreads = 512, kGrKeyGroups = 14;
 __host__ __device__ inline int gr_groups(int P) { return P > kGrThreads ? 1 : P * kGrKeyGroups > kGrThreads ? kGrThreads / P : kGrKeyGroups; }
-// NQ: pairs of a key's 16 lanes each, ceil(hs / 32) to 4 (bf16: 4 for 3). MASK: only what is seen is loaded, behind branches.
-template <typename T, int NQ, bool MASK>
+// MASK: only what is seen is loaded, behind branches.
+template <typename T, bool MASK>
 __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* __restrict__ qkv, T* __restrict__ kc, T* __restrict__ vc,
                                                                const float* __restrict__ rope, const int* __restrict__ pos,
                                                                T* __restrict__ y, int C, int nh, int S) {
   extern __shared__ __align__(16) char gr_lds[];
   __shared__ float red[kGrThreads / 64];
   typedef T pair __attribute__((ext_vector_type(2)));
+  constexpr int NQ = 4;  // pairs of a key for each of its 16 lanes, at a time
   const int m = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int hs = C / nh, P = hs / 2, p = pos[0], slot = p % S, nvis = p < S ? p + 1 : S;
   float* sc = reinterpret_cast<float*>(gr_lds);  // [S] scores, then weights
@@ -326,9 +328,11 @@ __global__ __launch_bounds__(kGrThreads) void g_rope_attention_kernel(const T* _
 // no LDS, keys and values pass once (running maximum and sum per 16 lanes, key group + 32 i) and the workgroup meets once, at the end.
 // A chain of three memory trips: the first 128 keys and values with the position (not in MASK), then its rotary pairs, then (from 128 keys on) the next
 // keys, a pass ahead.
-// us with the scores in LDS (the kernel above) and so, bf16: 10 heads of 78, 40 keys 5.4 and 3.9, 110 keys 5.7 and 4.0, 500 keys 18.7 and 7.0; 8 rows
-// of 32 heads of 80, 500 keys 28.4 and 11.9; fp32: 10 heads of 78, 110 keys 5.7 and 5.1, 500 keys 12.9 and 9.5. 10 workgroups: bound by the
-// chain, not by the 16 KB a head.
+// us with the scores in LDS (the kernel above) and so, bf16: 10 heads of 78, 40 keys 5.4 and 3.9, 110 keys 5.7 and 4.0, 500 keys 18.7 and 7.0 (launches one after the
+// other; in a decode step 110 keys take 5.0); 8 rows
+// of 32 heads of 80, 500 keys 28.4 and 11.9; fp32: 10 heads of 78, 110 keys 5.7 and 5.1, 500 keys 12.9 and 9.5; heads of
+// 100 and 128 in the first some 50 keys 6.2 to 6.6 and 6.4 to 6.9, later 1.1 to 1.3 times as fast. 10 workgroups: bound by the chain, not by the 16 KB a
+// head.
 template <typename T, int NQ, int U, bool MASK>
 __global__ __launch_bounds__(kGrThreads) void g_rope_attention16_kernel(const T* __restrict__ qkv, T* __restrict__ kc, T* __restrict__ vc,
                                                                  const float* __restrict__ rope, const int* __restrict__ pos,

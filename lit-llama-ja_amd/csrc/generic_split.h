@@ -1,8 +1,8 @@
 // fp32 products of more than GL_ROWS rows on the bf16 matrix cores: y = x . W^T for any M, N, K and strides.
 //
 // An fp32 value is the sum of three bf16 values (each the rest's nearest: 8 + 8 + 8 bits), and a product of two such sums needs six of the
-// nine partial products: the three left out are below 2^-26 of the product and of either sign. The bf16 rate is 16 times the fp32 one, so six
-// products leave 2.7 times its ceiling (157 TFLOP/s dense).
+// nine partial products: the three left out are together below 2^-24 of the product, 2^-27.5 in the root mean square over random
+// mantissas, and of either sign. The bf16 rate is 16 times the fp32 one, so six products leave 2.7 times its ceiling (157 TFLOP/s dense).
 //
 // A workgroup computes 16 MI rows x 128 columns, wave w all rows of columns 32 w .. +31. The weights go from memory to the wave's registers
 // (each wave has its own columns, so LDS would move them twice) and are split there, one tile of 32 values of K ahead; the rows of x are split
@@ -17,7 +17,8 @@
 // Both operands are multiplied by 2^24 before they are split and the sums by 2^-48 at the end: the lowest part of any fp32 value, the smallest
 // denormal's included, is then a normal bf16 number, and no part of a product falls below fp32's range (unscaled, rows of 1e-35 were 2.7e-6 from
 // float64, rows of 1e-37 2.6e-4; scaled 1.03e-7 as at any size). Sums past 2^79 and values past 2^103 leave the range at the other end and are
-// formed again as below. It costs an instruction a value: 301 rows 4096 -> 12288 216 us and 220, 11008 -> 4096 170 and 177, 780 -> 2048 the same.
+// formed again as below. It costs an instruction a value: 301 rows 4096 -> 12288 212 us and 215, 4096 -> 4096 70 and 72,
+// 11008 -> 4096 165 and 180, 780 -> 2048 the same.
 //
 // Up to kGgFineK without K ranges the sums of K's halves are kept apart from 8 tiles on (the second half starts at the same sign).
 //
@@ -26,8 +27,9 @@
 // 1.15e-6 in one chain, 1.40e-7 in the fp32 products before; K = 780 8.9e-8, 5.0e-7 and 9.1e-8).
 //
 // Bound: the bf16 rate at the clock that it sustains (about 1.3 PFLOP/s, 217 TFLOP/s in sixths); below some 40 rows the weights' bytes. us before
-// (v_mfma_f32_32x32x2_f32) and now: 301 rows 4096 -> 12288 268, 186 (163 TFLOP/s), 4096 -> 4096 101, 69, 11008 -> 4096 252, 161, 2048 rows 4096 -> 4096 539,
-// 386, 16 rows 4096 -> 12288 64, 36 (5.5 TB/s), 1000 rows 780 -> 2304 76, 42, 70 rows 780 -> 2304 22, 14.
+// (v_mfma_f32_32x32x2_f32) and now, weights from memory: 301 rows 4096 -> 12288 270, 215 (141 TFLOP/s), 4096 -> 4096 103, 72, 11008 -> 4096 267, 180,
+// 4096 -> 32000 695, 512 (154), 2048 rows 4096 -> 4096 534, 432 (159), 16 rows 4096 -> 12288 69, 48 (4.2 TB/s), 1000 rows 780 -> 2304 76, 43, 70 rows
+// 780 -> 2304 23, 14.
 #pragma once
 #include "common.h"
 #include "generic_gemm.h"

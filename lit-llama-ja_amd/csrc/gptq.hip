@@ -138,8 +138,8 @@ __device__ __forceinline__ float gptq_columns(const float* hs, const float (*dia
 // instruction every 4.75 cycles and one that waits for the last every 8.1, so length and number both count: 570 a group of 16 columns (890 with a row's 16 columns in every
 // lane's registers: 23.6 us at N = 4096; interleaving those updates with the chain, or Hinv1's values a step ahead: no faster). 16 rows put
 // N = 4096 on all 256 CUs, one wave per SIMD; above, more rows to a workgroup share Hinv1. us a block with the rows in LDS, Hinv1 waited for
-// column by column, and now: N = 256 33 and 17, 4096 35 and 19, 8192 38 and 21, 11008 54 and 31, 35008 171 and 88 (a block with an error out
-// of div_by's range is done twice).
+// column by column, and now: N = 256 33 and 17, 4096 35 and 19 (among the producer's other launches
+// 39 and 22), 8192 38 and 21, 11008 54 and 31, 35008 171 and 88 (a block with an error out of div_by's range is done twice).
 template <int ROWS>
 __global__ __launch_bounds__(ROWS * 16) void gptq_block_kernel(const float* __restrict__ hinv, int K, int i1, int blk, float* __restrict__ wt, int N,
                                                                const float* __restrict__ scale, const float* __restrict__ zero, float maxq,

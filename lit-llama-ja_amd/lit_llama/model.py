@@ -142,7 +142,8 @@ _GEMM_FMTS = (0, 1, 2, 3, 4)  # weight formats (low byte of wfmt; 4 = grouped in
 
 
 def _gemm_rows(fmts) -> int:
-    """GEMM_MIN_ROWS, or past its half where every format is bf16 or LLM.int8, whose slices past the second cost more than the tiles
+    """GEMM_MIN_ROWS, or past its half, the first slice, where every format is bf16 or LLM.int8: their second slice costs more than the tiles at every size,
+    while one slice is the faster for small models and the slower for 7B bf16; gptq.int8 crosses between 24 and 31 rows, int4 past 31
     (ms of a prompt, slices and GEMMs: 7B bf16 9 rows 6.6 and 5.9, 16 rows 7.0 and 6.0, 17 rows 9.8 and 6.0, 31 rows 12.6 and 6.1; LLM.int8 16 rows
     7.0 and 7.0, 17 rows 8.9 and 7.1, 31 rows 13.3 and 8.7; 49M 16 rows 1.07 and 1.11, 24 rows 1.22 and 1.10; int4 24 rows 4.5 and 5.7, 31 rows 5.2 and
     5.8; gptq.int8 24 rows 5.7 and 6.2, 31 rows 6.8 and 6.0)."""
