@@ -313,6 +313,10 @@ int llj_gptq_block(const float* hinv, int K, int i1, float* wt, int N, const flo
  * i1 + b <= K. llj_gptq_block is this with b = 128. */
 int llj_gptq_block_bs(const float* hinv, int K, int i1, int blocksize, float* wt, int N, const float* scale,
                       const float* zero, int bits, float* qt, float* err, float* loss, void* stream);
+/* llj_gptq_update behind the block of 128 before i1 (its errors: last), then llj_gptq_block of the block at i1, whose errors go to
+ * another buffer, in one launch; the same bits. wt's columns of the block keep their values from before the update. */
+int llj_gptq_next(const float* hinv, int K, int i1, const float* last, float* wt, int N, const float* scale, const float* zero, int bits,
+                  float* qt, float* err, float* loss, void* stream);
 /* GPTQQuantizer.find_params_weight (475-514), per channel: (scale, zero) of N rows of K fp32 weights; sym: the symmetric range. */
 int llj_gptq_params(const float* w, int N, int K, int bits, int sym, float* scale, float* zero, void* stream);
 /* collect_input_stats (516-530): H = keep H + (alpha x)^T (alpha x), x (T, K) row-major, dt 0 = bf16, 1 = fp32, H (K, K) fp32

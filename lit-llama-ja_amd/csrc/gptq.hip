@@ -13,9 +13,11 @@
 // Every arithmetic step is the reference's fp32 op in the reference's order, rounded on its own
 // (this file is built with -ffp-contract=off, lit_llama/_build.py), so a block reproduces the torch CPU
 // loop bitwise given the same W1 and Hinv1.
+#include <algorithm>
 #include <utility>
 
 #include "common.h"
+#include "gptq_tiles.h"
 
 namespace llj {
 
@@ -23,6 +25,10 @@ constexpr int kGptqBlock = 128;
 
 constexpr int kGptqSub = 16;          // columns held in registers at a time
 constexpr int kHs = kGptqBlock + 4;   // LDS row stride of Hinv1 (rows start on 16 bytes)
+constexpr int kHsRows = 80;
+// Hinv1 in LDS from the diagonal groups on: place of element (b, b), b % 16 == 0, row b + u at + u kHs. The rows of b >= 80 lie in the
+// columns that those of 128 - b leave free (42 KB for 68: three workgroups a CU beside the products of gptq_next_kernel).
+__device__ __forceinline__ int band(int b) { return b <= 64 ? b * kHs + b : (kGptqBlock - b) * kHs; }
 
 // a / b, correctly rounded, from y = 1 / b correctly rounded: two residual steps. The first makes the quotient faithful, the
 // second then gives the rounded one (Markstein, "Computation of elementary functions on the IBM RISC System/6000", 1990), for
@@ -52,7 +58,7 @@ struct Group {
   f32x4 d[kGptqSub / 4], rd[kGptqSub / 4];
   __device__ __forceinline__ void load(const float* hs, const float (*diag)[kGptqBlock], int b, int l) {
 #pragma unroll
-    for (int u = 0; u < kGptqSub; ++u) h[u] = hs[(b + u) * kHs + b + l];
+    for (int u = 0; u < kGptqSub; ++u) h[u] = hs[band(b) + u * kHs + l];
 #pragma unroll
     for (int c = 0; c < kGptqSub / 4; ++c) {
       d[c] = *reinterpret_cast<const f32x4*>(diag[0] + b + 4 * c);
@@ -112,7 +118,7 @@ __device__ __forceinline__ float gptq_columns(const float* hs, const float (*dia
       q_out[(size_t)(b + l) * N] = c.q_own;
       e_out[(size_t)(b + l) * N] = c.e_own;
     }
-    const float* h = hs + b * kHs + b + l;
+    const float* h = hs + band(b) + l;
     if (b + kGptqSub < blk) grp.load(hs, diag, b + kGptqSub, l);
     // the rest of the block: the group's updates of a column in increasing i, as the reference applies them one column i at a time
 #pragma unroll
@@ -140,51 +146,136 @@ __device__ __forceinline__ float gptq_columns(const float* hs, const float (*dia
 // N = 4096 on all 256 CUs, one wave per SIMD; above, more rows to a workgroup share Hinv1. us a block with the rows in LDS, Hinv1 waited for
 // column by column, and now: N = 256 33 and 17, 4096 35 and 19 (among the producer's other launches
 // 39 and 22), 8192 38 and 21, 11008 54 and 31, 35008 171 and 88 (a block with an error out of div_by's range is done twice).
-template <int ROWS>
-__global__ __launch_bounds__(ROWS * 16) void gptq_block_kernel(const float* __restrict__ hinv, int K, int i1, int blk, float* __restrict__ wt, int N,
-                                                               const float* __restrict__ scale, const float* __restrict__ zero, float maxq,
-                                                               float* __restrict__ qt, float* __restrict__ err, float* __restrict__ loss) {
-  __shared__ __align__(16) float hs[kGptqBlock * kHs];    // hs[i * kHs + j] = Hinv1[i][j]
-  __shared__ __align__(16) float diag[2][kGptqBlock];     // Hinv1[i][i], 1 / Hinv1[i][i]
+struct BlockArgs {
+  const float* hinv;
+  int K, i1, blk, N;  // the block's columns [i1, i1 + blk)
+  const float *scale, *zero;
+  float maxq;
+  float *qt, *err, *loss;
+};
+struct BlockLds {
+  float hs[kHsRows * kHs];     // Hinv1 (band)
+  float diag[2][kGptqBlock];  // Hinv1[i][i], 1 / Hinv1[i][i]
+};
+
+// The block's columns of rows n = .. + tid / 16. weights(r): this lane's 8 weights, asked for ahead of Hinv1 (EARLY) or behind the barrier after it.
+template <int ROWS, bool EARLY, typename F>
+__device__ __forceinline__ void gptq_rows(const BlockArgs& p, int n, BlockLds& s_, F weights) {
   constexpr int NT = ROWS * 16;
-  const int tid = threadIdx.x, t = tid >> 4, l = tid & 15;
-  const int n = blockIdx.x * ROWS + t;
-  const int nn = n < N ? n : N - 1;  // clamped: loads stay in bounds, stores are guarded
+  const int tid = threadIdx.x, l = tid & 15, K = p.K, i1 = p.i1, blk = p.blk;
+  const int nn = n < p.N ? n : p.N - 1;  // clamped: loads stay in bounds, stores are guarded
   float r[kGptqBlock / kGptqSub];
-  auto stage = [&] {
-#pragma unroll
-    for (int i = 0; i < kGptqBlock / kGptqSub; ++i) r[i] = i * kGptqSub < blk ? wt[(size_t)(i1 + i * kGptqSub + l) * N + nn] : 0.f;
-  };
-  stage();
-  const float s = scale[nn], z = zero[nn];
+  if (EARLY) weights(r);
+  const float s = p.scale[nn], z = p.zero[nn];
   bool fast = divides(s) && fabsf(z) < 0x1p30f;
   if (tid < blk) {
-    const float d = hinv[(size_t)(i1 + tid) * K + i1 + tid];
-    diag[0][tid] = d;
-    diag[1][tid] = __fdiv_rn(1.f, d);
+    const float d = p.hinv[(size_t)(i1 + tid) * K + i1 + tid];
+    s_.diag[0][tid] = d;
+    s_.diag[1][tid] = __fdiv_rn(1.f, d);
     fast = fast && divides(d);
   }
-  if (((K | i1) & 3) == 0 && ((uintptr_t)hinv & 15) == 0) {
+  auto at = [](int i, int j) { return band(i & ~15) + (i & 15) * kHs + j - (i & ~15); };
+  if (((K | i1) & 3) == 0 && ((uintptr_t)p.hinv & 15) == 0) {
     for (int v = tid; v < blk * (blk / 4); v += NT) {
       const int i = v / (blk / 4), j = v % (blk / 4) * 4;
-      *reinterpret_cast<f32x4*>(hs + i * kHs + j) = *reinterpret_cast<const f32x4*>(hinv + (size_t)(i1 + i) * K + i1 + j);
+      if (j >= (i & ~15)) *reinterpret_cast<f32x4*>(s_.hs + at(i, j)) = *reinterpret_cast<const f32x4*>(p.hinv + (size_t)(i1 + i) * K + i1 + j);
     }
   } else {
-    for (int v = tid; v < blk * blk; v += NT) hs[v / blk * kHs + v % blk] = hinv[(size_t)(i1 + v / blk) * K + i1 + v % blk];
+    for (int v = tid; v < blk * blk; v += NT) {
+      const int i = v / blk, j = v % blk;
+      if (j >= (i & ~15)) s_.hs[at(i, j)] = p.hinv[(size_t)(i1 + i) * K + i1 + j];
+    }
   }
   bool done = __syncthreads_and(fast);
-  const bool live = n < N;
-  float* q_out = qt + (size_t)i1 * N + nn;
-  float* e_out = err + nn;
+  if (!EARLY) weights(r);
+  const bool live = n < p.N;
+  float* q_out = p.qt + (size_t)i1 * p.N + nn;
+  float* e_out = p.err + nn;
   float sum = 0.f;
   Errors seen;
   if (done) {
-    sum = gptq_columns<true>(hs, diag, r, l, blk, s, z, maxq, live, q_out, e_out, N, seen);
+    sum = gptq_columns<true>(s_.hs, s_.diag, r, l, blk, s, z, p.maxq, live, q_out, e_out, p.N, seen);
     done = __syncthreads_and(seen.fit());
-    if (!done) stage();  // a quotient out of div_by's range: the block again
+    if (!done) weights(r);  // a quotient out of div_by's range: the block again
   }
-  if (!done) sum = gptq_columns<false>(hs, diag, r, l, blk, s, z, maxq, live, q_out, e_out, N, seen);
-  if (live && l == 0) loss[n] += sum;
+  if (!done) sum = gptq_columns<false>(s_.hs, s_.diag, r, l, blk, s, z, p.maxq, live, q_out, e_out, p.N, seen);
+  if (live && l == 0) p.loss[n] += sum;
+}
+
+template <int ROWS>
+__global__ __launch_bounds__(ROWS * 16) void gptq_block_kernel(BlockArgs p, const float* __restrict__ wt) {
+  __shared__ __align__(16) BlockLds lds;
+  const int n = blockIdx.x * ROWS + (threadIdx.x >> 4), nn = n < p.N ? n : p.N - 1, l = threadIdx.x & 15;
+  gptq_rows<ROWS, true>(p, n, lds, [&](float (&r)[kGptqBlock / kGptqSub]) {
+#pragma unroll
+    for (int i = 0; i < kGptqBlock / kGptqSub; ++i) r[i] = i * kGptqSub < p.blk ? wt[(size_t)(p.i1 + i * kGptqSub + l) * p.N + nn] : 0.f;
+  });
+}
+
+// The update behind one block of 128 and the column loop of the next in one launch. The first workgroups take 16 rows each: they take the
+// last block's errors off the next 128 columns -- their own rows of the product, 64 MFMAs a wave, operands from memory as the MFMA
+// wants them -- and run the columns; the others meanwhile take the errors off all later columns in 64 x 64 tiles, as gptq_update_kernel
+// does. Both form every sum as that kernel does: the same bits.
+//
+// Bound: the column loop's chain, some 20 us on one wave per SIMD, beside the products (31 us of their own in the mean at
+// 4096 x 4096), which fill the matrix cores that the chain leaves idle.
+template <bool VEC>
+__global__ __launch_bounds__(256) void gptq_next_kernel(BlockArgs p, const float* __restrict__ last, float* __restrict__ wt, int row_groups) {
+  typedef AtB<64, 64, float, VEC, false> G;
+  struct Rows {
+    BlockLds b;
+    float w[kGptqBlock * 17];  // the block's columns of the 16 rows
+  };
+  __shared__ __align__(16) unsigned char lds[sizeof(Rows) > G::kLds * 4 ? sizeof(Rows) : G::kLds * 4];
+  const int K = p.K, N = p.N, i0 = p.i1 - kGptqBlock;  // (the last block's first column)
+  if ((int)blockIdx.x >= row_groups) {
+    const int i3 = p.i1 + kGptqBlock, M = K - i3, mt = (M + 63) / 64, nt = (N + 63) / 64, t = xcd_run(blockIdx.x - row_groups, mt * nt);
+    if (t < 0) return;
+    const int m0 = t / nt * 64, n0 = t % nt * 64;
+    f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
+    G::run(p.hinv + (size_t)i0 * K + i3 + m0, K, M - m0, last + n0, N, N - n0, kGptqBlock, 1.f, reinterpret_cast<float*>(lds), acc, [&] {
+      G::load(old, [&](int i, int j) { return wt[(size_t)(i3 + min(m0 + i, M - 1)) * N + min(n0 + j, N - 1)]; });
+    });
+    G::both(acc, old, [&](int i, int j, float v, float w) {
+      const int m = m0 + i, n = n0 + j;
+      if (m < M && n < N) wt[(size_t)(i3 + m) * N + n] = w - v;
+    });
+    return;
+  }
+  __builtin_amdgcn_s_setprio(3);  // the longest chain of the launch
+  Rows& s = *reinterpret_cast<Rows*>(lds);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c = lane & 15, n0 = blockIdx.x * 16;
+  {
+    // wave: columns 32 wave .. + 32 of the block, lane: rows (of W) n0 + c
+    const float* a = p.hinv + (size_t)(i0 + q) * K + p.i1 + 32 * wave + c;
+    const float* b = last + (size_t)q * N + min(n0 + c, N - 1);
+    const float* w = wt + (size_t)(p.i1 + 32 * wave + 4 * q) * N + min(n0 + c, N - 1);
+    constexpr int KS = kGptqBlock / 4;
+    float av[KS][2], bv[KS], old[2][4];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      av[k][0] = a[(size_t)4 * k * K];
+      av[k][1] = a[(size_t)4 * k * K + 16];
+      bv[k] = b[(size_t)4 * k * N];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) old[i][r] = w[(size_t)(16 * i + r) * N];
+    f32x4 acc[2] = {};
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] = mma4(av[k][i], bv[k], acc[i]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s.w[(32 * wave + 16 * i + 4 * q + r) * 17 + c] = old[i][r] - acc[i][r];
+  }
+  gptq_rows<16, false>(p, n0 + (tid >> 4), s.b, [&](float (&r)[kGptqBlock / kGptqSub]) {
+#pragma unroll
+    for (int i = 0; i < kGptqBlock / kGptqSub; ++i) r[i] = s.w[(i * kGptqSub + (tid & 15)) * 17 + (tid >> 4)];
+  });
 }
 
 // pack_weight (quantization.py:374-388) of reconstructed weights Qt (K x N, fp32):
@@ -260,10 +351,8 @@ int llj_gptq_block_bs(const float* hinv, int K, int i1, int blocksize, float* wt
   LLJ_REQUIRE(K > 0 && N > 0 && i1 >= 0 && i1 % blocksize == 0 && i1 + blocksize <= K);
   LLJ_REQUIRE(bits == 2 || bits == 4 || bits == 8);
   LLJ_REQUIRE(hinv && wt && scale && zero && qt && err && loss);
-  const float maxq = (float)((1 << bits) - 1);
-#define LLJ_BLOCK(ROWS)                                                                                                                \
-  hipLaunchKernelGGL((gptq_block_kernel<ROWS>), dim3((N + ROWS - 1) / ROWS), dim3(ROWS * 16), 0, (hipStream_t)stream, hinv, K, i1,    \
-                     blocksize, wt, N, scale, zero, maxq, qt, err, loss)
+  const BlockArgs p = {hinv, K, i1, blocksize, N, scale, zero, (float)((1 << bits) - 1), qt, err, loss};
+#define LLJ_BLOCK(ROWS) hipLaunchKernelGGL((gptq_block_kernel<ROWS>), dim3((N + ROWS - 1) / ROWS), dim3(ROWS * 16), 0, (hipStream_t)stream, p, wt)
   if (N <= 4096) LLJ_BLOCK(16);
   else if (N <= 8192) LLJ_BLOCK(32);
   else LLJ_BLOCK(64);
@@ -275,6 +364,20 @@ int llj_gptq_block_bs(const float* hinv, int K, int i1, int blocksize, float* wt
 int llj_gptq_block(const float* hinv, int K, int i1, float* wt, int N, const float* scale, const float* zero,
                    int bits, float* qt, float* err, float* loss, void* stream) {
   return llj_gptq_block_bs(hinv, K, i1, kGptqBlock, wt, N, scale, zero, bits, qt, err, loss, stream);
+}
+
+int llj_gptq_next(const float* hinv, int K, int i1, const float* last, float* wt, int N, const float* scale, const float* zero, int bits,
+                  float* qt, float* err, float* loss, void* stream) {
+  LLJ_REQUIRE(K > 0 && N > 0 && i1 >= kGptqBlock && i1 % kGptqBlock == 0 && i1 + kGptqBlock <= K && (bits == 2 || bits == 4 || bits == 8));
+  LLJ_REQUIRE(hinv && last && wt && scale && zero && qt && err && err != last && loss);
+  const BlockArgs p = {hinv, K, i1, kGptqBlock, N, scale, zero, (float)((1 << bits) - 1), qt, err, loss};
+  const bool vec = K % 4 == 0 && N % 4 == 0 && (((uintptr_t)hinv | (uintptr_t)last) & 15) == 0;
+  const long M = K - i1 - kGptqBlock, tiles = ((M + 63) / 64) * ((N + 63) / 64), groups = (N + 15) / 16, grid = groups + (tiles + 7) / 8 * 8;
+  LLJ_REQUIRE(grid < (1l << 31));
+  if (vec) hipLaunchKernelGGL((gptq_next_kernel<true>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, p, last, wt, (int)groups);
+  else hipLaunchKernelGGL((gptq_next_kernel<false>), dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, p, last, wt, (int)groups);
+  LLJ_CHECK_LAUNCH();
+  return 0;
 }
 
 int llj_gptq_params(const float* w, int N, int K, int bits, int sym, float* scale, float* zero, void* stream) {

@@ -1,151 +1,19 @@
 // Matrix work of the GPTQ producer around the column loop (gptq.hip): the calibration Hessian, the inverse factor that the
 // loop reads, and the update of the columns behind a block (reference lit_llama/quantization.py:516-530, 549-566, 596).
 //
-// All three are C -= or += A^T B with both operands stored along their output index ("k-major": X of the Hessian is tokens x
-// columns, a block of the factor and the block's errors are 128 x columns), which v_mfma_f32_16x16x4_f32 takes from LDS without a
-// transposition: lane l reads element (k + l / 16, m + l % 16), rows 16 banks apart. One accumulator per output, ascending k.
+// All three are C -= or += A^T B (gptq_tiles.h).
 // Bound: the fp32 matrix rate (157 TFLOP/s dense). A wave's 16 k of a 64 x 64 tile are 16 MFMAs of 32 cycles for 16 reads of
 // 4 bytes a lane, so neither LDS nor the loads (the next tile's in registers while this one is multiplied) are near their limits.
 #include "common.h"
+#include "gptq_tiles.h"
 
 namespace llj {
 
 constexpr int kFactor = 128;  // columns per elimination step
 
-__device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
-// four consecutive elements, zeros from `left` on
-template <bool VEC>
-__device__ __forceinline__ f32x4 ld4(const float* p, int left) {
-  if constexpr (VEC) return left > 0 ? *reinterpret_cast<const f32x4*>(p) : f32x4{};
-  f32x4 v = {};
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (i < left) v[i] = p[i];
-  return v;
-}
-template <bool VEC>
-__device__ __forceinline__ f32x4 ld4(const bf16_t* p, int left) {
-  f32x4 v = {};
-  if constexpr (VEC) {
-    if (left > 0) {
-      const uint2 w = *reinterpret_cast<const uint2*>(p);
-      v = f32x4{bflo(w.x), bfhi(w.x), bflo(w.y), bfhi(w.y)};
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i < left) v[i] = bf2f(p[i]);
-  }
-  return v;
-}
-
-// acc = A^T B of one BM x BN tile by 256 threads (2 x 2 waves): A: kd x ma, B: kd x nb, k-major, pointers at the tile's first column,
-// ma / nb columns left from there (VEC: multiples of 4, rows aligned to four elements). SCALE: elements times alpha, rounded.
-template <int BM, int BN, typename S, bool VEC, bool SCALE>
-struct AtB {
-  static constexpr int KD = 32, SA = BM + 16, SB = BN + 16, MI = BM / 32, NI = BN / 32;
-  static constexpr int kLds = 2 * KD * (SA + SB);  // floats
-  static constexpr int TA = BM / 4, RA = 256 / TA, PA = KD / RA, TB = BN / 4, RB = 256 / TB, PB = KD / RB;
-
-  static __device__ __forceinline__ void run(const S* A, size_t lda, int ma, const S* B, size_t ldb, int nb, int kd, float alpha,
-                                             float* lds, f32x4 (&acc)[MI][NI]) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int ca = (tid % TA) * 4, cb = (tid % TB) * 4;
-    f32x4 fa[PA], fb[PB];
-    auto fetch = [&](int k) {
-#pragma unroll
-      for (int p = 0; p < PA; ++p) {
-        const int row = k + tid / TA + p * RA;
-        fa[p] = ld4<VEC>(A + (size_t)row * lda + ca, row < kd ? ma - ca : 0);
-      }
-#pragma unroll
-      for (int p = 0; p < PB; ++p) {
-        const int row = k + tid / TB + p * RB;
-        fb[p] = ld4<VEC>(B + (size_t)row * ldb + cb, row < kd ? nb - cb : 0);
-      }
-    };
-    auto stage = [&](int buf) {
-      float* a = lds + buf * KD * (SA + SB);
-      float* b = a + KD * SA;
-#pragma unroll
-      for (int p = 0; p < PA; ++p) *reinterpret_cast<f32x4*>(a + (tid / TA + p * RA) * SA + ca) = SCALE ? fa[p] * alpha : fa[p];
-#pragma unroll
-      for (int p = 0; p < PB; ++p) *reinterpret_cast<f32x4*>(b + (tid / TB + p * RB) * SB + cb) = SCALE ? fb[p] * alpha : fb[p];
-    };
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NI; ++j) acc[i][j] = f32x4{};
-    const int oa = (lane >> 4) * SA + (wave & 1) * (BM / 2) + (lane & 15), ob = (lane >> 4) * SB + (wave >> 1) * (BN / 2) + (lane & 15);
-    fetch(0);
-    stage(0);
-    for (int k = 0, t = 0; k < kd; k += KD, ++t) {
-      __syncthreads();  // tile t is staged, and every wave is done with the other buffer
-      if (k + KD < kd) fetch(k + KD);
-      const float* a = lds + (t & 1) * KD * (SA + SB) + oa;
-      const float* b = lds + (t & 1) * KD * (SA + SB) + KD * SA + ob;
-#pragma unroll
-      for (int q = 0; q < KD / 4; ++q) {
-        float va[MI], vb[NI];
-#pragma unroll
-        for (int i = 0; i < MI; ++i) va[i] = a[4 * q * SA + 16 * i];
-#pragma unroll
-        for (int j = 0; j < NI; ++j) vb[j] = b[4 * q * SB + 16 * j];
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NI; ++j) acc[i][j] = mma4(va[i], vb[j], acc[i][j]);
-      }
-      if (k + KD < kd) stage((t + 1) & 1);
-    }
-  }
-  // acc = f(row, column) of every output of the tile: all loads before the first use
-  template <typename F>
-  static __device__ __forceinline__ void load(f32x4 (&acc)[MI][NI], F f) {
-    each(acc, [&](int i, int j, float& v) { v = f(i, j); });
-  }
-  // f(row, column, sum) of every output of the tile
-  template <typename F>
-  static __device__ __forceinline__ void each(f32x4 (&acc)[MI][NI], F f) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NI; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float v = acc[i][j][r];
-          f((wave & 1) * (BM / 2) + 16 * i + 4 * (lane >> 4) + r, (wave >> 1) * (BN / 2) + 16 * j + (lane & 15), v);
-          acc[i][j][r] = v;
-        }
-  }
-  template <typename F>
-  static __device__ __forceinline__ void both(f32x4 (&acc)[MI][NI], f32x4 (&old)[MI][NI], F f) {
-    int at = 0;
-    each(acc, [&](int i, int j, float v) {
-      f(i, j, v, old[at / (4 * NI)][at / 4 % NI][at % 4]);
-      ++at;
-    });
-  }
-};
-
-// block b of a grid padded to a multiple of 8 -> its place in a list of n tiles that gives each XCD (b % 8) one run of neighbours
-__device__ __forceinline__ int xcd_run(int b, int n) {
-  const int per = (n + 7) / 8, t = (b & 7) * per + (b >> 3);
-  return (b >> 3) < per && t < n ? t : -1;
-}
-// t -> (i, j <= i) of a triangle's tiles, row by row
-__device__ __forceinline__ void triangle(int t, int& i, int& j) {
-  i = (int)((__builtin_sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
-  while (i * (i + 1) / 2 > t) --i;
-  while ((i + 1) * (i + 2) / 2 <= t) ++i;
-  j = t - i * (i + 1) / 2;
-}
-
 // H = keep H + (alpha X)^T (alpha X): the tiles on and below the diagonal, each written to its place and mirrored. The sums are those
-// of the library's product bit for bit (to 4,096 columns), at half its work: 2048 x 4096 422 us (83 TFLOP/s of the half) for 580 with
-// the two passes over H.
+// of the library's product bit for bit (to 4,096 columns), at half its work: 2048 x 4096 358 us (96 TFLOP/s of the half; 386 with one tile
+// ahead, read behind branches) for 580 with the two passes over H.
 template <int BT, typename S, bool VEC>
 __global__ __launch_bounds__(256) void gptq_gram_kernel(const S* __restrict__ x, int T, int K, float keep, float alpha, float* __restrict__ H) {
   typedef AtB<BT, BT, S, VEC, true> G;
@@ -156,7 +24,24 @@ __global__ __launch_bounds__(256) void gptq_gram_kernel(const S* __restrict__ x,
   triangle(t, ti, tj);
   const int m0 = ti * BT, n0 = tj * BT;
   f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
-  G::run(x + m0, K, K - m0, x + n0, K, K - n0, T, alpha, lds, acc);
+  // (a lane's four sums of an MFMA tile are neighbours in the mirrored place: whole vectors there, of H's own symmetric other half too)
+  const bool whole = VEC && m0 + BT <= K && n0 + BT <= K;
+  G::run(x + m0, K, K - m0, x + n0, K, K - n0, T, alpha, lds, acc, [&] {
+    if (!whole) return;
+    G::tiles([&](int a, int b, int i, int j) { old[a][b] = *reinterpret_cast<const f32x4*>(H + (size_t)(n0 + j) * K + m0 + i); });
+  });
+  if (whole) {
+    G::tiles([&](int a, int b, int i, int j) {
+      f32x4 h;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) h[r] = old[a][b][r] * keep + acc[a][b][r];
+      *reinterpret_cast<f32x4*>(H + (size_t)(n0 + j) * K + m0 + i) = h;
+      if (ti != tj)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) H[(size_t)(m0 + i + r) * K + n0 + j] = h[r];
+    });
+    return;
+  }
   G::load(old, [&](int i, int j) { return H[(size_t)min(m0 + i, K - 1) * K + min(n0 + j, K - 1)]; });
   G::both(acc, old, [&](int i, int j, float v, float h) {
     const int m = m0 + i, n = n0 + j;
@@ -178,8 +63,9 @@ __global__ __launch_bounds__(256) void gptq_update_kernel(const float* __restric
   if (t < 0) return;
   const int m0 = t / nt * BM, n0 = t % nt * BN;
   f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
-  G::run(hinv + (size_t)i1 * K + i2 + m0, K, M - m0, err + n0, N, N - n0, blk, 1.f, lds, acc);
-  G::load(old, [&](int i, int j) { return wt[(size_t)(i2 + min(m0 + i, M - 1)) * N + min(n0 + j, N - 1)]; });
+  G::run(hinv + (size_t)i1 * K + i2 + m0, K, M - m0, err + n0, N, N - n0, blk, 1.f, lds, acc, [&] {
+    G::load(old, [&](int i, int j) { return wt[(size_t)(i2 + min(m0 + i, M - 1)) * N + min(n0 + j, N - 1)]; });
+  });
   G::both(acc, old, [&](int i, int j, float v, float w) {
     const int m = m0 + i, n = n0 + j;
     if (m < M && n < N) wt[(size_t)(i2 + m) * N + n] = w - v;
@@ -334,7 +220,7 @@ __global__ __launch_bounds__(256) void gptq_panel_kernel(const float* __restrict
   if (n0 / kFactor == k) return;
   f32x4 acc[G::MI][G::NI];
   const size_t row = (size_t)k * kFactor;
-  G::run(xt + m0, kFactor, kFactor - m0, M + row * K + n0, K, K - n0, kFactor, 1.f, lds, acc);
+  G::run(xt + m0, kFactor, kFactor - m0, M + row * K + n0, K, K - n0, kFactor, 1.f, lds, acc, [] {});
   G::each(acc, [&](int i, int j, float v) { P[(row + m0 + i) * K + n0 + j] = v; });
 }
 
@@ -351,8 +237,8 @@ __global__ __launch_bounds__(256) void gptq_step_kernel(float* __restrict__ M, f
   if (blockIdx.x == 0) {
     __builtin_amdgcn_s_setprio(3);  // the longest chain of the launch, beside another workgroup's products
     f32x4 acc[D::MI][D::NI], old[D::MI][D::NI];
-    D::load(old, [&](int i, int j) { return M[(size_t)(r0 + i) * K + r0 + j]; });
-    D::run(p + r0, K, kFactor, p + r0, K, kFactor, kFactor, 1.f, lds, acc);
+    D::run(p + r0, K, kFactor, p + r0, K, kFactor, kFactor, 1.f, lds, acc,
+           [&] { D::load(old, [&](int i, int j) { return M[(size_t)(r0 + i) * K + r0 + j]; }); });
     __syncthreads();
     D::both(acc, old, [&](int i, int j, float v, float m) { lds[i * kFs + j] = j >= i ? m - v : 0.f; });
     const bool ok = factor_block(lds, &bad);
@@ -374,8 +260,8 @@ __global__ __launch_bounds__(256) void gptq_step_kernel(float* __restrict__ M, f
     n0 = r0 + i * 64;
   }
   f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
-  G::load(old, [&](int i, int j) { return M[(size_t)(m0 + i) * K + n0 + j]; });
-  G::run(p + m0, K, 64, p + n0, K, 64, kFactor, 1.f, lds, acc);
+  G::run(p + m0, K, 64, p + n0, K, 64, kFactor, 1.f, lds, acc,
+         [&] { G::load(old, [&](int i, int j) { return M[(size_t)(m0 + i) * K + n0 + j]; }); });
   const bool first = n0 / kFactor == k;
   G::both(acc, old, [&](int i, int j, float v, float m) { M[(size_t)(m0 + i) * K + n0 + j] = (first ? 0.f : m) - v; });
 }

@@ -48,6 +48,7 @@ SIGNATURES = {
     "llj_i8_gather_weight": [_P, _P, _I, _I, _P, _P, _I, _P],
     "llj_gptq_block": [_P, _I, _I, _P, _I, _P, _P, _I, _P, _P, _P, _P],
     "llj_gptq_block_bs": [_P, _I, _I, _I, _P, _I, _P, _P, _I, _P, _P, _P, _P],
+    "llj_gptq_next": [_P, _I, _I, _P, _P, _I, _P, _P, _I, _P, _P, _P, _P],
     "llj_gptq_gram": [_P, _I, _I, _I, _F, _F, _P, _P],
     "llj_gptq_update": [_P, _I, _I, _I, _P, _I, _P, _P],
     "llj_gptq_params": [_P, _I, _I, _I, _I, _P, _P, _P],

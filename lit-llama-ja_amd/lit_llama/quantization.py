@@ -574,7 +574,7 @@ class GPTQQuantizer:
                   _hip.stream())
         del W
         Qt = torch.empty_like(Wt)
-        Err = torch.empty((B, N), dtype=torch.float32, device=self.dev)
+        Err, Err_next = torch.empty((2, B, N), dtype=torch.float32, device=self.dev)
         loss = torch.zeros(N, dtype=torch.float32, device=self.dev)
         # the stored (scale, zero) -- rounded to the buffers' dtype, e.g. bf16 -- are what decode
         # dequantizes with, so the column loop's reconstructions and error feedback use them too
@@ -586,19 +586,26 @@ class GPTQQuantizer:
         if G == 1:
             scg[0] = self.scales.reshape(-1).float().contiguous()
             zrg[0] = self.zeros.reshape(-1).float().contiguous()
+        def update(i1):  # W[:, i1:] -= Err1 @ Hinv[i1 - B:i1, i1:] (596) behind the block before i1, transposed
+            _hip.call("llj_gptq_update", Hinv.data_ptr(), K, i1 - B, B, Err.data_ptr(), N, Wt.data_ptr(), s)
+
         for i1 in range(0, K, B):
-            i2 = i1 + B
             gi = i1 // g
-            if G > 1 and i1 % g == 0:  # reference 571-577: the group's params from W as updated so far
+            first = i1 == 0 or (G > 1 and i1 % g == 0)
+            if i1 and (first or B != 128):
+                update(i1)
+            if G > 1 and first:  # reference 571-577: the group's params from W as updated so far
                 gs, gz = self.find_params_weight(Wt[i1:i1 + g].t())
                 self.scales[:, gi] = gs.reshape(-1)
                 self.zeros[:, gi] = gz.reshape(-1)
                 scg[gi] = self.scales[:, gi].float().contiguous()
                 zrg[gi] = self.zeros[:, gi].float().contiguous()
-            _hip.call("llj_gptq_block_bs", Hinv.data_ptr(), K, i1, B, Wt.data_ptr(), N, scg[gi].data_ptr(),
-                      zrg[gi].data_ptr(), self.bits, Qt.data_ptr(), Err.data_ptr(), loss.data_ptr(), s)
-            # W[:, i2:] -= Err1 @ Hinv[i1:i2, i2:] (596), transposed
-            _hip.call("llj_gptq_update", Hinv.data_ptr(), K, i1, B, Err.data_ptr(), N, Wt.data_ptr(), s)
+            args = (Wt.data_ptr(), N, scg[gi].data_ptr(), zrg[gi].data_ptr(), self.bits, Qt.data_ptr())
+            if first or B != 128:
+                _hip.call("llj_gptq_block_bs", Hinv.data_ptr(), K, i1, B, *args, Err.data_ptr(), loss.data_ptr(), s)
+            else:  # the update and the block in one launch
+                _hip.call("llj_gptq_next", Hinv.data_ptr(), K, i1, Err.data_ptr(), *args, Err_next.data_ptr(), loss.data_ptr(), s)
+                Err, Err_next = Err_next, Err
         with torch.device(self.dev):  # (made on the host, its transposed empty codes took longer than the rest of this function)
             q_module = ColBlockQuantizedLinear(self.linear_module.in_features, self.linear_module.out_features,
                                                self.linear_module.bias is not None, bits=self.bits, tile_cols=self.groupsize)

@@ -587,6 +587,36 @@ def test_block_update_kernel(hip, N, K, i1, blk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("small", [1.0, 2.0 ** -70])  # quotients by reciprocals, and by divisions
+@pytest.mark.parametrize("N,K,i1", [(1, 256, 128), (37, 384, 128), (130, 384, 256), (4100, 512, 128)])
+def test_update_and_next_block_in_one_launch(hip, N, K, i1, small):
+    """llj_gptq_next is llj_gptq_update followed by llj_gptq_block, bit for bit: row counts off the tiles, off the 16 rows of a
+    workgroup and off four, the matrix's last block, later columns of one and of several tiles."""
+    from lit_llama import _hip
+    g = torch.Generator(device=dev).manual_seed(N)
+    hinv = torch.triu(torch.randn(K, K, generator=g, device=dev) * 0.02)
+    hinv.diagonal().uniform_(0.1, 3, generator=g)
+    w = torch.randn(K, N, generator=g, device=dev) * small
+    last = torch.randn(128, N, generator=g, device=dev) * small
+    scale = (torch.rand(N, generator=g, device=dev) * 0.3 + 0.05) * small
+    zero = torch.randint(4, 12, (N,), generator=g, device=dev).float()
+
+    def outputs():
+        return w.clone(), torch.full((K, N), 7.0, device=dev), torch.empty(128, N, device=dev), torch.zeros(N, device=dev)
+
+    w1, q1, e1, l1 = outputs()
+    _hip.call("llj_gptq_update", hinv.data_ptr(), K, i1 - 128, 128, last.data_ptr(), N, w1.data_ptr(), _st())
+    _hip.call("llj_gptq_block", hinv.data_ptr(), K, i1, w1.data_ptr(), N, scale.data_ptr(), zero.data_ptr(), 4, q1.data_ptr(), e1.data_ptr(),
+              l1.data_ptr(), _st())
+    w2, q2, e2, l2 = outputs()
+    _hip.call("llj_gptq_next", hinv.data_ptr(), K, i1, last.data_ptr(), w2.data_ptr(), N, scale.data_ptr(), zero.data_ptr(), 4, q2.data_ptr(),
+              e2.data_ptr(), l2.data_ptr(), _st())
+    torch.cuda.synchronize()
+    assert torch.equal(q1, q2) and torch.equal(e1, e2) and torch.equal(l1, l2)
+    assert torch.equal(w1[i1 + 128:], w2[i1 + 128:]) and torch.equal(w2[:i1 + 128], w[:i1 + 128])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bits,sym", [(4, False), (8, True), (2, False)])
 def test_row_parameters_kernel(hip, bits, sym):
     """find_params_weight on the device against the host's: rows of one sign, of zeros, with NaN and infinities."""
