@@ -77,29 +77,59 @@ __global__ __launch_bounds__(256) void gptq_update_kernel(const float* __restric
 // columns reversed, H = L L^T gives U as L^-1 reversed -- one elimination instead of two factorizations and a product. Blocks of 128
 // columns; step k turns row block k of [H | I] into P_k = L_kk^-1 [X_k | H_k] (gptq_panel_kernel) and takes P_k[:, i]^T P_k off every
 // later row block i (gptq_step_kernel): in H's upper triangle the next matrix to factor, in the lower one the growing L^-1.
-// The next diagonal block is factored by one workgroup of that launch while the others work on the rest: its chain of 128 pivots (about
-// 35 us) bounds a step, the products (2 K^3 / 3 in all, 0.3 ms at K = 4096) run beside it. K = 4096: 1.7 ms for 29.2 with the library's
-// three calls, K = 512: 0.18 for 3.1; error against float64 2.5e-7 for 1.1e-6 (8,192 rows).
+// The next diagonal block is factored by one workgroup of that launch while the others work on the rest: its chain (1.4 us
+// for its loads, 4 for its product, four times 2.9 for 32 pivots, 1.7 between them, 2 for the stores) bounds a step, the products (2 K^3 / 3 in
+// all, 0.3 ms at K = 4096) run beside it. K = 4096: 1.27 ms (39.6 us a step; 1.49 with the block's whole product, the other waves' updates before
+// the elimination and 4-byte stores) for 29.2 with the library's three calls, K = 512: 0.14 (35 a step; 0.17) for 3.1; error against float64 2.5e-7 for 1.1e-6 (8,192 rows).
 constexpr int kFs = kFactor + 16;  // LDS row stride of the diagonal block
 
 __device__ __forceinline__ float lane_value(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
 
 // S (LDS, 128 x 128, upper triangle, zeros below) -> L^-1 in the lower triangle with zeros above, S = L L^T. 32 columns at a time: one wave eliminates
-// the 32 x 32 block in registers (lane c a column of the block, lane 32 + c of the identity), the matrix cores do the rest.
+// the 32 x 32 block in registers (lane c a column of the block, lane 32 + c of the identity, which lies in the rows' padding), the matrix cores do
+// the rest: the other waves' products of one turn run beside the next turn's elimination, whose block that wave brings up to date itself.
 // Returns false (in every thread) if a pivot was not a positive normal number.
 __device__ __forceinline__ bool factor_block(float* S, int* bad) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c16 = lane & 15;
   if (tid == 0) *bad = 0;
+  for (int i = tid; i < 64 * 16; i += 256) S[(i >> 4) * kFs + kFactor + (i & 15)] = (i >> 4 & 31) == (i >> 9) * 16 + (i & 15) ? 1.f : 0.f;
+  auto update = [&](int s, int ib, int jb) {  // block (ib, jb) less its product of row block s
+    const float* p = S + 32 * s * kFs;
+    float* o = S + 32 * ib * kFs + 32 * jb;
+    f32x4 d[2][2] = {}, old[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[i][j][r] = o[(16 * i + 4 * q + r) * kFs + 16 * j + c16];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          d[i][j] = mma4(p[(4 * k + q) * kFs + 32 * ib + 16 * i + c16], p[(4 * k + q) * kFs + 32 * jb + 16 * j + c16], d[i][j]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * i + 4 * q + r, col = 16 * j + c16;
+          o[row * kFs + col] = ib == jb && row > col ? 0.f : old[i][j][r] - d[i][j][r];
+        }
+  };
   for (int s = 0; s < 4; ++s) {
     __syncthreads();
     if (wave == 0) {
+      if (s) update(s - 1, s, s);
       const int c = lane & 31;
       float* d = S + 32 * s * kFs + 32 * s;
+      const float* from = lane < 32 ? d + c : S + (c >> 4) * 32 * kFs + kFactor + (c & 15);
       float v[32];
 #pragma unroll
-      for (int i = 0; i < 32; ++i) v[i] = d[i * kFs + c];
-#pragma unroll
-      for (int i = 0; i < 32; ++i) v[i] = lane < 32 ? (i <= c ? v[i] : 0.f) : (i == c ? 1.f : 0.f);
+      for (int i = 0; i < 32; ++i) v[i] = from[i * kFs];
       bool ok = true;
 #pragma unroll
       for (int j = 0; j < 32; ++j) {
@@ -121,6 +151,13 @@ __device__ __forceinline__ bool factor_block(float* S, int* bad) {
         for (int i = 0; i < 32; ++i) d[i * kFs + c] = v[i];
       }
       if (!ok && lane == 0) *bad = 1;
+    } else if (s) {
+      int n = 0;
+      for (int ib = s; ib < 4; ++ib)
+        for (int jb = 0; jb < 4; ++jb) {
+          if ((jb >= s && jb < ib) || (ib == s && jb == s)) continue;
+          if (n++ % 3 == wave - 1) update(s - 1, ib, jb);
+        }
     }
     __syncthreads();
     if (wave != s) {  // the other 32-column blocks of these rows, times the block's inverse
@@ -141,60 +178,99 @@ __device__ __forceinline__ bool factor_block(float* S, int* bad) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) b[(16 * i + 4 * q + r) * kFs + 16 * j + c16] = o[i][j][r];
     }
-    __syncthreads();
-    int n = 0;
-    for (int ib = s + 1; ib < 4; ++ib)
-      for (int jb = 0; jb < 4; ++jb) {
-        if (jb > s && jb < ib) continue;
-        if ((n++ & 3) != wave) continue;
-        const float* p = S + 32 * s * kFs;
-        float* o = S + 32 * ib * kFs + 32 * jb;
-        f32x4 d[2][2] = {}, old[2][2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) old[i][j][r] = o[(16 * i + 4 * q + r) * kFs + 16 * j + c16];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-              d[i][j] = mma4(p[(4 * k + q) * kFs + 32 * ib + 16 * i + c16], p[(4 * k + q) * kFs + 32 * jb + 16 * j + c16], d[i][j]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[(16 * i + 4 * q + r) * kFs + 16 * j + c16] = old[i][j][r] - d[i][j][r];
-      }
   }
   __syncthreads();
   return *bad == 0;
 }
 
-// the factored block: its rows of P (zeros above the diagonal) and transposed for the panel product
+// the factored block: its rows of P (zeros above the diagonal) and transposed for the panel product, in whole vectors (4-byte stores: 7.8 us)
 __device__ __forceinline__ void put_block(const float* S, int k, int K, float* __restrict__ P, float* __restrict__ xt, bool ok, int* info) {
-  const int j = threadIdx.x & 127;
-#pragma unroll 8
-  for (int i = threadIdx.x >> 7; i < kFactor; i += 2) {
-    const float a = S[i * kFs + j], t = S[j * kFs + i];
-    P[((size_t)k * kFactor + i) * K + (size_t)k * kFactor + j] = j <= i ? a : 0.f;
-    xt[i * kFactor + j] = i <= j ? t : 0.f;
+  const int tid = threadIdx.x;
+#pragma unroll
+  for (int b = 0; b < kFactor / 8; ++b) {
+    const int i = 8 * b + (tid >> 5), j = 4 * (tid & 31);
+    f32x4 v = *reinterpret_cast<const f32x4*>(S + i * kFs + j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = j + e <= i ? v[e] : 0.f;
+    *reinterpret_cast<f32x4*>(P + ((size_t)k * kFactor + i) * K + (size_t)k * kFactor + j) = v;
   }
-  if (!ok && threadIdx.x == 0) *info = 1;
+#pragma unroll
+  for (int b = 0; b < kFactor / 8; ++b) {  // 16 columns of 16 rows a wave
+    const int i = 16 * (b >> 1) + (tid & 15), j = 64 * (b & 1) + 4 * (tid >> 4);
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = i <= j + e ? S[(j + e) * kFs + i] : 0.f;
+    *reinterpret_cast<f32x4*>(xt + i * kFactor + j) = v;
+  }
+  if (!ok && tid == 0) *info = 1;
 }
 
-// M (upper triangle) = H in the reversed order of perm (null: 0, 1, ..) with damp on the diagonal
+// S (LDS) = the upper triangle of M's diagonal block at r0 less X^T X, X: P's 128 x 128 block there, zeros below. Wave W: rows W and 7 - W of the
+// MFMA tiles, 9 of the triangle's 36.
+template <int W>
+__device__ __forceinline__ void diagonal_block(const float* __restrict__ M, const float* __restrict__ p, int r0, int K, float* S) {
+  const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, c = lane & 15;
+  f32x4 x[16], acc[9], old[9];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) x[i] = *reinterpret_cast<const f32x4*>(p + (size_t)(8 * i + (tid >> 5)) * K + r0 + 4 * (tid & 31));
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int t = 0; t < 9; ++t) f(t, t < 8 - W ? W : 7 - W, t < 8 - W ? W + t : t - 1);
+  };
+  each([&](int t, int m, int n) {
+    acc[t] = f32x4{};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) old[t][r] = M[(size_t)(r0 + 16 * m + 4 * q + r) * K + r0 + 16 * n + c];
+  });
+#pragma unroll
+  for (int i = 0; i < 16; ++i) *reinterpret_cast<f32x4*>(S + (8 * i + (tid >> 5)) * kFs + 4 * (tid & 31)) = x[i];
+  __syncthreads();
+  float v[2][8];  // tile columns W .. 7 of four k: both operands' values
+  auto read = [&](int s) {
+#pragma unroll
+    for (int j = W; j < 8; ++j) v[s & 1][j] = S[(4 * s + q) * kFs + 16 * j + c];
+  };
+  read(0);
+#pragma unroll
+  for (int s = 0; s < kFactor / 4; ++s) {
+    if (s + 1 < kFactor / 4) read(s + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    each([&](int t, int m, int n) { acc[t] = mma4(v[s & 1][m], v[s & 1][n], acc[t]); });
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) *reinterpret_cast<f32x4*>(S + (8 * i + (tid >> 5)) * kFs + 4 * (tid & 31)) = f32x4{};
+  __syncthreads();
+  each([&](int t, int m, int n) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * m + 4 * q + r, j = 16 * n + c;
+      if (j >= i) S[i * kFs + j] = old[t][r] - acc[t][r];
+    }
+  });
+}
+
+// M (upper triangle) = H in the reversed order of perm (null: 0, 1, ..) with damp on the diagonal, a row to a workgroup. ROW: through LDS, where the
+// gather costs least (4,096 columns: 74 us from memory).
+template <bool ROW>
 __global__ __launch_bounds__(256) void gptq_order_kernel(const float* __restrict__ H, const int64_t* __restrict__ perm, const float* __restrict__ damp,
                                                          int K, float* __restrict__ M) {
-  const int a = blockIdx.y, b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= K || b < a) return;
-  const int ra = K - 1 - a, rb = K - 1 - b;
-  const size_t i = perm ? (size_t)perm[ra] : ra, j = perm ? (size_t)perm[rb] : rb;
-  M[(size_t)a * K + b] = a == b ? H[i * K + j] + *damp : H[i * K + j];
+  extern __shared__ __align__(16) float row[];
+  const int a = blockIdx.x, ra = K - 1 - a;
+  const size_t i = perm ? (size_t)perm[ra] : ra;
+  const float* h = H + i * K;
+  const float d = *damp;
+  if (ROW) {
+    for (int b = threadIdx.x; b < K; b += 256) row[b] = h[b];
+    __syncthreads();
+  }
+#pragma unroll 4
+  for (int b = a + threadIdx.x; b < K; b += 256) {
+    const size_t j = perm ? (size_t)perm[K - 1 - b] : K - 1 - b;
+    const float v = ROW ? row[j] : h[j];
+    M[(size_t)a * K + b] = a == b ? v + d : v;
+  }
 }
 
 __global__ __launch_bounds__(256) void gptq_first_kernel(const float* __restrict__ M, int K, float* __restrict__ P, float* __restrict__ xt, int* info) {
@@ -224,23 +300,24 @@ __global__ __launch_bounds__(256) void gptq_panel_kernel(const float* __restrict
   G::each(acc, [&](int i, int j, float v) { P[(row + m0 + i) * K + n0 + j] = v; });
 }
 
-// Workgroup 0: the next diagonal block, updated and factored. The others: 64 x 64 tiles of the rows below, the lower triangle's columns
+constexpr int kStepLds = 21000;  // floats: the diagonal block's 18,432, and more than half a CU's LDS (4,096 columns: 41.8 us a step with two to a CU, 39.6 so)
+
+// Workgroup 0, alone on its CU: the next diagonal block, updated and factored. The others: 64 x 64 tiles of the rows below, the lower triangle's columns
 // up to block k (first sums in block k's own) and the upper triangle's.
 __global__ __launch_bounds__(256) void gptq_step_kernel(float* __restrict__ M, float* __restrict__ P, int k, int K, float* __restrict__ xt, int* info) {
-  typedef AtB<128, 128, float, true, false> D;
   typedef AtB<64, 64, float, true, false> G;
-  constexpr int kS = kFactor * kFs;
-  __shared__ __align__(16) float lds[kS > D::kLds ? kS : D::kLds];
+  __shared__ __align__(16) float lds[kStepLds];
   __shared__ int bad;
   const float* p = P + (size_t)k * kFactor * K;
   const int r0 = (k + 1) * kFactor;
   if (blockIdx.x == 0) {
     __builtin_amdgcn_s_setprio(3);  // the longest chain of the launch, beside another workgroup's products
-    f32x4 acc[D::MI][D::NI], old[D::MI][D::NI];
-    D::run(p + r0, K, kFactor, p + r0, K, kFactor, kFactor, 1.f, lds, acc,
-           [&] { D::load(old, [&](int i, int j) { return M[(size_t)(r0 + i) * K + r0 + j]; }); });
-    __syncthreads();
-    D::both(acc, old, [&](int i, int j, float v, float m) { lds[i * kFs + j] = j >= i ? m - v : 0.f; });
+    switch (uniform(threadIdx.x >> 6)) {  // (the same barriers on every way)
+      case 0: diagonal_block<0>(M, p, r0, K, lds); break;
+      case 1: diagonal_block<1>(M, p, r0, K, lds); break;
+      case 2: diagonal_block<2>(M, p, r0, K, lds); break;
+      default: diagonal_block<3>(M, p, r0, K, lds);
+    }
     const bool ok = factor_block(lds, &bad);
     put_block(lds, k + 1, K, P, xt, ok, info);
     return;
@@ -357,7 +434,8 @@ int llj_gptq_factor(const float* H, const int64_t* perm, const float* damp, int 
   LLJ_REQUIRE((((uintptr_t)M | (uintptr_t)P | (uintptr_t)xt) & 15) == 0);
   const hipStream_t s = (hipStream_t)stream;
   const int nb = K / kFactor;
-  hipLaunchKernelGGL(gptq_order_kernel, dim3((K + 255) / 256, K), dim3(256), 0, s, H, perm, damp, K, M);
+  if (K <= 16384) hipLaunchKernelGGL(gptq_order_kernel<true>, dim3(K), dim3(256), (size_t)K * 4, s, H, perm, damp, K, M);
+  else hipLaunchKernelGGL(gptq_order_kernel<false>, dim3(K), dim3(256), 0, s, H, perm, damp, K, M);
   hipLaunchKernelGGL(gptq_first_kernel, dim3(1), dim3(256), 0, s, M, K, P, xt, info);
   for (int k = 0; k < nb; ++k) {
     hipLaunchKernelGGL(gptq_panel_kernel, dim3(K / 64 * 2), dim3(256), 0, s, M, xt, k, K, P);

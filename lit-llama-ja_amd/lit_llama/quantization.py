@@ -528,7 +528,7 @@ class GPTQQuantizer:
         """The upper Cholesky factor of the damped H's inverse, columns in the order of perm (reference 549-566).
 
         One elimination of our own where the calibration rows determine H well (half as many again as columns): 4,096 columns
-        1.7 ms for 29.5 with the library's two factorizations and inverse, its error against float64 2.5e-7 for 1.1e-6. With
+        1.3 ms for 29.5 with the library's two factorizations and inverse, its error against float64 2.5e-7 for 1.1e-6. With
         fewer rows H is damping in most directions and the error feedback amplifies any rounding (other correct factors change
         1 to 5 % of the codes at 4,096 columns, 0.2 % from there on): those keep the library's. So does an H whose elimination
         meets a pivot that is not positive and normal, so that it is the library that decides whether that is an error."""
