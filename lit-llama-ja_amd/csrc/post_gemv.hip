@@ -2,7 +2,7 @@
 //
 // One row runs on rowdot.h, also as the residual streams (llj_streams_linear); 2 to 8 rows run on rows_gemv_kernel. 9 to 16 rows, rows
 // of values that do not fit its registers, any rows with LLJ_ACT_TILES and the row that is the residual after a sublayer
-// (llj_post_linear) run on post_gemv_kernel. Output bf16, plus a bias, optionally max(., 0)^2 or the clamped gated unit of
+// (llj_post_linear) run on post_gemv_kernel, 2 to 8 such rows (llj_post_rows) on post_rows_kernel. Output bf16, plus a bias, optionally max(., 0)^2 or the clamped gated unit of
 // interleaved columns (elem.h).
 #include <algorithm>
 #include <type_traits>
@@ -16,7 +16,7 @@ namespace llj {
 
 struct PostGemvParams {
   const bf16_t* A;  // plain: rows, stride lda
-  int lda;
+  int lda, ldt, ldx;  // post: row strides of t, of x and x'
   const bf16_t* t;  // post: sublayer output (C), norm weight (C), residual in / out (C)
   const bf16_t* w;
   const float* x;
@@ -372,6 +372,156 @@ static int post_gemv_launch(const PostGemvParams& p, int act, hipStream_t s) {
   }
 }
 
+// 2 to 8 rows that are the fp32 residual after a sublayer (as above for one), to the bits of postnorm.hip's launch and the plain form: row by row the
+// same sums over the same threads, the product's chunks on the same waves in the same order.
+// Bound: the weights' bytes. A launch of its own for the norm costs 2 to 2.7 us; here every workgroup forms the rows under its first weights in
+// flight, so that a CU's share of the columns is one workgroup: TW tiles side by side, NW waves and all their chunks (n = D, or D ahead) each, and past
+// 256 workgroups one such group after another. us in a graph, norm + product -> this (the product alone):
+//   2 rows: 2048 -> 8448 11.3 -> 9.5 (9.1)   2048 -> 6272 9.7 -> 7.2 (7.1)   4096 -> 16512 26.0 -> 23.3 (22.8)   4096 -> 12544 21.7 -> 18.9 (19.9)
+//   8 rows: 2048 -> 8448 11.8 -> 11.9 (9.6)  2048 -> 6272 9.8 -> 9.6 (7.5)   4096 -> 16512 27.6 -> 26.8 (25.0)   4096 -> 12544 23.3 -> 22.5 (20.4)
+// and of a program of 32 steps, whose rows come from other XCDs: 1B, 2 / 3 / 5 / 8 sequences 38.5 / 39.3 / 38.4 / 40.7 -> 35.1 / 37.0 / 37.3 / 39.4 ms, 7B,
+// 2 / 3 / 8 107.4 / 108.6 / 113.0 -> 101.5 / 105.0 / 110.9. (2048 -> 8448, 8 rows, with two tiles: 264 workgroups, 15.9; at 128 registers 19.6.)
+template <int NW, int TW, int D, int NV, int MR, int ACT, bool MORE>
+__global__ __launch_bounds__(NW * TW * 64) void post_rows_kernel(PostGemvParams p, int rounds) {
+  constexpr int NT = NW * TW * 64, RH = (MR + NT / 256 - 1) / (NT / 256);  // rows to 256 threads
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int K = p.K, KC = K >> 7, AS = K + 8;  // (rows 4 banks apart)
+  unsigned char* patch = smem;                                                      // [waves][4096] a chunk of weights each
+  float* rs = reinterpret_cast<float*>(smem + NW * TW * 4096);                      // [MR][4]
+  bf16_t* As = reinterpret_cast<bf16_t*>(smem + NW * TW * 4096 + MR * 16);          // [MR][AS]
+  float* red = reinterpret_cast<float*>(As + (size_t)MR * AS);                      // [rounds > 1 ? 2 : 1][waves][64][4]
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), team = wave / NW, w = wave % NW;
+  const int row = lane & 15, g = lane >> 4, tiles = p.N >> 4, step = gridDim.x * TW, first = blockIdx.x * TW + team;
+  unsigned char* mine = patch + wave * 4096;
+  u32x4 wr[D][4];
+  // (a load past the last tile fetches nothing, so that the count of loads in flight is the same everywhere)
+  const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 2 * p.N * K, 0x00020000);
+  const int lane_at = 2 * (g * K + 8 * row);
+  auto load = [&](int d, int tile, int c) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int at = tile < tiles ? lane_at + 2 * (tile * 16 + 4 * s) * K + 256 * c : 0x7ffffff0;
+      wr[d][s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(weights, at, 0, 2));  // non-temporal
+    }
+  };
+  // ---- the rows
+  const int part = tid >> 8, lt = tid & 255;
+  {
+    u32x4 tv[RH][NV], gv[NV];
+    float xv[RH][NV][8];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int k = 8 * (lt + 256 * v), kk = k < p.C ? k : 0;
+      gv[v] = *reinterpret_cast<const u32x4*>(p.w + kk);
+#pragma unroll
+      for (int r = 0; r < RH; ++r) {
+        const int m = part * RH + r < p.M ? part * RH + r : 0;
+        tv[r][v] = *reinterpret_cast<const u32x4*>(p.t + (size_t)m * p.ldt + kk);
+        ld8(p.x + (size_t)m * p.ldx + kk, xv[r][v]);
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, first, w + NW * d);
+#pragma unroll
+    for (int r = 0; r < RH; ++r) {
+      float ss = 0.f;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const bool in = 8 * (lt + 256 * v) < p.C;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float tt = (e & 1) ? bfhi(tv[r][v][e >> 1]) : bflo(tv[r][v][e >> 1]);
+          ss += in ? tt * tt : 0.f;
+        }
+      }
+      ss = wave_sum(ss);
+      if (lane == 0 && part * RH + r < MR) rs[(part * RH + r) * 4 + (wave & 3)] = ss;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RH; ++r) {
+      const int m = part * RH + r;
+      if (m >= MR) break;  // (uniform)
+      const f32x4 q = *reinterpret_cast<const f32x4*>(rs + 4 * m);
+      const float f = 1.f / sqrtf((q[0] + q[1] + q[2] + q[3]) / (float)p.C + p.eps);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const int k = 8 * (lt + 256 * v);
+        if (k >= K) continue;
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float tt = (e & 1) ? bfhi(tv[r][v][e >> 1]) : bflo(tv[r][v][e >> 1]);
+          const float gg = (e & 1) ? bfhi(gv[v][e >> 1]) : bflo(gv[v][e >> 1]);
+          o[e] = k < p.C ? xv[r][v][e] + tt * f * (1.f + gg) : 0.f;
+        }
+        st8(As + (size_t)m * AS + k, o);
+        if (k < p.C && m < p.M && (unsigned)(k >> 3) % gridDim.x == blockIdx.x) st8(p.xo + (size_t)m * p.ldx + k, o);
+      }
+    }
+    __syncthreads();
+  }
+  // ---- the products
+  const bf16_t* a0 = As + (size_t)(row & (MR - 1)) * AS + 8 * g;
+  const int n = KC / NW;  // a multiple of D
+  for (int t = 0; t < rounds; ++t) {
+    const int tile = first + t * step;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < n; i0 += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int c = w + NW * (i0 + d);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) *reinterpret_cast<u32x4*>(mine + 256 * (4 * s + g) + 16 * (row ^ (4 * s + g))) = wr[d][s];
+        const bool next = i0 + D >= n;  // (uniform) this chunk's registers take the next tile's
+        if (MORE) load(d, !next ? tile : t + 1 < rounds ? tile + step : tiles, next ? w + NW * d : c + NW * D);
+        u32x4 wt[4], a[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          wt[s] = *reinterpret_cast<const u32x4*>(mine + 256 * row + 16 * ((4 * s + g) ^ row));
+          a[s] = *reinterpret_cast<const u32x4*>(a0 + 128 * c + 32 * s);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = mfma_bf16(__builtin_bit_cast(bf16x8, a[s]), __builtin_bit_cast(bf16x8, wt[s]), acc);
+      }
+    }
+    float* sums = red + (t & 1) * NW * TW * 256;
+    *reinterpret_cast<f32x4*>(sums + (wave * 64 + lane) * 4) = acc;
+    __syncthreads();
+    for (int i = tid; i < TW * p.M * 16; i += NT) {
+      const int c = i & 15, m = (i >> 4) % p.M, tm = (i >> 4) / p.M, at = blockIdx.x * TW + tm + t * step;
+      float y = 0.f;
+#pragma unroll
+      for (int q = 0; q < NW; ++q) y += sums[((tm * NW + q) * 64 + (m >> 2) * 16 + c) * 4 + (m & 3)];
+      if (ACT == 1) y = fmaxf(y, 0.f) * fmaxf(y, 0.f);
+      if (at < tiles) p.out[(size_t)m * p.ldo + 16 * at + c] = f2bf(y);
+    }
+  }
+}
+
+template <int NW, int TW, int D, int NV, int MR>
+static int post_rows_go(const PostGemvParams& p, int act, hipStream_t s) {
+  const int units = (p.N / 16 + TW - 1) / TW, rounds = (units + 255) / 256, grid = (units + rounds - 1) / rounds;
+  const size_t lds = NW * TW * 4096 + MR * 16 + (size_t)MR * (p.K + 8) * 2 + (size_t)(rounds > 1 ? 2 : 1) * NW * TW * 1024;
+  auto go = [&](auto kern) -> int {
+    if (lds > 64 * 1024) {
+      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * TW * 64), lds, s, p, rounds);
+    LLJ_CHECK_LAUNCH();
+    return 0;
+  };
+  const bool more = rounds > 1 || p.K / 128 / NW > D;
+  if (act) return more ? go(post_rows_kernel<NW, TW, D, NV, MR, 1, true>) : go(post_rows_kernel<NW, TW, D, NV, MR, 1, false>);
+  return more ? go(post_rows_kernel<NW, TW, D, NV, MR, 0, true>) : go(post_rows_kernel<NW, TW, D, NV, MR, 0, false>);
+}
+template <int NW, int TW, int D, int NV>
+static int post_rows_m(const PostGemvParams& p, int act, hipStream_t s) {
+  if (p.M <= 2) return post_rows_go<NW, TW, D, NV, 2>(p, act, s);
+  return p.M <= 4 ? post_rows_go<NW, TW, D, NV, 4>(p, act, s) : post_rows_go<NW, TW, NW == 8 ? 2 : D, NV, 8>(p, act, s);  // (8 rows of 4096: registers)
+}
+
 constexpr int kPostMaxK = 28544;  // widest weight rows of the post form, whose row lies in LDS (96 KB with the waves' patches); llj_streams_linear keeps the same limit
 
 template <int PRO>
@@ -426,6 +576,24 @@ int llj_post_linear(int act, const void* t, const void* norm_w, float eps, const
   const int nt = post_threads(K), nv = (C / 8 + nt - 1) / nt;
   if (nv <= 1) return post_gemv_launch<1>(p, act, s);
   return post_gemv_launch<2>(p, act, s);  // C <= 8192 over 512 threads, C <= 4096 over 256
+}
+
+// whole rounds of chunks for every wave, and not the half-K forms' widths
+int llj_post_rows_ok(int M, int N, int K, int C) {
+  return M >= 2 && M <= 8 && C > 0 && C % 8 == 0 && C <= K && (K == 2048 || K == 4096) && N >= 4096 && N % 16 == 0 && N < (1 << 29) / K;
+}
+
+int llj_post_rows(int act, const void* t, int ldt, const void* norm_w, float eps, const float* x, float* x_out, int ldx, int C, const void* W,
+                  void* out, int ldo, int M, int N, int K, void* stream) {
+  LLJ_REQUIRE((act == 0 || act == 1) && t && norm_w && x && x_out && x != x_out && W && out && llj_post_rows_ok(M, N, K, C) && ldt >= C && ldx >= C &&
+              ldo >= N && (ldt & 7) == 0 && (ldx & 3) == 0 &&
+              (((uintptr_t)t | (uintptr_t)norm_w | (uintptr_t)x | (uintptr_t)x_out | (uintptr_t)W) & 15) == 0);
+  PostGemvParams p{};
+  p.t = (const bf16_t*)t; p.ldt = ldt; p.w = (const bf16_t*)norm_w; p.x = x; p.xo = x_out; p.ldx = ldx; p.eps = eps; p.C = C;
+  p.W = (const bf16_t*)W; p.out = (bf16_t*)out; p.ldo = ldo; p.M = M; p.N = N; p.K = K;
+  hipStream_t s = (hipStream_t)stream;
+  if (K == 2048) return N <= 8192 ? post_rows_m<4, 2, 4, 1>(p, act, s) : post_rows_m<4, 3, 4, 1>(p, act, s);
+  return post_rows_m<8, 1, 4, 2>(p, act, s);
 }
 
 int llj_streams_linear_ok(int streams, int C) { return streams >= 1 && streams <= kRdStreams && C % 8 == 0 && C > 0 && C <= 8192; }

@@ -117,14 +117,21 @@ class PackedLinear:
 
     def takes_post(self, M: int, width: int) -> bool:
         """Whether apply_post serves these rows."""
-        return self.dtype == torch.bfloat16 and M == 1 and width == self.K and width % 8 == 0 and width <= 8192
+        if self.dtype != torch.bfloat16 or width != self.K:
+            return False
+        if M == 1:
+            return width % 8 == 0 and width <= 8192
+        return self.tiles and self.bias is None and bool(_hip.lib().llj_post_rows_ok(M, self.Np, self.Kp, width))
 
-    def apply_post(self, t: torch.Tensor, norm: torch.Tensor, eps: float, x: torch.Tensor, x_out: torch.Tensor,
+    def apply_post(self, t: torch.Tensor, norm: torch.Tensor, eps: float, x: torch.Tensor, x_out: torch.Tensor, M: int,
                    out: torch.Tensor, st, relu2: bool = False) -> None:
-        """One row: x_out = x + norm(t) and out = x_out . W^T in one launch."""
-        _hip.call("llj_post_linear", int(relu2), t.data_ptr(), norm.data_ptr(), eps, x.data_ptr(), x_out.data_ptr(), self.K,
-                  self.w.data_ptr(), out.data_ptr(), self.Np, self.Kp, st)
-
+        """M rows: x_out = x + norm(t) and out = x_out . W^T in one launch."""
+        if M == 1:
+            _hip.call("llj_post_linear", int(relu2), t.data_ptr(), norm.data_ptr(), eps, x.data_ptr(), x_out.data_ptr(), self.K,
+                      self.w.data_ptr(), out.data_ptr(), self.Np, self.Kp, st)
+            return
+        _hip.call("llj_post_rows", int(relu2), t.data_ptr(), t.stride(0), norm.data_ptr(), eps, x.data_ptr(), x_out.data_ptr(),
+                  x.stride(0), self.K, self.w.data_ptr(), out.data_ptr(), out.stride(0), M, self.Np, self.Kp, st)
 
     def takes_streams(self, M: int, width: int, streams: int) -> bool:
         """Whether apply_streams serves these rows (7B: 6,272 columns 15.5 us against 16.4 with a launch of their own for the

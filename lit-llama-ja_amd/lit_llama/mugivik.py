@@ -27,6 +27,9 @@ from .state import Rows, SequenceState
 from .utils import find_multiple
 
 
+POST_ROWS = 8  # most rows of a product that closes the pending norm itself
+
+
 @dataclass(frozen=True)
 class MugivikLayer:
     mixer: object  # GLASpec or LatentSpec
@@ -108,7 +111,7 @@ class _Work(Scratch):
         # mixer outputs by width: padding columns stay zero
         self.y = {n: torch.zeros(M, lane_pad(n, dt), dtype=dt, device=dev) for n in {mx.out_width() for mx in m.mixers}}
         self.cur: dict = {}  # this call's latents by layer (prompt rows)
-        self.x2 = torch.empty_like(self.x) if M == 1 else None  # the residual's other place (fused post-norm products)
+        self.x2 = torch.empty_like(self.x) if M <= POST_ROWS else None  # the residual's other place (fused post-norm products)
 
 
 @register("Mugivik")
@@ -215,7 +218,7 @@ class Mugivik(HybridModel):
         copy of the residual after every layer.
 
         A sublayer leaves its output in w.t with its norm pending; the next product over the residual
-        closes it, in its own launch for one row (PackedLinear.apply_post) or in one before it."""
+        closes it, in its own launch for few rows (PackedLinear.apply_post) or in one before it."""
         M, C, eps = rows.M, self.config.n_embd, self.config.eps
         self._embed(rows, w, state, st)
         x, pending = w.x, None
@@ -231,7 +234,7 @@ class Mugivik(HybridModel):
             nonlocal x, pending
             if pending is not None and lin.takes_post(M, C) and taps is None:
                 other = w.x2 if x is w.x else w.x
-                lin.apply_post(w.t, pending, eps, x, other, out, st, relu2)
+                lin.apply_post(w.t, pending, eps, x, other, M, out, st, relu2)
                 x, pending = other, None
                 return
             if pending is not None:

@@ -153,6 +153,33 @@ def test_rows_on_tiles(hip, N, K, act):
         assert torch.equal(post, rows[8][0])
 
 
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 8])
+@pytest.mark.parametrize("K,C,N", [(2048, 2048, 4096), (2048, 1928, 8192), (2048, 2048, 8224), (2048, 2048, 12320), (4096, 4096, 4112), (4096, 3976, 8448)])
+def test_post_rows(hip, K, C, N, M):
+    """The residual's norm in front of 2 to 8 rows' product is the norm's launch and the product on the tiles, bit for bit: widths with and
+    without padding, one pair (or three) of column tiles to a workgroup and several in turn, the last one partial; nothing outside."""
+    from lit_llama import _hip
+
+    g = torch.Generator(device="cuda").manual_seed(N + M)
+    W = torch.zeros(N, K, dtype=torch.bfloat16, device="cuda")
+    W[:, :C] = torch.randn(N, C, generator=g, device="cuda") * C ** -0.5
+    t = torch.full((M, K + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    t[:, :C] = torch.randn(M, C, generator=g, device="cuda")
+    w = (0.3 * torch.randn(C, generator=g, device="cuda")).to(torch.bfloat16)
+    x = torch.full((M, C + 8), float("nan"), device="cuda")
+    x[:, :C] = torch.randn(M, C, generator=g, device="cuda")
+    for act in (0, 1):
+        xn, xb, xo = x.clone(), torch.empty(M, K, dtype=torch.bfloat16, device="cuda"), torch.full((M + 1, C + 8), 3.0, device="cuda")
+        want = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        got = torch.full((M + 1, N + 8), 3.0, dtype=torch.bfloat16, device="cuda")
+        call("llj_post_norm", t, K + 8, w, 1e-5, xn, C + 8, xb, K, None, None, M, C, 0)
+        call("llj_rows_linear", act | _hip.ACT_TILES, xb, K, W, None, want, N, M, N, K, 0.0, 0.0)
+        call("llj_post_rows", act, t, K + 8, w, 1e-5, x, xo, C + 8, C, W, got, N + 8, M, N, K)
+        assert torch.equal(got[:M, :N], want) and torch.equal(xo[:M, :C], xn[:, :C])
+        assert float((got[M] - 3.0).abs().max()) == 0.0 and float((got[:, N:] - 3.0).abs().max()) == 0.0
+        assert float((xo[M] - 3.0).abs().max()) == 0.0 and float((xo[:, C:] - 3.0).abs().max()) == 0.0
+
+
 @pytest.mark.parametrize("M", [1, 7, 40, 64, 154, 255])
 def test_packed_linear_on_tiles(hip, M):
     """PackedLinear(tiles=True): rows and prompts below 256 rows as the tiles and the unsplit product give them, bit for bit."""
