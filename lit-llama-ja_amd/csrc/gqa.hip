@@ -37,8 +37,8 @@ struct GqaParams {
   float scale;
 };
 
-__device__ __forceinline__ void turn_cs(const double* __restrict__ turns, int i, int pos, float& c, float& s) {
-  const double t = (double)pos * turns[i];
+__device__ __forceinline__ void turn_cs(double turns, int pos, float& c, float& s) {
+  const double t = (double)pos * turns;
   sincospif(2.f * (float)(t - rint(t)), &s, &c);
 }
 
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void gqa_prep_kernel(GqaParams p, int LG) {
   T* row = (T*)p.in + (size_t)m * p.ld;
   const int ps = p.pos[m], b = p.row_seq ? p.row_seq[m] : m;
   T* dst = (T*)p.cache + ((size_t)p.slot[b] * p.W + ps) * p.ldc;
-  for (int i = tid; i < n; i += 256) turn_cs(p.turns, i, ps, s_cs[i], s_cs[n + i]);
+  for (int i = tid; i < n; i += 256) turn_cs(p.turns[i], ps, s_cs[i], s_cs[n + i]);
   __syncthreads();
   const int l = tid & (LG - 1), per = 256 / LG;
   constexpr int E = VEC ? 8 : 1;
@@ -393,34 +393,11 @@ __global__ __launch_bounds__(256) void gqa_attend_kernel(GqaParams p, float* par
   const int sp = blockIdx.x, gh = blockIdx.y / HB, hb = blockIdx.y % HB, m = blockIdx.z;
   const int h0 = gh * R + 16 * hb, nh = R - 16 * hb < 16 ? R - 16 * hb : 16;
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), col = lane & 15, g = lane >> 4;
-  const int ps = p.pos[m], D = p.D, V = p.V;
-  const int steps = ps / 32 + 1, per = (steps + nsplit - 1) / nsplit;
-  const int s0 = sp * per, s1 = s0 + per < steps ? s0 + per : steps;
-  const bool owner = s0 < s1 && s1 == steps;
-  bf16_t* kb = (bf16_t*)p.cache + (size_t)p.slot[m] * p.W * p.ldc + gh * D;
-  bf16_t* vb = kb - gh * D + p.G * D + gh * V;
-  const u32x4 zero = {0, 0, 0, 0};
-  u32x4 kf[2][KT], vr[DB];
-  // (padding columns and keys past the position read a valid place; masked or multiplied by zeros)
-  auto fetch = [&](int t) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int key = 32 * t + 16 * j + col;
-      const bf16_t* kr = kb + (size_t)(key < ps ? key : ps) * p.ldc;
-#pragma unroll
-      for (int kk = 0; kk < KT; ++kk) {
-        const int c = 32 * kk + 8 * g;
-        kf[j][kk] = *reinterpret_cast<const u32x4*>(kr + (c < D ? c : 0));
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < DB; ++i) {
-      const int piece = lane + 64 * i, key = 32 * t + piece / (2 * DB), c = 8 * (piece % (2 * DB));
-      vr[i] = *reinterpret_cast<const u32x4*>(vb + (size_t)(key < ps ? key : ps) * p.ldc + (c < V ? c : 0));
-    }
-  };
-  // ---- queries and the new key: 16 lanes per head; their loads first (a lane's items as in the preparation kernel: pairs,
-  // then unrotated dimensions), then the first step's keys and values, all in flight over the angles
+  const int D = p.D, V = p.V;
+  // ---- queries and the new key: 16 lanes per head; their loads first, with the new value's (a lane's items as in the preparation
+  // kernel: pairs, then unrotated dimensions), while the position and the slot are on their way; then the first step's keys and values, all in
+  // flight over the angles. (The value's operands behind the barrier were 1 us of the owner's chain of 8: 8 ranges of 1,016
+  // keys 10.35 -> 9.9 us, the new key on another wave than the queries in that.)
   const bf16_t* row = (const bf16_t*)p.in + (size_t)m * p.ld;
   constexpr int NI = 2 * KT;  // items per lane, at most
   const int hh = tid >> 4, l = tid & 15, items = n + D - p.RD;
@@ -448,8 +425,38 @@ __global__ __launch_bounds__(256) void gqa_attend_kernel(GqaParams p, float* par
       kc[j] = ks[pair ? k + n : k];
     }
   }
+  const int vt = gh * V + (tid < V ? tid : 0);  // (V, n <= 256)
+  const bf16_t nv = row[p.ov + vt], fv = *(p.lam ? (const bf16_t*)p.first + (size_t)m * p.ldf + vt : row);
+  const float lam = *(p.lam ? p.lam : (const float*)p.cache);
+  const double turns = *(n ? p.turns + (tid < n ? tid : 0) : (const double*)p.cache);
+  const int ps = p.pos[m];
+  const int steps = ps / 32 + 1, per = (steps + nsplit - 1) / nsplit;
+  const int s0 = sp * per, s1 = s0 + per < steps ? s0 + per : steps;
+  const bool owner = s0 < s1 && s1 == steps;
+  bf16_t* kb = (bf16_t*)p.cache + (size_t)p.slot[m] * p.W * p.ldc + gh * D;
+  bf16_t* vb = kb - gh * D + p.G * D + gh * V;
+  const u32x4 zero = {0, 0, 0, 0};
+  u32x4 kf[2][KT], vr[DB];
+  // (padding columns and keys past the position read a valid place; masked or multiplied by zeros)
+  auto fetch = [&](int t) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int key = 32 * t + 16 * j + col;
+      const bf16_t* kr = kb + (size_t)(key < ps ? key : ps) * p.ldc;
+#pragma unroll
+      for (int kk = 0; kk < KT; ++kk) {
+        const int c = 32 * kk + 8 * g;
+        kf[j][kk] = *reinterpret_cast<const u32x4*>(kr + (c < D ? c : 0));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < DB; ++i) {
+      const int piece = lane + 64 * i, key = 32 * t + piece / (2 * DB), c = 8 * (piece % (2 * DB));
+      vr[i] = *reinterpret_cast<const u32x4*>(vb + (size_t)(key < ps ? key : ps) * p.ldc + (c < V ? c : 0));
+    }
+  };
   if (s0 + wave < s1) fetch(s0 + wave);
-  for (int i = tid; i < n; i += 256) turn_cs(p.turns, i, ps, cs[i], cs[n + i]);
+  if (tid < n) turn_cs(turns, ps, cs[tid], cs[n + tid]);
   for (int i = tid; i < 17 * QP / 8; i += 256) *reinterpret_cast<u32x4*>(Qs + 8 * i) = zero;
   __syncthreads();
   auto prepare = [&](const bf16_t (&a)[NI], const bf16_t (&c)[NI], bool live, bf16_t* out, bf16_t* out2) {
@@ -486,14 +493,13 @@ __global__ __launch_bounds__(256) void gqa_attend_kernel(GqaParams p, float* par
     }
   };
   prepare(qa, qc, qlive, Qs + hh * QP, nullptr);
-  if (owner && wave == 0) prepare(ka, kc, hh == 0, Kn, kb + (size_t)ps * p.ldc);
+  if (owner && wave == 3) prepare(ka, kc, hh == 12, Kn, kb + (size_t)ps * p.ldc);  // (the wave that has a query only beyond 12 heads)
   if (owner && tid < VW) {
     bf16_t o = 0;
     if (tid < V) {
-      float v = bf2f(row[p.ov + gh * V + tid]);
-      bf16_t* fr = p.first ? (bf16_t*)p.first + (size_t)m * p.ldf + gh * V + tid : nullptr;
-      if (p.lam) v = (1.f - *p.lam) * v + *p.lam * bf2f(*fr);
-      else if (fr) *fr = f2bf(v);
+      float v = bf2f(nv);
+      if (p.lam) v = (1.f - lam) * v + lam * bf2f(fv);
+      else if (p.first) ((bf16_t*)p.first)[(size_t)m * p.ldf + gh * V + tid] = f2bf(v);
       o = f2bf(v);
       vb[(size_t)ps * p.ldc + tid] = o;
     }
