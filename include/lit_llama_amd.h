@@ -142,6 +142,15 @@ int llj_attention(const void* q, const void* kcache, const void* vcache, void* y
 int llj_attention_prefill(const void* q, const void* kcache, const void* vcache, void* y, const int* pos, int B, int T,
                           int n_head, int head_size, int S, void* stream);
 
+/* One decode row in heads of 64 (8 <= n_head <= 16, C = 64 n_head): llj_attention with the heads' shares of attn.c_proj's product, parts[h][n] =
+ * sum_d y[64 h + d] W[n, 64 h + d] (fp32 [n_head][C], y rounded to bf16), W (C, C) bf16. llj_sums_swiglu adds them up. */
+int llj_attention_proj_ok(int n_head, int head_size, int S);
+int llj_attention_proj(const void* q, const void* kcache, const void* vcache, const int* pos, int n_head, int head_size, int S, const void* W,
+                       float* parts, void* stream);
+/* One row, bf16 weights (H, C), C <= 1024: x_out = x + sum of the parts (nparts <= 16 fp32 rows of C, the sum rounded to bf16), then llj_norm_swiglu
+ * of it. x_out must not be x. */
+int llj_sums_swiglu(const void* x, const float* parts, int nparts, void* x_out, const void* norm_w, float eps, const void* W1, const void* W2, void* h,
+                    int H, int C, void* stream);
 /* Split-K form of llj_attention for long caches: the valid keys of every (row, head) split into
  * nsplit equal ranges, one block each, writing unnormalized partials (outputs, max, sum) into
  * part_ws (llj_attention_ws_bytes(B*T, n_head, head_size, nsplit) bytes), merged in split order

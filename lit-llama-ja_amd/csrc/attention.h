@@ -70,10 +70,15 @@ __device__ __forceinline__ void attention_out(float v, bf16_t* __restrict__ y, u
   if (st) i8_emit_stats64(st, thr, m, h * HS + (d & ~63), ob, h);  // (uniform)
 }
 
+// also(): loads of the caller's, behind the first keys' and the query's. KEEP: the head's outputs, rounded to bf16, are left in lds
+// at attention_lds_floats (HS more floats), behind a barrier, and y is not written.
+struct NoLoads {
+  __device__ __forceinline__ void operator()() const {}
+};
 // count (with PART, else partials only; nsplit <= 64): zeroed arrival counters, one per (row, head), left zero: the last of the
 // ranges' blocks to finish merges them. The hand-off is device-scope stores, a wait for them, the counter, device-scope
 // loads; no block waits for another.
-template <int HS, int U, int NTH, bool PART = false, int SPECU = U / 2, bool ILV = false>
+template <int HS, int U, int NTH, bool PART = false, int SPECU = U / 2, bool ILV = false, bool KEEP = false, typename F = NoLoads>
 __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                const bf16_t* __restrict__ vc, bf16_t* __restrict__ y,
                                                const int* __restrict__ pos, int T, int S, int nh, float scale_log2,
@@ -81,7 +86,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
                                                int split = 0, float* __restrict__ part = nullptr,
                                                uint32_t* __restrict__ st = nullptr, float thr = 0.f,
                                                uint32_t* __restrict__ clr = nullptr, int clr_words = 0,
-                                               bool spec_ok = false, int* __restrict__ count = nullptr) {
+                                               bool spec_ok = false, int* __restrict__ count = nullptr, F also = F()) {
   constexpr int DPL = HS / 16;
   constexpr int NG = NTH / 16;
   constexpr int NWV = NTH / 64;
@@ -145,6 +150,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
     const size_t qo = (size_t)m * C + h * HS + sub * DPL;
     if constexpr (DPL == 8) {
       const uint4 a = *reinterpret_cast<const uint4*>(q + qo);
+      also();
       const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -153,6 +159,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
       }
     } else {
       const uint2 a = *reinterpret_cast<const uint2*>(q + qo);
+      also();
       qf[0] = bflo(a.x) * scale_log2;
       qf[1] = bfhi(a.x) * scale_log2;
       qf[2] = bflo(a.y) * scale_log2;
@@ -242,10 +249,13 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
         }
       }
       LLJ_STAMP(5);
+    } else if constexpr (KEEP) {
+      s_m[2 * NWV + NWV * HS + d] = round_bf(O / L);  // (past what is read here)
     } else {
       attention_out<HS>(O / L, y, st, thr, h, m, C);
     }
   }
+  if constexpr (KEEP) __syncthreads();
   LLJ_STAMP(5);
   if constexpr (PART) {
     if (!count) return;

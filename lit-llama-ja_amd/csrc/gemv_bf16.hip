@@ -30,6 +30,20 @@ int gemv_launch_bf16(int am, int ep, const GemvParams& p, hipStream_t s) {
 }
 }  // namespace llj
 
+using namespace llj;
+
 extern "C" {
 LLJ_TRACE_EXPORT(bf16)
+
+int llj_sums_swiglu(const void* x, const float* parts, int nparts, void* x_out, const void* norm_w, float eps, const void* W1, const void* W2, void* h,
+                    int H, int C, void* stream) {
+  LLJ_REQUIRE(x && parts && nparts >= 1 && nparts <= kRdSums && x_out && x_out != x && norm_w && W1 && W2 && h && H > 0 && C > 0 && C % 8 == 0 && C <= 1024 &&
+              (((uintptr_t)x | (uintptr_t)parts | (uintptr_t)norm_w | (uintptr_t)W1 | (uintptr_t)W2) & 15) == 0 && ((uintptr_t)x_out & 3) == 0);
+  RowDotParams r{};
+  r.A = (const bf16_t*)x; r.parts = parts; r.S = nparts; r.ao = (bf16_t*)x_out; r.w = (const bf16_t*)norm_w; r.eps = eps; r.K = r.C = C; r.N = 2 * H;
+  r.W = (const bf16_t*)W1; r.W2 = (const bf16_t*)W2; r.out = (bf16_t*)h;
+  if (nparts <= 8) return rowdot_go<2, 1, RD_SUMS + 8, RD_SWIGLU>(r, (hipStream_t)stream);
+  if (nparts <= 10) return rowdot_go<2, 1, RD_SUMS + 10, RD_SWIGLU>(r, (hipStream_t)stream);
+  return rowdot_go<2, 1, RD_SUMS + kRdSums, RD_SWIGLU>(r, (hipStream_t)stream);
+}
 }

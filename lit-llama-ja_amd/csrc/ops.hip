@@ -130,6 +130,36 @@ __global__ __launch_bounds__(NTH) void attention_kernel(const bf16_t* __restrict
                                            nullptr, st, thr, clr, clr_words, spec_ok != 0);
 }
 
+// One decode row's attention with the head's share of attn.c_proj: part[h][n] = sum_d y[h, d] Wp[n, HS h + d], y rounded to bf16 as a
+// launch of its own would store it; the next product adds the heads' shares up (rowdot.h, sums). A workgroup takes a head and 64 of Wp's rows, which are on
+// their way to registers (HS / 8 lanes and a piece of 16 bytes each to a row) over the attention's own memory trips; the head's other workgroups form
+// the same attention again, since a CU takes its 82 KB of Wp no faster than two launches take all of it. For small models, whose launches are
+// all latency. us a step of 49M (10 layers), launches of their own 193; a head's rows in one workgroup 201, in two 192, four 188, five 185, ten 183.
+template <int HS, int U, int NTH>
+__global__ __launch_bounds__(NTH) void attention_proj_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
+                                                             const int* __restrict__ pos, int S, int nh, float scale_log2, const bf16_t* __restrict__ W,
+                                                             float* __restrict__ part) {
+  constexpr int LR = HS / 8;  // lanes to a row
+  static_assert(NTH / LR == 64 && LR == 8);
+  __shared__ __align__(16) float lds[attention_lds_floats<HS, NTH>() + HS];
+  const int h = blockIdx.x, C = nh * HS, j = threadIdx.x % LR, n = 64 * blockIdx.y + threadIdx.x / LR;
+  u32x4 w;
+  attention_body<HS, U, NTH, false, U / 2, false, true>(
+      q, kc, vc, nullptr, pos, 1, S, nh, scale_log2, h, 0, lds, 1, 0, nullptr, nullptr, 0.f, nullptr, 0, true, nullptr,
+      [&] { w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(W + (size_t)n * C + h * HS + 8 * j)); });
+  const float* y = lds + attention_lds_floats<HS, NTH>() + 8 * j;
+  float a = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    a = fmaf(bflo(w[e]), y[2 * e], a);
+    a = fmaf(bfhi(w[e]), y[2 * e + 1], a);
+  }
+  a += dpp_f32<kDppXor1>(a);
+  a += dpp_f32<kDppXor2>(a);
+  a += dpp_f32<kDppHalfMirror>(a);
+  if (j == 0) __hip_atomic_store(part + (size_t)h * C + n, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // split-K attention over the keys (long contexts): block (head, row, split) -> partial
 template <int HS, int U, int NTH>
 __global__ __launch_bounds__(NTH) void attention_part_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
@@ -711,6 +741,19 @@ static int attention_run(const void* q, const void* kcache, const void* vcache, 
 int llj_attention(const void* q, const void* kcache, const void* vcache, void* y, const int* pos, int B, int T,
                   int n_head, int head_size, int S, void* stream) {
   return attention_run(q, kcache, vcache, y, pos, B, T, n_head, head_size, S, nullptr, 0.f, nullptr, 0, stream);
+}
+
+// 512 (where one bf16 row goes to rowdot.h) to 1024 values in heads of 64
+int llj_attention_proj_ok(int n_head, int head_size, int S) { return head_size == 64 && n_head >= 8 && n_head <= 16 && S > 0; }
+
+int llj_attention_proj(const void* q, const void* kcache, const void* vcache, const int* pos, int n_head, int head_size, int S, const void* W,
+                       float* part, void* stream) {
+  LLJ_REQUIRE(q && kcache && vcache && pos && W && part && llj_attention_proj_ok(n_head, head_size, S) &&
+              (((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)W) & 15) == 0);
+  hipLaunchKernelGGL((attention_proj_kernel<64, LLJ_ATT_U, 512>), dim3(n_head, n_head), dim3(512), 0, (hipStream_t)stream, (const bf16_t*)q,
+                     (const bf16_t*)kcache, (const bf16_t*)vcache, pos, S, n_head, 1.4426950408889634f / 8.f, (const bf16_t*)W, part);
+  LLJ_CHECK_LAUNCH();
+  return 0;
 }
 
 size_t llj_attention_ws_bytes(int rows, int n_head, int head_size, int nsplit) {

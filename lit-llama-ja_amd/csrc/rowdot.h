@@ -23,6 +23,8 @@
 // Prologues (the weights' first loads are in flight meanwhile):
 //   plain    the row from memory, bf16;
 //   norm     RMSNorm with the reference's bf16 rounding points (model.py:281-283);
+//   sums     that of the row plus the sum of up to 16 fp32 rows (a product's shares by heads, ops.hip), each rounded to bf16; the row so
+//            formed is written once to x';
 //   streams  the residual streams after a sublayer, the mixed row and its layer norm (streams.hip), the new streams written
 //            once to x'.
 #pragma once
@@ -31,7 +33,7 @@
 
 namespace llj {
 
-enum { RD_PLAIN = 0, RD_NORM = 1, RD_STREAMS = 2 };
+enum { RD_PLAIN = 0, RD_NORM = 1, RD_STREAMS = 2, RD_SUMS = 3 /* .. + 16: up to PRO - RD_SUMS rows */ };
 // RD_STORE: + bias (fp32 or NULL). RD_RESID: out += . RD_QKV: RoPE, q to out, k / v to the caches. RD_SWIGLU: silu(. W) * (. W2).
 // RD_RELU2: max(., 0)^2. RD_GLU: the clamped gated unit of interleaved columns (elem.h), biased.
 enum { RD_STORE = 0, RD_RESID = 1, RD_QKV = 2, RD_SWIGLU = 3, RD_RELU2 = 4, RD_GLU = 5 };
@@ -54,6 +56,8 @@ struct RowDotParams {
   const float* sm;
   const float* si;
   int S, ldx;
+  const float* parts;  // sums: S rows of C
+  bf16_t* ao;          // x'
   bf16_t* kcache;  // RD_QKV
   bf16_t* vcache;
   const float* rope;
@@ -62,6 +66,7 @@ struct RowDotParams {
 };
 
 constexpr int kRdStreams = 4;
+constexpr int kRdSums = 16;
 constexpr int kRdMaxC = 16384;
 
 // ONE: columns of the largest range where a single round of loads holds them, or 0.
@@ -134,12 +139,22 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
     for (int i = 0; i < NW; ++i) t += red[which][i];
     return t;
   };
-  if constexpr (PRO == RD_PLAIN || PRO == RD_NORM) {
+  if constexpr (PRO != RD_STREAMS) {
     u32x4 xv[SL], gv[SL];
+    constexpr int NS = PRO > RD_SUMS ? PRO - RD_SUMS : 1;
+    f32x4 pv[SL][NS][2];
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
       xv[s] = *reinterpret_cast<const u32x4*>(p.A + kv[s]);
-      if constexpr (PRO == RD_NORM) gv[s] = *reinterpret_cast<const u32x4*>(p.w + kv[s]);
+      if constexpr (PRO != RD_PLAIN) gv[s] = *reinterpret_cast<const u32x4*>(p.w + kv[s]);
+      if constexpr (PRO > RD_SUMS) {
+#pragma unroll
+        for (int q = 0; q < NS; ++q) {  // (past the last: a copy, not added)
+          const f32x4* from = reinterpret_cast<const f32x4*>(p.parts + (size_t)(q < p.S ? q : 0) * p.C + kv[s]);
+          pv[s][q][0] = from[0];
+          pv[s][q][1] = from[1];
+        }
+      }
     }
     first = operand(tid);
     fetch(0, c0);
@@ -151,7 +166,26 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
     for (int s = 0; s < SL; ++s)
 #pragma unroll
       for (int e = 0; e < 8; ++e) xf[s][e] = (e & 1) ? bfhi(xv[s][e >> 1]) : bflo(xv[s][e >> 1]);
-    if constexpr (PRO == RD_NORM) {
+    if constexpr (PRO > RD_SUMS) {
+#pragma unroll
+      for (int s = 0; s < SL; ++s) {
+        const int k = k0 + 512 * s;
+        float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < NS; ++q)
+          if (q < p.S) {  // (uniform)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] += pv[s][q][e >> 2][e & 3];
+          }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xf[s][e] = k < p.C ? round_bf(xf[s][e] + round_bf(y[e])) : 0.f;  // model.py:172
+        if (k < p.C && (unsigned)(k >> 3) % gridDim.x == blockIdx.x) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) st_out32(p.ao + k + 2 * e, pack2bf(xf[s][2 * e], xf[s][2 * e + 1]));
+        }
+      }
+    }
+    if constexpr (PRO != RD_PLAIN) {
       float ss = 0.f;
 #pragma unroll
       for (int s = 0; s < SL; ++s)
@@ -313,7 +347,7 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
 template <int NW, int SL, int PRO, int EPI>
 static int rowdot_go(const RowDotParams& p, hipStream_t s) {
   const int units = p.N / 2;
-  int grid = 2048 / NW;
+  int grid = (PRO > RD_SUMS ? 512 : 2048) / NW;  // (every workgroup of a sums prologue reads all of its rows: 49M 2048 198 us a step, 512 and 1024 185)
   grid = grid < units ? grid : units;
   // [column][NW * 4] sums of the largest range in 48 KiB (very wide outputs: more workgroups)
   const long most = 48 * 1024 / (NW * 16) - 2;

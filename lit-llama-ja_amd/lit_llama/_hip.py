@@ -130,6 +130,9 @@ SIGNATURES = {
     "llj_g_bias_act": [_I, _P, _I, _P, _P, _I, _I, _I, _F, _F, _I, _P],
     "llj_streams_embed": [_P, _P, _I, _F, _P, _P, _I, _I, _P, _P, _F, _P, _I, _I, _I, _I, _P],
     "llj_streams_step": [_P, _I, _P, _P, _P, _I, _I, _P, _P, _F, _P, _I, _P, _I, _I, _I, _P],
+    "llj_attention_proj_ok": [_I, _I, _I],
+    "llj_attention_proj": [_P, _P, _P, _P, _I, _I, _I, _P, _P, _P],
+    "llj_sums_swiglu": [_P, _P, _I, _P, _P, _F, _P, _P, _P, _I, _I, _P],
     "llj_post_rows": [_I, _P, _I, _P, _F, _P, _P, _I, _I, _P, _P, _I, _I, _I, _I, _P],
     "llj_post_rows_ok": [_I, _I, _I, _I],
     "llj_streams_linear_ok": [_I, _I],

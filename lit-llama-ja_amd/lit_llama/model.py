@@ -306,6 +306,13 @@ class _Work:
             nb = _hip.lib().llj_attention_ws_bytes(M, cfg.n_head, C // cfg.n_head, self.nsplit)
             self.att_ws = torch.empty(nb, dtype=torch.uint8, device=device)
             self.att_count = torch.zeros(M * cfg.n_head, dtype=torch.int32, device=device)
+        # one row of a small model, short cache: the attention leaves the heads' shares of c_proj, which the SwiGLU adds up
+        # (llj_attention_proj, llj_sums_swiglu) into the residual's other place
+        self.parts = self.x2 = None
+        if (M == 1 and self.nsplit <= 1 and not need_i8 and not gemm and C % cfg.n_head == 0
+                and _hip.lib().llj_attention_proj_ok(cfg.n_head, C // cfg.n_head, S)):
+            self.parts = torch.empty(cfg.n_head, C, dtype=torch.float32, device=device)
+            self.x2 = torch.empty_like(self.x)
         # one decode row, short cache: interleaved split partials merged in attn.c_proj (ATT_MERGE)
         self.att_merge = ATT_MERGE if (ATT_MERGE > 1 and M == 1 and self.nsplit <= 1 and not need_i8) else 0
         self.att_part = None
@@ -739,6 +746,14 @@ class LLaMA(nn.Module):
                           w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), rope.data_ptr(), pos.data_ptr(), B, T, C, nh,
                           S, r0, r, P(w.i8ws), P(rs), P(nst), w.npart, st)
             # 2. attention, 3. c_proj + residual
+            if w.parts is not None and T == 1 and fp == f1 == f2 == 1 and not w.hand:  # .. and 4.
+                _hip.call("llj_attention_proj", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), nh, C // nh, S, wp.data_ptr(),
+                          w.parts.data_ptr(), st)
+                _hip.call("llj_sums_swiglu", w.x.data_ptr(), w.parts.data_ptr(), nh, w.x2.data_ptr(), blk.rms_2.scale.data_ptr(),
+                          blk.rms_2.eps, w1.data_ptr(), w2.data_ptr(), w.h.data_ptr(), H, C, st)
+                w.x, w.x2 = w.x2, w.x
+                self._resid(fd, w.h, wd, sd, w.x, M, C, H, w, st)
+                continue
             if w.i8s and not w.flash:  # y's LLM.int8 statistics from the attention (clears h's block)
                 if w.att_ws is not None:
                     _hip.call("llj_attention_ranges", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(),

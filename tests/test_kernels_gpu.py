@@ -2192,3 +2192,42 @@ def test_gemm_qkv_tiles(hip, nh, hs, B, T_, S):
         v = y[:, 2 * C:].view(B, T_, nh, hs).transpose(1, 2)
         slots = ((pos.long()) % S)
         assert_bf16_close(outs[1][2][:, :, slots].float().cpu().numpy(), v.cpu().numpy(), "v rows", rel=2.0 ** -7, abs_frac=2e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,S,p,H", [(8, 96, 0, 1536), (10, 144, 63, 1792), (10, 144, 64, 1792), (10, 511, 510, 1792), (16, 40, 75, 256), (12, 8, 3, 16)])
+def test_attention_with_projection_shares(hip, nh, S, p, H):
+    """llj_attention_proj and llj_sums_swiglu against float64 on what each reads: one key, a speculative pass exactly, past it, the largest cache, a
+    wrapped ring, most and fewest heads. Bounds: the rounding of y (2^-9) through |Wp|, the bf16 roundings of x' and h."""
+    from lit_llama import _hip
+
+    g = torch.Generator(device="cuda").manual_seed(nh + p)
+    hs, C = 64, 64 * nh
+    q = torch.randn(C, generator=g, device="cuda").bfloat16()
+    kc, vc = (torch.randn(nh, S, hs, generator=g, device="cuda").bfloat16() for _ in range(2))
+    W = (torch.randn(C, C, generator=g, device="cuda") * C ** -0.5).bfloat16()
+    pos = torch.tensor([p], dtype=torch.int32, device="cuda")
+    parts = torch.full((nh, C), float("nan"), device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    _hip.call("llj_attention_proj", q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), nh, hs, S, W.data_ptr(), parts.data_ptr(), st)
+    n = min(p + 1, S)
+    s = torch.einsum("hd,hkd->hk", q.double().view(nh, hs), kc[:, :n].double()) / 8
+    y = torch.einsum("hk,hkd->hd", s.softmax(-1), vc[:, :n].double())
+    Wh = W.double().view(C, nh, hs)
+    want = torch.einsum("hd,nhd->hn", y, Wh)
+    bound = 2.0 ** -8 * torch.einsum("hd,nhd->hn", y.abs(), Wh.abs()) + 1e-6
+    assert ((parts.double() - want).abs() <= bound).all()
+
+    x = torch.randn(C, generator=g, device="cuda").bfloat16()
+    w = (1 + 0.1 * torch.randn(C, generator=g, device="cuda")).bfloat16()
+    w1, w2 = ((torch.randn(H, C, generator=g, device="cuda") * C ** -0.5).bfloat16() for _ in range(2))
+    xo, h = torch.zeros(C, dtype=torch.bfloat16, device="cuda"), torch.zeros(H, dtype=torch.bfloat16, device="cuda")
+    _hip.call("llj_sums_swiglu", x.data_ptr(), parts.data_ptr(), nh, xo.data_ptr(), w.data_ptr(), 1e-5, w1.data_ptr(), w2.data_ptr(), h.data_ptr(), H, C, st)
+    sums = parts.double().sum(0)
+    assert ((xo.double() - (x.double() + sums)).abs() <= 2.0 ** -8 * (sums.abs() + (x.double() + sums).abs()) + 1e-6).all()
+    ref, x2 = torch.zeros_like(h), xo.clone()
+    _hip.call("llj_norm_swiglu", 1, x2.data_ptr(), w.data_ptr(), 1e-5, w1.data_ptr(), None, w2.data_ptr(), None, ref.data_ptr(), 1, H, C, None, 0, None, None,
+              0, st)
+    torch.cuda.synchronize()
+    # (the same row through the product without the sums: the order of fp32 sums apart, one rounding of a, b and h)
+    assert ((h.double() - ref.double()).abs() <= 2.0 ** -7 * ref.double().abs() + 2e-3 * ref.double().abs().max()).all()
