@@ -52,7 +52,10 @@ static int gemm_run(int wfmt, GemmParams& p, void* ws, size_t ws_bytes, void* st
     p.gch = wfmt >> 8;
     return (p.sz && p.gch >= 1 && p.K % 128 == 0) ? gemm_split_launch<GWF_W4G, EP>(p, ws_bytes, s) : LLJ_EINVAL;
   }
-  if (wfmt == GWF_BF16) return gemm_bf16_run(EP, p, ws_bytes, s);
+  if (wfmt == GWF_BF16) {
+    const int rc = gemm_few_run(EP, p, s);
+    return rc < 0 ? gemm_bf16_run(EP, p, ws_bytes, s) : rc;
+  }
   if (wfmt == GWF_I8) {
     if (!p.sz || !p.i8ws || p.K % 128) return LLJ_EINVAL;
     if (!p.ao16 != !p.w16 || (p.ao16 && (p.kpad < 64 || p.kpad % 64))) return LLJ_EINVAL;

@@ -1688,5 +1688,6 @@ static inline int splitk_plan(int wfmt, int M, int N, int K, int* kcs_out) {
 
 // bf16 (N, K) weights, any epilogue of the plain GEMMs: instantiated in gemm_bf16.hip
 int gemm_bf16_run(int ep, const GemmParams& p, size_t ws_bytes, hipStream_t s);
+int gemm_few_run(int ep, const GemmParams& p, hipStream_t s);
 
 }  // namespace llj

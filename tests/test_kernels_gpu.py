@@ -2231,3 +2231,31 @@ def test_attention_with_projection_shares(hip, nh, S, p, H):
     torch.cuda.synchronize()
     # (the same row through the product without the sums: the order of fp32 sums apart, one rounding of a, b and h)
     assert ((h.double() - ref.double()).abs() <= 2.0 ** -7 * ref.double().abs() + 2e-3 * ref.double().abs().max()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(17, 640, 640), (32, 1920, 256), (33, 512, 384), (64, 384, 512), (63, 1536, 1024), (47, 640, 1792), (250, 512, 1536), (1, 128, 768)])
+def test_gemm_few_tiles_exact(hip, M, N, K):
+    """Small bf16 products (32 rows and 16 columns to a workgroup, K over its waves) on integer values, whose sums are exact in any order: shares of equal
+    and of different numbers of steps, a partial last block of rows; nothing outside, every epilogue but QKV's (which the prompt tests run)."""
+    from lit_llama import _hip
+
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    A = torch.full((M, K + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    A[:, :K] = torch.randint(-3, 4, (M, K), generator=g, device="cuda").float()
+    W = torch.randint(-2, 3, (N, K), generator=g, device="cuda").bfloat16()
+    st = torch.cuda.current_stream().cuda_stream
+    y = A[:, :K].double() @ W.double().T
+    out = torch.full((M + 1, N + 8), 3.0, dtype=torch.bfloat16, device="cuda")
+    _hip.call("llj_gemm_linear_ws", 1, A.data_ptr(), K + 8, W.data_ptr(), None, out.data_ptr(), N + 8, M, N, K, None, 0, st)
+    assert torch.equal(out[:M, :N], y.bfloat16())
+    r = torch.randint(-9, 9, (M + 1, N + 8), generator=g, device="cuda").bfloat16()
+    x = r.clone()
+    _hip.call("llj_gemm_resid_ws", 1, A.data_ptr(), K + 8, W.data_ptr(), None, x.data_ptr(), N + 8, M, N, K, None, 0, st)
+    assert torch.equal(x[:M, :N], (r[:M, :N].double() + y.bfloat16().double()).bfloat16())
+    h = r.clone()
+    _hip.call("llj_gemm_silu_mul_ws", 1, A.data_ptr(), K + 8, W.data_ptr(), None, h.data_ptr(), N + 8, M, N, K, None, 0, st)
+    want = torch.nn.functional.silu(r[:M, :N].double()) * y.bfloat16().double()
+    assert ((h[:M, :N].double() - want).abs() <= 2.0 ** -7 * want.abs() + 1e-30).all()
+    for t, o in ((out, torch.full_like(out, 3.0)), (x, r), (h, r)):
+        assert torch.equal(t[M], o[M]) and torch.equal(t[:, N:], o[:, N:])
