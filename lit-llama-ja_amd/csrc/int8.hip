@@ -217,16 +217,17 @@ __device__ __forceinline__ uint2 quant8(uint4 x, uint2 fl, float inv) {
 __device__ __forceinline__ uint32_t first_not_below(float thr) { return (__float_as_uint(thr) + 0xFFFFu) >> 16; }
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-// The whole activation preparation in ONE launch for decode batches (M <= 8 rows): one 1024-thread
-// block per k-block (kNSB blocks). Every block reads all M rows (four 256-thread groups, group g
+// The whole activation preparation in ONE launch for decode batches (M <= 8 rows): min(M, 4) 1024-thread
+// blocks per k-block (kNSB k-blocks). Every block reads all M rows (four 256-thread groups, group g
 // taking rows g and g + 4 with llj_rmsnorm's thread-to-vector map, so with norm_w the sums of
-// squares -- and xn -- are bit-identical to llj_rmsnorm's) and reduces each row's SCA = max of the
-// elements below the threshold itself (redundant across blocks, no grid-wide dependency); then it
-// finishes its own k-block: outlier flags, the list, part, the normalized rows (xn) and the
-// quantized rows (aq). Block 0 writes the header and SCA.
-// Bound by instructions and by the steps that follow each other: the 32 CUs each see all rows. 8 rows of 4096 with the norm,
-// us a launch: 7.5 -> 7.1 since the maxima are taken on pairs of bf16 bits, the rows' factors by every wave for itself and the
-// row loads issued ahead of the own item's place.
+// squares -- and xn -- are bit-identical to llj_rmsnorm's); block (b, q) reduces SCA = max of the
+// elements below the threshold of rows q and q + 4 itself (redundant across k-blocks, no grid-wide dependency)
+// and finishes them in k-block b: the normalized rows (xn) and the quantized rows (aq). Every block finds the k-block's
+// outlier flags, which take all rows; block (b, 0) writes them, the list and part, k-block 0 the header and SCA.
+// Bound by instructions and by the steps that follow each other: all blocks see all rows. The maxima are more than half of the
+// instructions; a block's own two rows are one wave a SIMD of them, beside which another group finds the flags.
+// One block per k-block for all rows -> this, us a launch in a graph: 8 rows of 4096 with the norm 6.7 -> 5.4 (with the hand-off
+// block 8.4 -> 7.2), 2 rows 6.3 -> 4.9, 3 rows of 5120 9.1 -> 6.6, 8 of 2048 6.4 -> 5.1.
 template <bool NORM, int VPT>
 __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restrict__ x, int lda,
                                                            const bf16_t* __restrict__ w, float eps,
@@ -236,11 +237,13 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
   constexpr int MR = 8;
   __shared__ int flag[1024];
   __shared__ __attribute__((aligned(16))) float red[MR][4];
-  __shared__ float mred[16][MR];
+  __shared__ float mred[4][2];
   __shared__ int pmax[MR];
   __shared__ uint4 vals[MR][1024 / 8];  // the own k-block's (normalized) rows, for aval
   const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int grp = tid >> 8, lt = tid & 255, gw = lt >> 6;  // row group, thread / wave within it
+  const int rq = blockIdx.y, nq = gridDim.y;  // this block's rows: rq and rq + 4
+  const int it = (tid - 256 * (rq + 1)) & 1023;  // place in the k-block's items: the group after the one that takes the maxima
   const I8Layout L = i8_layout(ws, M, K);
   const int nvec = K >> 3;
   const int k0 = b * kb, k1 = min(K, k0 + kb);
@@ -261,8 +264,8 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
     for (int j = 0; j < VPT; ++j) ga[j] = reinterpret_cast<const uint4*>(w)[lt + 256 * j < nvec ? lt + 256 * j : nvec - 1];
   }
   // own k-block item (row, vector; M * vpr <= 1024 on this path): its place is computed over the loads above
-  const bool own = tid < M * vpr;
-  const int om = own ? tid / vpr : 0, ov = own ? (k0 >> 3) + tid % vpr : 0;
+  const bool own = it < M * vpr;
+  const int om = own ? it / vpr : 0, ov = own ? (k0 >> 3) + it % vpr : 0;
   const uint4 oa = reinterpret_cast<const uint4*>(x + (size_t)om * lda)[ov];
   uint4 og = oa;
   if (NORM) og = reinterpret_cast<const uint4*>(w)[ov];
@@ -298,6 +301,7 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
   const uint32_t tb = first_not_below(thr), tb2 = tb | (tb << 16);
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
+    if (uniform(grp) != rq || rq + 4 * r >= M) break;  // (uniform)
     const float rn = NORM ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rows), uniform(grp + 4 * r))) : 1.f;
     const f32x2 rn2 = {rn, rn};
     u16x2 mx = {0, 0};
@@ -315,7 +319,7 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
     }
     const uint32_t top = max((uint32_t)mx[0], (uint32_t)mx[1]);
     const float m = wave_max(top >= 0x10000u - tb ? __uint_as_float((top + tb) << 16) : 0.f);  // (top + tb - 2^16: bf16 bits)
-    if (lane == 0) mred[tid >> 6][r] = to_f16f(m);  // wave (grp, gw): slot r <-> row grp + 4 r
+    if (lane == 0) mred[gw][r] = to_f16f(m);  // wave gw of the group: slot r <-> row rq + 4 r
   }
   if (!NORM) __syncthreads();  // flag / pmax zeroed before any thread sets them (NORM: synced above)
   // own k-block: normalize, flags, per-row maximum
@@ -327,7 +331,7 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
                     norm_pair(oa.w, og.w, rn));
   }
   if (own) {
-    if (NORM) reinterpret_cast<uint4*>(xn + (size_t)om * K)[ov] = on;
+    if (NORM && (om & 3) == rq) reinterpret_cast<uint4*>(xn + (size_t)om * K)[ov] = on;
     vals[om][ov - (k0 >> 3)] = on;
     const uint32_t ow[4] = {on.x, on.y, on.z, on.w};
     float mx = 0.f;
@@ -340,30 +344,26 @@ __global__ __launch_bounds__(1024) void i8_prep_one_kernel(const bf16_t* __restr
     atomicMax(&pmax[om], __float_as_int(mx));  // non-negative floats order as their bits
   }
   __syncthreads();
-  // SCA of row m: max over the 4 waves of its group (slot m >> 2)
-  if (own) {
-    const int g = om & 3, r = om >> 2;
-    const float sca = fmaxf(fmaxf(mred[4 * g][r], mred[4 * g + 1][r]), fmaxf(mred[4 * g + 2][r], mred[4 * g + 3][r]));
-    const float inv = sca > 0.f ? 127.f / sca : 0.f;
+  // SCA of row rq + 4 r: max over the 4 waves
+  auto sca_of = [&](int r) { return fmaxf(fmaxf(mred[0][r], mred[1][r]), fmaxf(mred[2][r], mred[3][r])); };
+  if (own && (om & 3) == rq) {
     const int c = 8 * ov - k0;
     const uint2 fb = make_uint2(flag[c] | (flag[c + 1] << 8) | (flag[c + 2] << 16) | (flag[c + 3] << 24),
                                 flag[c + 4] | (flag[c + 5] << 8) | (flag[c + 6] << 16) | (flag[c + 7] << 24));
+    const float sca = sca_of(om >> 2), inv = sca > 0.f ? 127.f / sca : 0.f;
     reinterpret_cast<uint2*>(L.aq + (size_t)om * K)[ov] = quant8(on, fb, inv);
     if (om == 0) reinterpret_cast<uint2*>(L.flag)[ov] = fb;
     if (b == 0 && ov == (k0 >> 3)) L.sca[om] = sca;
   }
-  if (tid < M) L.part[(size_t)b * M + tid] = __int_as_float(pmax[tid]);
-  if (b == 0 && tid == 0) *reinterpret_cast<I8WsHeader*>(ws) = I8WsHeader{M, K, kNSB, kb}, L.avh[0] = 1;  // aval written
-  if (st) {  // uniform: the decode hand-off block (i8ws.h) for the streamed int8 GEMVs (AM_I8Q)
-    if (b == 0 && tid < 8 * kI8StSlots) {  // SCA in slot 0, the other slots 0
-      const int m = tid;
-      float sca = 0.f;
-      if (m < M) {
-        const int g = m & 3, r = m >> 2;
-        sca = fmaxf(fmaxf(mred[4 * g][r], mred[4 * g + 1][r]), fmaxf(mred[4 * g + 2][r], mred[4 * g + 3][r]));
-      }
-      st[kI8StSca + tid] = __float_as_uint(sca);
-    }
+  if (rq == 0 && tid < M) L.part[(size_t)b * M + tid] = __int_as_float(pmax[tid]);
+  if (b == 0 && rq == 0 && tid == 0) *reinterpret_cast<I8WsHeader*>(ws) = I8WsHeader{M, K, kNSB, kb}, L.avh[0] = 1;  // aval written
+  if (st && b == 0 && tid < 8 * kI8StSlots) {  // the decode hand-off block (i8ws.h) for the streamed int8 GEMVs (AM_I8Q)
+    // SCA in slot 0, the other slots 0: every word is written by the block of its row, by block 0 where there is none
+    const int q = tid & 3;
+    if (q == rq || (rq == 0 && q >= nq)) st[kI8StSca + tid] = __float_as_uint(tid < M ? sca_of(tid >> 2) : 0.f);
+  }
+  if (rq != 0) return;
+  if (st) {  // uniform
     for (int wd = tid; 32 * wd < k1 - k0; wd += 1024) {  // this k-block's flag words (kb % 32 == 0)
       uint32_t bits = 0;
       for (int j = 0; j < 32 && 32 * wd + j < k1 - k0; ++j) bits |= (uint32_t)(flag[32 * wd + j] != 0) << j;
@@ -583,7 +583,7 @@ static int i8_prep_one(bool norm, const bf16_t* x, int lda, const bf16_t* w, flo
   if (!(thr >= 0x1p-14f && thr <= 65504.f)) return 1;
   hipStream_t s = (hipStream_t)stream;
 #define LLJ_P1(N, V) \
-  hipLaunchKernelGGL((i8_prep_one_kernel<N, V>), dim3(kNSB), dim3(1024), 0, s, x, lda, w, eps, xn, M, K, thr, (char*)ws, kb, st)
+  hipLaunchKernelGGL((i8_prep_one_kernel<N, V>), dim3(kNSB, M < 4 ? M : 4), dim3(1024), 0, s, x, lda, w, eps, xn, M, K, thr, (char*)ws, kb, st)
   if (norm) {
     if (vpt <= 2) LLJ_P1(true, 2); else LLJ_P1(true, 4);
   } else {

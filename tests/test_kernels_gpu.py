@@ -882,6 +882,34 @@ def _check_i8_ws(ws, a, M, K, thr=6.0):
     np.testing.assert_array_equal(ws[o_aq:o_aq + M * K].view(np.int8).reshape(M, K), q.astype(np.int8))
 
 
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("M,K", [(1, 256), (2, 4096), (3, 144), (4, 4096), (5, 8192), (6, 2048), (7, 4096), (8, 8192)])
+def test_i8_decode_prep_rows_over_blocks(hip, M, K, norm):
+    """The one-launch preparation gives every row to one of min(M, 4) blocks of a k-block: each word of the workspace and of the
+    hand-off block is written whatever they held (counts of rows below, at and past the four blocks)."""
+    rng = np.random.default_rng(11 * M + K)
+    x = bf16(rng.standard_normal((M, K)))
+    x[M - 1, rng.choice(K, 5, replace=False)] = 40.0  # outliers in the last row alone
+    xd, gd = T(x, torch.bfloat16), T(bf16(rng.uniform(0.5, 1.5, K)), torch.bfloat16)
+    xn = torch.zeros_like(xd)
+    ws = torch.full((hip.llj_i8_ws_bytes(M, K),), 255, dtype=torch.uint8, device=dev)
+    blk = torch.full((hip.llj_i8_rowstats_bytes(K) // 4,), -1, dtype=torch.int32, device=dev)
+    call(hip, "llj_i8_norm_rowstats", xd.data_ptr(), gd.data_ptr() if norm else None, 1e-5, xn.data_ptr(), M, K, 6.0, ws.data_ptr(),
+         blk.data_ptr(), st())
+    want = xd
+    if norm:
+        want = torch.zeros_like(xd)
+        call(hip, "llj_rmsnorm", xd.data_ptr(), gd.data_ptr(), 1e-5, want.data_ptr(), M, K, st())
+        assert torch.equal(want.view(torch.int16), xn.view(torch.int16))
+    a = want.float().cpu().numpy()
+    _check_i8_ws(ws.cpu().numpy(), a, M, K)
+    a16 = np.abs(a.astype(np.float16).astype(np.float32))
+    slots = blk.cpu().numpy()[16:16 + 512].view(np.float32).reshape(64, 8)
+    np.testing.assert_array_equal(slots[0, :M], np.where(a16 >= 6.0, 0.0, a16).max(1))
+    assert not slots[0, M:].any() and not slots[1:].any()
+    np.testing.assert_array_equal(_st_decode(blk, M, K)[1], (a16 >= 6.0).any(0))
+
+
 @pytest.mark.parametrize("wfmt", [0, 3, W4G_128])
 def test_long_k_residual_eight_waves_m1(hip, wfmt):
     """mlp.c_proj at 7B (K = 11008 >= 8192: 8-wave workgroups, M = 1 register prologue): every
