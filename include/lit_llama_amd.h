@@ -156,6 +156,14 @@ int llj_sums_swiglu(const void* x, const float* parts, int nparts, void* x_out, 
  * part_ws (llj_attention_ws_bytes(B*T, n_head, head_size, nsplit) bytes), merged in split order
  * by a second launch. nsplit <= 1 is llj_attention itself. Same softmax up to summation order. */
 size_t llj_attention_ws_bytes(int rows, int n_head, int head_size, int nsplit);
+/* The attention of M decode rows (M sequences at one position, M <= 2; bf16 weights: M = 1) and attn.c_proj with the residual add
+ * (x += y . W^T, model.py:172) in one launch: y (M, C = nh * hs) holds 0xFFFFFFFF words when it starts and the attention's output when it ends;
+ * the launch fills y_next with such words for the launch that takes it next. wfmt 0, 1 or 3; nsplit > 1: key ranges with part and zeroed
+ * count as in llj_attention_ranges; nstat_out as in llj_linear_resid (M > 1). llj_attention_resid_ok: what is taken. */
+int llj_attention_resid_ok(int wfmt, int M, int nh, int hs);
+int llj_attention_resid(int wfmt, const void* q, const void* kcache, const void* vcache, void* y, void* y_next, const int* pos, int M, int nh,
+                        int hs, int S, int nsplit, void* part, int* count, const void* W, const void* sz, void* x, float* nstat_out, void* stream);
+
 /* Decode attention (model.py:237) as nsplit <= 4 interleaved key splits per (row, head) whose
  * unnormalized partials (outputs, max, sum; llj_attention_ws_bytes layout) go to part_ws with no
  * combine launch: llj_linear_resid_attn merges them in attn.c_proj's prologue (one row). */

@@ -61,12 +61,16 @@ __device__ __forceinline__ void softmax_merge(float& mx, float& l, float* o, con
 template <int HS>
 constexpr int kAttPart = HS + 4;  // floats per partial record: HS outputs, max, sum, 2 pad (16-byte records)
 
-// y[m, h * HS + d] of thread d < HS, adjacent dims as one 4-byte store; with st the LLM.int8 statistics of y, one slot per head
-template <int HS>
+// y[m, h * HS + d] of thread d < HS, adjacent dims as one 4-byte store; with st the LLM.int8 statistics of y, one slot per head.
+// HAND: to workgroups of the same launch that wait for every word of y to differ from kNotYet (attend_proj.hip).
+constexpr uint32_t kNotYet = 0xFFFFFFFFu;  // two NaNs; as outputs they leave as two others
+template <int HS, bool HAND = false>
 __device__ __forceinline__ void attention_out(float v, bf16_t* __restrict__ y, uint32_t* st, float thr, int h, int m, int C) {
   const int d = threadIdx.x;
   const uint32_t ob = (uint32_t)f2bf(v), pr = lane_xor1(ob);
-  if (!(d & 1)) st_out32(y + (size_t)m * C + h * HS + d, ob | (pr << 16));
+  uint32_t w = ob | (pr << 16);
+  if (HAND && w == kNotYet) w = 0x7FFF7FFFu;
+  if (!(d & 1)) st_out32(y + (size_t)m * C + h * HS + d, w);
   if (st) i8_emit_stats64(st, thr, m, h * HS + (d & ~63), ob, h);  // (uniform)
 }
 
@@ -78,7 +82,8 @@ struct NoLoads {
 // count (with PART, else partials only; nsplit <= 64): zeroed arrival counters, one per (row, head), left zero: the last of the
 // ranges' blocks to finish merges them. The hand-off is device-scope stores, a wait for them, the counter, device-scope
 // loads; no block waits for another.
-template <int HS, int U, int NTH, bool PART = false, int SPECU = U / 2, bool ILV = false, bool KEEP = false, typename F = NoLoads>
+template <int HS, int U, int NTH, bool PART = false, int SPECU = U / 2, bool ILV = false, bool KEEP = false, bool HAND = false,
+          typename F = NoLoads>
 __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                const bf16_t* __restrict__ vc, bf16_t* __restrict__ y,
                                                const int* __restrict__ pos, int T, int S, int nh, float scale_log2,
@@ -252,7 +257,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
     } else if constexpr (KEEP) {
       s_m[2 * NWV + NWV * HS + d] = round_bf(O / L);  // (past what is read here)
     } else {
-      attention_out<HS>(O / L, y, st, thr, h, m, C);
+      attention_out<HS, HAND>(O / L, y, st, thr, h, m, C);
     }
   }
   if constexpr (KEEP) __syncthreads();
@@ -297,7 +302,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
         O += pc[e] * f;
       }
     }
-    attention_out<HS>(O / L, y, st, thr, h, m, C);
+    attention_out<HS, HAND>(O / L, y, st, thr, h, m, C);
   }
 }
 

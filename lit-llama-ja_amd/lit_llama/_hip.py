@@ -35,6 +35,7 @@ SIGNATURES = {
     "llj_norm_qkv_rope": [_I, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _I,
                           _P],
     "llj_attention_ranges": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _F, _P],
+    "llj_attention_resid": [_I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
     "llj_attention_split": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P],
     "llj_gemm_i8_linear": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
     "llj_gemm_i8_linear_ws": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
@@ -131,6 +132,7 @@ SIGNATURES = {
     "llj_streams_embed": [_P, _P, _I, _F, _P, _P, _I, _I, _P, _P, _F, _P, _I, _I, _I, _I, _P],
     "llj_streams_step": [_P, _I, _P, _P, _P, _I, _I, _P, _P, _F, _P, _I, _P, _I, _I, _I, _P],
     "llj_attention_proj_ok": [_I, _I, _I],
+    "llj_attention_resid_ok": [_I, _I, _I, _I],
     "llj_attention_proj": [_P, _P, _P, _P, _I, _I, _I, _P, _P, _P],
     "llj_sums_swiglu": [_P, _P, _I, _P, _P, _F, _P, _P, _P, _I, _I, _P],
     "llj_post_rows": [_I, _P, _I, _P, _F, _P, _P, _I, _I, _P, _P, _I, _I, _I, _I, _P],

@@ -32,7 +32,7 @@ import weakref
 import torch
 
 from . import _hip
-from .model import LLaMA, _Work, _enable_i8_handoff
+from .model import LLaMA, _Work, _enable_attend, _enable_i8_handoff
 from .state import Rows
 
 
@@ -127,14 +127,17 @@ class LLaMAProgram(_Program):
             need_i8 = any(q[0] == 2 for layer in s.specs["layers"] for q in layer) or s.specs["head"][0] == 2
             s.work = _Work(m.config, s.B, self.dev, need_i8, s.S)
             _enable_i8_handoff(s.work, s.specs)
+            _enable_attend(s.work, s.specs, s.B, 1, m.config.n_head)
 
     def reset_handoff(self):
-        """The LLM.int8 hand-off blocks (_Work.y_st / h_st) must be zero when a step starts; a
-        completed step leaves them so, a step that raised part-way may not: zero them again."""
+        """The LLM.int8 hand-off blocks (_Work.y_st / h_st) must be zero when a step starts, and the attention's output (y_hand)
+        empty; a completed step leaves them so, a step that raised part-way may not: set them again."""
         w = self.sess.work
         if w is not None and getattr(w, "y_st", None) is not None:
             w.y_st.zero_()
             w.h_st.zero_()
+        if w is not None and w.y_hand is not None:
+            w.y_hand.fill_(-1)
 
     def step(self, st) -> None:
         s = self.sess

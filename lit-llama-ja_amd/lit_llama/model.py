@@ -244,6 +244,16 @@ def _enable_i8_handoff(w: "_Work", specs) -> None:
     w.i8s = w.y_st is not None and all(s[0] == 2 for layer in specs["layers"] for s in layer)
 
 
+def _enable_attend(w: "_Work", specs, B: int, T: int, nh: int) -> None:
+    """Decode rows: the attention and attn.c_proj in one launch (llj_attention_resid) when every layer's c_proj takes it. y then
+    lies in one of three places: a launch reads its own and empties the next one's, the last layer's is not the first's."""
+    C, layers = w.x.shape[1], specs["layers"]
+    if (T == 1 and len(layers) > 1 and C % nh == 0 and w.parts is None and not (w.gemm or w.flash or w.att_merge)
+            and all(s[1][0] == layers[0][1][0] and s[1][1].data_ptr() % 16 == 0 for s in layers)
+            and _hip.lib().llj_attention_resid_ok(layers[0][1][0], B, nh, C // nh)):
+        w.y_hand = torch.full((3, B * C // 2), -1, dtype=torch.int32, device=w.x.device)
+
+
 class _Work:
     """Per-call scratch for M rows (allocated from torch's caching allocator)."""
 
@@ -264,9 +274,11 @@ class _Work:
             self.a2 = torch.empty(M, H, dtype=bf, device=device)
             self.h = torch.empty(M, H, dtype=bf, device=device)
             self.gemm = self.flash = self.pre = self.hand = False
+            self.y_hand = None
             self.i8ws = self.att_ws = self.nst = self.rs = None
             return
         self.gemm = gemm  # many rows: the prefill GEMMs (LLaMA._blocks_gemm)
+        self.y_hand = None  # _enable_attend
         self.flash = False  # T-row prompt attention on the MFMA flash kernel (set by LLaMA._run)
         self.x = torch.empty(M, C, dtype=bf, device=device)
         self.q = torch.empty(M, C, dtype=bf, device=device)
@@ -467,6 +479,7 @@ class LLaMA(nn.Module):
             w = _Work(cfg, M, dev, need_i8, S, gemm=self._gemm_ok(specs, M))
             w.flash = self._flash_ok(pos, T, S)
             _enable_i8_handoff(w, specs)
+            _enable_attend(w, specs, B, T, cfg.n_head)
         st = _hip.stream()
         ids = idx.reshape(-1).to(torch.int32)
         if w.generic:
@@ -754,7 +767,13 @@ class LLaMA(nn.Module):
                 w.x, w.x2 = w.x2, w.x
                 self._resid(fd, w.h, wd, sd, w.x, M, C, H, w, st)
                 continue
-            if w.i8s and not w.flash:  # y's LLM.int8 statistics from the attention (clears h's block)
+            if w.y_hand is not None:
+                n = len(specs["layers"])
+                y0, y1 = (2 if j == n - 1 and n % 2 else j % 2 for j in (i, (i + 1) % n))
+                _hip.call("llj_attention_resid", fp, w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y_hand[y0].data_ptr(),
+                          w.y_hand[y1].data_ptr(), pos.data_ptr(), M, nh, C // nh, S, w.nsplit, P(w.att_ws), P(w.att_count), wp.data_ptr(),
+                          P(sp), w.x.data_ptr(), P(w.nst) if w.hand and M > 1 else None, st)
+            elif w.i8s and not w.flash:  # y's LLM.int8 statistics from the attention (clears h's block)
                 if w.att_ws is not None:
                     _hip.call("llj_attention_ranges", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), w.y.data_ptr(), pos.data_ptr(),
                               B, T, nh, C // nh, S, w.nsplit, w.att_ws.data_ptr(), w.att_count.data_ptr(), w.y_st.data_ptr(),

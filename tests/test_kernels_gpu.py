@@ -2287,3 +2287,75 @@ def test_gemm_few_tiles_exact(hip, M, N, K):
     assert ((h[:M, :N].double() - want).abs() <= 2.0 ** -7 * want.abs() + 1e-30).all()
     for t, o in ((out, torch.full_like(out, 3.0)), (x, r), (h, r)):
         assert torch.equal(t[M], o[M]) and torch.equal(t[:, N:], o[:, N:])
+
+
+@pytest.mark.parametrize("wfmt,M,nh,S,p,nsplit", [(0, 1, 32, 80, 0, 1), (0, 1, 40, 96, 63, 1), (0, 1, 16, 96, 64, 1), (0, 2, 32, 600, 500, 3),
+                                                  (0, 2, 40, 70, 69, 1), (1, 1, 32, 1033, 1000, 5), (1, 1, 16, 40, 100, 1), (1, 1, 40, 130, 128, 1),
+                                                  (3, 1, 32, 600, 599, 3), (3, 2, 16, 96, 95, 1), (3, 2, 40, 520, 3, 3)])
+def test_attention_and_projection_in_one_launch(hip, wfmt, M, nh, S, p, nsplit):
+    """llj_attention_resid against the attention's launch, whose y it has bit for bit, and float64 on that y: five launches over two places for y, eagerly
+    and in a graph replayed three times (every place is empty again when it is used), ranges, one key, a wrapped ring, 1 to 5 rounds of chunks
+    to a wave. Bounds: the bf16 roundings of the product and of x', fp32 sums. A value that is all ones (the mark of a place not written
+    yet) still arrives, as NaN."""
+    rng = np.random.default_rng(nh + S)
+    hs, C = 128, 128 * nh
+    g = torch.Generator(device=dev).manual_seed(S)
+    W, Wd, szd = quant_operands(hip, rng, wfmt, C, C)
+    W = T(W).double()
+    q, x0 = (torch.randn(M, C, generator=g, device=dev).bfloat16() for _ in range(2))
+    kc, vc = (torch.randn(M, nh, S, hs, generator=g, device=dev).bfloat16() for _ in range(2))
+    pos = torch.tensor([p], dtype=torch.int32, device=dev)
+    part = torch.empty(max(16, M * nh * nsplit * (hs + 4) * 4), dtype=torch.uint8, device=dev)
+    count = torch.zeros(M * nh, dtype=torch.int32, device=dev)
+    y = torch.zeros(M, C, dtype=torch.bfloat16, device=dev)
+    if nsplit > 1:
+        call(hip, "llj_attention_ranges", q.data_ptr(), kc.data_ptr(), vc.data_ptr(), y.data_ptr(), pos.data_ptr(), M, 1, nh, hs, S, nsplit, part.data_ptr(),
+             count.data_ptr(), None, None, 0, 0.0, st())
+    else:
+        call(hip, "llj_attention", q.data_ptr(), kc.data_ptr(), vc.data_ptr(), y.data_ptr(), pos.data_ptr(), M, 1, nh, hs, S, st())
+    places = torch.full((2, M, C // 2), -1, dtype=torch.int32, device=dev)
+    nst = torch.zeros(C // 16, 16, device=dev)
+    x = torch.empty_like(x0)
+
+    def run(i, out, v=vc):
+        call(hip, "llj_attention_resid", wfmt, q.data_ptr(), kc.data_ptr(), v.data_ptr(), places[i % 2].data_ptr(), places[(i + 1) % 2].data_ptr(),
+             pos.data_ptr(), M, nh, hs, S, nsplit, part.data_ptr(), count.data_ptr(), Wd.data_ptr(), szd.data_ptr() if szd is not None else None,
+             out.data_ptr(), nst.data_ptr() if M > 1 else None, st())
+
+    prod = y.double() @ W.T
+    want = x0.double() + prod
+    bound = 2.0 ** -8 * (prod.abs() + want.abs()) + C * 2.0 ** -24 * (y.double().abs() @ W.abs().T)
+    if wfmt != 1:  # (the codes' offset is taken off at the end: sums of 128 + q or 2176 + q)
+        bound = bound + 2.0 ** -22 * (2 ** 4 if wfmt == 0 else 2 ** 8) * 0.02 * y.double().abs().sum(1, keepdim=True)
+    for i in range(5):
+        x.copy_(x0)
+        run(i, x)
+        assert torch.equal(places[i % 2].view(torch.bfloat16).view(M, C), y), i
+        assert (places[(i + 1) % 2] == -1).all()
+        assert ((x.double() - want).abs() <= bound).all(), i
+        if M > 1:
+            sq = (x.float() * x.float()).bfloat16().float().view(M, -1, 16).sum(-1)
+            np.testing.assert_allclose(nst[:, :M].T.cpu().numpy(), sq.cpu().numpy(), rtol=1e-6)
+    eager = x.clone()
+    s = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=s):
+        x.copy_(x0)
+        run(5, x)
+        x.copy_(x0)
+        run(6, x)
+        x.copy_(x0)
+        run(7, x)
+        x.copy_(x0)
+        run(8, x)
+    for _ in range(3):
+        x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(x, eager)
+    bad = vc.clone()
+    bad.view(torch.int16).fill_(-1)
+    run(9, x, bad)
+    torch.cuda.synchronize()
+    assert x.isnan().all()
