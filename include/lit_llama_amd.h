@@ -156,6 +156,15 @@ int llj_sums_swiglu(const void* x, const float* parts, int nparts, void* x_out, 
  * part_ws (llj_attention_ws_bytes(B*T, n_head, head_size, nsplit) bytes), merged in split order
  * by a second launch. nsplit <= 1 is llj_attention itself. Same softmax up to summation order. */
 size_t llj_attention_ws_bytes(int rows, int n_head, int head_size, int nsplit);
+/* One decode row through all L layers of a small bf16 model (model.py:162-175) in one launch. layers: L x 9 device pointers (a host array): rms_1 scale, c_attn,
+ * attn.c_proj, rms_2 scale, c_fc1, c_fc2, mlp.c_proj, K and V cache (n_head, S, hs); x (C) in and out; hand: llj_small_step_words(L, C, H) words, all
+ * 0xFFFFFFFF when it starts. llj_small_begin, the launch before it: those words, x = wte[idx[0]], pos[0] += 1. llj_small_step_ok: shapes taken. */
+int llj_small_step_ok(int L, int C, int H, int nh, int S);
+size_t llj_small_step_words(int L, int C, int H);
+int llj_small_begin(const int* idx, const void* wte, void* x, int C, int* pos, void* hand, int words, void* stream);
+int llj_small_step(const void* const* layers, int L, int C, int H, int nh, int S, float eps, const float* rope, const int* pos, void* x, void* hand,
+                   void* stream);
+
 /* The attention of M decode rows (M sequences at one position, M <= 2; bf16 weights: M = 1) and attn.c_proj with the residual add
  * (x += y . W^T, model.py:172) in one launch: y (M, C = nh * hs) holds 0xFFFFFFFF words when it starts and the attention's output when it ends;
  * the launch fills y_next with such words for the launch that takes it next. wfmt 0, 1 or 3; nsplit > 1: key ranges with part and zeroed

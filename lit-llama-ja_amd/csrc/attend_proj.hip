@@ -1,28 +1,21 @@
-// Decode rows: the attention over the K / V cache and attn.c_proj with its residual add (reference model.py:172, 218-240) in one launch.
-//
-// The first workgroups are the attention's (attention.h), the others own 16 columns of c_proj each. These bring all their weights to
-// registers while the attention runs, then read y until no word is kNotYet: y is its own signal, so that between the
-// attention's last store and the product there is one trip through the caches, where a launch of its own has its start, the trip
-// and the weights' bytes. The words return to kNotYet in the launch before the one that uses them next (`clear`).
+// One and two decode rows: the attention over the K / V cache and attn.c_proj with its residual add (reference model.py:172, 218-240) in one
+// launch. The first workgroups are the attention's (attention.h), the others own 16 columns of c_proj each and wait for y (handover.h).
 // us a pair in a graph, weights and caches from memory, two launches -> this (keys past 512 in ranges, as llj_attention_ranges):
 //   one row   int4  4096  8.4 -> 6.4 at 30 keys, 8.6 -> 6.5 at 70, 13.0 -> 11.3 at 500, 14.4 -> 12.7 at 1,000   5120  10.3 -> 7.9   2048  6.9 -> 5.3
 //             8-bit 4096  10.2 -> 7.8 at 90 keys, 16.1 -> 14.3 at 1,000
 //             bf16  4096  11.7 -> 9.6 at 70 keys, 17.5 -> 15.9 at 1,000   5120  21.1 -> 19.4 at 1,000   2048  7.7 -> 5.7 at 70
 //   two rows  4096  int4 9.1 -> 7.6 at 70 keys, 14.7 -> 13.2 at 500   8-bit 10.1 -> 9.0
 // Three and four rows gain 0.1 to 0.7 (with ranges nothing) and eight lose 2: every workgroup takes all rows past the caches.
-//
-// The waiting workgroups come after the attention's in the grid, and workgroups start in that order: whatever else runs on the
-// device, the ones waited for have started, and they wait for nobody. The wait is bounded all the same (kWaits; past it the
-// outputs are NaN).
 #include <algorithm>
 
 #include "attention.h"
 #include "common.h"
+#include "handover.h"
 #include "lit_llama_amd.h"
 
 namespace llj {
 
-enum { AP_W4 = 0, AP_BF16 = 1, AP_W8 = 3 };  // wfmt
+enum { AP_W4 = HC_W4, AP_BF16 = 1, AP_W8 = HC_W8 };  // wfmt
 
 struct AttendProjParams {
   const bf16_t *q, *kc, *vc;
@@ -42,103 +35,11 @@ struct AttendProjParams {
 };
 
 constexpr int kApNT = 512;
-constexpr int kWaits = 1 << 24;
-
 // words [at, at + 2) of y, both there or kNotYet in one of them
 __device__ __forceinline__ unsigned long long ap_word2(const uint32_t* y, int at) {
   return __hip_atomic_load(reinterpret_cast<const unsigned long long*>(y + at), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ bool ap_there(unsigned long long w) { return (uint32_t)w != kNotYet && (uint32_t)(w >> 32) != kNotYet; }
-
-__device__ __forceinline__ uint32_t ap_word(const uint32_t* y, int at) {
-  return __hip_atomic_load(y + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// acc += a . one MFMA step of codes (gemv_impl.h: W4P, and W8P as two nibble planes)
-template <int WF>
-__device__ __forceinline__ void ap_mfma(f32x4& acc, bf16x8 a, uint32_t lo, uint32_t hi, uint32_t msk, uint32_t mag, uint32_t mag_hi) {
-  auto codes = [&](uint32_t c, uint32_t m) {
-    return __builtin_bit_cast(bf16x8, make_uint4(and_or(c, msk, m), and_or(c >> 4, msk, m), and_or(c >> 8, msk, m), and_or(c >> 12, msk, m)));
-  };
-  acc = mfma_bf16(a, codes(lo, mag), acc);
-  if constexpr (WF == AP_W8) acc = mfma_bf16(a, codes(hi, mag_hi), acc);
-}
-
-// Up to MR rows of codes. Wave: chunks wave + 8 i of 128 values; lane: the codes of column n0 + lane % 16, 32 of a chunk's values.
-template <int WF, int MR, int NI>
-__device__ __forceinline__ void ap_codes(const AttendProjParams& p, int nt, unsigned char* smem) {
-  constexpr int NW = kApNT / 64, V = WF == AP_W8 ? 2 : 1, RS = NI * 128 + 8;  // (rows on other banks)
-  const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), C = p.C;
-  const int n0 = 16 * nt, KC = C >> 7, g = lane >> 4;
-  u32x4 w[NI][V];
-  const u32x4* src = reinterpret_cast<const u32x4*>(p.W) + (size_t)nt * KC * 64 * V + lane;
-  const int om = min((tid >> 4) & (MR - 1), p.M - 1), on = n0 + (tid & 15);  // the output of a thread: row, column
-  const float2 sz = p.sz[on];
-  const float x = bf2f(p.x[(size_t)om * C + on]);
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int v = 0; v < V; ++v) w[i][v] = __builtin_nontemporal_load(src + (size_t)(min(wave + NW * i, KC - 1) * V + v) * 64);
-  // this wave's own values of y: word `lane` of each of its chunks
-  bf16_t* ys = reinterpret_cast<bf16_t*>(smem) + wave * MR * RS;
-  uint32_t v[MR][NI];
-  for (int t = 0; t < kWaits; ++t) {
-    bool there = true;
-#pragma unroll
-    for (int m = 0; m < MR; ++m)
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        v[m][i] = ap_word(p.y, min(m, p.M - 1) * (C >> 1) + 64 * min(wave + NW * i, KC - 1) + lane);
-        there = there && v[m][i] != kNotYet;
-      }
-    if (__all(there)) break;
-    __builtin_amdgcn_s_sleep(1);
-  }
-  float* red = reinterpret_cast<float*>(smem + NW * MR * RS * 2);  // [NW][MR][16 + 4]
-#pragma unroll
-  for (int m = 0; m < MR; ++m) {
-    float rs = 0.f;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      reinterpret_cast<uint32_t*>(ys + m * RS)[64 * i + lane] = v[m][i];
-      if (wave + NW * i < KC) rs += bflo(v[m][i]) + bfhi(v[m][i]);
-    }
-    rs = wave_sum(rs);
-    if (lane == 0) red[(wave * MR + m) * 20 + 16] = rs;
-  }
-  uint32_t msk = 0x000F000Fu, mag = 0x43004300u, mag_hi = 0x45004500u;
-  asm volatile("" : "+s"(msk));
-  asm volatile("" : "+v"(mag), "+v"(mag_hi));
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    if (wave + NW * i >= KC) break;  // (uniform)
-#pragma unroll
-    for (int t = 0; t < 4; ++t)  // (the operand's rows past MR are those below again)
-      ap_mfma<WF>(acc, *reinterpret_cast<const bf16x8*>(ys + (lane & (MR - 1)) * RS + 128 * i + 32 * g + 8 * t), w[i][0][t], w[i][V - 1][t], msk, mag,
-                  mag_hi);
-  }
-  if (lane < 16) {
-#pragma unroll
-    for (int m = 0; m < MR; ++m) red[(wave * MR + m) * 20 + lane] = acc[m];
-  }
-  __syncthreads();
-  if (tid >= 64) return;
-  float y = 0.f, r = 0.f;
-#pragma unroll
-  for (int q = 0; q < NW; ++q) {
-    y += red[(q * MR + om) * 20 + (tid & 15)];
-    r += red[(q * MR + om) * 20 + 16];
-  }
-  const bool live = (tid >> 4) < p.M;
-  const float xn = round_bf(x + round_bf(sz.x * (y - sz.y * r)));  // model.py:172
-  const uint32_t o = (uint32_t)f2bf(xn), pr = lane_xor1(o);
-  if (live && !(tid & 1)) st_out32(p.x + (size_t)om * C + on, o | (pr << 16));
-  if (p.nstat) {  // uniform
-    const float sq = row16_sum(round_bf(xn * xn));
-    if (live && (tid & 15) == 0) st_out32(p.nstat + (size_t)nt * 16 + om, __float_as_uint(sq));
-  }
-}
 
 // One row of bf16. Wave: two columns; lane: values 512 i + 8 lane .. + 7 of both
 template <int NI>
@@ -187,7 +88,7 @@ __device__ __forceinline__ void ap_bf16_row(const AttendProjParams& p, int nt, u
 // NI: codes: rounds of 8 chunks of 128 that cover C; bf16: steps of 512. MR: most rows.
 template <int HS, int WF, int MR, bool RANGES, int NI>
 __global__ __launch_bounds__(kApNT) void attend_proj_kernel(AttendProjParams p) {
-  constexpr int NW = kApNT / 64, kProj = WF == AP_BF16 ? NI * 1024 : NW * MR * (NI * 256 + 16 + 80);
+  constexpr int NW = kApNT / 64, kProj = WF == AP_BF16 ? NI * 1024 : hand_codes_lds<NW, MR, NI>();
   __shared__ __align__(16) unsigned char smem[std::max(attention_lds_floats<HS, kApNT>() * 4, kProj)];
   if ((int)blockIdx.x < p.heads) {
     const int h = blockIdx.x % p.nh, rest = blockIdx.x / p.nh, m = MR > 1 ? rest % p.M : 0, split = MR > 1 ? rest / p.M : rest;
@@ -203,7 +104,7 @@ __global__ __launch_bounds__(kApNT) void attend_proj_kernel(AttendProjParams p) 
   if ((int)threadIdx.x < 8 * p.M)
     st_out32(p.clear + (size_t)(threadIdx.x >> 3) * (p.C >> 1) + 8 * nt + (threadIdx.x & 7), kNotYet);
   if constexpr (WF == AP_BF16) ap_bf16_row<NI>(p, nt, smem);
-  else ap_codes<WF, MR, NI>(p, nt, smem);
+  else hand_codes<WF, NW, MR, NI>(HandCodes{p.y, p.W, p.sz, p.x, p.nstat, p.M, p.C, p.C}, nt, smem);
 }
 
 template <int WF, int MR, bool RANGES, int NI>

@@ -10,6 +10,7 @@
 // softmax; the groups of a wave merge through lane swaps, the waves through LDS.
 #pragma once
 #include "common.h"
+#include "handover.h"
 #include "i8ws.h"
 
 namespace llj {
@@ -62,15 +63,13 @@ template <int HS>
 constexpr int kAttPart = HS + 4;  // floats per partial record: HS outputs, max, sum, 2 pad (16-byte records)
 
 // y[m, h * HS + d] of thread d < HS, adjacent dims as one 4-byte store; with st the LLM.int8 statistics of y, one slot per head.
-// HAND: to workgroups of the same launch that wait for every word of y to differ from kNotYet (attend_proj.hip).
-constexpr uint32_t kNotYet = 0xFFFFFFFFu;  // two NaNs; as outputs they leave as two others
+// HAND: to workgroups of the same launch that wait for y (handover.h).
 template <int HS, bool HAND = false>
 __device__ __forceinline__ void attention_out(float v, bf16_t* __restrict__ y, uint32_t* st, float thr, int h, int m, int C) {
   const int d = threadIdx.x;
   const uint32_t ob = (uint32_t)f2bf(v), pr = lane_xor1(ob);
-  uint32_t w = ob | (pr << 16);
-  if (HAND && w == kNotYet) w = 0x7FFF7FFFu;
-  if (!(d & 1)) st_out32(y + (size_t)m * C + h * HS + d, w);
+  const uint32_t w = ob | (pr << 16);
+  if (!(d & 1)) st_out32(y + (size_t)m * C + h * HS + d, HAND ? hand_word(w) : w);
   if (st) i8_emit_stats64(st, thr, m, h * HS + (d & ~63), ob, h);  // (uniform)
 }
 

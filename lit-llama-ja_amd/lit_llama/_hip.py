@@ -132,6 +132,9 @@ SIGNATURES = {
     "llj_streams_embed": [_P, _P, _I, _F, _P, _P, _I, _I, _P, _P, _F, _P, _I, _I, _I, _I, _P],
     "llj_streams_step": [_P, _I, _P, _P, _P, _I, _I, _P, _P, _F, _P, _I, _P, _I, _I, _I, _P],
     "llj_attention_proj_ok": [_I, _I, _I],
+    "llj_small_step_ok": [_I, _I, _I, _I, _I],
+    "llj_small_begin": [_P, _P, _P, _I, _P, _P, _I, _P],
+    "llj_small_step": [_P, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P],
     "llj_attention_resid_ok": [_I, _I, _I, _I],
     "llj_attention_proj": [_P, _P, _P, _P, _I, _I, _I, _P, _P, _P],
     "llj_sums_swiglu": [_P, _P, _I, _P, _P, _F, _P, _P, _P, _I, _I, _P],
@@ -157,6 +160,7 @@ SIZE_SIGNATURES = {
     "llj_attention_ws_bytes": [_I, _I, _I, _I],
     "llj_g_i8_ws_bytes": [_I, _I],
     "llj_i8_rowstats_bytes": [_I],
+    "llj_small_step_words": [_I, _I, _I],
     "llj_gemm_resid_ws_bytes": [_I, _I, _I, _I],
     "llj_gemm_swiglu_ws_bytes": [_I, _I, _I, _I],
     "llj_g_linear_ws_bytes": [_I, _I, _I, _I, _I],

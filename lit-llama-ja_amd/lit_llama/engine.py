@@ -32,7 +32,7 @@ import weakref
 import torch
 
 from . import _hip
-from .model import LLaMA, _Work, _enable_attend, _enable_i8_handoff
+from .model import LLaMA, _SmallStep, _Work, _enable_attend, _enable_i8_handoff
 from .state import Rows
 
 
@@ -121,6 +121,7 @@ class LLaMAProgram(_Program):
         s = self.sess
         m = s.model
         s.specs = m._layer_specs()
+        self.small = None
         if m._generic():  # the any-shape kernels (csrc/generic.hip)
             s.work = _Work(m.config, s.B, self.dev, False, s.S, generic=True, dtype=m.act_dtype())
         else:
@@ -128,6 +129,9 @@ class LLaMAProgram(_Program):
             s.work = _Work(m.config, s.B, self.dev, need_i8, s.S)
             _enable_i8_handoff(s.work, s.specs)
             _enable_attend(s.work, s.specs, s.B, 1, m.config.n_head)
+
+        if _SmallStep.ok(m, s.specs, s.B, s.S):
+            self.small = _SmallStep(m, s.specs, s.S)
 
     def reset_handoff(self):
         """The LLM.int8 hand-off blocks (_Work.y_st / h_st) must be zero when a step starts, and the attention's output (y_hand)
@@ -144,13 +148,16 @@ class LLaMAProgram(_Program):
         m, w, B = s.model, s.work, s.B
         cfg = m.config
         try:
-            if w.generic:
+            if self.small is not None:
+                self.small.step(m, s.cur, w.x, s.pos, st)
+            elif w.generic:
                 _hip.call("llj_g_embedding", s.cur.data_ptr(), m.transformer.wte.weight.data_ptr(), w.x.data_ptr(), B,
                           cfg.n_embd, s.pos.data_ptr(), w.dt, st)
             else:
                 _hip.call("llj_embedding", s.cur.data_ptr(), m.transformer.wte.weight.data_ptr(), w.x.data_ptr(), B,
                           cfg.n_embd, s.pos.data_ptr(), st)
-            m._blocks(w, s.specs, m.kv_caches, s.pos, B, 1, s.S, st)
+            if self.small is None:
+                m._blocks(w, s.specs, m.kv_caches, s.pos, B, 1, s.S, st)
             m._head(w.x, B, s.specs, s.logits, st, w)
         except BaseException:
             self.reset_handoff()

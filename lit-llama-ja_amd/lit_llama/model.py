@@ -23,6 +23,7 @@ any-shape kernels in fp32); there is no CPU path.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 import types
@@ -252,6 +253,39 @@ def _enable_attend(w: "_Work", specs, B: int, T: int, nh: int) -> None:
             and all(s[1][0] == layers[0][1][0] and s[1][1].data_ptr() % 16 == 0 for s in layers)
             and _hip.lib().llj_attention_resid_ok(layers[0][1][0], B, nh, C // nh)):
         w.y_hand = torch.full((3, B * C // 2), -1, dtype=torch.int32, device=w.x.device)
+
+
+class _SmallStep:
+    """A session's decode step of one row of a small bf16 model: all layers in one launch (llj_small_step)."""
+
+    def __init__(self, model: "LLaMA", specs, S: int):
+        cfg, L = model.config, _hip.lib()
+        C, H = cfg.n_embd, MLP.hidden(cfg)
+        self.shape = (cfg.n_layer, C, H, cfg.n_head, S)
+        self.eps = model.transformer.ln_f.eps
+        ptrs = []
+        for blk, (sa, sp, s1, s2, sd), (k, v) in zip(model.transformer.h, specs["layers"], model.kv_caches):
+            ptrs += [t.data_ptr() for t in (blk.rms_1.scale, sa[1], sp[1], blk.rms_2.scale, s1[1], s2[1], sd[1], k, v)]
+        self.layers = (ctypes.c_void_p * len(ptrs))(*ptrs)
+        self.words = int(L.llj_small_step_words(*self.shape[:3]))
+        self.hand = torch.empty(self.words, dtype=torch.int32, device=model.transformer.wte.weight.device)
+
+    @staticmethod
+    def ok(model: "LLaMA", specs, B: int, S: int) -> bool:
+        cfg, bf = model.config, torch.bfloat16
+        if B != 1 or len(specs["layers"]) != cfg.n_layer or not _hip.lib().llj_small_step_ok(cfg.n_layer, cfg.n_embd, MLP.hidden(cfg), cfg.n_head, S):
+            return False
+        norms = [n for blk in model.transformer.h for n in (blk.rms_1, blk.rms_2)]
+        dense = [s[1] for layer in specs["layers"] for s in layer if s[0] == 1]
+        return (len(dense) == 5 * cfg.n_layer and all(n.eps == model.transformer.ln_f.eps for n in norms)
+                and all(t.dtype == bf and t.is_contiguous() and t.data_ptr() % 8 == 0 for t in dense + [n.scale for n in norms] + [model.transformer.wte.weight])
+                and all(t.dtype == bf and t.data_ptr() % 4 == 0 for kv in model.kv_caches for t in kv))
+
+    def step(self, model: "LLaMA", cur, x, pos, st) -> None:
+        _hip.call("llj_small_begin", cur.data_ptr(), model.transformer.wte.weight.data_ptr(), x.data_ptr(), self.shape[1], pos.data_ptr(),
+                  self.hand.data_ptr(), self.words, st)
+        _hip.call("llj_small_step", ctypes.addressof(self.layers), *self.shape, self.eps, model.rope_cache.data_ptr(), pos.data_ptr(), x.data_ptr(),
+                  self.hand.data_ptr(), st)
 
 
 class _Work:

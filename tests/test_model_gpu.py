@@ -755,3 +755,37 @@ def test_generate_main_reads_reference_written_checkpoint(tmp_path, capsys, monk
     top = np.sort(logits, -1)[:, ::-1][:, :2]
     # oracle margins on this file are 1.3-44 % of max|logit| (bf16 path noise ~1 %): all steps are compared
     guarded(ids, ref_ids, top, 4, tol=0.01 * np.abs(logits).max())
+
+
+@pytest.mark.parametrize("n_embd,n_head,n_layer,P,S,steps", [(512, 8, 2, 3, 12, 30), (520, 10, 1, 1, 200, 20), (780, 10, 3, 130, 160, 12), (640, 10, 16, 64, 96, 6),
+                                                             (1024, 8, 2, 250, 300, 10), (768, 12, 2, 400, 512, 6)])
+def test_small_model_steps_in_one_launch(n_embd, n_head, n_layer, P, S, steps, monkeypatch):
+    """llj_small_step (all layers of a decode step in one launch) against the launches of their own, on given tokens: one to sixteen layers, heads of 52 to
+    128, partial pieces of 256 values, one to four passes of keys, a wrapped cache; as a graph's replays and eagerly the same bits. Bound: both
+    round to bf16 at the same places and add in other orders, which moves the logits as far as either is from the fp32 restatement."""
+    from lit_llama import engine
+
+    cfg = Cfg(block_size=640, n_layer=n_layer, n_head=n_head, n_embd=n_embd, vocab_size=512)
+    params = make_params(cfg, n_embd)
+    m = build(cfg, params)
+    rng = np.random.default_rng(n_embd)
+    ids = rng.integers(3, 512, P + steps)
+
+    def logits(small, graph=True):
+        with monkeypatch.context() as mp:
+            if not small:
+                mp.setattr(engine._SmallStep, "ok", staticmethod(lambda *a: False))
+            s = engine.DecodeSession(m, 1, S, P + steps + 1, top_k=1, use_graph=graph)
+            s.prefill(torch.from_numpy(ids[None, :P]).cuda())
+            assert (s.program.small is not None) == small
+            return torch.stack([s.feed([t])[0].float() for t in ids[P:]]).cpu().numpy()
+
+    one, eager, many = logits(True), logits(True, False), logits(False)
+    np.testing.assert_array_equal(one, eager)
+    assert np.isfinite(one).all()
+    far = np.linalg.norm(one - many) / np.linalg.norm(many)
+    assert far <= 0.02, far
+    if P + steps <= S:
+        want = O.OracleLLaMA(cfg, params).forward(ids[None].astype(np.int64))[0, P:]
+        err = [np.linalg.norm(x[:, : want.shape[1]] - want) / np.linalg.norm(want) for x in (one, many)]
+        assert err[0] <= 1.5 * err[1] + 2e-3, err
