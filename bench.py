@@ -759,7 +759,7 @@ def main():
                              "in_graph_frac": round(k_bytes / (in_graph[0] * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
                              "in_graph_source": f"profiles/{in_graph[1]} (rocprofv3 kernel trace of bench.py --decode-only)"}
                             if in_graph and head7 else {})},
-            "decode_path": "launch chain (5 fused launches per layer)",
+            "decode_path": "launch chain (4 fused launches per layer)",
             "step_roofline": {"bytes_per_step": sb, "achieved": round(step_gbs, 1), "frac": round(step_gbs / HBM_PEAK_GBS, 4),
                               "frac_of_achievable": round(step_gbs / ach, 4)},
             "reference_formula_tokens_per_s": round(r["tokens"] / (r["seconds"] + r["t_prefill"]), 2),
