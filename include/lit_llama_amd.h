@@ -156,14 +156,17 @@ int llj_sums_swiglu(const void* x, const float* parts, int nparts, void* x_out, 
  * part_ws (llj_attention_ws_bytes(B*T, n_head, head_size, nsplit) bytes), merged in split order
  * by a second launch. nsplit <= 1 is llj_attention itself. Same softmax up to summation order. */
 size_t llj_attention_ws_bytes(int rows, int n_head, int head_size, int nsplit);
-/* One decode row through all L layers of a small bf16 model (model.py:162-175) in one launch. layers: L x 9 device pointers (a host array): rms_1 scale, c_attn,
- * attn.c_proj, rms_2 scale, c_fc1, c_fc2, mlp.c_proj, K and V cache (n_head, S, hs); x (C) in and out; hand: llj_small_step_words(L, C, H) words, all
- * 0xFFFFFFFF when it starts. llj_small_begin, the launch before it: those words, x = wte[idx[0]], pos[0] += 1. llj_small_step_ok: shapes taken. */
+/* One decode row through all L layers of a small bf16 model (model.py:162-175) in one launch, and a second one that does what the first left undone
+ * where its workgroups waited long for one another (`waits` polls, 0: some milliseconds; beside other such launches). layers: L x 9 device pointers (a
+ * host array): rms_1 scale, c_attn, attn.c_proj, rms_2 scale, c_fc1, c_fc2, mlp.c_proj, K and V cache (n_head, S, hs); x (C): the row after them.
+ * hand: llj_small_step_words(L, C, H) words, set by llj_small_begin, the launch before it, which also takes wte[idx[0]] and adds 1 to
+ * pos[0]. failed: set to 1 if a wait of the second launch ran out (a second or more, or -waits polls of both launches for waits < 0), which its order of places rules
+ * out; x and the caches' new rows are then not valid. llj_small_step_ok: shapes taken. */
 int llj_small_step_ok(int L, int C, int H, int nh, int S);
 size_t llj_small_step_words(int L, int C, int H);
-int llj_small_begin(const int* idx, const void* wte, void* x, int C, int* pos, void* hand, int words, void* stream);
+int llj_small_begin(const int* idx, const void* wte, int L, int C, int H, int* pos, void* hand, void* stream);
 int llj_small_step(const void* const* layers, int L, int C, int H, int nh, int S, float eps, const float* rope, const int* pos, void* x, void* hand,
-                   void* stream);
+                   int* failed, int waits, void* stream);
 
 /* The attention of M decode rows (M sequences at one position, M <= 2; bf16 weights: M = 1) and attn.c_proj with the residual add
  * (x += y . W^T, model.py:172) in one launch: y (M, C = nh * hs) holds 0xFFFFFFFF words when it starts and the attention's output when it ends;

@@ -2,16 +2,19 @@
 //
 // Every 4-byte word of the row holds kNotYet until its two values are there. The workgroups that wait bring their weights to registers
 // first and then read the row, past the caches, until no word is kNotYet: one trip through the memory system between the last store and the
-// product, where a launch of its own has its start, the trip and the weights' bytes. The waiting workgroups come last in the grid, and
-// workgroups start in that order: whatever else runs on the device, the ones waited for have started, and they wait for nobody. The wait is
-// bounded all the same (kWaits; past it the outputs are NaN). Words return to kNotYet in the launch before the one that uses them next.
+// product, where a launch of its own has its start, the trip and the weights' bytes. Words return to kNotYet in the launch before the one that uses
+// them next.
+//
+// The workgroups waited for come first in the grid, but that does not mean that they have started: each XCD starts its share of a launch in that order,
+// nothing orders the starts on different XCDs, and waiting workgroups keep their places, so that those of several launches can stand in the
+// way of the ones that they wait for. Every wait is bounded, and a launch is right however its waits end: see there.
 #pragma once
 #include "common.h"
 
 namespace llj {
 
 constexpr uint32_t kNotYet = 0xFFFFFFFFu;  // two NaNs; as outputs they leave as two others
-constexpr int kWaits = 1 << 20;  // about a second
+constexpr int kWaits = 1 << 20;  // polls, each a trip past the caches: a second or more
 
 __device__ __forceinline__ uint32_t hand_word(uint32_t w) { return w == kNotYet ? 0x7FFF7FFFu : w; }
 __device__ __forceinline__ uint32_t get_word(const uint32_t* y, int at) {

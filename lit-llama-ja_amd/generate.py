@@ -60,12 +60,14 @@ def _run_session(sess, idx, max_new_tokens, eos_id):
             gen = sess.output()[0, T:]
             hit = (gen == eos_id).nonzero()
             if hit.numel():  # the reference returns idx[:input_pos]: the EOS token is excluded
+                sess.check()
                 return sess.output()[0, :T + int(hit[0, 0])].to(idx.dtype)
         if left == 0:
             break
         n = min(left, EOS_CHECK_EVERY) if eos_id is not None else left
         sess.decode(n)
         left -= n
+    sess.check()
     return sess.output()[0].to(idx.dtype)
 
 
@@ -84,6 +86,7 @@ def generate_batch(model: LLaMA, idx: torch.Tensor, max_new_tokens: int, *, max_
     sess.prefill(idx)
     if max_new_tokens > 1:
         sess.decode(max_new_tokens - 1)
+    sess.check()
     out = sess.output()
     out = [r.to(idx[0].dtype) for r in out] if isinstance(out, list) else out.to(idx[0].dtype)
     if eos_id is None:

@@ -133,8 +133,8 @@ SIGNATURES = {
     "llj_streams_step": [_P, _I, _P, _P, _P, _I, _I, _P, _P, _F, _P, _I, _P, _I, _I, _I, _P],
     "llj_attention_proj_ok": [_I, _I, _I],
     "llj_small_step_ok": [_I, _I, _I, _I, _I],
-    "llj_small_begin": [_P, _P, _P, _I, _P, _P, _I, _P],
-    "llj_small_step": [_P, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P],
+    "llj_small_begin": [_P, _P, _I, _I, _I, _P, _P, _P],
+    "llj_small_step": [_P, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P],
     "llj_attention_resid_ok": [_I, _I, _I, _I],
     "llj_attention_proj": [_P, _P, _P, _P, _I, _I, _I, _P, _P, _P],
     "llj_sums_swiglu": [_P, _P, _I, _P, _P, _F, _P, _P, _P, _I, _I, _P],

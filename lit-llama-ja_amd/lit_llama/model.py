@@ -267,8 +267,9 @@ class _SmallStep:
         for blk, (sa, sp, s1, s2, sd), (k, v) in zip(model.transformer.h, specs["layers"], model.kv_caches):
             ptrs += [t.data_ptr() for t in (blk.rms_1.scale, sa[1], sp[1], blk.rms_2.scale, s1[1], s2[1], sd[1], k, v)]
         self.layers = (ctypes.c_void_p * len(ptrs))(*ptrs)
-        self.words = int(L.llj_small_step_words(*self.shape[:3]))
-        self.hand = torch.empty(self.words, dtype=torch.int32, device=model.transformer.wte.weight.device)
+        self.hand = torch.empty(int(L.llj_small_step_words(*self.shape[:3])), dtype=torch.int32, device=model.transformer.wte.weight.device)
+        self.failed = torch.zeros(1, dtype=torch.int32, device=self.hand.device)
+        self.waits = 0  # the library's bound
 
     @staticmethod
     def ok(model: "LLaMA", specs, B: int, S: int) -> bool:
@@ -282,10 +283,10 @@ class _SmallStep:
                 and all(t.dtype == bf and t.data_ptr() % 4 == 0 for kv in model.kv_caches for t in kv))
 
     def step(self, model: "LLaMA", cur, x, pos, st) -> None:
-        _hip.call("llj_small_begin", cur.data_ptr(), model.transformer.wte.weight.data_ptr(), x.data_ptr(), self.shape[1], pos.data_ptr(),
-                  self.hand.data_ptr(), self.words, st)
-        _hip.call("llj_small_step", ctypes.addressof(self.layers), *self.shape, self.eps, model.rope_cache.data_ptr(), pos.data_ptr(), x.data_ptr(),
+        _hip.call("llj_small_begin", cur.data_ptr(), model.transformer.wte.weight.data_ptr(), *self.shape[:3], pos.data_ptr(),
                   self.hand.data_ptr(), st)
+        _hip.call("llj_small_step", ctypes.addressof(self.layers), *self.shape, self.eps, model.rope_cache.data_ptr(), pos.data_ptr(), x.data_ptr(),
+                  self.hand.data_ptr(), self.failed.data_ptr(), self.waits, st)
 
 
 class _Work:

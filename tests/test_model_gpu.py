@@ -789,3 +789,81 @@ def test_small_model_steps_in_one_launch(n_embd, n_head, n_layer, P, S, steps, m
         want = O.OracleLLaMA(cfg, params).forward(ids[None].astype(np.int64))[0, P:]
         err = [np.linalg.norm(x[:, : want.shape[1]] - want) / np.linalg.norm(want) for x in (one, many)]
         assert err[0] <= 1.5 * err[1] + 2e-3, err
+
+
+@pytest.mark.parametrize("n_embd,n_head,n_layer,S", [(640, 10, 3, 64), (520, 10, 1, 64), (780, 10, 2, 17), (1024, 8, 16, 40)])
+def test_small_model_step_done_again(n_embd, n_head, n_layer, S):
+    """llj_small_step whose first launch gives up at once (a bound of one poll a wait): the second one does what is left, in place of all the first, eagerly and in
+    a graph, over a wrapped cache; the logits differ by the order of nothing. With such a bound in both it says that it failed, and the next
+    prompt starts anew."""
+    from lit_llama import engine
+
+    cfg = Cfg(block_size=640, n_layer=n_layer, n_head=n_head, n_embd=n_embd, vocab_size=512)
+    m = build(cfg, make_params(cfg, 7))
+    ids = np.random.default_rng(7).integers(3, 512, 32)
+    prompt = torch.from_numpy(ids[None, :12]).cuda()
+
+    def session(waits, graph):
+        s = engine.DecodeSession(m, 1, S, 64, top_k=1, use_graph=graph)
+        s.prefill(prompt)
+        s.program.small.waits = waits
+        return s
+
+    def fed(waits, graph):
+        s = session(waits, graph)
+        out = torch.stack([s.feed([t])[0].clone() for t in ids[12:]])
+        undone = s.program.small.hand[-(n_embd // 2 + 32)]
+        assert (int(undone) != -1) == (waits == 1)
+        return out
+
+    want = fed(0, True)
+    assert want.isfinite().all()
+    for graph in (False, True):
+        assert torch.equal(fed(1, graph), want), graph
+    s = session(-1, False)
+    with pytest.raises(RuntimeError, match="waited too long"):
+        s.feed([int(ids[12])])
+    with pytest.raises(RuntimeError, match="waited too long"):
+        s.check()
+    s.prefill(prompt)
+    assert torch.equal(s.feed([int(ids[12])])[0], want[0])
+
+
+def test_small_model_steps_on_two_streams():
+    """Two sessions' steps at once, each launch of more workgroups than the chip holds: both end, with the bits that each has alone."""
+    import threading
+
+    from lit_llama import engine
+
+    cfg = Cfg(block_size=640, n_layer=16, n_head=10, n_embd=640, vocab_size=512)
+    models = [build(cfg, make_params(cfg, seed)) for seed in (1, 2)]
+    prompts = [torch.from_numpy(np.random.default_rng(seed).integers(3, 512, (1, 20))).cuda() for seed in (1, 2)]
+    n = 120
+    alone, both, streams = [], [None, None], [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+
+    def run(i):
+        with torch.cuda.stream(streams[i]):
+            s = engine.DecodeSession(models[i], 1, 200, 200, top_k=1)
+            s.prefill(prompts[i])
+            assert s.program.small is not None
+            s.capture()
+            start.wait(60)
+            s.decode(n)
+            return s.output().cpu(), s.logits.cpu()
+
+    start = threading.Barrier(1)
+    for i in range(2):
+        alone.append(run(i))
+    start = threading.Barrier(2)
+
+    def keep(i):
+        both[i] = run(i)
+
+    threads = [threading.Thread(target=keep, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    for a, b in zip(alone, both):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])

@@ -189,3 +189,29 @@ def test_graphs_dropped_during_a_capture_wait_for_its_end(monkeypatch):
     assert log.count("free") == 8 and log.count("step") == 2 and "freed inside" not in log
     drop(3)
     assert log.count("free") == 9  # two are kept
+
+
+def test_failed_step_raises(monkeypatch):
+    """A step that says on the device that it failed (a wait ran out): check() and the reads that wait for the steps raise, until the next prompt; a
+    program without such steps has nothing to check."""
+    import generate
+
+    monkeypatch.setattr("lit_llama._hip.require_device", lambda *a: None)
+    monkeypatch.setattr(DecodeSession, "decode", lambda self, n: None)
+    monkeypatch.setattr(DecodeSession, "prefill", lambda self, prompts: None)
+    model = _Model(LLaMAProgram)
+    model.transformer = types.SimpleNamespace(wte=types.SimpleNamespace(weight=torch.zeros(1)))
+    sess = DecodeSession(model, 1, 16, 16)
+    sess.lens, sess.steps_done, ids = [3], 2, torch.arange(3)
+    eos = int(sess.tokens[0, 3])
+    reads = [sess.check, lambda: sess.feed([1]), lambda: generate._run_session(sess, ids, 2, None), lambda: generate._run_session(sess, ids, 2, eos)]
+    for read in reads:
+        read()
+    sess.program.small = types.SimpleNamespace(failed=torch.zeros(1, dtype=torch.int32))
+    for read in reads:
+        read()
+    sess.program.small.failed.fill_(1)
+    for read in reads:
+        with pytest.raises(RuntimeError, match="waited too long"):
+            read()
+    DecodeSession(_Model(HybridProgram), 1, 16, 16).check()
