@@ -175,6 +175,10 @@ int llj_small_step(const void* const* layers, int L, int C, int H, int nh, int S
 int llj_attention_resid_ok(int wfmt, int M, int nh, int hs);
 int llj_attention_resid(int wfmt, const void* q, const void* kcache, const void* vcache, void* y, void* y_next, const int* pos, int M, int nh,
                         int hs, int S, int nsplit, void* part, int* count, const void* W, const void* sz, void* x, float* nstat_out, void* stream);
+/* The same with a bound on the polls of a wait for y (0: the library's, some milliseconds), past which a workgroup forms what is missing itself. */
+int llj_attention_resid_waits(int wfmt, const void* q, const void* kcache, const void* vcache, void* y, void* y_next, const int* pos, int M, int nh,
+                              int hs, int S, int nsplit, void* part, int* count, const void* W, const void* sz, void* x, float* nstat_out, int waits,
+                              void* stream);
 
 /* Decode attention (model.py:237) as nsplit <= 4 interleaved key splits per (row, head) whose
  * unnormalized partials (outputs, max, sum; llj_attention_ws_bytes layout) go to part_ws with no

@@ -78,9 +78,41 @@ __device__ __forceinline__ void attention_out(float v, bf16_t* __restrict__ y, u
 struct NoLoads {
   __device__ __forceinline__ void operator()() const {}
 };
+// The head's ranges merged, by threads d < HS: every range's pieces requested at once, added in range order (nsplit <= 64).
+template <int HS, bool HAND>
+__device__ __forceinline__ void attention_merge(const float* part, bf16_t* __restrict__ y, uint32_t* st, float thr, int h, int m, int nh, int nsplit) {
+  const int d = threadIdx.x, lane = d & 63;
+  const float* src = part + (size_t)(m * nh + h) * nsplit * kAttPart<HS>;
+  float O = 0.f;
+  constexpr int R = 16;
+  float pc[R];
+  auto pieces = [&](int s0) {  // (past the end: a copy, not used)
+#pragma unroll
+    for (int e = 0; e < R; ++e) pc[e] = get1(src + (size_t)min(s0 + e, nsplit - 1) * kAttPart<HS> + d);
+  };
+  pieces(0);
+  float2 ml = make_float2(-INFINITY, 0.f);  // lane s: range s (nsplit <= 64)
+  if (lane < nsplit) ml = get2(src + (size_t)lane * kAttPart<HS> + HS);
+  const float M = wave_max(ml.x);  // (in every lane: not inside the selection)
+  const float w = ml.x == -INFINITY ? 0.f : exp2f(ml.x - M);
+  auto of_range = [](float v, int s) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), s)); };
+  float L = 0.f;  // both sums in attention_combine_kernel's order: the same bits
+  for (int s0 = 0; s0 < nsplit; s0 += R) {
+    if (s0) pieces(s0);
+#pragma unroll
+    for (int e = 0; e < R; ++e) {
+      if (s0 + e >= nsplit) break;  // (uniform; s0 + e < 64)
+      const float f = of_range(w, s0 + e);
+      L += of_range(ml.y, s0 + e) * f;
+      O += pc[e] * f;
+    }
+  }
+  attention_out<HS, HAND>(O / L, y, st, thr, h, m, nh * HS);
+}
+
 // count (with PART, else partials only; nsplit <= 64): zeroed arrival counters, one per (row, head), left zero: the last of the
 // ranges' blocks to finish merges them. The hand-off is device-scope stores, a wait for them, the counter, device-scope
-// loads; no block waits for another.
+// loads; no block waits for another. HAND without count: the partials leave in the same way, for attention_merge.
 template <int HS, int U, int NTH, bool PART = false, int SPECU = U / 2, bool ILV = false, bool KEEP = false, bool HAND = false,
           typename F = NoLoads>
 __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
@@ -241,7 +273,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
     }
     if constexpr (PART) {  // unnormalized partial: outputs, then (max, sum)
       float* dst = part + ((size_t)(m * nh + h) * nsplit + split) * kAttPart<HS>;
-      if (count) {
+      if (HAND || count) {
         const float O1 = lane_xor1(O);
         if (!(d & 1)) put2(dst + d, O, O1);
         if (d == 0) put2(dst + HS, M, L);
@@ -263,7 +295,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
   LLJ_STAMP(5);
   if constexpr (PART) {
     if (!count) return;
-    // ---- the last of the ranges' blocks merges them: every range's pieces requested at once, added in range order
+    // ---- the last of the ranges' blocks merges them
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials are out
     __syncthreads();
     int* last = reinterpret_cast<int*>(s_m);
@@ -275,33 +307,7 @@ __device__ __forceinline__ void attention_body(const bf16_t* __restrict__ q, con
     }
     __syncthreads();
     if (!*last || threadIdx.x >= HS) return;
-    const int d = threadIdx.x, lane = d & 63;
-    const float* src = part + (size_t)(m * nh + h) * nsplit * kAttPart<HS>;
-    float O = 0.f;
-    constexpr int R = 16;
-    float pc[R];
-    auto pieces = [&](int s0) {  // (past the end: a copy, not used)
-#pragma unroll
-      for (int e = 0; e < R; ++e) pc[e] = get1(src + (size_t)min(s0 + e, nsplit - 1) * kAttPart<HS> + d);
-    };
-    pieces(0);
-    float2 ml = make_float2(-INFINITY, 0.f);  // lane s: range s (nsplit <= 64)
-    if (lane < nsplit) ml = get2(src + (size_t)lane * kAttPart<HS> + HS);
-    const float M = wave_max(ml.x);  // (in every lane: not inside the selection)
-    const float w = ml.x == -INFINITY ? 0.f : exp2f(ml.x - M);
-    auto of_range = [](float v, int s) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), s)); };
-    float L = 0.f;  // both sums in attention_combine_kernel's order: the same bits
-    for (int s0 = 0; s0 < nsplit; s0 += R) {
-      if (s0) pieces(s0);
-#pragma unroll
-      for (int e = 0; e < R; ++e) {
-        if (s0 + e >= nsplit) break;  // (uniform; s0 + e < 64)
-        const float f = of_range(w, s0 + e);
-        L += of_range(ml.y, s0 + e) * f;
-        O += pc[e] * f;
-      }
-    }
-    attention_out<HS, HAND>(O / L, y, st, thr, h, m, C);
+    attention_merge<HS, HAND>(part, y, st, thr, h, m, nh, nsplit);
   }
 }
 

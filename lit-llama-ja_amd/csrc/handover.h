@@ -40,14 +40,15 @@ struct HandCodes {
   bf16_t* x;          // residual (M, N), in place: x += y . W^T in bf16 (model.py:172-173)
   float* nstat;       // sums of squares of x', 16 columns a place (llj_linear_resid's nstat_out), or NULL
   int M, N, K;
+  int waits;  // polls of a wait
 };
 template <int NW, int MR, int NI>
-constexpr int hand_codes_lds() { return NW * MR * (NI * 256 + 16 + 80); }
+constexpr int hand_codes_lds() { return NW * (MR * (NI * 256 + 16 + 80) + 4); }
 
 // Columns 16 nt .. + 15 for up to MR rows, by NW waves. Wave: chunks wave + NW i of 128 values, at most NI; lane: the codes of column
-// lane % 16, 32 of a chunk's values.
+// lane % 16, 32 of a chunk's values. false (in every thread), with nothing written: a wait ran out.
 template <int WF, int NW, int MR, int NI>
-__device__ __forceinline__ void hand_codes(const HandCodes& p, int nt, unsigned char* smem) {
+__device__ __forceinline__ bool hand_codes(const HandCodes& p, int nt, unsigned char* smem) {
   constexpr int V = WF == HC_W8 ? 2 : 1, RS = NI * 128 + 8;  // (rows on other banks)
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6), KW = p.K >> 1;
   const int n0 = 16 * nt, KC = p.K >> 7, g = lane >> 4;
@@ -63,7 +64,8 @@ __device__ __forceinline__ void hand_codes(const HandCodes& p, int nt, unsigned 
   // this wave's own values of y: word `lane` of each of its chunks
   bf16_t* ys = reinterpret_cast<bf16_t*>(smem) + wave * MR * RS;
   uint32_t v[MR][NI];
-  for (int t = 0; t < kWaits; ++t) {
+  bool got = false;
+  for (int t = 0; t < p.waits; ++t) {
     bool there = true;
 #pragma unroll
     for (int m = 0; m < MR; ++m)
@@ -72,9 +74,12 @@ __device__ __forceinline__ void hand_codes(const HandCodes& p, int nt, unsigned 
         v[m][i] = get_word(p.y, min(m, p.M - 1) * KW + 64 * min(wave + NW * i, KC - 1) + lane);
         there = there && v[m][i] != kNotYet;
       }
-    if (__all(there)) break;
+    got = __all(there);
+    if (got) break;
     __builtin_amdgcn_s_sleep(1);
   }
+  int* all = reinterpret_cast<int*>(smem + NW * MR * (RS * 2 + 80));  // [NW]
+  if (lane == 0) all[wave] = got;
   float* red = reinterpret_cast<float*>(smem + NW * MR * RS * 2);  // [NW][MR][16 + 4]
 #pragma unroll
   for (int m = 0; m < MR; ++m) {
@@ -104,7 +109,11 @@ __device__ __forceinline__ void hand_codes(const HandCodes& p, int nt, unsigned 
     for (int m = 0; m < MR; ++m) red[(wave * MR + m) * 20 + lane] = acc[m];
   }
   __syncthreads();
-  if (tid >= 64) return;
+  int every = 1;
+#pragma unroll
+  for (int q = 0; q < NW; ++q) every &= all[q];
+  if (!every) return false;
+  if (tid >= 64) return true;
   float y = 0.f, r = 0.f;
 #pragma unroll
   for (int q = 0; q < NW; ++q) {
@@ -119,6 +128,7 @@ __device__ __forceinline__ void hand_codes(const HandCodes& p, int nt, unsigned 
     const float sq = row16_sum(round_bf(xn * xn));
     if (live && (tid & 15) == 0) st_out32(p.nstat + (size_t)nt * 16 + om, __float_as_uint(sq));
   }
+  return true;
 }
 
 }  // namespace llj

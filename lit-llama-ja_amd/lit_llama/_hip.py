@@ -36,6 +36,7 @@ SIGNATURES = {
                           _P],
     "llj_attention_ranges": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _F, _P],
     "llj_attention_resid": [_I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
+    "llj_attention_resid_waits": [_I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P],
     "llj_attention_split": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P],
     "llj_gemm_i8_linear": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
     "llj_gemm_i8_linear_ws": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],

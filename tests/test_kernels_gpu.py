@@ -2359,3 +2359,51 @@ def test_attention_and_projection_in_one_launch(hip, wfmt, M, nh, S, p, nsplit):
     run(9, x, bad)
     torch.cuda.synchronize()
     assert x.isnan().all()
+
+
+@pytest.mark.parametrize("wfmt,M,nh,S,p,nsplit", [(0, 1, 32, 96, 0, 1), (0, 2, 40, 600, 500, 3), (1, 1, 32, 1033, 1000, 5), (1, 1, 40, 130, 128, 1), (1, 1, 16, 40, 100, 1),
+                                                  (3, 1, 32, 700, 699, 2), (3, 2, 16, 2048, 2047, 8), (3, 2, 40, 96, 95, 1)])
+def test_attention_and_projection_without_waiting(hip, wfmt, M, nh, S, p, nsplit):
+    """llj_attention_resid_waits with a bound of one poll, so that the product's workgroups form what is missing of the attention themselves, beside its own
+    workgroups: the bits of the launch that waits, for y, x and the sums of squares, in three launches eagerly and three replays of a graph; the next
+    place empty, the counters zero again."""
+    rng = np.random.default_rng(nh + S + M)
+    hs, C = 128, 128 * nh
+    g = torch.Generator(device=dev).manual_seed(S)
+    _, Wd, szd = quant_operands(hip, rng, wfmt, C, C)
+    q, x0 = (torch.randn(M, C, generator=g, device=dev).bfloat16() for _ in range(2))
+    kc, vc = (torch.randn(M, nh, S, hs, generator=g, device=dev).bfloat16() for _ in range(2))
+    pos = torch.tensor([p], dtype=torch.int32, device=dev)
+    part = torch.zeros(max(16, M * nh * nsplit * (hs + 4) * 4), dtype=torch.uint8, device=dev)
+    count = torch.zeros(M * nh, dtype=torch.int32, device=dev)
+    y, y_next = torch.empty(2, M, C // 2, dtype=torch.int32, device=dev)
+    nst = torch.zeros(C // 16, 16, device=dev)
+    x = torch.empty_like(x0)
+
+    def run(waits):
+        y.fill_(-1)
+        y_next.zero_()
+        part.zero_()
+        x.copy_(x0)
+        call(hip, "llj_attention_resid_waits", wfmt, q.data_ptr(), kc.data_ptr(), vc.data_ptr(), y.data_ptr(), y_next.data_ptr(), pos.data_ptr(), M, nh, hs, S,
+             nsplit, part.data_ptr(), count.data_ptr(), Wd.data_ptr(), szd.data_ptr() if szd is not None else None, x.data_ptr(),
+             nst.data_ptr() if M > 1 else None, waits, st())
+
+    def results():
+        torch.cuda.synchronize()
+        assert (y_next == -1).all() and not count.any()
+        return [t.clone() for t in (y, x, nst)]
+
+    run(0)
+    want = results()
+    assert want[1].isfinite().all()
+    for _ in range(3):
+        run(1)
+        assert all(map(torch.equal, results(), want))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        run(1)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        assert all(map(torch.equal, results(), want))
