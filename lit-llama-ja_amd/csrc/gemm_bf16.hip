@@ -31,7 +31,7 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(GemmParams p) {
   u32x4 wv[S], av[S][MT];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int k = 32 * min(k0 + s, k1 - 1);  // (past the share: its last step again, times zeros)
+    const int k = 32 * min(k0 + s, k1 - 1);  // (past the share: its last step again, not used)
     wv[s] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(w + k));
 #pragma unroll
     for (int i = 0; i < MT; ++i) av[s][i] = *reinterpret_cast<const u32x4*>(a[i] + k);
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(512) void gemm_few_kernel(GemmParams p) {
   __builtin_amdgcn_sched_barrier(0);  // (else each step's loads move to its products)
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    if (k0 + s >= k1) wv[s] = u32x4{0u, 0u, 0u, 0u};
+    if (k0 + s >= k1) break;  // (uniform)
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[i] = mfma_bf16(__builtin_bit_cast(bf16x8, av[s][i]), __builtin_bit_cast(bf16x8, wv[s]), acc[i]);
   }

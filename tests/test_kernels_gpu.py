@@ -2289,6 +2289,25 @@ def test_gemm_few_tiles_exact(hip, M, N, K):
         assert torch.equal(t[M], o[M]) and torch.equal(t[:, N:], o[:, N:])
 
 
+@pytest.mark.parametrize("M,N,K", [(20, 640, 640), (33, 512, 384), (17, 128, 256), (40, 640, 1792)])
+def test_gemm_few_infinities(hip, M, N, K):
+    """An infinity in any step of K, the last ones of the waves' shares among them (shares shorter than the longest multiply nothing twice): its row is that
+    infinity where the weight is positive, minus it where it is negative, and the other rows stay finite and exact."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A = torch.randint(-3, 4, (M, K), generator=g, device="cuda").bfloat16()
+    W = (torch.randint(1, 3, (N, K), generator=g, device="cuda") * (1 - 2 * torch.randint(0, 2, (N, K), generator=g, device="cuda"))).bfloat16()
+    clean = A.double() @ W.double().T
+    st = torch.cuda.current_stream().cuda_stream
+    for step in range(K // 32):
+        a, m, k = A.clone(), step % M, 32 * step + 7 * step % 32
+        a[m, k] = float("inf") if step % 2 else float("-inf")
+        want = clean.bfloat16()
+        want[m] = a[m, k] * W[:, k].sign()
+        out = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda")
+        call(hip, "llj_gemm_linear_ws", 1, a.data_ptr(), K, W.data_ptr(), None, out.data_ptr(), N, M, N, K, None, 0, st)
+        assert torch.equal(out, want), step
+
+
 @pytest.mark.parametrize("wfmt,M,nh,S,p,nsplit", [(0, 1, 32, 80, 0, 1), (0, 1, 40, 96, 63, 1), (0, 1, 16, 96, 64, 1), (0, 2, 32, 600, 500, 3),
                                                   (0, 2, 40, 70, 69, 1), (1, 1, 32, 1033, 1000, 5), (1, 1, 16, 40, 100, 1), (1, 1, 40, 130, 128, 1),
                                                   (3, 1, 32, 600, 599, 3), (3, 2, 16, 96, 95, 1), (3, 2, 40, 520, 3, 3)])
