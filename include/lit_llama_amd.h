@@ -352,8 +352,8 @@ int llj_gptq_next(const float* hinv, int K, int i1, const float* last, float* wt
                   float* qt, float* err, float* loss, void* stream);
 /* GPTQQuantizer.find_params_weight (475-514), per channel: (scale, zero) of N rows of K fp32 weights; sym: the symmetric range. */
 int llj_gptq_params(const float* w, int N, int K, int bits, int sym, float* scale, float* zero, void* stream);
-/* collect_input_stats (516-530): H = keep H + (alpha x)^T (alpha x), x (T, K) row-major, dt 0 = bf16, 1 = fp32, H (K, K) fp32
- * symmetric. Any T, K; fp32 sums over the rows in order. */
+/* collect_input_stats (516-530): H = keep H + (alpha x)^T (alpha x), x (T, K) row-major, dt 0 = bf16, 1 = fp32, H (K, K) fp32.
+ * H must be symmetric (either half is read for both) and stays so. Any T, K, 4-byte aligned H; fp32 sums over the rows in order. */
 int llj_gptq_gram(const void* x, int dt, int T, int K, float keep, float alpha, float* H, void* stream);
 /* W (N, K) in the loop's layout and column order: wt (K, N) with wt[place[k]][n] = W[n][k] (place NULL: k), zero for dead[k]. */
 int llj_gptq_weight(const float* W, const int64_t* place, const void* dead, int N, int K, float* wt, void* stream);

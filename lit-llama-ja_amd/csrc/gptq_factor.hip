@@ -24,8 +24,9 @@ __global__ __launch_bounds__(256) void gptq_gram_kernel(const S* __restrict__ x,
   triangle(t, ti, tj);
   const int m0 = ti * BT, n0 = tj * BT;
   f32x4 acc[G::MI][G::NI], old[G::MI][G::NI];
-  // (a lane's four sums of an MFMA tile are neighbours in the mirrored place: whole vectors there, of H's own symmetric other half too)
-  const bool whole = VEC && m0 + BT <= K && n0 + BT <= K;
+  // (a lane's four sums of an MFMA tile are neighbours in the mirrored place: whole vectors there, of H's own symmetric other half too. VEC says
+  // nothing of where H begins.)
+  const bool whole = VEC && ((uintptr_t)H & 15) == 0 && m0 + BT <= K && n0 + BT <= K;
   G::run(x + m0, K, K - m0, x + n0, K, K - n0, T, alpha, lds, acc, [&] {
     if (!whole) return;
     G::tiles([&](int a, int b, int i, int j) { old[a][b] = *reinterpret_cast<const f32x4*>(H + (size_t)(n0 + j) * K + m0 + i); });

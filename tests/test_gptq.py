@@ -542,6 +542,27 @@ def test_hessian_kernel(hip, T, K, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,K", [(70, 128), (40, 1536)])
+def test_hessian_kernel_alignment(hip, T, K):
+    """H and x wherever they begin, both tile sizes: the bits of the aligned ones, nothing outside H."""
+    from lit_llama import _hip
+    g = torch.Generator(device=dev).manual_seed(K)
+    x = torch.randn(T, K, generator=g, device=dev)
+    h0 = torch.randn(K, K, generator=g, device=dev)
+    h0 = h0 + h0.t()
+    outs = []
+    for at_x, at_h in ((0, 0), (0, 1), (0, 2), (1, 0), (3, 3)):
+        xb, hb = torch.zeros(T * K + 4, device=dev), torch.full((K * K + 8,), 7.0, device=dev)
+        xb[at_x:at_x + T * K], hb[at_h:at_h + K * K] = x.view(-1), h0.view(-1)
+        _hip.call("llj_gptq_gram", xb[at_x:].data_ptr(), 1, T, K, 0.5, 0.25, hb[at_h:].data_ptr(), torch.cuda.current_stream().cuda_stream)
+        outs.append(hb[at_h:at_h + K * K].clone())
+        assert (hb[:at_h] == 7).all() and (hb[at_h + K * K:] == 7).all()
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    want = 0.5 * h0.double() + 0.0625 * (x.double().t() @ x.double())
+    assert ((outs[0].view(K, K).double() - want).abs() <= (T + 8) * 2.0 ** -24 * (want.abs() + 0.0625 * (x.abs().double().t() @ x.abs().double()))).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("K", [128, 256, 384, 1152])
 def test_inverse_factor_kernel(hip, K):
     """llj_gptq_factor against float64: one block, two, and several, with and without an order; the input stays as it is, zeros below
