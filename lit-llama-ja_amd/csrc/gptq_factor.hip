@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void gptq_update_kernel(const float* __restric
 // later row block i (gptq_step_kernel): in H's upper triangle the next matrix to factor, in the lower one the growing L^-1.
 // The next diagonal block is factored by one workgroup of that launch while the others work on the rest: its chain (1.4 us
 // for its loads, 4 for its product, four times 2.9 for 32 pivots, 1.7 between them, 2 for the stores) bounds a step, the products (2 K^3 / 3 in
-// all, 0.3 ms at K = 4096) run beside it. K = 4096: 1.27 ms (39.6 us a step; 1.49 with the block's whole product, the other waves' updates before
+// all, 0.3 ms at K = 4096) run beside it and bound it from 6,144 columns on. K = 4096: 1.27 ms (39.6 us a step; 1.49 with the block's whole product, the other waves' updates before
 // the elimination and 4-byte stores) for 29.2 with the library's three calls, K = 512: 0.14 (35 a step; 0.17) for 3.1; error against float64 2.5e-7 for 1.1e-6 (8,192 rows).
 constexpr int kFs = kFactor + 16;  // LDS row stride of the diagonal block
 
@@ -301,18 +301,24 @@ __global__ __launch_bounds__(256) void gptq_panel_kernel(const float* __restrict
   G::each(acc, [&](int i, int j, float v) { P[(row + m0 + i) * K + n0 + j] = v; });
 }
 
-constexpr int kStepLds = 21000;  // floats: the diagonal block's 18,432, and more than half a CU's LDS (4,096 columns: 41.8 us a step with two to a CU, 39.6 so)
+constexpr int kStepLds = kFactor * kFs, kStepAlone = 21000;  // floats: the diagonal block's, and more than half a CU's LDS
+// Tiles of a step up to which workgroup 0 has its CU to itself (ALONE), so that its chain is not held up: up to 8 tiles a CU the chain is the longer. Past that
+// the products are, and one workgroup of theirs a CU, which ALONE makes of them too, is too few. ms of a factor, all steps alone -> by this rule
+// (two a CU in all): 4,096 columns 1.31 -> 1.31 (1.39), 5,120 2.01 -> 1.82 (1.86), 6,144 3.08 -> 2.62 (2.65), 8,192 6.52 -> 5.31 (5.33),
+// 11,008 15.3 -> 12.3 (12.3), 13,824 29.5 -> 24.1 (24.1); with 1,536 tiles 4,096 columns take 1.35, with 3,072 5,120 take 1.95.
+constexpr long kAloneTiles = 2048;
 
-// Workgroup 0, alone on its CU: the next diagonal block, updated and factored. The others: 64 x 64 tiles of the rows below, the lower triangle's columns
+// Workgroup 0: the next diagonal block, updated and factored. The others: 64 x 64 tiles of the rows below, the lower triangle's columns
 // up to block k (first sums in block k's own) and the upper triangle's.
+template <bool ALONE>
 __global__ __launch_bounds__(256) void gptq_step_kernel(float* __restrict__ M, float* __restrict__ P, int k, int K, float* __restrict__ xt, int* info) {
   typedef AtB<64, 64, float, true, false> G;
-  __shared__ __align__(16) float lds[kStepLds];
+  __shared__ __align__(16) float lds[ALONE ? kStepAlone : kStepLds];
   __shared__ int bad;
   const float* p = P + (size_t)k * kFactor * K;
   const int r0 = (k + 1) * kFactor;
   if (blockIdx.x == 0) {
-    __builtin_amdgcn_s_setprio(3);  // the longest chain of the launch, beside another workgroup's products
+    __builtin_amdgcn_s_setprio(3);  // the longest chain of the launch (not ALONE: beside another workgroup's products)
     switch (uniform(threadIdx.x >> 6)) {  // (the same barriers on every way)
       case 0: diagonal_block<0>(M, p, r0, K, lds); break;
       case 1: diagonal_block<1>(M, p, r0, K, lds); break;
@@ -442,7 +448,9 @@ int llj_gptq_factor(const float* H, const int64_t* perm, const float* damp, int 
     hipLaunchKernelGGL(gptq_panel_kernel, dim3(K / 64 * 2), dim3(256), 0, s, M, xt, k, K, P);
     if (k + 1 == nb) break;
     const long R = (K - (k + 1) * kFactor) / 64, C = (k + 1) * kFactor / 64, tiles = R * C + R * (R + 1) / 2;
-    hipLaunchKernelGGL(gptq_step_kernel, dim3((unsigned)(1 + (tiles + 7) / 8 * 8)), dim3(256), 0, s, M, P, k, K, xt, info);
+    const dim3 grid((unsigned)(1 + (tiles + 7) / 8 * 8));
+    if (tiles <= kAloneTiles) hipLaunchKernelGGL(gptq_step_kernel<true>, grid, dim3(256), 0, s, M, P, k, K, xt, info);
+    else hipLaunchKernelGGL(gptq_step_kernel<false>, grid, dim3(256), 0, s, M, P, k, K, xt, info);
   }
   hipLaunchKernelGGL(gptq_reverse_kernel, dim3((K + 255) / 256, K), dim3(256), 0, s, P, K, M);
   LLJ_CHECK_LAUNCH();

@@ -563,7 +563,7 @@ def test_hessian_kernel_alignment(hip, T, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("K", [128, 256, 384, 1152])
+@pytest.mark.parametrize("K", [128, 256, 384, 1152, 4224])  # (4224: steps past kAloneTiles and steps up to it)
 def test_inverse_factor_kernel(hip, K):
     """llj_gptq_factor against float64: one block, two, and several, with and without an order; the input stays as it is, zeros below
     the diagonal. Its error is held to the library's chain's on the same matrix."""
