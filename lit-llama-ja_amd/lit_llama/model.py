@@ -794,7 +794,8 @@ class LLaMA(nn.Module):
                           w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), rope.data_ptr(), pos.data_ptr(), B, T, C, nh,
                           S, r0, r, P(w.i8ws), P(rs), P(nst), w.npart, st)
             # 2. attention, 3. c_proj + residual
-            if w.parts is not None and T == 1 and fp == f1 == f2 == 1 and not w.hand:  # .. and 4.
+            if (w.parts is not None and T == 1 and fp == f1 == f2 == 1 and not w.hand
+                    and (wp.data_ptr() | w1.data_ptr() | w2.data_ptr() | blk.rms_2.scale.data_ptr() | kc.data_ptr() | vc.data_ptr()) % 16 == 0):  # .. and 4.
                 _hip.call("llj_attention_proj", w.q.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), nh, C // nh, S, wp.data_ptr(),
                           w.parts.data_ptr(), st)
                 _hip.call("llj_sums_swiglu", w.x.data_ptr(), w.parts.data_ptr(), nh, w.x2.data_ptr(), blk.rms_2.scale.data_ptr(),

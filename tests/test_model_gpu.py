@@ -791,6 +791,36 @@ def test_small_model_steps_in_one_launch(n_embd, n_head, n_layer, P, S, steps, m
         assert err[0] <= 1.5 * err[1] + 2e-3, err
 
 
+@pytest.mark.parametrize("which", ["c_proj", "c_fc1", "c_fc2", "rms_2", "cache"])
+def test_small_model_operands_off_16_bytes(which):
+    """One-row forwards of a small model whose weights or caches begin 8 bytes off (views of larger buffers): taken, with the logits of aligned ones. The two
+    differ by the order of fp32 sums and the bf16 roundings behind them, 2 layers of some 2^-8 each."""
+    cfg = Cfg(block_size=64, n_layer=2, n_head=10, n_embd=640, vocab_size=512)
+    m = build(cfg, make_params(cfg, 3))
+    ids = torch.from_numpy(np.random.default_rng(3).integers(3, 512, (1, 12))).cuda()
+
+    def off(t):
+        v = torch.empty(t.numel() + 4, dtype=t.dtype, device=t.device)[4:].view(t.shape)
+        return v.copy_(t)
+
+    @torch.no_grad()
+    def logits(caches=None):
+        m.reset_cache()
+        m.kv_caches = caches or []
+        return torch.cat([m(ids[:, i:i + 1], 32, torch.tensor([i], device="cuda"))[0] for i in range(12)]).float()
+
+    want = logits()
+    caches = None
+    if which == "cache":
+        caches = [tuple(off(torch.zeros(1, 10, 32, 64, dtype=torch.bfloat16, device="cuda")) for _ in range(2)) for _ in range(2)]
+    for blk in m.transformer.h:
+        for owner, name in ((blk.attn.c_proj, "weight"), (blk.mlp.c_fc1, "weight"), (blk.mlp.c_fc2, "weight"), (blk.rms_2, "scale")):
+            if {"c_proj": blk.attn.c_proj, "c_fc1": blk.mlp.c_fc1, "c_fc2": blk.mlp.c_fc2, "rms_2": blk.rms_2}.get(which) is owner:
+                setattr(owner, name, torch.nn.Parameter(off(getattr(owner, name).data), requires_grad=False))
+    got = logits(caches)
+    assert got.isfinite().all() and (got - want).norm() <= 2 * 2.0 ** -7 * want.norm()
+
+
 @pytest.mark.parametrize("n_embd,n_head,n_layer,S", [(640, 10, 3, 64), (520, 10, 1, 64), (780, 10, 2, 17), (1024, 8, 16, 40)])
 def test_small_model_step_done_again(n_embd, n_head, n_layer, S):
     """llj_small_step whose first launch gives up at once (a bound of one poll a wait): the second one does what is left, in place of all the first, eagerly and in
