@@ -115,9 +115,9 @@ class PackedLinear:
             _hip.call("llj_gemm_bf16", act, a.data_ptr(), a.stride(0), self.w.data_ptr(), bias, out.data_ptr(),
                       out.stride(0), M, self.Np, self.Kp, limit, alpha, _hip.ptr(ws), nb, st)
 
-    def takes_post(self, M: int, width: int) -> bool:
-        """Whether apply_post serves these rows."""
-        if self.dtype != torch.bfloat16 or width != self.K:
+    def takes_post(self, M: int, width: int, norm: torch.Tensor) -> bool:
+        """Whether apply_post serves these rows and this norm (it reads 16-byte pieces; a checkpoint's tensors may begin anywhere)."""
+        if self.dtype != torch.bfloat16 or width != self.K or norm.data_ptr() % 16:
             return False
         if M == 1:
             return width % 8 == 0 and width <= 8192

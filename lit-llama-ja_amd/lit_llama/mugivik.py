@@ -232,7 +232,7 @@ class Mugivik(HybridModel):
 
         def product(lin, out, relu2=False):
             nonlocal x, pending
-            if pending is not None and lin.takes_post(M, C) and taps is None:
+            if pending is not None and lin.takes_post(M, C, pending) and taps is None:
                 other = w.x2 if x is w.x else w.x
                 lin.apply_post(w.t, pending, eps, x, other, M, out, st, relu2)
                 x, pending = other, None

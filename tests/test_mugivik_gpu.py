@@ -36,6 +36,28 @@ def test_whole_prompts(hip, name, dtype):
         check(got, oracle(cfg, w, toks), dtype, (name, n))
 
 
+def test_norms_off_16_bytes(hip):
+    """Norm weights that are views 8 bytes into a larger buffer: few rows close them in a launch of their own, to the bits of the products that close aligned
+    ones (one row: to a few roundings, its two forms add in other orders)."""
+    from lit_llama.mugivik import Mugivik, MugivikConfig
+
+    cfg = config(2048, 512, [gla(8, 64, 128), gla(8, 64, 128)], 4096)
+    t = {k: torch.from_numpy(v).to("cuda", torch.bfloat16) for k, v in weights(cfg, 4).items()}
+    moved = {k: torch.cat([v.new_zeros(4), v])[4:] if k.endswith((".norm1", ".norm2")) else v for k, v in t.items()}
+    toks, out = prompts(cfg, [8], seed=6)[0], []
+    for tensors in (t, moved):
+        m = Mugivik.from_tensors(MugivikConfig.from_dict(cfg), tensors)
+        assert all((w.data_ptr() % 16 != 0) == (tensors is moved) for w in m.norm1 + m.norm2)
+        assert m.mlps[0].up.takes_post(2, 2048, m.norm1[0]) == (tensors is t)
+        out.append([])
+        for n in (1, 2, 3, 8):
+            st = m.new_state(1)
+            out[-1].append(m.extend(st, st.alloc(1), [0], [toks[:n]]).float())
+    for a, b in list(zip(*out))[1:]:
+        assert torch.equal(a, b)
+    assert (out[0][0] - out[1][0]).norm() <= 2.0 ** -6 * out[0][0].norm()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(CONFIGS))
 def test_residual_after_every_layer(hip, name, dtype):
