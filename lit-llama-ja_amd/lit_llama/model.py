@@ -263,10 +263,10 @@ class _SmallStep:
         C, H = cfg.n_embd, MLP.hidden(cfg)
         self.shape = (cfg.n_layer, C, H, cfg.n_head, S)
         self.eps = model.transformer.ln_f.eps
-        ptrs = []
+        self.tensors = []  # kept: the model may replace its own (reset_cache, a new Parameter) while steps go on
         for blk, (sa, sp, s1, s2, sd), (k, v) in zip(model.transformer.h, specs["layers"], model.kv_caches):
-            ptrs += [t.data_ptr() for t in (blk.rms_1.scale, sa[1], sp[1], blk.rms_2.scale, s1[1], s2[1], sd[1], k, v)]
-        self.layers = (ctypes.c_void_p * len(ptrs))(*ptrs)
+            self.tensors += [blk.rms_1.scale, sa[1], sp[1], blk.rms_2.scale, s1[1], s2[1], sd[1], k, v]
+        self.layers = (ctypes.c_void_p * len(self.tensors))(*(t.data_ptr() for t in self.tensors))
         self.hand = torch.empty(int(L.llj_small_step_words(*self.shape[:3])), dtype=torch.int32, device=model.transformer.wte.weight.device)
         self.failed = torch.zeros(1, dtype=torch.int32, device=self.hand.device)
         self.waits = 0  # the library's bound

@@ -215,3 +215,20 @@ def test_failed_step_raises(monkeypatch):
         with pytest.raises(RuntimeError, match="waited too long"):
             read()
     DecodeSession(_Model(HybridProgram), 1, 16, 16).check()
+
+
+def test_small_step_keeps_what_it_points_to():
+    """A small model's step holds addresses of weights, norms and caches: it keeps them all alive when the model lets go of them."""
+    from lit_llama.model import LLaMA, LLaMAConfig, _SmallStep
+
+    model = LLaMA(LLaMAConfig(block_size=32, vocab_size=64, n_layer=2, n_head=8, n_embd=512)).to(torch.bfloat16)
+    model.kv_caches = [tuple(torch.zeros(1, 8, 32, 64, dtype=torch.bfloat16) for _ in range(2)) for _ in range(2)]
+    lins = [(b.attn.c_attn, b.attn.c_proj, b.mlp.c_fc1, b.mlp.c_fc2, b.mlp.c_proj) for b in model.transformer.h]
+    specs = {"layers": [[(1, lin.weight, None) for lin in layer] for layer in lins]}
+    step = _SmallStep(model, specs, 32)
+    at = [int(p) for p in step.layers]
+    held = [weakref.ref(t) for b, kv in zip(model.transformer.h, model.kv_caches) for t in (b.rms_1.scale, b.mlp.c_proj.weight, *kv)]
+    assert len(at) == 18 and {r().data_ptr() for r in held} <= set(at)
+    del model, specs, lins
+    gc.collect()
+    assert all(r() is not None for r in held)
