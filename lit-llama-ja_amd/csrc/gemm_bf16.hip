@@ -67,11 +67,12 @@ static int gemm_few_go(const GemmParams& p, hipStream_t s) {
   return 0;
 }
 
-// Up to 256 workgroups, of short sums 512 or 400,000 steps of K (the times above: 640 -> 1920 at 600 9.3 for the tiles' 9.6, at 960 11.3 for 10.0; 1024 -> 1024 at 512 8.1 for 10.7).
+// Up to 256 workgroups, of short sums 512 or 400,000 steps of K (the times above: 640 -> 1920 at 600 9.3 for the tiles' 9.6, at 960 11.3 for 10.0; 1024 -> 1024 at 512 8.1 for 10.7), but no more
+// than three a CU (256 -> 4608 at 864 7.8 for 6.7, 256 -> 4096 at 768 6.4 for 6.6 and at 1,024 7.8 for 6.6; 384 -> 8192 at 1,024 8.7 for 7.6, 384 -> 4096 at 768 6.9 for 7.6).
 // Only for the LLaMA entries: other models' logits move with the order of a product's sums. -1: not taken.
 int gemm_few_run(int ep, const GemmParams& p, hipStream_t s) {
   const long groups = (long)(p.N / 16) * ((p.M + 31) / 32);
-  if (p.M < 1 || p.K % 32 || p.K < 256 || p.K > 1792 || p.N % 16 || groups > (p.K > 1024 ? 256 : std::max(512, 400000 / p.K)) || (((uintptr_t)p.A | (uintptr_t)p.W) & 15) || (p.lda & 7)) return -1;
+  if (p.M < 1 || p.K % 32 || p.K < 256 || p.K > 1792 || p.N % 16 || groups > (p.K > 1024 ? 256 : std::min(768, std::max(512, 400000 / p.K))) || (((uintptr_t)p.A | (uintptr_t)p.W) & 15) || (p.lda & 7)) return -1;
   switch (ep) {
     case GEP_STORE: return gemm_few_go<GEP_STORE>(p, s);
     case GEP_RESID: return gemm_few_go<GEP_RESID>(p, s);

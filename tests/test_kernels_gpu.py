@@ -2262,7 +2262,7 @@ def test_attention_with_projection_shares(hip, nh, S, p, H):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(17, 640, 640), (32, 1920, 256), (33, 512, 384), (64, 384, 512), (63, 1536, 1024), (47, 640, 1792), (250, 512, 1536), (1, 128, 768)])
+@pytest.mark.parametrize("M,N,K", [(17, 640, 640), (32, 1920, 256), (33, 512, 384), (64, 384, 512), (63, 1536, 1024), (47, 640, 1792), (250, 512, 1536), (1, 128, 768), (96, 4096, 256), (96, 4608, 256)])
 def test_gemm_few_tiles_exact(hip, M, N, K):
     """Small bf16 products (32 rows and 16 columns to a workgroup, K over its waves) on integer values, whose sums are exact in any order: shares of equal
     and of different numbers of steps, a partial last block of rows; nothing outside, every epilogue but QKV's (which the prompt tests run)."""
