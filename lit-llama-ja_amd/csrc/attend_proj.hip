@@ -7,7 +7,11 @@
 //   two rows  4096  int4 9.3 -> 7.9 at 70 keys, 14.2 -> 13.3 at 500   8-bit 10.1 -> 9.2
 // The attention's workgroups may not have started when others wait for them (handover.h: beside three such launches at once, each XCD holding the
 // waiting workgroups of two). A workgroup whose wait runs out does the attention that is missing itself, to the same bits, and waits for nobody.
-// Three and four rows gain 0.1 to 0.7 (with ranges nothing) and eight lose 2: every workgroup takes all rows past the caches.
+// Three and four rows gain 0.1 to 0.7 (with ranges nothing) and eight lose 2: every workgroup takes all rows past the caches. Of two rows with eight
+// ranges 5120 gains nothing any more (int4 2,048 keys 27.5 -> 28.1, 600 keys 17.5 -> 16.6, 8-bit 30.5 -> 30.3 and 19.8 -> 19.6).
+// Widths: 4096 and 5120 of 7B and 13B, 2048 of models of that width with heads of 128. 6656 and 8192 (30B, 65B) are left out: one row of codes would
+// gain (int4 11.0 -> 9.4 and 13.2 -> 11.8 at 70 keys), two rows and bf16 with long caches would lose (6656: int4 23.8 -> 24.4, bf16 28.6 -> 30.7 at 1,000 keys;
+// 8192: two 8-bit rows 32.0 -> 39.0).
 #include <algorithm>
 
 #include "attention.h"

@@ -134,7 +134,10 @@ __global__ __launch_bounds__(NTH) void attention_kernel(const bf16_t* __restrict
 // launch of its own would store it; the next product adds the heads' shares up (rowdot.h, sums). A workgroup takes a head and 64 of Wp's rows, which are on
 // their way to registers (HS / 8 lanes and a piece of 16 bytes each to a row) over the attention's own memory trips; the head's other workgroups form
 // the same attention again, since a CU takes its 82 KB of Wp no faster than two launches take all of it. For small models, whose launches are
-// all latency. us a step of 49M (10 layers), launches of their own 193; a head's rows in one workgroup 201, in two 192, four 188, five 185, ten 183.
+// all latency, where small_step.hip does not take the step: forwards of one token outside a session and models of more than 16 layers. us a token, five
+// launches a layer -> four: 19M 340 -> 280, 49M 516 -> 416 (the host's calls), a session's step of 24 layers of 640 434 -> 411 at 30 tokens and 490 -> 482 at
+// 300, of 20 layers of 1024 404 -> 397 and 457 -> 449. (A session's step of 10 layers of 640 so, five launches 193: a head's rows in one
+// workgroup 201, in two 192, four 188, five 185, ten 183.)
 template <int HS, int U, int NTH>
 __global__ __launch_bounds__(NTH) void attention_proj_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
                                                              const int* __restrict__ pos, int S, int nh, float scale_log2, const bf16_t* __restrict__ W,

@@ -578,7 +578,8 @@ int llj_post_linear(int act, const void* t, const void* norm_w, float eps, const
   return post_gemv_launch<2>(p, act, s);  // C <= 8192 over 512 threads, C <= 4096 over 256
 }
 
-// whole rounds of chunks for every wave, and not the half-K forms' widths
+// K: the hybrid models' two widths, the two that were measured (above); every wave has whole rounds of its D chunks there. N: below 4096 columns the rows by
+// themselves take the half-K form, which adds in another order.
 int llj_post_rows_ok(int M, int N, int K, int C) {
   return M >= 2 && M <= 8 && C > 0 && C % 8 == 0 && C <= K && (K == 2048 || K == 4096) && N >= 4096 && N % 16 == 0 && N < (1 << 29) / K;
 }

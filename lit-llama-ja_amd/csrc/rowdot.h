@@ -347,7 +347,7 @@ __global__ __launch_bounds__(NW * 64) void rowdot_kernel(RowDotParams p) {
 template <int NW, int SL, int PRO, int EPI>
 static int rowdot_go(const RowDotParams& p, hipStream_t s) {
   const int units = p.N / 2;
-  int grid = (PRO > RD_SUMS ? 512 : 2048) / NW;  // (every workgroup of a sums prologue reads all of its rows: 49M 2048 198 us a step, 512 and 1024 185)
+  int grid = (PRO > RD_SUMS ? 512 : 2048) / NW;  // (every workgroup of a sums prologue reads all of its rows: a session's step of 10 layers of 640 with 2048 198 us, with 512 and 1024 185)
   grid = grid < units ? grid : units;
   // [column][NW * 4] sums of the largest range in 48 KiB (very wide outputs: more workgroups)
   const long most = 48 * 1024 / (NW * 16) - 2;

@@ -500,7 +500,12 @@ using namespace llj;
 
 extern "C" {
 
-// (up to 512 cache slots and from 512 values: what was measured, always for the better)
+// Up to 512 cache slots: a head's one workgroup walks all keys. us a session's step, this for launches of their own (those with heads of 64 as ops.hip's
+// shares), heads of 64 unless said:
+//   10 layers of 640  139 / 204 at 30 keys, 204 / 220 at 600 (640 slots), 222 / 221 at 740, 259 / 225 at 1,000   12 of 1024  185 / 267, 272 / 298, 292 / 303, 331 / 305
+//   12 layers of 780 (heads of 78)  194 / 234 at 30, 268 / 272 at 480, 290 / 278 at 600, 364 / 318 at 1,000   16 of 512, heads of 32  193 / 237, 272 / 266 at 480
+// From 512 values on, where one bf16 row's products run on rowdot.h. Any number of layers, though the second launch and the first one's clearing are 4 us of a step:
+// one layer takes 0.96 to 1.16 of its launches, two 0.88 to 1.14, three 0.84 to 1.12, six and more 0.75 to 1.03, the larger ones past 400 keys.
 int llj_small_step_ok(int L, int C, int H, int nh, int S) {
   return L >= 1 && L <= kSmLayers && nh >= 1 && C % nh == 0 && (C / nh) % 2 == 0 && C / nh <= 128 && C / nh >= 32 && C % 4 == 0 && C >= 512 && C <= 1024 &&
          H % 4 == 0 && H >= 2 * C && H <= 2816 && S >= 1 && S <= 512;

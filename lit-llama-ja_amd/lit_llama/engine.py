@@ -136,6 +136,7 @@ class LLaMAProgram(_Program):
 
         if _SmallStep.ok(m, s.specs, s.B, s.S):
             self.small = _SmallStep(m, s.specs, s.S)
+            s.work.parts = s.work.x2 = None  # (of the launches that it takes the place of)
 
     def reset_handoff(self):
         """The LLM.int8 hand-off blocks (_Work.y_st / h_st) must be zero when a step starts, and the attention's output (y_hand)

@@ -353,8 +353,8 @@ class _Work:
             nb = _hip.lib().llj_attention_ws_bytes(M, cfg.n_head, C // cfg.n_head, self.nsplit)
             self.att_ws = torch.empty(nb, dtype=torch.uint8, device=device)
             self.att_count = torch.zeros(M * cfg.n_head, dtype=torch.int32, device=device)
-        # one row of a small model, short cache: the attention leaves the heads' shares of c_proj, which the SwiGLU adds up
-        # (llj_attention_proj, llj_sums_swiglu) into the residual's other place
+        # one row of a small model, short cache, outside llj_small_step: the attention leaves the heads' shares of c_proj, which the SwiGLU
+        # adds up (llj_attention_proj, llj_sums_swiglu) into the residual's other place
         self.parts = self.x2 = None
         if (M == 1 and self.nsplit <= 1 and not need_i8 and not gemm and C % cfg.n_head == 0
                 and _hip.lib().llj_attention_proj_ok(cfg.n_head, C // cfg.n_head, S)):
