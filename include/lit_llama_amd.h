@@ -535,7 +535,7 @@ int llj_rows_linear(int act, const void* A, int lda, const void* W, const float*
 int llj_post_linear(int act, const void* t, const void* norm_w, float eps, const float* x, float* x_out, int C,
                     const void* W, void* out, int N, int K, void* stream);
 /* The same for 2 to 8 rows (strides ldt, ldx, ldo): llj_post_norm, then llj_rows_linear with LLJ_ACT_TILES, in one launch and to their bits.
- * llj_post_rows_ok: K of 2048 or 4096, N of 4096 columns on. */
+ * K of 2048 or 4096, N of 4096 columns on. llj_post_rows_ok: where it is the faster of the two. */
 int llj_post_rows_ok(int M, int N, int K, int C);
 int llj_post_rows(int act, const void* t, int ldt, const void* norm_w, float eps, const float* x, float* x_out, int ldx, int C, const void* W,
                   void* out, int ldo, int M, int N, int K, void* stream);

@@ -578,15 +578,25 @@ int llj_post_linear(int act, const void* t, const void* norm_w, float eps, const
   return post_gemv_launch<2>(p, act, s);  // C <= 8192 over 512 threads, C <= 4096 over 256
 }
 
-// K: the hybrid models' two widths, the two that were measured (above); every wave has whole rounds of its D chunks there. N: below 4096 columns the rows by
+// K: the hybrid models' two widths, the two that were measured; every wave has whole rounds of its D chunks there. N: below 4096 columns the rows by
 // themselves take the half-K form, which adds in another order.
-int llj_post_rows_ok(int M, int N, int K, int C) {
+static bool post_rows_takes(int M, int N, int K, int C) {
   return M >= 2 && M <= 8 && C > 0 && C % 8 == 0 && C <= K && (K == 2048 || K == 4096) && N >= 4096 && N % 16 == 0 && N < (1 << 29) / K;
+}
+
+// Where it is the faster. Up to 4 rows: everywhere (within 0.9 us where it is not). 5 to 8 rows cost every workgroup 1.3 us more, which pays where the product alone leaves
+// most of a round of 256 workgroups empty. us with the product before it, norm and product -> this, 5 / 8 rows:
+//   4096 ->  4352 21.4 / 22.5 -> 21.7 / 22.6   8448 25.3 / 27.5 -> 25.2 / 26.3   12544 30.6 / 31.4 -> 30.4 / 31.3   16512 34.2 / 36.8 -> 34.6 / 35.9, but
+//            4096 18.5 / 18.7 -> 20.1 / 21.2   7168 22.7 / 23.6 -> 24.0 / 24.6    8192 22.9 / 24.6 -> 24.6 / 25.8   12288 28.1 / 29.2 -> 29.8 / 31.0
+//   2048 ->  4352 13.5 / 14.0 -> 12.9 / 13.9   6272 13.8 / 15.4 -> 13.5 / 14.5    8448 15.6 / 17.1 -> 16.2 / 16.7, but
+//            4096 12.3 / 12.4 -> 12.8 / 13.5  12288 17.1 / 18.4 -> 18.2 / 18.7   12544 18.7 / 18.8 -> 20.1 / 20.6   26112 26.2 / 28.3 -> 26.9 / 27.5
+int llj_post_rows_ok(int M, int N, int K, int C) {
+  return post_rows_takes(M, N, K, C) && (M <= 4 || (K == 2048 ? N > 4096 && N < 12288 : (N / 16 - 1) % 256 < 64));
 }
 
 int llj_post_rows(int act, const void* t, int ldt, const void* norm_w, float eps, const float* x, float* x_out, int ldx, int C, const void* W,
                   void* out, int ldo, int M, int N, int K, void* stream) {
-  LLJ_REQUIRE((act == 0 || act == 1) && t && norm_w && x && x_out && x != x_out && W && out && llj_post_rows_ok(M, N, K, C) && ldt >= C && ldx >= C &&
+  LLJ_REQUIRE((act == 0 || act == 1) && t && norm_w && x && x_out && x != x_out && W && out && post_rows_takes(M, N, K, C) && ldt >= C && ldx >= C &&
               ldo >= N && (ldt & 7) == 0 && (ldx & 3) == 0 &&
               (((uintptr_t)t | (uintptr_t)norm_w | (uintptr_t)x | (uintptr_t)x_out | (uintptr_t)W) & 15) == 0);
   PostGemvParams p{};

@@ -284,3 +284,17 @@ def test_gptq_cli_tokenizer_selection(tmp_path):
 
     HFTok(WordLevel({"<pad>": 0, "a": 1}, unk_token="<pad>")).save(str(tmp_path / "t.json"))
     assert isinstance(tokenizer_for(tmp_path / "t.json"), HFTokenizer)
+
+
+@pytest.mark.parametrize("K", [2048, 4096])
+def test_post_rows_rule(K):
+    """llj_post_rows_ok on both sides of its lines: 5 to 8 rows only where the product alone leaves most of a round of 256 workgroups empty (K = 4096) or is
+    one round (2048), fewer rows everywhere; nothing that llj_post_rows refuses."""
+    from lit_llama import _hip
+
+    ok = lambda M, N, C=K: bool(_hip.lib().llj_post_rows_ok(M, N, K, C))  # noqa: E731
+    assert all(ok(M, N) for M in (2, 3, 4) for N in (4096, 8192, 12288, 20480))
+    few = {2048: (4096, 12288, 12544), 4096: (4096, 6144, 8192, 12288, 20480)}[K]
+    many = {2048: (4112, 6272, 8448, 12272), 4096: (4112, 5120, 8448, 12544, 16512)}[K]
+    assert not any(ok(M, N) for M in (5, 8) for N in few) and all(ok(M, N) for M in (5, 8) for N in many)
+    assert not (ok(1, 8448) or ok(9, 8448) or ok(2, 4080) or ok(2, 8440) or ok(2, 8448, K + 8) or ok(2, 8448, K - 4))
