@@ -2377,7 +2377,7 @@ def test_attention_and_projection_in_one_launch(hip, wfmt, M, nh, S, p, nsplit):
     bad.view(torch.int16).fill_(-1)
     run(9, x, bad)
     torch.cuda.synchronize()
-    assert x.isnan().all()
+    assert x.isnan().all() and (places[1] != -1).all() and places[1].view(torch.bfloat16).isnan().all()
 
 
 @pytest.mark.parametrize("wfmt,M,nh,S,p,nsplit", [(0, 1, 32, 96, 0, 1), (0, 2, 40, 600, 500, 3), (1, 1, 32, 1033, 1000, 5), (1, 1, 40, 130, 128, 1), (1, 1, 16, 40, 100, 1),

@@ -859,6 +859,29 @@ def test_small_model_step_done_again(n_embd, n_head, n_layer, S):
     assert torch.equal(s.feed([int(ids[12])])[0], want[0])
 
 
+@pytest.mark.parametrize("n_embd,n_head", [(640, 10), (780, 10)])
+def test_small_model_step_of_marks(n_embd, n_head):
+    """A token whose embedding is all ones, the mark of a word that is not there yet: as NaN it goes through every row of the step, no wait runs out and the
+    second launch has nothing to do; the next prompt's steps are as before it. An embedding with infinities likewise."""
+    from lit_llama import engine
+
+    cfg = Cfg(block_size=64, n_layer=3, n_head=n_head, n_embd=n_embd, vocab_size=512)
+    m = build(cfg, make_params(cfg, 9))
+    m.transformer.wte.weight.data[5].view(torch.int16).fill_(-1)
+    m.transformer.wte.weight.data[6, ::7] = float("inf")
+    ids = torch.from_numpy(np.random.default_rng(9).integers(7, 512, (1, 10))).cuda()
+    s = engine.DecodeSession(m, 1, 32, 32, top_k=1)
+    s.prefill(ids)
+    want = s.feed([7]).clone()
+    assert want.isfinite().all()
+    for token in (5, 6):
+        s.prefill(ids)
+        assert s.feed([token]).isnan().all()
+        assert int(s.program.small.hand[-(n_embd // 2 + 32)]) == -1 and int(s.program.small.failed) == 0
+        s.prefill(ids)
+        assert torch.equal(s.feed([7]), want)
+
+
 def test_small_model_steps_on_two_streams():
     """Two sessions' steps at once, each launch of more workgroups than the chip holds: both end, with the bits that each has alone."""
     import threading
