@@ -104,24 +104,25 @@ __device__ __forceinline__ bool ap_bf16_row(const AttendProjParams& p, int nt, u
 
 // The attention's workgroup of row m, head h and range split
 template <int HS, bool RANGES>
-__device__ __forceinline__ void ap_attend(const AttendProjParams& p, int h, int m, int split, int* count, float* lds) {
+__device__ __forceinline__ void ap_attend(const AttendProjParams& p, int h, int m, int split, int* count, bool spec, float* lds) {
   attention_body<HS, 4, kApNT, RANGES, 2, false, false, true>(p.q, p.kc, p.vc, reinterpret_cast<bf16_t*>(p.y), p.pos, 1, p.S, p.nh,
-                                                              p.scale_log2, h, m, lds, p.nsplit, split, p.part, nullptr, 0.f, nullptr, 0,
-                                                              p.heads <= 64, count);
+                                                              p.scale_log2, h, m, lds, p.nsplit, split, p.part, nullptr, 0.f, nullptr, 0, spec,
+                                                              count);
 }
 
 // Every head whose words are not all there, as its own workgroups form it (and store it too, when they come to run: the same values at the same
-// places). The workgroups start at different heads. All of y is there afterwards.
+// places). The workgroups start at different heads. All of y is there afterwards. (Its code costs the others: with requests ahead of the position and a loop
+// over one range 7B int4 took 1,035 us a step for 1,021.)
 template <int HS, bool RANGES>
 __device__ __forceinline__ void ap_missing(const AttendProjParams& p, int nt, float* lds) {
-  const int n = p.nh * p.M;
+  const int n = p.nh * p.M, splits = RANGES ? p.nsplit : 1;
   for (int i = 0; i < n; ++i) {
     const int at = (nt + i) % n, h = at % p.nh, m = at / p.nh;
     const uint32_t w = get_word(p.y, (m * p.C + h * HS) / 2 + (int)(threadIdx.x & (HS / 2 - 1)));
     if (__syncthreads_and(w != kNotYet)) continue;
-    for (int s = 0; s < p.nsplit; ++s) {
+    for (int s = 0; s < splits; ++s) {
       if (s) __syncthreads();  // (LDS)
-      ap_attend<HS, RANGES>(p, h, m, s, nullptr, lds);
+      ap_attend<HS, RANGES>(p, h, m, s, nullptr, false, lds);
     }
     if constexpr (RANGES) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials are out
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(kApNT) void attend_proj_kernel(AttendProjParams p) 
   __shared__ __align__(16) unsigned char smem[std::max(attention_lds_floats<HS, kApNT>() * 4, kProj)];
   if ((int)blockIdx.x < p.heads) {
     const int h = blockIdx.x % p.nh, rest = blockIdx.x / p.nh, m = MR > 1 ? rest % p.M : 0, split = MR > 1 ? rest / p.M : rest;
-    ap_attend<HS, RANGES>(p, h, m, split, p.count, reinterpret_cast<float*>(smem));
+    ap_attend<HS, RANGES>(p, h, m, split, p.count, p.heads <= 64, reinterpret_cast<float*>(smem));
     return;
   }
   const int nt = blockIdx.x - p.heads;
