@@ -302,11 +302,12 @@ __global__ __launch_bounds__(256) void gptq_panel_kernel(const float* __restrict
 }
 
 constexpr int kStepLds = kFactor * kFs, kStepAlone = 21000;  // floats: the diagonal block's, and more than half a CU's LDS
-// Tiles of a step up to which workgroup 0 has its CU to itself (ALONE), so that its chain is not held up: up to 8 tiles a CU the chain is the longer. Past that
+// Tiles of a step up to which workgroup 0 has its CU to itself (ALONE), so that its chain is not held up: up to some 8 tiles a CU the chain is the longer. Past that
 // the products are, and one workgroup of theirs a CU, which ALONE makes of them too, is too few. ms of a factor, all steps alone -> by this rule
-// (two a CU in all): 4,096 columns 1.31 -> 1.31 (1.39), 5,120 2.01 -> 1.82 (1.86), 6,144 3.08 -> 2.62 (2.65), 8,192 6.52 -> 5.31 (5.33),
-// 11,008 15.3 -> 12.3 (12.3), 13,824 29.5 -> 24.1 (24.1); with 1,536 tiles 4,096 columns take 1.35, with 3,072 5,120 take 1.95.
-constexpr long kAloneTiles = 2048;
+// (two a CU in all): 4,096 columns 1.28 -> 1.28 (1.39), 5,120 2.01 -> 1.80 (1.86), 6,144 3.08 -> 2.62 (2.65), 8,192 6.52 -> 5.31 (5.33),
+// 11,008 15.3 -> 12.3 (12.3), 13,824 29.5 -> 24.1 (24.1); with 1,536 tiles 4,096 columns take 1.35, with 2,048 1.31 (their first
+// steps have up to 2,077), with 3,072 5,120 take 1.95.
+constexpr long kAloneTiles = 2100;
 
 // Workgroup 0: the next diagonal block, updated and factored. The others: 64 x 64 tiles of the rows below, the lower triangle's columns
 // up to block k (first sums in block k's own) and the upper triangle's.
