@@ -328,25 +328,23 @@ def time_dominant_kernel(model, B, iters=10):
 
 # the dominant decode launch (W4, fused RMSNorm, SwiGLU; 4 waves, 2 chunks in flight, one row)
 DOMINANT = "llj::gemv_kernel<0, 2, 3, 4, 2, 1, 1>"
+GRAPH_STATS = "decode_graph_kernel_stats.csv"  # in profiles/
 
 
 def graph_kernel_us(kernel_prefix: str = "void " + DOMINANT):
-    """In-graph average duration of the dominant launch from the newest committed kernel trace of
-    the decode graph alone: profiles/<round>_graph_kernel_stats.csv, the rocprofv3 --kernel-trace
-    --stats summary of `bench.py --decode-only` (graph replays only: no isolated loop in the
-    process, so the average is over launches inside the captured chain). None when absent."""
+    """In-graph average duration of the dominant launch from the committed kernel trace of the decode graph alone
+    (GRAPH_STATS): the rocprofv3 --kernel-trace --stats summary of `bench.py --decode-only` (graph replays only: no isolated
+    loop in the process, so the average is over launches inside the captured chain). None when absent."""
     import csv
 
-    best = None
-    for p in sorted((REPO / "profiles").glob("r*_graph_kernel_stats.csv")):
-        try:
-            with open(p) as f:
-                for r in csv.DictReader(f):
-                    if r["Name"].startswith(kernel_prefix):
-                        best = (float(r["AverageNs"]) / 1e3, p.name)
-        except (OSError, KeyError, ValueError):
-            continue
-    return best
+    try:
+        with open(REPO / "profiles" / GRAPH_STATS) as f:
+            for r in csv.DictReader(f):
+                if r["Name"].startswith(kernel_prefix):
+                    return float(r["AverageNs"]) / 1e3, GRAPH_STATS
+    except (OSError, KeyError, ValueError):
+        pass
+    return None
 
 
 def achievable_read_gbs(gb: float = 4.0, iters: int = 5):
