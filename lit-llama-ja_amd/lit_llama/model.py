@@ -256,7 +256,7 @@ def _enable_attend(w: "_Work", specs, B: int, T: int, nh: int) -> None:
 
 
 class _SmallStep:
-    """A session's decode step of one row of a small bf16 model: all layers in one launch (llj_small_step)."""
+    """A session's decode step of one row of a small bf16 model: all layers in one launch, and one for what that left undone (llj_small_step)."""
 
     def __init__(self, model: "LLaMA", specs, S: int):
         cfg, L = model.config, _hip.lib()
